@@ -1,707 +1,776 @@
-// First-party CDNA4 flash attention (forward + backward) for the learner's
-// teacher-forced training pass and the engine's long-prompt prefill —
-// replaces torch SDPA (aotriton, Triton-derived) on the hot path
-// (reference distributed_actor.py:241-243 forward + loss.backward();
-// SURVEY.md §2.4-B "causal attention fwd/bwd" row; north star: no Triton).
+// Causal GQA flash attention, forward and backward, for the learner's
+// teacher-forced pass and the engine's prompt phase (reference
+// distributed_actor.py:241-243 forward + loss.backward()).
 //
-// Design (MFMA 16x16x32, online softmax, batched causal GQA):
-//  * The S-matrix is never materialized: per 64-row Q block (4 waves x 16
-//    rows), KV is streamed in 32-token tiles through LDS.
-//  * Every MFMA operand is a ROW-MAJOR fragment: QK^T is computed in the
-//    SWAPPED orientation ST[kv][q] = mfma(A=K rows, B=Q rows), so softmax
-//    statistics reduce over the register rows + two cross-lane shuffles,
-//    and P@V consumes a PRE-TRANSPOSED V (v_t = V^T, one cheap torch
-//    transpose per call) so its B fragments are row-major reads too.
-//  * The only layout conversion is D-layout (f32 accumulator) ->
-//    A/B-fragment (bf16), done in-register with v_cvt_pk_bf16_f32 + 8
-//    ds_bpermute per 16x32 fragment (guide T12's idea at 16x16 shape).
-//  * Backward runs in two passes with NO atomics: pass Q (q-block outer,
-//    recomputes ST from the saved row LSE, produces dQ) and pass KV
-//    (kv-block outer in the UNSWAPPED orientation, produces dK^T/dV^T).
-//    delta = rowsum(dO*O) is computed by the host in torch.
+// Layout. q, o, dout, dq are (B, Hq, T, D) and k, v, dk, dv (B, Hkv, T, D)
+// with any strides whose innermost one is 1: the model's (B, T, H, D)
+// projections go in and come out without a copy. The prompt phase passes
+// one flat (tokens, H, D) batch with row offsets instead of padded rows.
 //
-// Fragment mapping (mfma_f32_16x16x32_bf16, same as nf4_gemm.hip):
-//   A: lane l holds A[row = l&15][k = (l>>4)*8 + j]
-//   B: lane l holds B[col = l&15][k = (l>>4)*8 + j]   (D = A @ B^T)
-//   D: lane l, reg r -> row = (l>>4)*4 + r, col = l&15
+// Products run on MFMA 32x32x16. A wave owns 32 rows (queries in the
+// forward and the dQ pass, keys in the dK/dV pass) whose operands stay in
+// registers; the other side streams through LDS in double-buffered tiles,
+// fetched into registers one tile ahead. Scores are formed transposed,
+// ST[key][query] = K Q^T (dK/dV: S[query][key] = Q K^T), so that
+//  * a lane holds 16 scores of ONE query of each 32x32 block: the softmax
+//    reduces in registers and over one lane swap, and rescaling the output
+//    is a lane-local multiply;
+//  * the accumulator's rows {4h..4h+3, 8+4h..8+4h+3} (h = lane / 32) of a
+//    16-row step serve directly as the next product's k-slots: packing to
+//    bf16 is the only conversion. The other operand is read with the same
+//    k order, by LDS transpose reads from the row-major tile, so nothing is
+//    ever transposed in memory.
+// Bound: LDS reads (1 KB per MFMA and wave, 128 B/clk) run level with the
+// matrix cores here; two workgroups a CU let one's softmax overlap the
+// other's products.
+//
+// A tile row is XOR-swizzled in 16 B chunks by swz(row): 8 consecutive rows
+// read at one chunk (row fragments) and 4 rows read over 64 B (transpose
+// reads) both fall into different banks.
+//
+// The backward has two passes and no atomics: results do not depend on the
+// order of workgroups. dQ (query rows) also forms delta = rowsum(dO * O);
+// dK/dV (key rows) walks the query heads of its kv head and adds them up in
+// fp32 registers; where key blocks alone leave the chip idle, the heads are
+// split over workgroups that leave fp32 partials for a small sum kernel.
+//
+// Measured at B 16, 28/4 heads, T 1550, D 128 (275 GFLOP in the causal half,
+// forward): forward 425 us = 650 TFLOP/s, dQ 597 us, dK/dV 1208 us + 39 us for
+// the sum; 16-row waves on 16x16x32 with single-buffered tiles and transposed
+// copies of q, k, v, dout took 1161, 2097 and 3466 us + 1.9 ms of copies and
+// sums. What bounds them now: vector work beside the products (10 vector
+// instructions a product in the forward) at two waves a SIMD.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16v8;
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16v4;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16v2;
+typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+typedef __attribute__((address_space(3))) bf16v4 lds_bf16v4;
 
 namespace {
 
-constexpr int QB = 16;    // q rows per wave
-constexpr int KVB = 32;   // kv tile
-constexpr int NWAVE = 4;  // waves per block -> 64 q rows per block
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float LN2 = 0.6931471805599453f;
+constexpr int WROWS = 32;   // rows a wave owns
 
-DEV_INLINE float wave_xor_max(float v) {
-  v = fmaxf(v, __shfl_xor(v, 16, 64));
-  v = fmaxf(v, __shfl_xor(v, 32, 64));
-  return v;
+// Keys of a tile: two waves share the fetch of a smaller one, or their
+// prefetch registers would spill.
+template <int NW>
+constexpr int tile_rows() { return NW == 4 ? 64 : 32; }
+
+// element strides of a (B, H, T, D) operand
+struct Strides { int64_t b, h; int t; };
+
+DEV_INLINE f32x16 mfma(bf16v8 a, bf16v8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-DEV_INLINE float wave_xor_sum(float v) {
-  v += __shfl_xor(v, 16, 64);
-  v += __shfl_xor(v, 32, 64);
-  return v;
+DEV_INLINE f32x16 zero16() {
+  f32x16 z;
+  #pragma unroll
+  for (int i = 0; i < 16; ++i) z[i] = 0.f;
+  return z;
 }
 
-// Pack two f32 into one dword of bf16x2 (round-to-nearest-even).
-DEV_INLINE uint32_t cvt_pk_bf16(float lo, float hi) {
-  union { __hip_bfloat162 h; uint32_t u; } cv;
-  cv.h = __float22bfloat162_rn(float2{lo, hi});
-  return cv.u;
+// maximum and sum over the two half-waves
+DEV_INLINE float halves_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+DEV_INLINE float halves_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// D-layout -> A/B-fragment relayout.
-// Sources: two 16x16 D-layout tiles T0 (k-rows 0-15) and T1 (k-rows
-// 16-31) over the SAME preserved column index c = l&15; lane l holds
-// T[4*(l>>4)+r][l&15]. Target: bf16v8 with lane l = F[c = l&15]
-// [k = 8*(l>>4)+j]. Each lane pulls two packed dwords from source lanes
-// s0/s1 of T0 AND T1, then selects by its own group half.
-DEV_INLINE bf16v8 relayout_frag(const f32x4& t0, const f32x4& t1) {
-  const int l = threadIdx.x & 63;
-  const int g = l >> 4;
-  const int c = l & 15;
-  const uint32_t a0_0 = cvt_pk_bf16(t0[0], t0[1]);
-  const uint32_t a1_0 = cvt_pk_bf16(t0[2], t0[3]);
-  const uint32_t a0_1 = cvt_pk_bf16(t1[0], t1[1]);
-  const uint32_t a1_1 = cvt_pk_bf16(t1[2], t1[3]);
-  const int s0 = ((g & 1) << 5) + c;        // source lane: group 2*(g&1)
-  const int s1 = s0 + 16;                   // group 2*(g&1)+1
-  union { uint32_t w[4]; bf16v8 v; } out;
-  const uint32_t p00 = __shfl((int)a0_0, s0, 64), p01 = __shfl((int)a1_0, s0, 64);
-  const uint32_t p02 = __shfl((int)a0_0, s1, 64), p03 = __shfl((int)a1_0, s1, 64);
-  const uint32_t p10 = __shfl((int)a0_1, s0, 64), p11 = __shfl((int)a1_1, s0, 64);
-  const uint32_t p12 = __shfl((int)a0_1, s1, 64), p13 = __shfl((int)a1_1, s1, 64);
-  const bool hi = g >= 2;                   // k 16..31 -> T1
-  out.w[0] = hi ? p10 : p00;
-  out.w[1] = hi ? p11 : p01;
-  out.w[2] = hi ? p12 : p02;
-  out.w[3] = hi ? p13 : p03;
-  return out.v;
+// the wave's number as a scalar, so that branches on its rows are scalar too
+DEV_INLINE int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+
+template <int D>
+DEV_INLINE int swz(int row) {
+  return D == 128 ? ((row & 3) << 2) | ((row >> 2) & 3)
+                  : (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
 }
 
-// LDS tile staging: [ROWS][COLS] bf16 row-major with an XOR swizzle on
-// the 16-B column slot, MASKED to the row width (COLS/8 slots per row)
-// so it never escapes the row — (row & 15) << 4 for 256-B rows,
-// (row & 3) << 4 for 64-B rows. Readers use lds_frag with the same XOR.
-// Guards rows >= limit with zero fill.
-template <int COLS>
-DEV_INLINE int tile_off(int row, int cu) {
-  constexpr int SWZ_MASK = (COLS / 8) - 1;
-  return (row * (COLS * 2) + cu * 16) ^ ((row & SWZ_MASK) << 4);
-}
+// One ROWS x D tile: fetched into registers, then stored to LDS.
+template <int D, int ROWS, int NT>
+struct Tile {
+  static constexpr int UN = D / 8, STEP = NT / UN;     // rows NT threads cover
+  static constexpr int PER = ROWS / STEP;
+  static_assert(NT % UN == 0 && ROWS % STEP == 0, "tile does not divide");
+  u32x4 r[PER];
 
-template <int ROWS, int COLS>
-DEV_INLINE void stage_tile(char* lds, const __hip_bfloat16* src,
-                           int64_t src_row_stride, int rows_valid, int tid,
-                           int nthreads) {
-  constexpr int UN = COLS / 8;  // bf16x8 units per row
-  for (int i = tid; i < ROWS * UN; i += nthreads) {
-    const int row = i / UN;
-    const int cu = i % UN;
-    bf16x8 v;
-    if (row < rows_valid) {
-      v = *reinterpret_cast<const bf16x8*>(src + (int64_t)row * src_row_stride
-                                           + cu * 8);
+  // base is wave-uniform: a full tile's loads share one lane offset. Rows past
+  // the end repeat the last one, their weights are zero. (A branch around
+  // each load would make the loads wait for one another.)
+  DEV_INLINE void fetch(const __hip_bfloat16* base, int stride_t, int valid) {
+    const int row = threadIdx.x / UN, cu = threadIdx.x % UN;
+    if (valid >= ROWS) {
+      const int off = row * stride_t + cu * 8;
+      #pragma unroll
+      for (int i = 0; i < PER; ++i)
+        r[i] = *reinterpret_cast<const u32x4*>(base + (int64_t)(i * STEP) * stride_t + off);
     } else {
       #pragma unroll
-      for (int j = 0; j < 8; ++j) v.v[j] = f2bf(0.f);
+      for (int i = 0; i < PER; ++i)
+        r[i] = *reinterpret_cast<const u32x4*>(base + min(i * STEP + row, valid - 1) * stride_t
+                                               + cu * 8);
     }
-    *reinterpret_cast<bf16x8*>(lds + tile_off<COLS>(row, cu)) = v;
+  }
+  DEV_INLINE void store(char* lds) const {
+    #pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int row = i * STEP + threadIdx.x / UN, cu = threadIdx.x % UN;
+      *reinterpret_cast<u32x4*>(lds + row * (2 * D) + ((cu ^ swz<D>(row)) << 4)) = r[i];
+    }
+  }
+};
+
+// Lane offsets of the two kinds of fragment of a tile.
+template <int D>
+struct Frags {
+  int row_off;         // row fragment: row l&31, chunk h
+  int tr_lo, tr_hi;    // transpose reads: rows 4h + (l&15)/4 and 8 further
+
+  DEV_INLINE Frags() {
+    const int l = threadIdx.x & 63, h = l >> 5;
+    const int row = l & 31;
+    row_off = row * (2 * D) + ((h ^ swz<D>(row)) << 4);
+    const int x = ((l >> 4) & 1) * 2 + ((l & 3) >> 1);
+    const int r0 = 4 * h + ((l & 15) >> 2), r1 = r0 + 8;
+    tr_lo = r0 * (2 * D) + ((x ^ swz<D>(r0)) << 4) + (l & 1) * 8;
+    tr_hi = r1 * (2 * D) + ((x ^ swz<D>(r1)) << 4) + (l & 1) * 8;
+  }
+  // rows sub*32 + (l&31), elements ks*16 + h*8 ..
+  DEV_INLINE bf16v8 row(const char* lds, int sub, int ks) const {
+    return *reinterpret_cast<const bf16v8*>(lds + sub * (32 * 2 * D) + (row_off ^ (ks << 5)));
+  }
+  // element column dt*32 + (l&31), rows k0 + {4h.., 8+4h..}; k0 % 16 == 0
+  DEV_INLINE bf16v8 col(char* lds, int k0, int dt) const {
+    char* p = lds + k0 * (2 * D);
+    const bf16v4 a = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+        (lds_bf16v4*)(p + (tr_lo ^ (dt << 6))));
+    const bf16v4 b = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+        (lds_bf16v4*)(p + (tr_hi ^ (dt << 6))));
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+};
+
+// two floats rounded to nearest even (v_cvt_pk_bf16_f32)
+DEV_INLINE bf16v2 round2(float a, float b) {
+  return __builtin_convertvector(f32x2{a, b}, bf16v2);
+}
+
+// accumulator rows 8*k .. 8*k+7 of this lane as bf16 k-slots of a 16-row step
+DEV_INLINE bf16v8 pack8(const f32x16& s, int k) {
+  bf16v8 out;
+  #pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const bf16v2 v = round2(s[8 * k + 2 * j], s[8 * k + 2 * j + 1]);
+    out[2 * j] = v[0];
+    out[2 * j + 1] = v[1];
+  }
+  return out;
+}
+
+// row index within a 32-row block of accumulator register r
+DEV_INLINE int acc_row(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
+
+// this lane's row of a (rows, D) operand as fragments
+template <int D>
+DEV_INLINE void load_row(bf16v8 (&f)[D / 16], const __hip_bfloat16* base, int stride_t, int row) {
+  const int h = (threadIdx.x & 63) >> 5;
+  #pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks)
+    f[ks] = *reinterpret_cast<const bf16v8*>(base + (int64_t)row * stride_t + ks * 16 + h * 8);
+}
+
+// acc[dt] holds X^T (rows d, column = this lane's row): write the row times f.
+// Two half-waves hold alternating groups of four d; one swap makes 16 B runs.
+template <int D>
+DEV_INLINE void store_rows(const f32x16 (&acc)[D / 32], float f, __hip_bfloat16* row, bool valid) {
+  const int h = (threadIdx.x & 63) >> 5;
+  #pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt) {
+    #pragma unroll
+    for (int g = 0; g < 2; ++g) {       // d 16g .. 16g+15 of the 32
+      uint32_t w[4];
+      #pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        w[j] = __builtin_bit_cast(
+            uint32_t, round2(acc[dt][8 * g + 2 * j] * f, acc[dt][8 * g + 2 * j + 1] * f));
+      }
+      const auto x = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+      const auto y = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+      if (valid)
+        *reinterpret_cast<u32x4*>(row + dt * 32 + g * 16 + h * 8) = u32x4{x[0], y[0], x[1], y[1]};
+    }
   }
 }
 
-template <int COLS>
-DEV_INLINE bf16v8 lds_frag(const char* lds, int row, int col8) {
-  return *reinterpret_cast<const bf16v8*>(lds + tile_off<COLS>(row, col8));
+// The same rows in fp32 (partial sums of a head split).
+template <int D>
+DEV_INLINE void store_rows_f32(const f32x16 (&acc)[D / 32], float* row, bool valid) {
+  const int h = (threadIdx.x & 63) >> 5;
+  if (!valid) return;
+  #pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt)
+    #pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(row + dt * 32 + g * 8 + h * 4) =
+          f32x4{acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]};
+}
+
+// Workgroups go to the 8 XCDs in turn; give each XCD one contiguous share of
+// the work so that the heads and row blocks of a kv head meet in one L2.
+DEV_INLINE int xcd_share(int id, int total) {
+  const int x = id & 7, i = id >> 3, q = total >> 3, r = total & 7;
+  return x * q + min(x, r) + i;
 }
 
 // ---------------------------------------------------------------- forward
-// o[b,h,q,d], lse[b,h,q] from q/k/v. q,k: (B,H*/Hkv,T,D) row-major over
-// (T,D); v_t: (B,Hkv,D,T) (V pre-transposed). Causal. T arbitrary.
-template <int D>
-__global__ __launch_bounds__(256)
-void flash_fwd_kernel(const __hip_bfloat16* __restrict__ q,
-                      const __hip_bfloat16* __restrict__ k,
-                      const __hip_bfloat16* __restrict__ vt,
-                      __hip_bfloat16* __restrict__ o,
-                      float* __restrict__ lse,
-                      int B, int Hq, int Hkv, int T, int Tp, float scale) {
-  const int qblk = blockIdx.x;          // 64-row q block
-  const int h = blockIdx.y;
-  const int b = blockIdx.z;
-  const int kvh = h / (Hq / Hkv);
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int l = tid & 63;
-  const int lg = l >> 4;
-  const int lc = l & 15;
+// Lengths: T for every sequence, or rows cu[b] .. cu[b+1] of a flat batch.
+template <int D, int NW>
+__global__ __launch_bounds__(NW * 64, 2)
+void flash_fwd_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16* __restrict__ k,
+                      const __hip_bfloat16* __restrict__ v, __hip_bfloat16* __restrict__ o,
+                      float* __restrict__ lse, const int* __restrict__ cu, Strides sq, Strides sk,
+                      Strides sv, Strides so, int Hq, int Hkv, int T, int nq, float scale_log2) {
+  constexpr int KV = tile_rows<NW>(), NS = KV / 32, NT = NW * 64;
+  const int group = Hq / Hkv;
+  int id = xcd_share(blockIdx.x, gridDim.x);
+  const int hg = id % group;
+  id /= group;
+  const int qb = nq - 1 - id % nq;      // longest rows first
+  id /= nq;
+  const int kvh = id % Hkv, b = id / Hkv;
+  const int h = kvh * group + hg;
+  const int row0 = cu ? cu[b] : 0;
+  const int len = cu ? cu[b + 1] - row0 : T;
+  if (qb * (NW * WROWS) >= len) return;
 
-  const int q0 = qblk * (QB * NWAVE) + wave * QB;  // this wave's q rows
-  const int q_end = min(q0 + QB, T);  // waves past T still hit barriers
+  const int wave = wave_id(), l = threadIdx.x & 63, half = l >> 5;
+  const int q0 = qb * (NW * WROWS) + wave * WROWS;
+  const int qq = q0 + (l & 31);
+  const __hip_bfloat16* qp = q + b * sq.b + h * sq.h + (int64_t)row0 * sq.t;
+  const __hip_bfloat16* kp = k + b * sk.b + kvh * sk.h + (int64_t)row0 * sk.t;
+  const __hip_bfloat16* vp = v + b * sv.b + kvh * sv.h + (int64_t)row0 * sv.t;
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  char* k_lds = smem;                        // KVB x D bf16 (swizzled)
-  char* v_lds = k_lds + KVB * D * 2;         // D x KVB bf16 (swizzled)
-  float* o_lds = reinterpret_cast<float*>(v_lds + (size_t)D * KVB * 2);
-  // o_lds: per-wave 16 x D f32 staging for the epilogue (NWAVE*16*D)
+  constexpr int TB = KV * D * 2;
+  const Frags<D> fr;
+  bf16v8 qf[D / 16];
+  load_row<D>(qf, qp, sq.t, min(qq, len - 1));  // rows past the end are not stored
 
-  const __hip_bfloat16* qp = q + (((int64_t)b * Hq + h) * T) * D;
-  const __hip_bfloat16* kp = k + (((int64_t)b * Hkv + kvh) * T) * D;
-  const __hip_bfloat16* vp = vt + (((int64_t)b * Hkv + kvh) * D) * Tp;
-
-  // Q fragments: B[col = q-row = lc][kd = lg*8+j], one per 32-d step.
-  bf16v8 qf[D / 32];
-  {
-    const int row = q0 + lc;
-    #pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) {
-      if (row < T) {
-        qf[ks] = *reinterpret_cast<const bf16v8*>(
-            qp + (int64_t)row * D + ks * 32 + lg * 8);
-      } else {
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) qf[ks][j] = (__bf16)0.f;
-      }
-    }
-  }
-
-  float m_run = -1e30f;   // running max for this lane's q column
-  float l_run = 0.f;      // running denominator
-  f32x4 oacc[D / 16];     // O D-layout: col d = lc (+16*dt), row q = 4*lg+r
+  float m = -1e30f, lsum = 0.f;
+  f32x16 acc[D / 32];
   #pragma unroll
-  for (int dt = 0; dt < D / 16; ++dt) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < D / 32; ++dt) acc[dt] = zero16();
 
-  // causal: this BLOCK needs kv tiles up to the block's last q row
-  const int blk_q_end = min(qblk * (QB * NWAVE) + QB * NWAVE, T);
-  const int n_tiles = (blk_q_end + KVB - 1) / KVB;
-
-  for (int t = 0; t < n_tiles; ++t) {
-    const int kv0 = t * KVB;
-    const int kv_valid = min(KVB, T - kv0);
-    __syncthreads();
-    stage_tile<KVB, D>(k_lds, kp + (int64_t)kv0 * D, D, kv_valid, tid, 256);
-    stage_tile<D, KVB>(v_lds, vp + kv0, Tp, D, tid, 256);  // padded cols
-    __syncthreads();
-
-    if (q0 < T && kv0 <= q_end - 1) {
-      // ST[kv][q] tiles: kv subtile s (rows s*16..), cols = q block
-      f32x4 st[KVB / 16];
-      #pragma unroll
-      for (int s = 0; s < KVB / 16; ++s) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        #pragma unroll
-        for (int ks = 0; ks < D / 32; ++ks) {
-          const bf16v8 kf = lds_frag<D>(k_lds, s * 16 + lc, ks * 4 + lg);
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], acc,
-                                                        0, 0, 0);
-        }
-        st[s] = acc;
-      }
-      // scale + causal mask + running softmax (per q column = lane lc)
-      float tile_max = -1e30f;
-      #pragma unroll
-      for (int s = 0; s < KVB / 16; ++s) {
-        #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int kv = kv0 + s * 16 + 4 * lg + r;
-          const int qq = q0 + lc;
-          float v = st[s][r] * scale;
-          if (kv > qq || qq >= T) v = -1e30f;
-          st[s][r] = v;
-          tile_max = fmaxf(tile_max, v);
-        }
-      }
-      tile_max = wave_xor_max(tile_max);
-      const float m_new = fmaxf(m_run, tile_max);
-      const float alpha = __expf(m_run - m_new);
-      float psum = 0.f;
-      #pragma unroll
-      for (int s = 0; s < KVB / 16; ++s) {
-        #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float p = __expf(st[s][r] - m_new);
-          st[s][r] = p;
-          psum += p;
-        }
-      }
-      psum = wave_xor_sum(psum);
-      l_run = l_run * alpha + psum;
-      m_run = m_new;
-      // rescale O. The softmax stats live per LANE COLUMN (q = lc), but
-      // the accumulator's rows are q = 4*lg + r — fetch each row's alpha
-      // from the lane that owns that q column.
-      float alpha_row[4];
-      #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        alpha_row[r] = __shfl(alpha, 4 * lg + r, 64);
-      #pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) {
-        #pragma unroll
-        for (int r = 0; r < 4; ++r) oacc[dt][r] *= alpha_row[r];
-      }
-      // PV: A = PT^T fragments (relayout), B = v_t rows
-      const bf16v8 pa = relayout_frag(st[0], st[1]);
-      #pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) {
-        const bf16v8 vf = lds_frag<KVB>(v_lds, dt * 16 + lc, lg);
-        oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vf, oacc[dt],
-                                                           0, 0, 0);
-      }
-    }
-  }
-
-  // epilogue: normalize, stage O tile through LDS (D-layout columns ->
-  // row-major global), write lse. As with alpha, 1/l for accumulator row
-  // q = 4*lg+r lives in lane lc = 4*lg+r.
-  const float inv = (l_run > 0.f) ? 1.f / l_run : 0.f;
-  float inv_row[4];
-  #pragma unroll
-  for (int r = 0; r < 4; ++r) inv_row[r] = __shfl(inv, 4 * lg + r, 64);
-  float* ow = o_lds + (size_t)wave * QB * D;
-  #pragma unroll
-  for (int dt = 0; dt < D / 16; ++dt) {
-    #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int qq = 4 * lg + r;            // row within the wave's tile
-      ow[qq * D + dt * 16 + lc] = oacc[dt][r] * inv_row[r];
-    }
-  }
-  if (q0 < T && lg == 0) {
-    // lane lc owns q column q0+lc
-    if (q0 + lc < T)
-      lse[(((int64_t)b * Hq + h) * T) + q0 + lc] = m_run + __logf(l_run);
-  }
+  const int last = min((qb + 1) * (NW * WROWS), len);   // keys of this workgroup
+  const int n = (last + KV - 1) / KV;
+  Tile<D, KV, NT> tk, tv;
+  tk.fetch(kp, sk.t, len);
+  tv.fetch(vp, sv.t, len);
+  tk.store(smem);
+  tv.store(smem + TB);
   __syncthreads();
-  // coalesced store: each lane writes bf16x8 rows
-  for (int i = tid; i < NWAVE * QB * (D / 8); i += 256) {
-    const int w2 = i / (QB * D / 8);
-    const int rem = i % (QB * D / 8);
-    const int row = rem / (D / 8);
-    const int cu = rem % (D / 8);
-    const int qq = qblk * (QB * NWAVE) + w2 * QB + row;
-    if (qq < T) {
-      const float* src = o_lds + ((size_t)w2 * QB + row) * D + cu * 8;
-      bf16x8 vv;
+
+  for (int t = 0; t < n; ++t) {
+    const int kv0 = t * KV;
+    char* ks_ = smem + (t & 1) * (2 * TB);
+    char* vs_ = ks_ + TB;
+    if (t + 1 < n) {
+      tk.fetch(kp + (int64_t)(kv0 + KV) * sk.t, sk.t, len - kv0 - KV);
+      tv.fetch(vp + (int64_t)(kv0 + KV) * sv.t, sv.t, len - kv0 - KV);
+    }
+    if (kv0 <= q0 + WROWS - 1 && q0 < len) {            // wave-uniform
+      f32x16 st[NS];
       #pragma unroll
-      for (int j = 0; j < 8; ++j) vv.v[j] = f2bf(src[j]);
-      *reinterpret_cast<bf16x8*>(o + (((int64_t)b * Hq + h) * T + qq) * D
-                                 + cu * 8) = vv;
+      for (int s = 0; s < NS; ++s) {
+        st[s] = zero16();
+        #pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks) st[s] = mfma(fr.row(ks_, s, ks), qf[ks], st[s]);
+      }
+      if (kv0 + KV - 1 > q0) {                          // the diagonal
+        #pragma unroll
+        for (int s = 0; s < NS; ++s)
+          #pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (kv0 + s * 32 + acc_row(r, half) > qq) st[s][r] = -1e30f;
+      }
+      float mx = st[0][0];
+      #pragma unroll
+      for (int s = 0; s < NS; ++s)
+        #pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[s][r]);
+      // The subtracted maximum may lag by 2^8: weights stay far from fp32's
+      // range, and the accumulators are rescaled once or twice instead of at
+      // nearly every tile (one of 32 rows has a new maximum most of the time).
+      const float m_new = fmaxf(m, halves_max(mx) * scale_log2);
+      if (__any(m_new > m + 8.f)) {
+        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+        lsum *= alpha;
+        #pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+          #pragma unroll
+          for (int r = 0; r < 16; ++r) acc[dt][r] *= alpha;
+        m = m_new;
+      }
+      #pragma unroll
+      for (int s = 0; s < NS; ++s)
+        #pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          st[s][r] = __builtin_amdgcn_exp2f(st[s][r] * scale_log2 - m);
+          lsum += st[s][r];
+        }
+      #pragma unroll
+      for (int s = 0; s < NS; ++s)
+        #pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2) {
+          const bf16v8 p = pack8(st[s], k2);
+          #pragma unroll
+          for (int dt = 0; dt < D / 32; ++dt)
+            acc[dt] = mfma(fr.col(vs_, s * 32 + k2 * 16, dt), p, acc[dt]);
+        }
+    }
+    if (t + 1 < n) {
+      char* nk = smem + ((t + 1) & 1) * (2 * TB);
+      tk.store(nk);
+      tv.store(nk + TB);
+      __syncthreads();
     }
   }
+
+  lsum = halves_sum(lsum);
+  store_rows<D>(acc, 1.f / lsum, o + b * so.b + h * so.h + (int64_t)(row0 + qq) * so.t, qq < len);
+  if (lse != nullptr && half == 0 && qq < len)
+    lse[((int64_t)b * Hq + h) * T + qq] = m * LN2 + __logf(lsum);
 }
 
 // ------------------------------------------------------------- backward
-// Pass Q (dQ): q-block outer, kv loop; swapped orientation (like fwd).
-//   dPT[kv][q] = mfma(A=V rows, B=dO rows)
-//   PT[kv][q]  = exp(ST*scale - lse[q])   (ST recomputed)
-//   dST        = PT * (dPT - delta[q]) * scale
-//   dQ[q][d]  += mfma(A = relayout(dST), B = k_t rows)
-template <int D>
-__global__ __launch_bounds__(256)
-void flash_bwd_dq_kernel(const __hip_bfloat16* __restrict__ q,
-                         const __hip_bfloat16* __restrict__ k,
-                         const __hip_bfloat16* __restrict__ kt,
-                         const __hip_bfloat16* __restrict__ v,
-                         const __hip_bfloat16* __restrict__ dout,
-                         const float* __restrict__ lse,
-                         const float* __restrict__ delta,
-                         __hip_bfloat16* __restrict__ dq,
-                         int B, int Hq, int Hkv, int T, int Tp, float scale) {
-  const int qblk = blockIdx.x;
-  const int h = blockIdx.y;
-  const int b = blockIdx.z;
-  const int kvh = h / (Hq / Hkv);
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int l = tid & 63;
-  const int lg = l >> 4;
-  const int lc = l & 15;
-  const int q0 = qblk * (QB * NWAVE) + wave * QB;
-  const int q_end = min(q0 + QB, T);
+// dQ: P = exp(S*scale - lse), dS = P * (dP - delta), dQ = scale * dS K.
+template <int D, int NW>
+__global__ __launch_bounds__(NW * 64, 2)
+void flash_bwd_dq_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16* __restrict__ k,
+                         const __hip_bfloat16* __restrict__ v, const __hip_bfloat16* __restrict__ o,
+                         const __hip_bfloat16* __restrict__ dout, const float* __restrict__ lse,
+                         float* __restrict__ delta, __hip_bfloat16* __restrict__ dq, Strides sq,
+                         Strides sk, Strides sv, Strides so, Strides sdo, Strides sdq, int Hq,
+                         int Hkv, int T, int nq, float scale) {
+  constexpr int KV = tile_rows<NW>(), NS = KV / 32, NT = NW * 64;
+  const int group = Hq / Hkv;
+  int id = xcd_share(blockIdx.x, gridDim.x);
+  const int hg = id % group;
+  id /= group;
+  const int qb = nq - 1 - id % nq;
+  id /= nq;
+  const int kvh = id % Hkv, b = id / Hkv;
+  const int h = kvh * group + hg;
+
+  const int wave = wave_id(), l = threadIdx.x & 63, half = l >> 5;
+  const int q0 = qb * (NW * WROWS) + wave * WROWS;
+  const int qq = q0 + (l & 31);
+  const bool live = qq < T;
+  const __hip_bfloat16* kp = k + b * sk.b + kvh * sk.h;
+  const __hip_bfloat16* vp = v + b * sv.b + kvh * sv.h;
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  char* k_lds = smem;                          // KVB x D
-  char* kt_lds = k_lds + KVB * D * 2;          // D x KVB (K^T rows)
-  char* v_lds = kt_lds + (size_t)D * KVB * 2;  // KVB x D (V rows)
-  float* s_lds = reinterpret_cast<float*>(v_lds + (size_t)KVB * D * 2);
-
-  const int64_t bh = (int64_t)b * Hq + h;
-  const int64_t bkv = (int64_t)b * Hkv + kvh;
-  const __hip_bfloat16* qp = q + bh * T * D;
-  const __hip_bfloat16* kp = k + bkv * T * D;
-  const __hip_bfloat16* ktp = kt + bkv * D * Tp;
-  const __hip_bfloat16* vp = v + bkv * T * D;
-  const __hip_bfloat16* dop = dout + bh * T * D;
-
-  // Q and dO fragments (B-frags over d)
-  bf16v8 qf[D / 32], dof[D / 32];
+  constexpr int TB = KV * D * 2;
+  const Frags<D> fr;
+  bf16v8 qf[D / 16], dof[D / 16];
+  const int qrow = min(qq, T - 1);
+  load_row<D>(qf, q + b * sq.b + h * sq.h, sq.t, qrow);
+  load_row<D>(dof, dout + b * sdo.b + h * sdo.h, sdo.t, qrow);
+  float dl = 0.f;
   {
-    const int row = q0 + lc;
+    bf16v8 of[D / 16];
+    load_row<D>(of, o + b * so.b + h * so.h, so.t, qrow);
     #pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) {
-      if (row < T) {
-        qf[ks] = *reinterpret_cast<const bf16v8*>(
-            qp + (int64_t)row * D + ks * 32 + lg * 8);
-        dof[ks] = *reinterpret_cast<const bf16v8*>(
-            dop + (int64_t)row * D + ks * 32 + lg * 8);
-      } else {
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) { qf[ks][j] = (__bf16)0.f;
-                                      dof[ks][j] = (__bf16)0.f; }
-      }
-    }
+    for (int ks = 0; ks < D / 16; ++ks)
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) dl += (float)of[ks][j] * (float)dof[ks][j];
+    dl = halves_sum(dl);
   }
-  const float lse_q = (q0 + lc < T) ? lse[bh * T + q0 + lc] : 0.f;
-  const float delta_q = (q0 + lc < T) ? delta[bh * T + q0 + lc] : 0.f;
+  const int64_t at = ((int64_t)b * Hq + h) * T + qq;
+  const float scale_log2 = scale * LOG2E;
+  const float lse2 = live ? lse[at] * LOG2E : 1e30f;    // 1e30: weight zero
+  if (live && half == 0) delta[at] = dl;
 
-  f32x4 dqacc[D / 16];
+  f32x16 acc[D / 32];
   #pragma unroll
-  for (int dt = 0; dt < D / 16; ++dt) dqacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < D / 32; ++dt) acc[dt] = zero16();
 
-  const int blk_q_end = min(qblk * (QB * NWAVE) + QB * NWAVE, T);
-  const int n_tiles = (blk_q_end + KVB - 1) / KVB;
-
-  for (int t = 0; t < n_tiles; ++t) {
-    const int kv0 = t * KVB;
-    const int kv_valid = min(KVB, T - kv0);
-    __syncthreads();
-    stage_tile<KVB, D>(k_lds, kp + (int64_t)kv0 * D, D, kv_valid, tid, 256);
-    stage_tile<D, KVB>(kt_lds, ktp + kv0, Tp, D, tid, 256);
-    stage_tile<KVB, D>(v_lds, vp + (int64_t)kv0 * D, D, kv_valid, tid, 256);
-    __syncthreads();
-
-    if (q0 < T && kv0 <= q_end - 1) {
-      f32x4 st[KVB / 16], dpt[KVB / 16];
-      #pragma unroll
-      for (int s = 0; s < KVB / 16; ++s) {
-        f32x4 a1 = {0.f, 0.f, 0.f, 0.f}, a2 = {0.f, 0.f, 0.f, 0.f};
-        #pragma unroll
-        for (int ks = 0; ks < D / 32; ++ks) {
-          const bf16v8 kf = lds_frag<D>(k_lds, s * 16 + lc, ks * 4 + lg);
-          const bf16v8 vf = lds_frag<D>(v_lds, s * 16 + lc, ks * 4 + lg);
-          a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], a1, 0, 0, 0);
-          a2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, dof[ks], a2, 0, 0, 0);
-        }
-        st[s] = a1;
-        dpt[s] = a2;
-      }
-      // dST = PT * (dPT - delta) * scale with causal mask
-      #pragma unroll
-      for (int s = 0; s < KVB / 16; ++s) {
-        #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int kv = kv0 + s * 16 + 4 * lg + r;
-          const int qq = q0 + lc;
-          float p = 0.f;
-          if (kv <= qq && qq < T && kv < T)
-            p = __expf(st[s][r] * scale - lse_q);
-          st[s][r] = p * (dpt[s][r] - delta_q) * scale;
-        }
-      }
-      const bf16v8 da = relayout_frag(st[0], st[1]);
-      #pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) {
-        const bf16v8 ktf = lds_frag<KVB>(kt_lds, dt * 16 + lc, lg);
-        dqacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(da, ktf,
-                                                            dqacc[dt], 0, 0, 0);
-      }
-    }
-  }
-
-  // epilogue via LDS (same as fwd)
-  float* ow = s_lds + (size_t)wave * QB * D;
-  #pragma unroll
-  for (int dt = 0; dt < D / 16; ++dt) {
-    #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      ow[(4 * lg + r) * D + dt * 16 + lc] = dqacc[dt][r];
-  }
+  const int last = min((qb + 1) * (NW * WROWS), T);
+  const int n = (last + KV - 1) / KV;
+  Tile<D, KV, NT> tk, tv;
+  tk.fetch(kp, sk.t, T);
+  tv.fetch(vp, sv.t, T);
+  tk.store(smem);
+  tv.store(smem + TB);
   __syncthreads();
-  for (int i = tid; i < NWAVE * QB * (D / 8); i += 256) {
-    const int w2 = i / (QB * D / 8);
-    const int rem = i % (QB * D / 8);
-    const int row = rem / (D / 8);
-    const int cu = rem % (D / 8);
-    const int qq = qblk * (QB * NWAVE) + w2 * QB + row;
-    if (qq < T) {
-      const float* src = s_lds + ((size_t)w2 * QB + row) * D + cu * 8;
-      bf16x8 vv;
-      #pragma unroll
-      for (int j = 0; j < 8; ++j) vv.v[j] = f2bf(src[j]);
-      *reinterpret_cast<bf16x8*>(dq + (bh * T + qq) * D + cu * 8) = vv;
+
+  for (int t = 0; t < n; ++t) {
+    const int kv0 = t * KV;
+    char* ks_ = smem + (t & 1) * (2 * TB);
+    char* vs_ = ks_ + TB;
+    if (t + 1 < n) {
+      tk.fetch(kp + (int64_t)(kv0 + KV) * sk.t, sk.t, T - kv0 - KV);
+      tv.fetch(vp + (int64_t)(kv0 + KV) * sv.t, sv.t, T - kv0 - KV);
     }
+    #pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int c0 = kv0 + s * 32;
+      if (c0 > q0 + WROWS - 1 || q0 >= T) continue;     // wave-uniform
+      f32x16 st = zero16(), dp = zero16();
+      #pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks) st = mfma(fr.row(ks_, s, ks), qf[ks], st);
+      #pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks) dp = mfma(fr.row(vs_, s, ks), dof[ks], dp);
+      #pragma unroll
+      for (int r = 0; r < 16; ++r)
+        st[r] = __builtin_amdgcn_exp2f(st[r] * scale_log2 - lse2) * (dp[r] - dl);
+      if (c0 + 31 > q0) {                               // the diagonal
+        #pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (c0 + acc_row(r, half) > qq) st[r] = 0.f;
+      }
+      #pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2) {
+        const bf16v8 ds = pack8(st, k2);
+        #pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+          acc[dt] = mfma(fr.col(ks_, s * 32 + k2 * 16, dt), ds, acc[dt]);
+      }
+    }
+    if (t + 1 < n) {
+      char* nk = smem + ((t + 1) & 1) * (2 * TB);
+      tk.store(nk);
+      tv.store(nk + TB);
+      __syncthreads();
+    }
+  }
+  store_rows<D>(acc, scale, dq + b * sdq.b + h * sdq.h + (int64_t)qq * sdq.t, live);
+}
+
+// dK, dV of one kv head's 32*NW keys, summed over query heads
+// hs*part .. of its group. Partials (split > 1) go to fp32 (split, B, Hkv, T, D).
+template <int D, int NW>
+__global__ __launch_bounds__(NW * 64, 2)
+void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16* __restrict__ k,
+                          const __hip_bfloat16* __restrict__ v,
+                          const __hip_bfloat16* __restrict__ dout, const float* __restrict__ lse,
+                          const float* __restrict__ delta, __hip_bfloat16* __restrict__ dk,
+                          __hip_bfloat16* __restrict__ dv, float* __restrict__ pk,
+                          float* __restrict__ pv, Strides sq, Strides sk, Strides sv, Strides sdo,
+                          Strides sdk, Strides sdv, int Hq, int Hkv, int T, int nkv, int split,
+                          float scale) {
+  constexpr int QT = 32, NT = NW * 64;
+  const int group = Hq / Hkv;
+  int id = xcd_share(blockIdx.x, gridDim.x);
+  const int hs = id % split;
+  id /= split;
+  const int kb = id % nkv;              // longest columns first
+  id /= nkv;
+  const int kvh = id % Hkv, b = id / Hkv;
+  const int h0 = hs * group / split, h1 = (hs + 1) * group / split;
+
+  const int wave = wave_id(), l = threadIdx.x & 63, half = l >> 5;
+  const int kv0 = kb * (NW * WROWS) + wave * WROWS;
+  const int kk = kv0 + (l & 31);
+  const bool live = kk < T;
+
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int TB = QT * D * 2, SB = 2 * TB + QT * 8;  // Q, dO, lse, delta
+  constexpr int KB = NW * WROWS * D * 2;
+  const Frags<D> fr;
+  // V rows stay in registers, K rows in LDS: both in registers would leave
+  // 256 too few for the accumulators, one wave a SIMD, and copies to the
+  // accumulation registers around every product
+  {
+    Tile<D, NW * WROWS, NT> tk;
+    const int r0 = kb * (NW * WROWS);
+    tk.fetch(k + b * sk.b + kvh * sk.h + (int64_t)r0 * sk.t, sk.t, T - r0);
+    tk.store(smem);
+  }
+  bf16v8 vf[D / 16];
+  load_row<D>(vf, v + b * sv.b + kvh * sv.h, sv.t, min(kk, T - 1));
+  const float scale_log2 = scale * LOG2E;
+
+  f32x16 ak[D / 32], av[D / 32];
+  #pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt) { ak[dt] = zero16(); av[dt] = zero16(); }
+
+  const int first = kb * (NW * WROWS), n = (T - first + QT - 1) / QT * (h1 - h0);
+  Tile<D, QT, NT> tq, td;
+  float stat = 0.f;     // threads 0..31: lse, 32..63: delta of the tile's rows
+  int fh = kvh * group + h0, fr0 = first;              // the next tile to fetch
+  auto fetch = [&] {
+    tq.fetch(q + b * sq.b + fh * sq.h + (int64_t)fr0 * sq.t, sq.t, T - fr0);
+    td.fetch(dout + b * sdo.b + fh * sdo.h + (int64_t)fr0 * sdo.t, sdo.t, T - fr0);
+    if (threadIdx.x < 64) {
+      const int r = fr0 + (threadIdx.x & 31);
+      const float* p = (threadIdx.x < 32 ? lse : delta) + ((int64_t)b * Hq + fh) * T;
+      stat = p[min(r, T - 1)];
+      // rows past the end get weight exp(-huge) = 0
+      if (threadIdx.x < 32) stat = r < T ? stat * LOG2E : 1e30f;
+    }
+    fr0 += QT;
+    if (fr0 >= T) { fr0 = first; ++fh; }
+  };
+  auto store = [&](int i) {
+    char* s = smem + KB + (i & 1) * SB;
+    tq.store(s);
+    td.store(s + TB);
+    if (threadIdx.x < 64) reinterpret_cast<float*>(s + 2 * TB)[threadIdx.x] = stat;
+  };
+  fetch();
+  store(0);
+  __syncthreads();
+
+  int r0 = first;
+  for (int i = 0; i < n; ++i) {
+    char* qs = smem + KB + (i & 1) * SB;
+    char* ds_ = qs + TB;
+    const float* st_lse = reinterpret_cast<const float*>(ds_ + TB);
+    if (i + 1 < n) fetch();
+    if (r0 + QT - 1 >= kv0 && kv0 < T) {                // wave-uniform
+      f32x16 s = zero16(), dp = zero16();
+      #pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks) s = mfma(fr.row(qs, 0, ks), fr.row(smem, wave, ks), s);
+      #pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks) dp = mfma(fr.row(ds_, 0, ks), vf[ks], dp);
+      #pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 le = *reinterpret_cast<const f32x4*>(st_lse + 8 * g + 4 * half);
+        const f32x4 de = *reinterpret_cast<const f32x4*>(st_lse + 32 + 8 * g + 4 * half);
+        #pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          s[4 * g + j] = __builtin_amdgcn_exp2f(s[4 * g + j] * scale_log2 - le[j]);
+          dp[4 * g + j] = s[4 * g + j] * (dp[4 * g + j] - de[j]);
+        }
+      }
+      if (r0 < kv0 + WROWS - 1) {                       // the diagonal
+        #pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (r0 + acc_row(r, half) < kk) s[r] = dp[r] = 0.f;
+      }
+      #pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2) {
+        const bf16v8 p = pack8(s, k2), ds = pack8(dp, k2);
+        #pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt) {
+          av[dt] = mfma(fr.col(ds_, k2 * 16, dt), p, av[dt]);
+          ak[dt] = mfma(fr.col(qs, k2 * 16, dt), ds, ak[dt]);
+        }
+      }
+    }
+    r0 += QT;
+    if (r0 >= T) r0 = first;
+    if (i + 1 < n) {
+      store(i + 1);
+      __syncthreads();
+    }
+  }
+
+  if (split == 1) {
+    store_rows<D>(ak, scale, dk + b * sdk.b + kvh * sdk.h + (int64_t)kk * sdk.t, live);
+    store_rows<D>(av, 1.f, dv + b * sdv.b + kvh * sdv.h + (int64_t)kk * sdv.t, live);
+  } else {
+    const int64_t at = ((((int64_t)hs * (gridDim.x / (split * nkv * Hkv)) + b) * Hkv + kvh) * T + kk) * D;
+    store_rows_f32<D>(ak, pk + at, live);
+    store_rows_f32<D>(av, pv + at, live);
   }
 }
 
-// Pass KV (dK^T, dV^T): kv-block outer, UNSWAPPED orientation.
-//   S[q][kv]  = mfma(A=Q rows, B=K rows);  P = exp(S*scale - lse[q])
-//   dP[q][kv] = mfma(A=dO rows, B=V rows)
-//   dS        = P * (dP - delta[q]) * scale
-//   dV^T[d][kv] += mfma(A = dO^T rows, B = relayout(P))
-//   dK^T[d][kv] += mfma(A = q^T rows,  B = relayout(dS))
-// One wave owns 16 kv columns; the block owns 64 kv rows (KVT tile).
+// dK = scale * sum of partials, dV = sum of partials; 8 elements a thread.
 template <int D>
 __global__ __launch_bounds__(256)
-void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q,
-                          const __hip_bfloat16* __restrict__ qt,
-                          const __hip_bfloat16* __restrict__ k,
-                          const __hip_bfloat16* __restrict__ v,
-                          const __hip_bfloat16* __restrict__ dout,
-                          const __hip_bfloat16* __restrict__ dot_t,
-                          const float* __restrict__ lse,
-                          const float* __restrict__ delta,
-                          __hip_bfloat16* __restrict__ dkt,  // (B,Hq,D,T)
-                          __hip_bfloat16* __restrict__ dvt,   // per Q-HEAD
-                          int B, int Hq, int Hkv, int T, int Tp, float scale) {
-  constexpr int KB = 16;     // kv cols per wave
-  const int kvblk = blockIdx.x;          // 64 kv rows per block
-  const int h = blockIdx.y;              // q head (accumulate into kv head)
-  const int b = blockIdx.z;
-  const int group = Hq / Hkv;
-  const int kvh = h / group;
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6;
-  const int l = tid & 63;
-  const int lg = l >> 4;
-  const int lc = l & 15;
-  const int kv0 = kvblk * (KB * NWAVE) + wave * KB;  // wave's 16 kv cols
-
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  char* q_lds = smem;                            // QTile x D (Q rows)
-  char* do_lds = q_lds + KVB * D * 2;            // QTile x D (dO rows)
-  char* qt_lds = do_lds + KVB * D * 2;           // D x QTile (Q^T rows)
-  char* dot_lds = qt_lds + (size_t)D * KVB * 2;  // D x QTile (dO^T rows)
-
-  const int64_t bh = (int64_t)b * Hq + h;
-  const int64_t bkv = (int64_t)b * Hkv + kvh;
-  const __hip_bfloat16* qp = q + bh * T * D;
-  const __hip_bfloat16* qtp = qt + bh * D * Tp;
-  const __hip_bfloat16* kp = k + bkv * T * D;
-  const __hip_bfloat16* vp = v + bkv * T * D;
-  const __hip_bfloat16* dop = dout + bh * T * D;
-  const __hip_bfloat16* dotp = dot_t + bh * D * Tp;
-
-  // K and V fragments for this wave's 16 kv columns (B-frags over d)
-  bf16v8 kf[D / 32], vf[D / 32];
-  {
-    const int row = kv0 + lc;
+void flash_bwd_sum_kernel(const float* __restrict__ pk, const float* __restrict__ pv,
+                          __hip_bfloat16* __restrict__ dk, __hip_bfloat16* __restrict__ dv,
+                          Strides sdk, Strides sdv, int Hkv, int T, int64_t rows, int split,
+                          float scale) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = i / (D / 8);
+  const int c = (int)(i % (D / 8)) * 8;
+  if (row >= rows) return;
+  const int t = (int)(row % T);
+  const int64_t bh = row / T;
+  const int kvh = (int)(bh % Hkv);
+  const int64_t b = bh / Hkv;
+  float a[8] = {0, 0, 0, 0, 0, 0, 0, 0}, w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int s = 0; s < split; ++s) {
+    const int64_t at = (s * rows + row) * D + c;
     #pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) {
-      if (row < T) {
-        kf[ks] = *reinterpret_cast<const bf16v8*>(
-            kp + (int64_t)row * D + ks * 32 + lg * 8);
-        vf[ks] = *reinterpret_cast<const bf16v8*>(
-            vp + (int64_t)row * D + ks * 32 + lg * 8);
-      } else {
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) { kf[ks][j] = (__bf16)0.f;
-                                      vf[ks][j] = (__bf16)0.f; }
-      }
-    }
+    for (int j = 0; j < 8; ++j) { a[j] += pk[at + j]; w[j] += pv[at + j]; }
   }
-
-  f32x4 dkacc[D / 16], dvacc[D / 16];
+  bf16x8 x, y;
   #pragma unroll
-  for (int dt = 0; dt < D / 16; ++dt) {
-    dkacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    dvacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int j = 0; j < 8; ++j) { x.v[j] = f2bf(a[j] * scale); y.v[j] = f2bf(w[j]); }
+  *reinterpret_cast<bf16x8*>(dk + b * sdk.b + kvh * sdk.h + t * sdk.t + c) = x;
+  *reinterpret_cast<bf16x8*>(dv + b * sdv.b + kvh * sdv.h + t * sdv.t + c) = y;
+}
 
-  // causal: q tiles from the block's FIRST kv row onward
-  const int blk_kv0 = kvblk * (KB * NWAVE);
-  const int t0 = blk_kv0 / KVB;
-  const int n_tiles = (T + KVB - 1) / KVB;
+// A (B, H, T, D) operand whose rows can be read 16 B at a time as it lies.
+torch::Tensor rows16(const torch::Tensor& x) {
+  bool ok = x.stride(3) == 1 && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+  for (int d = 0; d < 3; ++d) ok = ok && (x.size(d) == 1 || x.stride(d) % 8 == 0);
+  ok = ok && x.stride(2) < (1 << 24);     // 64 rows of a tile within 32-bit offsets
+  return ok ? x : x.clone(at::MemoryFormat::Contiguous);
+}
 
-  for (int t = t0; t < n_tiles; ++t) {
-    const int tq0 = t * KVB;                 // 32 q rows per tile
-    const int q_valid = min(KVB, T - tq0);
-    __syncthreads();
-    stage_tile<KVB, D>(q_lds, qp + (int64_t)tq0 * D, D, q_valid, tid, 256);
-    stage_tile<KVB, D>(do_lds, dop + (int64_t)tq0 * D, D, q_valid, tid, 256);
-    stage_tile<D, KVB>(qt_lds, qtp + tq0, Tp, D, tid, 256);
-    stage_tile<D, KVB>(dot_lds, dotp + tq0, Tp, D, tid, 256);
-    __syncthreads();
+Strides strides(const torch::Tensor& x) {
+  return {x.stride(0), x.stride(1), (int)x.stride(2)};
+}
 
-    if (kv0 < T && tq0 + q_valid - 1 >= kv0) {
-      f32x4 s_t[KVB / 16], dp_t[KVB / 16];
-      #pragma unroll
-      for (int s = 0; s < KVB / 16; ++s) {
-        f32x4 a1 = {0.f, 0.f, 0.f, 0.f}, a2 = {0.f, 0.f, 0.f, 0.f};
-        #pragma unroll
-        for (int ks = 0; ks < D / 32; ++ks) {
-          // S[q][kv]: A = Q rows (LDS), B = K frags (regs)
-          const bf16v8 qfr = lds_frag<D>(q_lds, s * 16 + lc, ks * 4 + lg);
-          const bf16v8 dofr = lds_frag<D>(do_lds, s * 16 + lc, ks * 4 + lg);
-          a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qfr, kf[ks], a1, 0, 0, 0);
-          a2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dofr, vf[ks], a2, 0, 0, 0);
-        }
-        s_t[s] = a1;   // D-layout: col = kv = lc + kv0, row = q = tq0+s*16+4lg+r
-        dp_t[s] = a2;
-      }
-      f32x4 p_t[KVB / 16];
-      #pragma unroll
-      for (int s = 0; s < KVB / 16; ++s) {
-        #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int qq = tq0 + s * 16 + 4 * lg + r;
-          const int kv = kv0 + lc;
-          float p = 0.f;
-          if (kv <= qq && qq < T && kv < T)
-            p = __expf(s_t[s][r] * scale
-                       - lse[bh * T + min(qq, T - 1)]);
-          const float dlt = (qq < T) ? delta[bh * T + qq] : 0.f;
-          p_t[s][r] = p;
-          s_t[s][r] = p * (dp_t[s][r] - dlt) * scale;
-        }
-      }
-      const bf16v8 pb = relayout_frag(p_t[0], p_t[1]);    // B[kv][q-k]
-      const bf16v8 dsb = relayout_frag(s_t[0], s_t[1]);
-      #pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) {
-        const bf16v8 dotf = lds_frag<KVB>(dot_lds, dt * 16 + lc, lg);
-        const bf16v8 qtf = lds_frag<KVB>(qt_lds, dt * 16 + lc, lg);
-        dvacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(dotf, pb,
-                                                            dvacc[dt], 0, 0, 0);
-        dkacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qtf, dsb,
-                                                            dkacc[dt], 0, 0, 0);
-      }
-    }
-  }
+// A flat batch is one (1, H, tokens, D) operand for all sequences.
+Strides strides(const torch::Tensor& x, bool flat) {
+  return {flat ? 0 : x.stride(0), x.stride(1), (int)x.stride(2)};
+}
 
-  // per-Q-HEAD bf16 outputs (B,Hq,D,T): each (kvblk, h) block owns its
-  // region exclusively — no atomics; the host sums the GQA group in fp32
-  // (288 GB makes the extra head-resolved image free)
-  if (kv0 < T) {
-    #pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) {
-      #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int d = dt * 16 + 4 * lg + r;   // D-layout row = d
-        const int kv = kv0 + lc;              // col = kv
-        if (kv < T) {
-          const int64_t off = (bh * D + d) * T + kv;
-          dkt[off] = f2bf(dkacc[dt][r]);
-          dvt[off] = f2bf(dvacc[dt][r]);
-        }
-      }
-    }
-  }
-  (void)group;
+// The forward's running maximum and mask are those of unscaled scores: they
+// need scale > 0.
+torch::Tensor positive_scale(const torch::Tensor& q, double& scale) {
+  if (scale > 0) return q;
+  const bool zero = scale == 0;
+  scale = zero ? 1 : -scale;
+  return zero ? torch::zeros_like(q) : -q;
+}
+
+// An output laid out like the operand it belongs to, if that is dense.
+torch::Tensor like(const torch::Tensor& x) {
+  return x.is_non_overlapping_and_dense() ? torch::empty_like(x)
+                                          : torch::empty(x.sizes(), x.options());
+}
+
+const __hip_bfloat16* bf(const torch::Tensor& x) {
+  return reinterpret_cast<const __hip_bfloat16*>(x.data_ptr());
+}
+__hip_bfloat16* bfm(torch::Tensor& x) { return reinterpret_cast<__hip_bfloat16*>(x.data_ptr()); }
+
+void check_qkv(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& v) {
+  TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kBFloat16);
+  TORCH_CHECK(k.is_cuda() && v.is_cuda() && k.scalar_type() == at::kBFloat16 &&
+              v.scalar_type() == at::kBFloat16);
+  TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4);
+  TORCH_CHECK(k.size(0) == q.size(0) && k.size(2) == q.size(2) && k.size(3) == q.size(3) &&
+              v.sizes() == k.sizes(), "flash attention: k/v shape mismatch");
+  TORCH_CHECK(k.size(1) > 0 && q.size(1) % k.size(1) == 0);
+  TORCH_CHECK(q.size(3) == 64 || q.size(3) == 128, "flash attention: head_dim 64/128 only");
+}
+
+// 128-row workgroups (four waves share a tile) once they fill the chip
+// twice over; below that 64-row ones, which spread short batches wider.
+int waves_for(int64_t rows_of_heads, int T) { return rows_of_heads * ((T + 127) / 128) >= 512 ? 4 : 2; }
+
+#define FLASH_DISPATCH(D_, NW_, ...)                                             \
+  [&] {                                                                         \
+    if ((D_) == 128 && (NW_) == 4) { constexpr int D = 128, NW = 4; __VA_ARGS__; } \
+    else if ((D_) == 128) { constexpr int D = 128, NW = 2; __VA_ARGS__; }        \
+    else if ((NW_) == 4) { constexpr int D = 64, NW = 4; __VA_ARGS__; }          \
+    else { constexpr int D = 64, NW = 2; __VA_ARGS__; }                          \
+  }()
+
+void launch_fwd(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& v,
+                torch::Tensor& o, float* lse, const int* cu, int B, int T, double scale) {
+  const int Hq = q.size(1), Hkv = k.size(1);
+  const int nw = waves_for((int64_t)B * Hq, T);
+  const int nq = (T + nw * WROWS - 1) / (nw * WROWS);
+  const int64_t blocks = (int64_t)B * Hq * nq;
+  if (blocks == 0) return;
+  TORCH_CHECK(blocks < (1ll << 31), "flash attention: batch too large");
+  auto stream = at::cuda::getCurrentCUDAStream();
+  FLASH_DISPATCH(q.size(3), nw, {
+    const size_t smem = 4 * tile_rows<NW>() * D * 2;
+    hipLaunchKernelGGL((flash_fwd_kernel<D, NW>), dim3(blocks), dim3(NW * 64), smem, stream, bf(q),
+                       bf(k), bf(v), bfm(o), lse, cu, strides(q, cu), strides(k, cu),
+                       strides(v, cu), strides(o, cu), Hq, Hkv, T, nq, (float)scale * LOG2E);
+  });
+  HIP_CHECK_LAST();
 }
 
 }  // namespace
 
-std::vector<torch::Tensor> flash_attn_fwd(torch::Tensor q, torch::Tensor k,
-                                          torch::Tensor v, double scale) {
-  // q: (B, Hq, T, D); k, v: (B, Hkv, T, D) — causal, bf16
-  TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kBFloat16);
-  TORCH_CHECK(k.scalar_type() == at::kBFloat16 &&
-              v.scalar_type() == at::kBFloat16);
-  TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4);
-  const int B = q.size(0), Hq = q.size(1), T = q.size(2), D = q.size(3);
-  const int Hkv = k.size(1);
-  TORCH_CHECK(k.size(0) == B && k.size(2) == T && k.size(3) == D &&
-              v.sizes() == k.sizes(), "flash_attn_fwd: k/v shape mismatch");
-  TORCH_CHECK(Hq % Hkv == 0);
-  TORCH_CHECK(D == 64 || D == 128, "flash_attn_fwd: head_dim 64/128 only");
-  auto qc = q.contiguous(), kc = k.contiguous();
-  // transpose with columns padded to a multiple of 32 (KVB): keeps every
-  // bf16x8 staging read 16B-aligned and in-bounds for arbitrary T
-  const int Tp = (T + 31) / 32 * 32;
-  auto vt = torch::constant_pad_nd(v.transpose(2, 3), {0, Tp - T}, 0)
-                .contiguous();                 // (B, Hkv, D, Tp)
-  auto o = torch::empty_like(qc);
-  auto lse = torch::empty({B, Hq, T}, q.options().dtype(at::kFloat));
-  dim3 grid((T + QB * NWAVE - 1) / (QB * NWAVE), Hq, B), block(256);
-  const size_t smem = (size_t)KVB * D * 2 * 2 + (size_t)NWAVE * QB * D * 4;
-  auto stream = at::cuda::getCurrentCUDAStream();
-  #define LAUNCH_FWD(DV) \
-    hipLaunchKernelGGL((flash_fwd_kernel<DV>), grid, block, smem, stream, \
-        reinterpret_cast<const __hip_bfloat16*>(qc.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(kc.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(vt.data_ptr()), \
-        reinterpret_cast<__hip_bfloat16*>(o.data_ptr()), \
-        lse.data_ptr<float>(), B, Hq, Hkv, T, Tp, (float)scale)
-  if (D == 128) LAUNCH_FWD(128); else LAUNCH_FWD(64);
-  #undef LAUNCH_FWD
-  HIP_CHECK_LAST();
+std::vector<torch::Tensor> flash_attn_fwd(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                                          double scale) {
+  check_qkv(q, k, v);
+  auto qc = rows16(positive_scale(q, scale)), kc = rows16(k), vc = rows16(v);
+  auto o = like(qc);
+  auto lse = torch::empty({q.size(0), q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
+  launch_fwd(qc, kc, vc, o, lse.data_ptr<float>(), nullptr, q.size(0), q.size(2), scale);
   return {o, lse};
 }
 
-std::vector<torch::Tensor> flash_attn_bwd(torch::Tensor dout, torch::Tensor q,
-                                          torch::Tensor k, torch::Tensor v,
-                                          torch::Tensor o, torch::Tensor lse,
+// Causal attention inside each of the sequences cu[i] .. cu[i+1] of a flat
+// batch: q (tokens, Hq, D), k/v (tokens, Hkv, D), cu int32 (n+1,) rising from
+// 0 to tokens, max_len the longest of them.
+torch::Tensor flash_attn_varlen(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                                torch::Tensor cu, int64_t max_len, double scale) {
+  TORCH_CHECK(q.dim() == 3 && k.dim() == 3 && v.dim() == 3);
+  TORCH_CHECK(cu.is_cuda() && cu.scalar_type() == at::kInt && cu.is_contiguous() && cu.dim() == 1 &&
+              cu.numel() >= 1);
+  auto as4 = [](const torch::Tensor& x) { return x.transpose(0, 1).unsqueeze(0); };
+  auto q4 = as4(q), k4 = as4(k), v4 = as4(v);
+  check_qkv(q4, k4, v4);
+  TORCH_CHECK(max_len >= 0 && max_len <= q.size(0));
+  auto qc = rows16(positive_scale(q4, scale)), kc = rows16(k4), vc = rows16(v4);
+  auto out = torch::empty(q.sizes(), q.options());
+  auto o4 = as4(out);
+  launch_fwd(qc, kc, vc, o4, nullptr, cu.data_ptr<int>(), cu.numel() - 1, max_len, scale);
+  return out;
+}
+
+std::vector<torch::Tensor> flash_attn_bwd(torch::Tensor dout, torch::Tensor q, torch::Tensor k,
+                                          torch::Tensor v, torch::Tensor o, torch::Tensor lse,
                                           double scale) {
-  TORCH_CHECK(q.is_cuda() && q.scalar_type() == at::kBFloat16);
-  TORCH_CHECK(dout.scalar_type() == at::kBFloat16 &&
-              k.scalar_type() == at::kBFloat16 &&
-              v.scalar_type() == at::kBFloat16 &&
-              o.scalar_type() == at::kBFloat16 &&
+  check_qkv(q, k, v);
+  TORCH_CHECK(dout.scalar_type() == at::kBFloat16 && o.scalar_type() == at::kBFloat16 &&
               lse.scalar_type() == at::kFloat);
   TORCH_CHECK(dout.sizes() == q.sizes() && o.sizes() == q.sizes(),
               "flash_attn_bwd: dout/o shape mismatch");
-  const int B = q.size(0), Hq = q.size(1), T = q.size(2), D = q.size(3);
-  const int Hkv = k.size(1);
-  TORCH_CHECK(k.size(0) == B && k.size(2) == T && k.size(3) == D &&
-              v.sizes() == k.sizes(), "flash_attn_bwd: k/v shape mismatch");
-  auto qc = q.contiguous(), kc = k.contiguous(), vc = v.contiguous();
-  auto doc = dout.contiguous();
-  const int Tp = (T + 31) / 32 * 32;
-  auto kt = torch::constant_pad_nd(kc.transpose(2, 3), {0, Tp - T}, 0)
-                .contiguous();
-  auto qt = torch::constant_pad_nd(qc.transpose(2, 3), {0, Tp - T}, 0)
-                .contiguous();
-  auto dot_t = torch::constant_pad_nd(doc.transpose(2, 3), {0, Tp - T}, 0)
-                .contiguous();
-  auto delta = (doc.to(at::kFloat) * o.to(at::kFloat)).sum(-1);  // (B,Hq,T)
-  auto dq = torch::empty_like(qc);
-  auto dkt = torch::zeros({B, Hq, D, T}, q.options());
-  auto dvt = torch::zeros({B, Hq, D, T}, q.options());
-  auto stream = at::cuda::getCurrentCUDAStream();
-  dim3 block(256);
-  dim3 grid_q((T + QB * NWAVE - 1) / (QB * NWAVE), Hq, B);
-  const size_t smem_q = (size_t)KVB * D * 2 * 3 + (size_t)NWAVE * QB * D * 4;
-  #define LAUNCH_DQ(DV) \
-    hipLaunchKernelGGL((flash_bwd_dq_kernel<DV>), grid_q, block, smem_q, \
-        stream, \
-        reinterpret_cast<const __hip_bfloat16*>(qc.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(kc.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(kt.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(vc.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(doc.data_ptr()), \
-        lse.data_ptr<float>(), delta.data_ptr<float>(), \
-        reinterpret_cast<__hip_bfloat16*>(dq.data_ptr()), \
-        B, Hq, Hkv, T, Tp, (float)scale)
-  if (D == 128) LAUNCH_DQ(128); else LAUNCH_DQ(64);
-  #undef LAUNCH_DQ
-  dim3 grid_kv((T + 16 * NWAVE - 1) / (16 * NWAVE), Hq, B);
-  const size_t smem_kv = (size_t)KVB * D * 2 * 4;
-  #define LAUNCH_DKV(DV) \
-    hipLaunchKernelGGL((flash_bwd_dkv_kernel<DV>), grid_kv, block, smem_kv, \
-        stream, \
-        reinterpret_cast<const __hip_bfloat16*>(qc.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(qt.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(kc.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(vc.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(doc.data_ptr()), \
-        reinterpret_cast<const __hip_bfloat16*>(dot_t.data_ptr()), \
-        lse.data_ptr<float>(), delta.data_ptr<float>(), \
-        reinterpret_cast<__hip_bfloat16*>(dkt.data_ptr()), \
-        reinterpret_cast<__hip_bfloat16*>(dvt.data_ptr()), \
-        B, Hq, Hkv, T, Tp, (float)scale)
-  if (D == 128) LAUNCH_DKV(128); else LAUNCH_DKV(64);
-  #undef LAUNCH_DKV
-  HIP_CHECK_LAST();
+  const int B = q.size(0), Hq = q.size(1), T = q.size(2), Hkv = k.size(1);
+  TORCH_CHECK(lse.numel() == (int64_t)B * Hq * T, "flash_attn_bwd: lse shape mismatch");
+  auto qc = rows16(q), kc = rows16(k), vc = rows16(v), oc = rows16(o), doc = rows16(dout);
+  auto lsec = lse.contiguous();
+  auto delta = torch::empty_like(lsec);
+  auto dq = like(qc), dk = like(kc), dv = like(vc);
+  const int nw = waves_for((int64_t)B * Hq, T);
+  const int rows = nw * WROWS, nq = (T + rows - 1) / rows;
+  const int64_t blocks = (int64_t)B * Hq * nq, kv_blocks = (int64_t)B * Hkv * nq;
+  if (blocks == 0) return {dq, dk, dv};
+  TORCH_CHECK(blocks < (1ll << 31), "flash attention: batch too large");
   const int group = Hq / Hkv;
-  auto dk = dkt.view({B, Hkv, group, D, T}).to(at::kFloat).sum(2)
-                .transpose(2, 3).contiguous().to(at::kBFloat16);
-  auto dv = dvt.view({B, Hkv, group, D, T}).to(at::kFloat).sum(2)
-                .transpose(2, 3).contiguous().to(at::kBFloat16);
+  const int split = (int)std::min<int64_t>(group, (1024 + kv_blocks - 1) / kv_blocks);
+  torch::Tensor part;
+  float *pk = nullptr, *pv = nullptr;
+  if (split > 1) {
+    part = torch::empty({2, split, B, Hkv, T, q.size(3)}, lsec.options());
+    pk = part.data_ptr<float>();
+    pv = pk + part.numel() / 2;
+  }
+  auto stream = at::cuda::getCurrentCUDAStream();
+  FLASH_DISPATCH(q.size(3), nw, {
+    hipLaunchKernelGGL((flash_bwd_dq_kernel<D, NW>), dim3(blocks), dim3(NW * 64), 4 * tile_rows<NW>() * D * 2,
+                       stream, bf(qc), bf(kc), bf(vc), bf(oc), bf(doc), lsec.data_ptr<float>(),
+                       delta.data_ptr<float>(), bfm(dq), strides(qc), strides(kc), strides(vc),
+                       strides(oc), strides(doc), strides(dq), Hq, Hkv, T, nq, (float)scale);
+    hipLaunchKernelGGL((flash_bwd_dkv_kernel<D, NW>), dim3(kv_blocks * split), dim3(NW * 64),
+                       NW * WROWS * D * 2 + 2 * (2 * 32 * D * 2 + 32 * 8), stream, bf(qc), bf(kc), bf(vc), bf(doc),
+                       lsec.data_ptr<float>(), delta.data_ptr<float>(), bfm(dk), bfm(dv), pk, pv,
+                       strides(qc), strides(kc), strides(vc), strides(doc), strides(dk),
+                       strides(dv), Hq, Hkv, T, nq, split, (float)scale);
+    if (split > 1) {
+      const int64_t n = (int64_t)B * Hkv * T;
+      hipLaunchKernelGGL((flash_bwd_sum_kernel<D>), dim3((n * (D / 8) + 255) / 256), dim3(256), 0,
+                         stream, pk, pv, bfm(dk), bfm(dv), strides(dk), strides(dv), Hkv, T, n,
+                         split, (float)scale);
+    }
+  });
+  HIP_CHECK_LAST();
   return {dq, dk, dv};
 }

@@ -52,6 +52,9 @@ void lora_u(torch::Tensor x, torch::Tensor afrag, torch::Tensor u,
 torch::Tensor mfma_probe(torch::Tensor a, torch::Tensor b);
 std::vector<torch::Tensor> flash_attn_fwd(torch::Tensor q, torch::Tensor k,
                                           torch::Tensor v, double scale);
+torch::Tensor flash_attn_varlen(torch::Tensor q, torch::Tensor k,
+                                torch::Tensor v, torch::Tensor cu,
+                                int64_t max_len, double scale);
 std::vector<torch::Tensor> flash_attn_bwd(torch::Tensor dout, torch::Tensor q,
                                           torch::Tensor k, torch::Tensor v,
                                           torch::Tensor o, torch::Tensor lse,
@@ -94,6 +97,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma_probe", &mfma_probe, "16x16x32 bf16 MFMA mapping probe");
   m.def("flash_attn_fwd", &flash_attn_fwd,
         "causal GQA flash attention forward (returns o, lse)");
+  m.def("flash_attn_varlen", &flash_attn_varlen,
+        "causal GQA flash attention over a flat batch of sequences");
   m.def("flash_attn_bwd", &flash_attn_bwd,
         "causal GQA flash attention backward (returns dq, dk, dv)");
 }

@@ -1,0 +1,104 @@
+"""Kernels at the edges of their tiles, splits and layouts, against plain
+fp32 or fp64 torch."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ext():
+    from distrl_llm_amd.ops.build import build
+    return build()
+
+
+def _rand(shape, seed, std=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(shape, generator=g) * std).to("cuda", torch.bfloat16)
+
+
+def _rel(x, ref):
+    return float((x.double() - ref.double()).norm() / ref.double().norm().clamp_min(1e-30))
+
+
+# ------------------------------------------------------------------ flash
+# Bound: weights, dS and the outputs are each rounded to bf16 (2^-9 of the
+# value at most), everything else is fp32: three roundings, 3 * 2^-9 < 0.6 %.
+FLASH_REL = 3 * 2.0 ** -9
+
+
+def _flash_reference(q, k, v, dout, scale):
+    q, k, v = (t.detach().float().requires_grad_() for t in (q, k, v))
+    group, T = q.shape[1] // k.shape[1], q.shape[2]
+    s = q @ k.repeat_interleave(group, 1).transpose(2, 3).contiguous() * scale
+    s = s.masked_fill(torch.ones(T, T, dtype=torch.bool, device=q.device).triu(1), float("-inf"))
+    o = s.softmax(-1) @ v.repeat_interleave(group, 1)
+    return (o.detach(), *torch.autograd.grad(o, (q, k, v), dout.float()))
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,T,D", [
+    (1, 1, 1, 1, 64), (1, 2, 1, 31, 128), (2, 7, 1, 32, 64), (1, 4, 2, 33, 128),
+    (1, 3, 3, 64, 64), (2, 10, 2, 65, 128), (1, 28, 4, 127, 128), (1, 14, 2, 129, 64),
+    (3, 6, 2, 257, 128), (12, 28, 4, 193, 128), (20, 14, 2, 300, 64)])
+@pytest.mark.parametrize("layout", ["heads_first", "tokens_first", "sliced"])
+def test_flash_edges(B, Hq, Hkv, T, D, layout):
+    """Row blocks of 64 and 128 rows, key tiles of 32 and 64, ragged ends, a
+    head split with partial sums (few key blocks) and without; contiguous
+    operands, transposed projections, and rows cut out of a wider one at an
+    offset that is not a multiple of 16 bytes."""
+    from distrl_llm_amd.ops import functional as OF
+
+    def make(H, seed):
+        if layout == "heads_first":
+            return _rand((B, H, T, D), seed)
+        if layout == "tokens_first":
+            return _rand((B, T, H, D), seed).transpose(1, 2)
+        return _rand((B, T, H * D + 6), seed)[..., 3:3 + H * D].unflatten(2, (H, D)).transpose(1, 2)
+
+    q, k, v, dout = (make(H, i) for i, H in enumerate((Hq, Hkv, Hkv, Hq)))
+    scale = 1.3 * D ** -0.5
+    ref = _flash_reference(q, k, v, dout, scale)
+    leaves = [t.detach().requires_grad_() for t in (q, k, v)]
+    o = OF.flash_attention(*leaves, scale)
+    got = (o.detach(), *torch.autograd.grad(o, leaves, dout))
+    for name, x, r in zip(("o", "dq", "dk", "dv"), got, ref):
+        if name in ("dq", "dk") and T == 1:
+            # one key: the gradient is zero up to delta's fp32 rounding
+            assert float(x.float().abs().max()) < 1e-5
+            continue
+        assert _rel(x, r) < FLASH_REL, name
+
+
+def test_flash_scale_signs_and_far_scores():
+    """Scores hundreds below the maximum (forward: a saturated softmax's
+    gradients cancel, which the bound does not cover), negative and zero scale."""
+    from distrl_llm_amd.ops import functional as OF
+    q, k, v, dout = (_rand((1, 2, 150, 64), i, 2.0 if i < 2 else 1.0) for i in range(4))
+    for scale in (8.0, -8.0):
+        ref = _flash_reference(q, k, v, dout, scale)[0]
+        assert _rel(OF.flash_attention(q, k, v, scale), ref) < FLASH_REL
+    for scale in (-0.125, 0.0, 0.125):
+        ref = _flash_reference(q, k, v, dout, scale)
+        leaves = [t.detach().requires_grad_() for t in (q, k, v)]
+        o = OF.flash_attention(*leaves, scale)
+        got = (o.detach(), *torch.autograd.grad(o, leaves, dout))
+        for x, r in zip(got, ref):
+            if float(r.abs().max()) == 0.0:
+                assert float(x.float().abs().max()) == 0.0
+            else:
+                assert _rel(x, r) < FLASH_REL
+
+
+@pytest.mark.parametrize("lens", [[1], [5, 64, 65, 1, 200], [130, 3]])
+@pytest.mark.parametrize("H,KV,D", [(4, 2, 64), (7, 1, 128)])
+def test_flash_varlen(ext, lens, H, KV, D):
+    q, k, v = (_rand((sum(lens), h, D), i) for i, h in enumerate((H, KV, KV)))
+    cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0).to(torch.int32).cuda()
+    out = ext.flash_attn_varlen(q, k, v, cu, max(lens), D ** -0.5)
+    at = 0
+    for n in lens:
+        part = [t[at:at + n].transpose(0, 1).unsqueeze(0).contiguous() for t in (q, k, v)]
+        ref = _flash_reference(*part, torch.zeros_like(part[0]), D ** -0.5)[0][0].transpose(0, 1)
+        assert _rel(out[at:at + n], ref) < FLASH_REL
+        at += n
