@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Single-kernel vs two-stage sampler at decode shapes."""
+"""The sampler at decode shapes."""
 import sys, time, torch
 sys.path.insert(0, ".")
 from distrl_llm_amd.ops.build import build
@@ -10,7 +10,7 @@ for B in (160, 64, 512):
     logits = torch.randn(B, V, device=dev, dtype=torch.bfloat16)
     seeds = torch.randint(0, 2**31 - 1, (B,), device=dev, dtype=torch.int64)
     step = torch.zeros(1, dtype=torch.int64, device=dev)
-    for name in ("sample_tokens", "sample_tokens2"):
+    for name in ("sample_tokens",):
         fn = getattr(ext, name)
         run = lambda: fn(logits, 1.2, 0.95, 0, seeds, step)
         for _ in range(10): run()

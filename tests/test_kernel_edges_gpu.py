@@ -102,3 +102,95 @@ def test_flash_varlen(ext, lens, H, KV, D):
         ref = _flash_reference(*part, torch.zeros_like(part[0]), D ** -0.5)[0][0].transpose(0, 1)
         assert _rel(out[at:at + n], ref) < FLASH_REL
         at += n
+
+
+# ---------------------------------------------------------------- sampler
+
+def _splitmix64(x):
+    import numpy as np
+    with np.errstate(over="ignore"):
+        x = x + np.uint64(0x9E3779B97F4A7C15)
+        x = (x ^ (x >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+        x = (x ^ (x >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+    return x ^ (x >> np.uint64(31))
+
+
+def _sampled(logits, temperature, top_p, top_k, seeds, step):
+    """The sampler's definition, row by row in numpy: whole bins of 1/32 down
+    to the threshold, then the largest z - log(-log u)."""
+    import numpy as np
+    V, out = logits.shape[1], []
+    for row, seed in zip(logits.float().cpu().numpy(), seeds.tolist()):
+        z = (row - row.max()) * (np.float32(1) / np.float32(temperature))
+        inside = z > -32
+        bins = np.minimum(1023, (np.where(inside, -z, 0) * 32).astype(np.int64))
+        p = np.bincount(bins[inside], np.exp(z[inside].astype(np.float64)), 1024).cumsum()
+        c = np.bincount(bins[inside], minlength=1024).cumsum()
+        thr = 1023
+        if top_p < 1:
+            thr = min(thr, int(np.argmax(p >= top_p * p[-1])))
+        if 0 < top_k < V and c[-1] >= top_k:
+            thr = min(thr, int(np.argmax(c >= top_k)))
+        base = np.uint64(seed) ^ _splitmix64(np.uint64(0x5D21 + step))
+        h = _splitmix64(base ^ _splitmix64(np.arange(V, dtype=np.uint64)))
+        u = ((h >> np.uint64(40)).astype(np.float64) + 1) / 16777217.0
+        key = np.where(z >= -(thr + 1) / 32, z - np.log(-np.log(u)), -np.inf)
+        out.append(int(key.argmax()))
+    return out
+
+
+@pytest.mark.parametrize("B,V,dtype", [
+    (3, 8, "bfloat16"), (2, 4096, "bfloat16"), (2, 8200, "bfloat16"), (2, 32768, "bfloat16"),
+    (2, 65536, "bfloat16"), (2, 128256, "bfloat16"), (2, 152064, "bfloat16"),
+    (1, 160000, "bfloat16"), (2, 32003, "bfloat16"), (2, 32003, "float32"),
+    (2, 151936, "float32"), (1200, 40, "float32"), (300, 2056, "bfloat16")])
+@pytest.mark.parametrize("temperature,top_p,top_k", [
+    (1.0, 1.0, 0), (1.2, 0.95, 0), (0.7, 0.8, 50), (1.0, 1.0, 7)])
+def test_sampler_draws_as_defined(ext, B, V, dtype, temperature, top_p, top_k):
+    """One slice and several, aligned rows and others, each threshold, each
+    draw against the definition. The inputs put no cumulative sum within
+    rounding of top_p."""
+    g = torch.Generator().manual_seed(V + B)
+    logits = torch.randn(B, V, generator=g) * 2.5
+    logits[:, 3] += 9.0
+    logits = logits.to("cuda", getattr(torch, dtype))
+    seeds = torch.randint(0, 2 ** 31 - 1, (B,), generator=g)
+    got = ext.sample_tokens(logits, temperature, top_p, top_k, seeds.cuda(),
+                            torch.tensor([11], device="cuda"))
+    assert got.tolist() == _sampled(logits, temperature, top_p, top_k, seeds, 11)
+
+
+def test_sampler_odd_places_and_values(ext):
+    """A matrix that does not start on 16 bytes, rows with -inf, and a row
+    with nothing finite below its maximum."""
+    B, V = 4, 4096
+    g = torch.Generator().manual_seed(1)
+    flat = (torch.randn(B * V + 1, generator=g) * 2).to("cuda", torch.bfloat16)
+    logits = flat[1:].view(B, V)
+    logits[1, ::2] = float("-inf")
+    logits[2] = float("-inf")
+    logits[2, 77] = 1.0
+    seeds, step = torch.arange(B), torch.tensor([5], device="cuda")
+    for top_p in (1.0, 0.9):
+        for x in (logits, logits.clone()):
+            got = ext.sample_tokens(x, 1.0, top_p, 0, seeds.cuda(), step).tolist()
+            assert got == _sampled(logits, 1.0, top_p, 0, seeds, 5)
+            assert got[1] % 2 == 1 and got[2] == 77
+
+
+def test_sampler_in_a_graph(ext):
+    """Replays draw anew with the device step and match eager draws."""
+    logits = _rand((5, 32768), 2, 3.0)
+    seeds, step = torch.arange(5, device="cuda"), torch.zeros(1, dtype=torch.int64, device="cuda")
+    for top_p in (1.0, 0.9):
+        step.zero_()
+        ext.sample_tokens(logits, 1.0, top_p, 0, seeds, step)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = ext.sample_tokens(logits, 1.0, top_p, 0, seeds, step)
+        for i in range(4):
+            step.fill_(i)
+            graph.replay()
+            got = out.clone()
+            assert torch.equal(got, ext.sample_tokens(logits, 1.0, top_p, 0, seeds, step))
