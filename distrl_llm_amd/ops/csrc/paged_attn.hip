@@ -1,246 +1,284 @@
 // Paged-attention decode (GQA) over the block-paged KV pool — the decode
 // hot loop of the generation engine (reference counterpart: vLLM
-// paged_attention_v1/v2), written CDNA4-first:
+// paged_attention_v1/v2).
 //
-//   grid = (num_seqs, n_kv_heads, context_slices); one workgroup owns one
-//   (sequence, kv-head, context-slice) triple and the kv-head's whole
-//   group of query heads (GQA 7:1 on Qwen2.5-7B). 4 waves / 256 threads.
-//   The flash-decoding context split (chosen to fill the chip at decode
-//   batch sizes) emits unnormalized fp32 partials + (m, l) per slice,
-//   combined by paged_decode_combine_kernel.
-//   Phase 1 (scores): each LANE owns one context token — it streams that
-//   token's K row with bf16x8 loads and keeps one fp32 partial per query
-//   head in registers (GROUP is a template param so the per-head array
-//   stays in VGPRs); Q is staged in LDS and read as wave-uniform
-//   broadcasts. No cross-lane reduction at all.
-//   Phase 2: per-head softmax (wave-strided max/sum over the LDS scores).
-//   Phase 3 (PV): V streamed through LDS in 32-token tiles; each thread
-//   accumulates one (head, 8-dim) slice in registers; epilogue divides by
-//   the softmax denominator and stores bf16x8.
-//
-// K and V are each read exactly once from HBM per step; the kernel is
-// KV-bandwidth-bound as it should be.
+// One workgroup owns (sequence, kv head, slice of the context) with all query
+// heads of the kv head; its waves take 32 tokens each in turn and keep a
+// softmax of their own, joined once at the end. Per 32 tokens a wave
+//  * loads K rows straight into MFMA operands (16x16x32: lane = token row,
+//    16 B pieces) and forms S^T[token][head] = K Q^T, q and K exact in bf16,
+//    sums in fp32;
+//  * keeps the weights in fp32 and feeds them to the second product as two
+//    bf16 terms, p = hi + lo (error 2^-17 of p): the accumulator's token rows
+//    serve as k-slots as they lie;
+//  * passes V rows through a tile of its own in LDS and reads them back
+//    transposed (LDS transpose reads); no workgroup barrier in the loop.
+// The next 32 tokens' rows are in flight meanwhile (page numbers two ahead).
+// K and V are read once per sequence and kv head; bound by HBM.
+// 160 sequences of 420..1550 tokens sharing prompts, 28/4 heads of 128
+// (251 MB of distinct rows): 157 us with one lane a token on vector FMAs,
+// 76 us now; 3 sequences of 911..3777, 14/2 heads of 64: 43 -> 12.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
 
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16v8;
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16v4;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((address_space(3))) bf16v4 lds_bf16v4;
+
 namespace {
 
-constexpr int VTILE = 64;        // V tokens staged per LDS tile
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr int CHUNK = 32;        // tokens of a wave's step
 
-template <int D, int GROUP>
-__global__ __launch_bounds__(256)
-void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // (N,H,D)
-                         const __hip_bfloat16* __restrict__ kcache, // (nb,bs,KV,D)
+// 16 B chunk c of row r in a wave's V tile: rows read at one chunk (writes)
+// and 16 rows read over two chunks (transpose reads) spread over the banks.
+template <int D>
+DEV_INLINE int v_off(int r, int c) {
+  return r * (2 * D) + ((c ^ (D == 128 ? r & 15 : (r >> 1) & 7)) << 4);
+}
+
+template <int D, int NW>
+__global__ __launch_bounds__(NW * 64, 2)
+void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q_row_stride
+                         const __hip_bfloat16* __restrict__ kcache, // (nb, bs, KV, D)
                          const __hip_bfloat16* __restrict__ vcache,
-                         const int* __restrict__ block_tables,      // (N,max_nb)
+                         const int* __restrict__ block_tables,      // (N, max_nb)
                          const int* __restrict__ ctx_lens,          // (N,)
-                         __hip_bfloat16* __restrict__ out,          // (N,H,D)
-                         float* __restrict__ o_part,  // (CS,N,H,D) | null
-                         float* __restrict__ ml_part, // (CS,N,H,2) | null
-                         int H, int KV, int max_nb, int block_size,
-                         int Lpad, float scale, int64_t q_row_stride,
-                         int slice_len) {
-  const int seq = blockIdx.x;
-  const int kv = blockIdx.y;
-  const int zid = blockIdx.z;     // context slice (flash-decoding split)
-  const int Lall = ctx_lens[seq];
-  const int c0 = zid * slice_len;
-  const int L = min(Lall, c0 + slice_len);  // this slice: [c0, L)
-  const int tid = threadIdx.x;
+                         __hip_bfloat16* __restrict__ out,          // (N, H, D)
+                         float* __restrict__ o_part,                // (cs, N, H, D)
+                         float* __restrict__ ml_part,               // (cs, N, H, 2)
+                         int H, int KV, int max_nb, int block_size, int bs_shift,
+                         float scale_log2, int64_t q_row_stride, int slice_len) {
+  constexpr int KS = D / 32, DT = D / 16;
+  const int seq = blockIdx.x, kv = blockIdx.y, z = blockIdx.z, N = gridDim.x;
+  const int group = H / KV;
+  const int len = ctx_lens[seq];
+  const int c0 = z * slice_len, c1 = min(len, c0 + slice_len);
+  if (z > 0 && c0 >= len) return;       // an empty slice is not read
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l = threadIdx.x & 63, g = l >> 4, lr = l & 15;
 
-  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  float* q_lds = reinterpret_cast<float*>(smem_raw);          // GROUP*D
-  float* denom = q_lds + GROUP * D;                           // padded to 4
-  float* gmax = denom + ((GROUP + 3) & ~3);                   // slice maxes
-  float* scores = gmax + ((GROUP + 3) & ~3);                  // GROUP*Lpad
-  __hip_bfloat16* v_lds = reinterpret_cast<__hip_bfloat16*>(
-      scores + (size_t)GROUP * Lpad);                         // VTILE*D
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  char* tile = smem + wave * (CHUNK * D * 2);           // also 16 heads x D floats
+  float* ml_lds = reinterpret_cast<float*>(smem + NW * (CHUNK * D * 2));  // [NW][16][2]
+
+  bf16v8 qf[KS];
+  #pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const __hip_bfloat16* qp = q + seq * q_row_stride + (kv * group + min(lr, group - 1)) * D;
+    qf[ks] = *reinterpret_cast<const bf16v8*>(qp + ks * 32 + g * 8);   // spare columns repeat
+  }
+
+  float m = -1e30f, lsum = 0.f;
+  f32x4 acc[DT];
+  #pragma unroll
+  for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int* bt = block_tables + (int64_t)seq * max_nb;
-  const int64_t kv_row = (int64_t)KV * D;
-
-  // ---- stage Q (group heads of this kv head) into LDS as fp32 ----
-  for (int i = tid; i < GROUP * D; i += blockDim.x) {
-    const int h = kv * GROUP + i / D;
-    q_lds[i] = bf2f(q[(int64_t)seq * q_row_stride + h * D + i % D]) * scale;
-  }
-  __syncthreads();
-
-  // ---- phase 1: one token per lane, per-head partials in VGPRs ----
-  for (int t = c0 + tid; t < L; t += blockDim.x) {
-    const int64_t row = (int64_t)bt[t / block_size] * block_size
-                        + t % block_size;
-    const bf16x8* kp = reinterpret_cast<const bf16x8*>(
-        kcache + row * kv_row + (int64_t)kv * D);
-    float part[GROUP];
+  const int row_elems = KV * D;
+  bf16v8 kf[2][KS], vf[2][KS];
+  int page[2], slot[2];                 // this lane's two tokens of a chunk
+  auto lookup = [&](int t0) {
     #pragma unroll
-    for (int h = 0; h < GROUP; ++h) part[h] = 0.f;
+    for (int s = 0; s < 2; ++s) {
+      const int t = min(t0 + s * 16 + lr, c1 - 1);      // past the end: weight zero
+      const int b = bs_shift >= 0 ? t >> bs_shift : t / block_size;
+      slot[s] = t - b * block_size;
+      page[s] = bt[b];
+    }
+  };
+  auto offset = [&](int s) {
+    return ((int64_t)page[s] * block_size + slot[s]) * row_elems + kv * D + g * 8;
+  };
+
+  int t0 = c0 + wave * CHUNK;
+  if (t0 < c1) {
+    lookup(t0);
     #pragma unroll
-    for (int c = 0; c < D / 8; ++c) {
-      const bf16x8 kvec = kp[c];
-      float kf[8];
+    for (int s = 0; s < 2; ++s) {
+      const int64_t at = offset(s);
       #pragma unroll
-      for (int j = 0; j < 8; ++j) kf[j] = bf2f(kvec.v[j]);
-      #pragma unroll
-      for (int h = 0; h < GROUP; ++h) {
-        const float* qh = q_lds + h * D + c * 8;   // wave-uniform broadcast
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) part[h] += qh[j] * kf[j];
+      for (int ks = 0; ks < KS; ++ks) {
+        kf[s][ks] = *reinterpret_cast<const bf16v8*>(kcache + at + ks * 32);
+        vf[s][ks] = *reinterpret_cast<const bf16v8*>(vcache + at + ks * 32);
       }
     }
+    lookup(t0 + NW * CHUNK);
+  }
+  for (; t0 < c1; t0 += NW * CHUNK) {
+    const bool more = t0 + NW * CHUNK < c1;             // wave-uniform
+    int64_t at[2];
     #pragma unroll
-    for (int h = 0; h < GROUP; ++h) scores[(size_t)h * Lpad + (t - c0)] = part[h];
-  }
-  __syncthreads();
-
-  // ---- phase 2: per-head softmax over the LDS scores ----
-  const int wid = tid / WAVE;
-  const int wlane = tid % WAVE;
-  const int nw = blockDim.x / WAVE;
-  const int Ls = L - c0;  // tokens in this slice (may be <= 0)
-  for (int h = wid; h < GROUP; h += nw) {
-    float* s = scores + (size_t)h * Lpad;
-    float m = -1e30f;
-    for (int t = wlane; t < Ls; t += WAVE) m = fmaxf(m, s[t]);
-    m = wave_max(m);
-    float d = 0.f;
-    for (int t = wlane; t < Ls; t += WAVE) {
-      float e = __expf(s[t] - m);
-      s[t] = e;
-      d += e;
-    }
-    d = wave_sum(d);
-    if (wlane == 0) {
-      denom[h] = d;
-      gmax[h] = m;
-    }
-  }
-  __syncthreads();
-
-  // ---- phase 3: PV accumulation through LDS V tiles ----
-  constexpr int DV = D / 8;             // bf16x8 units per row
-  constexpr int UNITS = GROUP * DV;     // <= 16*16 = 256
-  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  const int u = tid;                    // one unit per thread (tid < UNITS)
-  const int uh = u / DV, ud = u % DV;
-
-  for (int base = 0; base < Ls; base += VTILE) {
-    const int tile = min(VTILE, Ls - base);
-    // stage V rows [base, base+tile) for this kv head
-    for (int i = tid; i < tile * DV; i += blockDim.x) {
-      const int tt = c0 + base + i / DV;
-      const int64_t row = (int64_t)bt[tt / block_size] * block_size
-                          + tt % block_size;
-      reinterpret_cast<bf16x8*>(v_lds)[i] =
-          *reinterpret_cast<const bf16x8*>(
-              vcache + row * kv_row + (int64_t)kv * D + (i % DV) * 8);
-    }
-    __syncthreads();
-    if (u < UNITS) {
-      const float* ps = scores + (size_t)uh * Lpad + base;
-      #pragma unroll 4
-      for (int j = 0; j < tile; ++j) {
-        const float p = ps[j];
-        const bf16x8 vv = reinterpret_cast<const bf16x8*>(v_lds)[j * DV + ud];
-        #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] += p * bf2f(vv.v[e]);
-      }
-    }
-    __syncthreads();
-  }
-
-  if (u < UNITS) {
-    const int h = kv * GROUP + uh;
-    if (o_part == nullptr) {
-      const float inv = 1.f / denom[uh];
-      bf16x8 o;
+    for (int s = 0; s < 2; ++s) at[s] = offset(s);
+    f32x4 st[2];
+    #pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      st[s] = f32x4{0.f, 0.f, 0.f, 0.f};
       #pragma unroll
-      for (int e = 0; e < 8; ++e) o.v[e] = f2bf(acc[e] * inv);
-      *reinterpret_cast<bf16x8*>(out + ((int64_t)seq * H + h) * D + ud * 8) = o;
+      for (int ks = 0; ks < KS; ++ks)
+        st[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s][ks], qf[ks], st[s], 0, 0, 0);
+    }
+    #pragma unroll
+    for (int s = 0; s < 2; ++s)
+      #pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        *reinterpret_cast<bf16v8*>(tile + v_off<D>(s * 16 + lr, ks * 4 + g)) = vf[s][ks];
+    if (more) {
+      #pragma unroll
+      for (int s = 0; s < 2; ++s)
+        #pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          kf[s][ks] = *reinterpret_cast<const bf16v8*>(kcache + at[s] + ks * 32);
+          vf[s][ks] = *reinterpret_cast<const bf16v8*>(vcache + at[s] + ks * 32);
+        }
+      lookup(t0 + 2 * NW * CHUNK);
+    }
+
+    // this lane: head lr, tokens t0 + 16 s + 4 g + r
+    float mx = -1e30f;
+    #pragma unroll
+    for (int s = 0; s < 2; ++s)
+      #pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        st[s][r] = t0 + s * 16 + g * 4 + r < c1 ? st[s][r] * scale_log2 : -1e30f;
+        mx = fmaxf(mx, st[s][r]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+    // the subtracted maximum may lag by 2^8 (see the rescaling's cost)
+    if (__any(mx > m + 8.f)) {
+      const float m_new = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - m_new);
+      lsum *= alpha;
+      #pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        #pragma unroll
+        for (int r = 0; r < 4; ++r) acc[dt][r] *= alpha;
+      m = m_new;
+    }
+    bf16v8 hi, lo;
+    #pragma unroll
+    for (int s = 0; s < 2; ++s)
+      #pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float p = __builtin_amdgcn_exp2f(st[s][r] - m);
+        lsum += p;
+        hi[s * 4 + r] = (__bf16)p;
+        lo[s * 4 + r] = (__bf16)(p - (float)hi[s * 4 + r]);
+      }
+    __builtin_amdgcn_wave_barrier();
+    #pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      // V^T: rows d = 16 dt + lr, k-slots = tokens 4g.. and 16 + 4g..
+      const int c = dt * 2 + ((l & 3) >> 1), r0 = 4 * g + (lr >> 2), e = (l & 1) * 8;
+      const bf16v4 a = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16v4*)(tile + v_off<D>(r0, c) + e));
+      const bf16v4 b = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16v4*)(tile + v_off<D>(r0 + 16, c) + e));
+      const bf16v8 vt = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, hi, acc[dt], 0, 0, 0);
+      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, lo, acc[dt], 0, 0, 0);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+
+  // join the waves: m, l per head, then the weighted sums
+  lsum += __shfl_xor(lsum, 16, WAVE);
+  lsum += __shfl_xor(lsum, 32, WAVE);
+  if (g == 0) {
+    ml_lds[(wave * 16 + lr) * 2] = m;
+    ml_lds[(wave * 16 + lr) * 2 + 1] = lsum;
+  }
+  float* o_tile = reinterpret_cast<float*>(tile);       // [16 heads][D]
+  #pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+    *reinterpret_cast<f32x4*>(o_tile + lr * D + dt * 16 + g * 4) = acc[dt];
+  __syncthreads();
+  const bool whole = len <= slice_len;                  // nothing to join outside
+  for (int i = threadIdx.x; i < group * (D / 4); i += NW * 64) {
+    const int h = i / (D / 4), d = i % (D / 4) * 4;
+    float top = -1e30f, total = 0.f;
+    #pragma unroll
+    for (int w = 0; w < NW; ++w) top = fmaxf(top, ml_lds[(w * 16 + h) * 2]);
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    #pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float f = __builtin_amdgcn_exp2f(ml_lds[(w * 16 + h) * 2] - top);
+      total += f * ml_lds[(w * 16 + h) * 2 + 1];
+      const f32x4 x = *reinterpret_cast<const f32x4*>(smem + w * (CHUNK * D * 2) + (h * D + d) * 4);
+      #pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] += f * x[r];
+    }
+    const int64_t head = (int64_t)seq * H + kv * group + h;
+    if (whole) {
+      const float inv = total > 0.f ? 1.f / total : 0.f;
+      bf16v4 y;
+      #pragma unroll
+      for (int r = 0; r < 4; ++r) y[r] = (__bf16)(o[r] * inv);
+      *reinterpret_cast<bf16v4*>(out + head * D + d) = y;
     } else {
-      // flash-decoding partial: unnormalized o + (m, l) per slice
-      const int64_t oz = (((int64_t)zid * gridDim.x + seq) * H + h) * D + ud * 8;
-      #pragma unroll
-      for (int e = 0; e < 8; ++e) o_part[oz + e] = acc[e];
-      if (ud == 0) {
-        const int64_t mz = (((int64_t)zid * gridDim.x + seq) * H + h) * 2;
-        ml_part[mz] = (Ls > 0) ? gmax[uh] : -1e30f;
-        ml_part[mz + 1] = (Ls > 0) ? denom[uh] : 0.f;
-      }
+      const int64_t at = (int64_t)z * N * H + head;
+      *reinterpret_cast<f32x4*>(o_part + at * D + d) = o;
+      if (d == 0) { ml_part[at * 2] = top; ml_part[at * 2 + 1] = total; }
     }
   }
 }
 
-// flash-decoding combine: out[seq,h] = sum_z w_z*o_z / sum_z w_z*l_z,
-// w_z = exp(m_z - max_z m_z). grid (N, H), D/64 elems per lane.
+// Joins the slices of a sequence that has more than one. grid (N, H), one wave.
 template <int D>
 __global__ __launch_bounds__(64)
 void paged_decode_combine_kernel(const float* __restrict__ o_part,
                                  const float* __restrict__ ml_part,
-                                 __hip_bfloat16* __restrict__ out,
-                                 int H, int cs) {
-  const int seq = blockIdx.x;
-  const int h = blockIdx.y;
-  const int N = gridDim.x;
-  const int lane = threadIdx.x;
-  float M = -1e30f;
-  for (int z = 0; z < cs; ++z)
-    M = fmaxf(M, ml_part[(((int64_t)z * N + seq) * H + h) * 2]);
-  float Lsum = 0.f;
-  float o[D / 64];
+                                 const int* __restrict__ ctx_lens,
+                                 __hip_bfloat16* __restrict__ out, int H, int slice_len) {
+  const int seq = blockIdx.x, h = blockIdx.y, N = gridDim.x, lane = threadIdx.x;
+  const int len = ctx_lens[seq];
+  if (len <= slice_len) return;                         // written already
+  const int n = (len + slice_len - 1) / slice_len;
+  const int64_t head = (int64_t)seq * H + h, step = (int64_t)N * H;
+  float top = -1e30f;
+  for (int z = 0; z < n; ++z) top = fmaxf(top, ml_part[(z * step + head) * 2]);
+  float total = 0.f, o[D / 64];
   #pragma unroll
   for (int e = 0; e < D / 64; ++e) o[e] = 0.f;
-  for (int z = 0; z < cs; ++z) {
-    const int64_t mz = (((int64_t)z * N + seq) * H + h) * 2;
-    const float w = __expf(ml_part[mz] - M);
-    Lsum += w * ml_part[mz + 1];
-    const int64_t oz = (((int64_t)z * N + seq) * H + h) * D;
+  for (int z = 0; z < n; ++z) {
+    const int64_t at = z * step + head;
+    const float w = __builtin_amdgcn_exp2f(ml_part[at * 2] - top);
+    total += w * ml_part[at * 2 + 1];
     #pragma unroll
-    for (int e = 0; e < D / 64; ++e)
-      o[e] += w * o_part[oz + lane + e * 64];
+    for (int e = 0; e < D / 64; ++e) o[e] += w * o_part[at * D + lane + e * 64];
   }
-  const float inv = 1.f / Lsum;
+  const float inv = 1.f / total;
   #pragma unroll
-  for (int e = 0; e < D / 64; ++e)
-    out[((int64_t)seq * H + h) * D + lane + e * 64] = f2bf(o[e] * inv);
+  for (int e = 0; e < D / 64; ++e) out[head * D + lane + e * 64] = f2bf(o[e] * inv);
 }
 
-template <int D, int GROUP>
-void launch(const torch::Tensor& q, const torch::Tensor& kcache,
-            const torch::Tensor& vcache, const torch::Tensor& bt,
-            const torch::Tensor& ctx, torch::Tensor& out, int H, int KV,
-            int max_nb, int block_size, int Lpad, float scale, size_t smem,
-            int64_t q_row_stride, int cs, int slice_len) {
-  const int N = q.size(0);
+template <int D, int NW>
+void launch_decode(const torch::Tensor& q, const torch::Tensor& kcache,
+                   const torch::Tensor& vcache, const torch::Tensor& bt,
+                   const torch::Tensor& ctx, torch::Tensor& out, int H, int KV,
+                   float scale, int64_t q_row_stride, int cs, int slice_len) {
+  const int N = q.size(0), block_size = kcache.size(1);
+  const int shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1;
   auto stream = at::cuda::getCurrentCUDAStream();
-  dim3 grid(N, KV, cs), block(256);
-  float* o_p = nullptr;
-  float* ml_p = nullptr;
-  torch::Tensor o_part, ml_part;
+  torch::Tensor part;
+  float *o_p = nullptr, *ml_p = nullptr;
   if (cs > 1) {
-    auto opts = out.options().dtype(at::kFloat);
-    o_part = torch::empty({cs, N, H, D}, opts);
-    ml_part = torch::empty({cs, N, H, 2}, opts);
-    o_p = o_part.data_ptr<float>();
-    ml_p = ml_part.data_ptr<float>();
+    const int64_t heads = (int64_t)cs * N * H;
+    part = torch::empty({heads * (D + 2)}, out.options().dtype(at::kFloat));
+    o_p = part.data_ptr<float>();
+    ml_p = o_p + heads * D;
   }
-  hipLaunchKernelGGL((paged_decode_kernel<D, GROUP>), grid, block, smem,
-                     stream,
+  auto* o = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
+  hipLaunchKernelGGL((paged_decode_kernel<D, NW>), dim3(N, KV, cs), dim3(NW * 64),
+                     NW * (CHUNK * D * 2 + 16 * 2 * 4), stream,
                      reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
                      reinterpret_cast<const __hip_bfloat16*>(kcache.data_ptr()),
                      reinterpret_cast<const __hip_bfloat16*>(vcache.data_ptr()),
-                     bt.data_ptr<int>(), ctx.data_ptr<int>(),
-                     reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                     o_p, ml_p,
-                     H, KV, max_nb, block_size, Lpad, scale, q_row_stride,
-                     slice_len);
-  if (cs > 1) {
-    hipLaunchKernelGGL((paged_decode_combine_kernel<D>), dim3(N, H), dim3(64),
-                       0, stream, o_p, ml_p,
-                       reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                       H, cs);
-  }
+                     bt.data_ptr<int>(), ctx.data_ptr<int>(), o, o_p, ml_p, H, KV,
+                     (int)bt.size(1), block_size, shift, scale * LOG2E, q_row_stride, slice_len);
+  if (cs > 1)
+    hipLaunchKernelGGL((paged_decode_combine_kernel<D>), dim3(N, H), dim3(64), 0, stream, o_p,
+                       ml_p, ctx.data_ptr<int>(), o, H, slice_len);
 }
 
 }  // namespace
@@ -256,6 +294,11 @@ torch::Tensor paged_attention_decode_strided(
   TORCH_CHECK(block_tables.scalar_type() == at::kInt &&
               ctx_lens.scalar_type() == at::kInt);
   const int N = q.size(0), H = (int)n_heads, D = (int)head_dim;
+  if (q_row_stride % 8 != 0 || reinterpret_cast<uintptr_t>(q.data_ptr()) % 16 != 0) {
+    // rows that 16 B loads cannot read
+    q = q.view({N, q_row_stride}).slice(1, 0, (int64_t)H * D).clone(at::MemoryFormat::Contiguous);
+    q_row_stride = (int64_t)H * D;
+  }
   const int KV = kcache.size(2);
   const int block_size = kcache.size(1);
   const int max_nb = block_tables.size(1);
@@ -264,42 +307,35 @@ torch::Tensor paged_attention_decode_strided(
 
   auto out = torch::empty({N, (int64_t)H, (int64_t)D}, q.options());
   if (N == 0) return out;
+  TORCH_CHECK((D == 128 && (group <= 2 || (group >= 4 && group <= 8))) ||
+              (D == 64 && (group == 1 || group == 2 || group == 4 || group == 7)),
+              "paged decode: unsupported (head_dim=", D, ", gqa group=", group, ")");
 
+  // Slices of the context (known here: a table's width, not its sequence's
+  // length). A round of loads takes ~4 us from cold pages, the joining kernel
+  // as long: few sequences run with eight waves in slices of 512 tokens, up to
+  // one workgroup a CU (16 sequences of 1500, 4 kv heads: 1 slice 25 us, 2: 18,
+  // 4: 14, 6: 19; 8 sequences of 4000, 8 kv heads: 63, 39, 29, 8 slices 34).
+  // More sequences fill the chip by themselves; two slices even out their
+  // lengths where they are long (the round above: 1 slice 80 us, 2: 76, 4: 79;
+  // 32 sequences of 700, 8 kv heads: 16, 18, 21).
   const int max_ctx = max_nb * block_size;
-  // flash-decoding context split: fill the chip (N*KV blocks alone leave
-  // most CUs idle at decode batch sizes) and shorten the per-block chain
-  // sweep-tuned: ~2048 blocks beats ~1024 at decode batch 160 (113 vs
-  // 137 us at ctx 800 — smaller LDS score tiles double the blocks/CU);
-  // cs=8+ loses to combine overhead (profiles/)
-  int cs = 1;
-  while (cs * 2 <= 8 && N * KV * cs < 2048
-         && (max_ctx + cs * 2 - 1) / (cs * 2) >= 128)
-    cs *= 2;
+  const int64_t blocks = (int64_t)N * KV;
+  const bool few = blocks < 256;
+  int cs = few ? (int)std::max<int64_t>(1, std::min<int64_t>(256 / blocks, CDIV(max_ctx, 512)))
+               : (blocks < 1024 && max_ctx >= 1024 ? 2 : 1);
   if (const char* e = getenv("DISTRL_PAGED_CS")) {
     cs = std::max(1, std::min(atoi(e), 16));
     while (cs > 1 && (max_ctx + cs - 1) / cs < 32) cs /= 2;
   }
-  const int slice_len = (max_ctx + cs - 1) / cs;
-  const int Lpad = slice_len + 4;  // +pad to stagger LDS banks across heads
-  size_t smem = (size_t)group * D * 4 + 2 * ((group + 3) & ~3) * 4
-                + (size_t)group * Lpad * 4 + (size_t)VTILE * D * 2;
-  TORCH_CHECK(smem <= 160 * 1024,
-              "context too long for single-pass decode kernel: ", max_ctx);
-
-  auto bt = block_tables;
-  auto ctx = ctx_lens;
-  const float sc = (float)scale;
-  #define CASE(DD, GG) \
-    if (D == DD && group == GG) { \
-      launch<DD, GG>(q, kcache, vcache, bt, ctx, out, H, KV, max_nb, \
-                     block_size, Lpad, sc, smem, q_row_stride, cs, \
-                     slice_len); \
-      HIP_CHECK_LAST(); return out; }
-  CASE(128, 7) CASE(128, 5) CASE(128, 4) CASE(128, 8) CASE(128, 6)
-  CASE(128, 2) CASE(128, 1) CASE(64, 7) CASE(64, 4) CASE(64, 2) CASE(64, 1)
-  #undef CASE
-  TORCH_CHECK(false, "paged decode: unsupported (head_dim=", D,
-              ", gqa group=", group, ")");
+  const int slice_len = std::max(1, CDIV(max_ctx, cs));
+  #define DECODE(DD, NN) launch_decode<DD, NN>(q, kcache, vcache, block_tables, ctx_lens, out, H, \
+                                               KV, (float)scale, q_row_stride, cs, slice_len)
+  if (D == 128) { if (few) DECODE(128, 8); else DECODE(128, 4); }
+  else { if (few) DECODE(64, 8); else DECODE(64, 4); }
+  #undef DECODE
+  HIP_CHECK_LAST();
+  return out;
 }
 
 

@@ -194,3 +194,59 @@ def test_sampler_in_a_graph(ext):
             graph.replay()
             got = out.clone()
             assert torch.equal(got, ext.sample_tokens(logits, 1.0, top_p, 0, seeds, step))
+
+
+# --------------------------------------------------- paged decode attention
+# Bound: the output's rounding, 2^-9 of each value at most; scores and sums are
+# fp32 and the weights carry 17 bits.
+DECODE_REL = 2.0 ** -8
+
+
+@pytest.mark.parametrize("H,KV,D", [(28, 4, 128), (5, 5, 128), (10, 2, 128), (14, 2, 64), (8, 8, 64)])
+@pytest.mark.parametrize("ctxs,width,bs", [
+    ([1, 2, 15, 16, 17, 31, 32, 33], 40, 16), ([100, 255, 256, 257, 511, 512, 513], 520, 16),
+    ([2048, 1, 1025], 2048, 16), ([5000, 3, 2049, 257], 5000, 16), ([77, 300], 333, 12),
+    ([400 + i for i in range(130)], 560, 16), ([60], 64, 1)])
+def test_paged_decode_edges(ext, H, KV, D, ctxs, width, bs):
+    """Chunk ends, one and several slices (also empty ones), eight and four
+    waves, page sizes that are no power of two; pages in random order, some
+    shared, and NaN in every row that no sequence holds."""
+    g = torch.Generator().manual_seed(len(ctxs) + H)
+    nb = (width + bs - 1) // bs
+    pages = nb * len(ctxs)
+    bt = torch.randperm(pages, generator=g).view(len(ctxs), nb).int()
+    bt[:, 0] = bt[0, 0]
+    q, kc, vc = (_rand(s, i) for i, s in enumerate(
+        ((len(ctxs), H, D), (pages, bs, KV, D), (pages, bs, KV, D))))
+    used = torch.zeros(pages, bs, dtype=torch.bool)
+    for i, n in enumerate(ctxs):
+        t = torch.arange(n)
+        used[bt[i, t // bs].long(), t % bs] = True
+    kc[~used.cuda()] = float("nan")
+    vc[~used.cuda()] = float("nan")
+    lens = torch.tensor(ctxs, dtype=torch.int32)
+    for scale in (D ** -0.5, -1.0):
+        out = ext.paged_attention_decode(q, kc, vc, bt.cuda(), lens.cuda(), scale)
+        for i, n in enumerate(ctxs):
+            t = torch.arange(n)
+            k, v = (c[bt[i, t // bs].long().cuda(), (t % bs).cuda()].double().transpose(0, 1)
+                    .repeat_interleave(H // KV, 0) for c in (kc, vc))
+            p = ((k @ q[i].double().unsqueeze(2)).squeeze(2) * scale).softmax(-1)
+            assert _rel(out[i], (p.unsqueeze(1) @ v).squeeze(1)) < DECODE_REL, (i, n)
+
+
+def test_paged_decode_reads_packed_rows(ext):
+    """Query heads at the head of wider rows, at any alignment."""
+    H, KV, D, N = 14, 2, 64, 3
+    kc, vc = _rand((9, 16, KV, D), 1), _rand((9, 16, KV, D), 2)
+    bt = torch.arange(9, dtype=torch.int32).view(3, 3).cuda()
+    lens = torch.tensor([48, 7, 33], dtype=torch.int32, device="cuda")
+    q = _rand((N, H, D), 3)
+    ref = ext.paged_attention_decode(q, kc, vc, bt, lens, 0.125)
+    for stride in (H * D + 2 * KV * D, H * D + 3):
+        flat = torch.zeros(N * stride + 1, dtype=torch.bfloat16, device="cuda")
+        for off in (0, 1):
+            rows = flat[off:off + N * stride].view(N, stride)
+            rows[:, :H * D] = q.view(N, -1)
+            out = ext.paged_attention_decode_strided(rows, H, D, stride, kc, vc, bt, lens, 0.125)
+            assert torch.equal(out, ref)
