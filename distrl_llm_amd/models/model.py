@@ -20,6 +20,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from ..ops import reference as R
+from . import fused_layer
 from .lora import LoRALinear
 from .spec import ModelSpec
 
@@ -128,7 +129,11 @@ class DecoderLayer(nn.Module):
                                                 dtype, device)
         self.mlp = MLP(spec, r, alpha, dropout, dtype, device)
 
-    def forward(self, x, cos, sin, attn_bias):
+    def forward(self, x, cos, sin, attn_bias, rotary=None):
+        """rotary: (int32 positions (B*T,), inverse frequencies, their
+        negatives): the rotation of cos and sin, for the fused nodes."""
+        if attn_bias is None and rotary is not None and fused_layer.usable(self, x):
+            return fused_layer.forward(self, x, rotary)
         x = x + self.self_attn(self.input_layernorm(x), cos, sin, attn_bias)
         x = x + self.mlp(self.post_attention_layernorm(x))
         return x
@@ -274,9 +279,15 @@ class CausalLM(nn.Module):
             bias = torch.zeros(B, 1, T, T, dtype=self.dtype_, device=input_ids.device)
             bias.masked_fill_(~allow, torch.finfo(self.dtype_).min)
 
+        rotary = None
+        if input_ids.is_cuda:
+            half = torch.arange(0, self.spec.head_dim, 2, device=input_ids.device,
+                                dtype=torch.float32)
+            inv_freq = 1.0 / (self.spec.rope_theta ** (half / self.spec.head_dim))
+            rotary = (position_ids.reshape(-1).to(torch.int32), inv_freq, -inv_freq)
         x = self.model.embed_tokens(input_ids)
         for layer in self.model.layers:
-            x = layer(x, cos, sin, bias)
+            x = layer(x, cos, sin, bias, rotary)
         return self.model.norm(x)
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:

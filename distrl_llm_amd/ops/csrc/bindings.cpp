@@ -5,6 +5,8 @@
 torch::Tensor rmsnorm_fwd(torch::Tensor x, torch::Tensor w, double eps);
 torch::Tensor rmsnorm_bwd(torch::Tensor dy, torch::Tensor x, torch::Tensor w,
                           double eps);
+torch::Tensor rmsnorm_bwd_add(torch::Tensor dy, torch::Tensor x,
+                              torch::Tensor w, torch::Tensor g, double eps);
 std::vector<torch::Tensor> add_rmsnorm_fwd(torch::Tensor x, torch::Tensor h,
                                            torch::Tensor w, double eps);
 torch::Tensor silu_mul_fwd(torch::Tensor gate, torch::Tensor up);
@@ -64,6 +66,8 @@ void adam8bit_step(torch::Tensor p, torch::Tensor g, torch::Tensor m_q,
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm_fwd", &rmsnorm_fwd, "RMSNorm forward (gfx950)");
   m.def("rmsnorm_bwd", &rmsnorm_bwd, "RMSNorm backward dx (gfx950)");
+  m.def("rmsnorm_bwd_add", &rmsnorm_bwd_add,
+        "RMSNorm backward dx plus the residual's gradient");
   m.def("add_rmsnorm_fwd", &add_rmsnorm_fwd,
         "fused residual add + RMSNorm forward");
   m.def("silu_mul_fwd", &silu_mul_fwd, "fused SiLU*mul forward");

@@ -52,14 +52,17 @@ __global__ void rmsnorm_fwd_f32(const float* __restrict__ x,
   for (int i = threadIdx.x; i < hidden; i += blockDim.x) yr[i] = xr[i] * r * w[i];
 }
 
-// dx = r*(dy*w) - r^3/H * x * sum(dy*w*x)
+// dx = r*(dy*w) - r^3/H * x * sum(dy*w*x), plus g where given: the gradient
+// that reaches x past the norm (the residual's), which saves a pass of its own
 __global__ void rmsnorm_bwd_bf16(const __hip_bfloat16* __restrict__ dy,
                                  const __hip_bfloat16* __restrict__ x,
                                  const __hip_bfloat16* __restrict__ w,
+                                 const __hip_bfloat16* __restrict__ g,
                                  __hip_bfloat16* __restrict__ dx,
                                  int hidden, float eps) {
   __shared__ float red[16];
   const int64_t row = blockIdx.x;
+  const bf16x8* gr = reinterpret_cast<const bf16x8*>(g + row * hidden);
   const bf16x8* dyr = reinterpret_cast<const bf16x8*>(dy + row * hidden);
   const bf16x8* xr = reinterpret_cast<const bf16x8*>(x + row * hidden);
   const bf16x8* wr = reinterpret_cast<const bf16x8*>(w);
@@ -82,11 +85,13 @@ __global__ void rmsnorm_bwd_bf16(const __hip_bfloat16* __restrict__ dy,
   const float r = rsqrtf(ss / hidden + eps);
   const float c = r * r * r * dot / hidden;
   for (int i = threadIdx.x; i < nvec; i += blockDim.x) {
-    bf16x8 xv = xr[i], dyv = dyr[i], wv = wr[i], o;
+    bf16x8 xv = xr[i], dyv = dyr[i], wv = wr[i], gv, o;
+    if (g) gv = gr[i];
     #pragma unroll
     for (int j = 0; j < 8; ++j) {
       float dyw = bf2f(dyv.v[j]) * bf2f(wv.v[j]);
-      o.v[j] = f2bf(dyw * r - bf2f(xv.v[j]) * c);
+      float d = dyw * r - bf2f(xv.v[j]) * c;
+      o.v[j] = f2bf(g ? d + bf2f(gv.v[j]) : d);
     }
     dxr[i] = o;
   }
@@ -157,6 +162,7 @@ torch::Tensor rmsnorm_bwd(torch::Tensor dy, torch::Tensor x, torch::Tensor w,
                        reinterpret_cast<const __hip_bfloat16*>(dy.data_ptr()),
                        reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()),
                        reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()),
+                       (const __hip_bfloat16*)nullptr,
                        reinterpret_cast<__hip_bfloat16*>(dx.data_ptr()),
                        hidden, (float)eps);
   } else {
@@ -166,6 +172,29 @@ torch::Tensor rmsnorm_bwd(torch::Tensor dy, torch::Tensor x, torch::Tensor w,
                        w.data_ptr<float>(), dx.data_ptr<float>(),
                        hidden, (float)eps);
   }
+  HIP_CHECK_LAST();
+  return dx;
+}
+
+// dx = g + rmsnorm's dx (bf16)
+torch::Tensor rmsnorm_bwd_add(torch::Tensor dy, torch::Tensor x, torch::Tensor w,
+                              torch::Tensor g, double eps) {
+  TORCH_CHECK(dy.is_cuda() && dy.is_contiguous() && x.is_contiguous() && g.is_contiguous());
+  TORCH_CHECK(dy.scalar_type() == at::kBFloat16 && x.scalar_type() == at::kBFloat16 &&
+              w.scalar_type() == at::kBFloat16 && g.scalar_type() == at::kBFloat16);
+  TORCH_CHECK(dy.sizes() == x.sizes() && g.sizes() == x.sizes() && w.numel() == x.size(-1));
+  const int hidden = x.size(-1);
+  TORCH_CHECK(hidden % 8 == 0);
+  const int64_t rows = x.numel() / hidden;
+  auto dx = torch::empty_like(x);
+  if (rows == 0) return dx;
+  hipLaunchKernelGGL(rmsnorm_bwd_bf16, dim3(rows), dim3(256), 0,
+                     at::cuda::getCurrentCUDAStream(),
+                     reinterpret_cast<const __hip_bfloat16*>(dy.data_ptr()),
+                     reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()),
+                     reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()),
+                     reinterpret_cast<const __hip_bfloat16*>(g.data_ptr()),
+                     reinterpret_cast<__hip_bfloat16*>(dx.data_ptr()), hidden, (float)eps);
   HIP_CHECK_LAST();
   return dx;
 }

@@ -250,3 +250,107 @@ def test_paged_decode_reads_packed_rows(ext):
             rows[:, :H * D] = q.view(N, -1)
             out = ext.paged_attention_decode_strided(rows, H, D, stride, kc, vc, bt, lens, 0.125)
             assert torch.equal(out, ref)
+
+
+# ----------------------------------------------------- fused layer, rotary
+
+def _train_model(name, **kw):
+    from distrl_llm_amd.models import CausalLM, get_spec
+    model = CausalLM(get_spec(name), lora_r=8, lora_alpha=16, dtype=torch.bfloat16,
+                     device=torch.device("cuda"), **kw).random_init(3)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    with torch.no_grad():
+        for n, p in model.named_parameters():
+            if n.endswith(("lora_B", "bias")):
+                p.copy_(torch.randn(p.shape, generator=g, device="cuda") * 0.05)
+            elif "norm" in n:
+                p.copy_(1 + 0.1 * torch.randn(p.shape, generator=g, device="cuda"))
+    return model.train()
+
+
+def _grads(model, ids, mask, dout):
+    out = model.forward_hidden(ids, mask)
+    params = [p for p in model.parameters() if p.requires_grad]
+    return [out.detach(), *torch.autograd.grad(out, params, dout)]
+
+
+@pytest.mark.parametrize("name", ["small-qwen2", "small-qwen3"])
+@pytest.mark.parametrize("B,T", [(1, 1), (2, 77), (3, 200)])
+def test_fused_layer_matches_modules(name, B, T):
+    """Hidden states and adapter gradients against the same model in fp64 on
+    the CPU: no further off than the module path (1.3 times leaves room for
+    other roundings of the same size), with padding at the ends."""
+    from distrl_llm_amd.models import CausalLM, fused_layer
+    model = _train_model(name)
+    g = torch.Generator().manual_seed(T)
+    ids = torch.randint(0, model.spec.vocab_size, (B, T), generator=g).cuda()
+    lens = torch.randint(max(1, T // 2), T + 1, (B,), generator=g)
+    mask = (torch.arange(T)[None] < lens[:, None]).long().cuda()
+    dout = _rand((B, T, model.spec.hidden_size), 9) * mask.unsqueeze(-1)
+    exact = CausalLM(model.spec, lora_r=8, lora_alpha=16, dtype=torch.float64)
+    exact.load_state_dict({k: v.double().cpu() for k, v in model.state_dict().items()})
+    ref = _grads(exact.train(), ids.cpu(), mask.cpu(), dout.double().cpu())
+    real = mask.bool().cpu()
+    fused = _grads(model, ids, mask, dout)
+    usable = fused_layer.usable
+    fused_layer.usable = lambda layer, x: False
+    try:
+        plain = _grads(model, ids, mask, dout)
+    finally:
+        fused_layer.usable = usable
+    fused, plain, ref = ([x.double().cpu() for x in xs] for xs in (fused, plain, ref))
+    fused[0], plain[0], ref[0] = (xs[0][real] for xs in (fused, plain, ref))
+    assert _rel(fused[0], ref[0]) < 1.3 * _rel(plain[0], ref[0]) + 2.0 ** -9
+    # the adapters' gradients together: one tensor's alone, from few tokens, is
+    # a single rounding or two of luck
+    fused, plain, ref = (torch.cat([x.reshape(-1) for x in xs[1:]]) for xs in (fused, plain, ref))
+    assert _rel(fused, ref) < 1.3 * _rel(plain, ref) + 2.0 ** -9
+
+
+def test_fused_layer_steps_aside():
+    """Hooks, dropout, inference and frozen shapes keep the modules."""
+    from distrl_llm_amd.models import fused_layer
+    model = _train_model("small-qwen2")
+    layer = model.model.layers[0]
+    x = _rand((1, 5, model.spec.hidden_size), 1)
+    assert fused_layer.usable(layer, x)
+    with torch.no_grad():
+        assert not fused_layer.usable(layer, x)
+    assert not fused_layer.usable(layer, x.float())
+    seen = []
+    handle = layer.mlp.up_proj.register_forward_hook(lambda m, i, o: seen.append(o))
+    model.forward_hidden(torch.zeros(1, 5, dtype=torch.long, device="cuda"))
+    assert len(seen) == 1
+    handle.remove()
+    assert fused_layer.usable(layer, x)
+    dropped = _train_model("small-qwen2", lora_dropout=0.1).model.layers[0]
+    assert not fused_layer.usable(dropped, x)
+    assert fused_layer.usable(dropped.eval(), x)
+
+
+@pytest.mark.parametrize("T,H,KV,D", [(1, 1, 1, 16), (5, 14, 2, 64), (9, 28, 4, 128), (7, 3, 1, 24),
+                                      (6, 4, 2, 48)])
+def test_rope_inplace_units(ext, T, H, KV, D):
+    """Vector and element rotation at odd head counts and sizes. Bound: one
+    bf16 rounding, and the fast sine's 2^-10 at these angles."""
+    q, k = _rand((T, H, D), 1), _rand((T, KV, D), 2)
+    pos = torch.randint(0, 3000, (T,), dtype=torch.int32, device="cuda")
+    inv = 1.0 / (1e4 ** (torch.arange(0, D, 2, device="cuda").float() / D))
+    a = (pos.double()[:, None] * inv.double())[:, None]
+    ref = []
+    for x in (q, k):
+        x1, x2 = x.double().chunk(2, -1)
+        ref.append(torch.cat([x1 * a.cos() - x2 * a.sin(), x2 * a.cos() + x1 * a.sin()], -1))
+    ext.rope_inplace(q, k, pos, inv)
+    assert _rel(q, ref[0]) < 2.0 ** -8 and _rel(k, ref[1]) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("rows,hidden", [(1, 8), (3, 896), (2, 2056)])
+def test_rmsnorm_bwd_add(ext, rows, hidden):
+    """One rounding of the sum instead of two."""
+    x, dy, g = (_rand((rows, hidden), i) for i in range(3))
+    w = _rand((hidden,), 4)
+    xr = x.double().requires_grad_()
+    y = xr * torch.rsqrt((xr * xr).mean(-1, keepdim=True) + 1e-6) * w.double()
+    ref = g.double() + torch.autograd.grad(y, xr, dy.double())[0]
+    assert _rel(ext.rmsnorm_bwd_add(dy, x, w, g, 1e-6), ref) < 2.0 ** -9
