@@ -10,8 +10,8 @@ sums accumulate inside the products (beta = 1, in place), the adapters of
 projections that share an input share one down product, and rotary, norm and
 activation passes are one kernel each: ~65 launches.
 
-A micro-batch of three short samples on a 24-layer 0.5B model: SHORT ms to
-SHORT2 ms; 16 x 1550 tokens on a 28-layer 1.5B model: ROUND to ROUND2 ms.
+A micro-batch of three short samples on a 24-layer 0.5B model: 58 ms to
+34 ms; 16 x 1550 tokens on a 28-layer 1.5B model: 380 to 239 ms.
 """
 
 from __future__ import annotations
