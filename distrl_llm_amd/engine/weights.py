@@ -35,7 +35,10 @@ class LayerWeights:
                  "gateup_w4", "gateup_amax", "down_w4", "down_amax",
                  "qkv_afrag", "qkv_bfrag", "o_afrag", "o_bfrag",
                  "gateup_afrag", "gateup_bfrag", "down_afrag", "down_bfrag",
-                 "qkv_r", "o_r", "gateup_r", "down_r")
+                 "qkv_r", "o_r", "gateup_r", "down_r",
+                 # the down site's bf16 base image and its adapter (rank
+                 # padded, scale folded into B) for steps of few sequences
+                 "down_base", "down_a", "down_b")
 
 
 def _effective(mod) -> torch.Tensor:
@@ -167,6 +170,14 @@ class FusedWeights:
                 setattr(lw, f"{name}_afrag", af)
                 setattr(lw, f"{name}_bfrag", bf)
             setattr(lw, f"{name}_r", r_pad)
+            if name == "down" and mods[0].weight.numel() > 0:
+                lw.down_base = mods[0].weight
+                if old_af is None:
+                    lw.down_a = A.to(torch.bfloat16).contiguous()
+                    lw.down_b = B.to(torch.bfloat16).contiguous()
+                else:
+                    lw.down_a.copy_(A)
+                    lw.down_b.copy_(B)
 
     @torch.no_grad()
     def refresh(self):

@@ -17,7 +17,9 @@ void rope_inplace(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
 void rope_scatter_qkv(torch::Tensor qkv, torch::Tensor positions,
                       torch::Tensor slots, torch::Tensor inv_freq,
                       torch::Tensor key_cache, torch::Tensor value_cache,
-                      int64_t H, int64_t KV, int64_t D);
+                      int64_t H, int64_t KV, int64_t D,
+                      c10::optional<torch::Tensor> q_norm,
+                      c10::optional<torch::Tensor> k_norm, double eps);
 torch::Tensor silu_mul_packed(torch::Tensor gu);
 torch::Tensor prefill_attention(torch::Tensor q, torch::Tensor k,
                                 torch::Tensor v, torch::Tensor tile_q0,
@@ -48,6 +50,13 @@ torch::Tensor nf4_gemm(torch::Tensor x, torch::Tensor w4f, torch::Tensor amaxf,
                        int64_t N, int64_t K, int64_t r);
 void lora_u(torch::Tensor x, torch::Tensor afrag, torch::Tensor u,
             int64_t r, int64_t ksplit);
+bool skinny_gemm_takes(int64_t M, int64_t N, int64_t K);
+torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
+                          c10::optional<torch::Tensor> bias,
+                          c10::optional<torch::Tensor> res,
+                          c10::optional<torch::Tensor> norm_w, double eps,
+                          c10::optional<torch::Tensor> u,
+                          c10::optional<torch::Tensor> ub);
 torch::Tensor mfma_probe(torch::Tensor a, torch::Tensor b);
 std::vector<torch::Tensor> flash_attn_fwd(torch::Tensor q, torch::Tensor k,
                                           torch::Tensor v, double scale);
@@ -74,7 +83,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_mul_bwd", &silu_mul_bwd, "fused SiLU*mul backward");
   m.def("rope_inplace", &rope_inplace, "fused in-place RoPE (q,k)");
   m.def("rope_scatter_qkv", &rope_scatter_qkv,
-        "fused packed-qkv RoPE + paged KV scatter");
+        "packed-qkv per-head norms (optional) + RoPE + paged KV scatter",
+        py::arg("qkv"), py::arg("positions"), py::arg("slots"),
+        py::arg("inv_freq"), py::arg("key_cache"), py::arg("value_cache"),
+        py::arg("H"), py::arg("KV"), py::arg("D"),
+        py::arg("q_norm") = py::none(), py::arg("k_norm") = py::none(),
+        py::arg("eps") = 0.0);
   m.def("silu_mul_packed", &silu_mul_packed, "SiLU*mul on packed [gate|up]");
   m.def("paged_attention_decode_strided", &paged_attention_decode_strided,
         "paged GQA decode attention (packed-q rows)");
@@ -94,6 +108,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("nf4_gemm", &nf4_gemm,
         "fused nf4-dequant MFMA GEMM with bias + LoRA-B epilogue");
   m.def("lora_u", &lora_u, "split-K LoRA A projection (u = x @ A^T)");
+  m.def("skinny_gemm_takes", &skinny_gemm_takes,
+        "whether skinny_gemm takes (M, N, K)");
+  m.def("skinny_gemm", &skinny_gemm,
+        "x W^T for few rows, with norm, bias, residual or SiLU*mul",
+        py::arg("x"), py::arg("w"), py::arg("mode"),
+        py::arg("bias") = py::none(), py::arg("res") = py::none(),
+        py::arg("norm_w") = py::none(), py::arg("eps") = 0.0,
+        py::arg("u") = py::none(), py::arg("ub") = py::none());
   m.def("mfma_probe", &mfma_probe, "16x16x32 bf16 MFMA mapping probe");
   m.def("flash_attn_fwd", &flash_attn_fwd,
         "causal GQA flash attention forward (returns o, lse)");

@@ -135,12 +135,85 @@ __global__ void rope_scatter_qkv_kernel(__hip_bfloat16* __restrict__ qkv,
   }
 }
 
+// The same for D 64 and 128 with 16 B accesses: 8 pairs a thread, so a head
+// takes D/16 neighbouring lanes, which also norm it (q_norm, k_norm: RMS norm
+// of each head before the rotation, rounded to bf16 in between as a separate
+// norm's output is; as torch operations it cost fourteen launches a layer).
+__global__ __launch_bounds__(256)
+void rope_scatter_vec_kernel(__hip_bfloat16* __restrict__ qkv, const int* __restrict__ positions,
+                             const int64_t* __restrict__ slots,
+                             const float* __restrict__ inv_freq,
+                             __hip_bfloat16* __restrict__ key_cache,
+                             __hip_bfloat16* __restrict__ value_cache,
+                             const __hip_bfloat16* __restrict__ q_norm,
+                             const __hip_bfloat16* __restrict__ k_norm, float eps, int H, int KV,
+                             int D) {
+  const int t = blockIdx.x, half = D / 2, per = half / 8;
+  const int64_t slot = slots[t];
+  const float pos = (float)positions[t];
+  __hip_bfloat16* base = qkv + (int64_t)t * (H + 2 * KV) * D;
+  const int c = threadIdx.x % per * 8;          // 256 % per == 0: fixed
+  float cs[8], sn[8];
+  #pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float a = pos * inv_freq[c + j];
+    sn[j] = __sinf(a);
+    cs[j] = __cosf(a);
+  }
+  const int rot = (H + KV) * per, all = rot + KV * D / 8;
+  // whole heads stay together: rot and the step are multiples of per
+  for (int u = threadIdx.x; u < all; u += 256) {
+    if (u >= rot) {                             // a value unit
+      const int i = u - rot;
+      if (slot >= 0)
+        reinterpret_cast<bf16x8*>(value_cache)[slot * (KV * D / 8) + i] =
+            reinterpret_cast<const bf16x8*>(base + (H + KV) * D)[i];
+      continue;
+    }
+    const int head = u / per;
+    __hip_bfloat16* p = base + head * D + c;
+    const bf16x8 a = *reinterpret_cast<const bf16x8*>(p);
+    const bf16x8 b = *reinterpret_cast<const bf16x8*>(p + half);
+    float x1[8], x2[8];
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) { x1[j] = bf2f(a.v[j]); x2[j] = bf2f(b.v[j]); }
+    const __hip_bfloat16* nw = head < H ? q_norm : k_norm;
+    if (nw) {
+      float ss = 0.f;
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) ss += x1[j] * x1[j] + x2[j] * x2[j];
+      for (int off = per / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, WAVE);
+      const float r = rsqrtf(ss / D + eps);
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        x1[j] = bf2f(f2bf(x1[j] * r * bf2f(nw[c + j])));
+        x2[j] = bf2f(f2bf(x2[j] * r * bf2f(nw[c + half + j])));
+      }
+    }
+    bf16x8 x, y;
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      x.v[j] = f2bf(x1[j] * cs[j] - x2[j] * sn[j]);
+      y.v[j] = f2bf(x2[j] * cs[j] + x1[j] * sn[j]);
+    }
+    *reinterpret_cast<bf16x8*>(p) = x;
+    *reinterpret_cast<bf16x8*>(p + half) = y;
+    if (head >= H && slot >= 0) {
+      __hip_bfloat16* kd = key_cache + (slot * KV + head - H) * D + c;
+      *reinterpret_cast<bf16x8*>(kd) = x;
+      *reinterpret_cast<bf16x8*>(kd + half) = y;
+    }
+  }
+}
+
 }  // namespace
 
 void rope_scatter_qkv(torch::Tensor qkv, torch::Tensor positions,
                       torch::Tensor slots, torch::Tensor inv_freq,
                       torch::Tensor key_cache, torch::Tensor value_cache,
-                      int64_t H, int64_t KV, int64_t D) {
+                      int64_t H, int64_t KV, int64_t D,
+                      c10::optional<torch::Tensor> q_norm,
+                      c10::optional<torch::Tensor> k_norm, double eps) {
   TORCH_CHECK(qkv.is_cuda() && qkv.is_contiguous());
   TORCH_CHECK(qkv.scalar_type() == at::kBFloat16);
   TORCH_CHECK(positions.scalar_type() == at::kInt);
@@ -148,7 +221,28 @@ void rope_scatter_qkv(torch::Tensor qkv, torch::Tensor positions,
   const int T = qkv.size(0);
   TORCH_CHECK(qkv.size(1) == (H + 2 * KV) * D);
   TORCH_CHECK((KV * D) % 8 == 0);
+  auto norm = [&](const c10::optional<torch::Tensor>& w) {
+    if (!w) return (const __hip_bfloat16*)nullptr;
+    TORCH_CHECK(w->is_cuda() && w->is_contiguous() && w->scalar_type() == at::kBFloat16 &&
+                w->numel() == D, "rope_scatter_qkv: head norm weight");
+    return reinterpret_cast<const __hip_bfloat16*>(w->data_ptr());
+  };
+  const auto *qn = norm(q_norm), *kn = norm(k_norm);
+  const bool vec = (D == 64 || D == 128) && reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0;
+  TORCH_CHECK(vec || (!qn && !kn), "rope_scatter_qkv: head norms need head_dim 64 or 128");
   if (T == 0) return;
+  if (vec) {
+    hipLaunchKernelGGL(rope_scatter_vec_kernel, dim3(T), dim3(256), 0,
+                       at::cuda::getCurrentCUDAStream(),
+                       reinterpret_cast<__hip_bfloat16*>(qkv.data_ptr()),
+                       positions.data_ptr<int>(), slots.data_ptr<int64_t>(),
+                       inv_freq.data_ptr<float>(),
+                       reinterpret_cast<__hip_bfloat16*>(key_cache.data_ptr()),
+                       reinterpret_cast<__hip_bfloat16*>(value_cache.data_ptr()), qn, kn,
+                       (float)eps, (int)H, (int)KV, (int)D);
+    HIP_CHECK_LAST();
+    return;
+  }
   const int smem = D * sizeof(float);
   hipLaunchKernelGGL(rope_scatter_qkv_kernel, dim3(T), dim3(256), smem,
                      at::cuda::getCurrentCUDAStream(),

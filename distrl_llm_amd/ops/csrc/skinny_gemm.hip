@@ -1,0 +1,249 @@
+// Products of a decode step with few rows: y = x W^T for M <= 64 rows,
+// W (N, K) bf16, fp32 sums, with what stands around the product in the same
+// launch: the RMS norm of x before it; bias, residual sum or SiLU*mul after it.
+//
+// Such a product only streams W. A workgroup owns 16 rows of W (for SiLU*mul 16
+// gate rows and their 16 up rows) and its waves split K, so that small matrices
+// spread over the chip (few rows of W: 8 a workgroup); a wave has up to ten steps of its share of W and x in
+// flight, straight into MFMA operands (16x16x32: lane = row, 16 B pieces).
+// Partial sums meet in LDS. The norm needs no pass of its own: the waves
+// multiply x by the norm weight as they read it and sum its squares on the way,
+// 1/rms scales the finished row.
+// A step of a few sequences is bound by its launches' latency (~4 us each) as
+// much as by bytes, hence the fusions: on the 0.5B model at 8 rows a layer took
+// 67 us in 11 launches, 39 in 7 now (gate|up + SiLU 17 + 5 -> 11.6 us, down and
+// output 8.3 and 6.8 -> 8.8 and 4.6 with the residual sum, qkv 6.8 -> 4.9; the two
+// norms' 4.8 each are in them).
+#include <torch/extension.h>
+#include <ATen/cuda/CUDAContext.h>
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16v8;
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16v4;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+namespace {
+
+enum { PLAIN = 0, RESIDUAL = 1, GLU = 2 };
+
+// Steps of K a wave has in flight: what its registers hold.
+template <int MT, int KW, int ACC, bool NORM>
+constexpr int in_flight() {
+  const int n = 96 / (4 * (ACC + MT + (NORM ? 1 : 0)));
+  return n > 10 ? 10 : n;
+}
+
+template <int MT, int KW, int MODE, bool NORM>
+__global__ __launch_bounds__(KW * 64)
+void skinny_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat16* __restrict__ w,
+                        const __hip_bfloat16* __restrict__ bias,
+                        const __hip_bfloat16* __restrict__ res,
+                        const __hip_bfloat16* __restrict__ norm_w,
+                        const __hip_bfloat16* __restrict__ u,    // (M, R): y += u ub^T
+                        const __hip_bfloat16* __restrict__ ub,   // (N, R)
+                        __hip_bfloat16* __restrict__ y, int M, int N, int K, int R, int tr, float eps) {
+  constexpr int ACC = MODE == GLU ? 2 : 1, U = in_flight<MT, KW, ACC, NORM>();
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  f32x4* red = reinterpret_cast<f32x4*>(smem);            // [KW][ACC][MT][64]
+  __shared__ float squares[NORM ? KW * MT * 16 : 1];      // of x, [KW][MT][16 rows]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l = threadIdx.x & 63, g = l >> 4, lr = l & 15;
+  const int n0 = blockIdx.x * tr, wr = min(lr, tr - 1);   // spare rows repeat
+  const int steps = K / 32, s0 = wave * steps / KW, s1 = (wave + 1) * steps / KW;
+
+  const __hip_bfloat16* wp[ACC];
+  #pragma unroll
+  for (int a = 0; a < ACC; ++a) wp[a] = w + (int64_t)(n0 + a * N + wr) * K + g * 8;
+  f32x4 acc[ACC][MT];
+  #pragma unroll
+  for (int a = 0; a < ACC; ++a)
+    #pragma unroll
+    for (int t = 0; t < MT; ++t) acc[a][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int row[MT];
+  float ss[MT];
+  #pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    row[t] = min(t * 16 + lr, M - 1);                     // spare rows repeat
+    ss[t] = 0.f;
+  }
+
+  for (int s = s0; s < s1; s += U) {
+    bf16v8 wf[U][ACC], xf[U][MT], nf[U];
+    #pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int k = min(s + i, s1 - 1) * 32;              // past the end: the last again
+      #pragma unroll
+      for (int a = 0; a < ACC; ++a) wf[i][a] = *reinterpret_cast<const bf16v8*>(wp[a] + k);
+      #pragma unroll
+      for (int t = 0; t < MT; ++t)
+        xf[i][t] = *reinterpret_cast<const bf16v8*>(x + (int64_t)row[t] * K + k + g * 8);
+      if (NORM) nf[i] = *reinterpret_cast<const bf16v8*>(norm_w + k + g * 8);
+    }
+    #pragma unroll
+    for (int i = 0; i < U; ++i)
+      if (s + i < s1) {                                   // wave-uniform
+        #pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          if (NORM) {
+            #pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float v = (float)xf[i][t][j];
+              ss[t] += v * v;
+              xf[i][t][j] = (__bf16)(v * (float)nf[i][j]);
+            }
+          }
+          #pragma unroll
+          for (int a = 0; a < ACC; ++a)
+            acc[a][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i][a], xf[i][t], acc[a][t],
+                                                                0, 0, 0);
+        }
+      }
+  }
+  if (NORM) {
+    #pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      ss[t] += __shfl_xor(ss[t], 16, WAVE);
+      ss[t] += __shfl_xor(ss[t], 32, WAVE);
+      if (g == 0) squares[(wave * MT + t) * 16 + lr] = ss[t];
+    }
+  }
+  if (MODE == RESIDUAL && wave == 0) {      // an adapter: more of K, elsewhere
+    for (int k = g * 8; k < R; k += 32) {
+      const bf16v8 b = *reinterpret_cast<const bf16v8*>(ub + (int64_t)(n0 + wr) * R + k);
+      #pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            b, *reinterpret_cast<const bf16v8*>(u + (int64_t)row[t] * R + k), acc[0][t], 0, 0, 0);
+    }
+  }
+
+  #pragma unroll
+  for (int a = 0; a < ACC; ++a)
+    #pragma unroll
+    for (int t = 0; t < MT; ++t) red[((wave * ACC + a) * MT + t) * 64 + l] = acc[a][t];
+  __syncthreads();
+  // lane of tile t: row m = 16 t + lr of x, columns n0 + 4 g + 0..3
+  for (int t = wave; t < MT; t += KW) {
+    const int m = t * 16 + lr, n = n0 + g * 4;
+    f32x4 sum[ACC];
+    #pragma unroll
+    for (int a = 0; a < ACC; ++a) {
+      sum[a] = red[(a * MT + t) * 64 + l];
+      #pragma unroll
+      for (int v = 1; v < KW; ++v) sum[a] += red[((v * ACC + a) * MT + t) * 64 + l];
+    }
+    if (NORM) {
+      float sq = 0.f;
+      #pragma unroll
+      for (int v = 0; v < KW; ++v) sq += squares[(v * MT + t) * 16 + lr];
+      const float r = rsqrtf(sq / K + eps);
+      #pragma unroll
+      for (int a = 0; a < ACC; ++a) sum[a] *= r;
+    }
+    if (m >= M || g * 4 >= tr) continue;
+    const int64_t at = (int64_t)m * N + n;
+    bf16v4 o;
+    if (MODE == GLU) {
+      #pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        // gate and up round as the separate product's output does
+        const float gt = (float)(__bf16)sum[0][r], up = (float)(__bf16)sum[ACC - 1][r];
+        o[r] = (__bf16)(gt / (1.f + __expf(-gt)) * up);
+      }
+    } else {
+      bf16v4 add;
+      if (MODE == RESIDUAL) add = *reinterpret_cast<const bf16v4*>(res + at);
+      else if (bias) add = *reinterpret_cast<const bf16v4*>(bias + n);
+      #pragma unroll
+      for (int r = 0; r < 4; ++r)
+        o[r] = (__bf16)(MODE == RESIDUAL || bias ? sum[0][r] + (float)add[r] : sum[0][r]);
+    }
+    *reinterpret_cast<bf16v4*>(y + at) = o;
+  }
+}
+
+bool aligned16(const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+const __hip_bfloat16* ptr(const torch::Tensor& t) {
+  return reinterpret_cast<const __hip_bfloat16*>(t.data_ptr());
+}
+
+}  // namespace
+
+// Whether skinny_gemm takes the shape: rows of x, columns of y (the activation's
+// for SiLU*mul), K.
+bool skinny_gemm_takes(int64_t M, int64_t N, int64_t K) {
+  return M >= 1 && M <= 64 && N >= 16 && N % 16 == 0 && K >= 512 && K % 32 == 0;
+}
+
+// mode 0: x W^T (+ bias); 1: res + x W^T (+ u ub^T); 2: silu(x Wg^T) * (x Wu^T)
+// with w = [Wg; Wu]. norm_w: x is RMS-normed first.
+torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
+                          c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> res,
+                          c10::optional<torch::Tensor> norm_w, double eps,
+                          c10::optional<torch::Tensor> u, c10::optional<torch::Tensor> ub) {
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() && aligned16(x));
+  TORCH_CHECK(w.is_cuda() && w.dim() == 2 && w.is_contiguous() && aligned16(w));
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16);
+  TORCH_CHECK(mode >= PLAIN && mode <= GLU && w.size(1) == x.size(1));
+  const int M = x.size(0), K = x.size(1), N = mode == GLU ? w.size(0) / 2 : w.size(0);
+  TORCH_CHECK(mode != GLU || w.size(0) % 2 == 0);
+  TORCH_CHECK(skinny_gemm_takes(M, N, K), "skinny_gemm: unsupported shape (", M, ", ", N, ", ", K, ")");
+  auto check = [&](const c10::optional<torch::Tensor>& t, int64_t n, const char* what) {
+    if (!t) return (const __hip_bfloat16*)nullptr;
+    TORCH_CHECK(t->is_cuda() && t->is_contiguous() && t->scalar_type() == at::kBFloat16 &&
+                t->numel() == n && aligned16(*t), "skinny_gemm: ", what);
+    return ptr(*t);
+  };
+  const auto* b = check(bias, N, "bias");
+  const auto* r = check(res, (int64_t)M * N, "residual");
+  const auto* nw = check(norm_w, K, "norm weight");
+  const int R = u ? (int)u->size(-1) : 0;
+  TORCH_CHECK(u.has_value() == ub.has_value() && (!u || (mode == RESIDUAL && R % 32 == 0)),
+              "skinny_gemm: adapter");
+  const auto* up = check(u, (int64_t)M * R, "adapter input");
+  const auto* ubp = check(ub, (int64_t)N * R, "adapter weight");
+  TORCH_CHECK((mode == RESIDUAL) == (r != nullptr) && (b == nullptr || mode == PLAIN));
+  auto y = torch::empty({M, N}, x.options());
+  auto* o = reinterpret_cast<__hip_bfloat16*>(y.data_ptr());
+  auto stream = at::cuda::getCurrentCUDAStream();
+  // Rows of W a workgroup takes and waves that share its K, from sweeps of both
+  // at 8 rows and cold weights (us; rows/waves): N 896, K 4864: 16/4 11.8,
+  // 16/16 10.6, 8/16 8.6, 4/16 7.8; N 1536, K 8960: 19.4, 19.6, 15.3, 24.0;
+  // N 2560, K 9728: 22.7, 20.3, 28.0; N 1152, K 896: 4.6 (8/4 4.3, 8/16 8.0);
+  // N 1536, K 1536: 7.1 (8/4 6.3, 8/8 5.7); SiLU*mul of N 8960, K 1536: 16/4
+  // 20.6, 16/8 18.1; N 9728, K 2560: 36, 33; N 4864, K 896: 11.4, 11.5.
+  // Fewer rows a workgroup reach more CUs but re-read x; more waves shorten
+  // the chain of loads until joining them costs more.
+  const int tiles = N / 16, steps = K / 32, tr = tiles <= 128 ? 8 : 16;
+  int kw = tiles <= 256 ? (steps >= 64 ? 16 : steps >= 32 ? 8 : 4)
+                        : (mode == GLU && steps >= 48 ? 8 : 4);
+  if (mode == GLU && M > 32) kw = std::min(kw, 8);     // 64 KB of partial sums
+  auto go = [&](auto mt_, auto kw_, auto mode_, auto norm_) {
+    constexpr int MT = decltype(mt_)::value, KW = decltype(kw_)::value,
+                  MODE = decltype(mode_)::value;
+    constexpr bool NORM = decltype(norm_)::value;
+    const size_t smem = KW * (MODE == GLU ? 2 : 1) * MT * 64 * 16;
+    hipLaunchKernelGGL((skinny_gemm_kernel<MT, KW, MODE, NORM>), dim3(N / tr), dim3(KW * 64), smem,
+                       stream, ptr(x), ptr(w), b, r, nw, up, ubp, o, M, N, K, R, tr, (float)eps);
+  };
+  auto by_norm = [&](auto mt_, auto kw_, auto mode_) {
+    if (nw) go(mt_, kw_, mode_, std::true_type{}); else go(mt_, kw_, mode_, std::false_type{});
+  };
+  auto by_mode = [&](auto mt_, auto kw_) {
+    if (mode == PLAIN) by_norm(mt_, kw_, std::integral_constant<int, PLAIN>{});
+    else if (mode == RESIDUAL) go(mt_, kw_, std::integral_constant<int, RESIDUAL>{}, std::false_type{});
+    else by_norm(mt_, kw_, std::integral_constant<int, GLU>{});
+  };
+  auto by_kw = [&](auto mt_) {
+    if (kw == 16) by_mode(mt_, std::integral_constant<int, 16>{});
+    else if (kw == 8) by_mode(mt_, std::integral_constant<int, 8>{});
+    else by_mode(mt_, std::integral_constant<int, 4>{});
+  };
+  TORCH_CHECK(mode != RESIDUAL || !nw, "skinny_gemm: norm with a residual sum");
+  if (M <= 16) by_kw(std::integral_constant<int, 1>{});
+  else if (M <= 32) by_kw(std::integral_constant<int, 2>{});
+  else by_kw(std::integral_constant<int, 4>{});
+  HIP_CHECK_LAST();
+  return y;
+}

@@ -354,3 +354,55 @@ def test_rmsnorm_bwd_add(ext, rows, hidden):
     y = xr * torch.rsqrt((xr * xr).mean(-1, keepdim=True) + 1e-6) * w.double()
     ref = g.double() + torch.autograd.grad(y, xr, dy.double())[0]
     assert _rel(ext.rmsnorm_bwd_add(dy, x, w, g, 1e-6), ref) < 2.0 ** -9
+
+
+# ------------------------------------------------------------ skinny products
+
+@pytest.mark.parametrize("M", [1, 8, 15, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(16, 512), (896, 896), (2064, 544), (4112, 4864), (256, 8960)])
+def test_skinny_gemm(ext, M, N, K):
+    """Every wave count and row tile, K that does not divide among the waves;
+    bias, residual with an adapter, SiLU*mul, with and without the norm.
+    Bounds: one rounding of the result (2^-9) over fp32 sums; the norm rounds
+    its output first, SiLU*mul its two inputs."""
+    x, w, b = _rand((M, K), 1), _rand((2 * N, K), 2, K ** -0.5), _rand((N,), 3)
+    res, u, ub = _rand((M, N), 4), _rand((M, 64), 5), _rand((N, 64), 6, 0.1)
+    nw = _rand((K,), 7, 0.1) + 1
+    xd, wd = x.double(), w[:N].contiguous()
+    assert _rel(ext.skinny_gemm(x, wd, 0), xd @ wd.double().t()) < 2.0 ** -8
+    assert _rel(ext.skinny_gemm(x, wd, 0, b), xd @ wd.double().t() + b.double()) < 2.0 ** -8
+    ref = res.double() + xd @ wd.double().t()
+    assert _rel(ext.skinny_gemm(x, wd, 1, res=res), ref) < 2.0 ** -8
+    assert _rel(ext.skinny_gemm(x, wd, 1, res=res, u=u, ub=ub),
+                ref + u.double() @ ub.double().t()) < 2.0 ** -8
+    normed = xd * torch.rsqrt((xd * xd).mean(-1, keepdim=True) + 1e-6) * nw.double()
+    for inp, kw, bound in ((xd, {}, 2.0 ** -7), (normed, {"norm_w": nw, "eps": 1e-6}, 2.0 ** -6)):
+        gate, up = (inp @ w.double().t()).chunk(2, -1)
+        assert _rel(ext.skinny_gemm(x, w, 2, **kw), torch.nn.functional.silu(gate) * up) < bound
+        assert _rel(ext.skinny_gemm(x, wd, 0, b, **kw),
+                    inp @ wd.double().t() + b.double()) < bound
+
+
+@pytest.mark.parametrize("D,H,KV", [(64, 3, 1), (128, 28, 4)])
+def test_rope_scatter_norms(ext, D, H, KV):
+    """Per-head norms, rotation and cache write of packed projections, a
+    skipped slot among them, against the separate kernels."""
+    T = 5
+    qkv, wq, wk = _rand((T, (H + 2 * KV) * D), 1), _rand((D,), 2, 0.1) + 1, _rand((D,), 3, 0.1) + 1
+    pos = torch.randint(0, 2000, (T,), dtype=torch.int32, device="cuda")
+    slots = torch.tensor([3, -1, 40, 0, 17], device="cuda")
+    inv = 1.0 / (1e4 ** (torch.arange(0, D, 2, device="cuda").float() / D))
+    for norms in ((), (wq, wk, 1e-6)):
+        q, k, v = (t.reshape(T, -1, D).contiguous()
+                   for t in qkv.split([H * D, KV * D, KV * D], 1))
+        if norms:
+            q, k = ext.rmsnorm_fwd(q, wq, 1e-6), ext.rmsnorm_fwd(k, wk, 1e-6)
+        ext.rope_inplace(q, k, pos, inv)
+        kc, vc = torch.zeros(2, 3, 16, KV, D, dtype=torch.bfloat16, device="cuda")
+        ext.kv_cache_scatter(k, v, kc, vc, slots.int())
+        packed, kc2, vc2 = qkv.clone(), torch.zeros_like(kc), torch.zeros_like(vc)
+        ext.rope_scatter_qkv(packed, pos, slots, inv, kc2, vc2, H, KV, D, *norms)
+        # norm sums in another order: the last bit may differ
+        assert _rel(packed[:, :H * D].reshape(q.shape), q) < 2.0 ** -9
+        assert _rel(kc2, kc) < 2.0 ** -9
+        assert torch.equal(vc2, vc)
