@@ -245,7 +245,12 @@ class Engine:
                                     + p % self.pool.block_size)
             q.context_len = L
         slot_mapping = torch.tensor(slot_mapping, dtype=torch.long, device=device)
+        last_idx = torch.tensor([sum(lens[:i + 1]) - 1 for i in range(len(lens))],
+                                dtype=torch.long, device=device)
 
+        if self._prefill_packs():
+            x = self._prefill_packed(input_ids, positions, slot_mapping, lens)
+            return self.model.logits(x[last_idx])
         x = self.model.model.embed_tokens(input_ids)
         for li, layer in enumerate(self.model.model.layers):
             h = layer.input_layernorm(x)
@@ -265,10 +270,71 @@ class Engine:
             u = self._proj(layer.mlp.up_proj, h2)
             x = x + self._proj(layer.mlp.down_proj, OF.silu_mul(g, u))
         x = self.model.model.norm(x)
-
-        last_idx = torch.tensor([sum(lens[:i + 1]) - 1 for i in range(len(lens))],
-                                dtype=torch.long, device=device)
         return self.model.logits(x[last_idx])
+
+    def _prefill_packs(self) -> bool:
+        """Whether the prompt phase can run on packed rows: bf16 on the GPU,
+        bf16 base weights at hand, sizes the packed kernels take."""
+        f, s = self.fused, self.spec
+        return (self.device.type == "cuda" and self.dtype == torch.bfloat16
+                and f is not None and f._built and not f.nf4
+                and s.head_dim in (64, 128)
+                and os.environ.get("DISTRL_PREFILL_VARLEN") != "1")
+
+    def _prefill_packed(self, input_ids, positions, slots, lens):
+        """The layers over one flat batch of prompts -> normed hidden states.
+        Projections go into packed rows, [q|k|v] and [gate|up], which the
+        rotary + cache, attention (row offsets instead of padding) and
+        activation kernels read as they lie. Adapters stay beside the base
+        weights here (a merged weight would round small ones away); without
+        any, the packed decode weights are the base weights."""
+        from ..ops.functional import _require_ext
+        ext, s, m = _require_ext("prefill"), self.spec, self.model
+        qs, kvs, eps = s.q_size, s.kv_size, s.rms_norm_eps
+        T, H, KV, D = input_ids.shape[0], s.num_heads, s.num_kv_heads, s.head_dim
+        pos32 = positions.to(torch.int32)
+        cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0) \
+            .to(torch.int32).to(self.device)
+
+        def packed(x, mods, merged, bias):
+            if all(mod.r == 0 for mod in mods):
+                return F.linear(x, merged, bias)
+            out = x.new_empty(T, sum(mod.out_features for mod in mods))
+            for mod, y in zip(mods, out.split([mod.out_features
+                                               for mod in mods], 1)):
+                if mod.bias is None:
+                    torch.mm(x, mod.weight.t(), out=y)
+                else:
+                    torch.addmm(mod.bias, x, mod.weight.t(), out=y)
+                if mod.r > 0:
+                    y.addmm_(x @ mod.lora_A.t(), mod.lora_B.t(),
+                             alpha=mod.scale)
+            return out
+
+        res = m.model.embed_tokens(input_ids)
+        h = ext.rmsnorm_fwd(res, self.fused.layers[0].in_norm, eps)
+        for li, (layer, lw) in enumerate(zip(m.model.layers,
+                                             self.fused.layers)):
+            at, mlp = layer.self_attn, layer.mlp
+            qkv = packed(h, (at.q_proj, at.k_proj, at.v_proj), lw.qkv_w,
+                         lw.qkv_b)
+            norms = ((at.q_norm.weight, at.k_norm.weight, eps)
+                     if s.qk_norm else ())
+            ext.rope_scatter_qkv(qkv, pos32, slots, self._inv_freq,
+                                 self.pool.key[li], self.pool.value[li],
+                                 H, KV, D, *norms)
+            q, k, v = (t.unflatten(1, (-1, D))
+                       for t in qkv.split([qs, kvs, kvs], 1))
+            o = ext.flash_attn_varlen(q, k, v, cu, max(lens), self.scale)
+            o = self._proj(at.o_proj, o.view(T, qs))
+            h, res = ext.add_rmsnorm_fwd(res, o, lw.post_norm, eps)
+            gu = packed(h, (mlp.gate_proj, mlp.up_proj), lw.gateup_w, None)
+            d = self._proj(mlp.down_proj, ext.silu_mul_packed(gu))
+            last = li + 1 == len(self.fused.layers)
+            h, res = ext.add_rmsnorm_fwd(
+                res, d, m.model.norm.weight if last
+                else self.fused.layers[li + 1].in_norm, eps)
+        return h
 
     def _qk_norm(self, at, q, k):
         """Qwen3 per-head q/k RMSNorm over head_dim, applied before RoPE

@@ -49,6 +49,19 @@ def _effective(mod) -> torch.Tensor:
     return w
 
 
+def _merge_into(mod, out: torch.Tensor) -> None:
+    """out <- the module's effective weight."""
+    if mod.r > 0 and out.is_cuda and out.dtype == torch.bfloat16 \
+            and mod.lora_A.dtype == out.dtype == mod.weight.dtype:
+        from ..ops.functional import _require_ext
+        ext = _require_ext("lora_merge")
+        if ext is not None and ext.lora_merge_takes(mod.in_features, mod.r):
+            ext.lora_merge(mod.weight.detach(), mod.lora_A.detach(),
+                           mod.lora_B.detach(), out, float(mod.scale))
+            return
+    out.copy_(_effective(mod))
+
+
 class FusedWeights:
     def __init__(self, model, use_nf4: bool = True):
         self.model = model
@@ -222,19 +235,17 @@ class FusedWeights:
 
     def _refresh_merged(self, lw: "LayerWeights", layer, first: bool):
         at, mlp = layer.self_attn, layer.mlp
-        qkv = torch.cat([_effective(at.q_proj), _effective(at.k_proj),
-                         _effective(at.v_proj)], dim=0).contiguous()
-        gateup = torch.cat([_effective(mlp.gate_proj),
-                            _effective(mlp.up_proj)], dim=0).contiguous()
-        o_w = _effective(at.o_proj).contiguous()
-        down_w = _effective(mlp.down_proj).contiguous()
-        if first:
-            lw.qkv_w = qkv
-            lw.gateup_w = gateup
-            lw.o_w = o_w
-            lw.down_w = down_w
-        else:
-            lw.qkv_w.copy_(qkv)
-            lw.gateup_w.copy_(gateup)
-            lw.o_w.copy_(o_w)
-            lw.down_w.copy_(down_w)
+        for name, mods in (("qkv_w", [at.q_proj, at.k_proj, at.v_proj]),
+                           ("gateup_w", [mlp.gate_proj, mlp.up_proj]),
+                           ("o_w", [at.o_proj]), ("down_w", [mlp.down_proj])):
+            if first:
+                m = mods[0]
+                if len(mods) == 1 and m.r == 0:
+                    setattr(lw, name, m.weight.contiguous())
+                else:
+                    setattr(lw, name, m.weight.new_empty(
+                        sum(m.out_features for m in mods), m.in_features))
+            # IN PLACE: captured decode steps hold these storages
+            rows = getattr(lw, name).split([m.out_features for m in mods])
+            for m, out in zip(mods, rows):
+                _merge_into(m, out)

@@ -406,3 +406,55 @@ def test_rope_scatter_norms(ext, D, H, KV):
         assert _rel(packed[:, :H * D].reshape(q.shape), q) < 2.0 ** -9
         assert _rel(kc2, kc) < 2.0 ** -9
         assert torch.equal(vc2, vc)
+
+
+# ---------------------------------------------- merged weights, prompt phase
+
+@pytest.mark.parametrize("N,K,r", [(1, 32, 8), (17, 288, 8), (130, 256, 32), (128, 1056, 40),
+                                   (70, 544, 128)])
+def test_lora_merge(ext, N, K, r):
+    """Row and column remainders, ranks that do not fill a product step. One
+    rounding of an fp32 sum."""
+    w, a, b = _rand((N, K), 1), _rand((r, K), 2, 0.3), _rand((N, r), 3, 0.3)
+    out = torch.full((N + 1, K), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ext.lora_merge(w, a, b, out[:N], 0.5)
+    assert _rel(out[:N], w.double() + 0.5 * b.double() @ a.double()) < 2.0 ** -9
+    assert bool(out[N].isnan().all())
+
+
+@pytest.mark.parametrize("name", ["small-qwen2", "small-qwen3"])
+@pytest.mark.parametrize("lora_r,four_bit", [(0, False), (8, False), (8, True), (12, False)])
+def test_packed_prefill_matches_modules(name, lora_r, four_bit):
+    """Logits and cache rows of a ragged batch against the module path (two
+    bf16 paths of the same products: 2 %), and the merged weights against
+    W + scale * B A at a rank the kernel takes and one it does not."""
+    from distrl_llm_amd.config import EngineConfig
+    from distrl_llm_amd.engine import Engine
+    from distrl_llm_amd.engine.kvcache import Sequence
+    from distrl_llm_amd.models import CausalLM, get_spec
+    model = CausalLM(get_spec(name), lora_r=lora_r, lora_alpha=16, dtype=torch.bfloat16,
+                     device=torch.device("cuda")).random_init(3).eval()
+    with torch.no_grad():
+        for n, p in model.named_parameters():
+            if n.endswith(("lora_B", "bias")):
+                p.copy_(_rand(p.shape, 7, 0.05))
+    if four_bit:
+        model.quantize_nf4_()
+    g = torch.Generator().manual_seed(1)
+    prompts = [torch.randint(0, 4096, (n,), generator=g).tolist() for n in (3, 64, 129, 1)]
+    got = []
+    for packs in (True, False):
+        eng = Engine(model, EngineConfig(max_seq_length=256, num_kv_blocks=32, max_num_seqs=8))
+        eng.fused.refresh()
+        if not packs:
+            eng._prefill_packs = lambda: False
+        logits = eng._prefill_batch([Sequence(i, p, i) for i, p in enumerate(prompts)])
+        got.append((logits, eng.pool.key, eng.pool.value))
+    for x, y in zip(*got):
+        assert _rel(x, y) < 0.02
+    at = model.model.layers[1].self_attn
+    w = at.k_proj.weight.double()
+    if lora_r:
+        w = w + at.k_proj.scale * at.k_proj.lora_B.double() @ at.k_proj.lora_A.double()
+    q = model.spec.q_size
+    assert _rel(eng.fused.layers[1].qkv_w[q:q + model.spec.kv_size], w) < 2.0 ** -8
