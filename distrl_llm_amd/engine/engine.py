@@ -549,8 +549,10 @@ class Engine:
             if r > 0:
                 o0, rt = site_off[site]
                 u = u_pool[li, :, o0:o0 + rt]
-                ksplit = max(1, min(8, 512 // max(1, ((N_batch + 15) // 16)
-                                                 * (rt // 16))))
+                # a thousand waves, none under eight steps: with eight splits
+                # a wave of the deep-K site walked 74 steps in turn (32 us)
+                tiles = (N_batch + 15) // 16 * (rt // 16)
+                ksplit = max(1, min(K_in // 256, 1024 // tiles))
                 ext.lora_u(x, getattr(lw, f"{site}_afrag"), u, rt, ksplit)
                 return ext.nf4_gemm(x, getattr(lw, f"{site}_w4"),
                                     getattr(lw, f"{site}_amax"), bias, u,

@@ -391,31 +391,23 @@ void lora_u_kernel(const __hip_bfloat16* __restrict__ x,   // (M, K)
 
   const int m = mt * 16 + lrow;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  // software-pipelined 2-deep: issue next k-steps' fragments while the
-  // current MFMA runs (the bare loop serializes on load latency)
-  auto load_af = [&](int kstep, bf16v8& af, uint4& bw) {
-    if (m < M) {
-      af = *reinterpret_cast<const bf16v8*>(
-          x + (int64_t)m * K + kstep * 32 + lk * 8);
-    } else {
-      #pragma unroll
-      for (int j = 0; j < 8; ++j) af[j] = (__bf16)0.f;
+  // eight steps' fragments in flight; rows past M repeat the last one and are
+  // not written
+  constexpr int U = 8;
+  const __hip_bfloat16* xr = x + (int64_t)min(m, M - 1) * K + lk * 8;
+  const uint32_t* ar = afrag + (int64_t)rt * ksteps * 64 * 4 + l * 4;
+  for (int s = k0; s < k1; s += U) {
+    bf16v8 af[U], bw[U];
+    #pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int k = min(s + i, k1 - 1);
+      af[i] = *reinterpret_cast<const bf16v8*>(xr + k * 32);
+      bw[i] = *reinterpret_cast<const bf16v8*>(ar + (int64_t)k * 64 * 4);
     }
-    bw = *reinterpret_cast<const uint4*>(
-        afrag + ((int64_t)rt * ksteps + kstep) * 64 * 4 + l * 4);
-  };
-  bf16v8 af_c, af_n;
-  uint4 bw_c, bw_n;
-  if (k0 < k1) load_af(k0, af_c, bw_c);
-  if (k0 + 1 < k1) load_af(k0 + 1, af_n, bw_n);
-  for (int kstep = k0; kstep < k1; ++kstep) {
-    bf16v8 af_f;
-    uint4 bw_f;
-    if (kstep + 2 < k1) load_af(kstep + 2, af_f, bw_f);
-    const bf16v8 bf = *reinterpret_cast<const bf16v8*>(&bw_c);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af_c, bf, acc, 0, 0, 0);
-    af_c = af_n; bw_c = bw_n;
-    af_n = af_f; bw_n = bw_f;
+    #pragma unroll
+    for (int i = 0; i < U; ++i)
+      if (s + i < k1)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bw[i], acc, 0, 0, 0);
   }
   #pragma unroll
   for (int rr = 0; rr < 4; ++rr) {
