@@ -41,8 +41,13 @@ torch::Tensor sample_tokens(torch::Tensor logits, double temperature,
                             torch::Tensor step);
 std::vector<torch::Tensor> logprob_lse_fwd(torch::Tensor logits,
                                            torch::Tensor targets);
+std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits,
+                                            torch::Tensor targets,
+                                            torch::Tensor mask,
+                                            torch::Tensor rewards, double scale);
 torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets,
-                               torch::Tensor w, torch::Tensor lse);
+                               torch::Tensor w, torch::Tensor lse,
+                               c10::optional<torch::Tensor> dloss);
 torch::Tensor nf4_gemm(torch::Tensor x, torch::Tensor w4f, torch::Tensor amaxf,
                        c10::optional<torch::Tensor> bias,
                        c10::optional<torch::Tensor> u,
@@ -105,8 +110,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sample_tokens2", &sample_tokens, "sample_tokens by its other name");
   m.def("logprob_lse_fwd", &logprob_lse_fwd,
         "per-token log p(target) + LSE, one streaming pass");
+  m.def("logprob_loss_fwd", &logprob_loss_fwd,
+        "masked PG/GRPO loss, its row weights and the LSE");
   m.def("logprob_loss_bwd", &logprob_loss_bwd,
-        "dlogits for the masked PG/GRPO loss");
+        "dlogits for the masked PG/GRPO loss", py::arg("logits"),
+        py::arg("targets"), py::arg("w"), py::arg("lse"),
+        py::arg("dloss") = py::none());
   m.def("adam8bit_step", &adam8bit_step, "fused blockwise 8-bit Adam step");
   m.def("nf4_gemm", &nf4_gemm,
         "fused nf4-dequant MFMA GEMM with bias + LoRA-B epilogue");

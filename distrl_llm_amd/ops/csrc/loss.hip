@@ -15,62 +15,101 @@ DEV_INLINE float ld(const T* p, int64_t i);
 template <> DEV_INLINE float ld<__hip_bfloat16>(const __hip_bfloat16* p, int64_t i) { return bf2f(p[i]); }
 template <> DEV_INLINE float ld<float>(const float* p, int64_t i) { return p[i]; }
 
-// one workgroup per (b, t) row; single streaming pass, online logsumexp.
+// One workgroup per (b, t) row; single streaming pass, online logsumexp: a
+// thread takes 16 values at a time, compares their maximum with its own once
+// and then sums exponentials without branches (value by value, with two
+// branches and an equality test for the target each, vector work held it to
+// 3.4 TB/s: 215 us for 2408 rows of 152064, 178 now).
 template <typename T>
 __global__ __launch_bounds__(256)
 void logprob_lse_kernel(const T* __restrict__ logits,
                         const int64_t* __restrict__ targets,
                         float* __restrict__ token_logp,
                         float* __restrict__ lse_out, int V) {
+  constexpr float LOG2E = 1.4426950408889634f;
+  constexpr bool BF16 = std::is_same<T, __hip_bfloat16>::value;
   __shared__ float red[16];
-  __shared__ float tgt_logit_s;
   const int64_t row = blockIdx.x;
   const T* lr = logits + row * V;
-  const int64_t tgt = targets[row];
 
-  float m = -1e30f, s = 0.f;
-  if constexpr (std::is_same<T, __hip_bfloat16>::value) {
+  float m = -1e30f, s = 0.f;     // s: sum of 2^((x - m) log2 e)
+  auto take = [&](const float* x, int n) {
+    float top = m;
+    #pragma unroll
+    for (int j = 0; j < n; ++j) top = fmaxf(top, x[j]);
+    if (top > m) {
+      s *= __builtin_amdgcn_exp2f((m - top) * LOG2E);
+      m = top;
+    }
+    const float c = m * LOG2E;
+    #pragma unroll
+    for (int j = 0; j < n; ++j) s += __builtin_amdgcn_exp2f(x[j] * LOG2E - c);
+  };
+  int done = 0;
+  if constexpr (BF16) {
     const bf16x8* l8 = reinterpret_cast<const bf16x8*>(lr);
     const int nvec = V / 8;
-    for (int i = threadIdx.x; i < nvec; i += blockDim.x) {
-      bf16x8 v = l8[i];
+    int i = threadIdx.x;
+    for (; i + 256 < nvec; i += 512) {
+      const bf16x8 v = l8[i], u = l8[i + 256];
+      float x[16];
       #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float x = bf2f(v.v[j]);
-        if (i * 8 + j == (int)tgt) tgt_logit_s = x;
-        if (x > m) {
-          s = s * __expf(m - x) + 1.f;
-          m = x;
-        } else {
-          s += __expf(x - m);
-        }
-      }
+      for (int j = 0; j < 8; ++j) { x[j] = bf2f(v.v[j]); x[8 + j] = bf2f(u.v[j]); }
+      take(x, 16);
     }
-    for (int i = nvec * 8 + threadIdx.x; i < V; i += blockDim.x) {
-      float x = ld(lr, i);
-      if (i == (int)tgt) tgt_logit_s = x;
-      if (x > m) { s = s * __expf(m - x) + 1.f; m = x; }
-      else s += __expf(x - m);
+    if (i < nvec) {
+      const bf16x8 v = l8[i];
+      float x[8];
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = bf2f(v.v[j]);
+      take(x, 8);
     }
-  } else {
-    for (int i = threadIdx.x; i < V; i += blockDim.x) {
-      float x = ld(lr, i);
-      if (i == tgt) tgt_logit_s = x;   // exactly one thread hits it
-      if (x > m) {
-        s = s * __expf(m - x) + 1.f;
-        m = x;
-      } else {
-        s += __expf(x - m);
-      }
-    }
+    done = nvec * 8;
+  }
+  for (int i = done + threadIdx.x; i < V; i += 256) {
+    const float x = ld(lr, i);
+    take(&x, 1);
   }
   // combine per-thread (m, s): M = max m; S = sum s_i * exp(m_i - M)
   const float M = block_max(m, red);
-  const float S = block_sum(s * __expf(m - M), red);
+  const float S = block_sum(s * __builtin_amdgcn_exp2f((m - M) * LOG2E), red);
   if (threadIdx.x == 0) {
     const float lse = M + __logf(S);
+    const int64_t tgt = targets[row];
     lse_out[row] = lse;
-    token_logp[row] = tgt_logit_s - lse;
+    token_logp[row] = (tgt >= 0 && tgt < V ? ld(lr, tgt) : 0.f) - lse;
+  }
+}
+
+// Row weights and the loss itself: w[b, t] = mask * coef_b with
+// coef_b = -reward_b / max(sum mask, 1) / B * scale, loss = sum w * token_logp.
+// One wave a sequence and turn.
+template <typename M>
+__global__ __launch_bounds__(1024)
+void loss_reduce_kernel(const float* __restrict__ token_logp, const M* __restrict__ mask,
+                        const float* __restrict__ rewards, float* __restrict__ w,
+                        float* __restrict__ loss, int B, int T, float scale) {
+  __shared__ float part[16];
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x & (WAVE - 1);
+  float total = 0.f;
+  for (int b = wave; b < B; b += 16) {
+    const int64_t at = (int64_t)b * T;
+    float n = 0.f, sum = 0.f;
+    for (int t = lane; t < T; t += WAVE) {
+      const float k = (float)mask[at + t];
+      n += k;
+      sum += token_logp[at + t] * k;
+    }
+    const float coef = -rewards[b] / fmaxf(wave_sum(n), 1.f) / B * scale;
+    for (int t = lane; t < T; t += WAVE) w[at + t] = (float)mask[at + t] * coef;
+    total += wave_sum(sum) * coef;
+  }
+  if (lane == 0) part[wave] = total;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float sum = 0.f;
+    for (int i = 0; i < 16; ++i) sum += part[i];
+    *loss = sum;
   }
 }
 
@@ -80,11 +119,12 @@ void loss_bwd_kernel(const T* __restrict__ logits,
                      const int64_t* __restrict__ targets,
                      const float* __restrict__ w,
                      const float* __restrict__ lse,
+                     const float* __restrict__ dloss,   // scalar, or null: 1
                      T* __restrict__ dlogits, int V) {
   const int64_t row = blockIdx.x;
   const T* lr = logits + row * V;
   T* dr = dlogits + row * V;
-  const float wv = w[row];
+  const float wv = dloss ? w[row] * *dloss : w[row];
   const float l = lse[row];
   const int64_t tgt = targets[row];
   if constexpr (std::is_same<T, __hip_bfloat16>::value) {
@@ -158,9 +198,42 @@ std::vector<torch::Tensor> logprob_lse_fwd(torch::Tensor logits,
   return {token_logp, lse};
 }
 
+// The masked PG/GRPO loss of logits (B, T, V): {loss, row weights (B, T), lse}.
+// mask int64 or fp32, rewards fp32.
+std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits, torch::Tensor targets,
+                                            torch::Tensor mask, torch::Tensor rewards,
+                                            double scale) {
+  TORCH_CHECK(logits.dim() == 3 && mask.is_cuda() && rewards.is_cuda());
+  const int B = logits.size(0), T = logits.size(1);
+  TORCH_CHECK(mask.numel() == (int64_t)B * T && targets.numel() == (int64_t)B * T &&
+              rewards.numel() == B, "logprob_loss: shape mismatch");
+  TORCH_CHECK(mask.is_contiguous() && rewards.is_contiguous() &&
+              rewards.scalar_type() == at::kFloat);
+  auto lp = logprob_lse_fwd(logits, targets);
+  auto w = torch::empty_like(lp[0]);
+  auto loss = torch::empty({}, lp[0].options());
+  auto stream = at::cuda::getCurrentCUDAStream();
+  #define REDUCE(M)                                                                   \
+    hipLaunchKernelGGL(loss_reduce_kernel<M>, dim3(1), dim3(1024), 0, stream,         \
+                       lp[0].data_ptr<float>(), mask.data_ptr<M>(),                   \
+                       rewards.data_ptr<float>(), w.data_ptr<float>(),                \
+                       loss.data_ptr<float>(), B, T, (float)scale)
+  if (mask.scalar_type() == at::kLong) REDUCE(int64_t);
+  else { TORCH_CHECK(mask.scalar_type() == at::kFloat); REDUCE(float); }
+  #undef REDUCE
+  HIP_CHECK_LAST();
+  return {loss, w, lp[1]};
+}
+
 torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets,
-                               torch::Tensor w, torch::Tensor lse) {
+                               torch::Tensor w, torch::Tensor lse,
+                               c10::optional<torch::Tensor> dloss) {
   TORCH_CHECK(logits.is_cuda() && logits.is_contiguous());
+  const float* dl = nullptr;
+  if (dloss) {
+    TORCH_CHECK(dloss->is_cuda() && dloss->numel() == 1 && dloss->scalar_type() == at::kFloat);
+    dl = dloss->data_ptr<float>();
+  }
   const int V = logits.size(-1);
   const int64_t rows = logits.numel() / V;
   auto dlogits = torch::empty_like(logits);
@@ -173,13 +246,13 @@ torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets,
     hipLaunchKernelGGL(loss_bwd_kernel<__hip_bfloat16>, grid, block, 0, stream,
                        reinterpret_cast<const __hip_bfloat16*>(logits.data_ptr()),
                        targets.contiguous().data_ptr<int64_t>(),
-                       wc.data_ptr<float>(), lsec.data_ptr<float>(),
+                       wc.data_ptr<float>(), lsec.data_ptr<float>(), dl,
                        reinterpret_cast<__hip_bfloat16*>(dlogits.data_ptr()), V);
   } else {
     hipLaunchKernelGGL(loss_bwd_kernel<float>, grid, block, 0, stream,
                        logits.data_ptr<float>(),
                        targets.contiguous().data_ptr<int64_t>(),
-                       wc.data_ptr<float>(), lsec.data_ptr<float>(),
+                       wc.data_ptr<float>(), lsec.data_ptr<float>(), dl,
                        dlogits.data_ptr<float>(), V);
   }
   HIP_CHECK_LAST();

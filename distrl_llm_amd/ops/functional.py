@@ -306,29 +306,35 @@ class _LogprobLossFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, targets, mask, rewards, loss_scale):
         ext = _require_ext("logprob_loss") if logits.is_cuda else None
-        m = mask.to(torch.float32)
-        denom = m.sum(-1).clamp_min(1.0)
-        coef = -rewards.to(torch.float32) / denom / logits.shape[0] * loss_scale
         logits = logits.contiguous()
         if ext is not None:
-            tok, lse = ext.logprob_lse_fwd(logits, targets.contiguous())
+            # int64 masks are read as they are
+            m = mask if mask.dtype == torch.int64 else mask.to(torch.float32)
+            loss, w, lse = ext.logprob_loss_fwd(
+                logits, targets.contiguous(), m.contiguous(),
+                rewards.to(torch.float32).contiguous(), float(loss_scale))
         else:
+            m = mask.to(torch.float32)
+            denom = m.sum(-1).clamp_min(1.0)
+            coef = (-rewards.to(torch.float32) / denom / logits.shape[0]
+                    * loss_scale)
             logp = logits.float().log_softmax(-1)
             tok = logp.gather(-1, targets.unsqueeze(-1)).squeeze(-1)
             lse = torch.logsumexp(logits.float(), -1)
-        loss = ((tok * m).sum(-1) * coef).sum()
-        ctx.save_for_backward(logits, targets, m, coef, lse)
+            loss = ((tok * m).sum(-1) * coef).sum()
+            w = m * coef.unsqueeze(-1)
+        ctx.save_for_backward(logits, targets, w, lse)
         ctx.used_ext = ext is not None
         return loss
 
     @staticmethod
     def backward(ctx, dloss):
-        logits, targets, m, coef, lse = ctx.saved_tensors
-        w = (m * coef.unsqueeze(-1)) * dloss.float()
+        logits, targets, w, lse = ctx.saved_tensors
         if ctx.used_ext:
-            ext = get_extension()
-            dlogits = ext.logprob_loss_bwd(logits, targets, w, lse)
+            dlogits = get_extension().logprob_loss_bwd(
+                logits, targets.contiguous(), w, lse, dloss.float())
         else:
+            w = w * dloss.float()
             probs = (logits.float() - lse.unsqueeze(-1)).exp()
             dlogits = probs * (-w).unsqueeze(-1)
             dlogits.scatter_add_(-1, targets.unsqueeze(-1), w.unsqueeze(-1))

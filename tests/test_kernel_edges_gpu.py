@@ -458,3 +458,38 @@ def test_packed_prefill_matches_modules(name, lora_r, four_bit):
         w = w + at.k_proj.scale * at.k_proj.lora_B.double() @ at.k_proj.lora_A.double()
     q = model.spec.q_size
     assert _rel(eng.fused.layers[1].qkv_w[q:q + model.spec.kv_size], w) < 2.0 ** -8
+
+
+# ------------------------------------------------------------------- loss
+
+@pytest.mark.parametrize("B,T,V,dtype", [
+    (1, 1, 8, "bfloat16"), (2, 3, 4095, "bfloat16"), (17, 5, 4104, "bfloat16"),
+    (3, 70, 6000, "float32"), (2, 2, 152064, "bfloat16")])
+@pytest.mark.parametrize("mask_dtype", [torch.int64, torch.bool, torch.float32])
+def test_loss_edges(B, T, V, dtype, mask_dtype):
+    """Vector remainders and odd row places, more sequences than waves, empty
+    masks, each mask type, a scaled loss. fp32 sums: 1e-5 of the largest term;
+    the gradient is rounded to the logits' type once."""
+    from distrl_llm_amd.ops import functional as OF
+    g = torch.Generator().manual_seed(V)
+    logits = (torch.randn(B, T, V, generator=g) * 3).to("cuda", getattr(torch, dtype))
+    logits[..., 1] = float("-inf")
+    targets = torch.randint(2, V, (B, T), generator=g).cuda()
+    mask = (torch.rand(B, T, generator=g) < 0.7).to(mask_dtype).cuda()
+    mask[-1] = 0
+    rewards = torch.randn(B, generator=g).cuda()
+    leaf = logits.detach().requires_grad_()
+    loss = OF.logprob_loss(leaf, targets, mask, rewards, 0.25)
+    grad, = torch.autograd.grad(loss * 3.0, leaf)
+    exact = logits.double().requires_grad_()
+    m = mask.double()
+    tok = exact.log_softmax(-1).gather(-1, targets.unsqueeze(-1)).squeeze(-1)
+    ref = -((tok * m).sum(-1) / m.sum(-1).clamp_min(1) * rewards.double()).mean() * 0.25
+    ref_grad, = torch.autograd.grad(ref * 3.0, exact)
+    ref_grad = ref_grad.nan_to_num(0.0)
+    assert abs(float(loss) - float(ref)) < 1e-5 * float((tok * m).abs().max() * rewards.abs().max()
+                                                        + 1e-30)
+    if float(ref_grad.norm()) == 0.0:
+        assert float(grad.float().abs().max()) == 0.0
+    else:
+        assert _rel(grad, ref_grad) < (2.0 ** -8 if dtype == "bfloat16" else 1e-5)
