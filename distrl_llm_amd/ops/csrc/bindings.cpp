@@ -68,6 +68,11 @@ void lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b,
 torch::Tensor mfma_probe(torch::Tensor a, torch::Tensor b);
 std::vector<torch::Tensor> flash_attn_fwd(torch::Tensor q, torch::Tensor k,
                                           torch::Tensor v, double scale);
+torch::Tensor flash_attention(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                              double scale);
+torch::Tensor logprob_loss(torch::Tensor logits, torch::Tensor targets,
+                           torch::Tensor mask, torch::Tensor rewards,
+                           double scale);
 torch::Tensor flash_attn_varlen(torch::Tensor q, torch::Tensor k,
                                 torch::Tensor v, torch::Tensor cu,
                                 int64_t max_len, double scale);
@@ -133,6 +138,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("mfma_probe", &mfma_probe, "16x16x32 bf16 MFMA mapping probe");
   m.def("flash_attn_fwd", &flash_attn_fwd,
         "causal GQA flash attention forward (returns o, lse)");
+  m.def("flash_attention", &flash_attention,
+        "differentiable causal GQA flash attention");
+  m.def("logprob_loss", &logprob_loss, "differentiable masked PG/GRPO loss");
   m.def("flash_attn_varlen", &flash_attn_varlen,
         "causal GQA flash attention over a flat batch of sequences");
   m.def("flash_attn_bwd", &flash_attn_bwd,

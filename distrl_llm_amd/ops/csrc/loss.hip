@@ -258,3 +258,34 @@ torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets,
   HIP_CHECK_LAST();
   return dlogits;
 }
+
+// The differentiable loss: a node of the C++ engine.
+namespace {
+
+struct LogprobLoss : public torch::autograd::Function<LogprobLoss> {
+  static torch::Tensor forward(torch::autograd::AutogradContext* ctx, torch::Tensor logits,
+                               torch::Tensor targets, torch::Tensor mask, torch::Tensor rewards,
+                               double scale) {
+    logits = logits.contiguous();
+    targets = targets.contiguous();
+    // int64 masks are read as they are
+    auto m = mask.scalar_type() == at::kLong ? mask : mask.to(at::kFloat);
+    auto r = logprob_loss_fwd(logits, targets, m.contiguous(),
+                              rewards.to(at::kFloat).contiguous(), scale);
+    ctx->save_for_backward({logits, targets, r[1], r[2]});
+    return r[0];
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto s = ctx->get_saved_variables();
+    auto d = logprob_loss_bwd(s[0], s[1], s[2], s[3], grads[0].to(at::kFloat));
+    return {d, torch::Tensor(), torch::Tensor(), torch::Tensor(), torch::Tensor()};
+  }
+};
+
+}  // namespace
+
+torch::Tensor logprob_loss(torch::Tensor logits, torch::Tensor targets, torch::Tensor mask,
+                           torch::Tensor rewards, double scale) {
+  return LogprobLoss::apply(logits, targets, mask, rewards, scale);
+}

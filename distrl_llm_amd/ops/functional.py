@@ -263,34 +263,14 @@ def nf4_linear(x, w4f, amaxf, packed, absmax, bias, N: int, K: int):
 
 # --------------------------------------------------- flash attention
 
-class _FlashAttnFn(torch.autograd.Function):
-    """First-party CDNA4 causal GQA flash attention (ops/csrc/attention.hip)
-    — the learner's training attention without aotriton/Triton (SURVEY.md
-    §2.4-B row "causal attention fwd/bwd"; reference hot path
-    distributed_actor.py:241-243 + loss.backward())."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, scale):
-        ext = _require_ext("flash_attention")
-        o, lse = ext.flash_attn_fwd(q, k, v, float(scale))
-        ctx.save_for_backward(q, k, v, o, lse)
-        ctx.scale = float(scale)
-        return o
-
-    @staticmethod
-    def backward(ctx, dout):
-        q, k, v, o, lse = ctx.saved_tensors
-        ext = _require_ext("flash_attention")
-        dq, dk, dv = ext.flash_attn_bwd(dout.to(q.dtype), q, k, v, o, lse,
-                                        ctx.scale)
-        return dq, dk, dv, None
-
-
 def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                     scale: float) -> torch.Tensor:
-    """Causal GQA attention, (B, H, T, D) layout, bf16. k/v carry the KV
-    head count natively (no repeat_interleave materialization)."""
-    return _FlashAttnFn.apply(q, k, v, scale)
+    """Causal GQA attention (ops/csrc/attention.hip; reference hot path
+    distributed_actor.py:241-243 + loss.backward()): (B, H, T, D) in any
+    strides, bf16. k/v carry the KV head count natively (no
+    repeat_interleave materialization)."""
+    return _require_ext("flash_attention").flash_attention(q, k, v,
+                                                           float(scale))
 
 
 # ------------------------------------------------------------ fused loss
@@ -305,40 +285,26 @@ class _LogprobLossFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, logits, targets, mask, rewards, loss_scale):
-        ext = _require_ext("logprob_loss") if logits.is_cuda else None
+        m = mask.to(torch.float32)
+        denom = m.sum(-1).clamp_min(1.0)
+        coef = (-rewards.to(torch.float32) / denom / logits.shape[0]
+                * loss_scale)
         logits = logits.contiguous()
-        if ext is not None:
-            # int64 masks are read as they are
-            m = mask if mask.dtype == torch.int64 else mask.to(torch.float32)
-            loss, w, lse = ext.logprob_loss_fwd(
-                logits, targets.contiguous(), m.contiguous(),
-                rewards.to(torch.float32).contiguous(), float(loss_scale))
-        else:
-            m = mask.to(torch.float32)
-            denom = m.sum(-1).clamp_min(1.0)
-            coef = (-rewards.to(torch.float32) / denom / logits.shape[0]
-                    * loss_scale)
-            logp = logits.float().log_softmax(-1)
-            tok = logp.gather(-1, targets.unsqueeze(-1)).squeeze(-1)
-            lse = torch.logsumexp(logits.float(), -1)
-            loss = ((tok * m).sum(-1) * coef).sum()
-            w = m * coef.unsqueeze(-1)
-        ctx.save_for_backward(logits, targets, w, lse)
-        ctx.used_ext = ext is not None
+        logp = logits.float().log_softmax(-1)
+        tok = logp.gather(-1, targets.unsqueeze(-1)).squeeze(-1)
+        lse = torch.logsumexp(logits.float(), -1)
+        loss = ((tok * m).sum(-1) * coef).sum()
+        ctx.save_for_backward(logits, targets, m, coef, lse)
         return loss
 
     @staticmethod
     def backward(ctx, dloss):
-        logits, targets, w, lse = ctx.saved_tensors
-        if ctx.used_ext:
-            dlogits = get_extension().logprob_loss_bwd(
-                logits, targets.contiguous(), w, lse, dloss.float())
-        else:
-            w = w * dloss.float()
-            probs = (logits.float() - lse.unsqueeze(-1)).exp()
-            dlogits = probs * (-w).unsqueeze(-1)
-            dlogits.scatter_add_(-1, targets.unsqueeze(-1), w.unsqueeze(-1))
-            dlogits = dlogits.to(logits.dtype)
+        logits, targets, m, coef, lse = ctx.saved_tensors
+        w = (m * coef.unsqueeze(-1)) * dloss.float()
+        probs = (logits.float() - lse.unsqueeze(-1)).exp()
+        dlogits = probs * (-w).unsqueeze(-1)
+        dlogits.scatter_add_(-1, targets.unsqueeze(-1), w.unsqueeze(-1))
+        dlogits = dlogits.to(logits.dtype)
         return dlogits, None, None, None, None
 
 
@@ -347,4 +313,9 @@ def logprob_loss(logits: torch.Tensor, targets: torch.Tensor, mask: torch.Tensor
     """PG/GRPO loss on answer-region logits. logits (B, T, V); targets/mask
     (B, T); rewards (B,). ``loss_scale`` folds the reference's
     loss/num_batches scaling (reference distributed_actor.py:382)."""
+    if logits.is_cuda:
+        ext = _require_ext("logprob_loss")
+        if ext is not None:
+            return ext.logprob_loss(logits, targets, mask, rewards,
+                                    float(loss_scale))
     return _LogprobLossFn.apply(logits, targets, mask, rewards, loss_scale)
