@@ -307,8 +307,11 @@ class Engine:
                 else:
                     torch.addmm(mod.bias, x, mod.weight.t(), out=y)
                 if mod.r > 0:
-                    y.addmm_(x @ mod.lora_A.t(), mod.lora_B.t(),
-                             alpha=mod.scale)
+                    u = x @ mod.lora_A.t()
+                    if ext.lora_merge_takes(mod.out_features, mod.r):
+                        ext.lora_add(y, u, mod.lora_B, True, mod.scale)
+                    else:
+                        y.addmm_(u, mod.lora_B.t(), alpha=mod.scale)
             return out
 
         res = m.model.embed_tokens(input_ids)

@@ -70,10 +70,19 @@ def _scaled_mm(a, b, scale, out=None):
     return torch.addmm(out, a, b, beta=0.0, alpha=scale, out=out)
 
 
+def _add(y, u, m, scale=1.0):
+    """y += scale * u m, in place; m as it lies or a transposed view."""
+    ext, flip = _ext(), not m.is_contiguous()
+    if ext.lora_merge_takes(y.shape[1], u.shape[1]):
+        ext.lora_add(y, u, m.t() if flip else m, flip, scale)
+        return y
+    return y.addmm_(u, m, alpha=scale)
+
+
 def _project(x, u, weight, bias, B, scale):
     """x W^T + b + scale * u B^T."""
     y = x @ weight.t() if bias is None else torch.addmm(bias, x, weight.t())
-    return y.addmm_(u, B.t(), alpha=scale)
+    return _add(y, u, B.t(), scale)
 
 
 class _Attention(torch.autograd.Function):
@@ -106,7 +115,7 @@ class _Attention(torch.autograd.Function):
         o2 = o.transpose(1, 2).reshape(B * T, s.q_size)
         uo = o2 @ Ao.t()
         y = torch.addmm(x, o2, at.o_proj.weight.t())
-        y.addmm_(uo, Bo.t(), alpha=at.o_proj.scale)
+        _add(y, uo, Bo.t(), at.o_proj.scale)
         ctx.save_for_backward(x, h, A, u, Bq, Bk, Bv, Ao, Bo, q, k, v, o, lse,
                               uo, pos, back_freq, q0, k0)
         ctx.at, ctx.norm, ctx.shape = at, norm, shape
@@ -125,7 +134,7 @@ class _Attention(torch.autograd.Function):
 
         duo = _scaled_mm(g, Bo, at.o_proj.scale)
         dAo, dBo = duo.t() @ o2, _scaled_mm(g.t(), uo, at.o_proj.scale)
-        do = (g @ at.o_proj.weight).addmm_(duo, Ao)
+        do = _add(g @ at.o_proj.weight, duo, Ao)
         do = do.view(B, T, s.num_heads, s.head_dim).transpose(1, 2)
         dq, dk, dv = ext.flash_attn_bwd(do, q, k, v, o, lse, at.scale)
         dq, dk, dv = (t.transpose(1, 2).reshape(rows, -1, s.head_dim)
@@ -151,7 +160,7 @@ class _Attention(torch.autograd.Function):
             dh = dq @ at.q_proj.weight
             dh.addmm_(dk, at.k_proj.weight)
             dh.addmm_(dv, at.v_proj.weight)
-            dh.addmm_(du, A)
+            _add(dh, du, A)
             dx = ext.rmsnorm_bwd_add(dh, x, norm.weight, g, norm.eps)
         return (dx, None, None, None, None, dAq, dBs[0], dAk, dBs[1],
                 dAv, dBs[2], dAo, dBo)
@@ -174,7 +183,7 @@ class _FeedForward(torch.autograd.Function):
         act = ext.silu_mul_fwd(gate, up)
         ud = act @ Ad.t()
         y = torch.addmm(x, act, mlp.down_proj.weight.t())
-        y.addmm_(ud, Bd.t(), alpha=mlp.down_proj.scale)
+        _add(y, ud, Bd.t(), mlp.down_proj.scale)
         ctx.save_for_backward(x, h, A, u, Bg, Bu, Ad, Bd, gate, up, act, ud)
         ctx.mlp, ctx.norm = mlp, norm
         return y
@@ -187,7 +196,7 @@ class _FeedForward(torch.autograd.Function):
         g = g.contiguous()
         dud = _scaled_mm(g, Bd, mlp.down_proj.scale)
         dAd, dBd = dud.t() @ act, _scaled_mm(g.t(), ud, mlp.down_proj.scale)
-        dact = (g @ mlp.down_proj.weight).addmm_(dud, Ad)
+        dact = _add(g @ mlp.down_proj.weight, dud, Ad)
         dgate, dup = ext.silu_mul_bwd(dact, gate, up)
         ranks = [Bg.shape[1], Bu.shape[1]]
         du = g.new_empty(g.shape[0], sum(ranks))
@@ -201,7 +210,7 @@ class _FeedForward(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             dh = dgate @ mlp.gate_proj.weight
             dh.addmm_(dup, mlp.up_proj.weight)
-            dh.addmm_(du, A)
+            _add(dh, du, A)
             dx = ext.rmsnorm_bwd_add(dh, x, norm.weight, g, norm.eps)
         return dx, None, None, dAg, dBg, dAu, dBu, dAd, dBd
 

@@ -5,10 +5,22 @@
 // One read of W and one write of out, 16 B a lane; B A comes from MFMA
 // 16x16x32 on the way (one product per 16 x 16 x 32 of r): A's tile lies in
 // LDS and is read transposed, with the columns of two products interleaved so
-// that a lane ends up with 8 consecutive k of one row. Bound: memory.
+// that a lane ends up with 8 consecutive k of one row. Bound: memory; the
+// eight loads of a row's 256 columns are all in flight before the products
+// (two at a time: 8.6 us where this takes 5.0, a chain of waits).
 // As torch operations (fp32 product, two conversions, scale, sum, concatenation
 // and copy into the captured storage) the 7B model's refresh took 44 ms,
-// 13 ms now for 2 x 13 GB (with the 4-bit site's adapter packs).
+// 13 ms with two loads in flight; 61 us for a projection of 18944 x 3584, of
+// which a copy of that size takes 55.
+//
+// The same kernel adds an adapter's output to the rows of a product, in place:
+// y += scale * u B^T (TA: A given as (K, r), staged as it lies) and
+// y += scale * u A. r 32, rows x columns, the library's addmm against this:
+// 128 x 896 3.9 and 5.3 us, 2408 x 3584 10 and 12, 2408 x 18944 41 and 40,
+// 4816 x 3584 160 and 19. On the GPU that is a draw below 4000 rows, but the
+// library's call costs 19 us of host time and this one 4, and short
+// micro-batches wait for the host: a pass of the 0.5B model over 3 x 308 tokens
+// 34.2 -> 28.0 ms; the 1.5B model's over 16 x 1550 is unchanged (within 1%).
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
@@ -21,55 +33,78 @@ typedef __attribute__((address_space(3))) bf16v4 lds_bf16v4;
 namespace {
 
 constexpr int KC = 256;            // columns of a workgroup
-constexpr int ROWS = 128;          // rows of a workgroup, 16 a wave and turn
+constexpr int STEPS = KC / 32;     // loads of W in flight
 
+// w and out may be one; rows of w and out are ldw elements apart, those of b
+// ldb. TA: a is (K, r).
+template <bool TA>
 __global__ __launch_bounds__(256)
-void lora_merge_kernel(const __hip_bfloat16* __restrict__ w, const __hip_bfloat16* __restrict__ a,
-                       const __hip_bfloat16* __restrict__ b, __hip_bfloat16* __restrict__ out,
-                       int N, int K, int r, float scale) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];   // A: [r32][KC], rows 16 B apart
+void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict__ a,
+                       const __hip_bfloat16* __restrict__ b, __hip_bfloat16* out, int N, int K,
+                       int r, int rows, int64_t ldw, int ldb, float scale) {
+  // A: [r32][KC], TA: [KC][r32], rows 16 B apart
+  extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int RS = KC * 2 + 16;
   const int k0 = blockIdx.x * KC, r32 = (r + 31) / 32 * 32;
+  const int ts = r32 * 2 + 16;
   for (int i = threadIdx.x; i < r32 * (KC / 8); i += 256) {
-    const int row = i / (KC / 8), c = i % (KC / 8);
+    const int row = TA ? i / (r32 / 8) : i / (KC / 8), c = TA ? i % (r32 / 8) : i % (KC / 8);
     bf16v8 v;
     #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (__bf16)0.f;
-    if (row < r && k0 + c * 8 < K)
-      v = *reinterpret_cast<const bf16v8*>(a + (int64_t)row * K + k0 + c * 8);
-    *reinterpret_cast<bf16v8*>(smem + row * RS + c * 16) = v;
+    if (TA ? k0 + row < K && c * 8 < r : row < r && k0 + c * 8 < K)
+      v = *reinterpret_cast<const bf16v8*>(TA ? a + (int64_t)(k0 + row) * r + c * 8
+                                              : a + (int64_t)row * K + k0 + c * 8);
+    *reinterpret_cast<bf16v8*>(smem + row * (TA ? ts : RS) + c * 16) = v;
   }
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63, g = l >> 4, lr = l & 15;
-  for (int n0 = blockIdx.y * ROWS + wave * 16; n0 < min(N, (int)(blockIdx.y + 1) * ROWS); n0 += 64) {
-    const int n = min(n0 + lr, N - 1);
-    #pragma unroll 2
-    for (int kk = 0; kk < KC; kk += 32) {
-      if (k0 + kk >= K) break;                          // K % 32 == 0
-      const int64_t at = (int64_t)n * K + k0 + kk + g * 8;
-      const bf16v8 wv = *reinterpret_cast<const bf16v8*>(w + at);
-      f32x4 d[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-      for (int s = 0; s < r32; s += 32) {
-        bf16v8 bv;
+  const int end = min(N, (int)(blockIdx.y + 1) * rows);
+  for (int n0 = blockIdx.y * rows + wave * 16; n0 < end; n0 += 64) {
+    const __hip_bfloat16* wrow = w + min(n0 + lr, N - 1) * ldw + g * 8;
+    const __hip_bfloat16* brow = b + (int64_t)min(n0 + lr, N - 1) * ldb;
+    bf16v8 wv[STEPS];
+    #pragma unroll
+    for (int i = 0; i < STEPS; ++i)                     // K % 32 == 0
+      wv[i] = *reinterpret_cast<const bf16v8*>(wrow + min(k0 + i * 32, K - 32));
+    f32x4 d[STEPS][2];
+    #pragma unroll
+    for (int i = 0; i < STEPS; ++i)
+      d[i][0] = d[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < r32; s += 32) {
+      bf16v8 bv = *reinterpret_cast<const bf16v8*>(brow + min(s + g * 8, r - 8));
+      if (s + g * 8 >= r) {                             // r % 8 == 0
         #pragma unroll
         for (int j = 0; j < 8; ++j) bv[j] = (__bf16)0.f;
-        if (s + g * 8 < r)                              // r % 8 == 0
-          bv = *reinterpret_cast<const bf16v8*>(b + (int64_t)n * r + s + g * 8);
+      }
+      #pragma unroll
+      for (int i = 0; i < STEPS; ++i) {
         #pragma unroll
         for (int t = 0; t < 2; ++t) {
           // rows s + 8 g + 0..7 of A; lane i gets column 8 (i/4) + i%4 + 4 t
-          char* p = smem + (s + g * 8 + (lr >> 2)) * RS + (kk + (lr & 3) * 8 + t * 4) * 2;
-          const bf16v4 x = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16v4*)p);
-          const bf16v4 y = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16v4*)(p + 4 * RS));
-          const bf16v8 av = __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
-          d[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, d[t], 0, 0, 0);
+          bf16v8 av;
+          if (TA) {
+            const int k = i * 32 + (lr >> 2) * 8 + (lr & 3) + t * 4;
+            av = *reinterpret_cast<const bf16v8*>(smem + k * ts + (s + g * 8) * 2);
+          } else {
+            char* p = smem + (s + g * 8 + (lr >> 2)) * RS + (i * 32 + (lr & 3) * 8 + t * 4) * 2;
+            const bf16v4 x = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16v4*)p);
+            const bf16v4 y = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16v4*)(p + 4 * RS));
+            av = __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
+          }
+          d[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, d[i][t], 0, 0, 0);
         }
       }
+    }
+    #pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
       bf16v8 o;
       #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = (__bf16)((float)wv[j] + scale * d[j >> 2][j & 3]);
-      if (n0 + lr < N) *reinterpret_cast<bf16v8*>(out + at) = o;
+      for (int j = 0; j < 8; ++j)
+        o[j] = (__bf16)((float)wv[i][j] + scale * d[i][j >> 2][j & 3]);
+      if (n0 + lr < N && k0 + i * 32 < K)
+        *reinterpret_cast<bf16v8*>(out + (n0 + lr) * ldw + k0 + i * 32 + g * 8) = o;
     }
   }
 }
@@ -78,19 +113,50 @@ void lora_merge_kernel(const __hip_bfloat16* __restrict__ w, const __hip_bfloat1
 
 bool lora_merge_takes(int64_t K, int64_t r) { return K % 32 == 0 && r % 8 == 0 && r >= 8 && r <= 128; }
 
-void lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b, torch::Tensor out, double scale) {
-  TORCH_CHECK(w.dim() == 2 && a.dim() == 2 && b.dim() == 2);
-  const int N = w.size(0), K = w.size(1), r = a.size(0);
-  TORCH_CHECK(a.size(1) == K && b.size(0) == N && b.size(1) == r && out.sizes() == w.sizes());
+namespace {
+
+const __hip_bfloat16* lptr(const torch::Tensor& t) {
+  return reinterpret_cast<const __hip_bfloat16*>(t.data_ptr());
+}
+
+// rows of a (rows, columns) operand that 16 B accesses can walk
+bool lrows(const torch::Tensor& t) {
+  return t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() == 2 && t.stride(1) == 1 &&
+         t.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+
+void launch_merge(const torch::Tensor& w, const torch::Tensor& a, const torch::Tensor& b,
+                  torch::Tensor& out, bool ta, double scale) {
+  const int N = w.size(0), K = w.size(1), r = b.size(1);
   TORCH_CHECK(lora_merge_takes(K, r), "lora_merge: unsupported K ", K, " or rank ", r);
-  for (const auto& t : {w, a, b, out})
-    TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.scalar_type() == at::kBFloat16 &&
-                reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0, "lora_merge: operand");
+  TORCH_CHECK((ta ? a.size(0) : a.size(1)) == K && (ta ? a.size(1) : a.size(0)) == r &&
+              b.size(0) == N && out.sizes() == w.sizes(), "lora_merge: shape mismatch");
+  TORCH_CHECK(lrows(w) && lrows(b) && lrows(out) && lrows(a) && a.is_contiguous() &&
+              w.stride(0) == out.stride(0), "lora_merge: operand");
   if (N == 0) return;
-  auto p = [](const torch::Tensor& t) { return reinterpret_cast<const __hip_bfloat16*>(t.data_ptr()); };
-  hipLaunchKernelGGL(lora_merge_kernel, dim3(CDIV(K, KC), CDIV(N, ROWS)), dim3(256),
-                     (r + 31) / 32 * 32 * (KC * 2 + 16), at::cuda::getCurrentCUDAStream(), p(w),
-                     p(a), p(b), reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), N, K, r,
-                     (float)scale);
+  // 4096 tiles fill the chip eight deep: then a staged A serves four turns,
+  // below that every 64 rows get a workgroup of their own.
+  const int rows = (int64_t)CDIV(K, KC) * CDIV(N, 64) >= 4096 ? 256 : 64;
+  const dim3 grid(CDIV(K, KC), CDIV(N, rows)), block(256);
+  auto stream = at::cuda::getCurrentCUDAStream();
+  auto* o = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
+  const int r32 = (r + 31) / 32 * 32, smem = ta ? KC * (r32 * 2 + 16) : r32 * (KC * 2 + 16);
+  hipLaunchKernelGGL(ta ? lora_merge_kernel<true> : lora_merge_kernel<false>, grid, block, smem,
+                     stream, lptr(w), lptr(a), lptr(b), o, N, K, r, rows, w.stride(0),
+                     (int)b.stride(0), (float)scale);
   HIP_CHECK_LAST();
+}
+
+}  // namespace
+
+void lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b, torch::Tensor out, double scale) {
+  TORCH_CHECK(w.dim() == 2 && a.dim() == 2 && b.dim() == 2 && out.dim() == 2);
+  launch_merge(w, a, b, out, false, scale);
+}
+
+// y (M, N) += scale * u (M, r) m, m (r, N), or (N, r) if transposed; rows of y
+// and u in any strides of whole 16 bytes.
+void lora_add(torch::Tensor y, torch::Tensor u, torch::Tensor m, bool transposed, double scale) {
+  TORCH_CHECK(y.dim() == 2 && u.dim() == 2 && m.dim() == 2);
+  launch_merge(y, m, u, y, transposed, scale);
 }

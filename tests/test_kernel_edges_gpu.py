@@ -422,6 +422,21 @@ def test_lora_merge(ext, N, K, r):
     assert bool(out[N].isnan().all())
 
 
+@pytest.mark.parametrize("M,N,r", [(1, 32, 8), (17, 288, 8), (130, 256, 32), (129, 1056, 40),
+                                   (70, 544, 96), (33, 64, 128)])
+def test_lora_add(ext, M, N, r):
+    """In place on rows cut out of wider ones, the matrix in both layouts."""
+    wide, uw, m = _rand((M, N + 64), 1), _rand((M, r + 32), 2), _rand((r, N), 3, 0.3)
+    before = wide.clone()
+    ref = before[:, 32:32 + N].double() + 0.5 * uw[:, 16:16 + r].double() @ m.double()
+    for mat, flip in ((m, False), (m.t().contiguous(), True)):
+        wide.copy_(before)
+        ext.lora_add(wide[:, 32:32 + N], uw[:, 16:16 + r], mat, flip, 0.5)
+        assert _rel(wide[:, 32:32 + N], ref) < 2.0 ** -8
+        assert torch.equal(wide[:, :32], before[:, :32])
+        assert torch.equal(wide[:, 32 + N:], before[:, 32 + N:])
+
+
 @pytest.mark.parametrize("name", ["small-qwen2", "small-qwen3"])
 @pytest.mark.parametrize("lora_r,four_bit", [(0, False), (8, False), (8, True), (12, False)])
 def test_packed_prefill_matches_modules(name, lora_r, four_bit):
@@ -487,6 +502,7 @@ def test_loss_edges(B, T, V, dtype, mask_dtype):
     ref = -((tok * m).sum(-1) / m.sum(-1).clamp_min(1) * rewards.double()).mean() * 0.25
     ref_grad, = torch.autograd.grad(ref * 3.0, exact)
     ref_grad = ref_grad.nan_to_num(0.0)
+    loss, ref, tok = loss.detach(), ref.detach(), tok.detach()
     assert abs(float(loss) - float(ref)) < 1e-5 * float((tok * m).abs().max() * rewards.abs().max()
                                                         + 1e-30)
     if float(ref_grad.norm()) == 0.0:
