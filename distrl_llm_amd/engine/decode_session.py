@@ -7,7 +7,8 @@ finished mask, output buffer, sampler seed/step counters) in device
 tensors, pre-allocates each sequence's worst-case KV blocks up front (the
 admission control already reserved them), and expresses one decode step as
 a fixed tensor program over those buffers — embed -> 28 layers (HIP
-rmsnorm / rope / kv-scatter / paged-attention + hipBLASLt projections) ->
+rmsnorm / rope / kv-scatter / paged-attention + hipBLASLt projections, or
+skinny products for few sequences) ->
 LM head -> fused sampler -> in-graph state advance. That program is
 captured once into a hipGraph and replayed per token (SURVEY.md §2.4-A:
 "hipGraph-captured decode step" north star); the host loop is just

@@ -62,11 +62,10 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
                           c10::optional<torch::Tensor> norm_w, double eps,
                           c10::optional<torch::Tensor> u,
                           c10::optional<torch::Tensor> ub);
-bool lora_merge_takes(int64_t K, int64_t r);
-void lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b,
+bool lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b,
                 torch::Tensor out, double scale);
-void lora_add(torch::Tensor y, torch::Tensor u, torch::Tensor m,
-              bool transposed, double scale);
+bool lora_add(torch::Tensor y, torch::Tensor u, torch::Tensor m,
+              double scale, c10::optional<torch::Tensor> res);
 torch::Tensor mfma_probe(torch::Tensor a, torch::Tensor b);
 std::vector<torch::Tensor> flash_attn_fwd(torch::Tensor q, torch::Tensor k,
                                           torch::Tensor v, double scale);
@@ -135,9 +134,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("bias") = py::none(), py::arg("res") = py::none(),
         py::arg("norm_w") = py::none(), py::arg("eps") = 0.0,
         py::arg("u") = py::none(), py::arg("ub") = py::none());
-  m.def("lora_merge_takes", &lora_merge_takes, "whether lora_merge takes (K, rank)");
   m.def("lora_merge", &lora_merge, "out = W + scale * B A, one pass");
-  m.def("lora_add", &lora_add, "y += scale * u m (or m^T), in place");
+  m.def("lora_add", &lora_add, "y += scale * u m (+ res) in place; false: not these operands",
+        py::arg("y"), py::arg("u"), py::arg("m"), py::arg("scale"),
+        py::arg("res") = c10::nullopt);
   m.def("mfma_probe", &mfma_probe, "16x16x32 bf16 MFMA mapping probe");
   m.def("flash_attn_fwd", &flash_attn_fwd,
         "causal GQA flash attention forward (returns o, lse)");

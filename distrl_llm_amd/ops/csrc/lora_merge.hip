@@ -35,13 +35,14 @@ namespace {
 constexpr int KC = 256;            // columns of a workgroup
 constexpr int STEPS = KC / 32;     // loads of W in flight
 
-// w and out may be one; rows of w and out are ldw elements apart, those of b
+// w and out may be one; res (or none) is added to the same sum; rows of w and out are ldw elements apart, those of b
 // ldb. TA: a is (K, r).
 template <bool TA>
 __global__ __launch_bounds__(256)
 void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict__ a,
-                       const __hip_bfloat16* __restrict__ b, __hip_bfloat16* out, int N, int K,
-                       int r, int rows, int64_t ldw, int ldb, float scale) {
+                       const __hip_bfloat16* __restrict__ b, const __hip_bfloat16* __restrict__ res,
+                       __hip_bfloat16* out, int N, int K, int r, int rows, int64_t ldw, int ldb,
+                       int64_t ldr, float scale) {
   // A: [r32][KC], TA: [KC][r32], rows 16 B apart
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int RS = KC * 2 + 16;
@@ -68,6 +69,13 @@ void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict
     #pragma unroll
     for (int i = 0; i < STEPS; ++i)                     // K % 32 == 0
       wv[i] = *reinterpret_cast<const bf16v8*>(wrow + min(k0 + i * 32, K - 32));
+    bf16v8 rv[STEPS];
+    if (res) {
+      #pragma unroll
+      for (int i = 0; i < STEPS; ++i)
+        rv[i] = *reinterpret_cast<const bf16v8*>(res + min(n0 + lr, N - 1) * ldr + g * 8 +
+                                                 min(k0 + i * 32, K - 32));
+    }
     f32x4 d[STEPS][2];
     #pragma unroll
     for (int i = 0; i < STEPS; ++i)
@@ -101,8 +109,10 @@ void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict
     for (int i = 0; i < STEPS; ++i) {
       bf16v8 o;
       #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        o[j] = (__bf16)((float)wv[i][j] + scale * d[i][j >> 2][j & 3]);
+      for (int j = 0; j < 8; ++j) {
+        const float t = (float)wv[i][j] + scale * d[i][j >> 2][j & 3];
+        o[j] = (__bf16)(res ? t + (float)rv[i][j] : t);
+      }
       if (n0 + lr < N && k0 + i * 32 < K)
         *reinterpret_cast<bf16v8*>(out + (n0 + lr) * ldw + k0 + i * 32 + g * 8) = o;
     }
@@ -111,7 +121,7 @@ void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict
 
 }  // namespace
 
-bool lora_merge_takes(int64_t K, int64_t r) { return K % 32 == 0 && r % 8 == 0 && r >= 8 && r <= 128; }
+static bool lora_merge_takes(int64_t K, int64_t r) { return K % 32 == 0 && r % 8 == 0 && r >= 8 && r <= 128; }
 
 namespace {
 
@@ -125,38 +135,48 @@ bool lrows(const torch::Tensor& t) {
          t.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 
-void launch_merge(const torch::Tensor& w, const torch::Tensor& a, const torch::Tensor& b,
-                  torch::Tensor& out, bool ta, double scale) {
+// out = w + scale * b a, or b a^T (ta); false: not these operands
+bool launch_merge(const torch::Tensor& w, const torch::Tensor& a, const torch::Tensor& b,
+                  const torch::Tensor& out, bool ta, double scale,
+                  const c10::optional<torch::Tensor>& res = c10::nullopt) {
+  if (w.dim() != 2 || a.dim() != 2 || b.dim() != 2) return false;
   const int N = w.size(0), K = w.size(1), r = b.size(1);
-  TORCH_CHECK(lora_merge_takes(K, r), "lora_merge: unsupported K ", K, " or rank ", r);
-  TORCH_CHECK((ta ? a.size(0) : a.size(1)) == K && (ta ? a.size(1) : a.size(0)) == r &&
-              b.size(0) == N && out.sizes() == w.sizes(), "lora_merge: shape mismatch");
-  TORCH_CHECK(lrows(w) && lrows(b) && lrows(out) && lrows(a) && a.is_contiguous() &&
-              w.stride(0) == out.stride(0), "lora_merge: operand");
-  if (N == 0) return;
+  if (!lora_merge_takes(K, r) || (ta ? a.size(0) : a.size(1)) != K ||
+      (ta ? a.size(1) : a.size(0)) != r || b.size(0) != N || out.sizes() != w.sizes() ||
+      !lrows(w) || !lrows(b) || !lrows(out) || !lrows(a) || !a.is_contiguous() ||
+      w.stride(0) != out.stride(0))
+    return false;
+  if (res && (!lrows(*res) || res->sizes() != w.sizes())) return false;
+  if (N == 0) return true;
   // 4096 tiles fill the chip eight deep: then a staged A serves four turns,
   // below that every 64 rows get a workgroup of their own.
   const int rows = (int64_t)CDIV(K, KC) * CDIV(N, 64) >= 4096 ? 256 : 64;
   const dim3 grid(CDIV(K, KC), CDIV(N, rows)), block(256);
   auto stream = at::cuda::getCurrentCUDAStream();
-  auto* o = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
   const int r32 = (r + 31) / 32 * 32, smem = ta ? KC * (r32 * 2 + 16) : r32 * (KC * 2 + 16);
   hipLaunchKernelGGL(ta ? lora_merge_kernel<true> : lora_merge_kernel<false>, grid, block, smem,
-                     stream, lptr(w), lptr(a), lptr(b), o, N, K, r, rows, w.stride(0),
-                     (int)b.stride(0), (float)scale);
+                     stream, lptr(w), lptr(a), lptr(b), res ? lptr(*res) : nullptr,
+                     reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), N, K, r, rows,
+                     w.stride(0), (int)b.stride(0), res ? res->stride(0) : 0, (float)scale);
   HIP_CHECK_LAST();
+  return true;
 }
 
 }  // namespace
 
-void lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b, torch::Tensor out, double scale) {
-  TORCH_CHECK(w.dim() == 2 && a.dim() == 2 && b.dim() == 2 && out.dim() == 2);
-  launch_merge(w, a, b, out, false, scale);
+// out = w + scale * b a. False, and nothing done, for operands that 16 B
+// accesses or the tiles can't take.
+bool lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b, torch::Tensor out, double scale) {
+  return launch_merge(w, a, b, out, false, scale);
 }
 
-// y (M, N) += scale * u (M, r) m, m (r, N), or (N, r) if transposed; rows of y
-// and u in any strides of whole 16 bytes.
-void lora_add(torch::Tensor y, torch::Tensor u, torch::Tensor m, bool transposed, double scale) {
-  TORCH_CHECK(y.dim() == 2 && u.dim() == 2 && m.dim() == 2);
-  launch_merge(y, m, u, y, transposed, scale);
+// y (M, N) += scale * u (M, r) m (r, N), then + res if given: one rounding for
+// all of it. m as it lies or a transposed view, rows of y, u and res in any
+// strides of whole 16 bytes. False, and nothing done, for other operands: the
+// caller takes the library's product.
+bool lora_add(torch::Tensor y, torch::Tensor u, torch::Tensor m, double scale,
+              c10::optional<torch::Tensor> res) {
+  if (m.dim() != 2) return false;
+  const bool ta = m.stride(1) != 1;
+  return launch_merge(y, ta ? m.t() : m, u, y, ta, scale, res);
 }

@@ -417,7 +417,7 @@ def test_lora_merge(ext, N, K, r):
     rounding of an fp32 sum."""
     w, a, b = _rand((N, K), 1), _rand((r, K), 2, 0.3), _rand((N, r), 3, 0.3)
     out = torch.full((N + 1, K), float("nan"), dtype=torch.bfloat16, device="cuda")
-    ext.lora_merge(w, a, b, out[:N], 0.5)
+    assert ext.lora_merge(w, a, b, out[:N], 0.5)
     assert _rel(out[:N], w.double() + 0.5 * b.double() @ a.double()) < 2.0 ** -9
     assert bool(out[N].isnan().all())
 
@@ -429,12 +429,22 @@ def test_lora_add(ext, M, N, r):
     wide, uw, m = _rand((M, N + 64), 1), _rand((M, r + 32), 2), _rand((r, N), 3, 0.3)
     before = wide.clone()
     ref = before[:, 32:32 + N].double() + 0.5 * uw[:, 16:16 + r].double() @ m.double()
-    for mat, flip in ((m, False), (m.t().contiguous(), True)):
+    for mat in (m, m.t().contiguous().t()):
         wide.copy_(before)
-        ext.lora_add(wide[:, 32:32 + N], uw[:, 16:16 + r], mat, flip, 0.5)
+        assert ext.lora_add(wide[:, 32:32 + N], uw[:, 16:16 + r], mat, 0.5)
         assert _rel(wide[:, 32:32 + N], ref) < 2.0 ** -8
         assert torch.equal(wide[:, :32], before[:, :32])
         assert torch.equal(wide[:, 32 + N:], before[:, 32 + N:])
+    wide.copy_(before)
+    res = _rand((M, N + 32), 4)[:, 16:16 + N]
+    assert ext.lora_add(wide[:, 32:32 + N], uw[:, 16:16 + r], m, 0.5, res)
+    assert _rel(wide[:, 32:32 + N], ref + res.double()) < 2.0 ** -8
+    # refused, nothing written: unaligned rows, strided columns, other types
+    assert not ext.lora_add(wide[:, 4:4 + N], uw[:, 16:16 + r], m, 0.5)
+    assert not ext.lora_add(wide[:, :N], uw[:, 4:4 + r], m, 0.5)
+    assert not ext.lora_add(wide[:, :N], uw[:, :r].float(), m, 0.5)
+    assert not ext.lora_add(wide[:, :N], uw[:, :r], m.flip(0)[:, ::2], 0.5)
+    assert torch.equal(wide[:, :32], before[:, :32])
 
 
 @pytest.mark.parametrize("name", ["small-qwen2", "small-qwen3"])
