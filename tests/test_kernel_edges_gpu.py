@@ -90,6 +90,24 @@ def test_flash_scale_signs_and_far_scores():
                 assert _rel(x, r) < FLASH_REL
 
 
+@pytest.mark.parametrize("B,H,D", [(1, 2, 64), (1, 2, 128), (300, 2, 64), (300, 2, 128)])
+def test_flash_leading_weight(B, H, D):
+    """A key that takes the lead in a later tile, by 0..8 in log2 over the 64
+    before it, and the only one with a value: its weight carries no rounding, so
+    the output has only its own (2^-8 of the value; 2^-16 for the fp32 sums)."""
+    from distrl_llm_amd.ops import functional as OF
+    T, lead = 160, 64
+    q, k, v = (torch.zeros(B, H, T, D, dtype=torch.bfloat16, device="cuda") for _ in range(3))
+    # scores q[0] * 1 / 8 against zeros
+    q[..., 0] = torch.linspace(0.1, 44.0, B * H * T, device="cuda").view(B, H, T)
+    k[:, :, lead, 0] = 1.0
+    v[:, :, lead] = 1.0
+    out = OF.flash_attention(q, k, v, 0.125)[:, :, lead:].double()
+    s = (q[:, :, lead:, 0].double() * 0.125).exp()
+    ref = (s / (s + torch.arange(lead, T, device="cuda").double()))[..., None]
+    assert float(((out - ref).abs() / ref).max()) < 2.0 ** -8 + 2.0 ** -16
+
+
 @pytest.mark.parametrize("lens", [[1], [5, 64, 65, 1, 200], [130, 3]])
 @pytest.mark.parametrize("H,KV,D", [(4, 2, 64), (7, 1, 128)])
 def test_flash_varlen(ext, lens, H, KV, D):
