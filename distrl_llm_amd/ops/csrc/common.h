@@ -68,17 +68,12 @@ DEV_INLINE float block_max(float x, float* red) {
   return out;
 }
 
-// ---- hash RNG (counter-based; deterministic per (seed, idx)) ----
+// ---- hash (counter-based random numbers) ----
 DEV_INLINE uint64_t splitmix64(uint64_t x) {
   x += 0x9E3779B97F4A7C15ull;
   x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
   x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
   return x ^ (x >> 31);
-}
-// uniform in (0, 1]
-DEV_INLINE float hash_uniform(uint64_t seed, uint64_t idx) {
-  uint64_t h = splitmix64(seed ^ splitmix64(idx));
-  return ((h >> 40) + 1.0f) * (1.0f / 16777217.0f);
 }
 
 #define HIP_CHECK_LAST()                                                     \

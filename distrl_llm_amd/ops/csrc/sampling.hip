@@ -75,12 +75,13 @@ DEV_INLINE uint64_t mix_index(uint32_t idx) {
   return x ^ (x >> 31);
 }
 
-// z - log(-log u) with hash_uniform's u; neither logarithm's argument is ever
-// denormal.
+// z - log(-log u), u = (the hash's upper 24 bits + 1) / 2^24, kept below 1: u = 1
+// would make the key infinite and draw the element whatever its probability.
+// Neither logarithm's argument is ever denormal.
 DEV_INLINE float gumbel_key(uint64_t seed, int idx, float z) {
   constexpr float LN2 = 0.6931471805599453f;
   const uint64_t h = splitmix64(seed ^ mix_index((uint32_t)idx));
-  const float u = ((h >> 40) + 1.0f) * (1.0f / 16777217.0f);
+  const float u = (float)min((uint32_t)(h >> 40) + 1u, (1u << 24) - 1u) * 0x1p-24f;
   return z - LN2 * __builtin_amdgcn_logf(-LN2 * __builtin_amdgcn_logf(u));
 }
 

@@ -1,6 +1,7 @@
 """Kernels at the edges of their tiles, splits and layouts, against plain
 fp32 or fp64 torch."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -125,7 +126,6 @@ def test_flash_varlen(ext, lens, H, KV, D):
 # ---------------------------------------------------------------- sampler
 
 def _splitmix64(x):
-    import numpy as np
     with np.errstate(over="ignore"):
         x = x + np.uint64(0x9E3779B97F4A7C15)
         x = (x ^ (x >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
@@ -136,7 +136,6 @@ def _splitmix64(x):
 def _sampled(logits, temperature, top_p, top_k, seeds, step):
     """The sampler's definition, row by row in numpy: whole bins of 1/32 down
     to the threshold, then the largest z - log(-log u)."""
-    import numpy as np
     V, out = logits.shape[1], []
     for row, seed in zip(logits.float().cpu().numpy(), seeds.tolist()):
         z = (row - row.max()) * (np.float32(1) / np.float32(temperature))
@@ -151,7 +150,7 @@ def _sampled(logits, temperature, top_p, top_k, seeds, step):
             thr = min(thr, int(np.argmax(c >= top_k)))
         base = np.uint64(seed) ^ _splitmix64(np.uint64(0x5D21 + step))
         h = _splitmix64(base ^ _splitmix64(np.arange(V, dtype=np.uint64)))
-        u = ((h >> np.uint64(40)).astype(np.float64) + 1) / 16777217.0
+        u = np.minimum((h >> np.uint64(40)).astype(np.float64) + 1, 2 ** 24 - 1) / 2 ** 24
         key = np.where(z >= -(thr + 1) / 32, z - np.log(-np.log(u)), -np.inf)
         out.append(int(key.argmax()))
     return out
@@ -194,6 +193,24 @@ def test_sampler_odd_places_and_values(ext):
             got = ext.sample_tokens(x, 1.0, top_p, 0, seeds.cuda(), step).tolist()
             assert got == _sampled(logits, 1.0, top_p, 0, seeds, 5)
             assert got[1] % 2 == 1 and got[2] == 77
+
+
+def test_sampler_largest_variate(ext):
+    """Index 39387 of this row hashes to the largest 24 bits there are. Its key
+    is z + 16.64 and not infinite: at z = -18 it does not win over the maximum."""
+    V, at = 152064, 39387
+    h = _splitmix64(np.uint64(203) ^ _splitmix64(np.uint64(0x5D21)) ^ _splitmix64(np.uint64(at)))
+    assert int(h >> np.uint64(40)) == 2 ** 24 - 1
+    logits = torch.full((1, V), -40.0)
+    logits[0, 7], logits[0, at] = 0.0, -18.0
+    logits, seeds = logits.to("cuda", torch.bfloat16), torch.tensor([203])
+    for top_k in (0, 2):
+        got = ext.sample_tokens(logits, 1.0, 1.0, top_k, seeds.cuda(), torch.tensor([0], device="cuda"))
+        assert got.tolist() == _sampled(logits, 1.0, 1.0, top_k, seeds, 0) == [7]
+    # and does where its probability allows it: -0.5 + 16.64
+    logits[0, at] = -0.5
+    got = ext.sample_tokens(logits, 1.0, 1.0, 0, seeds.cuda(), torch.tensor([0], device="cuda"))
+    assert got.tolist() == [at]
 
 
 def test_sampler_in_a_graph(ext):
