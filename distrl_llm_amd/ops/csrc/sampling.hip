@@ -315,7 +315,7 @@ void slice_draw_kernel(const T* __restrict__ logits, int V, int per, float inv_t
   const T* lr = logits + (int64_t)row * V;
   const int i1 = min(V, (sl + 1) * per);
   const float m = row_max(ms, row, S);
-  float zmin = ZDRAW;
+  float zlow = ZDRAW;
   if (BY_P || BY_K) {
     Crossing<float> cp;
     Crossing<int> ck;
@@ -325,7 +325,8 @@ void slice_draw_kernel(const T* __restrict__ logits, int V, int per, float inv_t
     int thr = NBINS - 1;
     if (BY_P) thr = min(thr, cp.bin * IN_GROUP + crossing(h.bin_p[at], cp.before, target).bin);
     if (BY_K) thr = min(thr, ck.bin * IN_GROUP + crossing(h.bin_c[at], ck.before, top_k).bin);
-    zmin = fmaxf(-(thr + 1) * (ZRANGE / NBINS), ZDRAW);
+    // the bins up to thr are z > -(thr + 1) / 32; the edge itself lies in the next
+    zlow = fmaxf(-(thr + 1) * (ZRANGE / NBINS), ZDRAW);
   }
   DrawQueue dq{queue + (tid / WAVE) * 128, row_seed(seeds, step, row)};
   float x[8], next[8];
@@ -338,7 +339,7 @@ void slice_draw_kernel(const T* __restrict__ logits, int V, int per, float inv_t
     #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const float z = (x[k] - m) * inv_temp;
-      dq.push(z >= zmin, id[k], z);
+      dq.push(z > zlow, id[k], z);
     }
   }
   dq.draw(dq.count);

@@ -151,7 +151,8 @@ def _sampled(logits, temperature, top_p, top_k, seeds, step):
         base = np.uint64(seed) ^ _splitmix64(np.uint64(0x5D21 + step))
         h = _splitmix64(base ^ _splitmix64(np.arange(V, dtype=np.uint64)))
         u = np.minimum((h >> np.uint64(40)).astype(np.float64) + 1, 2 ** 24 - 1) / 2 ** 24
-        key = np.where(z >= -(thr + 1) / 32, z - np.log(-np.log(u)), -np.inf)
+        kept = np.where(inside, bins <= thr, thr == 1023)
+        key = np.where(kept, z - np.log(-np.log(u)), -np.inf)
         out.append(int(key.argmax()))
     return out
 
@@ -211,6 +212,22 @@ def test_sampler_largest_variate(ext):
     logits[0, at] = -0.5
     got = ext.sample_tokens(logits, 1.0, 1.0, 0, seeds.cuda(), torch.tensor([0], device="cuda"))
     assert got.tolist() == [at]
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_sampler_threshold_on_a_bin_edge(ext, dtype):
+    """Logits whose distance from the maximum is a whole number of bins: an
+    entry on the threshold bin's lower edge belongs to the next bin, dropped."""
+    B, V = 64, 4096
+    logits = torch.full((B, V), -20.0)
+    logits[:, 5], logits[:, 9], logits[:, 11] = 7.5, 7.46875, 7.4375
+    logits, seeds = logits.to("cuda", getattr(torch, dtype)), torch.arange(B)
+    step = torch.tensor([0], device="cuda")
+    for top_p, top_k, kept in ((1.0, 1, {5}), (0.2, 0, {5}), (1.0, 2, {5, 9}), (0.5, 0, {5, 9}),
+                               (0.9, 0, {5, 9, 11})):
+        got = ext.sample_tokens(logits, 1.0, top_p, top_k, seeds.cuda(), step).tolist()
+        assert set(got) == kept
+        assert got == _sampled(logits, 1.0, top_p, top_k, seeds, 0)
 
 
 def test_sampler_in_a_graph(ext):
