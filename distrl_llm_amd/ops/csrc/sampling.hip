@@ -7,8 +7,10 @@
 // cumulative probability reaches top_p (or the count top_k). The draw is the
 // argmax of z - log(-log u) over the kept set, u a counter-based hash of
 // (seed of the row, step, element): the step is read from device memory, so a
-// replayed graph draws anew, and the draw does not depend on how the row was
-// split over workgroups.
+// replayed graph draws anew. Slices add their probabilities up as integers of
+// 2^-32, whose sum does not hang on their order: a call repeats itself exactly.
+// How a row was split over workgroups (by the number of rows) shows only where
+// a cumulative probability lies within fp32 rounding of top_p.
 //
 // A row is cut into slices, so that any number of rows fills the chip: a
 // maximum pass; with a threshold two histogram passes, first over 32 groups of
@@ -154,11 +156,13 @@ DEV_INLINE float wave_total(float x) {   // lanes 0..31, in their order
 }
 
 // Sums of a row's groups and of the bins of the crossing groups, in global
-// memory: probability and count.
+// memory: probability in units of 2^-32 (a row's is below V < 2^31) and count.
 struct Hist {
-  float *group_p, *bin_p;     // (B, 32) each
+  unsigned long long *group_p, *bin_p;     // (B, 32) each
   int *group_c, *bin_c;
 };
+
+DEV_INLINE float prob(unsigned long long x) { return (float)x * 0x1p-32f; }
 
 // The row's crossing groups, from the group sums: every wave computes them.
 template <bool BY_P, bool BY_K>
@@ -166,7 +170,7 @@ DEV_INLINE void crossing_groups(const Hist& h, int row, float top_p, int top_k,
                                 Crossing<float>& cp, Crossing<int>& ck, float& target) {
   const int at = row * GROUPS + (threadIdx.x & 31);
   if (BY_P) {
-    const float x = h.group_p[at];
+    const float x = prob(h.group_p[at]);
     target = top_p * wave_total(x);
     cp = crossing(x, 0.f, target);
   }
@@ -233,7 +237,7 @@ void slice_max_kernel(const T* __restrict__ logits, int V, int per, float* __res
     if (threadIdx.x == 0) { top[row] = 0ull; done[row] = 0; }
     if (h.group_p && threadIdx.x < 32) {
       const int at = row * 32 + threadIdx.x;
-      h.group_p[at] = h.bin_p[at] = 0.f;
+      h.group_p[at] = h.bin_p[at] = 0ull;
       h.group_c[at] = h.bin_c[at] = 0;
     }
   }
@@ -289,7 +293,9 @@ void slice_hist_kernel(const T* __restrict__ logits, int V, int per, float inv_t
       #pragma unroll
       for (int i = 0; i < 4; ++i) v += hp[b * 256 + i * WAVE + lane];
       v = wave_sum(v);
-      if (lane == 0 && v != 0.f) atomicAdd(&(FINE ? h.bin_p : h.group_p)[row * 32 + b], v);
+      if (lane == 0 && v != 0.f)
+        atomicAdd(&(FINE ? h.bin_p : h.group_p)[row * 32 + b],
+                  (unsigned long long)(v * 0x1p32f + 0.5f));
     }
     if (BY_K) {
       int v = 0;
@@ -323,7 +329,7 @@ void slice_draw_kernel(const T* __restrict__ logits, int V, int per, float inv_t
     crossing_groups<BY_P, BY_K>(h, row, top_p, top_k, cp, ck, target);
     const int at = row * 32 + (tid & 31);
     int thr = NBINS - 1;
-    if (BY_P) thr = min(thr, cp.bin * IN_GROUP + crossing(h.bin_p[at], cp.before, target).bin);
+    if (BY_P) thr = min(thr, cp.bin * IN_GROUP + crossing(prob(h.bin_p[at]), cp.before, target).bin);
     if (BY_K) thr = min(thr, ck.bin * IN_GROUP + crossing(h.bin_c[at], ck.before, top_k).bin);
     // the bins up to thr are z > -(thr + 1) / 32; the edge itself lies in the next
     zlow = fmaxf(-(thr + 1) * (ZRANGE / NBINS), ZDRAW);
@@ -376,19 +382,21 @@ void sample_slices(const T* logits, int B, int V, float inv_t, float top_p, int 
   int S = 1;
   while (S < 64 && (int64_t)B * S < 1024 && V / (2 * S) >= 2048) S *= 2;
   const int per = (CDIV(V, S) + 7) / 8 * 8;
-  auto ws = torch::empty({B * (int64_t)(12 + 4 * S + (filtering ? 4 * 4 * 32 : 0))},
+  auto ws = torch::empty({B * (int64_t)(12 + 4 * S + (filtering ? (8 + 4) * 2 * 32 : 0))},
                          out.options().dtype(at::kByte));
   char* w = reinterpret_cast<char*>(ws.data_ptr());
   auto* top = reinterpret_cast<unsigned long long*>(w);
-  int* done = reinterpret_cast<int*>(w + 8ll * B);
-  float* ms = reinterpret_cast<float*>(w + 12ll * B);
+  w += 8ll * B;
   Hist h{};
   if (filtering) {
-    h.group_p = ms + (int64_t)B * S;
+    h.group_p = reinterpret_cast<unsigned long long*>(w);
     h.bin_p = h.group_p + 32ll * B;
     h.group_c = reinterpret_cast<int*>(h.bin_p + 32ll * B);
     h.bin_c = h.group_c + 32ll * B;
+    w = reinterpret_cast<char*>(h.bin_c + 32ll * B);
   }
+  int* done = reinterpret_cast<int*>(w);
+  float* ms = reinterpret_cast<float*>(w + 4ll * B);
   auto stream = at::cuda::getCurrentCUDAStream();
   const dim3 grid(B, S), block(256);
   hipLaunchKernelGGL((slice_max_kernel<T, VEC>), grid, block, 0, stream, logits, V, per, ms, top,

@@ -230,6 +230,20 @@ def test_sampler_threshold_on_a_bin_edge(ext, dtype):
         assert got == _sampled(logits, 1.0, top_p, top_k, seeds, 0)
 
 
+def test_sampler_repeats_itself(ext):
+    """64 equal rows with one seed draw one token, also where a cumulative
+    probability falls on top_p within rounding: slices finish in any order."""
+    V, step = 32768, torch.tensor([0], device="cuda")
+    for i in range(20):
+        row = torch.randn(1, V, generator=torch.Generator().manual_seed(i)) * 2
+        z = (row[0] - row[0].max()).double()
+        p = torch.bincount((-z * 32).long().clamp(max=1023), z.exp()).cumsum(0)
+        rows, top_p = row.cuda().expand(64, -1).contiguous(), float((p[150 + i] / p[-1]).float())
+        for seed in range(100):
+            seeds = torch.full((64,), seed, device="cuda")
+            assert len(set(ext.sample_tokens(rows, 1.0, top_p, 0, seeds, step).tolist())) == 1
+
+
 def test_sampler_in_a_graph(ext):
     """Replays draw anew with the device step and match eager draws."""
     logits = _rand((5, 32768), 2, 3.0)
