@@ -15,6 +15,16 @@ DEV_INLINE float ld(const T* p, int64_t i);
 template <> DEV_INLINE float ld<__hip_bfloat16>(const __hip_bfloat16* p, int64_t i) { return bf2f(p[i]); }
 template <> DEV_INLINE float ld<float>(const float* p, int64_t i) { return p[i]; }
 
+// Eight values at any element: rows of an odd vocabulary, or of a matrix that
+// starts inside another, lie on 2 bytes. One 16-byte access all the same, which
+// needs no alignment in device memory.
+DEV_INLINE bf16x8 load8(const __hip_bfloat16* p) {
+  bf16x8 v;
+  __builtin_memcpy(&v, p, sizeof v);
+  return v;
+}
+DEV_INLINE void store8(__hip_bfloat16* p, const bf16x8& v) { __builtin_memcpy(p, &v, sizeof v); }
+
 // One workgroup per (b, t) row; single streaming pass, online logsumexp: a
 // thread takes 16 values at a time, compares their maximum with its own once
 // and then sums exponentials without branches (value by value, with two
@@ -47,18 +57,17 @@ void logprob_lse_kernel(const T* __restrict__ logits,
   };
   int done = 0;
   if constexpr (BF16) {
-    const bf16x8* l8 = reinterpret_cast<const bf16x8*>(lr);
     const int nvec = V / 8;
     int i = threadIdx.x;
     for (; i + 256 < nvec; i += 512) {
-      const bf16x8 v = l8[i], u = l8[i + 256];
+      const bf16x8 v = load8(lr + i * 8), u = load8(lr + (i + 256) * 8);
       float x[16];
       #pragma unroll
       for (int j = 0; j < 8; ++j) { x[j] = bf2f(v.v[j]); x[8 + j] = bf2f(u.v[j]); }
       take(x, 16);
     }
     if (i < nvec) {
-      const bf16x8 v = l8[i];
+      const bf16x8 v = load8(lr + i * 8);
       float x[8];
       #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = bf2f(v.v[j]);
@@ -128,8 +137,6 @@ void loss_bwd_kernel(const T* __restrict__ logits,
   const float l = lse[row];
   const int64_t tgt = targets[row];
   if constexpr (std::is_same<T, __hip_bfloat16>::value) {
-    const bf16x8* l8 = reinterpret_cast<const bf16x8*>(lr);
-    bf16x8* d8 = reinterpret_cast<bf16x8*>(dr);
     const int nvec = V / 8;
     for (int i = threadIdx.x; i < nvec; i += blockDim.x) {
       bf16x8 o;
@@ -137,14 +144,14 @@ void loss_bwd_kernel(const T* __restrict__ logits,
         #pragma unroll
         for (int j = 0; j < 8; ++j) o.v[j] = f2bf(0.f);
       } else {
-        bf16x8 v = l8[i];
+        const bf16x8 v = load8(lr + i * 8);
         #pragma unroll
         for (int j = 0; j < 8; ++j) {
           float p = __expf(bf2f(v.v[j]) - l);
           o.v[j] = f2bf(wv * ((i * 8 + j == (int)tgt ? 1.f : 0.f) - p));
         }
       }
-      d8[i] = o;
+      store8(dr + i * 8, o);
     }
     for (int i = nvec * 8 + threadIdx.x; i < V; i += blockDim.x) {
       float g = 0.f;

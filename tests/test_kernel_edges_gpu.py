@@ -585,3 +585,21 @@ def test_loss_edges(B, T, V, dtype, mask_dtype):
         assert float(grad.float().abs().max()) == 0.0
     else:
         assert _rel(grad, ref_grad) < (2.0 ** -8 if dtype == "bfloat16" else 1e-5)
+
+
+@pytest.mark.parametrize("off,V", [(1, 4096), (3, 4103), (0, 32003), (1, 7)])
+def test_loss_rows_at_any_element(ext, off, V):
+    """A matrix that starts inside another and rows of an odd vocabulary give
+    what aligned ones do, forward bit for bit; the gradient rounds once."""
+    rows = 5
+    flat = _rand((rows * V + off,), V, 3.0)
+    logits, targets = flat[off:].view(rows, V), torch.arange(rows, device="cuda")
+    w = torch.linspace(0.0, 1.0, rows, device="cuda")
+    tok, lse = ext.logprob_lse_fwd(logits, targets)
+    grad = ext.logprob_loss_bwd(logits, targets, w, lse)
+    logp = logits.double().log_softmax(-1)
+    ref = w.double()[:, None] * (torch.nn.functional.one_hot(targets, V) - logp.exp())
+    assert torch.allclose(tok.double(), logp[torch.arange(rows), targets], rtol=0, atol=1e-5)
+    assert _rel(grad, ref) < 2.0 ** -8
+    aligned = logits.clone()
+    assert all(torch.equal(a, b) for a, b in zip((tok, lse), ext.logprob_lse_fwd(aligned, targets)))
