@@ -308,14 +308,40 @@ class _LogprobLossFn(torch.autograd.Function):
         return dlogits, None, None, None, None
 
 
+class _TokenLogpFn(torch.autograd.Function):
+    """log p(target) of every row of logits, on the GPU."""
+
+    @staticmethod
+    def forward(ctx, logits, targets):
+        logits = logits.contiguous()
+        tok, lse = _require_ext("logprob_loss").logprob_lse_fwd(logits,
+                                                                targets)
+        ctx.save_for_backward(logits, targets, lse)
+        return tok
+
+    @staticmethod
+    def backward(ctx, dtok):
+        logits, targets, lse = ctx.saved_tensors
+        return _require_ext("logprob_loss").logprob_loss_bwd(
+            logits, targets, dtok.float(), lse), None
+
+
 def logprob_loss(logits: torch.Tensor, targets: torch.Tensor, mask: torch.Tensor,
                  rewards: torch.Tensor, loss_scale: float = 1.0) -> torch.Tensor:
     """PG/GRPO loss on answer-region logits. logits (B, T, V); targets/mask
     (B, T); rewards (B,). ``loss_scale`` folds the reference's
     loss/num_batches scaling (reference distributed_actor.py:382)."""
     if logits.is_cuda:
-        ext = _require_ext("logprob_loss")
-        if ext is not None:
+        ext, lead = _require_ext("logprob_loss"), logits.shape[:-1]
+        if (len(lead) == 2 and targets.shape == mask.shape == lead
+                and rewards.shape == lead[:1] and mask.is_cuda
+                and rewards.is_cuda):
             return ext.logprob_loss(logits, targets, mask, rewards,
                                     float(loss_scale))
+        # rows without a batch, one reward or mask for all: torch broadcasts
+        tok = _TokenLogpFn.apply(logits, targets.reshape(lead))
+        m = mask.to(torch.float32)
+        coef = (-rewards.to(torch.float32) / m.sum(-1).clamp_min(1.0)
+                / logits.shape[0] * loss_scale)
+        return ((tok * m).sum(-1) * coef).sum()
     return _LogprobLossFn.apply(logits, targets, mask, rewards, loss_scale)

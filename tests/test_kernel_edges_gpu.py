@@ -603,3 +603,27 @@ def test_loss_rows_at_any_element(ext, off, V):
     assert _rel(grad, ref) < 2.0 ** -8
     aligned = logits.clone()
     assert all(torch.equal(a, b) for a, b in zip((tok, lse), ext.logprob_lse_fwd(aligned, targets)))
+
+
+@pytest.mark.parametrize("lead,mask_shape,reward_shape,host", [
+    ((6,), (6,), (), False), ((6,), (6,), (1,), False), ((3, 6), (3, 6), (), False),
+    ((3, 6), (3, 6), (1,), False), ((3, 6), (1, 6), (3,), False), ((3, 6), (6,), (3,), False),
+    ((3, 6), (3, 1), (3,), False), ((3, 6), (3, 6), (), True), ((2, 3, 6), (3, 6), (2, 3), False)])
+def test_loss_broadcasts(lead, mask_shape, reward_shape, host):
+    """Shapes that torch broadcasts, against the formula in fp64 (fp32 sums,
+    the gradient rounded to bf16 once)."""
+    from distrl_llm_amd.ops import functional as OF
+    V = 40
+    logits = _rand((*lead, V), 1, 2.0).requires_grad_()
+    targets = torch.randint(0, V, lead, generator=torch.Generator().manual_seed(2)).cuda()
+    mask = (_rand(mask_shape, 3) > -0.5).long()
+    rewards = torch.randn(reward_shape, generator=torch.Generator().manual_seed(4))
+    rewards = rewards if host else rewards.cuda()
+    loss = OF.logprob_loss(logits, targets, mask, rewards, 0.5)
+    grad, = torch.autograd.grad(loss, logits)
+    x = logits.detach().double().requires_grad_()
+    tok = x.log_softmax(-1).gather(-1, targets.unsqueeze(-1)).squeeze(-1)
+    m = mask.double()
+    ref = ((tok * m).sum(-1) * (-rewards.cuda().double() / m.sum(-1).clamp_min(1) / lead[0] * 0.5)).sum()
+    assert float((loss - ref).detach().abs()) < 1e-5 * float(tok.detach().abs().max())
+    assert _rel(grad, torch.autograd.grad(ref, x)[0]) < 2.0 ** -8
