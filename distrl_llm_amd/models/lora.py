@@ -103,11 +103,9 @@ class LoRALinear(nn.Module):
             # addmm folds the scale and the accumulation into the adapter
             # GEMM itself (no separate mul/add kernels in the hot path)
             y2 = y.reshape(-1, self.out_features)
-            # without autograd y is this call's own: add in place
-            add = (torch.addmm if torch.is_grad_enabled()
-                   else torch.Tensor.addmm_)
-            y = add(y2, u.reshape(-1, self.r), self.lora_B.t(),
-                    beta=1.0, alpha=self.scale).view_as(y)
+            # (not addmm_, which autocast and vmap do not cover)
+            y = torch.addmm(y2, u.reshape(-1, self.r), self.lora_B.t(),
+                            beta=1.0, alpha=self.scale).view_as(y)
         return y
 
     def extra_repr(self) -> str:

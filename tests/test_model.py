@@ -169,6 +169,27 @@ def test_lora_dropout_train_eval_semantics():
     assert torch.equal(c, d)  # eval: deterministic, no dropping
 
 
+def test_lora_linear_under_autocast_and_vmap():
+    """fp32 weights without autograd: under bf16 autocast, and with one B for
+    each of several adapters."""
+    from distrl_llm_amd.models.lora import LoRALinear
+    m = LoRALinear(16, 8, True, 4, 8.0, 0.0, torch.float32)
+    g = torch.Generator().manual_seed(0)
+    x, Bs = torch.randn(3, 16, generator=g), torch.randn(5, 8, 4, generator=g)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.copy_(torch.randn(p.shape, generator=g))
+        ref = m(x)
+        with torch.autocast("cpu", torch.bfloat16):
+            y = m(x)
+        assert y.dtype == torch.bfloat16
+        torch.testing.assert_close(y.float(), ref, rtol=0.05, atol=0.2)
+        call = torch.func.functional_call
+        ys = torch.func.vmap(lambda b: call(m, {"lora_B": b}, (x,)))(Bs)
+        for y, b in zip(ys, Bs):
+            torch.testing.assert_close(y, call(m, {"lora_B": b}, (x,)))
+
+
 def test_spec_registry_resolution_and_shapes():
     """Registry name resolution for every supported family/size, and
     internal dimension consistency (published architecture shapes)."""
