@@ -19,34 +19,42 @@ from __future__ import annotations
 
 import torch
 from torch.autograd.function import once_differentiable
+from torch.nn.modules.module import _has_any_global_hook
 
 from .lora import LoRALinear
 
 
 def _hooked(module) -> bool:
-    return bool(module._forward_hooks or module._forward_pre_hooks
-                or module._backward_hooks or module._backward_pre_hooks)
+    """Whether calling the module does more than its class's forward."""
+    d = vars(module)
+    return bool(d["_forward_hooks"] or d["_forward_pre_hooks"]
+                or d["_backward_hooks"] or d["_backward_pre_hooks"]
+                or "forward" in d)
 
 
 def _trainable(mod: LoRALinear) -> bool:
-    return (mod.r > 0 and mod.weight.numel() > 0
-            and mod.weight.dtype == torch.bfloat16
-            and mod.lora_A.dtype == torch.bfloat16
-            and mod.lora_B.dtype == torch.bfloat16
-            and not mod.weight.requires_grad
-            and (mod.bias is None or not mod.bias.requires_grad)
-            and (isinstance(mod.lora_dropout, torch.nn.Identity)
-                 or not mod.training or mod.lora_dropout.p == 0.0))
+    if type(mod) is not LoRALinear or mod.r <= 0:
+        return False
+    w, b, drop, bf16 = mod.weight, mod.bias, mod.lora_dropout, torch.bfloat16
+    return (w.dtype == mod.lora_A.dtype == mod.lora_B.dtype == bf16
+            and w.numel() > 0 and not w.requires_grad
+            and (b is None or not b.requires_grad)
+            and (isinstance(drop, torch.nn.Identity)
+                 or not mod.training or drop.p == 0.0)
+            and not _hooked(drop))
 
 
 def usable(layer, x) -> bool:
     """Whether the layer's forward on x may take the fused nodes: everything
     else (CPU, other types, dropout, freed base weights, hooks on a part,
-    no adapter, inference) stays with the modules."""
+    parts of another class, no adapter, inference) stays with the modules."""
     if not (x.is_cuda and x.dtype == torch.bfloat16
-            and torch.is_grad_enabled()):
+            and torch.is_grad_enabled()) or _has_any_global_hook():
         return False
+    from .model import MLP, Attention, RMSNorm
     at, mlp = layer.self_attn, layer.mlp
+    if type(at) is not Attention or type(mlp) is not MLP:
+        return False
     linears = (at.q_proj, at.k_proj, at.v_proj, at.o_proj,
                mlp.gate_proj, mlp.up_proj, mlp.down_proj)
     norms = [layer.input_layernorm, layer.post_attention_layernorm]
@@ -54,7 +62,8 @@ def usable(layer, x) -> bool:
         norms += [at.q_norm, at.k_norm]
     return (at.spec.head_dim in (64, 128)
             and all(_trainable(m) for m in linears)
-            and all(n.weight.dtype == torch.bfloat16
+            and at.o_proj.bias is None and mlp.down_proj.bias is None
+            and all(type(n) is RMSNorm and n.weight.dtype == torch.bfloat16
                     and not n.weight.requires_grad for n in norms)
             and not any(_hooked(m) for m in (*linears, *norms, at, mlp)))
 

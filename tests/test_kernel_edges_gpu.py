@@ -389,6 +389,21 @@ def test_fused_layer_steps_aside():
     assert len(seen) == 1
     handle.remove()
     assert fused_layer.usable(layer, x)
+    handle = torch.nn.modules.module.register_module_forward_hook(
+        lambda m, i, o: seen.append(m) if m is layer.mlp.up_proj else None)
+    model.forward_hidden(torch.zeros(1, 5, dtype=torch.long, device="cuda"))
+    handle.remove()
+    assert len(seen) == 2
+    norm, layer.input_layernorm = layer.input_layernorm, torch.nn.Identity()
+    assert not fused_layer.usable(layer, x)
+    layer.input_layernorm = norm
+    layer.mlp.down_proj.bias = torch.nn.Parameter(x[0, 0].clone(), requires_grad=False)
+    assert not fused_layer.usable(layer, x)
+    layer.mlp.down_proj.bias = None
+    layer.mlp.forward = lambda y: y
+    assert not fused_layer.usable(layer, x)
+    del layer.mlp.forward
+    assert fused_layer.usable(layer, x)
     dropped = _train_model("small-qwen2", lora_dropout=0.1).model.layers[0]
     assert not fused_layer.usable(dropped, x)
     assert fused_layer.usable(dropped.eval(), x)
