@@ -130,52 +130,59 @@ class _Attention(torch.autograd.Function):
         o2 = o.transpose(1, 2).reshape(B * T, s.q_size)
         uo = o2 @ Ao.t()
         y = _residual(x, o2, uo, at.o_proj.weight, Bo, at.o_proj.scale)
+        head_norms = ((at.q_norm.weight, at.k_norm.weight) if s.qk_norm
+                      else (None, None))
         ctx.save_for_backward(x, h, A, u, Bq, Bk, Bv, Ao, Bo, q, k, v, o, lse,
-                              uo, pos, back_freq, q0, k0)
-        ctx.at, ctx.norm, ctx.shape = at, norm, shape
+                              uo, pos, back_freq, q0, k0, *head_norms,
+                              norm.weight, at.o_proj.weight,
+                              *(m.weight for m in mods))
+        ctx.spec, ctx.shape, ctx.scale = s, shape, at.scale
+        ctx.scales = [m.scale for m in (*mods, at.o_proj)]
+        ctx.eps = (norm.eps, *((at.q_norm.eps, at.k_norm.eps) if s.qk_norm
+                               else ()))
         return y
 
     @staticmethod
     @once_differentiable
     def backward(ctx, g):
         (x, h, A, u, Bq, Bk, Bv, Ao, Bo, q, k, v, o, lse, uo, pos, back_freq,
-         q0, k0) = ctx.saved_tensors
-        ext, at, norm = _ext(), ctx.at, ctx.norm
-        s, (B, T) = at.spec, ctx.shape
+         q0, k0, q_norm, k_norm, norm, Wo, *Ws) = ctx.saved_tensors
+        ext, s, (B, T) = _ext(), ctx.spec, ctx.shape
+        *scales, scale_o = ctx.scales
         g = g.contiguous()
         rows = B * T
         o2 = o.transpose(1, 2).reshape(rows, s.q_size)
 
-        duo = _scaled_mm(g, Bo, at.o_proj.scale)
-        dAo, dBo = duo.t() @ o2, _scaled_mm(g.t(), uo, at.o_proj.scale)
-        do = _add(g @ at.o_proj.weight, duo, Ao)
+        duo = _scaled_mm(g, Bo, scale_o)
+        dAo, dBo = duo.t() @ o2, _scaled_mm(g.t(), uo, scale_o)
+        do = _add(g @ Wo, duo, Ao)
         do = do.view(B, T, s.num_heads, s.head_dim).transpose(1, 2)
-        dq, dk, dv = ext.flash_attn_bwd(do, q, k, v, o, lse, at.scale)
+        dq, dk, dv = ext.flash_attn_bwd(do, q, k, v, o, lse, ctx.scale)
         dq, dk, dv = (t.transpose(1, 2).reshape(rows, -1, s.head_dim)
                       for t in (dq, dk, dv))
         # a rotation's gradient is the rotation by the negative angle
         ext.rope_inplace(dq, dk, pos, back_freq)
         if q0 is not None:
-            dq = ext.rmsnorm_bwd(dq, q0, at.q_norm.weight, at.q_norm.eps)
-            dk = ext.rmsnorm_bwd(dk, k0, at.k_norm.weight, at.k_norm.eps)
+            dq = ext.rmsnorm_bwd(dq, q0, q_norm, ctx.eps[1])
+            dk = ext.rmsnorm_bwd(dk, k0, k_norm, ctx.eps[2])
         dq, dk, dv = (t.reshape(rows, -1) for t in (dq, dk, dv))
 
         ranks = [Bq.shape[1], Bk.shape[1], Bv.shape[1]]
         du = g.new_empty(rows, sum(ranks))
         dBs = []
-        for d, m, b, p, part in zip(
-                (dq, dk, dv), (at.q_proj, at.k_proj, at.v_proj),
-                (Bq, Bk, Bv), u.split(ranks, 1), du.split(ranks, 1)):
-            _scaled_mm(d, b, m.scale, out=part)
-            dBs.append(_scaled_mm(d.t(), p, m.scale))
+        for d, scale, b, p, part in zip(
+                (dq, dk, dv), scales, (Bq, Bk, Bv), u.split(ranks, 1),
+                du.split(ranks, 1)):
+            _scaled_mm(d, b, scale, out=part)
+            dBs.append(_scaled_mm(d.t(), p, scale))
         dAq, dAk, dAv = (du.t() @ h).split(ranks)
         dx = None
         if ctx.needs_input_grad[0]:
-            dh = dq @ at.q_proj.weight
-            dh.addmm_(dk, at.k_proj.weight)
-            dh.addmm_(dv, at.v_proj.weight)
+            dh = dq @ Ws[0]
+            dh.addmm_(dk, Ws[1])
+            dh.addmm_(dv, Ws[2])
             _add(dh, du, A)
-            dx = ext.rmsnorm_bwd_add(dh, x, norm.weight, g, norm.eps)
+            dx = ext.rmsnorm_bwd_add(dh, x, norm, g, ctx.eps[0])
         return (dx, None, None, None, None, dAq, dBs[0], dAk, dBs[1],
                 dAv, dBs[2], dAo, dBo)
 
@@ -198,34 +205,37 @@ class _FeedForward(torch.autograd.Function):
         ud = act @ Ad.t()
         y = _residual(x, act, ud, mlp.down_proj.weight, Bd,
                       mlp.down_proj.scale)
-        ctx.save_for_backward(x, h, A, u, Bg, Bu, Ad, Bd, gate, up, act, ud)
-        ctx.mlp, ctx.norm = mlp, norm
+        mods = (mlp.gate_proj, mlp.up_proj, mlp.down_proj)
+        ctx.save_for_backward(x, h, A, u, Bg, Bu, Ad, Bd, gate, up, act, ud,
+                              norm.weight, *(m.weight for m in mods))
+        ctx.scales, ctx.eps = [m.scale for m in mods], norm.eps
         return y
 
     @staticmethod
     @once_differentiable
     def backward(ctx, g):
-        x, h, A, u, Bg, Bu, Ad, Bd, gate, up, act, ud = ctx.saved_tensors
-        ext, mlp, norm = _ext(), ctx.mlp, ctx.norm
+        (x, h, A, u, Bg, Bu, Ad, Bd, gate, up, act, ud, norm, Wg, Wu,
+         Wd) = ctx.saved_tensors
+        ext, (scale_g, scale_u, scale_d) = _ext(), ctx.scales
         g = g.contiguous()
-        dud = _scaled_mm(g, Bd, mlp.down_proj.scale)
-        dAd, dBd = dud.t() @ act, _scaled_mm(g.t(), ud, mlp.down_proj.scale)
-        dact = _add(g @ mlp.down_proj.weight, dud, Ad)
+        dud = _scaled_mm(g, Bd, scale_d)
+        dAd, dBd = dud.t() @ act, _scaled_mm(g.t(), ud, scale_d)
+        dact = _add(g @ Wd, dud, Ad)
         dgate, dup = ext.silu_mul_bwd(dact, gate, up)
         ranks = [Bg.shape[1], Bu.shape[1]]
         du = g.new_empty(g.shape[0], sum(ranks))
         (ug, uu), (dug, duu) = u.split(ranks, 1), du.split(ranks, 1)
-        _scaled_mm(dgate, Bg, mlp.gate_proj.scale, out=dug)
-        _scaled_mm(dup, Bu, mlp.up_proj.scale, out=duu)
-        dBg = _scaled_mm(dgate.t(), ug, mlp.gate_proj.scale)
-        dBu = _scaled_mm(dup.t(), uu, mlp.up_proj.scale)
+        _scaled_mm(dgate, Bg, scale_g, out=dug)
+        _scaled_mm(dup, Bu, scale_u, out=duu)
+        dBg = _scaled_mm(dgate.t(), ug, scale_g)
+        dBu = _scaled_mm(dup.t(), uu, scale_u)
         dAg, dAu = (du.t() @ h).split(ranks)
         dx = None
         if ctx.needs_input_grad[0]:
-            dh = dgate @ mlp.gate_proj.weight
-            dh.addmm_(dup, mlp.up_proj.weight)
+            dh = dgate @ Wg
+            dh.addmm_(dup, Wu)
             _add(dh, du, A)
-            dx = ext.rmsnorm_bwd_add(dh, x, norm.weight, g, norm.eps)
+            dx = ext.rmsnorm_bwd_add(dh, x, norm, g, ctx.eps)
         return dx, None, None, dAg, dBg, dAu, dBu, dAd, dBd
 
 

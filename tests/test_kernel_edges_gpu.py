@@ -409,6 +409,19 @@ def test_fused_layer_steps_aside():
     assert fused_layer.usable(dropped.eval(), x)
 
 
+@pytest.mark.parametrize("part", ["self_attn.k_proj", "self_attn.o_proj", "mlp.up_proj",
+                                  "mlp.down_proj", "input_layernorm", "post_attention_layernorm"])
+def test_fused_layer_notices_changed_weights(part):
+    """A weight written in place between the passes: an error, as with the
+    modules, not the gradient of another weight."""
+    model = _train_model("small-qwen2")
+    out = model.forward_hidden(torch.zeros(1, 5, dtype=torch.long, device="cuda"))
+    with torch.no_grad():
+        model.model.layers[1].get_submodule(part).weight.mul_(2.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.float().sum().backward()
+
+
 @pytest.mark.parametrize("T,H,KV,D", [(1, 1, 1, 16), (5, 14, 2, 64), (9, 28, 4, 128), (7, 3, 1, 24),
                                       (6, 4, 2, 48)])
 def test_rope_inplace_units(ext, T, H, KV, D):
