@@ -54,7 +54,8 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
   constexpr int KS = D / 32, DT = D / 16;
   const int seq = blockIdx.x, kv = blockIdx.y, z = blockIdx.z, N = gridDim.x;
   const int group = H / KV;
-  const int len = ctx_lens[seq];
+  // no further than the block table and the slices laid out for it reach
+  const int len = min(ctx_lens[seq], max_nb * block_size);
   const int c0 = z * slice_len, c1 = min(len, c0 + slice_len);
   if (z > 0 && c0 >= len) return;       // an empty slice is not read
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -229,9 +230,10 @@ __global__ __launch_bounds__(64)
 void paged_decode_combine_kernel(const float* __restrict__ o_part,
                                  const float* __restrict__ ml_part,
                                  const int* __restrict__ ctx_lens,
-                                 __hip_bfloat16* __restrict__ out, int H, int slice_len) {
+                                 __hip_bfloat16* __restrict__ out, int H, int slice_len,
+                                 int max_ctx) {
   const int seq = blockIdx.x, h = blockIdx.y, N = gridDim.x, lane = threadIdx.x;
-  const int len = ctx_lens[seq];
+  const int len = min(ctx_lens[seq], max_ctx);
   if (len <= slice_len) return;                         // written already
   const int n = (len + slice_len - 1) / slice_len;
   const int64_t head = (int64_t)seq * H + h, step = (int64_t)N * H;
@@ -278,7 +280,8 @@ void launch_decode(const torch::Tensor& q, const torch::Tensor& kcache,
                      (int)bt.size(1), block_size, shift, scale * LOG2E, q_row_stride, slice_len);
   if (cs > 1)
     hipLaunchKernelGGL((paged_decode_combine_kernel<D>), dim3(N, H), dim3(64), 0, stream, o_p,
-                       ml_p, ctx.data_ptr<int>(), o, H, slice_len);
+                       ml_p, ctx.data_ptr<int>(), o, H, slice_len,
+                       (int)bt.size(1) * block_size);
 }
 
 }  // namespace

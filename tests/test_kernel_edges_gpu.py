@@ -301,6 +301,20 @@ def test_paged_decode_edges(ext, H, KV, D, ctxs, width, bs):
             assert _rel(out[i], (p.unsqueeze(1) @ v).squeeze(1)) < DECODE_REL, (i, n)
 
 
+@pytest.mark.parametrize("N,nb", [(3, 5), (3, 129), (300, 9)])
+def test_paged_decode_stays_in_its_table(ext, N, nb):
+    """A context length beyond the block table counts as the table's end, with
+    one slice and with several."""
+    H, KV, D, bs = 8, 2, 128, 16
+    kc, vc = _rand((nb + 1, bs, KV, D), 1), _rand((nb + 1, bs, KV, D), 2)
+    bt = torch.randperm(nb, generator=torch.Generator().manual_seed(N)).int().expand(N, -1)
+    bt, q = bt.contiguous().cuda(), _rand((N, H, D), 3)
+    lens = torch.full((N,), nb * bs, dtype=torch.int32, device="cuda")
+    ref = ext.paged_attention_decode(q, kc, vc, bt, lens, 0.1)
+    lens[::2] += 3 * bs * nb + 5
+    assert torch.equal(ext.paged_attention_decode(q, kc, vc, bt, lens, 0.1), ref)
+
+
 def test_paged_decode_reads_packed_rows(ext):
     """Query heads at the head of wider rows, at any alignment."""
     H, KV, D, N = 14, 2, 64, 3
