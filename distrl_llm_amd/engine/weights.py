@@ -139,6 +139,8 @@ class FusedWeights:
     def _refresh_nf4_adapters(self, lw: "LayerWeights", layer, sites=None):
         """Per-round: stack the A matrices and build the block-diagonal,
         scale-folded B matrix per fused site, prepacked into fragments."""
+        if self.lora_r == 0:
+            return
         from ..models.quant import prepack_bf16_fragments
         at, mlp = layer.self_attn, layer.mlp
         for name, mods in (("qkv", [at.q_proj, at.k_proj, at.v_proj]),

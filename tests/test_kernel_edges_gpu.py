@@ -593,6 +593,29 @@ def test_packed_prefill_matches_modules(name, lora_r, four_bit):
     assert _rel(eng.fused.layers[1].qkv_w[q:q + model.spec.kv_size], w) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("env", [("DISTRL_HYBRID_DOWN", "1"), ("DISTRL_DECODE_NF4", "1")])
+@pytest.mark.parametrize("n", [1, 40])
+def test_four_bit_decode_without_adapter(monkeypatch, env, n):
+    """A 4-bit model with no adapter through the 4-bit kernels (few rows and
+    many) against its bf16 image: the cache rows that a decode step writes (two
+    bf16 paths of the same products: 2 %)."""
+    from distrl_llm_amd.config import EngineConfig, SamplingParams
+    from distrl_llm_amd.engine import Engine
+    from distrl_llm_amd.models import CausalLM, get_spec
+    model = CausalLM(get_spec("small-qwen2"), dtype=torch.bfloat16,
+                     device=torch.device("cuda")).random_init(3).eval()
+    model.quantize_nf4_()
+    pools = []
+    for name, value in (env, ("DISTRL_HYBRID_DOWN", "0")):
+        with monkeypatch.context() as m:
+            m.setenv(name, value)
+            eng = Engine(model, EngineConfig(max_seq_length=64, num_kv_blocks=128, max_num_seqs=64))
+            assert (eng.fused.nf4 or eng.fused.hybrid_down) == (value == "1")
+            eng.generate([[1, 2, 3, 4, 5]], SamplingParams(max_tokens=2, temperature=0.0, n=n))
+            pools.append(torch.stack([eng.pool.key, eng.pool.value]))
+    assert _rel(*pools) < 0.02
+
+
 # ------------------------------------------------------------------- loss
 
 @pytest.mark.parametrize("B,T,V,dtype", [
