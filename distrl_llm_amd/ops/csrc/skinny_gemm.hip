@@ -162,7 +162,11 @@ void skinny_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat
   }
 }
 
-bool aligned16(const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+// An operand as 16 B loads can read it: a parameter cut out of a larger buffer
+// may start anywhere.
+torch::Tensor at16(const torch::Tensor& t) {
+  return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.clone();
+}
 
 const __hip_bfloat16* ptr(const torch::Tensor& t) {
   return reinterpret_cast<const __hip_bfloat16*>(t.data_ptr());
@@ -182,17 +186,20 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
                           c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> res,
                           c10::optional<torch::Tensor> norm_w, double eps,
                           c10::optional<torch::Tensor> u, c10::optional<torch::Tensor> ub) {
-  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() && aligned16(x));
-  TORCH_CHECK(w.is_cuda() && w.dim() == 2 && w.is_contiguous() && aligned16(w));
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous());
+  TORCH_CHECK(w.is_cuda() && w.dim() == 2 && w.is_contiguous());
   TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16);
   TORCH_CHECK(mode >= PLAIN && mode <= GLU && w.size(1) == x.size(1));
   const int M = x.size(0), K = x.size(1), N = mode == GLU ? w.size(0) / 2 : w.size(0);
   TORCH_CHECK(mode != GLU || w.size(0) % 2 == 0);
   TORCH_CHECK(skinny_gemm_takes(M, N, K), "skinny_gemm: unsupported shape (", M, ", ", N, ", ", K, ")");
-  auto check = [&](const c10::optional<torch::Tensor>& t, int64_t n, const char* what) {
+  x = at16(x);
+  w = at16(w);
+  auto check = [&](c10::optional<torch::Tensor>& t, int64_t n, const char* what) {
     if (!t) return (const __hip_bfloat16*)nullptr;
     TORCH_CHECK(t->is_cuda() && t->is_contiguous() && t->scalar_type() == at::kBFloat16 &&
-                t->numel() == n && aligned16(*t), "skinny_gemm: ", what);
+                t->numel() == n, "skinny_gemm: ", what);
+    t = at16(*t);
     return ptr(*t);
   };
   const auto* b = check(bias, N, "bias");

@@ -491,6 +491,25 @@ def test_skinny_gemm(ext, M, N, K):
                     inp @ wd.double().t() + b.double()) < bound
 
 
+def test_skinny_gemm_operands_anywhere(ext):
+    """Each operand in turn at an odd element of a buffer: the same results."""
+    M, N, K, R = 5, 64, 512, 32
+
+    def odd(t):
+        flat = t.new_empty(t.numel() + 1)
+        flat[1:] = t.reshape(-1)
+        return flat[1:].view(t.shape)
+
+    ops = {"x": _rand((M, K), 1), "w": _rand((N, K), 2, 0.05), "bias": _rand((N,), 3),
+           "norm_w": _rand((K,), 4), "res": _rand((M, N), 5), "u": _rand((M, R), 6),
+           "ub": _rand((N, R), 7)}
+    for mode, names in ((0, ("x", "w", "bias", "norm_w")), (1, ("x", "w", "res", "u", "ub"))):
+        ref = ext.skinny_gemm(mode=mode, eps=1e-6, **{n: ops[n] for n in names})
+        for name in names:
+            args = {n: odd(ops[n]) if n == name else ops[n] for n in names}
+            assert torch.equal(ext.skinny_gemm(mode=mode, eps=1e-6, **args), ref), name
+
+
 @pytest.mark.parametrize("D,H,KV", [(64, 3, 1), (128, 28, 4)])
 def test_rope_scatter_norms(ext, D, H, KV):
     """Per-head norms, rotation and cache write of packed projections, a
