@@ -218,6 +218,9 @@ class FusedWeights:
                 self.layers.append(lw)
             else:
                 lw = self.layers[li]
+                if lw.qkv_b is not None:
+                    torch.cat([at.q_proj.bias, at.k_proj.bias,
+                               at.v_proj.bias], out=lw.qkv_b)
             if self.nf4:
                 if first:
                     self._build_nf4_base(lw, layer)

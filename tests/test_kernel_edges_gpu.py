@@ -612,6 +612,29 @@ def test_packed_prefill_matches_modules(name, lora_r, four_bit):
     assert _rel(eng.fused.layers[1].qkv_w[q:q + model.spec.kv_size], w) < 2.0 ** -8
 
 
+def test_packed_prefill_after_a_changed_bias():
+    """Weights and biases written in place between two generations."""
+    from distrl_llm_amd.config import EngineConfig
+    from distrl_llm_amd.engine import Engine
+    from distrl_llm_amd.engine.kvcache import Sequence
+    from distrl_llm_amd.models import CausalLM, get_spec
+    model = CausalLM(get_spec("small-qwen2"), dtype=torch.bfloat16,
+                     device=torch.device("cuda")).random_init(3).eval()
+    eng = Engine(model, EngineConfig(max_seq_length=64, num_kv_blocks=32, max_num_seqs=8))
+    eng.fused.refresh()
+    at = model.model.layers[0].self_attn
+    with torch.no_grad():
+        at.k_proj.bias.add_(3.0)
+        at.v_proj.weight.mul_(-1.0)
+    eng.fused.refresh()
+    logits = [eng._prefill_batch([Sequence(0, [5, 6, 7], 0)])]
+    key = eng.pool.key.clone()
+    eng._prefill_packs = lambda: False
+    eng.pool.allocator.reset()
+    logits.append(eng._prefill_batch([Sequence(1, [5, 6, 7], 1)]))
+    assert _rel(*logits) < 0.02 and _rel(key, eng.pool.key) < 0.02
+
+
 @pytest.mark.parametrize("env", [("DISTRL_HYBRID_DOWN", "1"), ("DISTRL_DECODE_NF4", "1")])
 @pytest.mark.parametrize("n", [1, 40])
 def test_four_bit_decode_without_adapter(monkeypatch, env, n):
