@@ -279,7 +279,24 @@ class Engine:
         return (self.device.type == "cuda" and self.dtype == torch.bfloat16
                 and f is not None and f._built and not f.nf4
                 and s.head_dim in (64, 128)
-                and os.environ.get("DISTRL_PREFILL_VARLEN") != "1")
+                and os.environ.get("DISTRL_PREFILL_VARLEN") != "1"
+                and not self._prefill_hooked())
+
+    def _prefill_hooked(self) -> bool:
+        """Whether a module that the packed rows pass by has hooks."""
+        from ..models.fused_layer import _hooked, _has_any_global_hook
+        if _has_any_global_hook() or _hooked(self.model.model.norm):
+            return True
+        for layer in self.model.model.layers:
+            at, mlp = layer.self_attn, layer.mlp
+            linears = (at.q_proj, at.k_proj, at.v_proj, at.o_proj,
+                       mlp.gate_proj, mlp.up_proj, mlp.down_proj)
+            if any(map(_hooked, (layer.input_layernorm, *linears,
+                                 layer.post_attention_layernorm))):
+                return True
+            if any(m.r > 0 and _hooked(m.lora_dropout) for m in linears):
+                return True
+        return False
 
     def _prefill_packed(self, input_ids, positions, slots, lens):
         """The layers over one flat batch of prompts -> normed hidden states.
@@ -327,10 +344,11 @@ class Engine:
             q, k, v = (t.unflatten(1, (-1, D))
                        for t in qkv.split([qs, kvs, kvs], 1))
             o = ext.flash_attn_varlen(q, k, v, cu, max(lens), self.scale)
-            o = self._proj(at.o_proj, o.view(T, qs))
+            o = packed(o.view(T, qs), (at.o_proj,), lw.o_w, None)
             h, res = ext.add_rmsnorm_fwd(res, o, lw.post_norm, eps)
             gu = packed(h, (mlp.gate_proj, mlp.up_proj), lw.gateup_w, None)
-            d = self._proj(mlp.down_proj, ext.silu_mul_packed(gu))
+            d = packed(ext.silu_mul_packed(gu), (mlp.down_proj,), lw.down_w,
+                       None)
             last = li + 1 == len(self.fused.layers)
             h, res = ext.add_rmsnorm_fwd(
                 res, d, m.model.norm.weight if last

@@ -635,6 +635,32 @@ def test_packed_prefill_after_a_changed_bias():
     assert _rel(*logits) < 0.02 and _rel(key, eng.pool.key) < 0.02
 
 
+@pytest.mark.parametrize("part", ["layers.1.self_attn.q_proj", "layers.0.mlp.down_proj", "norm",
+                                  "layers.1.input_layernorm", None])
+def test_packed_prefill_leaves_hooks_their_modules(part):
+    """A hook on a module, or on all of them, sees the prompt's rows."""
+    from distrl_llm_amd.config import EngineConfig, SamplingParams
+    from distrl_llm_amd.engine import Engine
+    from distrl_llm_amd.models import CausalLM, get_spec
+    model = CausalLM(get_spec("small-qwen2"), lora_r=8, dtype=torch.bfloat16,
+                     device=torch.device("cuda")).random_init(3).eval()
+    eng = Engine(model, EngineConfig(max_seq_length=64, num_kv_blocks=32, max_num_seqs=8))
+    mod, seen = model.model.get_submodule(part or "layers.0.mlp.gate_proj"), []
+
+    def hook(m, i, o):
+        if m is mod:
+            seen.append(o.shape[0])
+
+    handle = (mod.register_forward_hook(hook) if part
+              else torch.nn.modules.module.register_module_forward_hook(hook))
+    try:
+        eng.generate([[5, 6, 7]], SamplingParams(max_tokens=2, temperature=0.0))
+    finally:
+        handle.remove()
+    assert seen == [3]
+    assert eng._prefill_packs()
+
+
 @pytest.mark.parametrize("env", [("DISTRL_HYBRID_DOWN", "1"), ("DISTRL_DECODE_NF4", "1")])
 @pytest.mark.parametrize("n", [1, 40])
 def test_four_bit_decode_without_adapter(monkeypatch, env, n):
