@@ -287,7 +287,9 @@ class CausalLM(nn.Module):
             rotary = (position_ids.reshape(-1).to(torch.int32), inv_freq, -inv_freq)
         x = self.model.embed_tokens(input_ids)
         for layer in self.model.layers:
-            x = layer(x, cos, sin, bias, rotary)
+            # a layer of another class takes what the modules need
+            x = (layer(x, cos, sin, bias, rotary)
+                 if isinstance(layer, DecoderLayer) else layer(x, cos, sin, bias))
         return self.model.norm(x)
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:

@@ -169,6 +169,27 @@ def test_lora_dropout_train_eval_semantics():
     assert torch.equal(c, d)  # eval: deterministic, no dropping
 
 
+def test_forward_with_wrapped_layers(tiny_model):
+    """A layer replaced by a module around it, which takes a decoder layer's
+    four arguments."""
+    class Around(torch.nn.Module):
+        def __init__(self, layer):
+            super().__init__()
+            self.layer = layer
+
+        def forward(self, x, cos, sin, attn_bias):
+            return self.layer(x, cos, sin, attn_bias)
+
+    ids = torch.randint(0, 2048, (1, 6))
+    ref = tiny_model(ids)
+    layers = tiny_model.model.layers
+    layers[0] = Around(layers[0])
+    try:
+        assert torch.equal(tiny_model(ids), ref)
+    finally:
+        layers[0] = layers[0].layer
+
+
 def test_lora_linear_under_autocast_and_vmap():
     """fp32 weights without autograd: under bf16 autocast, and with one B for
     each of several adapters."""
