@@ -35,8 +35,8 @@ namespace {
 constexpr int KC = 256;            // columns of a workgroup
 constexpr int STEPS = KC / 32;     // loads of W in flight
 
-// w and out may be one; res (or none) is added to the same sum; rows of w and out are ldw elements apart, those of b
-// ldb. TA: a is (K, r).
+// w and out may be one; res (or none) is added to the same sum. Rows of w and
+// out are ldw elements apart, those of b ldb. TA: a is (K, r).
 template <bool TA>
 __global__ __launch_bounds__(256)
 void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict__ a,
@@ -146,6 +146,7 @@ bool launch_merge(const torch::Tensor& w, const torch::Tensor& a, const torch::T
       !lrows(w) || !lrows(b) || !lrows(out) || !lrows(a) || !a.is_contiguous() ||
       w.stride(0) != out.stride(0))
     return false;
+  if (N > 1 && out.stride(0) < K) return false;         // rows over one another
   if (res && (!lrows(*res) || res->sizes() != w.sizes())) return false;
   if (N == 0) return true;
   // 4096 tiles fill the chip eight deep: then a staged A serves four turns,

@@ -571,6 +571,10 @@ def test_lora_add(ext, M, N, r):
     assert not ext.lora_add(wide[:, :N], uw[:, 4:4 + r], m, 0.5)
     assert not ext.lora_add(wide[:, :N], uw[:, :r].float(), m, 0.5)
     assert not ext.lora_add(wide[:, :N], uw[:, :r], m.flip(0)[:, ::2], 0.5)
+    if M > 1:
+        same, over = _rand((1, N), 5).expand(M, N), _rand((M * 32 + N,), 6).as_strided((M, N), (16, 1))
+        for y in (same, over):
+            assert not ext.lora_add(y, uw[:, 16:16 + r], m, 0.5)
     assert torch.equal(wide[:, :32], before[:, :32])
 
 
