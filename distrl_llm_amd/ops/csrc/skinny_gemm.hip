@@ -1,4 +1,4 @@
-// Products of a decode step with few rows: y = x W^T for M <= 64 rows,
+// Products of a decode step with few rows: y = x W^T for M <= 32 rows,
 // W (N, K) bf16, fp32 sums, with what stands around the product in the same
 // launch: the RMS norm of x before it; bias, residual sum or SiLU*mul after it.
 //
@@ -177,7 +177,7 @@ const __hip_bfloat16* ptr(const torch::Tensor& t) {
 // Whether skinny_gemm takes the shape: rows of x, columns of y (the activation's
 // for SiLU*mul), K.
 bool skinny_gemm_takes(int64_t M, int64_t N, int64_t K) {
-  return M >= 1 && M <= 64 && N >= 16 && N % 16 == 0 && K >= 512 && K % 32 == 0;
+  return M >= 1 && M <= 32 && N >= 16 && N % 16 == 0 && K >= 512 && K % 32 == 0;
 }
 
 // mode 0: x W^T (+ bias); 1: res + x W^T (+ u ub^T); 2: silu(x Wg^T) * (x Wu^T)
@@ -223,9 +223,8 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
   // Fewer rows a workgroup reach more CUs but re-read x; more waves shorten
   // the chain of loads until joining them costs more.
   const int tiles = N / 16, steps = K / 32, tr = tiles <= 128 ? 8 : 16;
-  int kw = tiles <= 256 ? (steps >= 64 ? 16 : steps >= 32 ? 8 : 4)
+  const int kw = tiles <= 256 ? (steps >= 64 ? 16 : steps >= 32 ? 8 : 4)
                         : (mode == GLU && steps >= 48 ? 8 : 4);
-  if (mode == GLU && M > 32) kw = std::min(kw, 8);     // 64 KB of partial sums
   auto go = [&](auto mt_, auto kw_, auto mode_, auto norm_) {
     constexpr int MT = decltype(mt_)::value, KW = decltype(kw_)::value,
                   MODE = decltype(mode_)::value;
@@ -249,8 +248,7 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
   };
   TORCH_CHECK(mode != RESIDUAL || !nw, "skinny_gemm: norm with a residual sum");
   if (M <= 16) by_kw(std::integral_constant<int, 1>{});
-  else if (M <= 32) by_kw(std::integral_constant<int, 2>{});
-  else by_kw(std::integral_constant<int, 4>{});
+  else by_kw(std::integral_constant<int, 2>{});
   HIP_CHECK_LAST();
   return y;
 }

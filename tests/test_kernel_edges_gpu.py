@@ -466,7 +466,7 @@ def test_rmsnorm_bwd_add(ext, rows, hidden):
 
 # ------------------------------------------------------------ skinny products
 
-@pytest.mark.parametrize("M", [1, 8, 15, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("M", [1, 8, 15, 16, 17, 32])
 @pytest.mark.parametrize("N,K", [(16, 512), (896, 896), (2064, 544), (4112, 4864), (256, 8960)])
 def test_skinny_gemm(ext, M, N, K):
     """Every wave count and row tile, K that does not divide among the waves;
@@ -483,6 +483,7 @@ def test_skinny_gemm(ext, M, N, K):
     assert _rel(ext.skinny_gemm(x, wd, 1, res=res), ref) < 2.0 ** -8
     assert _rel(ext.skinny_gemm(x, wd, 1, res=res, u=u, ub=ub),
                 ref + u.double() @ ub.double().t()) < 2.0 ** -8
+    assert not ext.skinny_gemm_takes(33, N, K)          # one row further
     normed = xd * torch.rsqrt((xd * xd).mean(-1, keepdim=True) + 1e-6) * nw.double()
     for inp, kw, bound in ((xd, {}, 2.0 ** -7), (normed, {"norm_w": nw, "eps": 1e-6}, 2.0 ** -6)):
         gate, up = (inp @ w.double().t()).chunk(2, -1)
