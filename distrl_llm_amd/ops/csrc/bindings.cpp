@@ -41,10 +41,6 @@ torch::Tensor sample_tokens(torch::Tensor logits, double temperature,
                             torch::Tensor step);
 std::vector<torch::Tensor> logprob_lse_fwd(torch::Tensor logits,
                                            torch::Tensor targets);
-std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits,
-                                            torch::Tensor targets,
-                                            torch::Tensor mask,
-                                            torch::Tensor rewards, double scale);
 torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets,
                                torch::Tensor w, torch::Tensor lse,
                                c10::optional<torch::Tensor> dloss);
@@ -113,11 +109,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "paged GQA decode attention");
   m.def("sample_tokens", &sample_tokens,
         "fused temperature/top-k/top-p categorical sampling");
-  m.def("sample_tokens2", &sample_tokens, "sample_tokens by its other name");
   m.def("logprob_lse_fwd", &logprob_lse_fwd,
         "per-token log p(target) + LSE, one streaming pass");
-  m.def("logprob_loss_fwd", &logprob_loss_fwd,
-        "masked PG/GRPO loss, its row weights and the LSE");
   m.def("logprob_loss_bwd", &logprob_loss_bwd,
         "dlogits for the masked PG/GRPO loss", py::arg("logits"),
         py::arg("targets"), py::arg("w"), py::arg("lse"),

@@ -207,9 +207,9 @@ std::vector<torch::Tensor> logprob_lse_fwd(torch::Tensor logits,
 
 // The masked PG/GRPO loss of logits (B, T, V): {loss, row weights (B, T), lse}.
 // mask int64 or fp32, rewards fp32.
-std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits, torch::Tensor targets,
-                                            torch::Tensor mask, torch::Tensor rewards,
-                                            double scale) {
+static std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits, torch::Tensor targets,
+                                                   torch::Tensor mask, torch::Tensor rewards,
+                                                   double scale) {
   TORCH_CHECK(logits.dim() == 3 && mask.is_cuda() && rewards.is_cuda());
   const int B = logits.size(0), T = logits.size(1);
   TORCH_CHECK(mask.numel() == (int64_t)B * T && targets.numel() == (int64_t)B * T &&

@@ -135,8 +135,7 @@ def test_paged_attention_decode(ext, D, H, KV, ctxs):
 
 # -------------------------------------------------------------- sampling
 
-@pytest.mark.parametrize("impl", ["sample_tokens", "sample_tokens2"])
-def test_sample_tokens_distribution(ext, impl):
+def test_sample_tokens_distribution(ext):
     """Statistical check: a peaked 3-token distribution sampled many times
     matches the renormalized top-p categorical within tolerance."""
     torch.manual_seed(6)
@@ -149,7 +148,7 @@ def test_sample_tokens_distribution(ext, impl):
     rows = logits.expand(n, V).contiguous()
     seeds = torch.arange(n, device=_dev(), dtype=torch.int64) * 7919 + 13
     step = torch.zeros(1, dtype=torch.int64, device=_dev())
-    fn = getattr(ext, impl)
+    fn = ext.sample_tokens
     out = fn(rows, 1.0, 1.0, 0, seeds, step)
     counts = torch.bincount(out.cpu(), minlength=V).float() / n
     assert abs(counts[10] - 0.6) < 0.04
@@ -169,15 +168,14 @@ def test_sample_tokens_distribution(ext, impl):
     assert (out3 == 10).all()
 
 
-@pytest.mark.parametrize("impl", ["sample_tokens", "sample_tokens2"])
-def test_sample_tokens_temperature(ext, impl):
+def test_sample_tokens_temperature(ext):
     V = 128
     logits = torch.zeros(2000, V, device=_dev())
     logits[:, 5] = 2.0
     seeds = torch.arange(2000, device=_dev(), dtype=torch.int64)
     step = torch.zeros(1, dtype=torch.int64, device=_dev())
     # low temperature sharpens: nearly all mass on token 5
-    out = getattr(ext, impl)(logits, 0.05, 1.0, 0, seeds, step)
+    out = ext.sample_tokens(logits, 0.05, 1.0, 0, seeds, step)
     assert (out == 5).float().mean() > 0.99
 
 
