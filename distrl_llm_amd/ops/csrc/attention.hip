@@ -35,7 +35,7 @@
 // split over workgroups that leave fp32 partials for a small sum kernel.
 //
 // Measured at B 16, 28/4 heads, T 1550, D 128 (275 GFLOP in the causal half,
-// forward): forward 425 us = 650 TFLOP/s, dQ 597 us, dK/dV 1208 us + 39 us for
+// forward): forward 440 us = 625 TFLOP/s, dQ 597 us, dK/dV 1208 us + 39 us for
 // the sum; 16-row waves on 16x16x32 with single-buffered tiles and transposed
 // copies of q, k, v, dout took 1161, 2097 and 3466 us + 1.9 ms of copies and
 // sums. What bounds them now: vector work beside the products (10 vector

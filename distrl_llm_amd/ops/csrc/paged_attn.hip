@@ -54,9 +54,9 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
   constexpr int KS = D / 32, DT = D / 16;
   const int seq = blockIdx.x, kv = blockIdx.y, z = blockIdx.z, N = gridDim.x;
   const int group = H / KV;
-  // no further than the block table and the slices laid out for it reach
-  const int len = min(ctx_lens[seq], max_nb * block_size);
-  const int c0 = z * slice_len, c1 = min(len, c0 + slice_len);
+  const int len = ctx_lens[seq];
+  // no further than the block table reaches
+  const int c0 = z * slice_len, c1 = min(len, min(c0 + slice_len, max_nb * block_size));
   if (z > 0 && c0 >= len) return;       // an empty slice is not read
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63, g = l >> 4, lr = l & 15;
@@ -148,7 +148,9 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
       }
     mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
     mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
-    // the subtracted maximum may lag by 2^8 (see the rescaling's cost)
+    // The subtracted maximum may lag by 2^8: rescaling the sums at every chunk
+    // would cost as much as weighing V. The weights' two terms carry 17 bits
+    // whatever their size, so nothing is lost by it.
     if (__any(mx > m + 8.f)) {
       const float m_new = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - m_new);
       lsum *= alpha;
@@ -194,7 +196,7 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
   for (int dt = 0; dt < DT; ++dt)
     *reinterpret_cast<f32x4*>(o_tile + lr * D + dt * 16 + g * 4) = acc[dt];
   __syncthreads();
-  const bool whole = len <= slice_len;                  // nothing to join outside
+  const bool whole = len <= slice_len || gridDim.z == 1;  // nothing to join outside
   for (int i = threadIdx.x; i < group * (D / 4); i += NW * 64) {
     const int h = i / (D / 4), d = i % (D / 4) * 4;
     float top = -1e30f, total = 0.f;
@@ -231,11 +233,11 @@ void paged_decode_combine_kernel(const float* __restrict__ o_part,
                                  const float* __restrict__ ml_part,
                                  const int* __restrict__ ctx_lens,
                                  __hip_bfloat16* __restrict__ out, int H, int slice_len,
-                                 int max_ctx) {
+                                 int cs) {
   const int seq = blockIdx.x, h = blockIdx.y, N = gridDim.x, lane = threadIdx.x;
-  const int len = min(ctx_lens[seq], max_ctx);
+  const int len = ctx_lens[seq];
   if (len <= slice_len) return;                         // written already
-  const int n = (len + slice_len - 1) / slice_len;
+  const int n = min((len + slice_len - 1) / slice_len, cs);
   const int64_t head = (int64_t)seq * H + h, step = (int64_t)N * H;
   float top = -1e30f;
   for (int z = 0; z < n; ++z) top = fmaxf(top, ml_part[(z * step + head) * 2]);
@@ -280,8 +282,7 @@ void launch_decode(const torch::Tensor& q, const torch::Tensor& kcache,
                      (int)bt.size(1), block_size, shift, scale * LOG2E, q_row_stride, slice_len);
   if (cs > 1)
     hipLaunchKernelGGL((paged_decode_combine_kernel<D>), dim3(N, H), dim3(64), 0, stream, o_p,
-                       ml_p, ctx.data_ptr<int>(), o, H, slice_len,
-                       (int)bt.size(1) * block_size);
+                       ml_p, ctx.data_ptr<int>(), o, H, slice_len, cs);
 }
 
 }  // namespace
@@ -319,6 +320,10 @@ torch::Tensor paged_attention_decode_strided(
   // as long: few sequences run with eight waves in slices of 512 tokens, up to
   // one workgroup a CU (16 sequences of 1500, 4 kv heads: 1 slice 25 us, 2: 18,
   // 4: 14, 6: 19; 8 sequences of 4000, 8 kv heads: 63, 39, 29, 8 slices 34).
+  // From 129 workgroups on one slice is left of that, right up to some 2000
+  // tokens (40 sequences of 1550, 4 kv heads: 26, 2: 32, 4: 35; 30 of 500, 8 kv
+  // heads: 13, 2: 18) and up to a fifth too slow beyond (33 of 4000, 4 kv heads:
+  // 61, 3: 55, 4: 51; 63 of them: 89, 2: 91, 4: 96).
   // More sequences fill the chip by themselves; two slices even out their
   // lengths where they are long (the round above: 1 slice 80 us, 2: 76, 4: 79;
   // 32 sequences of 700, 8 kv heads: 16, 18, 21).
