@@ -18,11 +18,11 @@
 // and the draw, whose last slice of a row writes the token. A thread adds into
 // histogram columns of its own, so nothing collides and no atomics are needed:
 // LDS float atomics into 1024 shared bins took ~3 clocks a lane (124 us for
-// 160 rows of 152064), the two passes take 42 us.
+// 160 rows of 152064), the two passes take 44 us.
 // An element that is kept costs ~330 cycles of hashing a wave, so sparse ones
 // are gathered into full waves first. 160 rows of 152064 at top_p 0.95: 284 us
-// as eight launches with one serial thread a row for the threshold, 94 us now
-// (draw 46, histograms 42, maximum 6), bound by the draw's integer products;
+// as eight launches with one serial thread a row for the threshold, 95 us now
+// (draw 46, histograms 44, maximum 9), bound by the draw's integer products;
 // one row of 151936 without a threshold 24.6 -> 11.3 us, bound by two launches.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
