@@ -313,9 +313,11 @@ class Engine:
         cu = torch.tensor([0] + lens, dtype=torch.int32).cumsum(0) \
             .to(torch.int32).to(self.device)
 
-        def packed(x, mods, merged, bias):
+        def packed(x, lw, site):
+            mods = lw.mods[site]
             if all(mod.r == 0 for mod in mods):
-                return F.linear(x, merged, bias)
+                return F.linear(x, lw.rows(site),
+                                lw.qkv_b if site == "qkv" else None)
             out = x.new_empty(T, sum(mod.out_features for mod in mods))
             for mod, y in zip(mods, out.split([mod.out_features
                                                for mod in mods], 1)):
@@ -333,9 +335,8 @@ class Engine:
         h = ext.rmsnorm_fwd(res, self.fused.layers[0].in_norm, eps)
         for li, (layer, lw) in enumerate(zip(m.model.layers,
                                              self.fused.layers)):
-            at, mlp = layer.self_attn, layer.mlp
-            qkv = packed(h, (at.q_proj, at.k_proj, at.v_proj), lw.qkv_w,
-                         lw.qkv_b)
+            at = layer.self_attn
+            qkv = packed(h, lw, "qkv")
             norms = ((at.q_norm.weight, at.k_norm.weight, eps)
                      if s.qk_norm else ())
             ext.rope_scatter_qkv(qkv, pos32, slots, self._inv_freq,
@@ -344,11 +345,10 @@ class Engine:
             q, k, v = (t.unflatten(1, (-1, D))
                        for t in qkv.split([qs, kvs, kvs], 1))
             o = ext.flash_attn_varlen(q, k, v, cu, max(lens), self.scale)
-            o = packed(o.view(T, qs), (at.o_proj,), lw.o_w, None)
+            o = packed(o.view(T, qs), lw, "o")
             h, res = ext.add_rmsnorm_fwd(res, o, lw.post_norm, eps)
-            gu = packed(h, (mlp.gate_proj, mlp.up_proj), lw.gateup_w, None)
-            d = packed(ext.silu_mul_packed(gu), (mlp.down_proj,), lw.down_w,
-                       None)
+            gu = packed(h, lw, "gateup")
+            d = packed(ext.silu_mul_packed(gu), lw, "down")
             last = li + 1 == len(self.fused.layers)
             h, res = ext.add_rmsnorm_fwd(
                 res, d, m.model.norm.weight if last
@@ -479,10 +479,11 @@ class Engine:
         """Single-token batched decode forward over device-side state —
         the hipGraph-capturable step body (all inputs are device tensors).
 
-        GPU path: merged-LoRA fused weights (one qkv GEMM, one gate|up
-        GEMM per layer), fused rope+KV-scatter, strided-q paged attention,
-        fused residual-add+RMSNorm and packed SiLU*mul — 9 kernels/layer;
-        about six for few sequences, on skinny products.
+        GPU path: merged-LoRA fused weights (one qkv and one gate|up product
+        a layer), rotation with the cache write, strided-q paged attention,
+        residual sum with the norm. Up to 16 sequences run on skinny
+        products, up to 160 on streamed ones, both on weights in tiles; more
+        on the library's.
         """
         if self.device.type == "cuda":
             return self._decode_forward_fused(input_ids, positions,
@@ -532,9 +533,12 @@ class Engine:
         # kernels accumulate into per-(layer, site) slices)
         hybrid_down = (not nf4) and getattr(self.fused, "hybrid_down", False)
         skinny = not nf4 and self._skinny(N_batch)
+        streamed = not skinny and self._streamed(N_batch)
+        if hybrid_down and not skinny and not streamed:
+            self.fused.ensure_nf4_down()
         u_pool = None
         site_off = {}
-        if (nf4 or hybrid_down) and r > 0 and not skinny:
+        if (nf4 or hybrid_down) and r > 0 and not skinny and not streamed:
             off = 0
             for site in (("qkv", "o", "gateup", "down") if nf4
                          else ("down",)):
@@ -562,9 +566,8 @@ class Engine:
             the down site runs the fused nf4 kernel even in merged mode —
             it beats hipBLASLt on that deep-K shape)."""
             if not nf4 and not (hybrid_down and site == "down"):
-                if site == "qkv":
-                    return F.linear(x, lw.qkv_w, lw.qkv_b)
-                return F.linear(x, getattr(lw, f"{site}_w"))
+                return F.linear(x, lw.rows(site),
+                                lw.qkv_b if site == "qkv" else None)
             bias = lw.qkv_b if site == "qkv" else None
             if r > 0:
                 o0, rt = site_off[site]
@@ -582,41 +585,77 @@ class Engine:
                                 getattr(lw, f"{site}_amax"), bias, None,
                                 None, N_out, K_in, 0)
 
+        def head_norms(li):
+            """The norm weights are engine-lifetime parameter storages, so
+            captured graphs stay valid."""
+            if not s.qk_norm:
+                return ()
+            at = m.model.layers[li].self_attn
+            return at.q_norm.weight, at.k_norm.weight, eps
+
         def attend(qkv, li):
             """Rotation, cache write and attention of one layer's packed
-            projections (in place); the norm weights are engine-lifetime
-            parameter storages, so captured graphs stay valid."""
-            norms = ()
-            if s.qk_norm:
-                at = m.model.layers[li].self_attn
-                norms = (at.q_norm.weight, at.k_norm.weight, eps)
+            projections (in place)."""
             ext.rope_scatter_qkv(qkv, pos32, slot_mapping, self._inv_freq,
                                  self.pool.key[li], self.pool.value[li],
                                  s.num_heads, s.num_kv_heads, s.head_dim,
-                                 *norms)
+                                 *head_norms(li))
             return ext.paged_attention_decode_strided(
                 qkv, s.num_heads, s.head_dim, qs + 2 * kvs,
                 self.pool.key[li], self.pool.value[li], block_tables,
                 context_lens, self.scale).view(-1, qs)
 
         res = m.model.embed_tokens(input_ids)
+        apart = hybrid_down and r > 0
         if skinny:
             # few sequences: the products carry the norms, the residual sums
             # and the activation along
+            t = self.fused.tiled
+
+            def weight(lw, site):
+                return lw.tiles[site] if t else lw.rows(site)
+
             for li, lw in enumerate(lws):
-                qkv = ext.skinny_gemm(res, lw.qkv_w, 0, bias=lw.qkv_b,
-                                      norm_w=lw.in_norm, eps=eps)
-                res = ext.skinny_gemm(attend(qkv, li), lw.o_w, 1, res=res)
-                act = ext.skinny_gemm(res, lw.gateup_w, 2,
-                                      norm_w=lw.post_norm, eps=eps)
-                if hybrid_down and r > 0:
+                qkv = ext.skinny_gemm(res, weight(lw, "qkv"), 0, bias=lw.qkv_b,
+                                      norm_w=lw.in_norm, eps=eps, tiles=t)
+                res = ext.skinny_gemm(attend(qkv, li), weight(lw, "o"), 1,
+                                      res=res, tiles=t)
+                act = ext.skinny_gemm(res, weight(lw, "gateup"), 2,
+                                      norm_w=lw.post_norm, eps=eps, tiles=t)
+                if apart:
                     # the 4-bit site keeps its adapter beside the base image
-                    u = ext.skinny_gemm(act, lw.down_a, 0)
-                    res = ext.skinny_gemm(act, lw.down_base, 1, res=res, u=u,
-                                          ub=lw.down_b)
+                    u = ext.skinny_gemm(act, lw.down_a, 0, tiles=t)
+                    base = lw.tiles["down"] if t else lw.mods["down"][0].weight
+                    res = ext.skinny_gemm(act, base, 1, res=res, u=u,
+                                          ub=lw.down_b, tiles=t)
                 else:
-                    res = ext.skinny_gemm(act, lw.down_w, 1, res=res)
+                    res = ext.skinny_gemm(act, weight(lw, "down"), 1, res=res,
+                                          tiles=t)
             return m.logits(ext.rmsnorm_fwd(res, m.model.norm.weight, eps))
+
+        if streamed:
+            h = ext.rmsnorm_fwd(res, lws[0].in_norm, eps)
+            for li, lw in enumerate(lws):
+                q = ext.rope_scatter_join(
+                    ext.stream_gemm(h, lw.tiles["qkv"]), lw.qkv_b, pos32,
+                    slot_mapping, self._inv_freq, self.pool.key[li],
+                    self.pool.value[li], s.num_heads, s.num_kv_heads,
+                    s.head_dim, *head_norms(li))
+                o = ext.paged_attention_decode_strided(
+                    q, s.num_heads, s.head_dim, qs, self.pool.key[li],
+                    self.pool.value[li], block_tables, context_lens,
+                    self.scale).view(-1, qs)
+                h, res = ext.add_rmsnorm_join(
+                    ext.stream_gemm(o, lw.tiles["o"]), res, lw.post_norm, eps)
+                act = ext.stream_glu(h, lw.tiles["gateup"])
+                next_w = (lws[li + 1].in_norm if li + 1 < len(lws)
+                          else m.model.norm.weight)
+                # the 4-bit site's adapter: more rows of W, joined in fp32
+                h, res = ext.add_rmsnorm_join(
+                    ext.stream_gemm(act, lw.tiles["down"],
+                                    lw.down_a if apart else None),
+                    res, next_w, eps, lw.down_bt if apart else None)
+            return m.logits(h)
 
         h = ext.rmsnorm_fwd(res, lws[0].in_norm, eps)
         for li, lw in enumerate(lws):
@@ -647,6 +686,22 @@ class Engine:
                 and fits(n, s.hidden_size, s.q_size)
                 and fits(n, s.intermediate_size, s.hidden_size)
                 and fits(n, s.hidden_size, s.intermediate_size))
+
+    def _streamed(self, n: int) -> bool:
+        """Whether a decode step of n sequences runs on the products that
+        stream weights in tiles and join their partial sums in the kernels
+        behind them."""
+        from ..ops.build import get_extension
+        s, f, takes = self.spec, self.fused, get_extension().stream_gemm_takes
+        norms = [lw.in_norm for lw in f.layers] + [lw.post_norm for lw in f.layers]
+        return (f.tiled and s.head_dim in (64, 128) and s.hidden_size <= 8192
+                and (not f.hybrid_down or f.lora_r <= 128)
+                and takes(n, s.q_size + 2 * s.kv_size, s.hidden_size)
+                and takes(n, s.hidden_size, s.q_size)
+                and takes(n, 2 * s.intermediate_size, s.hidden_size)
+                and takes(n, s.hidden_size, s.intermediate_size)
+                and all(w.dtype == torch.bfloat16 and w.data_ptr() % 16 == 0
+                        for w in (*norms, self.model.model.norm.weight)))
 
     # ----------------------------------------------------------- forking
 

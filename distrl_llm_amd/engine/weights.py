@@ -9,8 +9,8 @@ between rounds, so the engine folds it once per weight-sync:
 and concatenates the per-site projections — one qkv GEMM (q|k|v) and one
 gate|up GEMM per layer — halving GEMM launches and giving hipBLASLt fatter
 N at decode's skinny M. A refresh writes each projection's merged weight
-straight into the packed storage, one kernel a projection: ~13 ms for 7B,
-once per generation round.
+straight into the packed storage, one kernel a projection, once per
+generation round.
 
 Replaces the reference's per-generate adapter hot-swap into vLLM
 (``load_lora`` inside every fast_generate, reference
@@ -27,8 +27,15 @@ import torch
 
 
 class LayerWeights:
-    __slots__ = ("qkv_w", "qkv_b", "o_w", "gateup_w", "down_w",
-                 "in_norm", "post_norm",
+    """One layer's decode weights, by site: qkv, o, gateup, down.
+
+    ``tiles[site]``: the merged weight in the tiles that the decode products
+    read (ops/csrc/stream_gemm.hip); ``tiles`` is None where the sizes do not
+    tile.
+    ``rows(site)``: the same row-major, for the library's products; laid out
+    when first asked for and kept current by every later refresh."""
+
+    __slots__ = ("layer", "tiles", "_rows", "down_apart", "qkv_b", "in_norm", "post_norm",
                  # nf4 fragment packs (base, built once) + adapter fragment
                  # packs (rebuilt per refresh) for the fused nf4 GEMM path
                  "qkv_w4", "qkv_amax", "o_w4", "o_amax",
@@ -36,9 +43,70 @@ class LayerWeights:
                  "qkv_afrag", "qkv_bfrag", "o_afrag", "o_bfrag",
                  "gateup_afrag", "gateup_bfrag", "down_afrag", "down_bfrag",
                  "qkv_r", "o_r", "gateup_r", "down_r",
-                 # the down site's bf16 base image and its adapter (rank
-                 # padded, scale folded into B) for steps of few sequences
-                 "down_base", "down_a", "down_b")
+                 # the 4-bit down site beside its bf16 base image: the adapter
+                 # (rank padded, scale folded into B), A as rows or in tiles,
+                 # B as (hidden, r) and (r, hidden)
+                 "down_a", "down_b", "down_bt")
+
+    def __init__(self, layer):
+        self.layer = layer
+        self.tiles, self._rows = None, {}
+        self.down_apart = False     # tiles["down"] without its adapter
+
+    @property
+    def mods(self):
+        at, mlp = self.layer.self_attn, self.layer.mlp
+        return {"qkv": (at.q_proj, at.k_proj, at.v_proj), "o": (at.o_proj,),
+                "gateup": (mlp.gate_proj, mlp.up_proj),
+                "down": (mlp.down_proj,)}
+
+    def rows(self, site: str) -> torch.Tensor:
+        if site not in self._rows:
+            self._rows[site] = None
+            self._fill_rows(site)
+        return self._rows[site]
+
+    def refresh_rows(self):
+        for site in self._rows:
+            self._fill_rows(site)
+
+    def _fill_rows(self, site: str) -> None:
+        mods, out = self.mods[site], self._rows[site]
+        if len(mods) == 1 and mods[0].r == 0:
+            self._rows[site] = mods[0].weight.detach().contiguous()
+            return
+        if out is None:
+            out = self._rows[site] = mods[0].weight.new_empty(
+                sum(m.out_features for m in mods), mods[0].in_features)
+        # IN PLACE: captured decode steps hold these storages
+        if self.tiles is not None and not (site == "down" and self.down_apart):
+            out.copy_(_untiled(self.tiles[site], site == "gateup"))
+            return
+        for m, rows in zip(mods, out.split([m.out_features for m in mods])):
+            _merge_into(m, rows)
+
+    qkv_w = property(lambda self: self.rows("qkv"))
+    o_w = property(lambda self: self.rows("o"))
+    gateup_w = property(lambda self: self.rows("gateup"))
+    down_w = property(lambda self: self.rows("down"))
+
+
+def _tiled(w: torch.Tensor, glu: bool = False) -> torch.Tensor:
+    """(N, K) row-major -> tiles of 32 rows x 16 of K, [K half][row][8
+    elements]; glu: [gate; up] as 16 gate and 16 up rows a tile."""
+    N, K = w.shape
+    if glu:
+        w = w.view(2, N // 32, 16, K).transpose(0, 1)
+    return w.reshape(N // 32, 32, K // 16, 2, 8).permute(0, 2, 3, 1, 4) \
+        .reshape(N, K)
+
+
+def _untiled(t: torch.Tensor, glu: bool = False) -> torch.Tensor:
+    N, K = t.shape
+    w = t.view(N // 32, K // 16, 2, 32, 8).permute(0, 3, 1, 2, 4)
+    if glu:
+        w = w.reshape(N // 32, 2, 16, K).transpose(0, 1)
+    return w.reshape(N, K)
 
 
 def _effective(mod) -> torch.Tensor:
@@ -59,6 +127,23 @@ def _merge_into(mod, out: torch.Tensor) -> None:
                 mod.lora_B.detach(), out, float(mod.scale)):
             return
     out.copy_(_effective(mod))
+
+
+def _merge_tiles(mods, out: torch.Tensor, glu: bool, adapters: bool = True) -> None:
+    """out, in tiles <- the modules' weights one below the other (glu: a
+    SiLU*mul pair), with their adapters or without."""
+    from ..ops.functional import _require_ext
+    ext, row = _require_ext("decode weights"), 0
+    for m in mods:
+        ab = ((m.lora_A.detach(), m.lora_B.detach(), float(m.scale))
+              if adapters and m.r > 0 else ())
+        w = m.weight.detach()
+        if ({t.dtype for t in (w, *ab[:2])} != {torch.bfloat16}
+                or not ext.weight_tiles(w, out, row, glu, *ab)):
+            out.copy_(_tiled(torch.cat(
+                [_effective(m) if adapters else m.weight for m in mods]), glu))
+            return
+        row += 16 if glu else m.out_features
 
 
 class FusedWeights:
@@ -113,6 +198,15 @@ class FusedWeights:
             and q0.weight.is_cuda and shapes_ok
             and os.environ.get("DISTRL_HYBRID_DOWN", "1") == "1")
         self.lora_r = q0.r
+        # the decode products read weights in tiles
+        self.tiled = bool(
+            not self.nf4 and q0.weight.is_cuda
+            and q0.weight.dtype == torch.bfloat16 and s.hidden_size % 64 == 0
+            and s.q_size % 64 == 0 and s.kv_size % 32 == 0
+            and s.intermediate_size % 64 == 0)
+        # the 4-bit kernel's packs of the down site: only steps beyond the
+        # streamed products' rows use them
+        self._nf4_down = False
 
     @staticmethod
     def _nf4_cat(mods):
@@ -184,14 +278,37 @@ class FusedWeights:
                 setattr(lw, f"{name}_afrag", af)
                 setattr(lw, f"{name}_bfrag", bf)
             setattr(lw, f"{name}_r", r_pad)
-            if name == "down" and mods[0].weight.numel() > 0:
-                lw.down_base = mods[0].weight
-                if old_af is None:
-                    lw.down_a = A.to(torch.bfloat16).contiguous()
-                    lw.down_b = B.to(torch.bfloat16).contiguous()
-                else:
-                    lw.down_a.copy_(A)
-                    lw.down_b.copy_(B)
+
+    def ensure_nf4_down(self):
+        """The 4-bit kernel's packs of the down site, built when a step first
+        needs them; every later refresh renews the adapter's."""
+        if self._nf4_down:
+            return
+        from ..models.quant import prepack_nf4_fragments
+        for layer, lw in zip(self.model.model.layers, self.layers):
+            packed, absmax, N, K = self._nf4_cat([layer.mlp.down_proj])
+            lw.down_w4, lw.down_amax = prepack_nf4_fragments(packed, absmax,
+                                                             N, K)
+            self._refresh_nf4_adapters(lw, layer, sites=("down",))
+        self._nf4_down = True
+
+    def _refresh_down_adapter(self, lw: "LayerWeights"):
+        """The 4-bit down site's adapter beside the bf16 base image."""
+        m, = lw.mods["down"]
+        r_pad = (m.r + 31) // 32 * 32
+        A = m.lora_A.detach().to(torch.bfloat16)
+        B = (m.lora_B.detach() * m.scale).to(torch.bfloat16)
+        if r_pad != m.r:
+            A = torch.cat([A, A.new_zeros(r_pad - m.r, A.shape[1])])
+            B = torch.cat([B, B.new_zeros(B.shape[0], r_pad - m.r)], 1)
+        new = {"down_a": _tiled(A) if self.tiled else A, "down_b": B,
+               "down_bt": B.t()}
+        for name, t in new.items():
+            # IN PLACE: captured decode steps hold these storages
+            if hasattr(lw, name):
+                getattr(lw, name).copy_(t)
+            else:
+                setattr(lw, name, t.contiguous().clone())
 
     @torch.no_grad()
     def refresh(self):
@@ -202,12 +319,11 @@ class FusedWeights:
         only the adapter fragment packs (A stacks, block-diagonal scaled B)
         are rebuilt per refresh — the adapter stays exact bf16.
         """
-        model = self.model
         first = not self._built
-        for li, layer in enumerate(model.model.layers):
+        for li, layer in enumerate(self.model.model.layers):
             at = layer.self_attn
             if first:
-                lw = LayerWeights()
+                lw = LayerWeights(layer)
                 if at.q_proj.bias is not None:
                     lw.qkv_b = torch.cat([at.q_proj.bias, at.k_proj.bias,
                                           at.v_proj.bias]).contiguous()
@@ -225,31 +341,25 @@ class FusedWeights:
                 if first:
                     self._build_nf4_base(lw, layer)
                 self._refresh_nf4_adapters(lw, layer)
-            else:
-                self._refresh_merged(lw, layer, first)
-                if self.hybrid_down:
-                    if first:
-                        from ..models.quant import prepack_nf4_fragments
-                        packed, absmax, N, K = self._nf4_cat(
-                            [layer.mlp.down_proj])
-                        lw.down_w4, lw.down_amax = prepack_nf4_fragments(
-                            packed, absmax, N, K)
+                continue
+            if self.tiled:
+                self._refresh_tiles(lw)
+            lw.refresh_rows()
+            if self.hybrid_down:
+                if self.lora_r > 0:
+                    self._refresh_down_adapter(lw)
+                if self._nf4_down:
                     self._refresh_nf4_adapters(lw, layer, sites=("down",))
         self._built = True
 
-    def _refresh_merged(self, lw: "LayerWeights", layer, first: bool):
-        at, mlp = layer.self_attn, layer.mlp
-        for name, mods in (("qkv_w", [at.q_proj, at.k_proj, at.v_proj]),
-                           ("gateup_w", [mlp.gate_proj, mlp.up_proj]),
-                           ("o_w", [at.o_proj]), ("down_w", [mlp.down_proj])):
-            if first:
-                m = mods[0]
-                if len(mods) == 1 and m.r == 0:
-                    setattr(lw, name, m.weight.contiguous())
-                else:
-                    setattr(lw, name, m.weight.new_empty(
-                        sum(m.out_features for m in mods), m.in_features))
+    def _refresh_tiles(self, lw: "LayerWeights"):
+        if lw.tiles is None:
+            lw.tiles = {
+                site: mods[0].weight.new_empty(
+                    sum(m.out_features for m in mods), mods[0].in_features)
+                for site, mods in lw.mods.items()}
+            lw.down_apart = self.hybrid_down and self.lora_r > 0
+        for site, mods in lw.mods.items():
             # IN PLACE: captured decode steps hold these storages
-            rows = getattr(lw, name).split([m.out_features for m in mods])
-            for m, out in zip(mods, rows):
-                _merge_into(m, out)
+            _merge_tiles(mods, lw.tiles[site], site == "gateup",
+                         not (site == "down" and lw.down_apart))

@@ -57,7 +57,27 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
                           c10::optional<torch::Tensor> res,
                           c10::optional<torch::Tensor> norm_w, double eps,
                           c10::optional<torch::Tensor> u,
-                          c10::optional<torch::Tensor> ub);
+                          c10::optional<torch::Tensor> ub, bool tiles);
+bool stream_gemm_takes(int64_t M, int64_t N, int64_t K);
+torch::Tensor stream_glu(torch::Tensor x, torch::Tensor w);
+torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
+                          c10::optional<torch::Tensor> w2);
+bool weight_tiles(torch::Tensor w, torch::Tensor out, int64_t row, bool glu,
+                  c10::optional<torch::Tensor> a,
+                  c10::optional<torch::Tensor> b, double scale);
+std::vector<torch::Tensor> add_rmsnorm_join(torch::Tensor parts,
+                                            torch::Tensor res, torch::Tensor w,
+                                            double eps,
+                                            c10::optional<torch::Tensor> bt);
+torch::Tensor rope_scatter_join(torch::Tensor parts,
+                                c10::optional<torch::Tensor> bias,
+                                torch::Tensor positions, torch::Tensor slots,
+                                torch::Tensor inv_freq, torch::Tensor key_cache,
+                                torch::Tensor value_cache, int64_t H,
+                                int64_t KV, int64_t D,
+                                c10::optional<torch::Tensor> q_norm,
+                                c10::optional<torch::Tensor> k_norm,
+                                double eps);
 bool lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b,
                 torch::Tensor out, double scale);
 bool lora_add(torch::Tensor y, torch::Tensor u, torch::Tensor m,
@@ -126,7 +146,31 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("x"), py::arg("w"), py::arg("mode"),
         py::arg("bias") = py::none(), py::arg("res") = py::none(),
         py::arg("norm_w") = py::none(), py::arg("eps") = 0.0,
-        py::arg("u") = py::none(), py::arg("ub") = py::none());
+        py::arg("u") = py::none(), py::arg("ub") = py::none(),
+        py::arg("tiles") = false);
+  m.def("stream_gemm_takes", &stream_gemm_takes,
+        "whether stream_gemm and stream_glu take (M, N, K)");
+  m.def("stream_glu", &stream_glu,
+        "silu(x Wg^T) * (x Wu^T) for some tens of rows, W in tiles");
+  m.def("stream_gemm", &stream_gemm,
+        "fp32 partial sums of x [w; w2]^T, W in tiles", py::arg("x"),
+        py::arg("w"), py::arg("w2") = py::none());
+  m.def("weight_tiles", &weight_tiles,
+        "rows of W (+ scale * B A) into tiles; false: not these operands",
+        py::arg("w"), py::arg("out"), py::arg("row"), py::arg("glu"),
+        py::arg("a") = py::none(), py::arg("b") = py::none(),
+        py::arg("scale") = 0.0);
+  m.def("add_rmsnorm_join", &add_rmsnorm_join,
+        "residual + partial sums (+ adapter), then RMSNorm", py::arg("parts"),
+        py::arg("res"), py::arg("w"), py::arg("eps"),
+        py::arg("bt") = py::none());
+  m.def("rope_scatter_join", &rope_scatter_join,
+        "partial sums of [q|k|v] + bias -> norms, RoPE, KV scatter; returns q",
+        py::arg("parts"), py::arg("bias"), py::arg("positions"),
+        py::arg("slots"), py::arg("inv_freq"), py::arg("key_cache"),
+        py::arg("value_cache"), py::arg("H"), py::arg("KV"), py::arg("D"),
+        py::arg("q_norm") = py::none(), py::arg("k_norm") = py::none(),
+        py::arg("eps") = 0.0);
   m.def("lora_merge", &lora_merge, "out = W + scale * B A, one pass");
   m.def("lora_add", &lora_add, "y += scale * u m (+ res) in place; false: not these operands",
         py::arg("y"), py::arg("u"), py::arg("m"), py::arg("scale"),

@@ -68,6 +68,27 @@ DEV_INLINE float block_max(float x, float* red) {
   return out;
 }
 
+// ---- partial sums ----
+// v[0..7] += 8 elements of n arrays `step` elements apart, four of them in
+// flight at a time
+DEV_INLINE void add_parts8(float (&v)[8], const float* p, int64_t step, int n) {
+  for (int z = 0; z < n; z += 4) {
+    f32x4v a[4], b[4];
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* q = p + min(z + i, n - 1) * step;
+      a[i] = *reinterpret_cast<const f32x4v*>(q);
+      b[i] = *reinterpret_cast<const f32x4v*>(q + 4);
+    }
+    #pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (z + i < n) {
+        #pragma unroll
+        for (int j = 0; j < 4; ++j) { v[j] += a[i].v[j]; v[4 + j] += b[i].v[j]; }
+      }
+  }
+}
+
 // ---- hash (counter-based random numbers) ----
 DEV_INLINE uint64_t splitmix64(uint64_t x) {
   x += 0x9E3779B97F4A7C15ull;

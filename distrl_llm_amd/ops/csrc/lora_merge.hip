@@ -36,13 +36,15 @@ constexpr int KC = 256;            // columns of a workgroup
 constexpr int STEPS = KC / 32;     // loads of W in flight
 
 // w and out may be one; res (or none) is added to the same sum. Rows of w and
-// out are ldw elements apart, those of b ldb. TA: a is (K, r).
-template <bool TA>
+// out are ldw elements apart, those of b ldb. TA: a is (K, r). TILES: out in
+// tiles of 32 rows x 16 of K, [K half][row][8 elements], row n of w at row + n of
+// out, or (glu) at row + n in blocks of 16 of every 32; r may be 0.
+template <bool TA, bool TILES = false>
 __global__ __launch_bounds__(256)
 void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict__ a,
                        const __hip_bfloat16* __restrict__ b, const __hip_bfloat16* __restrict__ res,
                        __hip_bfloat16* out, int N, int K, int r, int rows, int64_t ldw, int ldb,
-                       int64_t ldr, float scale) {
+                       int64_t ldr, float scale, int row0, int glu) {
   // A: [r32][KC], TA: [KC][r32], rows 16 B apart
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int RS = KC * 2 + 16;
@@ -113,8 +115,13 @@ void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict
         const float t = (float)wv[i][j] + scale * d[i][j >> 2][j & 3];
         o[j] = (__bf16)(res ? t + (float)rv[i][j] : t);
       }
-      if (n0 + lr < N && k0 + i * 32 < K)
-        *reinterpret_cast<bf16v8*>(out + (n0 + lr) * ldw + k0 + i * 32 + g * 8) = o;
+      if (n0 + lr < N && k0 + i * 32 < K) {
+        const int n = n0 + lr, k = k0 + i * 32 + g * 8, row = row0 + (glu ? n + (n & ~15) : n);
+        const int64_t at = TILES ? (int64_t)(row >> 5) * K * 32 + (k >> 4) * 512 + (k & 8) * 32 +
+                                       (row & 31) * 8
+                                 : n * ldw + k;
+        *reinterpret_cast<bf16v8*>(out + at) = o;
+      }
     }
   }
 }
@@ -158,7 +165,7 @@ bool launch_merge(const torch::Tensor& w, const torch::Tensor& a, const torch::T
   hipLaunchKernelGGL(ta ? lora_merge_kernel<true> : lora_merge_kernel<false>, grid, block, smem,
                      stream, lptr(w), lptr(a), lptr(b), res ? lptr(*res) : nullptr,
                      reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), N, K, r, rows,
-                     w.stride(0), (int)b.stride(0), res ? res->stride(0) : 0, (float)scale);
+                     w.stride(0), (int)b.stride(0), res ? res->stride(0) : 0, (float)scale, 0, 0);
   HIP_CHECK_LAST();
   return true;
 }
@@ -169,6 +176,40 @@ bool launch_merge(const torch::Tensor& w, const torch::Tensor& a, const torch::T
 // accesses or the tiles can't take.
 bool lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b, torch::Tensor out, double scale) {
   return launch_merge(w, a, b, out, false, scale);
+}
+
+// Rows row .. of a weight in tiles (out: (rows, K), K % 32 == 0, see the kernel)
+// <- w, or w + scale * b a. glu: w is gate (row 0) or up (row 16) of a SiLU*mul
+// pair. False, and nothing done, for operands that 16 B accesses can't take.
+bool weight_tiles(torch::Tensor w, torch::Tensor out, int64_t row, bool glu,
+                  c10::optional<torch::Tensor> a, c10::optional<torch::Tensor> b, double scale) {
+  TORCH_CHECK(out.is_cuda() && out.is_contiguous() && out.dim() == 2 &&
+              out.scalar_type() == at::kBFloat16 && out.size(0) % 32 == 0);
+  if (w.dim() != 2 || !lrows(w) || w.size(1) != out.size(1) || w.size(1) % 32 != 0) return false;
+  const int N = w.size(0), K = w.size(1);
+  TORCH_CHECK(row >= 0 && (glu ? (row == 0 || row == 16) && N % 16 == 0 && 2 * N == out.size(0)
+                               : row + N <= out.size(0)),
+              "weight_tiles: rows past the end");
+  TORCH_CHECK(reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0);
+  int r = 0;
+  if (a) {
+    TORCH_CHECK(b.has_value());
+    if (a->dim() != 2 || b->dim() != 2 || !lrows(*a) || !a->is_contiguous() || !lrows(*b))
+      return false;
+    r = a->size(0);
+    TORCH_CHECK(a->size(1) == K && b->size(0) == N && b->size(1) == r, "weight_tiles: adapter");
+    if (!lora_merge_takes(K, r)) return false;
+  }
+  if (N == 0) return true;
+  const int rows = (int64_t)CDIV(K, KC) * CDIV(N, 64) >= 4096 ? 256 : 64;
+  const int smem = CDIV(r, 32) * 32 * (KC * 2 + 16);
+  hipLaunchKernelGGL((lora_merge_kernel<false, true>), dim3(CDIV(K, KC), CDIV(N, rows)), dim3(256),
+                     smem, at::cuda::getCurrentCUDAStream(), lptr(w), r ? lptr(*a) : nullptr,
+                     r ? lptr(*b) : nullptr, nullptr,
+                     reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), N, K, r, rows, w.stride(0),
+                     r ? (int)b->stride(0) : 0, 0, (float)scale, (int)row, (int)glu);
+  HIP_CHECK_LAST();
+  return true;
 }
 
 // y (M, N) += scale * u (M, r) m (r, N), then + res if given: one rounding for

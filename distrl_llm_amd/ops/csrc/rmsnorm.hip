@@ -262,3 +262,109 @@ std::vector<torch::Tensor> add_rmsnorm_fwd(torch::Tensor x, torch::Tensor h,
   HIP_CHECK_LAST();
   return {y, res};
 }
+
+// ---- the same behind a product that left partial sums (S, rows, hidden + r):
+// res' = res + their sum (+ u bt, u the sum of the last r columns, bt (r, hidden)
+// an adapter's output weights), y = rmsnorm(res') * w. One workgroup a row, 8
+// columns a thread: all of a row's loads are in flight at once.
+namespace {
+
+template <int VPT>
+__global__ __launch_bounds__(512)
+void add_rmsnorm_join_kernel(const float* __restrict__ parts, const __hip_bfloat16* __restrict__ x,
+                             const __hip_bfloat16* __restrict__ bt,
+                             const __hip_bfloat16* __restrict__ w, __hip_bfloat16* __restrict__ y,
+                             __hip_bfloat16* __restrict__ res, int rows, int hidden, int r, int S,
+                             float eps) {
+  __shared__ float red[16], us[128];
+  const int64_t row = blockIdx.x, ld = hidden + r, step = rows * ld;
+  const float* pr = parts + row * ld;
+  for (int j = threadIdx.x; j < r; j += blockDim.x) {
+    float u = 0.f;
+    for (int z = 0; z < S; ++z) u += pr[z * step + hidden + j];
+    us[j] = u;
+  }
+  float v[VPT][8];
+  #pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int n = (k * blockDim.x + threadIdx.x) * 8;
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) v[k][j] = 0.f;
+    if (n >= hidden) continue;
+    const bf16x8 xv = *reinterpret_cast<const bf16x8*>(x + row * hidden + n);
+    add_parts8(v[k], pr + n, step, S);
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) v[k][j] += bf2f(xv.v[j]);
+  }
+  if (r > 0) {
+    __syncthreads();
+    #pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+      const int n = (k * blockDim.x + threadIdx.x) * 8;
+      if (n >= hidden) continue;
+      #pragma unroll 8
+      for (int i = 0; i < r; ++i) {
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(bt + (int64_t)i * hidden + n);
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) v[k][j] += us[i] * bf2f(b.v[j]);
+      }
+    }
+  }
+  float ss = 0.f;
+  #pragma unroll
+  for (int k = 0; k < VPT; ++k)
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) ss += v[k][j] * v[k][j];
+  ss = block_sum(ss, red);
+  const float rn = rsqrtf(ss / hidden + eps);
+  #pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int n = (k * blockDim.x + threadIdx.x) * 8;
+    if (n >= hidden) continue;
+    const bf16x8 wv = *reinterpret_cast<const bf16x8*>(w + n);
+    bf16x8 o, s;
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      s.v[j] = f2bf(v[k][j]);
+      o.v[j] = f2bf(bf2f(s.v[j]) * rn * bf2f(wv.v[j]));
+    }
+    *reinterpret_cast<bf16x8*>(res + row * hidden + n) = s;
+    *reinterpret_cast<bf16x8*>(y + row * hidden + n) = o;
+  }
+}
+
+}  // namespace
+
+// {rmsnorm(res') * w, res'}, res' = res + the parts' sum (+ the adapter)
+std::vector<torch::Tensor> add_rmsnorm_join(torch::Tensor parts, torch::Tensor res, torch::Tensor w,
+                                            double eps, c10::optional<torch::Tensor> bt) {
+  TORCH_CHECK(res.is_cuda() && res.is_contiguous() && res.dim() == 2 &&
+              res.scalar_type() == at::kBFloat16);
+  TORCH_CHECK(parts.is_cuda() && parts.is_contiguous() && parts.dim() == 3 &&
+              parts.scalar_type() == at::kFloat && parts.size(1) == res.size(0));
+  const int rows = res.size(0), hidden = res.size(1), r = (int)parts.size(2) - hidden;
+  TORCH_CHECK(w.is_cuda() && w.is_contiguous() && w.scalar_type() == at::kBFloat16 &&
+              w.numel() == hidden);
+  TORCH_CHECK(hidden % 8 == 0 && hidden <= 8192 && r >= 0 && r <= 128 && r % 8 == 0,
+              "add_rmsnorm_join: unsupported shape");
+  TORCH_CHECK((r > 0) == bt.has_value());
+  if (bt)
+    TORCH_CHECK(bt->is_cuda() && bt->is_contiguous() && bt->scalar_type() == at::kBFloat16 &&
+                bt->dim() == 2 && bt->size(0) == r && bt->size(1) == hidden);
+  for (const auto* t : {&res, &w})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "add_rmsnorm_join: alignment");
+  TORCH_CHECK(!bt || reinterpret_cast<uintptr_t>(bt->data_ptr()) % 16 == 0);
+  auto y = torch::empty_like(res), out = torch::empty_like(res);
+  if (rows == 0) return {y, out};
+  const int threads = std::min(512, CDIV(hidden / 8, 64) * 64);
+  auto bf = [](const torch::Tensor& t) { return reinterpret_cast<__hip_bfloat16*>(t.data_ptr()); };
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(threads), 0, at::cuda::getCurrentCUDAStream(),
+                       parts.data_ptr<float>(), bf(res), bt ? bf(*bt) : nullptr, bf(w), bf(y),
+                       bf(out), rows, hidden, r, (int)parts.size(0), (float)eps);
+  };
+  if (hidden <= 4096) go(add_rmsnorm_join_kernel<1>);
+  else go(add_rmsnorm_join_kernel<2>);
+  HIP_CHECK_LAST();
+  return {y, out};
+}

@@ -33,7 +33,7 @@ constexpr int in_flight() {
   return n > 10 ? 10 : n;
 }
 
-template <int MT, int KW, int MODE, bool NORM>
+template <int MT, int KW, int MODE, bool NORM, bool TILES>
 __global__ __launch_bounds__(KW * 64)
 void skinny_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat16* __restrict__ w,
                         const __hip_bfloat16* __restrict__ bias,
@@ -53,7 +53,15 @@ void skinny_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat
 
   const __hip_bfloat16* wp[ACC];
   #pragma unroll
-  for (int a = 0; a < ACC; ++a) wp[a] = w + (int64_t)(n0 + a * N + wr) * K + g * 8;
+  for (int a = 0; a < ACC; ++a) {
+    if (TILES) {
+      // row of the tile; SiLU*mul: 16 gate and 16 up rows
+      const int n = MODE == GLU ? (n0 + wr) / 16 * 32 + a * 16 + (n0 + wr) % 16 : n0 + wr;
+      wp[a] = w + (int64_t)(n >> 5) * K * 32 + (g >> 1) * 512 + (g & 1) * 256 + (n & 31) * 8;
+    } else {
+      wp[a] = w + (int64_t)(n0 + a * N + wr) * K + g * 8;
+    }
+  }
   f32x4 acc[ACC][MT];
   #pragma unroll
   for (int a = 0; a < ACC; ++a)
@@ -73,7 +81,7 @@ void skinny_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat
     for (int i = 0; i < U; ++i) {
       const int k = min(s + i, s1 - 1) * 32;              // past the end: the last again
       #pragma unroll
-      for (int a = 0; a < ACC; ++a) wf[i][a] = *reinterpret_cast<const bf16v8*>(wp[a] + k);
+      for (int a = 0; a < ACC; ++a) wf[i][a] = *reinterpret_cast<const bf16v8*>(wp[a] + k * (TILES ? 32 : 1));
       #pragma unroll
       for (int t = 0; t < MT; ++t)
         xf[i][t] = *reinterpret_cast<const bf16v8*>(x + (int64_t)row[t] * K + k + g * 8);
@@ -185,7 +193,8 @@ bool skinny_gemm_takes(int64_t M, int64_t N, int64_t K) {
 torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
                           c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> res,
                           c10::optional<torch::Tensor> norm_w, double eps,
-                          c10::optional<torch::Tensor> u, c10::optional<torch::Tensor> ub) {
+                          c10::optional<torch::Tensor> u, c10::optional<torch::Tensor> ub,
+                          bool tiles) {
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous());
   TORCH_CHECK(w.is_cuda() && w.dim() == 2 && w.is_contiguous());
   TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16);
@@ -193,6 +202,7 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
   const int M = x.size(0), K = x.size(1), N = mode == GLU ? w.size(0) / 2 : w.size(0);
   TORCH_CHECK(mode != GLU || w.size(0) % 2 == 0);
   TORCH_CHECK(skinny_gemm_takes(M, N, K), "skinny_gemm: unsupported shape (", M, ", ", N, ", ", K, ")");
+  TORCH_CHECK(!tiles || w.size(0) % 32 == 0, "skinny_gemm: rows of W in tiles");
   x = at16(x);
   w = at16(w);
   auto check = [&](c10::optional<torch::Tensor>& t, int64_t n, const char* what) {
@@ -222,16 +232,20 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
   // 20.6, 16/8 18.1; N 9728, K 2560: 36, 33; N 4864, K 896: 11.4, 11.5.
   // Fewer rows a workgroup reach more CUs but re-read x; more waves shorten
   // the chain of loads until joining them costs more.
-  const int tiles = N / 16, steps = K / 32, tr = tiles <= 128 ? 8 : 16;
-  const int kw = tiles <= 256 ? (steps >= 64 ? 16 : steps >= 32 ? 8 : 4)
+  const int nt = N / 16, steps = K / 32, tr = nt <= 128 ? 8 : 16;
+  const int kw = nt <= 256 ? (steps >= 64 ? 16 : steps >= 32 ? 8 : 4)
                         : (mode == GLU && steps >= 48 ? 8 : 4);
-  auto go = [&](auto mt_, auto kw_, auto mode_, auto norm_) {
+  auto launch = [&](auto mt_, auto kw_, auto mode_, auto norm_, auto tiles_) {
     constexpr int MT = decltype(mt_)::value, KW = decltype(kw_)::value,
                   MODE = decltype(mode_)::value;
     constexpr bool NORM = decltype(norm_)::value;
     const size_t smem = KW * (MODE == GLU ? 2 : 1) * MT * 64 * 16;
-    hipLaunchKernelGGL((skinny_gemm_kernel<MT, KW, MODE, NORM>), dim3(N / tr), dim3(KW * 64), smem,
+    hipLaunchKernelGGL((skinny_gemm_kernel<MT, KW, MODE, NORM, decltype(tiles_)::value>), dim3(N / tr), dim3(KW * 64), smem,
                        stream, ptr(x), ptr(w), b, r, nw, up, ubp, o, M, N, K, R, tr, (float)eps);
+  };
+  auto go = [&](auto mt_, auto kw_, auto mode_, auto norm_) {
+    if (tiles) launch(mt_, kw_, mode_, norm_, std::true_type{});
+    else launch(mt_, kw_, mode_, norm_, std::false_type{});
   };
   auto by_norm = [&](auto mt_, auto kw_, auto mode_) {
     if (nw) go(mt_, kw_, mode_, std::true_type{}); else go(mt_, kw_, mode_, std::false_type{});

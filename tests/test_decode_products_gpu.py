@@ -1,0 +1,167 @@
+"""Decode products on weights in tiles and the kernels that join their partial
+sums, at the edges of their tiles and splits, against fp64 torch."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ext():
+    from distrl_llm_amd.ops.build import build
+    return build()
+
+
+def _rand(shape, seed, std=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(shape, generator=g) * std).to("cuda", torch.bfloat16)
+
+
+def _rel(x, ref):
+    return float((x.double() - ref.double()).norm() / ref.double().norm().clamp_min(1e-30))
+
+
+def _tiles(ext, *ws, glu=False):
+    out = torch.empty(sum(w.shape[0] for w in ws), ws[0].shape[1], dtype=torch.bfloat16,
+                      device="cuda")
+    row = 0
+    for w in ws:
+        assert ext.weight_tiles(w, out, row, glu)
+        row += 16 if glu else w.shape[0]
+    return out
+
+
+@pytest.mark.parametrize("N1,N2,K", [(32, 32, 32), (64, 96, 288), (256, 32, 1056)])
+@pytest.mark.parametrize("r", [0, 8, 40])
+def test_weight_tiles(ext, N1, N2, K, r):
+    """Tiles of two matrices one below the other, with an adapter and without,
+    are the torch permutation of the row-major kernel's results, and back."""
+    from distrl_llm_amd.engine.weights import _tiled, _untiled
+    ws, out = [_rand((N, K), i) for i, N in enumerate((N1, N2))], _rand((N1 + N2, K), 9)
+    row, rows = 0, []
+    for i, w in enumerate(ws):
+        a, b = _rand((r, K), 3 + i, 0.1), _rand((w.shape[0], r), 5 + i, 0.1)
+        rows.append(w.clone())
+        if r:
+            assert ext.lora_merge(w, a, b, rows[-1], 0.5)
+        assert ext.weight_tiles(w, out, row, False, *((a, b, 0.5) if r else ()))
+        row += w.shape[0]
+    rows = torch.cat(rows)
+    assert torch.equal(out, _tiled(rows)) and torch.equal(_untiled(out), rows)
+    if N1 % 32 == 0 and N1 == N2:
+        assert torch.equal(_tiles(ext, *ws, glu=True), _tiled(torch.cat(ws), True))
+        assert torch.equal(_untiled(_tiles(ext, *ws, glu=True), True), torch.cat(ws))
+    # refused: a row-major matrix that 16 B loads can't walk
+    assert not ext.weight_tiles(_rand((N1, K + 2), 1)[:, 1:K + 1], out, 0, False)
+
+
+@pytest.mark.parametrize("M", [1, 17, 32, 33, 96, 128, 129, 160])
+@pytest.mark.parametrize("N,K", [(32, 64), (96, 192), (1152, 896), (2048, 1536), (160, 8960)])
+def test_stream_gemm(ext, M, N, K):
+    """Every row tile and cut, ragged last workgroups, more rows of W behind;
+    SiLU*mul. Bounds: fp32 sums (some K roundings of 2^-24); one rounding of
+    the activation's result."""
+    x, w, a = _rand((M, K), 1), _rand((N, K), 2, K ** -0.5), _rand((32, K), 3)
+    xd, ref = x.double(), x.double() @ w.double().t()
+    got = ext.stream_gemm(x, _tiles(ext, w))
+    assert got.shape[1:] == (M, N) and _rel(got.sum(0), ref) < 1e-5
+    got = ext.stream_gemm(x, _tiles(ext, w), _tiles(ext, a)).sum(0)
+    assert _rel(got[:, :N], ref) < 1e-5 and _rel(got[:, N:], xd @ a.double().t()) < 1e-5
+    up = _rand((N, K), 4, K ** -0.5)
+    ref = torch.nn.functional.silu(ref) * (xd @ up.double().t())
+    assert _rel(ext.stream_glu(x, _tiles(ext, w, up, glu=True)), ref) < 2.0 ** -8
+    assert not ext.stream_gemm_takes(161, N, K)         # one row further
+
+
+@pytest.mark.parametrize("M", [1, 8, 17, 32])
+@pytest.mark.parametrize("N,K", [(32, 512), (896, 896), (2080, 544), (4128, 4864)])
+def test_skinny_gemm_tiles(ext, M, N, K):
+    """The same results from tiles as from rows."""
+    x, w, b = _rand((M, K), 1), _rand((2 * N, K), 2, K ** -0.5), _rand((N,), 3)
+    res, u, ub = _rand((M, N), 4), _rand((M, 64), 5), _rand((N, 64), 6, 0.1)
+    kw = {"norm_w": _rand((K,), 7, 0.1) + 1, "eps": 1e-6}
+    half = w[:N].contiguous()
+    t, tg = _tiles(ext, half), _tiles(ext, half, w[N:], glu=True)
+    for mode, rows, tiles, args in (
+            (0, half, t, {"bias": b}), (0, half, t, {"bias": b, **kw}),
+            (1, half, t, {"res": res, "u": u, "ub": ub}), (2, w, tg, {}), (2, w, tg, kw)):
+        assert torch.equal(ext.skinny_gemm(x, tiles, mode, tiles=True, **args),
+                           ext.skinny_gemm(x, rows, mode, **args))
+
+
+@pytest.mark.parametrize("S", [1, 3, 4, 9])
+@pytest.mark.parametrize("rows,hidden,r", [(1, 64, 0), (5, 896, 32), (33, 4096, 64), (2, 4160, 128),
+                                           (3, 8192, 0)])
+def test_add_rmsnorm_join(ext, S, rows, hidden, r):
+    """Bounds: the residual rounded once, its norm from the rounded values."""
+    g = torch.Generator(device="cuda").manual_seed(S)
+    parts = torch.randn((S, rows, hidden + r), generator=g, device="cuda")
+    res, w, bt = _rand((rows, hidden), 1), _rand((hidden,), 2, 0.1) + 1, _rand((r, hidden), 3, 0.1)
+    y, out = ext.add_rmsnorm_join(parts, res, w, 1e-6, bt if r else None)
+    total = parts.double().sum(0)
+    ref = res.double() + total[:, :hidden] + total[:, hidden:] @ bt.double()
+    assert _rel(out, ref) < 2.0 ** -8
+    assert _rel(y, ref * torch.rsqrt((ref * ref).mean(-1, keepdim=True) + 1e-6) * w.double()) \
+        < 2.0 ** -7
+
+
+@pytest.mark.parametrize("H,KV,D", [(14, 2, 64), (28, 4, 128), (3, 1, 64), (64, 8, 128)])
+@pytest.mark.parametrize("S,bias,norms", [(1, False, False), (3, True, False), (6, False, True)])
+def test_rope_scatter_join(ext, H, KV, D, S, bias, norms):
+    """Against the rotation of the summed rows (its inputs rounded to bf16: two
+    roundings more); a row without a slot leaves the cache alone."""
+    T, width = 5, (H + 2 * KV) * D
+    g = torch.Generator(device="cuda").manual_seed(S)
+    parts = torch.randn((S, T, width), generator=g, device="cuda")
+    b = _rand((width,), 1) if bias else None
+    nw = (_rand((D,), 2, 0.1) + 1, _rand((D,), 3, 0.1) + 1, 1e-6) if norms else ()
+    pos = torch.tensor([0, 7, 1, 1500, 3], dtype=torch.int32, device="cuda")
+    slots = torch.tensor([4, 0, -1, 9, 2], device="cuda")
+    inv = 1.0 / 1e4 ** (torch.arange(0, D, 2, device="cuda").float() / D)
+    cache = [_rand((12, KV, D), 4 + i) for i in range(2)]
+    got = [c.clone() for c in cache]
+    q = ext.rope_scatter_join(parts, b, pos, slots, inv, *got, H, KV, D, *nw)
+    qkv = parts.sum(0) + (b.float() if bias else 0)
+    qkv = qkv.to(torch.bfloat16)
+    ext.rope_scatter_qkv(qkv, pos, slots, inv, *cache, H, KV, D, *nw)
+    assert _rel(q, qkv[:, :H * D]) < 3 * 2.0 ** -9
+    for x, y in zip(got, cache):
+        assert _rel(x, y) < 3 * 2.0 ** -9 and torch.equal(x[5], y[5])
+
+
+@pytest.mark.parametrize("name,four_bit,lora_r", [("small-qwen2", False, 8), ("small-qwen2", True, 8),
+                                                  ("small-qwen3", True, 0), ("small-qwen3", False, 12)])
+@pytest.mark.parametrize("n", [3, 40, 161])
+def test_decode_step_matches_modules(name, four_bit, lora_r, n):
+    """Steps of few, of tens and of more sequences after a changed adapter, twice
+    through the cached graph: the cache rows they write against a teacher-forced
+    pass of the modules (two bf16 paths of the same products: 3 %)."""
+    from distrl_llm_amd.config import EngineConfig, SamplingParams
+    from distrl_llm_amd.engine import Engine
+    from distrl_llm_amd.models import CausalLM, get_spec
+    model = CausalLM(get_spec(name), lora_r=lora_r, dtype=torch.bfloat16,
+                     device=torch.device("cuda")).random_init(3).eval()
+    if four_bit:
+        model.quantize_nf4_()
+    eng = Engine(model, EngineConfig(max_seq_length=64, num_kv_blocks=2 * n + 8, max_num_seqs=256))
+    prompt, sp = [5, 6, 7, 8, 9], SamplingParams(max_tokens=4, temperature=0.0, n=n)
+    for seed in (7, 8):
+        with torch.no_grad():
+            for key, p in model.named_parameters():
+                if key.endswith(("lora_B", "bias")):
+                    p.copy_(_rand(p.shape, seed, 0.05))
+        eng.pool.allocator.reset()
+        tokens = eng.generate([prompt], sp)[0][0]
+        ids, ref = torch.tensor([prompt + tokens[:3]], device="cuda"), []
+        hooks = [l.self_attn.v_proj.register_forward_hook(lambda m, i, o: ref.append(o[0].detach()))
+                 for l in model.model.layers]
+        with torch.no_grad():
+            model(ids)
+        for h in hooks:
+            h.remove()
+        # the first candidate's page: the prompt's rows, then three steps'
+        rows = [v.flatten(1) for v in eng.pool.value.flatten(1, 2)]
+        for layer, want in zip(rows, ref):
+            at = (layer[:, None, :] - want[0]).abs().sum(-1).argmin().item()
+            assert _rel(layer[at:at + 8], want) < 0.03
