@@ -101,14 +101,12 @@ def _project(x, u, weight, bias, B, scale):
 
 
 class _Attention(torch.autograd.Function):
-    """x + o_proj(attention(qkv_proj(norm(x)))) over rows x (B*T, hidden)."""
+    """x + o_proj(attention(qkv_proj(norm(x)))) over rows x (rows, hidden)."""
 
     @staticmethod
-    def forward(ctx, x, shape, rotary, at, norm, Aq, Bq, Ak, Bk, Av, Bv, Ao,
-                Bo):
+    def forward(ctx, x, rotary, at, norm, Aq, Bq, Ak, Bk, Av, Bv, Ao, Bo):
         ext, s = _ext(), at.spec
-        pos, inv_freq, back_freq = rotary
-        B, T = shape
+        pos, inv_freq, back_freq, cu, longest = rotary
         h = ext.rmsnorm_fwd(x, norm.weight, norm.eps)
         A = torch.cat([Aq, Ak, Av])
         u = h @ A.t()
@@ -124,19 +122,18 @@ class _Attention(torch.autograd.Function):
             q = ext.rmsnorm_fwd(q0, at.q_norm.weight, at.q_norm.eps)
             k = ext.rmsnorm_fwd(k0, at.k_norm.weight, at.k_norm.eps)
         ext.rope_inplace(q, k, pos, inv_freq)
-        heads = (B, T, -1, s.head_dim)
-        q, k, v = (t.view(heads).transpose(1, 2) for t in (q, k, v))
-        o, lse = ext.flash_attn_fwd(q, k, v, at.scale)
-        o2 = o.transpose(1, 2).reshape(B * T, s.q_size)
+        v = v.view(-1, s.num_kv_heads, s.head_dim)
+        o, lse = ext.flash_varlen_fwd(q, k, v, cu, longest, at.scale)
+        o2 = o.view(-1, s.q_size)
         uo = o2 @ Ao.t()
         y = _residual(x, o2, uo, at.o_proj.weight, Bo, at.o_proj.scale)
         head_norms = ((at.q_norm.weight, at.k_norm.weight) if s.qk_norm
                       else (None, None))
         ctx.save_for_backward(x, h, A, u, Bq, Bk, Bv, Ao, Bo, q, k, v, o, lse,
-                              uo, pos, back_freq, q0, k0, *head_norms,
+                              uo, pos, back_freq, cu, q0, k0, *head_norms,
                               norm.weight, at.o_proj.weight,
                               *(m.weight for m in mods))
-        ctx.spec, ctx.shape, ctx.scale = s, shape, at.scale
+        ctx.spec, ctx.longest, ctx.scale = s, longest, at.scale
         ctx.scales = [m.scale for m in (*mods, at.o_proj)]
         ctx.eps = (norm.eps, *((at.q_norm.eps, at.k_norm.eps) if s.qk_norm
                                else ()))
@@ -146,20 +143,18 @@ class _Attention(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, g):
         (x, h, A, u, Bq, Bk, Bv, Ao, Bo, q, k, v, o, lse, uo, pos, back_freq,
-         q0, k0, q_norm, k_norm, norm, Wo, *Ws) = ctx.saved_tensors
-        ext, s, (B, T) = _ext(), ctx.spec, ctx.shape
+         cu, q0, k0, q_norm, k_norm, norm, Wo, *Ws) = ctx.saved_tensors
+        ext, s = _ext(), ctx.spec
         *scales, scale_o = ctx.scales
         g = g.contiguous()
-        rows = B * T
-        o2 = o.transpose(1, 2).reshape(rows, s.q_size)
+        rows = g.shape[0]
+        o2 = o.view(rows, s.q_size)
 
         duo = _scaled_mm(g, Bo, scale_o)
         dAo, dBo = duo.t() @ o2, _scaled_mm(g.t(), uo, scale_o)
         do = _add(g @ Wo, duo, Ao)
-        do = do.view(B, T, s.num_heads, s.head_dim).transpose(1, 2)
-        dq, dk, dv = ext.flash_attn_bwd(do, q, k, v, o, lse, ctx.scale)
-        dq, dk, dv = (t.transpose(1, 2).reshape(rows, -1, s.head_dim)
-                      for t in (dq, dk, dv))
+        dq, dk, dv = ext.flash_varlen_bwd(do.view_as(o), q, k, v, o, lse, cu,
+                                          ctx.longest, ctx.scale)
         # a rotation's gradient is the rotation by the negative angle
         ext.rope_inplace(dq, dk, pos, back_freq)
         if q0 is not None:
@@ -183,8 +178,8 @@ class _Attention(torch.autograd.Function):
             dh.addmm_(dv, Ws[2])
             _add(dh, du, A)
             dx = ext.rmsnorm_bwd_add(dh, x, norm, g, ctx.eps[0])
-        return (dx, None, None, None, None, dAq, dBs[0], dAk, dBs[1],
-                dAv, dBs[2], dAo, dBo)
+        return (dx, None, None, None, dAq, dBs[0], dAk, dBs[1], dAv, dBs[2],
+                dAo, dBo)
 
 
 class _FeedForward(torch.autograd.Function):
@@ -239,13 +234,22 @@ class _FeedForward(torch.autograd.Function):
         return dx, None, None, dAg, dBg, dAu, dBu, dAd, dBd
 
 
+def rotary(head_dim: int, theta: float, positions, cu, longest: int):
+    """What the nodes need to know of the rows: int32 positions (rows,), fp32
+    inverse frequencies and their negatives, the first row of every sequence
+    and the end (int32), the most rows of one."""
+    half = torch.arange(0, head_dim, 2, device=positions.device,
+                        dtype=torch.float32)
+    inv_freq = 1.0 / (theta ** (half / head_dim))
+    return positions.to(torch.int32), inv_freq, -inv_freq, cu, longest
+
+
 def forward(layer, x, rotary):
-    """The layer on x (B, T, hidden); rotary: int32 positions (B*T,), fp32
-    inverse frequencies and their negatives."""
+    """The layer on x, (B, T, hidden) or (rows, hidden); see rotary()."""
     at, mlp = layer.self_attn, layer.mlp
     shape = x.shape
     y = _Attention.apply(
-        x.reshape(-1, shape[-1]).contiguous(), shape[:2], rotary, at,
+        x.reshape(-1, shape[-1]).contiguous(), rotary, at,
         layer.input_layernorm,
         *(w for m in (at.q_proj, at.k_proj, at.v_proj, at.o_proj)
           for w in (m.lora_A, m.lora_B)))

@@ -130,8 +130,8 @@ class DecoderLayer(nn.Module):
         self.mlp = MLP(spec, r, alpha, dropout, dtype, device)
 
     def forward(self, x, cos, sin, attn_bias, rotary=None):
-        """rotary: (int32 positions (B*T,), inverse frequencies, their
-        negatives): the rotation of cos and sin, for the fused nodes."""
+        """rotary: the rotation of cos and sin and the rows of the sequences,
+        for the fused nodes (fused_layer.rotary)."""
         if attn_bias is None and rotary is not None and fused_layer.usable(self, x):
             return fused_layer.forward(self, x, rotary)
         x = x + self.self_attn(self.input_layernorm(x), cos, sin, attn_bias)
@@ -281,15 +281,45 @@ class CausalLM(nn.Module):
 
         rotary = None
         if input_ids.is_cuda:
-            half = torch.arange(0, self.spec.head_dim, 2, device=input_ids.device,
-                                dtype=torch.float32)
-            inv_freq = 1.0 / (self.spec.rope_theta ** (half / self.spec.head_dim))
-            rotary = (position_ids.reshape(-1).to(torch.int32), inv_freq, -inv_freq)
+            rotary = fused_layer.rotary(
+                self.spec.head_dim, self.spec.rope_theta,
+                position_ids.reshape(-1),
+                torch.arange(0, B * T + 1, T, dtype=torch.int32,
+                             device=input_ids.device), T)
         x = self.model.embed_tokens(input_ids)
         for layer in self.model.layers:
             # a layer of another class takes what the modules need
             x = (layer(x, cos, sin, bias, rotary)
                  if isinstance(layer, DecoderLayer) else layer(x, cos, sin, bias))
+        return self.model.norm(x)
+
+    def takes_rows(self) -> bool:
+        """Whether forward_rows takes this model now: every layer runs on its
+        fused nodes, and nothing hooks or replaces a part that it passes by."""
+        inner = self.model
+        embed = inner.embed_tokens
+        plain = (type(self) is CausalLM and type(inner) is _Inner
+                 and type(embed) is nn.Embedding and type(inner.norm) is RMSNorm
+                 and not {"forward", "forward_hidden", "logits"} & set(vars(self)))
+        return plain and embed.weight.is_cuda and all(
+            type(layer) is DecoderLayer and not fused_layer._hooked(layer)
+            and fused_layer.usable(layer, embed.weight)
+            for layer in inner.layers) and not any(
+            map(fused_layer._hooked,
+                [m for m in (self, inner, embed, inner.norm, self.lm_head)
+                 if m is not None]))
+
+    def forward_rows(self, input_ids: torch.Tensor, lens) -> torch.Tensor:
+        """forward_hidden of sequences that lie one behind the other, lens
+        tokens each, input_ids (rows,) -> (rows, H): no row is padding."""
+        host = torch.tensor([0, *lens], dtype=torch.int32).cumsum(0)
+        cu = host.to(torch.int32).to(input_ids.device)
+        pos = torch.cat([torch.arange(n) for n in lens]).to(input_ids.device)
+        rotary = fused_layer.rotary(self.spec.head_dim, self.spec.rope_theta,
+                                    pos, cu, max(lens))
+        x = self.model.embed_tokens(input_ids)
+        for layer in self.model.layers:
+            x = fused_layer.forward(layer, x, rotary)
         return self.model.norm(x)
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:

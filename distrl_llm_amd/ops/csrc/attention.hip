@@ -67,6 +67,17 @@ constexpr int tile_rows() { return NW == 4 ? 64 : 32; }
 // element strides of a (B, H, T, D) operand
 struct Strides { int64_t b, h; int t; };
 
+// The sequences of a batch: T rows each, or rows cu[b] .. cu[b + 1] of a flat
+// one. A (batch, heads, rows) array of numbers lies b * heads * T apart, or as
+// (heads, rows of the flat batch).
+struct Seqs {
+  const int* cu;
+  int T;            // rows of each, or of the longest
+  int64_t b, h;     // of a query head's numbers
+  DEV_INLINE int first(int i) const { return cu ? cu[i] : 0; }
+  DEV_INLINE int len(int i) const { return cu ? cu[i + 1] - cu[i] : T; }
+};
+
 DEV_INLINE f32x16 mfma(bf16v8 a, bf16v8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
@@ -234,13 +245,12 @@ DEV_INLINE int xcd_share(int id, int total) {
 }
 
 // ---------------------------------------------------------------- forward
-// Lengths: T for every sequence, or rows cu[b] .. cu[b+1] of a flat batch.
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, 2)
 void flash_fwd_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16* __restrict__ k,
                       const __hip_bfloat16* __restrict__ v, __hip_bfloat16* __restrict__ o,
-                      float* __restrict__ lse, const int* __restrict__ cu, Strides sq, Strides sk,
-                      Strides sv, Strides so, int Hq, int Hkv, int T, int nq, float scale_log2) {
+                      float* __restrict__ lse, Seqs seqs, Strides sq, Strides sk, Strides sv,
+                      Strides so, int Hq, int Hkv, int nq, float scale_log2) {
   constexpr int KV = tile_rows<NW>(), NS = KV / 32, NT = NW * 64;
   const int group = Hq / Hkv;
   int id = xcd_share(blockIdx.x, gridDim.x);
@@ -250,8 +260,7 @@ void flash_fwd_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16
   id /= nq;
   const int kvh = id % Hkv, b = id / Hkv;
   const int h = kvh * group + hg;
-  const int row0 = cu ? cu[b] : 0;
-  const int len = cu ? cu[b + 1] - row0 : T;
+  const int row0 = seqs.first(b), len = seqs.len(b);
   if (qb * (NW * WROWS) >= len) return;
 
   const int wave = wave_id(), l = threadIdx.x & 63, half = l >> 5;
@@ -351,7 +360,7 @@ void flash_fwd_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16
   lsum = halves_sum(lsum);
   store_rows<D>(acc, 1.f / lsum, o + b * so.b + h * so.h + (int64_t)(row0 + qq) * so.t, qq < len);
   if (lse != nullptr && half == 0 && qq < len)
-    lse[((int64_t)b * Hq + h) * T + qq] = m * LN2 + __logf(lsum);
+    lse[b * seqs.b + h * seqs.h + row0 + qq] = m * LN2 + __logf(lsum);
 }
 
 // ------------------------------------------------------------- backward
@@ -361,9 +370,9 @@ __global__ __launch_bounds__(NW * 64, 2)
 void flash_bwd_dq_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16* __restrict__ k,
                          const __hip_bfloat16* __restrict__ v, const __hip_bfloat16* __restrict__ o,
                          const __hip_bfloat16* __restrict__ dout, const float* __restrict__ lse,
-                         float* __restrict__ delta, __hip_bfloat16* __restrict__ dq, Strides sq,
-                         Strides sk, Strides sv, Strides so, Strides sdo, Strides sdq, int Hq,
-                         int Hkv, int T, int nq, float scale) {
+                         float* __restrict__ delta, __hip_bfloat16* __restrict__ dq, Seqs seqs,
+                         Strides sq, Strides sk, Strides sv, Strides so, Strides sdo, Strides sdq,
+                         int Hq, int Hkv, int nq, float scale) {
   constexpr int KV = tile_rows<NW>(), NS = KV / 32, NT = NW * 64;
   const int group = Hq / Hkv;
   int id = xcd_share(blockIdx.x, gridDim.x);
@@ -373,19 +382,21 @@ void flash_bwd_dq_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloa
   id /= nq;
   const int kvh = id % Hkv, b = id / Hkv;
   const int h = kvh * group + hg;
+  const int row0 = seqs.first(b), T = seqs.len(b);
+  if (qb * (NW * WROWS) >= T) return;
 
   const int wave = wave_id(), l = threadIdx.x & 63, half = l >> 5;
   const int q0 = qb * (NW * WROWS) + wave * WROWS;
   const int qq = q0 + (l & 31);
   const bool live = qq < T;
-  const __hip_bfloat16* kp = k + b * sk.b + kvh * sk.h;
-  const __hip_bfloat16* vp = v + b * sv.b + kvh * sv.h;
+  const __hip_bfloat16* kp = k + b * sk.b + kvh * sk.h + (int64_t)row0 * sk.t;
+  const __hip_bfloat16* vp = v + b * sv.b + kvh * sv.h + (int64_t)row0 * sv.t;
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int TB = KV * D * 2;
   const Frags<D> fr;
   bf16v8 qf[D / 16], dof[D / 16];
-  const int qrow = min(qq, T - 1);
+  const int qrow = row0 + min(qq, T - 1);
   load_row<D>(qf, q + b * sq.b + h * sq.h, sq.t, qrow);
   load_row<D>(dof, dout + b * sdo.b + h * sdo.h, sdo.t, qrow);
   float dl = 0.f;
@@ -398,7 +409,7 @@ void flash_bwd_dq_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloa
       for (int j = 0; j < 8; ++j) dl += (float)of[ks][j] * (float)dof[ks][j];
     dl = halves_sum(dl);
   }
-  const int64_t at = ((int64_t)b * Hq + h) * T + qq;
+  const int64_t at = b * seqs.b + h * seqs.h + row0 + qq;
   const float scale_log2 = scale * LOG2E;
   const float lse2 = live ? lse[at] * LOG2E : 1e30f;    // 1e30: weight zero
   if (live && half == 0) delta[at] = dl;
@@ -456,11 +467,12 @@ void flash_bwd_dq_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloa
       __syncthreads();
     }
   }
-  store_rows<D>(acc, scale, dq + b * sdq.b + h * sdq.h + (int64_t)qq * sdq.t, live);
+  store_rows<D>(acc, scale, dq + b * sdq.b + h * sdq.h + (int64_t)(row0 + qq) * sdq.t, live);
 }
 
 // dK, dV of one kv head's 32*NW keys, summed over query heads
-// hs*part .. of its group. Partials (split > 1) go to fp32 (split, B, Hkv, T, D).
+// hs*part .. of its group. Partials (split > 1) go to fp32 (split, B, Hkv, T, D),
+// part_rows rows a share.
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, 2)
 void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16* __restrict__ k,
@@ -468,9 +480,9 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
                           const __hip_bfloat16* __restrict__ dout, const float* __restrict__ lse,
                           const float* __restrict__ delta, __hip_bfloat16* __restrict__ dk,
                           __hip_bfloat16* __restrict__ dv, float* __restrict__ pk,
-                          float* __restrict__ pv, Strides sq, Strides sk, Strides sv, Strides sdo,
-                          Strides sdk, Strides sdv, int Hq, int Hkv, int T, int nkv, int split,
-                          float scale) {
+                          float* __restrict__ pv, Seqs seqs, Strides sq, Strides sk, Strides sv,
+                          Strides sdo, Strides sdk, Strides sdv, int Hq, int Hkv, int nkv, int split,
+                          int64_t part_rows, float scale) {
   constexpr int QT = 32, NT = NW * 64;
   const int group = Hq / Hkv;
   int id = xcd_share(blockIdx.x, gridDim.x);
@@ -479,6 +491,8 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
   const int kb = id % nkv;              // longest columns first
   id /= nkv;
   const int kvh = id % Hkv, b = id / Hkv;
+  const int row0 = seqs.first(b), T = seqs.len(b);
+  if (kb * (NW * WROWS) >= T) return;
   const int h0 = hs * group / split, h1 = (hs + 1) * group / split;
 
   const int wave = wave_id(), l = threadIdx.x & 63, half = l >> 5;
@@ -496,11 +510,11 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
   {
     Tile<D, NW * WROWS, NT> tk;
     const int r0 = kb * (NW * WROWS);
-    tk.fetch(k + b * sk.b + kvh * sk.h + (int64_t)r0 * sk.t, sk.t, T - r0);
+    tk.fetch(k + b * sk.b + kvh * sk.h + (int64_t)(row0 + r0) * sk.t, sk.t, T - r0);
     tk.store(smem);
   }
   bf16v8 vf[D / 16];
-  load_row<D>(vf, v + b * sv.b + kvh * sv.h, sv.t, min(kk, T - 1));
+  load_row<D>(vf, v + b * sv.b + kvh * sv.h, sv.t, row0 + min(kk, T - 1));
   const float scale_log2 = scale * LOG2E;
 
   f32x16 ak[D / 32], av[D / 32];
@@ -512,11 +526,11 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
   float stat = 0.f;     // threads 0..31: lse, 32..63: delta of the tile's rows
   int fh = kvh * group + h0, fr0 = first;              // the next tile to fetch
   auto fetch = [&] {
-    tq.fetch(q + b * sq.b + fh * sq.h + (int64_t)fr0 * sq.t, sq.t, T - fr0);
-    td.fetch(dout + b * sdo.b + fh * sdo.h + (int64_t)fr0 * sdo.t, sdo.t, T - fr0);
+    tq.fetch(q + b * sq.b + fh * sq.h + (int64_t)(row0 + fr0) * sq.t, sq.t, T - fr0);
+    td.fetch(dout + b * sdo.b + fh * sdo.h + (int64_t)(row0 + fr0) * sdo.t, sdo.t, T - fr0);
     if (threadIdx.x < 64) {
       const int r = fr0 + (threadIdx.x & 31);
-      const float* p = (threadIdx.x < 32 ? lse : delta) + ((int64_t)b * Hq + fh) * T;
+      const float* p = (threadIdx.x < 32 ? lse : delta) + b * seqs.b + fh * seqs.h + row0;
       stat = p[min(r, T - 1)];
       // rows past the end get weight exp(-huge) = 0
       if (threadIdx.x < 32) stat = r < T ? stat * LOG2E : 1e30f;
@@ -580,10 +594,11 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
   }
 
   if (split == 1) {
-    store_rows<D>(ak, scale, dk + b * sdk.b + kvh * sdk.h + (int64_t)kk * sdk.t, live);
-    store_rows<D>(av, 1.f, dv + b * sdv.b + kvh * sdv.h + (int64_t)kk * sdv.t, live);
+    store_rows<D>(ak, scale, dk + b * sdk.b + kvh * sdk.h + (int64_t)(row0 + kk) * sdk.t, live);
+    store_rows<D>(av, 1.f, dv + b * sdv.b + kvh * sdv.h + (int64_t)(row0 + kk) * sdv.t, live);
   } else {
-    const int64_t at = ((((int64_t)hs * (gridDim.x / (split * nkv * Hkv)) + b) * Hkv + kvh) * T + kk) * D;
+    // rows as the query heads' numbers lie, of Hkv heads
+    const int64_t at = (hs * part_rows + b * (seqs.b / Hq) * Hkv + kvh * seqs.h + row0 + kk) * D;
     store_rows_f32<D>(ak, pk + at, live);
     store_rows_f32<D>(av, pv + at, live);
   }
@@ -677,6 +692,11 @@ int waves_for(int64_t rows_of_heads, int T) { return rows_of_heads * ((T + 127) 
     else { constexpr int D = 64, NW = 2; __VA_ARGS__; }                          \
   }()
 
+// B sequences of T rows, or (cu) of up to T rows of one flat batch
+Seqs sequences(const torch::Tensor& q, const int* cu, int T) {
+  return {cu, T, cu ? 0 : q.size(1) * q.size(2), q.size(2)};
+}
+
 void launch_fwd(const torch::Tensor& q, const torch::Tensor& k, const torch::Tensor& v,
                 torch::Tensor& o, float* lse, const int* cu, int B, int T, double scale) {
   const int Hq = q.size(1), Hkv = k.size(1);
@@ -689,10 +709,77 @@ void launch_fwd(const torch::Tensor& q, const torch::Tensor& k, const torch::Ten
   FLASH_DISPATCH(q.size(3), nw, {
     const size_t smem = 4 * tile_rows<NW>() * D * 2;
     hipLaunchKernelGGL((flash_fwd_kernel<D, NW>), dim3(blocks), dim3(NW * 64), smem, stream, bf(q),
-                       bf(k), bf(v), bfm(o), lse, cu, strides(q, cu), strides(k, cu),
-                       strides(v, cu), strides(o, cu), Hq, Hkv, T, nq, (float)scale * LOG2E);
+                       bf(k), bf(v), bfm(o), lse, sequences(q, cu, T), strides(q, cu),
+                       strides(k, cu), strides(v, cu), strides(o, cu), Hq, Hkv, nq,
+                       (float)scale * LOG2E);
   });
   HIP_CHECK_LAST();
+}
+
+std::vector<torch::Tensor> launch_bwd(const torch::Tensor& dout, const torch::Tensor& q,
+                                      const torch::Tensor& k, const torch::Tensor& v,
+                                      const torch::Tensor& o, const torch::Tensor& lse,
+                                      const int* cu, int B, int T, double scale) {
+  check_qkv(q, k, v);
+  TORCH_CHECK(dout.scalar_type() == at::kBFloat16 && o.scalar_type() == at::kBFloat16 &&
+              lse.scalar_type() == at::kFloat);
+  TORCH_CHECK(dout.sizes() == q.sizes() && o.sizes() == q.sizes(),
+              "flash_attn_bwd: dout/o shape mismatch");
+  const int Hq = q.size(1), Hkv = k.size(1);
+  const int64_t rows_all = q.size(0) * q.size(2);
+  TORCH_CHECK(lse.numel() == Hq * rows_all, "flash_attn_bwd: lse shape mismatch");
+  auto qc = rows16(q), kc = rows16(k), vc = rows16(v), oc = rows16(o), doc = rows16(dout);
+  auto lsec = lse.contiguous();
+  auto delta = torch::empty_like(lsec);
+  auto dq = like(qc), dk = like(kc), dv = like(vc);
+  const int nw = waves_for((int64_t)B * Hq, T);
+  const int rows = nw * WROWS, nq = (T + rows - 1) / rows;
+  const int64_t blocks = (int64_t)B * Hq * nq, kv_blocks = (int64_t)B * Hkv * nq;
+  if (blocks == 0) return {dq, dk, dv};
+  TORCH_CHECK(blocks < (1ll << 31), "flash attention: batch too large");
+  const int group = Hq / Hkv;
+  const int split = (int)std::min<int64_t>(group, (1024 + kv_blocks - 1) / kv_blocks);
+  torch::Tensor part;
+  float *pk = nullptr, *pv = nullptr;
+  if (split > 1) {
+    part = torch::empty({2, split, Hkv * rows_all, q.size(3)}, lsec.options());
+    pk = part.data_ptr<float>();
+    pv = pk + part.numel() / 2;
+  }
+  const Seqs seqs = sequences(q, cu, T);
+  auto st = [&](const torch::Tensor& x) { return strides(x, cu); };
+  auto stream = at::cuda::getCurrentCUDAStream();
+  FLASH_DISPATCH(q.size(3), nw, {
+    hipLaunchKernelGGL((flash_bwd_dq_kernel<D, NW>), dim3(blocks), dim3(NW * 64), 4 * tile_rows<NW>() * D * 2,
+                       stream, bf(qc), bf(kc), bf(vc), bf(oc), bf(doc), lsec.data_ptr<float>(),
+                       delta.data_ptr<float>(), bfm(dq), seqs, st(qc), st(kc), st(vc), st(oc),
+                       st(doc), st(dq), Hq, Hkv, nq, (float)scale);
+    hipLaunchKernelGGL((flash_bwd_dkv_kernel<D, NW>), dim3(kv_blocks * split), dim3(NW * 64),
+                       NW * WROWS * D * 2 + 2 * (2 * 32 * D * 2 + 32 * 8), stream, bf(qc), bf(kc), bf(vc), bf(doc),
+                       lsec.data_ptr<float>(), delta.data_ptr<float>(), bfm(dk), bfm(dv), pk, pv,
+                       seqs, st(qc), st(kc), st(vc), st(doc), st(dk), st(dv), Hq, Hkv, nq, split,
+                       Hkv * rows_all, (float)scale);
+    if (split > 1) {
+      const int64_t n = Hkv * rows_all;
+      hipLaunchKernelGGL((flash_bwd_sum_kernel<D>), dim3((n * (D / 8) + 255) / 256), dim3(256), 0,
+                         stream, pk, pv, bfm(dk), bfm(dv), strides(dk), strides(dv), Hkv,
+                         (int)q.size(2), n, split, (float)scale);
+    }
+  });
+  HIP_CHECK_LAST();
+  return {dq, dk, dv};
+}
+
+// A flat (tokens, H, D) batch as one (1, H, tokens, D) operand
+torch::Tensor flat4(const torch::Tensor& x) {
+  TORCH_CHECK(x.dim() == 3);
+  return x.transpose(0, 1).unsqueeze(0);
+}
+
+void check_cu(const torch::Tensor& q, const torch::Tensor& cu, int64_t max_len) {
+  TORCH_CHECK(cu.is_cuda() && cu.scalar_type() == at::kInt && cu.is_contiguous() && cu.dim() == 1 &&
+              cu.numel() >= 1);
+  TORCH_CHECK(max_len >= 0 && max_len <= q.size(0));
 }
 
 }  // namespace
@@ -709,71 +796,41 @@ std::vector<torch::Tensor> flash_attn_fwd(torch::Tensor q, torch::Tensor k, torc
 
 // Causal attention inside each of the sequences cu[i] .. cu[i+1] of a flat
 // batch: q (tokens, Hq, D), k/v (tokens, Hkv, D), cu int32 (n+1,) rising from
-// 0 to tokens, max_len the longest of them.
-torch::Tensor flash_attn_varlen(torch::Tensor q, torch::Tensor k, torch::Tensor v,
-                                torch::Tensor cu, int64_t max_len, double scale) {
-  TORCH_CHECK(q.dim() == 3 && k.dim() == 3 && v.dim() == 3);
-  TORCH_CHECK(cu.is_cuda() && cu.scalar_type() == at::kInt && cu.is_contiguous() && cu.dim() == 1 &&
-              cu.numel() >= 1);
-  auto as4 = [](const torch::Tensor& x) { return x.transpose(0, 1).unsqueeze(0); };
-  auto q4 = as4(q), k4 = as4(k), v4 = as4(v);
+// 0 to tokens, max_len the longest of them. {output, log-sum-exp (Hq, tokens)}.
+std::vector<torch::Tensor> flash_varlen_fwd(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                                            torch::Tensor cu, int64_t max_len, double scale) {
+  auto q4 = flat4(q), k4 = flat4(k), v4 = flat4(v);
+  check_cu(q, cu, max_len);
   check_qkv(q4, k4, v4);
-  TORCH_CHECK(max_len >= 0 && max_len <= q.size(0));
   auto qc = rows16(positive_scale(q4, scale)), kc = rows16(k4), vc = rows16(v4);
   auto out = torch::empty(q.sizes(), q.options());
-  auto o4 = as4(out);
-  launch_fwd(qc, kc, vc, o4, nullptr, cu.data_ptr<int>(), cu.numel() - 1, max_len, scale);
-  return out;
+  auto lse = torch::empty({q.size(1), q.size(0)}, q.options().dtype(at::kFloat));
+  auto o4 = flat4(out);
+  launch_fwd(qc, kc, vc, o4, lse.data_ptr<float>(), cu.data_ptr<int>(), cu.numel() - 1, max_len,
+             scale);
+  return {out, lse};
+}
+
+torch::Tensor flash_attn_varlen(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                                torch::Tensor cu, int64_t max_len, double scale) {
+  return flash_varlen_fwd(q, k, v, cu, max_len, scale)[0];
 }
 
 std::vector<torch::Tensor> flash_attn_bwd(torch::Tensor dout, torch::Tensor q, torch::Tensor k,
                                           torch::Tensor v, torch::Tensor o, torch::Tensor lse,
                                           double scale) {
-  check_qkv(q, k, v);
-  TORCH_CHECK(dout.scalar_type() == at::kBFloat16 && o.scalar_type() == at::kBFloat16 &&
-              lse.scalar_type() == at::kFloat);
-  TORCH_CHECK(dout.sizes() == q.sizes() && o.sizes() == q.sizes(),
-              "flash_attn_bwd: dout/o shape mismatch");
-  const int B = q.size(0), Hq = q.size(1), T = q.size(2), Hkv = k.size(1);
-  TORCH_CHECK(lse.numel() == (int64_t)B * Hq * T, "flash_attn_bwd: lse shape mismatch");
-  auto qc = rows16(q), kc = rows16(k), vc = rows16(v), oc = rows16(o), doc = rows16(dout);
-  auto lsec = lse.contiguous();
-  auto delta = torch::empty_like(lsec);
-  auto dq = like(qc), dk = like(kc), dv = like(vc);
-  const int nw = waves_for((int64_t)B * Hq, T);
-  const int rows = nw * WROWS, nq = (T + rows - 1) / rows;
-  const int64_t blocks = (int64_t)B * Hq * nq, kv_blocks = (int64_t)B * Hkv * nq;
-  if (blocks == 0) return {dq, dk, dv};
-  TORCH_CHECK(blocks < (1ll << 31), "flash attention: batch too large");
-  const int group = Hq / Hkv;
-  const int split = (int)std::min<int64_t>(group, (1024 + kv_blocks - 1) / kv_blocks);
-  torch::Tensor part;
-  float *pk = nullptr, *pv = nullptr;
-  if (split > 1) {
-    part = torch::empty({2, split, B, Hkv, T, q.size(3)}, lsec.options());
-    pk = part.data_ptr<float>();
-    pv = pk + part.numel() / 2;
-  }
-  auto stream = at::cuda::getCurrentCUDAStream();
-  FLASH_DISPATCH(q.size(3), nw, {
-    hipLaunchKernelGGL((flash_bwd_dq_kernel<D, NW>), dim3(blocks), dim3(NW * 64), 4 * tile_rows<NW>() * D * 2,
-                       stream, bf(qc), bf(kc), bf(vc), bf(oc), bf(doc), lsec.data_ptr<float>(),
-                       delta.data_ptr<float>(), bfm(dq), strides(qc), strides(kc), strides(vc),
-                       strides(oc), strides(doc), strides(dq), Hq, Hkv, T, nq, (float)scale);
-    hipLaunchKernelGGL((flash_bwd_dkv_kernel<D, NW>), dim3(kv_blocks * split), dim3(NW * 64),
-                       NW * WROWS * D * 2 + 2 * (2 * 32 * D * 2 + 32 * 8), stream, bf(qc), bf(kc), bf(vc), bf(doc),
-                       lsec.data_ptr<float>(), delta.data_ptr<float>(), bfm(dk), bfm(dv), pk, pv,
-                       strides(qc), strides(kc), strides(vc), strides(doc), strides(dk),
-                       strides(dv), Hq, Hkv, T, nq, split, (float)scale);
-    if (split > 1) {
-      const int64_t n = (int64_t)B * Hkv * T;
-      hipLaunchKernelGGL((flash_bwd_sum_kernel<D>), dim3((n * (D / 8) + 255) / 256), dim3(256), 0,
-                         stream, pk, pv, bfm(dk), bfm(dv), strides(dk), strides(dv), Hkv, T, n,
-                         split, (float)scale);
-    }
-  });
-  HIP_CHECK_LAST();
-  return {dq, dk, dv};
+  return launch_bwd(dout, q, k, v, o, lse, nullptr, q.size(0), q.size(2), scale);
+}
+
+// {dq, dk, dv} of flash_varlen_fwd, (tokens, H, D)
+std::vector<torch::Tensor> flash_varlen_bwd(torch::Tensor dout, torch::Tensor q, torch::Tensor k,
+                                            torch::Tensor v, torch::Tensor o, torch::Tensor lse,
+                                            torch::Tensor cu, int64_t max_len, double scale) {
+  check_cu(q, cu, max_len);
+  auto r = launch_bwd(flat4(dout), flat4(q), flat4(k), flat4(v), flat4(o), lse, cu.data_ptr<int>(),
+                      cu.numel() - 1, max_len, scale);
+  for (auto& t : r) t = t.squeeze(0).transpose(0, 1);
+  return r;
 }
 
 // The differentiable call: a node of the C++ engine (from Python, node and

@@ -90,9 +90,19 @@ torch::Tensor flash_attention(torch::Tensor q, torch::Tensor k, torch::Tensor v,
 torch::Tensor logprob_loss(torch::Tensor logits, torch::Tensor targets,
                            torch::Tensor mask, torch::Tensor rewards,
                            double scale);
+torch::Tensor logprob_rows(torch::Tensor logits, torch::Tensor targets,
+                           torch::Tensor w);
 torch::Tensor flash_attn_varlen(torch::Tensor q, torch::Tensor k,
                                 torch::Tensor v, torch::Tensor cu,
                                 int64_t max_len, double scale);
+std::vector<torch::Tensor> flash_varlen_fwd(torch::Tensor q, torch::Tensor k,
+                                            torch::Tensor v, torch::Tensor cu,
+                                            int64_t max_len, double scale);
+std::vector<torch::Tensor> flash_varlen_bwd(torch::Tensor dout, torch::Tensor q,
+                                            torch::Tensor k, torch::Tensor v,
+                                            torch::Tensor o, torch::Tensor lse,
+                                            torch::Tensor cu, int64_t max_len,
+                                            double scale);
 std::vector<torch::Tensor> flash_attn_bwd(torch::Tensor dout, torch::Tensor q,
                                           torch::Tensor k, torch::Tensor v,
                                           torch::Tensor o, torch::Tensor lse,
@@ -181,8 +191,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("flash_attention", &flash_attention,
         "differentiable causal GQA flash attention");
   m.def("logprob_loss", &logprob_loss, "differentiable masked PG/GRPO loss");
+  m.def("logprob_rows", &logprob_rows,
+        "differentiable weighted sum of token log-probabilities");
   m.def("flash_attn_varlen", &flash_attn_varlen,
         "causal GQA flash attention over a flat batch of sequences");
+  m.def("flash_varlen_fwd", &flash_varlen_fwd,
+        "the same with its log-sum-exp");
+  m.def("flash_varlen_bwd", &flash_varlen_bwd, "its backward (dq, dk, dv)");
   m.def("flash_attn_bwd", &flash_attn_bwd,
         "causal GQA flash attention backward (returns dq, dk, dv)");
 }

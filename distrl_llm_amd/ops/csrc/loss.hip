@@ -122,6 +122,17 @@ void loss_reduce_kernel(const float* __restrict__ token_logp, const M* __restric
   }
 }
 
+// sum of w * token_logp over rows, in an order of its own for every row count
+__global__ __launch_bounds__(1024)
+void loss_rows_kernel(const float* __restrict__ token_logp, const float* __restrict__ w,
+                      float* __restrict__ loss, int64_t rows) {
+  __shared__ float red[16];
+  float sum = 0.f;
+  for (int64_t i = threadIdx.x; i < rows; i += 1024) sum += w[i] * token_logp[i];
+  sum = block_sum(sum, red);
+  if (threadIdx.x == 0) *loss = sum;
+}
+
 template <typename T>
 __global__ __launch_bounds__(256)
 void loss_bwd_kernel(const T* __restrict__ logits,
@@ -295,4 +306,40 @@ struct LogprobLoss : public torch::autograd::Function<LogprobLoss> {
 torch::Tensor logprob_loss(torch::Tensor logits, torch::Tensor targets, torch::Tensor mask,
                            torch::Tensor rewards, double scale) {
   return LogprobLoss::apply(logits, targets, mask, rewards, scale);
+}
+
+// The same sum for rows that carry weights of their own: sum_i w_i log p(target_i)
+// of logits (rows, V); no gradient for the weights.
+namespace {
+
+struct LogprobRows : public torch::autograd::Function<LogprobRows> {
+  static torch::Tensor forward(torch::autograd::AutogradContext* ctx, torch::Tensor logits,
+                               torch::Tensor targets, torch::Tensor w) {
+    TORCH_CHECK(logits.dim() == 2 && targets.is_cuda() && w.is_cuda() &&
+                targets.numel() == logits.size(0) && w.numel() == logits.size(0) &&
+                w.scalar_type() == at::kFloat, "logprob_rows: shape mismatch");
+    logits = logits.contiguous();
+    targets = targets.contiguous();
+    w = w.contiguous();
+    auto lp = logprob_lse_fwd(logits, targets);
+    auto loss = torch::empty({}, lp[0].options());
+    hipLaunchKernelGGL(loss_rows_kernel, dim3(1), dim3(1024), 0, at::cuda::getCurrentCUDAStream(),
+                       lp[0].data_ptr<float>(), w.data_ptr<float>(), loss.data_ptr<float>(),
+                       logits.size(0));
+    HIP_CHECK_LAST();
+    ctx->save_for_backward({logits, targets, w, lp[1]});
+    return loss;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto s = ctx->get_saved_variables();
+    auto d = logprob_loss_bwd(s[0], s[1], s[2], s[3], grads[0].to(at::kFloat));
+    return {d, torch::Tensor(), torch::Tensor()};
+  }
+};
+
+}  // namespace
+
+torch::Tensor logprob_rows(torch::Tensor logits, torch::Tensor targets, torch::Tensor w) {
+  return LogprobRows::apply(logits, targets, w);
 }

@@ -345,3 +345,10 @@ def logprob_loss(logits: torch.Tensor, targets: torch.Tensor, mask: torch.Tensor
                 / logits.shape[0] * loss_scale)
         return ((tok * m).sum(-1) * coef).sum()
     return _LogprobLossFn.apply(logits, targets, mask, rewards, loss_scale)
+
+
+def logprob_rows(logits: torch.Tensor, targets: torch.Tensor,
+                 w: torch.Tensor) -> torch.Tensor:
+    """sum_i w_i log p(target_i) of logits (rows, V) on the GPU: logprob_loss
+    for rows of any number of sequences, each with its weight in the loss."""
+    return _require_ext("logprob_rows").logprob_rows(logits, targets, w)

@@ -59,6 +59,11 @@ class Learner:
 
     # ------------------------------------------------------- tokenization
 
+    def _encode(self, problems: Sequence[str], answers: Sequence[str]):
+        P, A = self.max_prompt_tokens, self.max_new_tokens
+        return [(self.tokenizer.encode(p)[:P], self.tokenizer.encode(a)[:A])
+                for p, a in zip(problems, answers)]
+
     def _encode_batch(self, problems: Sequence[str], answers: Sequence[str]):
         """Packed right-padded layout: [prompt(<=max_prompt) | answer
         (<=max_new) | pad]. Keeps the reference's truncation semantics
@@ -69,8 +74,7 @@ class Learner:
         """
         P, A = self.max_prompt_tokens, self.max_new_tokens
         B = len(problems)
-        enc = [(self.tokenizer.encode(p)[:P], self.tokenizer.encode(a)[:A])
-               for p, a in zip(problems, answers)]
+        enc = self._encode(problems, answers)
         T = max(len(pi) + len(ai) for pi, ai in enc)
         T = min((T + 7) // 8 * 8, P + A)  # pad batch length to multiple of 8
         A_max = max(max(len(ai) for _, ai in enc), 1)
@@ -96,8 +100,38 @@ class Learner:
 
     # -------------------------------------------------------------- loss
 
+    def _rows_loss(self, enc, rewards: torch.Tensor,
+                   loss_scale: float) -> torch.Tensor:
+        """The loss on rows without padding: samples one behind the other
+        through the layers, and only the rows that predict an answer's token
+        through the LM head, each with its weight in the loss. Where answers
+        run from half the longest to all of it, a quarter of a padded
+        micro-batch is padding."""
+        lens = [len(p) + len(a) for p, a in enc]
+        n_ans = [len(a) for _, a in enc]
+        first, at = 0, []
+        for (p, a), n in zip(enc, lens):
+            start = first + max(len(p) - 1, 0)
+            at.append(torch.arange(start, start + len(a)))
+            first += n
+        dev, n_ans = self.device, torch.tensor(n_ans)
+        ids = torch.tensor([t for p, a in enc for t in p + a]).to(dev)
+        targets = torch.tensor([t for _, a in enc for t in a]).to(dev)
+        share = (-loss_scale / (n_ans * len(enc))).repeat_interleave(n_ans)
+        sample = torch.arange(len(enc)).repeat_interleave(n_ans)
+        hidden = self.model.forward_rows(ids, [n for n in lens if n])
+        logits = self.model.logits(hidden.index_select(0, torch.cat(at).to(dev)))
+        return OF.logprob_rows(logits, targets,
+                               rewards[sample.to(dev)] * share.to(dev))
+
     def _micro_loss(self, problems, answers, rewards: torch.Tensor,
                     loss_scale: float) -> torch.Tensor:
+        takes_rows = getattr(self.model, "takes_rows", None)
+        if (takes_rows is not None and takes_rows()
+                and type(self)._encode_batch is Learner._encode_batch):
+            enc = self._encode(problems, answers)
+            if any(a for _, a in enc):
+                return self._rows_loss(enc, rewards, loss_scale)
         input_ids, attn, targets, ans_mask, gidx = self._encode_batch(
             problems, answers)
         hidden = self.model.forward_hidden(input_ids, attn)

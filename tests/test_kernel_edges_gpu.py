@@ -765,3 +765,74 @@ def test_loss_broadcasts(lead, mask_shape, reward_shape, host):
     ref = ((tok * m).sum(-1) * (-rewards.cuda().double() / m.sum(-1).clamp_min(1) / lead[0] * 0.5)).sum()
     assert float((loss - ref).detach().abs()) < 1e-5 * float(tok.detach().abs().max())
     assert _rel(grad, torch.autograd.grad(ref, x)[0]) < 2.0 ** -8
+
+
+# ------------------------------------------------- training without padding
+
+@pytest.mark.parametrize("lens", [[1], [33, 1, 64, 65], [200, 5, 129]])
+@pytest.mark.parametrize("H,KV,D", [(4, 2, 64), (7, 1, 128), (14, 2, 64)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_flash_varlen_backward(ext, lens, H, KV, D, packed):
+    """Each sequence of a flat batch against itself alone; rows of their own
+    and cut out of wider ones."""
+    T = sum(lens)
+    rows = _rand((T, (H + 2 * KV) * D), 1)
+    q, k, v = (t.unflatten(1, (-1, D)) for t in rows.split([H * D, KV * D, KV * D], 1))
+    if not packed:
+        q, k, v = (t.contiguous() for t in (q, k, v))
+    dout = _rand((T, H, D), 2, 0.1)
+    cu = torch.tensor([0, *lens]).cumsum(0).to("cuda", torch.int32)
+    o, lse = ext.flash_varlen_fwd(q, k, v, cu, max(lens), D ** -0.5)
+    got = (o, *ext.flash_varlen_bwd(dout, q, k, v, o, lse, cu, max(lens), D ** -0.5))
+    start = 0
+    for n in lens:
+        part = [t[start:start + n].transpose(0, 1).unsqueeze(0) for t in (q, k, v, dout)]
+        for x, y in zip(got, _flash_reference(*part, D ** -0.5)):
+            # a single row's dq and dk are 0: fp32 roundings of terms of dout's size
+            off = (x[start:start + n].transpose(0, 1).double() - y[0].double()).norm()
+            assert off < FLASH_REL * y.double().norm() + 2.0 ** -18 * dout.double().norm()
+        start += n
+
+
+@pytest.mark.parametrize("rows,V", [(1, 7), (3, 4103), (1500, 4096)])
+def test_logprob_rows(ext, rows, V):
+    """Value and gradient against fp64; rows of weight zero. Bounds: bf16
+    gradient, and for the value as many fp32 roundings as there are rows."""
+    from distrl_llm_amd.ops import functional as OF
+    logits, g = _rand((rows, V), 1, 2.0).requires_grad_(), torch.Generator().manual_seed(2)
+    targets = torch.randint(0, V, (rows,), generator=g).cuda()
+    w = torch.randn(rows, generator=g).cuda() * (torch.arange(rows, device="cuda") % 3 != 1)
+    loss = OF.logprob_rows(logits, targets, w)
+    grad, = torch.autograd.grad(loss * 2, logits)
+    x = logits.detach().double().requires_grad_()
+    terms = x.log_softmax(-1).gather(1, targets[:, None])[:, 0] * w.double()
+    ref, = torch.autograd.grad(terms.sum() * 2, x)
+    assert abs(float(loss) - float(terms.sum())) < 1e-5 * float(terms.abs().sum())
+    assert _rel(grad, ref) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("prompts,answers", [([9, 30, 1], [40, 7, 100]), ([0, 5, 3], [4, 0, 6]),
+                                             ([3], [1]), ([4, 2], [0, 0])])
+def test_learner_rows_match_padding(prompts, answers):
+    """Loss and adapter gradients without padding against the padded batch (two
+    bf16 paths of the same sums: 1 %), with empty prompts and answers; a hook
+    on a part keeps the padded batch."""
+    from distrl_llm_amd.train.learner import Learner
+    from distrl_llm_amd.utils.tokenizer import ByteTokenizer
+    model = _train_model("small-qwen2")
+    learner = Learner(model, ByteTokenizer(model.spec.vocab_size), lr=1e-4, max_prompt_tokens=64,
+                      max_new_tokens=128, train_batch_size=4)
+    enc = [([5 + i] * p, [7 + i + j % 9 for j in range(a)])
+           for i, (p, a) in enumerate(zip(prompts, answers))]
+    learner._encode = lambda problems, answers: enc
+    rewards, got = torch.tensor([0.5, -1.0, 0.8][:len(enc)], device="cuda"), []
+    for rows in (True, False):
+        if not rows:
+            handle = model.model.norm.register_forward_hook(lambda m, i, o: None)
+        assert model.takes_rows() == rows
+        loss = learner._micro_loss(enc, enc, rewards, 0.5)
+        grads = torch.autograd.grad(loss, learner.params, allow_unused=True)
+        got.append((loss.detach(), torch.cat([g.reshape(-1).double() for g in grads])))
+    handle.remove()
+    assert abs(float(got[0][0]) - float(got[1][0])) < 0.01 * abs(float(got[1][0])) + 1e-6
+    assert _rel(got[0][1], got[1][1]) < 0.01 or not any(answers)
