@@ -6,13 +6,14 @@ The module-by-module layer launches ~200 kernels forward and backward, most
 of them elementwise passes between the products (residual adds, adapter
 scaling, gradient sums of projections that share an input, rotary steps,
 head transposes), and short micro-batches are bound by launching them. Here
-sums accumulate inside the products (beta = 1, in place), the adapters of
-projections that share an input share one down product, and rotary, norm and
-activation passes are one kernel each: ~65 launches.
-
-A micro-batch of three short samples on a 24-layer 0.5B model: 58 ms to
-28 ms (34 with the library adding the adapters); 16 x 1550 tokens on a
-28-layer 1.5B model: 380 to 239 ms.
+an adapter is more of its projection: u = scale * x A^T lies beside x in one
+matrix, [x | u], and one product with [W | B] gives every projection of that
+input, adapters and (beta = 1) the residual in its fp32 sums; backward is
+[dY | dU] [W; A]. Laying W out beside its adapter costs a copy of the weights,
+37 us a layer of the 1.5B model forward and as long backward, where adding the
+adapters' outputs to 18800 rows in passes of their own took 750. Adapter
+gradients are one launch and its sum (ops/csrc/adapter_grads.hip). Rotary, norm
+and activation passes are one kernel each: ~38 launches.
 """
 
 from __future__ import annotations
@@ -61,6 +62,7 @@ def usable(layer, x) -> bool:
     if at.spec.qk_norm:
         norms += [at.q_norm, at.k_norm]
     return (at.spec.head_dim in (64, 128)
+            and at.spec.hidden_size % 8 == at.spec.intermediate_size % 8 == 0
             and all(_trainable(m) for m in linears)
             and at.o_proj.bias is None and mlp.down_proj.bias is None
             and all(type(n) is RMSNorm and n.weight.dtype == torch.bfloat16
@@ -73,6 +75,11 @@ def _ext():
     return _require_ext("fused decoder layer")
 
 
+def _add(y, u, m, scale=1.0):
+    """y += scale * u m, in place; m as it lies or a transposed view."""
+    return y if _ext().lora_add(y, u, m, scale) else y.addmm_(u, m, alpha=scale)
+
+
 def _scaled_mm(a, b, scale, out=None):
     """scale * a @ b, the scale in the product's epilogue."""
     if out is None:
@@ -80,24 +87,59 @@ def _scaled_mm(a, b, scale, out=None):
     return torch.addmm(out, a, b, beta=0.0, alpha=scale, out=out)
 
 
-def _add(y, u, m, scale=1.0):
-    """y += scale * u m, in place; m as it lies or a transposed view."""
-    return y if _ext().lora_add(y, u, m, scale) else y.addmm_(u, m, alpha=scale)
+def _padded(ranks) -> int:
+    """Columns that adapters of such ranks get beside their input."""
+    return (sum(ranks) + 7) // 8 * 8
 
 
-def _residual(res, x, u, weight, B, scale):
-    """res + x W^T + scale * u B^T. The residual joins in the last sum: added
-    in the product, it would be rounded at its own size twice."""
-    y = x @ weight.t()
-    if _ext().lora_add(y, u, B.t(), scale, res):
-        return y
-    return y.addmm_(u, B.t(), alpha=scale).add_(res)
+def _beside(x, width: int):
+    """A matrix of x's rows, `width` columns and some more; its two parts."""
+    return x, x[:, :width], x[:, width:]
 
 
-def _project(x, u, weight, bias, B, scale):
-    """x W^T + b + scale * u B^T."""
-    y = x @ weight.t() if bias is None else torch.addmm(bias, x, weight.t())
-    return _add(y, u, B.t(), scale)
+def _down(x, u, As, scales) -> None:
+    """u <- the adapters' scaled inputs side by side, zeros in spare columns."""
+    ranks = [a.shape[0] for a in As]
+    A = torch.cat(As) if len(As) > 1 else As[0]
+    if len(set(scales)) == 1:
+        _scaled_mm(x, A.t(), scales[0], out=u[:, :sum(ranks)])
+    else:
+        for a, part, scale in zip(As, u[:, :sum(ranks)].split(ranks, 1), scales):
+            _scaled_mm(x, a.t(), scale, out=part)
+    if u.shape[1] > sum(ranks):
+        u[:, sum(ranks):].zero_()
+
+
+def _product(xu, W, mods):
+    """xu W^T + the modules' biases."""
+    if all(m.bias is None for m in mods):
+        return xu @ W.t()
+    return torch.addmm(torch.cat([
+        m.bias if m.bias is not None else xu.new_zeros(m.out_features)
+        for m in mods]), xu, W.t())
+
+
+def _up(dys, us, Bs, scales) -> None:
+    """us <- the gradients of the adapters' inputs."""
+    for dy, u, b, scale in zip(dys, us, Bs, scales):
+        _scaled_mm(dy, b, scale, out=u)
+
+
+def _sums(jobs):
+    """p^T y of every (y, p, transposed) over the rows: gradients of A, or of B
+    (transposed). Ranks that the kernel does not take go through the library."""
+    own = [i for i, (y, p, _) in enumerate(jobs)
+           if p.shape[1] % 8 == 0 and 8 <= p.shape[1] <= 128
+           and y.shape[1] % 8 == 0 and p.shape[0] > 0]
+    out = [None] * len(jobs)
+    if own:
+        got = _ext().adapter_grads(*map(list, zip(*(jobs[i] for i in own))))
+        for i, g in zip(own, got):
+            out[i] = g
+    for i, (y, p, transposed) in enumerate(jobs):
+        if out[i] is None:
+            out[i] = y.t() @ p if transposed else p.t() @ y
+    return out
 
 
 class _Attention(torch.autograd.Function):
@@ -107,34 +149,40 @@ class _Attention(torch.autograd.Function):
     def forward(ctx, x, rotary, at, norm, Aq, Bq, Ak, Bk, Av, Bv, Ao, Bo):
         ext, s = _ext(), at.spec
         pos, inv_freq, back_freq, cu, longest = rotary
-        h = ext.rmsnorm_fwd(x, norm.weight, norm.eps)
-        A = torch.cat([Aq, Ak, Av])
-        u = h @ A.t()
-        uq, uk, uv = u.split([Aq.shape[0], Ak.shape[0], Av.shape[0]], 1)
+        rows, hidden = x.shape
         mods = (at.q_proj, at.k_proj, at.v_proj)
-        q, k, v = (_project(h, p, m.weight, m.bias, b, m.scale)
-                   for m, p, b in zip(mods, (uq, uk, uv), (Bq, Bk, Bv)))
-        q = q.view(-1, s.num_heads, s.head_dim)
-        k = k.view(-1, s.num_kv_heads, s.head_dim)
+        scales = [m.scale for m in (*mods, at.o_proj)]
+        As, Bs, Ws = [Aq, Ak, Av], [Bq, Bk, Bv], [m.weight for m in mods]
+        pad = _padded([a.shape[0] for a in As])
+        hu, h, u = _beside(x.new_empty(rows, hidden + pad), hidden)
+        ext.rmsnorm_fwd_into(x, norm.weight, norm.eps, h)
+        _down(h, u, As, scales[:3])
+        W = ext.adapted_weight(Ws, As, Bs, pad, False)
+        qkv = _product(hu, W, mods)
+        q, k, v = (t.unflatten(1, (-1, s.head_dim))
+                   for t in qkv.split([s.q_size, s.kv_size, s.kv_size], 1))
         q0 = k0 = None
         if s.qk_norm:
-            q0, k0 = q, k
+            q0, k0 = q.contiguous(), k.contiguous()
             q = ext.rmsnorm_fwd(q0, at.q_norm.weight, at.q_norm.eps)
             k = ext.rmsnorm_fwd(k0, at.k_norm.weight, at.k_norm.eps)
-        ext.rope_inplace(q, k, pos, inv_freq)
-        v = v.view(-1, s.num_kv_heads, s.head_dim)
-        o, lse = ext.flash_varlen_fwd(q, k, v, cu, longest, at.scale)
-        o2 = o.view(-1, s.q_size)
-        uo = o2 @ Ao.t()
-        y = _residual(x, o2, uo, at.o_proj.weight, Bo, at.o_proj.scale)
+        ext.rope_rows(q, k, pos, inv_freq)
+        pad_o = _padded([Ao.shape[0]])
+        ou, o, uo = _beside(x.new_empty(rows, s.q_size + pad_o), s.q_size)
+        lse = ext.flash_varlen_fwd(q, k, v, cu, longest, at.scale,
+                                   o.unflatten(1, (-1, s.head_dim)))[1]
+        _down(o, uo, [Ao], scales[3:])
+        Wo = at.o_proj.weight
+        # the residual joins the product's sum: one rounding for all of it
+        y = torch.addmm(x, ou, ext.adapted_weight([Wo], [Ao], [Bo], pad_o,
+                                                  False).t())
         head_norms = ((at.q_norm.weight, at.k_norm.weight) if s.qk_norm
                       else (None, None))
-        ctx.save_for_backward(x, h, A, u, Bq, Bk, Bv, Ao, Bo, q, k, v, o, lse,
-                              uo, pos, back_freq, cu, q0, k0, *head_norms,
-                              norm.weight, at.o_proj.weight,
-                              *(m.weight for m in mods))
+        ctx.save_for_backward(x, hu, ou, q, k, v, lse, pos, back_freq, cu, q0,
+                              k0, *head_norms, norm.weight, Ao, Bo, Wo,
+                              *As, *Bs, *Ws)
         ctx.spec, ctx.longest, ctx.scale = s, longest, at.scale
-        ctx.scales = [m.scale for m in (*mods, at.o_proj)]
+        ctx.scales = scales
         ctx.eps = (norm.eps, *((at.q_norm.eps, at.k_norm.eps) if s.qk_norm
                                else ()))
         return y
@@ -142,44 +190,45 @@ class _Attention(torch.autograd.Function):
     @staticmethod
     @once_differentiable
     def backward(ctx, g):
-        (x, h, A, u, Bq, Bk, Bv, Ao, Bo, q, k, v, o, lse, uo, pos, back_freq,
-         cu, q0, k0, q_norm, k_norm, norm, Wo, *Ws) = ctx.saved_tensors
+        (x, hu, ou, q, k, v, lse, pos, back_freq, cu, q0, k0, q_norm, k_norm,
+         norm, Ao, Bo, Wo, *rest) = ctx.saved_tensors
+        As, Bs, Ws = rest[:3], rest[3:6], rest[6:]
         ext, s = _ext(), ctx.spec
         *scales, scale_o = ctx.scales
         g = g.contiguous()
-        rows = g.shape[0]
-        o2 = o.view(rows, s.q_size)
+        rows, hidden = x.shape
+        _, h, u = _beside(hu, hidden)
+        _, o2, uo = _beside(ou, s.q_size)
+        o = o2.unflatten(1, (-1, s.head_dim))
 
         duo = _scaled_mm(g, Bo, scale_o)
-        dAo, dBo = duo.t() @ o2, _scaled_mm(g.t(), uo, scale_o)
-        do = _add(g @ Wo, duo, Ao)
-        dq, dk, dv = ext.flash_varlen_bwd(do.view_as(o), q, k, v, o, lse, cu,
-                                          ctx.longest, ctx.scale)
+        do = _add(g @ Wo, duo, Ao).view(rows, -1, s.head_dim)
+        sizes, ranks = [s.q_size, s.kv_size, s.kv_size], [a.shape[0] for a in As]
+        pad, width = _padded(ranks), sum(sizes)
+        dyu, dy, du = _beside(x.new_empty(rows, width + pad), width)
+        dys, dus = dy.split(sizes, 1), du[:, :sum(ranks)].split(ranks, 1)
+        dq, dk, dv = (t.unflatten(1, (-1, s.head_dim)) for t in dys)
+        ext.flash_varlen_bwd(do, q, k, v, o, lse, cu, ctx.longest, ctx.scale,
+                             dq, dk, dv)
         # a rotation's gradient is the rotation by the negative angle
-        ext.rope_inplace(dq, dk, pos, back_freq)
+        ext.rope_rows(dq, dk, pos, back_freq)
         if q0 is not None:
-            dq = ext.rmsnorm_bwd(dq, q0, q_norm, ctx.eps[1])
-            dk = ext.rmsnorm_bwd(dk, k0, k_norm, ctx.eps[2])
-        dq, dk, dv = (t.reshape(rows, -1) for t in (dq, dk, dv))
-
-        ranks = [Bq.shape[1], Bk.shape[1], Bv.shape[1]]
-        du = g.new_empty(rows, sum(ranks))
-        dBs = []
-        for d, scale, b, p, part in zip(
-                (dq, dk, dv), scales, (Bq, Bk, Bv), u.split(ranks, 1),
-                du.split(ranks, 1)):
-            _scaled_mm(d, b, scale, out=part)
-            dBs.append(_scaled_mm(d.t(), p, scale))
-        dAq, dAk, dAv = (du.t() @ h).split(ranks)
+            dq.copy_(ext.rmsnorm_bwd(dq.contiguous(), q0, q_norm, ctx.eps[1]))
+            dk.copy_(ext.rmsnorm_bwd(dk.contiguous(), k0, k_norm, ctx.eps[2]))
+        _up(dys, dus, Bs, scales)
+        if pad > sum(ranks):
+            du[:, sum(ranks):].zero_()
+        us = u[:, :sum(ranks)].split(ranks, 1)
+        dA, dAo, dBo, *dBs = _sums(
+            [(h, du, False), (o2, duo, False), (g, uo[:, :Ao.shape[0]], True),
+             *((y, p, True) for y, p in zip(dys, us))])
+        dAs = dA[:sum(ranks)].split(ranks)
         dx = None
         if ctx.needs_input_grad[0]:
-            dh = dq @ Ws[0]
-            dh.addmm_(dk, Ws[1])
-            dh.addmm_(dv, Ws[2])
-            _add(dh, du, A)
+            dh = dyu @ ext.adapted_weight(Ws, As, Bs, pad, True)
             dx = ext.rmsnorm_bwd_add(dh, x, norm, g, ctx.eps[0])
-        return (dx, None, None, None, dAq, dBs[0], dAk, dBs[1], dAv, dBs[2],
-                dAo, dBo)
+        return (dx, None, None, None, dAs[0], dBs[0], dAs[1], dBs[1], dAs[2],
+                dBs[2], dAo, dBo)
 
 
 class _FeedForward(torch.autograd.Function):
@@ -188,50 +237,65 @@ class _FeedForward(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, mlp, norm, Ag, Bg, Au, Bu, Ad, Bd):
         ext = _ext()
-        h = ext.rmsnorm_fwd(x, norm.weight, norm.eps)
-        A = torch.cat([Ag, Au])
-        u = h @ A.t()
-        ug, uu = u.split([Ag.shape[0], Au.shape[0]], 1)
-        gate = _project(h, ug, mlp.gate_proj.weight, mlp.gate_proj.bias, Bg,
-                        mlp.gate_proj.scale)
-        up = _project(h, uu, mlp.up_proj.weight, mlp.up_proj.bias, Bu,
-                      mlp.up_proj.scale)
-        act = ext.silu_mul_fwd(gate, up)
-        ud = act @ Ad.t()
-        y = _residual(x, act, ud, mlp.down_proj.weight, Bd,
-                      mlp.down_proj.scale)
-        mods = (mlp.gate_proj, mlp.up_proj, mlp.down_proj)
-        ctx.save_for_backward(x, h, A, u, Bg, Bu, Ad, Bd, gate, up, act, ud,
-                              norm.weight, *(m.weight for m in mods))
-        ctx.scales, ctx.eps = [m.scale for m in mods], norm.eps
+        rows, hidden = x.shape
+        mods = (mlp.gate_proj, mlp.up_proj)
+        scales = [m.scale for m in (*mods, mlp.down_proj)]
+        As, Bs, Ws = [Ag, Au], [Bg, Bu], [m.weight for m in mods]
+        pad = _padded([a.shape[0] for a in As])
+        hu, h, u = _beside(x.new_empty(rows, hidden + pad), hidden)
+        ext.rmsnorm_fwd_into(x, norm.weight, norm.eps, h)
+        _down(h, u, As, scales[:2])
+        W = ext.adapted_weight(Ws, As, Bs, pad, False)
+        gu = _product(hu, W, mods)
+        pad_d, inner = _padded([Ad.shape[0]]), gu.shape[1] // 2
+        au, act, ud = _beside(x.new_empty(rows, inner + pad_d), inner)
+        ext.silu_mul_packed_into(gu, act)
+        _down(act, ud, [Ad], scales[2:])
+        Wd = mlp.down_proj.weight
+        y = torch.addmm(x, au, ext.adapted_weight([Wd], [Ad], [Bd], pad_d,
+                                                  False).t())
+        ctx.save_for_backward(x, hu, gu, au, norm.weight, Ad, Bd, Wd, *As, *Bs,
+                              *Ws)
+        ctx.scales, ctx.eps = scales, norm.eps
         return y
 
     @staticmethod
     @once_differentiable
     def backward(ctx, g):
-        (x, h, A, u, Bg, Bu, Ad, Bd, gate, up, act, ud, norm, Wg, Wu,
-         Wd) = ctx.saved_tensors
-        ext, (scale_g, scale_u, scale_d) = _ext(), ctx.scales
-        g = g.contiguous()
-        dud = _scaled_mm(g, Bd, scale_d)
-        dAd, dBd = dud.t() @ act, _scaled_mm(g.t(), ud, scale_d)
-        dact = _add(g @ Wd, dud, Ad)
-        dgate, dup = ext.silu_mul_bwd(dact, gate, up)
-        ranks = [Bg.shape[1], Bu.shape[1]]
-        du = g.new_empty(g.shape[0], sum(ranks))
-        (ug, uu), (dug, duu) = u.split(ranks, 1), du.split(ranks, 1)
-        _scaled_mm(dgate, Bg, scale_g, out=dug)
-        _scaled_mm(dup, Bu, scale_u, out=duu)
-        dBg = _scaled_mm(dgate.t(), ug, scale_g)
-        dBu = _scaled_mm(dup.t(), uu, scale_u)
-        dAg, dAu = (du.t() @ h).split(ranks)
+        x, hu, gu, au, norm, Ad, Bd, Wd, *rest = ctx.saved_tensors
+        As, Bs, Ws = rest[:2], rest[2:4], rest[4:]
+        ext, (*scales, scale_d) = _ext(), ctx.scales
+        rows, hidden = x.shape
+        inner, ranks = gu.shape[1] // 2, [a.shape[0] for a in As]
+        _, h, u = _beside(hu, hidden)
+        _, act, ud = _beside(au, inner)
+
+        # [g | dud]: the adapter's share of dact joins the product
+        pad_d = _padded([Ad.shape[0]])
+        gd, g2, dud = _beside(x.new_empty(rows, hidden + pad_d), hidden)
+        g2.copy_(g)
+        _scaled_mm(g2, Bd, scale_d, out=dud[:, :Ad.shape[0]])
+        if pad_d > Ad.shape[0]:
+            dud[:, Ad.shape[0]:].zero_()
+        dact = gd @ ext.adapted_weight([Wd], [Ad], [Bd], pad_d, True)
+        pad = _padded(ranks)
+        dyu, dy, du = _beside(x.new_empty(rows, 2 * inner + pad), 2 * inner)
+        ext.silu_mul_bwd_packed(dact, gu, dy)
+        dys, dus = dy.chunk(2, 1), du[:, :sum(ranks)].split(ranks, 1)
+        _up(dys, dus, Bs, scales)
+        if pad > sum(ranks):
+            du[:, sum(ranks):].zero_()
+        us = u[:, :sum(ranks)].split(ranks, 1)
+        dA, dAd, dBd, *dBs = _sums(
+            [(h, du, False), (act, dud[:, :Ad.shape[0]], False),
+             (g2, ud[:, :Ad.shape[0]], True),
+             *((y, p, True) for y, p in zip(dys, us))])
+        dAs = dA[:sum(ranks)].split(ranks)
         dx = None
         if ctx.needs_input_grad[0]:
-            dh = dgate @ Wg
-            dh.addmm_(dup, Wu)
-            _add(dh, du, A)
-            dx = ext.rmsnorm_bwd_add(dh, x, norm, g, ctx.eps)
-        return dx, None, None, dAg, dBg, dAu, dBu, dAd, dBd
+            dh = dyu @ ext.adapted_weight(Ws, As, Bs, pad, True)
+            dx = ext.rmsnorm_bwd_add(dh, x, norm, g.contiguous(), ctx.eps)
+        return dx, None, None, dAs[0], dBs[0], dAs[1], dBs[1], dAd, dBd
 
 
 def rotary(head_dim: int, theta: float, positions, cu, longest: int):

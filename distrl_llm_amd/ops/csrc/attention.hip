@@ -719,7 +719,8 @@ void launch_fwd(const torch::Tensor& q, const torch::Tensor& k, const torch::Ten
 std::vector<torch::Tensor> launch_bwd(const torch::Tensor& dout, const torch::Tensor& q,
                                       const torch::Tensor& k, const torch::Tensor& v,
                                       const torch::Tensor& o, const torch::Tensor& lse,
-                                      const int* cu, int B, int T, double scale) {
+                                      const int* cu, int B, int T, double scale,
+                                      std::vector<torch::Tensor> grads = {}) {
   check_qkv(q, k, v);
   TORCH_CHECK(dout.scalar_type() == at::kBFloat16 && o.scalar_type() == at::kBFloat16 &&
               lse.scalar_type() == at::kFloat);
@@ -731,11 +732,12 @@ std::vector<torch::Tensor> launch_bwd(const torch::Tensor& dout, const torch::Te
   auto qc = rows16(q), kc = rows16(k), vc = rows16(v), oc = rows16(o), doc = rows16(dout);
   auto lsec = lse.contiguous();
   auto delta = torch::empty_like(lsec);
-  auto dq = like(qc), dk = like(kc), dv = like(vc);
+  if (grads.empty()) grads = {like(qc), like(kc), like(vc)};
+  auto &dq = grads[0], &dk = grads[1], &dv = grads[2];
   const int nw = waves_for((int64_t)B * Hq, T);
   const int rows = nw * WROWS, nq = (T + rows - 1) / rows;
   const int64_t blocks = (int64_t)B * Hq * nq, kv_blocks = (int64_t)B * Hkv * nq;
-  if (blocks == 0) return {dq, dk, dv};
+  if (blocks == 0) return grads;
   TORCH_CHECK(blocks < (1ll << 31), "flash attention: batch too large");
   const int group = Hq / Hkv;
   const int split = (int)std::min<int64_t>(group, (1024 + kv_blocks - 1) / kv_blocks);
@@ -767,13 +769,20 @@ std::vector<torch::Tensor> launch_bwd(const torch::Tensor& dout, const torch::Te
     }
   });
   HIP_CHECK_LAST();
-  return {dq, dk, dv};
+  return grads;
 }
 
 // A flat (tokens, H, D) batch as one (1, H, tokens, D) operand
 torch::Tensor flat4(const torch::Tensor& x) {
   TORCH_CHECK(x.dim() == 3);
   return x.transpose(0, 1).unsqueeze(0);
+}
+
+// an output that the kernels can write as it lies
+void check_out(const torch::Tensor& out, const torch::Tensor& like) {
+  TORCH_CHECK(out.is_cuda() && out.sizes() == like.sizes() && out.scalar_type() == at::kBFloat16);
+  const auto o4 = flat4(out);
+  TORCH_CHECK(rows16(o4).is_same(o4), "flash attention: output rows on 16 bytes");
 }
 
 void check_cu(const torch::Tensor& q, const torch::Tensor& cu, int64_t max_len) {
@@ -796,14 +805,17 @@ std::vector<torch::Tensor> flash_attn_fwd(torch::Tensor q, torch::Tensor k, torc
 
 // Causal attention inside each of the sequences cu[i] .. cu[i+1] of a flat
 // batch: q (tokens, Hq, D), k/v (tokens, Hkv, D), cu int32 (n+1,) rising from
-// 0 to tokens, max_len the longest of them. {output, log-sum-exp (Hq, tokens)}.
+// 0 to tokens, max_len the longest of them. {output, log-sum-exp (Hq, tokens)};
+// into: where the output goes, rows of a wider matrix.
 std::vector<torch::Tensor> flash_varlen_fwd(torch::Tensor q, torch::Tensor k, torch::Tensor v,
-                                            torch::Tensor cu, int64_t max_len, double scale) {
+                                            torch::Tensor cu, int64_t max_len, double scale,
+                                            c10::optional<torch::Tensor> into) {
   auto q4 = flat4(q), k4 = flat4(k), v4 = flat4(v);
   check_cu(q, cu, max_len);
   check_qkv(q4, k4, v4);
   auto qc = rows16(positive_scale(q4, scale)), kc = rows16(k4), vc = rows16(v4);
-  auto out = torch::empty(q.sizes(), q.options());
+  auto out = into ? *into : torch::empty(q.sizes(), q.options());
+  check_out(out, q);
   auto lse = torch::empty({q.size(1), q.size(0)}, q.options().dtype(at::kFloat));
   auto o4 = flat4(out);
   launch_fwd(qc, kc, vc, o4, lse.data_ptr<float>(), cu.data_ptr<int>(), cu.numel() - 1, max_len,
@@ -813,7 +825,7 @@ std::vector<torch::Tensor> flash_varlen_fwd(torch::Tensor q, torch::Tensor k, to
 
 torch::Tensor flash_attn_varlen(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                                 torch::Tensor cu, int64_t max_len, double scale) {
-  return flash_varlen_fwd(q, k, v, cu, max_len, scale)[0];
+  return flash_varlen_fwd(q, k, v, cu, max_len, scale, c10::nullopt)[0];
 }
 
 std::vector<torch::Tensor> flash_attn_bwd(torch::Tensor dout, torch::Tensor q, torch::Tensor k,
@@ -822,15 +834,16 @@ std::vector<torch::Tensor> flash_attn_bwd(torch::Tensor dout, torch::Tensor q, t
   return launch_bwd(dout, q, k, v, o, lse, nullptr, q.size(0), q.size(2), scale);
 }
 
-// {dq, dk, dv} of flash_varlen_fwd, (tokens, H, D)
-std::vector<torch::Tensor> flash_varlen_bwd(torch::Tensor dout, torch::Tensor q, torch::Tensor k,
-                                            torch::Tensor v, torch::Tensor o, torch::Tensor lse,
-                                            torch::Tensor cu, int64_t max_len, double scale) {
+// dq, dk, dv of flash_varlen_fwd into (tokens, H, D) tensors, rows of wider ones
+void flash_varlen_bwd(torch::Tensor dout, torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                      torch::Tensor o, torch::Tensor lse, torch::Tensor cu, int64_t max_len,
+                      double scale, torch::Tensor dq, torch::Tensor dk, torch::Tensor dv) {
   check_cu(q, cu, max_len);
-  auto r = launch_bwd(flat4(dout), flat4(q), flat4(k), flat4(v), flat4(o), lse, cu.data_ptr<int>(),
-                      cu.numel() - 1, max_len, scale);
-  for (auto& t : r) t = t.squeeze(0).transpose(0, 1);
-  return r;
+  check_out(dq, q);
+  check_out(dk, k);
+  check_out(dv, v);
+  launch_bwd(flat4(dout), flat4(q), flat4(k), flat4(v), flat4(o), lse, cu.data_ptr<int>(),
+             cu.numel() - 1, max_len, scale, {flat4(dq), flat4(dk), flat4(dv)});
 }
 
 // The differentiable call: a node of the C++ engine (from Python, node and

@@ -14,6 +14,8 @@ std::vector<torch::Tensor> silu_mul_bwd(torch::Tensor dy, torch::Tensor gate,
                                         torch::Tensor up);
 void rope_inplace(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
                   torch::Tensor inv_freq);
+void rope_rows(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
+               torch::Tensor inv_freq);
 void rope_scatter_qkv(torch::Tensor qkv, torch::Tensor positions,
                       torch::Tensor slots, torch::Tensor inv_freq,
                       torch::Tensor key_cache, torch::Tensor value_cache,
@@ -97,12 +99,23 @@ torch::Tensor flash_attn_varlen(torch::Tensor q, torch::Tensor k,
                                 int64_t max_len, double scale);
 std::vector<torch::Tensor> flash_varlen_fwd(torch::Tensor q, torch::Tensor k,
                                             torch::Tensor v, torch::Tensor cu,
-                                            int64_t max_len, double scale);
-std::vector<torch::Tensor> flash_varlen_bwd(torch::Tensor dout, torch::Tensor q,
-                                            torch::Tensor k, torch::Tensor v,
-                                            torch::Tensor o, torch::Tensor lse,
-                                            torch::Tensor cu, int64_t max_len,
-                                            double scale);
+                                            int64_t max_len, double scale,
+                                            c10::optional<torch::Tensor> into);
+void flash_varlen_bwd(torch::Tensor dout, torch::Tensor q, torch::Tensor k,
+                      torch::Tensor v, torch::Tensor o, torch::Tensor lse,
+                      torch::Tensor cu, int64_t max_len, double scale,
+                      torch::Tensor dq, torch::Tensor dk, torch::Tensor dv);
+std::vector<torch::Tensor> adapter_grads(std::vector<torch::Tensor> y,
+                                         std::vector<torch::Tensor> p,
+                                         std::vector<int64_t> by_col);
+torch::Tensor adapted_weight(std::vector<torch::Tensor> w,
+                             std::vector<torch::Tensor> a,
+                             std::vector<torch::Tensor> b, int64_t pad,
+                             bool back);
+void rmsnorm_fwd_into(torch::Tensor x, torch::Tensor w, double eps,
+                      torch::Tensor out);
+void silu_mul_packed_into(torch::Tensor gu, torch::Tensor out);
+void silu_mul_bwd_packed(torch::Tensor dy, torch::Tensor gu, torch::Tensor out);
 std::vector<torch::Tensor> flash_attn_bwd(torch::Tensor dout, torch::Tensor q,
                                           torch::Tensor k, torch::Tensor v,
                                           torch::Tensor o, torch::Tensor lse,
@@ -122,6 +135,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_mul_fwd", &silu_mul_fwd, "fused SiLU*mul forward");
   m.def("silu_mul_bwd", &silu_mul_bwd, "fused SiLU*mul backward");
   m.def("rope_inplace", &rope_inplace, "fused in-place RoPE (q,k)");
+  m.def("rope_rows", &rope_rows, "the same on rows of wider matrices");
   m.def("rope_scatter_qkv", &rope_scatter_qkv,
         "packed-qkv per-head norms (optional) + RoPE + paged KV scatter",
         py::arg("qkv"), py::arg("positions"), py::arg("slots"),
@@ -196,8 +210,21 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("flash_attn_varlen", &flash_attn_varlen,
         "causal GQA flash attention over a flat batch of sequences");
   m.def("flash_varlen_fwd", &flash_varlen_fwd,
-        "the same with its log-sum-exp");
-  m.def("flash_varlen_bwd", &flash_varlen_bwd, "its backward (dq, dk, dv)");
+        "the same with its log-sum-exp", py::arg("q"), py::arg("k"),
+        py::arg("v"), py::arg("cu"), py::arg("max_len"), py::arg("scale"),
+        py::arg("into") = py::none());
+  m.def("flash_varlen_bwd", &flash_varlen_bwd,
+        "its backward, into dq, dk and dv");
+  m.def("adapter_grads", &adapter_grads,
+        "p^T y of several operands, summed over the rows");
+  m.def("adapted_weight", &adapted_weight,
+        "[W | B] or [W; A] of projections of one input");
+  m.def("rmsnorm_fwd_into", &rmsnorm_fwd_into,
+        "RMSNorm forward into rows of a wider matrix");
+  m.def("silu_mul_packed_into", &silu_mul_packed_into,
+        "SiLU*mul of [gate | up] into rows of a wider matrix");
+  m.def("silu_mul_bwd_packed", &silu_mul_bwd_packed,
+        "its backward into [dgate | dup]");
   m.def("flash_attn_bwd", &flash_attn_bwd,
         "causal GQA flash attention backward (returns dq, dk, dv)");
 }

@@ -222,3 +222,92 @@ bool lora_add(torch::Tensor y, torch::Tensor u, torch::Tensor m, double scale,
   const bool ta = m.stride(1) != 1;
   return launch_merge(y, ta ? m.t() : m, u, y, ta, scale, res);
 }
+
+// ---- base and adapter weights as one matrix, so that one product does both:
+// [x | u] [W | B]^T and [dY | du] [W; A], the adapter's sum in the product's fp32.
+namespace {
+
+struct Parts {
+  const __hip_bfloat16 *w[3], *a[3], *b[3];
+  int row[4], col[4];                   // first row and adapter column of each, and the ends
+  int n;
+};
+
+// 16 B a thread. BACK: (rows + pad, K), A below W; else (rows, K + pad), B beside
+// W, zeros where a row has another projection's columns.
+template <bool BACK>
+__global__ __launch_bounds__(256)
+void adapted_weight_kernel(Parts q, __hip_bfloat16* __restrict__ out, int K, int pad) {
+  const int cpr = (BACK ? K : K + pad) / 8, rows = q.row[q.n];
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = id / cpr;
+  const int c = (int)(id % cpr) * 8;
+  if (row >= (BACK ? rows + pad : rows)) return;
+  bf16x8 v;
+  if (row < rows && c < K) {
+    int i = 0;
+    while (i + 1 < q.n && row >= q.row[i + 1]) ++i;
+    v = *reinterpret_cast<const bf16x8*>(q.w[i] + (row - q.row[i]) * K + c);
+  } else {
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) v.v[j] = f2bf(0.f);
+    if (BACK) {
+      const int r = (int)row - rows;
+      for (int i = 0; i < q.n; ++i)
+        if (r >= q.col[i] && r < q.col[i + 1])
+          v = *reinterpret_cast<const bf16x8*>(q.a[i] + (int64_t)(r - q.col[i]) * K + c);
+    } else {
+      int i = 0;
+      while (i + 1 < q.n && row >= q.row[i + 1]) ++i;
+      const int r = q.col[i + 1] - q.col[i];
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int k = c - K + j - q.col[i];
+        if (k >= 0 && k < r) v.v[j] = q.b[i][(row - q.row[i]) * r + k];
+      }
+    }
+  }
+  *reinterpret_cast<bf16x8*>(out + id * 8) = v;
+}
+
+torch::Tensor dense16(const torch::Tensor& t) {
+  TORCH_CHECK(t.is_cuda() && t.dim() == 2 && t.scalar_type() == at::kBFloat16);
+  auto c = t.contiguous();
+  return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 ? c : c.clone();
+}
+
+}  // namespace
+
+// Up to three projections of one input, one below the other: w[i] (N_i, K), a[i]
+// (r_i, K), b[i] (N_i, r_i); pad >= the ranks' sum, both multiples of 8 as K is.
+torch::Tensor adapted_weight(std::vector<torch::Tensor> w, std::vector<torch::Tensor> a,
+                             std::vector<torch::Tensor> b, int64_t pad, bool back) {
+  const int n = (int)w.size(), K = (int)w.at(0).size(1);
+  TORCH_CHECK(n <= 3 && a.size() == w.size() && b.size() == w.size() && K % 8 == 0 && pad % 8 == 0);
+  Parts q{};
+  q.n = n;
+  for (int i = 0; i < n; ++i) {
+    w[i] = dense16(w[i]);
+    a[i] = dense16(a[i]);
+    b[i] = dense16(b[i]);
+    const int N = w[i].size(0), r = a[i].size(0);
+    TORCH_CHECK(w[i].size(1) == K && a[i].size(1) == K && b[i].size(0) == N && b[i].size(1) == r,
+                "adapted_weight: shape mismatch");
+    q.w[i] = lptr(w[i]);
+    q.a[i] = lptr(a[i]);
+    q.b[i] = lptr(b[i]);
+    q.row[i + 1] = q.row[i] + N;
+    q.col[i + 1] = q.col[i] + r;
+  }
+  TORCH_CHECK(q.col[n] <= pad);
+  const int64_t rows = q.row[n];
+  auto out = back ? torch::empty({rows + pad, K}, w[0].options())
+                  : torch::empty({rows, K + pad}, w[0].options());
+  if (out.numel() == 0) return out;
+  hipLaunchKernelGGL(back ? adapted_weight_kernel<true> : adapted_weight_kernel<false>,
+                     dim3(CDIV(out.numel() / 8, 256)), dim3(256), 0,
+                     at::cuda::getCurrentCUDAStream(), q,
+                     reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), K, (int)pad);
+  HIP_CHECK_LAST();
+  return out;
+}

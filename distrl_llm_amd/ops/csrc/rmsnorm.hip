@@ -14,12 +14,12 @@ namespace {
 __global__ void rmsnorm_fwd_bf16(const __hip_bfloat16* __restrict__ x,
                                  const __hip_bfloat16* __restrict__ w,
                                  __hip_bfloat16* __restrict__ y,
-                                 int hidden, float eps) {
+                                 int hidden, int64_t ldy, float eps) {
   __shared__ float red[16];
   const int64_t row = blockIdx.x;
   const bf16x8* xr = reinterpret_cast<const bf16x8*>(x + row * hidden);
   const bf16x8* wr = reinterpret_cast<const bf16x8*>(w);
-  bf16x8* yr = reinterpret_cast<bf16x8*>(y + row * hidden);
+  bf16x8* yr = reinterpret_cast<bf16x8*>(y + row * ldy);
   const int nvec = hidden / 8;
 
   float ss = 0.f;
@@ -136,7 +136,7 @@ torch::Tensor rmsnorm_fwd(torch::Tensor x, torch::Tensor w, double eps) {
                        reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()),
                        reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()),
                        reinterpret_cast<__hip_bfloat16*>(y.data_ptr()),
-                       hidden, (float)eps);
+                       hidden, (int64_t)hidden, (float)eps);
   } else {
     TORCH_CHECK(x.scalar_type() == at::kFloat, "rmsnorm: bf16 or fp32 only");
     hipLaunchKernelGGL(rmsnorm_fwd_f32, grid, block, 0, stream,
@@ -145,6 +145,24 @@ torch::Tensor rmsnorm_fwd(torch::Tensor x, torch::Tensor w, double eps) {
   }
   HIP_CHECK_LAST();
   return y;
+}
+
+// The same into rows of a wider matrix: out (rows, hidden), bf16
+void rmsnorm_fwd_into(torch::Tensor x, torch::Tensor w, double eps, torch::Tensor out) {
+  const int hidden = x.size(-1);
+  TORCH_CHECK(x.is_cuda() && x.is_contiguous() && x.dim() == 2 && x.scalar_type() == at::kBFloat16);
+  TORCH_CHECK(w.scalar_type() == at::kBFloat16 && w.numel() == hidden && w.is_contiguous());
+  TORCH_CHECK(out.sizes() == x.sizes() && out.scalar_type() == at::kBFloat16 && out.is_cuda() &&
+              out.stride(1) == 1 && out.stride(0) % 8 == 0 && hidden % 8 == 0 &&
+              reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0, "rmsnorm_fwd_into: output");
+  if (x.size(0) == 0) return;
+  hipLaunchKernelGGL(rmsnorm_fwd_bf16, dim3(x.size(0)), dim3(256), 0,
+                     at::cuda::getCurrentCUDAStream(),
+                     reinterpret_cast<const __hip_bfloat16*>(x.data_ptr()),
+                     reinterpret_cast<const __hip_bfloat16*>(w.data_ptr()),
+                     reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), hidden, out.stride(0),
+                     (float)eps);
+  HIP_CHECK_LAST();
 }
 
 torch::Tensor rmsnorm_bwd(torch::Tensor dy, torch::Tensor x, torch::Tensor w,

@@ -47,7 +47,8 @@ __global__ void rope_inplace_kernel(__hip_bfloat16* __restrict__ q,
 __global__ __launch_bounds__(256)
 void rope_inplace_vec_kernel(__hip_bfloat16* __restrict__ q, __hip_bfloat16* __restrict__ k,
                              const int* __restrict__ positions,
-                             const float* __restrict__ inv_freq, int T, int H, int KV, int D) {
+                             const float* __restrict__ inv_freq, int T, int H, int KV, int D,
+                             int64_t ldq, int64_t ldk) {
   const int t = blockIdx.x * 4 + threadIdx.x / WAVE, lane = threadIdx.x & (WAVE - 1);
   if (t >= T) return;
   const int half = D / 2, per = half / 8;        // units of a head
@@ -65,8 +66,7 @@ void rope_inplace_vec_kernel(__hip_bfloat16* __restrict__ q, __hip_bfloat16* __r
         cs[j] = __cosf(a);
       }
     }
-    __hip_bfloat16* p = (head < H ? q + ((int64_t)t * H + head) * D
-                                  : k + ((int64_t)t * KV + head - H) * D) + c;
+    __hip_bfloat16* p = (head < H ? q + t * ldq + head * D : k + t * ldk + (head - H) * D) + c;
     const bf16x8 a = *reinterpret_cast<const bf16x8*>(p);
     const bf16x8 b = *reinterpret_cast<const bf16x8*>(p + half);
     bf16x8 x, y;
@@ -367,27 +367,35 @@ torch::Tensor rope_scatter_join(torch::Tensor parts, c10::optional<torch::Tensor
   return q;
 }
 
-void rope_inplace(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
-                  torch::Tensor inv_freq) {
-  TORCH_CHECK(q.is_cuda() && q.is_contiguous() && k.is_contiguous());
-  TORCH_CHECK(q.scalar_type() == at::kBFloat16);
+// q (T, H, D), k (T, KV, D), whose rows may lie apart
+void rope_rows(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
+               torch::Tensor inv_freq) {
+  // heads of a row follow one another
+  auto rows = [](const torch::Tensor& x) {
+    return x.dim() == 3 && (x.size(2) <= 1 || x.stride(2) == 1) &&
+           (x.size(1) <= 1 || x.stride(1) == x.size(2));
+  };
+  TORCH_CHECK(q.is_cuda() && rows(q) && rows(k));
+  TORCH_CHECK(q.scalar_type() == at::kBFloat16 && k.scalar_type() == at::kBFloat16);
   TORCH_CHECK(positions.scalar_type() == at::kInt);
   const int T = q.size(0), H = q.size(1), D = q.size(2);
   const int KV = k.size(1);
   TORCH_CHECK(k.size(0) == T && k.size(2) == D);
   if (T == 0) return;
   auto aligned = [](const torch::Tensor& x) {
-    return reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+    return reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && x.stride(0) % 8 == 0;
   };
   if (D % 16 == 0 && aligned(q) && aligned(k)) {
     hipLaunchKernelGGL(rope_inplace_vec_kernel, dim3((T + 3) / 4), dim3(256), 0,
                        at::cuda::getCurrentCUDAStream(),
                        reinterpret_cast<__hip_bfloat16*>(q.data_ptr()),
                        reinterpret_cast<__hip_bfloat16*>(k.data_ptr()),
-                       positions.data_ptr<int>(), inv_freq.data_ptr<float>(), T, H, KV, D);
+                       positions.data_ptr<int>(), inv_freq.data_ptr<float>(), T, H, KV, D,
+                       q.stride(0), k.stride(0));
     HIP_CHECK_LAST();
     return;
   }
+  TORCH_CHECK(q.is_contiguous() && k.is_contiguous());
   const int smem = D * sizeof(float);
   hipLaunchKernelGGL(rope_inplace_kernel, dim3(T), dim3(256), smem,
                      at::cuda::getCurrentCUDAStream(),
@@ -396,4 +404,10 @@ void rope_inplace(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
                      positions.data_ptr<int>(), inv_freq.data_ptr<float>(),
                      H, KV, D);
   HIP_CHECK_LAST();
+}
+
+void rope_inplace(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
+                  torch::Tensor inv_freq) {
+  TORCH_CHECK(q.is_contiguous() && k.is_contiguous());
+  rope_rows(q, k, positions, inv_freq);
 }

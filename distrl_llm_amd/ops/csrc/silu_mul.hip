@@ -119,11 +119,11 @@ std::vector<torch::Tensor> silu_mul_bwd(torch::Tensor dy, torch::Tensor gate,
 namespace {
 __global__ void silu_mul_packed_bf16(const __hip_bfloat16* __restrict__ gu,
                                      __hip_bfloat16* __restrict__ out,
-                                     int fvec /* F/8 */) {
+                                     int fvec /* F/8 */, int64_t ldo) {
   const int64_t row = blockIdx.x;
   const bf16x8* g8 = reinterpret_cast<const bf16x8*>(gu + row * 2 * fvec * 8);
   const bf16x8* u8 = g8 + fvec;
-  bf16x8* o8 = reinterpret_cast<bf16x8*>(out + row * fvec * 8);
+  bf16x8* o8 = reinterpret_cast<bf16x8*>(out + row * ldo);
   for (int i = threadIdx.x; i < fvec; i += blockDim.x) {
     bf16x8 g = g8[i], u = u8[i], o;
     #pragma unroll
@@ -136,19 +136,71 @@ __global__ void silu_mul_packed_bf16(const __hip_bfloat16* __restrict__ gu,
 }
 }  // namespace
 
-torch::Tensor silu_mul_packed(torch::Tensor gu) {
+// out (rows, F), rows any multiple of 16 bytes apart
+void silu_mul_packed_into(torch::Tensor gu, torch::Tensor out) {
   TORCH_CHECK(gu.is_cuda() && gu.is_contiguous() && gu.dim() == 2);
-  TORCH_CHECK(gu.scalar_type() == at::kBFloat16);
-  const int64_t N = gu.size(0);
-  const int64_t F = gu.size(1) / 2;
-  TORCH_CHECK(F % 8 == 0);
-  auto out = torch::empty({N, F}, gu.options());
-  if (N == 0) return out;
+  TORCH_CHECK(gu.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16);
+  const int64_t N = gu.size(0), F = gu.size(1) / 2;
+  TORCH_CHECK(F % 8 == 0 && out.is_cuda() && out.dim() == 2 && out.size(0) == N &&
+              out.size(1) == F && out.stride(1) == 1 && out.stride(0) % 8 == 0 &&
+              reinterpret_cast<uintptr_t>(out.data_ptr()) % 16 == 0, "silu_mul_packed: output");
+  if (N == 0) return;
   hipLaunchKernelGGL(silu_mul_packed_bf16, dim3(N), dim3(256), 0,
                      at::cuda::getCurrentCUDAStream(),
                      reinterpret_cast<const __hip_bfloat16*>(gu.data_ptr()),
                      reinterpret_cast<__hip_bfloat16*>(out.data_ptr()),
-                     (int)(F / 8));
+                     (int)(F / 8), out.stride(0));
   HIP_CHECK_LAST();
+}
+
+torch::Tensor silu_mul_packed(torch::Tensor gu) {
+  TORCH_CHECK(gu.dim() == 2);
+  auto out = torch::empty({gu.size(0), gu.size(1) / 2}, gu.options());
+  silu_mul_packed_into(gu, out);
   return out;
+}
+
+// ---- its backward: dy (N, F), gu (N, 2F) -> out (N, 2F) = [dgate | dup]
+namespace {
+__global__ __launch_bounds__(256)
+void silu_mul_bwd_packed_kernel(const __hip_bfloat16* __restrict__ dy,
+                                const __hip_bfloat16* __restrict__ gu,
+                                __hip_bfloat16* __restrict__ out, int fvec, int64_t ldo) {
+  const int64_t row = blockIdx.x;
+  const bf16x8* d8 = reinterpret_cast<const bf16x8*>(dy) + row * fvec;
+  const bf16x8* g8 = reinterpret_cast<const bf16x8*>(gu) + row * 2 * fvec;
+  bf16x8* o8 = reinterpret_cast<bf16x8*>(out + row * ldo);
+  for (int i = threadIdx.x; i < fvec; i += 256) {
+    const bf16x8 d = d8[i], g = g8[i], u = g8[fvec + i];
+    bf16x8 og, ou;
+    #pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float gf = bf2f(g.v[j]), df = bf2f(d.v[j]);
+      const float sig = 1.f / (1.f + __expf(-gf));
+      og.v[j] = f2bf(df * bf2f(u.v[j]) * sig * (1.f + gf * (1.f - sig)));
+      ou.v[j] = f2bf(df * gf * sig);
+    }
+    o8[i] = og;
+    o8[fvec + i] = ou;
+  }
+}
+}  // namespace
+
+void silu_mul_bwd_packed(torch::Tensor dy, torch::Tensor gu, torch::Tensor out) {
+  TORCH_CHECK(dy.is_cuda() && dy.is_contiguous() && dy.dim() == 2 &&
+              dy.scalar_type() == at::kBFloat16);
+  const int64_t N = dy.size(0), F = dy.size(1);
+  TORCH_CHECK(gu.is_cuda() && gu.is_contiguous() && gu.scalar_type() == at::kBFloat16 &&
+              gu.dim() == 2 && gu.size(0) == N && gu.size(1) == 2 * F && F % 8 == 0);
+  TORCH_CHECK(out.is_cuda() && out.scalar_type() == at::kBFloat16 && out.sizes() == gu.sizes() &&
+              out.stride(1) == 1 && out.stride(0) % 8 == 0);
+  for (const auto* t : {&dy, &gu, &out})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "silu_mul_bwd: alignment");
+  if (N == 0) return;
+  hipLaunchKernelGGL(silu_mul_bwd_packed_kernel, dim3(N), dim3(256), 0,
+                     at::cuda::getCurrentCUDAStream(),
+                     reinterpret_cast<const __hip_bfloat16*>(dy.data_ptr()),
+                     reinterpret_cast<const __hip_bfloat16*>(gu.data_ptr()),
+                     reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), (int)(F / 8), out.stride(0));
+  HIP_CHECK_LAST();
 }

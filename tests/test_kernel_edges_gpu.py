@@ -783,8 +783,19 @@ def test_flash_varlen_backward(ext, lens, H, KV, D, packed):
     dout = _rand((T, H, D), 2, 0.1)
     cu = torch.tensor([0, *lens]).cumsum(0).to("cuda", torch.int32)
     o, lse = ext.flash_varlen_fwd(q, k, v, cu, max(lens), D ** -0.5)
-    got = (o, *ext.flash_varlen_bwd(dout, q, k, v, o, lse, cu, max(lens), D ** -0.5))
-    start = 0
+    wide = torch.full((T, (H + 2 * KV) * D + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+    grads = [t.unflatten(1, (-1, D)) for t in wide[:, :-8].split([H * D, KV * D, KV * D], 1)]
+    if not packed:
+        grads = [torch.empty_like(t) for t in (q, k, v)]
+    else:       # the output into a wider matrix too
+        room = torch.empty((T, H * D + 8), dtype=torch.bfloat16, device="cuda")
+        ext.flash_varlen_fwd(q, k, v, cu, max(lens), D ** -0.5,
+                             room[:, :H * D].unflatten(1, (H, D)))
+        assert torch.equal(room[:, :H * D], o.flatten(1))
+        o = room[:, :H * D].unflatten(1, (H, D))
+    ext.flash_varlen_bwd(dout, q, k, v, o, lse, cu, max(lens), D ** -0.5, *grads)
+    assert (wide[:, -8:] == 7).all()
+    got, start = (o, *grads), 0
     for n in lens:
         part = [t[start:start + n].transpose(0, 1).unsqueeze(0) for t in (q, k, v, dout)]
         for x, y in zip(got, _flash_reference(*part, D ** -0.5)):
@@ -792,6 +803,70 @@ def test_flash_varlen_backward(ext, lens, H, KV, D, packed):
             off = (x[start:start + n].transpose(0, 1).double() - y[0].double()).norm()
             assert off < FLASH_REL * y.double().norm() + 2.0 ** -18 * dout.double().norm()
         start += n
+
+
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 700, 5000])
+@pytest.mark.parametrize("shapes", [[(8, 8)], [(128, 32), (136, 40), (1000, 64), (256, 96), (64, 128),
+                                               (1536, 32)]])
+def test_adapter_grads(ext, rows, shapes):
+    """Ends of the row steps, column blocks and rank tiles, several operands at
+    once, in place and cut out of wider rows; both layouts of the output. Bound:
+    fp32 sums, one rounding."""
+    ys, ps = [], []
+    for i, (N, r) in enumerate(shapes):
+        ys.append(_rand((rows, N + 8), 2 * i)[:, 8:] if i % 2 else _rand((rows, N), 2 * i))
+        ps.append(_rand((rows, r + 3), 2 * i + 1)[:, 3:] if i % 3 == 2 else
+                  _rand((rows, r), 2 * i + 1))
+    for flip in (0, 1):
+        by_col = [(i + flip) % 2 for i in range(len(shapes))]
+        for y, p, c, got in zip(ys, ps, by_col, ext.adapter_grads(ys, ps, by_col)):
+            ref = p.double().t() @ y.double()
+            assert _rel(got, ref.t() if c else ref) < 2.0 ** -8
+    assert all((t == 0).all() for t in ext.adapter_grads([ys[0][:0]], [ps[0][:0]], [0]))
+
+
+@pytest.mark.parametrize("N,K,ranks,pad", [((16, 8, 24), 64, (8, 8, 8), 24), ((40, 24), 136, (5, 12), 24),
+                                           ((64,), 8, (32,), 32)])
+def test_adapted_weight(ext, N, K, ranks, pad):
+    ws, As, Bs = ([_rand(s, i) for i, s in enumerate(shapes)] for shapes in (
+        [(n, K) for n in N], [(r, K) for r in ranks], list(zip(N, ranks))))
+    odd = ws[0].new_empty(ws[0].numel() + 1)[1:].view(ws[0].shape).copy_(ws[0])
+    z = torch.zeros(pad - sum(ranks), K, device="cuda", dtype=torch.bfloat16)
+    beside = torch.block_diag(*Bs, z[:0, :0].new_zeros(0, pad - sum(ranks)))
+    for w0 in (ws[0], odd):
+        w = [w0, *ws[1:]]
+        assert torch.equal(ext.adapted_weight(w, As, Bs, pad, False),
+                           torch.cat([torch.cat(ws), beside], 1))
+        assert torch.equal(ext.adapted_weight(w, As, Bs, pad, True), torch.cat([*ws, *As, z]))
+
+
+@pytest.mark.parametrize("rows,F", [(1, 8), (5, 2056), (33, 4864)])
+def test_activation_and_norm_into_wider_rows(ext, rows, F):
+    """The same numbers as into matrices of their own, nothing beside them."""
+    gu, dy, w = _rand((rows, 2 * F), 1), _rand((rows, F), 2), _rand((F,), 3)
+    gate, up = (t.contiguous() for t in gu.chunk(2, 1))
+    act, back = (torch.full((rows, n + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+                 for n in (F, 2 * F))
+    ext.silu_mul_packed_into(gu, act[:, :F])
+    ext.silu_mul_bwd_packed(dy, gu, back[:, :-8])
+    assert torch.equal(act[:, :F], ext.silu_mul_fwd(gate, up))
+    assert torch.equal(back[:, :-8], torch.cat(ext.silu_mul_bwd(dy, gate, up), 1))
+    ext.rmsnorm_fwd_into(dy, w, 1e-6, act[:, :F])
+    assert torch.equal(act[:, :F], ext.rmsnorm_fwd(dy, w, 1e-6))
+    assert (act[:, F:] == 7).all() and (back[:, -8:] == 7).all()
+
+
+@pytest.mark.parametrize("T,H,KV,D", [(1, 1, 1, 64), (9, 14, 2, 64), (5, 12, 2, 128)])
+def test_rope_rows(ext, T, H, KV, D):
+    wide = _rand((T, (H + 2 * KV) * D + 8), 1)
+    q, k = (t.unflatten(1, (-1, D)) for t in wide[:, :(H + KV) * D].split([H * D, KV * D], 1))
+    pos = torch.arange(T, dtype=torch.int32, device="cuda") * 37
+    inv = 1.0 / 1e4 ** (torch.arange(0, D, 2, device="cuda").float() / D)
+    ref, rest = [q.contiguous(), k.contiguous()], wide[:, (H + KV) * D:].clone()
+    ext.rope_inplace(*ref, pos, inv)
+    ext.rope_rows(q, k, pos, inv)
+    assert torch.equal(q, ref[0]) and torch.equal(k, ref[1])
+    assert torch.equal(wide[:, (H + KV) * D:], rest)
 
 
 @pytest.mark.parametrize("rows,V", [(1, 7), (3, 4103), (1500, 4096)])
