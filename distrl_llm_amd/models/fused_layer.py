@@ -9,7 +9,7 @@ head transposes), and short micro-batches are bound by launching them. Here
 an adapter is more of its projection: u = scale * x A^T lies beside x in one
 matrix, [x | u], and one product with [W | B] gives every projection of that
 input, adapters and (beta = 1) the residual in its fp32 sums; backward is
-[dY | dU] [W; A]. Laying W out beside its adapter costs a copy of the weights,
+[dY | du] [W; A]. Laying W out beside its adapter costs a copy of the weights,
 37 us a layer of the 1.5B model forward and as long backward, where adding the
 adapters' outputs to 18800 rows in passes of their own took 750. Adapter
 gradients are one launch and its sum (ops/csrc/adapter_grads.hip). Rotary, norm
@@ -75,11 +75,6 @@ def _ext():
     return _require_ext("fused decoder layer")
 
 
-def _add(y, u, m, scale=1.0):
-    """y += scale * u m, in place; m as it lies or a transposed view."""
-    return y if _ext().lora_add(y, u, m, scale) else y.addmm_(u, m, alpha=scale)
-
-
 def _scaled_mm(a, b, scale, out=None):
     """scale * a @ b, the scale in the product's epilogue."""
     if out is None:
@@ -125,6 +120,20 @@ def _up(dys, us, Bs, scales) -> None:
         _scaled_mm(dy, b, scale, out=u)
 
 
+def _through(g, W, A, B, scale):
+    """g W + du A with du = scale * g B, from one product of [g | du]; g and du
+    as parts of that matrix."""
+    (rows, N), r = g.shape, A.shape[0]
+    pad = _padded([r])
+    gd, g2, du = _beside(g.new_empty(rows, N + pad), N)
+    g2.copy_(g)
+    _scaled_mm(g, B, scale, out=du[:, :r])
+    if pad > r:
+        du[:, r:].zero_()
+    return (gd @ _ext().stack_transposed([W, A], [0, N], N + pad).t(), g2,
+            du[:, :r])
+
+
 def _sums(jobs):
     """p^T y of every (y, p, transposed) over the rows: gradients of A, or of B
     (transposed). Ranks that the kernel does not take go through the library."""
@@ -157,7 +166,7 @@ class _Attention(torch.autograd.Function):
         hu, h, u = _beside(x.new_empty(rows, hidden + pad), hidden)
         ext.rmsnorm_fwd_into(x, norm.weight, norm.eps, h)
         _down(h, u, As, scales[:3])
-        W = ext.adapted_weight(Ws, As, Bs, pad, False)
+        W = ext.adapted_weight(Ws, Bs, pad)
         qkv = _product(hu, W, mods)
         q, k, v = (t.unflatten(1, (-1, s.head_dim))
                    for t in qkv.split([s.q_size, s.kv_size, s.kv_size], 1))
@@ -174,8 +183,7 @@ class _Attention(torch.autograd.Function):
         _down(o, uo, [Ao], scales[3:])
         Wo = at.o_proj.weight
         # the residual joins the product's sum: one rounding for all of it
-        y = torch.addmm(x, ou, ext.adapted_weight([Wo], [Ao], [Bo], pad_o,
-                                                  False).t())
+        y = torch.addmm(x, ou, ext.adapted_weight([Wo], [Bo], pad_o).t())
         head_norms = ((at.q_norm.weight, at.k_norm.weight) if s.qk_norm
                       else (None, None))
         ctx.save_for_backward(x, hu, ou, q, k, v, lse, pos, back_freq, cu, q0,
@@ -201,8 +209,8 @@ class _Attention(torch.autograd.Function):
         _, o2, uo = _beside(ou, s.q_size)
         o = o2.unflatten(1, (-1, s.head_dim))
 
-        duo = _scaled_mm(g, Bo, scale_o)
-        do = _add(g @ Wo, duo, Ao).view(rows, -1, s.head_dim)
+        do, g2, duo = _through(g, Wo, Ao, Bo, scale_o)
+        do = do.view(rows, -1, s.head_dim)
         sizes, ranks = [s.q_size, s.kv_size, s.kv_size], [a.shape[0] for a in As]
         pad, width = _padded(ranks), sum(sizes)
         dyu, dy, du = _beside(x.new_empty(rows, width + pad), width)
@@ -220,12 +228,14 @@ class _Attention(torch.autograd.Function):
             du[:, sum(ranks):].zero_()
         us = u[:, :sum(ranks)].split(ranks, 1)
         dA, dAo, dBo, *dBs = _sums(
-            [(h, du, False), (o2, duo, False), (g, uo[:, :Ao.shape[0]], True),
+            [(h, du, False), (o2, duo, False), (g2, uo[:, :Ao.shape[0]], True),
              *((y, p, True) for y, p in zip(dys, us))])
         dAs = dA[:sum(ranks)].split(ranks)
         dx = None
         if ctx.needs_input_grad[0]:
-            dh = dyu @ ext.adapted_weight(Ws, As, Bs, pad, True)
+            at = [sum(sizes[:i]) for i in range(3)]
+            at += [width + sum(ranks[:i]) for i in range(3)]
+            dh = dyu @ ext.stack_transposed([*Ws, *As], at, width + pad).t()
             dx = ext.rmsnorm_bwd_add(dh, x, norm, g, ctx.eps[0])
         return (dx, None, None, None, dAs[0], dBs[0], dAs[1], dBs[1], dAs[2],
                 dBs[2], dAo, dBo)
@@ -245,15 +255,14 @@ class _FeedForward(torch.autograd.Function):
         hu, h, u = _beside(x.new_empty(rows, hidden + pad), hidden)
         ext.rmsnorm_fwd_into(x, norm.weight, norm.eps, h)
         _down(h, u, As, scales[:2])
-        W = ext.adapted_weight(Ws, As, Bs, pad, False)
+        W = ext.adapted_weight(Ws, Bs, pad)
         gu = _product(hu, W, mods)
         pad_d, inner = _padded([Ad.shape[0]]), gu.shape[1] // 2
         au, act, ud = _beside(x.new_empty(rows, inner + pad_d), inner)
         ext.silu_mul_packed_into(gu, act)
         _down(act, ud, [Ad], scales[2:])
         Wd = mlp.down_proj.weight
-        y = torch.addmm(x, au, ext.adapted_weight([Wd], [Ad], [Bd], pad_d,
-                                                  False).t())
+        y = torch.addmm(x, au, ext.adapted_weight([Wd], [Bd], pad_d).t())
         ctx.save_for_backward(x, hu, gu, au, norm.weight, Ad, Bd, Wd, *As, *Bs,
                               *Ws)
         ctx.scales, ctx.eps = scales, norm.eps
@@ -270,31 +279,37 @@ class _FeedForward(torch.autograd.Function):
         _, h, u = _beside(hu, hidden)
         _, act, ud = _beside(au, inner)
 
-        # [g | dud]: the adapter's share of dact joins the product
-        pad_d = _padded([Ad.shape[0]])
-        gd, g2, dud = _beside(x.new_empty(rows, hidden + pad_d), hidden)
-        g2.copy_(g)
-        _scaled_mm(g2, Bd, scale_d, out=dud[:, :Ad.shape[0]])
-        if pad_d > Ad.shape[0]:
-            dud[:, Ad.shape[0]:].zero_()
-        dact = gd @ ext.adapted_weight([Wd], [Ad], [Bd], pad_d, True)
+        g = g.contiguous()
+        dact, g2, dud = _through(g, Wd, Ad, Bd, scale_d)
+        # [dgate | du | dup]
         pad = _padded(ranks)
-        dyu, dy, du = _beside(x.new_empty(rows, 2 * inner + pad), 2 * inner)
-        ext.silu_mul_bwd_packed(dact, gu, dy)
-        dys, dus = dy.chunk(2, 1), du[:, :sum(ranks)].split(ranks, 1)
-        _up(dys, dus, Bs, scales)
+        dyu = x.new_empty(rows, 2 * inner + pad)
+        dgate, du, dup = dyu.split([inner, pad, inner], 1)
+        ext.silu_mul_bwd_packed(dact, gu, dgate, dup)
+        dus = du[:, :sum(ranks)].split(ranks, 1)
+        _up((dgate, dup), dus, Bs, scales)
         if pad > sum(ranks):
             du[:, sum(ranks):].zero_()
         us = u[:, :sum(ranks)].split(ranks, 1)
         dA, dAd, dBd, *dBs = _sums(
-            [(h, du, False), (act, dud[:, :Ad.shape[0]], False),
-             (g2, ud[:, :Ad.shape[0]], True),
-             *((y, p, True) for y, p in zip(dys, us))])
+            [(h, du, False), (act, dud, False), (g2, ud[:, :Ad.shape[0]], True),
+             *((y, p, True) for y, p in zip((dgate, dup), us))])
         dAs = dA[:sum(ranks)].split(ranks)
         dx = None
         if ctx.needs_input_grad[0]:
-            dh = dyu @ ext.adapted_weight(Ws, As, Bs, pad, True)
-            dx = ext.rmsnorm_bwd_add(dh, x, norm, g.contiguous(), ctx.eps)
+            at = [0, inner, inner + ranks[0], inner + pad]
+            W = ext.stack_transposed([Ws[0], *As, Ws[1]], at, 2 * inner + pad)
+            half = inner + ranks[0]
+            if rows >= 8192 and hidden <= 2048 and half % 8 == 0:
+                # few columns from many rows: the library's product of twice
+                # the K takes up to three times as long (18793 x 17984 x 1536:
+                # 1080 us, in two 790; from 4000 rows or for 2560 columns one
+                # is the faster)
+                dh = dyu[:, :half] @ W[:, :half].t()
+                dh.addmm_(dyu[:, half:], W[:, half:].t())
+            else:
+                dh = dyu @ W.t()
+            dx = ext.rmsnorm_bwd_add(dh, x, norm, g, ctx.eps)
         return dx, None, None, dAs[0], dBs[0], dAs[1], dBs[1], dAd, dBd
 
 

@@ -109,13 +109,14 @@ std::vector<torch::Tensor> adapter_grads(std::vector<torch::Tensor> y,
                                          std::vector<torch::Tensor> p,
                                          std::vector<int64_t> by_col);
 torch::Tensor adapted_weight(std::vector<torch::Tensor> w,
-                             std::vector<torch::Tensor> a,
-                             std::vector<torch::Tensor> b, int64_t pad,
-                             bool back);
+                             std::vector<torch::Tensor> b, int64_t pad);
+torch::Tensor stack_transposed(std::vector<torch::Tensor> w,
+                               std::vector<int64_t> at, int64_t cols);
 void rmsnorm_fwd_into(torch::Tensor x, torch::Tensor w, double eps,
                       torch::Tensor out);
 void silu_mul_packed_into(torch::Tensor gu, torch::Tensor out);
-void silu_mul_bwd_packed(torch::Tensor dy, torch::Tensor gu, torch::Tensor out);
+void silu_mul_bwd_packed(torch::Tensor dy, torch::Tensor gu,
+                         torch::Tensor dgate, torch::Tensor dup);
 std::vector<torch::Tensor> flash_attn_bwd(torch::Tensor dout, torch::Tensor q,
                                           torch::Tensor k, torch::Tensor v,
                                           torch::Tensor o, torch::Tensor lse,
@@ -218,13 +219,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("adapter_grads", &adapter_grads,
         "p^T y of several operands, summed over the rows");
   m.def("adapted_weight", &adapted_weight,
-        "[W | B] or [W; A] of projections of one input");
+        "[W | B] of projections of one input");
+  m.def("stack_transposed", &stack_transposed,
+        "matrices of K columns side by side, transposed");
   m.def("rmsnorm_fwd_into", &rmsnorm_fwd_into,
         "RMSNorm forward into rows of a wider matrix");
   m.def("silu_mul_packed_into", &silu_mul_packed_into,
         "SiLU*mul of [gate | up] into rows of a wider matrix");
   m.def("silu_mul_bwd_packed", &silu_mul_bwd_packed,
-        "its backward into [dgate | dup]");
+        "its backward into dgate and dup");
   m.def("flash_attn_bwd", &flash_attn_bwd,
         "causal GQA flash attention backward (returns dq, dk, dv)");
 }

@@ -160,16 +160,20 @@ torch::Tensor silu_mul_packed(torch::Tensor gu) {
   return out;
 }
 
-// ---- its backward: dy (N, F), gu (N, 2F) -> out (N, 2F) = [dgate | dup]
+// ---- its backward: dy (N, F), gu (N, 2F) -> dgate, dup (N, F), rows any multiple
+// of 16 bytes apart
 namespace {
 __global__ __launch_bounds__(256)
 void silu_mul_bwd_packed_kernel(const __hip_bfloat16* __restrict__ dy,
                                 const __hip_bfloat16* __restrict__ gu,
-                                __hip_bfloat16* __restrict__ out, int fvec, int64_t ldo) {
+                                __hip_bfloat16* __restrict__ dgate,
+                                __hip_bfloat16* __restrict__ dup, int fvec, int64_t ldg,
+                                int64_t ldu) {
   const int64_t row = blockIdx.x;
   const bf16x8* d8 = reinterpret_cast<const bf16x8*>(dy) + row * fvec;
   const bf16x8* g8 = reinterpret_cast<const bf16x8*>(gu) + row * 2 * fvec;
-  bf16x8* o8 = reinterpret_cast<bf16x8*>(out + row * ldo);
+  bf16x8* dg8 = reinterpret_cast<bf16x8*>(dgate + row * ldg);
+  bf16x8* du8 = reinterpret_cast<bf16x8*>(dup + row * ldu);
   for (int i = threadIdx.x; i < fvec; i += 256) {
     const bf16x8 d = d8[i], g = g8[i], u = g8[fvec + i];
     bf16x8 og, ou;
@@ -180,27 +184,31 @@ void silu_mul_bwd_packed_kernel(const __hip_bfloat16* __restrict__ dy,
       og.v[j] = f2bf(df * bf2f(u.v[j]) * sig * (1.f + gf * (1.f - sig)));
       ou.v[j] = f2bf(df * gf * sig);
     }
-    o8[i] = og;
-    o8[fvec + i] = ou;
+    dg8[i] = og;
+    du8[i] = ou;
   }
 }
 }  // namespace
 
-void silu_mul_bwd_packed(torch::Tensor dy, torch::Tensor gu, torch::Tensor out) {
+void silu_mul_bwd_packed(torch::Tensor dy, torch::Tensor gu, torch::Tensor dgate,
+                         torch::Tensor dup) {
   TORCH_CHECK(dy.is_cuda() && dy.is_contiguous() && dy.dim() == 2 &&
               dy.scalar_type() == at::kBFloat16);
   const int64_t N = dy.size(0), F = dy.size(1);
   TORCH_CHECK(gu.is_cuda() && gu.is_contiguous() && gu.scalar_type() == at::kBFloat16 &&
               gu.dim() == 2 && gu.size(0) == N && gu.size(1) == 2 * F && F % 8 == 0);
-  TORCH_CHECK(out.is_cuda() && out.scalar_type() == at::kBFloat16 && out.sizes() == gu.sizes() &&
-              out.stride(1) == 1 && out.stride(0) % 8 == 0);
-  for (const auto* t : {&dy, &gu, &out})
+  for (const auto* t : {&dgate, &dup})
+    TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kBFloat16 && t->sizes() == dy.sizes() &&
+                t->stride(1) == 1 && t->stride(0) % 8 == 0, "silu_mul_bwd_packed: output");
+  for (const auto* t : {&dy, &gu, &dgate, &dup})
     TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "silu_mul_bwd: alignment");
   if (N == 0) return;
   hipLaunchKernelGGL(silu_mul_bwd_packed_kernel, dim3(N), dim3(256), 0,
                      at::cuda::getCurrentCUDAStream(),
                      reinterpret_cast<const __hip_bfloat16*>(dy.data_ptr()),
                      reinterpret_cast<const __hip_bfloat16*>(gu.data_ptr()),
-                     reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), (int)(F / 8), out.stride(0));
+                     reinterpret_cast<__hip_bfloat16*>(dgate.data_ptr()),
+                     reinterpret_cast<__hip_bfloat16*>(dup.data_ptr()), (int)(F / 8),
+                     dgate.stride(0), dup.stride(0));
   HIP_CHECK_LAST();
 }

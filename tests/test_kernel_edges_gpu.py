@@ -831,13 +831,19 @@ def test_adapted_weight(ext, N, K, ranks, pad):
     ws, As, Bs = ([_rand(s, i) for i, s in enumerate(shapes)] for shapes in (
         [(n, K) for n in N], [(r, K) for r in ranks], list(zip(N, ranks))))
     odd = ws[0].new_empty(ws[0].numel() + 1)[1:].view(ws[0].shape).copy_(ws[0])
-    z = torch.zeros(pad - sum(ranks), K, device="cuda", dtype=torch.bfloat16)
-    beside = torch.block_diag(*Bs, z[:0, :0].new_zeros(0, pad - sum(ranks)))
+    beside = torch.block_diag(*Bs, ws[0].new_zeros(0, pad - sum(ranks)))
     for w0 in (ws[0], odd):
         w = [w0, *ws[1:]]
-        assert torch.equal(ext.adapted_weight(w, As, Bs, pad, False),
-                           torch.cat([torch.cat(ws), beside], 1))
-        assert torch.equal(ext.adapted_weight(w, As, Bs, pad, True), torch.cat([*ws, *As, z]))
+        assert torch.equal(ext.adapted_weight(w, Bs, pad), torch.cat([torch.cat(ws), beside], 1))
+        # a gap of zeros between the first matrix and the rest
+        stack, at = [w0, *As, *ws[1:]], [0]
+        for t in stack[:-1]:
+            at.append(at[-1] + t.shape[0] + (8 if len(at) == 1 else 0))
+        cols = (at[-1] + stack[-1].shape[0] + 7) // 8 * 8
+        ref = torch.zeros(cols, K, device="cuda", dtype=torch.bfloat16)
+        for t, i in zip(stack, at):
+            ref[i:i + t.shape[0]] = t
+        assert torch.equal(ext.stack_transposed(stack, at, cols), ref.t())
 
 
 @pytest.mark.parametrize("rows,F", [(1, 8), (5, 2056), (33, 4864)])
@@ -848,12 +854,13 @@ def test_activation_and_norm_into_wider_rows(ext, rows, F):
     act, back = (torch.full((rows, n + 8), 7.0, dtype=torch.bfloat16, device="cuda")
                  for n in (F, 2 * F))
     ext.silu_mul_packed_into(gu, act[:, :F])
-    ext.silu_mul_bwd_packed(dy, gu, back[:, :-8])
+    ext.silu_mul_bwd_packed(dy, gu, back[:, :F], back[:, F + 8:])
     assert torch.equal(act[:, :F], ext.silu_mul_fwd(gate, up))
-    assert torch.equal(back[:, :-8], torch.cat(ext.silu_mul_bwd(dy, gate, up), 1))
+    ref = ext.silu_mul_bwd(dy, gate, up)
+    assert torch.equal(back[:, :F], ref[0]) and torch.equal(back[:, F + 8:], ref[1])
     ext.rmsnorm_fwd_into(dy, w, 1e-6, act[:, :F])
     assert torch.equal(act[:, :F], ext.rmsnorm_fwd(dy, w, 1e-6))
-    assert (act[:, F:] == 7).all() and (back[:, -8:] == 7).all()
+    assert (act[:, F:] == 7).all() and (back[:, F:F + 8] == 7).all()
 
 
 @pytest.mark.parametrize("T,H,KV,D", [(1, 1, 1, 64), (9, 14, 2, 64), (5, 12, 2, 128)])
