@@ -593,17 +593,20 @@ class Engine:
             at = m.model.layers[li].self_attn
             return at.q_norm.weight, at.k_norm.weight, eps
 
-        def attend(qkv, li):
+        # joins the slices of long contexts; zero between calls
+        if getattr(self, "_arrived", None) is None:
+            self._arrived = torch.zeros(
+                (self.cfg.max_num_seqs + 16) * s.num_kv_heads,  # waves are padded
+                dtype=torch.int32, device=input_ids.device)
+
+        def attend(qkv, li, bias=None):
             """Rotation, cache write and attention of one layer's packed
-            projections (in place)."""
-            ext.rope_scatter_qkv(qkv, pos32, slot_mapping, self._inv_freq,
-                                 self.pool.key[li], self.pool.value[li],
-                                 s.num_heads, s.num_kv_heads, s.head_dim,
-                                 *head_norms(li))
-            return ext.paged_attention_decode_strided(
-                qkv, s.num_heads, s.head_dim, qs + 2 * kvs,
+            projections, or of their partial sums and the bias."""
+            return ext.paged_decode_packed(
+                qkv, bias, pos32, slot_mapping, self._inv_freq,
                 self.pool.key[li], self.pool.value[li], block_tables,
-                context_lens, self.scale).view(-1, qs)
+                context_lens, self._arrived, s.num_heads, self.scale,
+                *head_norms(li))
 
         res = m.model.embed_tokens(input_ids)
         apart = hybrid_down and r > 0
@@ -636,15 +639,7 @@ class Engine:
         if streamed:
             h = ext.rmsnorm_fwd(res, lws[0].in_norm, eps)
             for li, lw in enumerate(lws):
-                q = ext.rope_scatter_join(
-                    ext.stream_gemm(h, lw.tiles["qkv"]), lw.qkv_b, pos32,
-                    slot_mapping, self._inv_freq, self.pool.key[li],
-                    self.pool.value[li], s.num_heads, s.num_kv_heads,
-                    s.head_dim, *head_norms(li))
-                o = ext.paged_attention_decode_strided(
-                    q, s.num_heads, s.head_dim, qs, self.pool.key[li],
-                    self.pool.value[li], block_tables, context_lens,
-                    self.scale).view(-1, qs)
+                o = attend(ext.stream_gemm(h, lw.tiles["qkv"]), li, lw.qkv_b)
                 h, res = ext.add_rmsnorm_join(
                     ext.stream_gemm(o, lw.tiles["o"]), res, lw.post_norm, eps)
                 act = ext.stream_glu(h, lw.tiles["gateup"])

@@ -71,15 +71,13 @@ std::vector<torch::Tensor> add_rmsnorm_join(torch::Tensor parts,
                                             torch::Tensor res, torch::Tensor w,
                                             double eps,
                                             c10::optional<torch::Tensor> bt);
-torch::Tensor rope_scatter_join(torch::Tensor parts,
-                                c10::optional<torch::Tensor> bias,
-                                torch::Tensor positions, torch::Tensor slots,
-                                torch::Tensor inv_freq, torch::Tensor key_cache,
-                                torch::Tensor value_cache, int64_t H,
-                                int64_t KV, int64_t D,
-                                c10::optional<torch::Tensor> q_norm,
-                                c10::optional<torch::Tensor> k_norm,
-                                double eps);
+torch::Tensor paged_decode_packed(
+    torch::Tensor qkv, c10::optional<torch::Tensor> bias,
+    torch::Tensor positions, torch::Tensor slots, torch::Tensor inv_freq,
+    torch::Tensor kcache, torch::Tensor vcache, torch::Tensor block_tables,
+    torch::Tensor ctx_lens, torch::Tensor arrived, int64_t n_heads,
+    double scale, c10::optional<torch::Tensor> q_norm,
+    c10::optional<torch::Tensor> k_norm, double eps);
 bool lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b,
                 torch::Tensor out, double scale);
 bool lora_add(torch::Tensor y, torch::Tensor u, torch::Tensor m,
@@ -189,11 +187,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual + partial sums (+ adapter), then RMSNorm", py::arg("parts"),
         py::arg("res"), py::arg("w"), py::arg("eps"),
         py::arg("bt") = py::none());
-  m.def("rope_scatter_join", &rope_scatter_join,
-        "partial sums of [q|k|v] + bias -> norms, RoPE, KV scatter; returns q",
-        py::arg("parts"), py::arg("bias"), py::arg("positions"),
-        py::arg("slots"), py::arg("inv_freq"), py::arg("key_cache"),
-        py::arg("value_cache"), py::arg("H"), py::arg("KV"), py::arg("D"),
+  m.def("paged_decode_packed", &paged_decode_packed,
+        "packed [q|k|v] or its partial sums -> norms, RoPE, KV scatter, "
+        "paged decode attention",
+        py::arg("qkv"), py::arg("bias"), py::arg("positions"),
+        py::arg("slots"), py::arg("inv_freq"), py::arg("kcache"),
+        py::arg("vcache"), py::arg("block_tables"), py::arg("ctx_lens"),
+        py::arg("arrived"), py::arg("n_heads"), py::arg("scale"),
         py::arg("q_norm") = py::none(), py::arg("k_norm") = py::none(),
         py::arg("eps") = 0.0);
   m.def("lora_merge", &lora_merge, "out = W + scale * B A, one pass");

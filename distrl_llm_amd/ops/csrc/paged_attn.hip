@@ -5,15 +5,25 @@
 // One workgroup owns (sequence, kv head, slice of the context) with all query
 // heads of the kv head; its waves take 32 tokens each in turn and keep a
 // softmax of their own, joined once at the end. Per 32 tokens a wave
-//  * loads K rows straight into MFMA operands (16x16x32: lane = token row,
-//    16 B pieces) and forms S^T[token][head] = K Q^T, q and K exact in bf16,
-//    sums in fp32;
+//  * loads whole K and V rows, neighbouring lanes neighbouring 16 B pieces, and
+//    passes both through tiles of its own in LDS (K straight into MFMA operands,
+//    a row a lane, touched a cache line a lane: the round below 74.7 us, 70.4
+//    now, three long chats 11.3 and 10.6); no workgroup barrier in the loop;
+//  * forms S^T[token][head] = K Q^T (16x16x32), q and K exact in bf16, sums in
+//    fp32;
 //  * keeps the weights in fp32 and feeds them to the second product as two
 //    bf16 terms, p = hi + lo (error 2^-17 of p): the accumulator's token rows
 //    serve as k-slots as they lie;
-//  * passes V rows through a tile of its own in LDS and reads them back
-//    transposed (LDS transpose reads); no workgroup barrier in the loop.
+//  * reads V back transposed (LDS transpose reads).
 // The next 32 tokens' rows are in flight meanwhile (page numbers two ahead).
+//
+// The engine's step fuses what stands before it: the workgroup of (sequence, kv
+// head) takes its heads from the projections' packed rows, or from a product's
+// partial sums and the bias, norms and rotates them, writes the new token's key
+// and value into the cache and attends over them from LDS, while the first rows
+// of the context are on their way. Slices of one sequence are joined by the last
+// of them to end. As kernels of their own rotation and join took 7.7 and 4.6 us a
+// layer at 160 sequences, 3.0 and 1.3 at eight.
 // K and V are read once per sequence and kv head; bound by HBM.
 // 160 sequences of 420..1550 tokens sharing prompts, 28/4 heads of 128
 // (251 MB of distinct rows): 157 us with one lane a token on vector FMAs,
@@ -39,7 +49,25 @@ DEV_INLINE int v_off(int r, int c) {
   return r * (2 * D) + ((c ^ (D == 128 ? r & 15 : (r >> 1) & 7)) << 4);
 }
 
-template <int D, int NW>
+// What the fused kernel makes its queries, keys and values from: packed rows
+// [q heads | k heads | v heads], as bf16 or as fp32 partial sums (splits, N, width)
+struct Packed {
+  const __hip_bfloat16* rows;
+  const float* parts;
+  int splits;
+  const __hip_bfloat16* bias;                 // of the parts, or null
+  const int* positions;
+  const int64_t* slots;                       // cache rows; negative: none
+  const float* inv_freq;
+  const __hip_bfloat16 *q_norm, *k_norm;      // or null
+  float eps;
+  __hip_bfloat16 *kcache, *vcache;
+  int* arrived;                               // (N, KV), zero before and after
+};
+
+enum { QUERIES = 0, ROWS = 1, PARTS = 2 };
+
+template <int D, int NW, int SRC>
 __global__ __launch_bounds__(NW * 64, 2)
 void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q_row_stride
                          const __hip_bfloat16* __restrict__ kcache, // (nb, bs, KV, D)
@@ -50,8 +78,9 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
                          float* __restrict__ o_part,                // (cs, N, H, D)
                          float* __restrict__ ml_part,               // (cs, N, H, 2)
                          int H, int KV, int max_nb, int block_size, int bs_shift,
-                         float scale_log2, int64_t q_row_stride, int slice_len) {
+                         float scale_log2, int64_t q_row_stride, int slice_len, Packed src) {
   constexpr int KS = D / 32, DT = D / 16;
+  constexpr int LPR = D / 8, RPL = 64 / LPR, NL = CHUNK / RPL;   // lanes of a row, rows of a load
   const int seq = blockIdx.x, kv = blockIdx.y, z = blockIdx.z, N = gridDim.x;
   const int group = H / KV;
   const int len = ctx_lens[seq];
@@ -62,15 +91,12 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
   const int l = threadIdx.x & 63, g = l >> 4, lr = l & 15;
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  char* tile = smem + wave * (CHUNK * D * 2);           // also 16 heads x D floats
-  float* ml_lds = reinterpret_cast<float*>(smem + NW * (CHUNK * D * 2));  // [NW][16][2]
-
-  bf16v8 qf[KS];
-  #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const __hip_bfloat16* qp = q + seq * q_row_stride + (kv * group + min(lr, group - 1)) * D;
-    qf[ks] = *reinterpret_cast<const bf16v8*>(qp + ks * 32 + g * 8);   // spare columns repeat
-  }
+  char* ktile = smem + wave * (2 * CHUNK * D * 2);      // also 16 heads x D floats
+  char* tile = ktile + CHUNK * D * 2;
+  float* ml_lds = reinterpret_cast<float*>(smem + NW * (2 * CHUNK * D * 2));  // [NW][16][2]
+  // fused: the heads' queries, then the new token's key and value
+  __hip_bfloat16* fresh = reinterpret_cast<__hip_bfloat16*>(ml_lds + NW * 32);
+  const int last = SRC == QUERIES ? 0x7fffffff : len - 1;
 
   float m = -1e30f, lsum = 0.f;
   f32x4 acc[DT];
@@ -79,62 +105,144 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
 
   const int* bt = block_tables + (int64_t)seq * max_nb;
   const int row_elems = KV * D;
-  bf16v8 kf[2][KS], vf[2][KS];
-  int page[2], slot[2];                 // this lane's two tokens of a chunk
+  bf16v8 kf[NL], vf[NL];
+  int row;                              // of the pool, of this lane's token l % 32 of a chunk
   auto lookup = [&](int t0) {
-    #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int t = min(t0 + s * 16 + lr, c1 - 1);      // past the end: weight zero
-      const int b = bs_shift >= 0 ? t >> bs_shift : t / block_size;
-      slot[s] = t - b * block_size;
-      page[s] = bt[b];
-    }
+    const int t = min(t0 + (l & 31), c1 - 1);           // past the end: weight zero
+    const int b = bs_shift >= 0 ? t >> bs_shift : t / block_size;
+    row = bt[b] * block_size + (t - b * block_size);
   };
-  auto offset = [&](int s) {
-    return ((int64_t)page[s] * block_size + slot[s]) * row_elems + kv * D + g * 8;
+  auto load = [&] {
+    #pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int64_t at = (int64_t)__shfl(row, i * RPL + l / LPR, WAVE) * row_elems + kv * D +
+                         (l % LPR) * 8;
+      kf[i] = *reinterpret_cast<const bf16v8*>(kcache + at);
+      vf[i] = *reinterpret_cast<const bf16v8*>(vcache + at);
+    }
   };
 
   int t0 = c0 + wave * CHUNK;
   if (t0 < c1) {
     lookup(t0);
+    load();
+    lookup(t0 + NW * CHUNK);
+  }
+  bf16v8 qf[KS];
+  if constexpr (SRC == QUERIES) {
     #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int64_t at = offset(s);
+    for (int ks = 0; ks < KS; ++ks) {
+      const __hip_bfloat16* qp = q + seq * q_row_stride + (kv * group + min(lr, group - 1)) * D;
+      qf[ks] = *reinterpret_cast<const bf16v8*>(qp + ks * 32 + g * 8);   // spare columns repeat
+    }
+  } else {
+    // eight rotation pairs a thread, so a head takes D / 16 neighbouring lanes;
+    // then the value, eight elements a thread
+    constexpr int PER = D / 16;
+    const int width = (H + 2 * KV) * D;
+    const bool owner = z + 1 == (int)gridDim.z || c0 + slice_len >= len;
+    auto take = [&](float (&x)[8], int at) {
+      if constexpr (SRC == ROWS) {
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(src.rows + (int64_t)seq * width + at);
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = bf2f(v.v[j]);
+      } else {
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = 0.f;
+        if (src.bias) {
+          const bf16x8 v = *reinterpret_cast<const bf16x8*>(src.bias + at);
+          #pragma unroll
+          for (int j = 0; j < 8; ++j) x[j] = bf2f(v.v[j]);
+        }
+        add_parts8(x, src.parts + (int64_t)seq * width + at, (int64_t)N * width, src.splits);
+      }
+    };
+    const int64_t slot = src.slots[seq];
+    const int units = (group + (owner ? 1 : 0)) * PER, all = units + (owner ? D / 8 : 0);
+    for (int u = threadIdx.x; u < all; u += NW * 64) {
+      bf16x8 x, y;
+      if (u >= units) {
+        const int c = (u - units) * 8;
+        float v[8];
+        take(v, (H + KV + kv) * D + c);
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) x.v[j] = f2bf(v[j]);
+        *reinterpret_cast<bf16x8*>(fresh + (group + 1) * D + c) = x;
+        if (slot >= 0)
+          *reinterpret_cast<bf16x8*>(src.vcache + (slot * KV + kv) * D + c) = x;
+        continue;
+      }
+      const int head = u / PER, c = u % PER * 8;        // head == group: the key
+      const int at = (head < group ? kv * group + head : H + kv) * D + c;
+      float x1[8], x2[8];
+      take(x1, at);
+      take(x2, at + D / 2);
+      const __hip_bfloat16* nw = head < group ? src.q_norm : src.k_norm;
+      if (nw) {
+        float ss = 0.f;
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) ss += x1[j] * x1[j] + x2[j] * x2[j];
+        #pragma unroll
+        for (int off = PER / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, WAVE);
+        const float r = rsqrtf(ss / D + src.eps);
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          x1[j] *= r * bf2f(nw[c + j]);
+          x2[j] *= r * bf2f(nw[c + D / 2 + j]);
+        }
+      }
+      const float pos = (float)src.positions[seq];
       #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        kf[s][ks] = *reinterpret_cast<const bf16v8*>(kcache + at + ks * 32);
-        vf[s][ks] = *reinterpret_cast<const bf16v8*>(vcache + at + ks * 32);
+      for (int j = 0; j < 8; ++j) {
+        const float a = pos * src.inv_freq[c + j], sn = __sinf(a), cs = __cosf(a);
+        x.v[j] = f2bf(x1[j] * cs - x2[j] * sn);
+        y.v[j] = f2bf(x2[j] * cs + x1[j] * sn);
+      }
+      *reinterpret_cast<bf16x8*>(fresh + head * D + c) = x;
+      *reinterpret_cast<bf16x8*>(fresh + head * D + c + D / 2) = y;
+      if (head == group && slot >= 0) {
+        __hip_bfloat16* kd = src.kcache + (slot * KV + kv) * D + c;
+        *reinterpret_cast<bf16x8*>(kd) = x;
+        *reinterpret_cast<bf16x8*>(kd + D / 2) = y;
       }
     }
-    lookup(t0 + NW * CHUNK);
+    __syncthreads();
+    #pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = *reinterpret_cast<const bf16v8*>(fresh + min(lr, group - 1) * D + ks * 32 + g * 8);
   }
   for (; t0 < c1; t0 += NW * CHUNK) {
     const bool more = t0 + NW * CHUNK < c1;             // wave-uniform
-    int64_t at[2];
+    if (SRC != QUERIES && t0 + CHUNK > last) {
+      // the new token, and what repeats it past the end: its row of the cache may
+      // not be written yet
+      #pragma unroll
+      for (int i = 0; i < NL; ++i)
+        if (t0 + i * RPL + l / LPR >= last) {
+          kf[i] = *reinterpret_cast<const bf16v8*>(fresh + group * D + l % LPR * 8);
+          vf[i] = *reinterpret_cast<const bf16v8*>(fresh + (group + 1) * D + l % LPR * 8);
+        }
+    }
     #pragma unroll
-    for (int s = 0; s < 2; ++s) at[s] = offset(s);
+    for (int i = 0; i < NL; ++i) {
+      const int r = i * RPL + l / LPR, c = l % LPR;
+      *reinterpret_cast<bf16v8*>(ktile + v_off<D>(r, c)) = kf[i];
+      *reinterpret_cast<bf16v8*>(tile + v_off<D>(r, c)) = vf[i];
+    }
+    if (more) {
+      load();
+      lookup(t0 + 2 * NW * CHUNK);
+    }
+    __builtin_amdgcn_wave_barrier();
     f32x4 st[2];
     #pragma unroll
     for (int s = 0; s < 2; ++s) {
       st[s] = f32x4{0.f, 0.f, 0.f, 0.f};
       #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
-        st[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s][ks], qf[ks], st[s], 0, 0, 0);
-    }
-    #pragma unroll
-    for (int s = 0; s < 2; ++s)
-      #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        *reinterpret_cast<bf16v8*>(tile + v_off<D>(s * 16 + lr, ks * 4 + g)) = vf[s][ks];
-    if (more) {
-      #pragma unroll
-      for (int s = 0; s < 2; ++s)
-        #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          kf[s][ks] = *reinterpret_cast<const bf16v8*>(kcache + at[s] + ks * 32);
-          vf[s][ks] = *reinterpret_cast<const bf16v8*>(vcache + at[s] + ks * 32);
-        }
-      lookup(t0 + 2 * NW * CHUNK);
+        st[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            *reinterpret_cast<const bf16v8*>(ktile + v_off<D>(s * 16 + lr, ks * 4 + g)), qf[ks],
+            st[s], 0, 0, 0);
     }
 
     // this lane: head lr, tokens t0 + 16 s + 4 g + r
@@ -191,7 +299,7 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
     ml_lds[(wave * 16 + lr) * 2] = m;
     ml_lds[(wave * 16 + lr) * 2 + 1] = lsum;
   }
-  float* o_tile = reinterpret_cast<float*>(tile);       // [16 heads][D]
+  float* o_tile = reinterpret_cast<float*>(ktile);      // [16 heads][D]
   #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
     *reinterpret_cast<f32x4*>(o_tile + lr * D + dt * 16 + g * 4) = acc[dt];
@@ -207,7 +315,7 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
     for (int w = 0; w < NW; ++w) {
       const float f = __builtin_amdgcn_exp2f(ml_lds[(w * 16 + h) * 2] - top);
       total += f * ml_lds[(w * 16 + h) * 2 + 1];
-      const f32x4 x = *reinterpret_cast<const f32x4*>(smem + w * (CHUNK * D * 2) + (h * D + d) * 4);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(smem + w * (2 * CHUNK * D * 2) + (h * D + d) * 4);
       #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] += f * x[r];
     }
@@ -222,6 +330,38 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
       const int64_t at = (int64_t)z * N * H + head;
       *reinterpret_cast<f32x4*>(o_part + at * D + d) = o;
       if (d == 0) { ml_part[at * 2] = top; ml_part[at * 2 + 1] = total; }
+    }
+  }
+  if constexpr (SRC != QUERIES) {
+    if (whole) return;
+    // the last slice of the sequence and kv head to end joins them
+    __shared__ int before;
+    __threadfence();
+    __syncthreads();
+    const int n = min((len + slice_len - 1) / slice_len, (int)gridDim.z);
+    int* arrived = src.arrived + seq * KV + kv;
+    if (threadIdx.x == 0) before = atomicAdd(arrived, 1);
+    __syncthreads();
+    if (before != n - 1) return;
+    __threadfence();
+    if (threadIdx.x == 0) atomicExch(arrived, 0);
+    for (int i = threadIdx.x; i < group * (D / 4); i += NW * 64) {
+      const int h = i / (D / 4), d = i % (D / 4) * 4;
+      const int64_t head = (int64_t)seq * H + kv * group + h, step = (int64_t)N * H;
+      float top = -1e30f, total = 0.f;
+      for (int s = 0; s < n; ++s) top = fmaxf(top, ml_part[(s * step + head) * 2]);
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < n; ++s) {
+        const int64_t at = s * step + head;
+        const float f = __builtin_amdgcn_exp2f(ml_part[at * 2] - top);
+        total += f * ml_part[at * 2 + 1];
+        o += *reinterpret_cast<const f32x4*>(o_part + at * D + d) * f;
+      }
+      const float inv = total > 0.f ? 1.f / total : 0.f;
+      bf16v4 y;
+      #pragma unroll
+      for (int r = 0; r < 4; ++r) y[r] = (__bf16)(o[r] * inv);
+      *reinterpret_cast<bf16v4*>(out + head * D + d) = y;
     }
   }
 }
@@ -256,12 +396,12 @@ void paged_decode_combine_kernel(const float* __restrict__ o_part,
   for (int e = 0; e < D / 64; ++e) out[head * D + lane + e * 64] = f2bf(o[e] * inv);
 }
 
-template <int D, int NW>
-void launch_decode(const torch::Tensor& q, const torch::Tensor& kcache,
+template <int D, int NW, int SRC>
+void launch_decode(const __hip_bfloat16* q, const torch::Tensor& kcache,
                    const torch::Tensor& vcache, const torch::Tensor& bt,
-                   const torch::Tensor& ctx, torch::Tensor& out, int H, int KV,
-                   float scale, int64_t q_row_stride, int cs, int slice_len) {
-  const int N = q.size(0), block_size = kcache.size(1);
+                   const torch::Tensor& ctx, torch::Tensor& out, int N, int H, int KV,
+                   float scale, int64_t q_row_stride, int cs, int slice_len, const Packed& src) {
+  const int block_size = kcache.size(1);
   const int shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1;
   auto stream = at::cuda::getCurrentCUDAStream();
   torch::Tensor part;
@@ -273,16 +413,57 @@ void launch_decode(const torch::Tensor& q, const torch::Tensor& kcache,
     ml_p = o_p + heads * D;
   }
   auto* o = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
-  hipLaunchKernelGGL((paged_decode_kernel<D, NW>), dim3(N, KV, cs), dim3(NW * 64),
-                     NW * (CHUNK * D * 2 + 16 * 2 * 4), stream,
-                     reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()),
-                     reinterpret_cast<const __hip_bfloat16*>(kcache.data_ptr()),
+  const int smem = NW * (2 * CHUNK * D * 2 + 16 * 2 * 4) + (SRC == QUERIES ? 0 : (H / KV + 2) * D * 2);
+  hipLaunchKernelGGL((paged_decode_kernel<D, NW, SRC>), dim3(N, KV, cs), dim3(NW * 64), smem,
+                     stream, q, reinterpret_cast<const __hip_bfloat16*>(kcache.data_ptr()),
                      reinterpret_cast<const __hip_bfloat16*>(vcache.data_ptr()),
                      bt.data_ptr<int>(), ctx.data_ptr<int>(), o, o_p, ml_p, H, KV,
-                     (int)bt.size(1), block_size, shift, scale * LOG2E, q_row_stride, slice_len);
-  if (cs > 1)
+                     (int)bt.size(1), block_size, shift, scale * LOG2E, q_row_stride, slice_len,
+                     src);
+  if (SRC == QUERIES && cs > 1)
     hipLaunchKernelGGL((paged_decode_combine_kernel<D>), dim3(N, H), dim3(64), 0, stream, o_p,
                        ml_p, ctx.data_ptr<int>(), o, H, slice_len, cs);
+}
+
+// Slices of the context (known here: a table's width, not its sequence's
+// length). A round of loads takes ~4 us from cold pages, joining as long: few
+// sequences run with eight waves in slices of 512 tokens, up to one workgroup a
+// CU (3 sequences of 911..3777, 2 kv heads: 1 slice 18 us, 2: 13.5, 4: 11.1, 8:
+// 11.5; 16 of 1500, 4 kv heads: 18.4, 18.2, 4: 16.8, 6: 21; 8 of 4000, 8 kv heads:
+// 37, 30, 29, 8: 35). From 129 workgroups on one slice is left of that, a fifth
+// too slow at most (33 of 4000, 4 kv heads: 50, 2: 61, 3: 50, 4: 57). More
+// sequences fill the chip by themselves (the round above: 60.2 us, 2: 59.8, 4:
+// 62; 10 x 16 of 180..380: 21, 2: 27; 63 of 4000: 100, 2: 101).
+int slices(int64_t blocks, int max_ctx) {
+  int cs = blocks < 256 ? (int)std::max<int64_t>(1, std::min<int64_t>(256 / blocks, CDIV(max_ctx, 512)))
+                        : 1;
+  if (const char* e = getenv("DISTRL_PAGED_CS")) {
+    cs = std::max(1, std::min(atoi(e), 16));
+    while (cs > 1 && (max_ctx + cs - 1) / cs < 32) cs /= 2;
+  }
+  return cs;
+}
+
+// out (N, H, D) by the kernel for its sizes
+template <int SRC>
+void decode(const __hip_bfloat16* q, const torch::Tensor& kcache, const torch::Tensor& vcache,
+            const torch::Tensor& bt, const torch::Tensor& ctx, torch::Tensor& out, int N, int H,
+            int KV, int D, double scale, int64_t q_row_stride, const Packed& src) {
+  const int group = H / KV, max_ctx = bt.size(1) * kcache.size(1);
+  TORCH_CHECK(H % KV == 0 && group <= 16, "GQA group too large");
+  if (N == 0) return;
+  TORCH_CHECK((D == 128 && (group <= 2 || (group >= 4 && group <= 8))) ||
+              (D == 64 && (group == 1 || group == 2 || group == 4 || group == 7)),
+              "paged decode: unsupported (head_dim=", D, ", gqa group=", group, ")");
+  const int64_t blocks = (int64_t)N * KV;
+  const bool few = blocks < 256;
+  const int cs = slices(blocks, max_ctx), slice_len = std::max(1, CDIV(max_ctx, cs));
+  #define DECODE(DD, NN) launch_decode<DD, NN, SRC>(q, kcache, vcache, bt, ctx, out, N, H, KV, \
+                                                    (float)scale, q_row_stride, cs, slice_len, src)
+  if (D == 128) { if (few) DECODE(128, 8); else DECODE(128, 4); }
+  else { if (few) DECODE(64, 8); else DECODE(64, 4); }
+  #undef DECODE
+  HIP_CHECK_LAST();
 }
 
 }  // namespace
@@ -303,46 +484,67 @@ torch::Tensor paged_attention_decode_strided(
     q = q.view({N, q_row_stride}).slice(1, 0, (int64_t)H * D).clone(at::MemoryFormat::Contiguous);
     q_row_stride = (int64_t)H * D;
   }
-  const int KV = kcache.size(2);
-  const int block_size = kcache.size(1);
-  const int max_nb = block_tables.size(1);
-  const int group = H / KV;
-  TORCH_CHECK(H % KV == 0 && group <= 16, "GQA group too large");
-
   auto out = torch::empty({N, (int64_t)H, (int64_t)D}, q.options());
-  if (N == 0) return out;
-  TORCH_CHECK((D == 128 && (group <= 2 || (group >= 4 && group <= 8))) ||
-              (D == 64 && (group == 1 || group == 2 || group == 4 || group == 7)),
-              "paged decode: unsupported (head_dim=", D, ", gqa group=", group, ")");
+  decode<QUERIES>(reinterpret_cast<const __hip_bfloat16*>(q.data_ptr()), kcache, vcache,
+                  block_tables, ctx_lens, out, N, H, kcache.size(2), D, scale, q_row_stride, {});
+  return out;
+}
 
-  // Slices of the context (known here: a table's width, not its sequence's
-  // length). A round of loads takes ~4 us from cold pages, the joining kernel
-  // as long: few sequences run with eight waves in slices of 512 tokens, up to
-  // one workgroup a CU (16 sequences of 1500, 4 kv heads: 1 slice 25 us, 2: 18,
-  // 4: 14, 6: 19; 8 sequences of 4000, 8 kv heads: 63, 39, 29, 8 slices 34).
-  // From 129 workgroups on one slice is left of that, right up to some 2000
-  // tokens (40 sequences of 1550, 4 kv heads: 26, 2: 32, 4: 35; 30 of 500, 8 kv
-  // heads: 13, 2: 18) and up to a fifth too slow beyond (33 of 4000, 4 kv heads:
-  // 61, 3: 55, 4: 51; 63 of them: 89, 2: 91, 4: 96).
-  // More sequences fill the chip by themselves; two slices even out their
-  // lengths where they are long (the round above: 1 slice 80 us, 2: 76, 4: 79;
-  // 32 sequences of 700, 8 kv heads: 16, 18, 21).
-  const int max_ctx = max_nb * block_size;
-  const int64_t blocks = (int64_t)N * KV;
-  const bool few = blocks < 256;
-  int cs = few ? (int)std::max<int64_t>(1, std::min<int64_t>(256 / blocks, CDIV(max_ctx, 512)))
-               : (blocks < 1024 && max_ctx >= 1024 ? 2 : 1);
-  if (const char* e = getenv("DISTRL_PAGED_CS")) {
-    cs = std::max(1, std::min(atoi(e), 16));
-    while (cs > 1 && (max_ctx + cs - 1) / cs < 32) cs /= 2;
+// One decode step's attention from the packed projections [q | k | v] of its N
+// tokens, (N, (H + 2 KV) D) bf16 or (splits, N, ...) fp32 partial sums without
+// their bias: head norms (if given), rotation, the new keys and values into the
+// cache, attention over it. Returns (N, H D). arrived: int32, N KV zeros at least,
+// which it leaves zero; calls that may overlap need one each.
+torch::Tensor paged_decode_packed(torch::Tensor qkv, c10::optional<torch::Tensor> bias,
+                                  torch::Tensor positions, torch::Tensor slots,
+                                  torch::Tensor inv_freq, torch::Tensor kcache,
+                                  torch::Tensor vcache, torch::Tensor block_tables,
+                                  torch::Tensor ctx_lens, torch::Tensor arrived, int64_t n_heads,
+                                  double scale, c10::optional<torch::Tensor> q_norm,
+                                  c10::optional<torch::Tensor> k_norm, double eps) {
+  const bool parts = qkv.dim() == 3;
+  TORCH_CHECK(qkv.is_cuda() && qkv.is_contiguous() && (parts || qkv.dim() == 2) &&
+              qkv.scalar_type() == (parts ? at::kFloat : at::kBFloat16));
+  const int N = qkv.size(-2), H = (int)n_heads, KV = kcache.size(2), D = kcache.size(3);
+  TORCH_CHECK(qkv.size(-1) == (int64_t)(H + 2 * KV) * D && (parts || !bias));
+  TORCH_CHECK(kcache.is_contiguous() && vcache.is_contiguous() && vcache.sizes() == kcache.sizes() &&
+              kcache.scalar_type() == at::kBFloat16 && vcache.scalar_type() == at::kBFloat16);
+  TORCH_CHECK(positions.scalar_type() == at::kInt && slots.scalar_type() == at::kLong &&
+              positions.numel() == N && slots.numel() == N && inv_freq.numel() == D / 2 &&
+              inv_freq.scalar_type() == at::kFloat);
+  TORCH_CHECK(block_tables.scalar_type() == at::kInt && block_tables.is_contiguous() &&
+              block_tables.size(0) == N && ctx_lens.scalar_type() == at::kInt &&
+              ctx_lens.numel() == N);
+  TORCH_CHECK(arrived.is_cuda() && arrived.scalar_type() == at::kInt && arrived.is_contiguous() &&
+              arrived.numel() >= (int64_t)N * KV);
+  auto vec = [&](const c10::optional<torch::Tensor>& w, int64_t n) {
+    if (!w) return (const __hip_bfloat16*)nullptr;
+    TORCH_CHECK(w->is_cuda() && w->is_contiguous() && w->scalar_type() == at::kBFloat16 &&
+                w->numel() == n, "paged_decode_packed: norm weight or bias");
+    return reinterpret_cast<const __hip_bfloat16*>(w->data_ptr());
+  };
+  Packed src{};
+  src.bias = vec(bias, qkv.size(-1));
+  src.q_norm = vec(q_norm, D);
+  src.k_norm = vec(k_norm, D);
+  for (const void* p : {(const void*)qkv.data_ptr(), (const void*)src.bias})
+    TORCH_CHECK(reinterpret_cast<uintptr_t>(p) % 16 == 0, "paged_decode_packed: alignment");
+  src.positions = positions.data_ptr<int>();
+  src.slots = slots.data_ptr<int64_t>();
+  src.inv_freq = inv_freq.data_ptr<float>();
+  src.eps = (float)eps;
+  src.kcache = reinterpret_cast<__hip_bfloat16*>(kcache.data_ptr());
+  src.vcache = reinterpret_cast<__hip_bfloat16*>(vcache.data_ptr());
+  src.arrived = arrived.data_ptr<int>();
+  auto out = torch::empty({N, (int64_t)H * D}, qkv.options().dtype(at::kBFloat16));
+  if (parts) {
+    src.parts = qkv.data_ptr<float>();
+    src.splits = qkv.size(0);
+    decode<PARTS>(nullptr, kcache, vcache, block_tables, ctx_lens, out, N, H, KV, D, scale, 0, src);
+  } else {
+    src.rows = reinterpret_cast<const __hip_bfloat16*>(qkv.data_ptr());
+    decode<ROWS>(nullptr, kcache, vcache, block_tables, ctx_lens, out, N, H, KV, D, scale, 0, src);
   }
-  const int slice_len = std::max(1, CDIV(max_ctx, cs));
-  #define DECODE(DD, NN) launch_decode<DD, NN>(q, kcache, vcache, block_tables, ctx_lens, out, H, \
-                                               KV, (float)scale, q_row_stride, cs, slice_len)
-  if (D == 128) { if (few) DECODE(128, 8); else DECODE(128, 4); }
-  else { if (few) DECODE(64, 8); else DECODE(64, 4); }
-  #undef DECODE
-  HIP_CHECK_LAST();
   return out;
 }
 

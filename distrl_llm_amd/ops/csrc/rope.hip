@@ -206,84 +206,6 @@ void rope_scatter_vec_kernel(__hip_bfloat16* __restrict__ qkv, const int* __rest
   }
 }
 
-// The same behind a product that left partial sums (S, T, (H + 2 KV) D): they
-// and the bias are added up on the way, q goes to (T, H D).
-__global__ __launch_bounds__(512)
-void rope_scatter_join_kernel(const float* __restrict__ parts, int S,
-                              const __hip_bfloat16* __restrict__ bias, __hip_bfloat16* __restrict__ q,
-                              const int* __restrict__ positions, const int64_t* __restrict__ slots,
-                              const float* __restrict__ inv_freq,
-                              __hip_bfloat16* __restrict__ key_cache,
-                              __hip_bfloat16* __restrict__ value_cache,
-                              const __hip_bfloat16* __restrict__ q_norm,
-                              const __hip_bfloat16* __restrict__ k_norm, float eps, int H, int KV,
-                              int D) {
-  const int t = blockIdx.x, half = D / 2, per = half / 8;
-  const int64_t slot = slots[t], width = (int64_t)(H + 2 * KV) * D, step = gridDim.x * width;
-  const float pos = (float)positions[t];
-  const float* base = parts + t * width;
-  auto add_up = [&](float (&v)[8], int at) {
-    #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = 0.f;
-    if (bias) {
-      const bf16x8 b = *reinterpret_cast<const bf16x8*>(bias + at);
-      #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = bf2f(b.v[j]);
-    }
-    add_parts8(v, base + at, step, S);
-  };
-  const int c = threadIdx.x % per * 8;          // the block is a multiple of per: fixed
-  float cs[8], sn[8];
-  #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const float a = pos * inv_freq[c + j];
-    sn[j] = __sinf(a);
-    cs[j] = __cosf(a);
-  }
-  const int rot = (H + KV) * per, all = rot + KV * D / 8;
-  for (int u = threadIdx.x; u < all; u += blockDim.x) {
-    if (u >= rot) {                             // a value unit
-      if (slot < 0) continue;
-      const int i = u - rot;
-      float v[8];
-      add_up(v, (H + KV) * D + i * 8);
-      bf16x8 o;
-      #pragma unroll
-      for (int j = 0; j < 8; ++j) o.v[j] = f2bf(v[j]);
-      reinterpret_cast<bf16x8*>(value_cache)[slot * (KV * D / 8) + i] = o;
-      continue;
-    }
-    const int head = u / per;
-    float x1[8], x2[8];
-    add_up(x1, head * D + c);
-    add_up(x2, head * D + c + half);
-    const __hip_bfloat16* nw = head < H ? q_norm : k_norm;
-    if (nw) {
-      float ss = 0.f;
-      #pragma unroll
-      for (int j = 0; j < 8; ++j) ss += x1[j] * x1[j] + x2[j] * x2[j];
-      for (int off = per / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, WAVE);
-      const float r = rsqrtf(ss / D + eps);
-      #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        x1[j] *= r * bf2f(nw[c + j]);
-        x2[j] *= r * bf2f(nw[c + half + j]);
-      }
-    }
-    bf16x8 x, y;
-    #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      x.v[j] = f2bf(x1[j] * cs[j] - x2[j] * sn[j]);
-      y.v[j] = f2bf(x2[j] * cs[j] + x1[j] * sn[j]);
-    }
-    if (head >= H && slot < 0) continue;
-    __hip_bfloat16* p = head < H ? q + ((int64_t)t * H + head) * D + c
-                                 : key_cache + (slot * KV + head - H) * D + c;
-    *reinterpret_cast<bf16x8*>(p) = x;
-    *reinterpret_cast<bf16x8*>(p + half) = y;
-  }
-}
-
 }  // namespace
 
 void rope_scatter_qkv(torch::Tensor qkv, torch::Tensor positions,
@@ -331,40 +253,6 @@ void rope_scatter_qkv(torch::Tensor qkv, torch::Tensor positions,
                      reinterpret_cast<__hip_bfloat16*>(value_cache.data_ptr()),
                      (int)H, (int)KV, (int)D);
   HIP_CHECK_LAST();
-}
-
-torch::Tensor rope_scatter_join(torch::Tensor parts, c10::optional<torch::Tensor> bias,
-                                torch::Tensor positions, torch::Tensor slots,
-                                torch::Tensor inv_freq, torch::Tensor key_cache,
-                                torch::Tensor value_cache, int64_t H, int64_t KV, int64_t D,
-                                c10::optional<torch::Tensor> q_norm,
-                                c10::optional<torch::Tensor> k_norm, double eps) {
-  TORCH_CHECK(parts.is_cuda() && parts.is_contiguous() && parts.dim() == 3 &&
-              parts.scalar_type() == at::kFloat);
-  TORCH_CHECK(positions.scalar_type() == at::kInt && slots.scalar_type() == at::kLong);
-  const int T = parts.size(1);
-  TORCH_CHECK(parts.size(2) == (H + 2 * KV) * D && positions.numel() == T && slots.numel() == T);
-  TORCH_CHECK(D == 64 || D == 128, "rope_scatter_join: head_dim 64 or 128");
-  auto vec = [&](const c10::optional<torch::Tensor>& w, int64_t n) {
-    if (!w) return (const __hip_bfloat16*)nullptr;
-    TORCH_CHECK(w->is_cuda() && w->is_contiguous() && w->scalar_type() == at::kBFloat16 &&
-                w->numel() == n, "rope_scatter_join: norm weight or bias");
-    return reinterpret_cast<const __hip_bfloat16*>(w->data_ptr());
-  };
-  const auto *b = vec(bias, parts.size(2)), *qn = vec(q_norm, D), *kn = vec(k_norm, D);
-  TORCH_CHECK(reinterpret_cast<uintptr_t>(b) % 16 == 0, "rope_scatter_join: bias on 16 bytes");
-  auto q = torch::empty({T, H * D}, parts.options().dtype(at::kBFloat16));
-  if (T == 0) return q;
-  const int units = (H + KV) * (D / 16) + KV * D / 8;
-  hipLaunchKernelGGL(rope_scatter_join_kernel, dim3(T), dim3(std::min(512, CDIV(units, 64) * 64)), 0,
-                     at::cuda::getCurrentCUDAStream(), parts.data_ptr<float>(), (int)parts.size(0),
-                     b, reinterpret_cast<__hip_bfloat16*>(q.data_ptr()), positions.data_ptr<int>(),
-                     slots.data_ptr<int64_t>(), inv_freq.data_ptr<float>(),
-                     reinterpret_cast<__hip_bfloat16*>(key_cache.data_ptr()),
-                     reinterpret_cast<__hip_bfloat16*>(value_cache.data_ptr()), qn, kn, (float)eps,
-                     (int)H, (int)KV, (int)D);
-  HIP_CHECK_LAST();
-  return q;
 }
 
 // q (T, H, D), k (T, KV, D), whose rows may lie apart

@@ -106,28 +106,49 @@ def test_add_rmsnorm_join(ext, S, rows, hidden, r):
         < 2.0 ** -7
 
 
-@pytest.mark.parametrize("H,KV,D", [(14, 2, 64), (28, 4, 128), (3, 1, 64), (64, 8, 128)])
-@pytest.mark.parametrize("S,bias,norms", [(1, False, False), (3, True, False), (6, False, True)])
-def test_rope_scatter_join(ext, H, KV, D, S, bias, norms):
-    """Against the rotation of the summed rows (its inputs rounded to bf16: two
-    roundings more); a row without a slot leaves the cache alone."""
-    T, width = 5, (H + 2 * KV) * D
-    g = torch.Generator(device="cuda").manual_seed(S)
-    parts = torch.randn((S, T, width), generator=g, device="cuda")
+@pytest.mark.parametrize("H,KV,D", [(14, 2, 64), (28, 4, 128), (8, 8, 64), (64, 8, 128)])
+@pytest.mark.parametrize("N,longest,bs", [(1, 1, 16), (5, 40, 16), (3, 2500, 16), (9, 700, 24),
+                                          (130, 90, 16)])
+@pytest.mark.parametrize("S,bias,norms", [(0, False, False), (1, True, False), (5, False, True)])
+def test_paged_decode_packed(ext, H, KV, D, N, longest, bs, S, bias, norms):
+    """Against rotation with cache write and attention as two calls on the
+    summed rows (their inputs rounded to bf16: a few roundings more): one slice
+    and several, more than once with the same counters, a row of the cache that
+    holds no number before it is written, a token without a slot."""
+    width, g = (H + 2 * KV) * D, torch.Generator(device="cuda").manual_seed(N)
+    lens = torch.randint(1, longest + 1, (N,), generator=g, device="cuda", dtype=torch.int32)
+    lens[0] = longest
+    nb = (longest + bs - 1) // bs
+    pages = torch.randperm(N * nb, generator=g, device="cuda").view(N, nb).int()
+    pos = (lens - 1).int()
+    slots = pages.gather(1, (pos // bs).long()[:, None])[:, 0].long() * bs + pos % bs
+    cache = [_rand((N * nb, bs, KV, D), 4 + i) for i in range(2)]
+    for c in cache:
+        c.view(-1, KV, D)[slots] = float("nan")
+    parts = torch.randn((max(S, 1), N, width), generator=g, device="cuda")
     b = _rand((width,), 1) if bias else None
     nw = (_rand((D,), 2, 0.1) + 1, _rand((D,), 3, 0.1) + 1, 1e-6) if norms else ()
-    pos = torch.tensor([0, 7, 1, 1500, 3], dtype=torch.int32, device="cuda")
-    slots = torch.tensor([4, 0, -1, 9, 2], device="cuda")
     inv = 1.0 / 1e4 ** (torch.arange(0, D, 2, device="cuda").float() / D)
-    cache = [_rand((12, KV, D), 4 + i) for i in range(2)]
+    rows = (parts.sum(0) + (b.float() if bias else 0)).to(torch.bfloat16)
+    arrived = torch.zeros(N * KV, dtype=torch.int32, device="cuda")
+    ref_cache, ref_rows = [c.clone() for c in cache], rows.clone()
+    ext.rope_scatter_qkv(ref_rows, pos, slots, inv, *ref_cache, H, KV, D, *nw)
+    queries = ref_rows[:, :H * D].reshape(N, H, D).contiguous()
+    ref = ext.paged_attention_decode(queries, *ref_cache, pages, lens,
+                                     D ** -0.5).flatten(1)
+    for _ in range(2):
+        got = [c.clone() for c in cache]
+        out = ext.paged_decode_packed(parts if S else rows, b if S else None, pos, slots, inv, *got,
+                                      pages, lens, arrived, H, D ** -0.5, *nw)
+        assert _rel(out, ref) < (5e-3 if longest == 1 else 0.02)
+        for x, y in zip(got, ref_cache):
+            assert _rel(x, y) < 3 * 2.0 ** -9
+        assert not arrived.any()
+    slots[-1] = -1
     got = [c.clone() for c in cache]
-    q = ext.rope_scatter_join(parts, b, pos, slots, inv, *got, H, KV, D, *nw)
-    qkv = parts.sum(0) + (b.float() if bias else 0)
-    qkv = qkv.to(torch.bfloat16)
-    ext.rope_scatter_qkv(qkv, pos, slots, inv, *cache, H, KV, D, *nw)
-    assert _rel(q, qkv[:, :H * D]) < 3 * 2.0 ** -9
-    for x, y in zip(got, cache):
-        assert _rel(x, y) < 3 * 2.0 ** -9 and torch.equal(x[5], y[5])
+    ext.paged_decode_packed(parts if S else rows, b if S else None, pos, slots, inv, *got, pages,
+                            lens, arrived, H, D ** -0.5, *nw)
+    assert got[0].isnan().any(-1).sum() == KV
 
 
 @pytest.mark.parametrize("name,four_bit,lora_r", [("small-qwen2", False, 8), ("small-qwen2", True, 8),
