@@ -73,7 +73,11 @@ class LayerWeights:
     def _fill_rows(self, site: str) -> None:
         mods, out = self.mods[site], self._rows[site]
         if len(mods) == 1 and mods[0].r == 0:
-            self._rows[site] = mods[0].weight.detach().contiguous()
+            w = mods[0].weight.detach()
+            if out is None:
+                self._rows[site] = w.contiguous()
+            elif out.data_ptr() != w.data_ptr():    # replaced since
+                out.copy_(w)
             return
         if out is None:
             out = self._rows[site] = mods[0].weight.new_empty(
@@ -146,6 +150,13 @@ def _merge_tiles(mods, out: torch.Tensor, glu: bool, adapters: bool = True) -> N
         row += 16 if glu else m.out_features
 
 
+def _room_for(size: int, device) -> bool:
+    """Whether so many bytes can be allocated, a twentieth of the card left."""
+    free, total = torch.cuda.mem_get_info(device)
+    free += torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+    return size <= free - total // 20
+
+
 class FusedWeights:
     def __init__(self, model, use_nf4: bool = True):
         self.model = model
@@ -198,12 +209,17 @@ class FusedWeights:
             and q0.weight.is_cuda and shapes_ok
             and os.environ.get("DISTRL_HYBRID_DOWN", "1") == "1")
         self.lora_r = q0.r
-        # the decode products read weights in tiles
+        # the decode products read weights in tiles, where the tiles and the
+        # row-major weights that prompts and larger steps read fit beside the
+        # model (a 70B model without an adapter keeps row-major ones alone)
         self.tiled = bool(
             not self.nf4 and q0.weight.is_cuda
             and q0.weight.dtype == torch.bfloat16 and s.hidden_size % 64 == 0
             and s.q_size % 64 == 0 and s.kv_size % 32 == 0
-            and s.intermediate_size % 64 == 0)
+            and s.intermediate_size % 64 == 0
+            and _room_for(2 * s.num_layers * 2 * s.hidden_size * (
+                2 * s.q_size + 2 * s.kv_size + 3 * s.intermediate_size),
+                q0.weight.device))
         # the 4-bit kernel's packs of the down site: only steps beyond the
         # streamed products' rows use them
         self._nf4_down = False

@@ -186,3 +186,37 @@ def test_decode_step_matches_modules(name, four_bit, lora_r, n):
         for layer, want in zip(rows, ref):
             at = (layer[:, None, :] - want[0]).abs().sum(-1).argmin().item()
             assert _rel(layer[at:at + 8], want) < 0.03
+
+
+def test_replaced_weight_reaches_row_major_storage():
+    """A weight without an adapter that is another tensor at the next refresh:
+    the storage that captured steps hold follows it."""
+    from distrl_llm_amd.engine.weights import FusedWeights
+    from distrl_llm_amd.models import CausalLM, get_spec
+    model = CausalLM(get_spec("small-qwen2"), dtype=torch.bfloat16,
+                     device=torch.device("cuda")).random_init(3)
+    fused = FusedWeights(model)
+    fused.refresh()
+    at, lw = model.model.layers[0].self_attn, fused.layers[0]
+    held = lw.rows("o")
+    at.o_proj.weight.data = _rand(at.o_proj.weight.shape, 5)
+    fused.refresh()
+    assert lw.rows("o") is held and torch.equal(held, at.o_proj.weight)
+
+
+def test_no_tiles_without_room(monkeypatch):
+    """Where a second copy of the weights does not fit, steps run row-major."""
+    from distrl_llm_amd.config import EngineConfig, SamplingParams
+    from distrl_llm_amd.engine import Engine, weights
+    from distrl_llm_amd.models import CausalLM, get_spec
+    model = CausalLM(get_spec("small-qwen2"), dtype=torch.bfloat16,
+                     device=torch.device("cuda")).random_init(3).eval()
+    tokens = []
+    for room in (True, False):
+        monkeypatch.setattr(weights, "_room_for", lambda size, device: room)
+        eng = Engine(model, EngineConfig(max_seq_length=64, num_kv_blocks=96, max_num_seqs=64))
+        assert eng.fused.tiled == room
+        tokens.append([eng.generate([[5, 6, 7]], SamplingParams(max_tokens=2, temperature=0.0, n=n))
+                       for n in (3, 40)])
+        assert (eng.fused.layers[0].tiles is None) != room
+    assert len(tokens[0][1][0]) == len(tokens[1][1][0]) == 40
