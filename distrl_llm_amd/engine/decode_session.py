@@ -91,15 +91,21 @@ class DecodeSession:
         e = self.engine
         bs = e.pool.block_size
         pos = self.positions
-        blk = torch.div(pos, bs, rounding_mode="floor")
-        slot = (self.block_tables.gather(1, blk.unsqueeze(1)).squeeze(1).long()
-                * bs + pos % bs)
+        ext = None
+        if pos.is_cuda:
+            from ..ops.build import get_extension
+            ext = get_extension()
+        if ext is not None:
+            slot, pos = ext.decode_slots(pos, self.block_tables, bs)
+        else:
+            blk = torch.div(pos, bs, rounding_mode="floor")
+            slot = (self.block_tables.gather(1, blk.unsqueeze(1)).squeeze(1)
+                    .long() * bs + pos % bs)
         logits = e._decode_forward(self.tokens, pos, slot, self.block_tables,
                                    self.ctx_lens)
         if self.sp.temperature > 0.0:
             if logits.is_cuda:
-                from ..ops.build import get_extension
-                sampled = get_extension().sample_tokens(
+                sampled = ext.sample_tokens(
                     logits, float(self.sp.temperature),
                     float(self.sp.top_p), int(self.sp.top_k), self.seeds,
                     self.step_idx)
@@ -114,6 +120,11 @@ class DecodeSession:
                                            generator=e.generator)
         else:
             sampled = logits.argmax(-1)
+        if ext is not None:
+            ext.decode_advance(sampled, self.tokens, self.positions,
+                               self.ctx_lens, self.limit_pos, self.finished,
+                               self.step_idx, self.out_buf, self.eos)
+            return
         self.out_buf.index_copy_(0, self.step_idx, sampled.unsqueeze(0))
 
         was_finished = self.finished

@@ -71,6 +71,11 @@ std::vector<torch::Tensor> add_rmsnorm_join(torch::Tensor parts,
                                             torch::Tensor res, torch::Tensor w,
                                             double eps,
                                             c10::optional<torch::Tensor> bt);
+std::vector<torch::Tensor> decode_slots(torch::Tensor positions, torch::Tensor tables,
+                                        int64_t block_size);
+void decode_advance(torch::Tensor sampled, torch::Tensor tokens, torch::Tensor positions,
+                    torch::Tensor ctx_lens, torch::Tensor limits, torch::Tensor finished,
+                    torch::Tensor step, torch::Tensor out, c10::optional<int64_t> eos);
 torch::Tensor paged_decode_packed(
     torch::Tensor qkv, c10::optional<torch::Tensor> bias,
     torch::Tensor positions, torch::Tensor slots, torch::Tensor inv_freq,
@@ -187,6 +192,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual + partial sums (+ adapter), then RMSNorm", py::arg("parts"),
         py::arg("res"), py::arg("w"), py::arg("eps"),
         py::arg("bt") = py::none());
+  m.def("decode_slots", &decode_slots, "cache rows and int32 positions of a step");
+  m.def("decode_advance", &decode_advance, "a step's tokens into the session's state");
   m.def("paged_decode_packed", &paged_decode_packed,
         "packed [q|k|v] or its partial sums -> norms, RoPE, KV scatter, "
         "paged decode attention",

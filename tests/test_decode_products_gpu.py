@@ -220,3 +220,30 @@ def test_no_tiles_without_room(monkeypatch):
                        for n in (3, 40)])
         assert (eng.fused.layers[0].tiles is None) != room
     assert len(tokens[0][1][0]) == len(tokens[1][1][0]) == 40
+
+
+@pytest.mark.parametrize("N,bs,eos", [(1, 16, None), (8, 16, 3), (300, 24, 3)])
+def test_decode_state(ext, N, bs, eos):
+    """Three steps against the same in torch operations: sequences that end at
+    their limit, with eos, and long before."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+
+    def ints(hi, *shape):
+        return torch.randint(0, hi, shape, generator=g, device="cuda")
+
+    tables, pos = ints(1000, N, 9).int(), ints(8 * bs, N)
+    limits, fin = pos + ints(4, N), ints(3, N) == 0
+    state = [ints(5, N), pos.clone(), pos.int() + 1, limits, fin.clone(),
+             torch.zeros(1, dtype=torch.long, device="cuda"), torch.zeros(4, N, dtype=torch.long, device="cuda")]
+    tok, ctx, out = state[0].clone(), state[2].clone(), state[6].clone()
+    for step in range(3):
+        slots, pos32 = ext.decode_slots(state[1], tables, bs)
+        assert torch.equal(slots, tables.gather(1, (pos // bs)[:, None])[:, 0].long() * bs + pos % bs)
+        assert pos32.dtype == torch.int32 and torch.equal(pos32, pos.int())
+        new = ints(5, N)
+        ext.decode_advance(new, *state, eos)
+        out[step], go = new, ~fin
+        fin = fin | (pos + 1 >= limits) | ((new == eos) if eos is not None else False)
+        tok, pos, ctx = torch.where(go, new, tok), pos + go, ctx + go.int()
+        for a, b in zip(state, (tok, pos, ctx, limits, fin, torch.tensor([step + 1], device="cuda"), out)):
+            assert torch.equal(a, b)
