@@ -1,0 +1,324 @@
+// The two halves of a decoder layer in LoRA training, each forward and backward as
+// one call: attention and feed-forward with their norms, adapted projections and
+// residual sums. The autograd nodes around them are models/fused_layer.py.
+//
+// An adapter is more of its projection: u = scale * x A^T lies beside x in one
+// matrix, [x | u], and one product with [W | B] gives every projection of that
+// input, adapters and (beta = 1) the residual in its fp32 sums; backward is
+// [dY | du] [W; A].
+//
+// Native because short micro-batches wait for the host: the same launches from
+// Python took 25.0 ms a pass of the 0.5B model over three short samples, of which
+// the GPU worked 11.
+#include <torch/extension.h>
+
+using at::Tensor;
+using Tensors = std::vector<Tensor>;
+using Ints = std::vector<int64_t>;
+using Optional = c10::optional<Tensor>;
+
+Tensor rmsnorm_fwd(Tensor x, Tensor w, double eps);
+Tensor rmsnorm_bwd(Tensor dy, Tensor x, Tensor w, double eps);
+Tensor rmsnorm_bwd_add(Tensor dy, Tensor x, Tensor w, Tensor g, double eps);
+void rmsnorm_fwd_into(Tensor x, Tensor w, double eps, Tensor out);
+void rope_rows(Tensor q, Tensor k, Tensor positions, Tensor inv_freq);
+Tensors flash_varlen_fwd(Tensor q, Tensor k, Tensor v, Tensor cu, int64_t max_len, double scale,
+                         Optional into);
+void flash_varlen_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, Tensor cu,
+                      int64_t max_len, double scale, Tensor dq, Tensor dk, Tensor dv);
+Tensors adapter_grads(Tensors y, Tensors p, Ints by_col);
+Tensor adapted_weight(Tensors w, Tensors b, int64_t pad);
+Tensor stack_transposed(Tensors w, Ints at, int64_t cols);
+void silu_mul_packed_into(Tensor gu, Tensor out);
+void silu_mul_bwd_packed(Tensor dy, Tensor gu, Tensor dgate, Tensor dup);
+
+namespace {
+
+// every operand is bf16 already
+struct NoAutocast {
+  c10::impl::ExcludeDispatchKeyGuard guard{c10::DispatchKey::AutocastCUDA};
+};
+
+Tensor columns(const Tensor& t, int64_t from, int64_t n) { return t.narrow(1, from, n); }
+
+Tensor heads(const Tensor& t, int64_t head_dim) {
+  return t.view({t.size(0), t.size(1) / head_dim, head_dim});
+}
+
+// out <- scale * a b, the scale in the product's epilogue
+void scaled_mm(const Tensor& a, const Tensor& b, double scale, Tensor out) {
+  at::addmm_out(out, out, a, b, 0., scale);
+}
+
+// Adapters of projections that share an input, or of one: A (r, K), B (N, r).
+struct Adapters {
+  Tensors A, B;
+  std::vector<double> scales;
+  Ints ranks, at;           // at: first column of each among the inputs u
+  int64_t sum = 0, pad;     // pad: the columns they get beside their input
+
+  Adapters(Tensors a, Tensors b, std::vector<double> s)
+      : A(std::move(a)), B(std::move(b)), scales(std::move(s)) {
+    TORCH_CHECK(!A.empty() && A.size() == B.size() && A.size() == scales.size());
+    for (const auto& t : A) {
+      at.push_back(sum);
+      ranks.push_back(t.size(0));
+      sum += t.size(0);
+    }
+    pad = (sum + 7) / 8 * 8;
+  }
+
+  Tensor part(const Tensor& u, size_t i) const { return columns(u, at[i], ranks[i]); }
+
+  void clear_spare(const Tensor& u) const {
+    if (pad > sum) columns(u, sum, pad - sum).zero_();
+  }
+
+  // u <- the adapters' scaled inputs side by side, zeros in spare columns
+  void down(const Tensor& x, const Tensor& u) const {
+    bool same = true;
+    for (double s : scales) same = same && s == scales[0];
+    if (same) {
+      scaled_mm(x, (A.size() > 1 ? at::cat(A) : A[0]).t(), scales[0], columns(u, 0, sum));
+    } else {
+      for (size_t i = 0; i < A.size(); ++i) scaled_mm(x, A[i].t(), scales[i], part(u, i));
+    }
+    clear_spare(u);
+  }
+
+  // du <- the gradients of the adapters' inputs
+  void up(const Tensors& dy, const Tensor& du) const {
+    for (size_t i = 0; i < B.size(); ++i) scaled_mm(dy[i], B[i], scales[i], part(du, i));
+    clear_spare(du);
+  }
+};
+
+// xu W^T + the projections' biases
+Tensor product(const Tensor& xu, const Tensor& W, const std::vector<Optional>& bias,
+               const Ints& sizes) {
+  bool any = false;
+  for (const auto& b : bias) any = any || b;
+  if (!any) return at::mm(xu, W.t());
+  Tensors all;
+  for (size_t i = 0; i < bias.size(); ++i)
+    all.push_back(bias[i] ? *bias[i] : at::zeros({sizes[i]}, xu.options()));
+  return at::addmm(at::cat(all), xu, W.t());
+}
+
+struct Through { Tensor dx, g, du; };
+
+// g W + du A with du = scale * g B, from one product of [g | du]; g and du as parts
+// of that matrix
+Through through(const Tensor& g, const Tensor& W, const Adapters& ad) {
+  const int64_t N = g.size(1);
+  auto gd = at::empty({g.size(0), N + ad.pad}, g.options());
+  auto g2 = columns(gd, 0, N), du = columns(gd, N, ad.pad);
+  g2.copy_(g);
+  ad.up({g}, du);
+  return {at::mm(gd, stack_transposed({W, ad.A[0]}, {0, N}, N + ad.pad).t()), g2, ad.part(du, 0)};
+}
+
+struct Job { Tensor y, p; bool by_col; };
+
+// p^T y of every job over the rows: gradients of A, or of B (by_col, transposed).
+// Ranks that the kernel does not take go through the library.
+Tensors sums(const std::vector<Job>& jobs) {
+  Tensors out(jobs.size()), y, p;
+  Ints by_col, own;
+  for (size_t i = 0; i < jobs.size(); ++i) {
+    const auto& j = jobs[i];
+    const int64_t r = j.p.size(1);
+    if (r % 8 == 0 && r >= 8 && r <= 128 && j.y.size(1) % 8 == 0 && j.p.size(0) > 0) {
+      own.push_back(i);
+      y.push_back(j.y);
+      p.push_back(j.p);
+      by_col.push_back(j.by_col);
+    } else {
+      out[i] = j.by_col ? at::mm(j.y.t(), j.p) : at::mm(j.p.t(), j.y);
+    }
+  }
+  if (!own.empty()) {
+    auto got = adapter_grads(y, p, by_col);
+    for (size_t i = 0; i < own.size(); ++i) out[own[i]] = got[i];
+  }
+  return out;
+}
+
+// gradients of the adapters in the order of their parameters: A, B of each
+Tensors in_order(const Adapters& ad, const Tensor& dA, const Tensor* dB) {
+  Tensors out;
+  for (size_t i = 0; i < ad.A.size(); ++i) {
+    out.push_back(dA.narrow(0, ad.at[i], ad.ranks[i]));
+    out.push_back(dB[i]);
+  }
+  return out;
+}
+
+}  // namespace
+
+// y = x + o_proj(attention(qkv_proj(norm(x)))) over rows x of sequences that begin
+// at cu. W, A, B, scales: q, k, v, o. Returns y and what backward needs:
+// [x | u] of the projections, [attention | u] of o, q, k, v, lse and, with head
+// norms, q and k before them.
+Tensors attention_half_fwd(Tensor x, Tensor norm, double eps, Tensors W,
+                           std::vector<Optional> bias, Tensors A, Tensors B,
+                           std::vector<double> scales, Optional q_norm, Optional k_norm,
+                           double q_eps, double k_eps, Tensor pos, Tensor inv_freq, Tensor cu,
+                           int64_t longest, double scale, int64_t head_dim) {
+  NoAutocast plain;
+  TORCH_CHECK(W.size() == 4 && A.size() == 4 && B.size() == 4 && scales.size() == 4 &&
+              bias.size() == 3 && q_norm.has_value() == k_norm.has_value());
+  const int64_t rows = x.size(0), hidden = x.size(1);
+  const Adapters in({A[0], A[1], A[2]}, {B[0], B[1], B[2]}, {scales[0], scales[1], scales[2]});
+  const Adapters o_ad({A[3]}, {B[3]}, {scales[3]});
+  const Ints sizes = {W[0].size(0), W[1].size(0), W[2].size(0)};
+
+  auto hu = at::empty({rows, hidden + in.pad}, x.options());
+  auto h = columns(hu, 0, hidden);
+  rmsnorm_fwd_into(x, norm, eps, h);
+  in.down(h, columns(hu, hidden, in.pad));
+  auto qkv = product(hu, adapted_weight({W[0], W[1], W[2]}, in.B, in.pad), bias, sizes);
+  auto q = heads(columns(qkv, 0, sizes[0]), head_dim);
+  auto k = heads(columns(qkv, sizes[0], sizes[1]), head_dim);
+  auto v = heads(columns(qkv, sizes[0] + sizes[1], sizes[2]), head_dim);
+  Tensor q0, k0;
+  if (q_norm) {
+    q0 = q.contiguous();
+    k0 = k.contiguous();
+    q = rmsnorm_fwd(q0, *q_norm, q_eps);
+    k = rmsnorm_fwd(k0, *k_norm, k_eps);
+  }
+  rope_rows(q, k, pos, inv_freq);
+  auto ou = at::empty({rows, sizes[0] + o_ad.pad}, x.options());
+  auto o = columns(ou, 0, sizes[0]);
+  auto lse = flash_varlen_fwd(q, k, v, cu, longest, scale, heads(o, head_dim))[1];
+  o_ad.down(o, columns(ou, sizes[0], o_ad.pad));
+  // the residual joins the product's sum: one rounding for all of it
+  auto y = at::addmm(x, ou, adapted_weight({W[3]}, o_ad.B, o_ad.pad).t());
+  return {y, hu, ou, q, k, v, lse, q0, k0};
+}
+
+// dx (undefined unless wanted), then the gradients of A and B of q, k, v, o.
+Tensors attention_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tensors W, Tensors A,
+                           Tensors B, std::vector<double> scales, Optional q_norm,
+                           Optional k_norm, double q_eps, double k_eps, Tensor pos,
+                           Tensor back_freq, Tensor cu, int64_t longest, double scale, Tensor hu,
+                           Tensor ou, Tensor q, Tensor k, Tensor v, Tensor lse, Optional q0,
+                           Optional k0, bool want_dx) {
+  NoAutocast plain;
+  const int64_t rows = x.size(0), hidden = x.size(1), head_dim = q.size(2);
+  const Adapters in({A[0], A[1], A[2]}, {B[0], B[1], B[2]}, {scales[0], scales[1], scales[2]});
+  const Adapters o_ad({A[3]}, {B[3]}, {scales[3]});
+  const Ints sizes = {W[0].size(0), W[1].size(0), W[2].size(0)};
+  const int64_t width = sizes[0] + sizes[1] + sizes[2];
+  g = g.contiguous();
+  auto h = columns(hu, 0, hidden), u = columns(hu, hidden, in.pad);
+  auto o = columns(ou, 0, sizes[0]), uo = columns(ou, sizes[0], o_ad.ranks[0]);
+
+  const auto [dO, g2, duo] = through(g, W[3], o_ad);
+  auto dyu = at::empty({rows, width + in.pad}, x.options());
+  const Tensors dys = {columns(dyu, 0, sizes[0]), columns(dyu, sizes[0], sizes[1]),
+                       columns(dyu, sizes[0] + sizes[1], sizes[2])};
+  auto du = columns(dyu, width, in.pad);
+  auto dq = heads(dys[0], head_dim), dk = heads(dys[1], head_dim), dv = heads(dys[2], head_dim);
+  flash_varlen_bwd(heads(dO, head_dim), q, k, v, heads(o, head_dim), lse, cu, longest, scale, dq,
+                   dk, dv);
+  // a rotation's gradient is the rotation by the negative angle
+  rope_rows(dq, dk, pos, back_freq);
+  if (q0) {
+    dq.copy_(rmsnorm_bwd(dq.contiguous(), *q0, *q_norm, q_eps));
+    dk.copy_(rmsnorm_bwd(dk.contiguous(), *k0, *k_norm, k_eps));
+  }
+  in.up(dys, du);
+  auto s = sums({{h, du, false},
+                 {o, duo, false},
+                 {g2, uo, true},
+                 {dys[0], in.part(u, 0), true},
+                 {dys[1], in.part(u, 1), true},
+                 {dys[2], in.part(u, 2), true}});
+  Tensors out = in_order(in, s[0], &s[3]);
+  out.push_back(s[1]);
+  out.push_back(s[2]);
+  Tensor dx;
+  if (want_dx) {
+    const auto WA = stack_transposed({W[0], W[1], W[2], A[0], A[1], A[2]},
+                                     {0, sizes[0], sizes[0] + sizes[1], width, width + in.at[1],
+                                      width + in.at[2]}, width + in.pad);
+    dx = rmsnorm_bwd_add(at::mm(dyu, WA.t()), x, norm, g, eps);
+  }
+  out.insert(out.begin(), dx);
+  return out;
+}
+
+// y = x + down_proj(silu(gate_proj(norm(x))) * up_proj(norm(x))) over rows x. W, A,
+// B, scales: gate, up, down. Returns y, [x | u], [gate | up], [act | u].
+Tensors feed_forward_half_fwd(Tensor x, Tensor norm, double eps, Tensors W,
+                              std::vector<Optional> bias, Tensors A, Tensors B,
+                              std::vector<double> scales) {
+  NoAutocast plain;
+  TORCH_CHECK(W.size() == 3 && A.size() == 3 && B.size() == 3 && scales.size() == 3 &&
+              bias.size() == 2);
+  const int64_t rows = x.size(0), hidden = x.size(1), inner = W[0].size(0);
+  const Adapters in({A[0], A[1]}, {B[0], B[1]}, {scales[0], scales[1]});
+  const Adapters d_ad({A[2]}, {B[2]}, {scales[2]});
+  auto hu = at::empty({rows, hidden + in.pad}, x.options());
+  auto h = columns(hu, 0, hidden);
+  rmsnorm_fwd_into(x, norm, eps, h);
+  in.down(h, columns(hu, hidden, in.pad));
+  auto gu = product(hu, adapted_weight({W[0], W[1]}, in.B, in.pad), bias, {inner, inner});
+  auto au = at::empty({rows, inner + d_ad.pad}, x.options());
+  auto act = columns(au, 0, inner);
+  silu_mul_packed_into(gu, act);
+  d_ad.down(act, columns(au, inner, d_ad.pad));
+  auto y = at::addmm(x, au, adapted_weight({W[2]}, d_ad.B, d_ad.pad).t());
+  return {y, hu, gu, au};
+}
+
+// dx (undefined unless wanted), then the gradients of A and B of gate, up, down.
+Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tensors W, Tensors A,
+                              Tensors B, std::vector<double> scales, Tensor hu, Tensor gu,
+                              Tensor au, bool want_dx) {
+  NoAutocast plain;
+  const int64_t rows = x.size(0), hidden = x.size(1), inner = W[0].size(0);
+  const Adapters in({A[0], A[1]}, {B[0], B[1]}, {scales[0], scales[1]});
+  const Adapters d_ad({A[2]}, {B[2]}, {scales[2]});
+  g = g.contiguous();
+  auto h = columns(hu, 0, hidden), u = columns(hu, hidden, in.pad);
+  auto act = columns(au, 0, inner), ud = columns(au, inner, d_ad.ranks[0]);
+
+  const auto [dact, g2, dud] = through(g, W[2], d_ad);
+  // [dgate | du | dup]
+  auto dyu = at::empty({rows, 2 * inner + in.pad}, x.options());
+  auto dgate = columns(dyu, 0, inner), du = columns(dyu, inner, in.pad),
+       dup = columns(dyu, inner + in.pad, inner);
+  silu_mul_bwd_packed(dact, gu, dgate, dup);
+  in.up({dgate, dup}, du);
+  auto s = sums({{h, du, false},
+                 {act, dud, false},
+                 {g2, ud, true},
+                 {dgate, in.part(u, 0), true},
+                 {dup, in.part(u, 1), true}});
+  Tensors out = in_order(in, s[0], &s[3]);
+  out.push_back(s[1]);
+  out.push_back(s[2]);
+  Tensor dx;
+  if (want_dx) {
+    const auto WA = stack_transposed({W[0], A[0], A[1], W[1]},
+                                     {0, inner, inner + in.ranks[0], inner + in.pad},
+                                     2 * inner + in.pad);
+    const int64_t half = inner + in.ranks[0], rest = inner + in.pad - in.ranks[0];
+    Tensor dh;
+    if (rows >= 8192 && hidden <= 2048 && half % 8 == 0) {
+      // few columns from many rows: the library's product of twice the K takes up
+      // to three times as long (18793 x 17984 x 1536: 1080 us, in two 790; from 4000
+      // rows or for 2560 columns one is the faster)
+      dh = at::mm(columns(dyu, 0, half), columns(WA, 0, half).t());
+      dh.addmm_(columns(dyu, half, rest), columns(WA, half, rest).t());
+    } else {
+      dh = at::mm(dyu, WA.t());
+    }
+    dx = rmsnorm_bwd_add(dh, x, norm, g, eps);
+  }
+  out.insert(out.begin(), dx);
+  return out;
+}

@@ -120,6 +120,34 @@ void rmsnorm_fwd_into(torch::Tensor x, torch::Tensor w, double eps,
 void silu_mul_packed_into(torch::Tensor gu, torch::Tensor out);
 void silu_mul_bwd_packed(torch::Tensor dy, torch::Tensor gu,
                          torch::Tensor dgate, torch::Tensor dup);
+std::vector<torch::Tensor> attention_half_fwd(
+    torch::Tensor x, torch::Tensor norm, double eps,
+    std::vector<torch::Tensor> W, std::vector<c10::optional<torch::Tensor>> bias,
+    std::vector<torch::Tensor> A, std::vector<torch::Tensor> B,
+    std::vector<double> scales, c10::optional<torch::Tensor> q_norm,
+    c10::optional<torch::Tensor> k_norm, double q_eps, double k_eps,
+    torch::Tensor pos, torch::Tensor inv_freq, torch::Tensor cu,
+    int64_t longest, double scale, int64_t head_dim);
+std::vector<torch::Tensor> attention_half_bwd(
+    torch::Tensor g, torch::Tensor x, torch::Tensor norm, double eps,
+    std::vector<torch::Tensor> W, std::vector<torch::Tensor> A,
+    std::vector<torch::Tensor> B, std::vector<double> scales,
+    c10::optional<torch::Tensor> q_norm, c10::optional<torch::Tensor> k_norm,
+    double q_eps, double k_eps, torch::Tensor pos, torch::Tensor back_freq,
+    torch::Tensor cu, int64_t longest, double scale, torch::Tensor hu,
+    torch::Tensor ou, torch::Tensor q, torch::Tensor k, torch::Tensor v,
+    torch::Tensor lse, c10::optional<torch::Tensor> q0,
+    c10::optional<torch::Tensor> k0, bool want_dx);
+std::vector<torch::Tensor> feed_forward_half_fwd(
+    torch::Tensor x, torch::Tensor norm, double eps,
+    std::vector<torch::Tensor> W, std::vector<c10::optional<torch::Tensor>> bias,
+    std::vector<torch::Tensor> A, std::vector<torch::Tensor> B,
+    std::vector<double> scales);
+std::vector<torch::Tensor> feed_forward_half_bwd(
+    torch::Tensor g, torch::Tensor x, torch::Tensor norm, double eps,
+    std::vector<torch::Tensor> W, std::vector<torch::Tensor> A,
+    std::vector<torch::Tensor> B, std::vector<double> scales, torch::Tensor hu,
+    torch::Tensor gu, torch::Tensor au, bool want_dx);
 std::vector<torch::Tensor> flash_attn_bwd(torch::Tensor dout, torch::Tensor q,
                                           torch::Tensor k, torch::Tensor v,
                                           torch::Tensor o, torch::Tensor lse,
@@ -192,6 +220,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual + partial sums (+ adapter), then RMSNorm", py::arg("parts"),
         py::arg("res"), py::arg("w"), py::arg("eps"),
         py::arg("bt") = py::none());
+  m.def("attention_half_fwd", &attention_half_fwd,
+        "an adapted layer's attention half");
+  m.def("attention_half_bwd", &attention_half_bwd);
+  m.def("feed_forward_half_fwd", &feed_forward_half_fwd,
+        "an adapted layer's feed-forward half");
+  m.def("feed_forward_half_bwd", &feed_forward_half_bwd);
   m.def("decode_slots", &decode_slots, "cache rows and int32 positions of a step");
   m.def("decode_advance", &decode_advance, "a step's tokens into the session's state");
   m.def("paged_decode_packed", &paged_decode_packed,
