@@ -120,6 +120,8 @@ void rmsnorm_fwd_into(torch::Tensor x, torch::Tensor w, double eps,
 void silu_mul_packed_into(torch::Tensor gu, torch::Tensor out);
 void silu_mul_bwd_packed(torch::Tensor dy, torch::Tensor gu,
                          torch::Tensor dgate, torch::Tensor dup);
+bool adapter_input(torch::Tensor x, std::vector<torch::Tensor> m,
+                   std::vector<double> scales, torch::Tensor out, bool k_major);
 std::vector<torch::Tensor> attention_half_fwd(
     torch::Tensor x, torch::Tensor norm, double eps,
     std::vector<torch::Tensor> W, std::vector<c10::optional<torch::Tensor>> bias,
@@ -220,6 +222,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual + partial sums (+ adapter), then RMSNorm", py::arg("parts"),
         py::arg("res"), py::arg("w"), py::arg("eps"),
         py::arg("bt") = py::none());
+  m.def("adapter_input", &adapter_input, "scaled inputs of LoRA adapters");
   m.def("attention_half_fwd", &attention_half_fwd,
         "an adapted layer's attention half");
   m.def("attention_half_bwd", &attention_half_bwd);

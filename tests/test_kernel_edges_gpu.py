@@ -825,6 +825,41 @@ def test_adapter_grads(ext, rows, shapes):
     assert all((t == 0).all() for t in ext.adapter_grads([ys[0][:0]], [ps[0][:0]], [0]))
 
 
+@pytest.mark.parametrize("rows", [1, 31, 33, 700, 17000])
+@pytest.mark.parametrize("K,ranks,pad", [(8, (8,), 8), (136, (32, 32, 32), 96), (896, (8, 24), 40),
+                                         (1000, (64,), 64), (264, (40, 48, 40), 128),
+                                         (4864, (32,), 32)])
+def test_adapter_input(ext, rows, K, ranks, pad):
+    """Ends of the row, K and column tiles, adapters side by side with a scale
+    each, zeros in spare columns, cut out of wider rows, both layouts of the
+    adapter. Bound: fp32 sums, one rounding."""
+    if rows * K > 2e7:
+        K = 392
+    x = _rand((rows, K + 8), 1)[:, 8:]
+    ms, scales = [_rand((r, K), 2 + i) for i, r in enumerate(ranks)], [0.5 + i for i in range(len(ranks))]
+    wide = torch.full((rows, pad + 16), 7.0, dtype=torch.bfloat16, device="cuda")
+    out = wide[:, 8:8 + pad]
+    ref = x.double() @ torch.cat([m.double() * s for m, s in zip(ms, scales)]).t()
+    assert ext.adapter_input(x, ms, scales, out, False)
+    assert _rel(out[:, :sum(ranks)], ref) < 2.0 ** -8
+    assert (out[:, sum(ranks):] == 0).all() and (wide[:, :8] == 7).all() and (wide[:, 8 + pad:] == 7).all()
+    out.fill_(7.0)
+    assert ext.adapter_input(x, [torch.cat(ms).t().contiguous()], [2.0], out, True)
+    assert _rel(out[:, :sum(ranks)], x.double() @ torch.cat(ms).double().t() * 2) < 2.0 ** -8
+    assert (out[:, sum(ranks):] == 0).all() and (wide[:, :8] == 7).all() and (wide[:, 8 + pad:] == 7).all()
+
+
+def test_adapter_input_refuses(ext):
+    """What 16 B accesses or the tiles can't take is left to the caller."""
+    x, m, out = _rand((5, 64), 1), _rand((8, 64), 2), _rand((5, 8), 3)
+    assert ext.adapter_input(x, [m], [1.0], out, False)
+    assert not ext.adapter_input(x[:, 1:57], [m[:, :56].contiguous()], [1.0], out, False)
+    assert not ext.adapter_input(x, [m[:5].contiguous()], [1.0], out, False)
+    assert not ext.adapter_input(x, [m], [1.0], out[:1].expand(5, 8), False)
+    assert not ext.adapter_input(x, [_rand((136, 64), 4)], [1.0], _rand((5, 136), 5), False)
+    assert not ext.adapter_input(x.float(), [m], [1.0], out, False)
+
+
 @pytest.mark.parametrize("N,K,ranks,pad", [((16, 8, 24), 64, (8, 8, 8), 24), ((40, 24), 136, (5, 12), 24),
                                            ((64,), 8, (32,), 32)])
 def test_adapted_weight(ext, N, K, ranks, pad):
