@@ -35,11 +35,13 @@
 // split over workgroups that leave fp32 partials for a small sum kernel.
 //
 // Measured at B 16, 28/4 heads, T 1550, D 128 (275 GFLOP in the causal half,
-// forward): forward 440 us = 625 TFLOP/s, dQ 597 us, dK/dV 1208 us + 39 us for
-// the sum; 16-row waves on 16x16x32 with single-buffered tiles and transposed
-// copies of q, k, v, dout took 1161, 2097 and 3466 us + 1.9 ms of copies and
-// sums. What bounds them now: vector work beside the products (10 vector
-// instructions a product in the forward) at two waves a SIMD.
+// forward): forward 390 us = 705 TFLOP/s, backward 1177 us. It was 440 and 1845 with
+// waits for the next tile's loads inside the dK/dV step (a row statistic used
+// behind a branch, fragments spilled or not waited for before the loop, 64-bit
+// addresses in registers) and pairs of heads one after the other; 16-row waves on
+// 16x16x32 with single-buffered tiles and transposed copies of q, k, v, dout took
+// 1161 and 5563 us + 1.9 ms of copies and sums. What bounds them now: LDS reads and
+// vector work beside the products at two waves a SIMD.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
@@ -142,6 +144,25 @@ struct Tile {
   }
 };
 
+// A tile whose loads take one 32-bit offset a lane: rows past the end read as zero.
+template <int D, int ROWS, int NT>
+struct Rows : Tile<D, ROWS, NT> {
+  using T = Tile<D, ROWS, NT>;
+  int off;          // bytes, of this lane's first 16
+
+  DEV_INLINE explicit Rows(int stride_t)
+      : off(((int)threadIdx.x / T::UN * stride_t + (int)threadIdx.x % T::UN * 8) * 2) {}
+
+  DEV_INLINE void fetch(const __hip_bfloat16* base, int stride_t, int valid) {
+    // stride_t < 2^24: 64 rows stay within 2^31 bytes
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<__hip_bfloat16*>(base), 0, ((min(valid, ROWS) - 1) * stride_t + D) * 2, 0x00027000);
+    #pragma unroll
+    for (int i = 0; i < T::PER; ++i)
+      this->r[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + i * T::STEP * stride_t * 2, 0, 0);
+  }
+};
+
 // Lane offsets of the two kinds of fragment of a tile.
 template <int D>
 struct Frags {
@@ -201,6 +222,18 @@ DEV_INLINE void load_row(bf16v8 (&f)[D / 16], const __hip_bfloat16* base, int st
     f[ks] = *reinterpret_cast<const bf16v8*>(base + (int64_t)row * stride_t + ks * 16 + h * 8);
 }
 
+// Waits for fragments here: left to their first use, in a loop, the wait would be
+// for the loop's own loads as well, in every step.
+template <int D>
+DEV_INLINE void arrived(bf16v8 (&f)[D / 16]) {
+  #pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) {
+    u32x4 x = __builtin_bit_cast(u32x4, f[ks]);
+    asm volatile("" : "+v"(x));
+    f[ks] = __builtin_bit_cast(bf16v8, x);
+  }
+}
+
 // acc[dt] holds X^T (rows d, column = this lane's row): write the row times f.
 // Two half-waves hold alternating groups of four d; one swap makes 16 B runs.
 template <int D>
@@ -237,11 +270,24 @@ DEV_INLINE void store_rows_f32(const f32x16 (&acc)[D / 32], float* row, bool val
           f32x4{acc[dt][4 * g], acc[dt][4 * g + 1], acc[dt][4 * g + 2], acc[dt][4 * g + 3]};
 }
 
-// Workgroups go to the 8 XCDs in turn; give each XCD one contiguous share of
-// the work so that the heads and row blocks of a kv head meet in one L2.
-DEV_INLINE int xcd_share(int id, int total) {
-  const int x = id & 7, i = id >> 3, q = total >> 3, r = total & 7;
-  return x * q + min(x, r) + i;
+// What workgroup id works on: a kv head of a sequence (pair), a block of its rows
+// (longest first) and a query head or share of them.
+struct Place { int pair, block, part; };
+
+// Longest blocks first over all pairs, so that short ones fill the end. Workgroups
+// go to the 8 XCDs in turn; where they divide, each XCD gets pairs of its own, whose
+// heads and row blocks meet in one L2. (Pair by pair, every pair's longest block
+// first, the last pair's ended late: backward at (16, 28/4, 1550, 128) 1339 us for
+// 1230, (8, 64/8, 1024, 128) 733 for 636.)
+DEV_INLINE Place place(int id, int pairs, int blocks, int parts) {
+  int x = 0, n = pairs * parts;
+  if (pairs % 8 == 0) {
+    x = id & 7;
+    id >>= 3;
+    n >>= 3;
+  }
+  const int r = id % n;
+  return {(x * n + r) / parts, id / n, r % parts};
 }
 
 // ---------------------------------------------------------------- forward
@@ -253,12 +299,8 @@ void flash_fwd_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16
                       Strides so, int Hq, int Hkv, int nq, float scale_log2) {
   constexpr int KV = tile_rows<NW>(), NS = KV / 32, NT = NW * 64;
   const int group = Hq / Hkv;
-  int id = xcd_share(blockIdx.x, gridDim.x);
-  const int hg = id % group;
-  id /= group;
-  const int qb = nq - 1 - id % nq;      // longest rows first
-  id /= nq;
-  const int kvh = id % Hkv, b = id / Hkv;
+  const Place at = place(blockIdx.x, gridDim.x / (nq * group), nq, group);
+  const int qb = nq - 1 - at.block, hg = at.part, kvh = at.pair % Hkv, b = at.pair / Hkv;
   const int h = kvh * group + hg;
   const int row0 = seqs.first(b), len = seqs.len(b);
   if (qb * (NW * WROWS) >= len) return;
@@ -283,7 +325,7 @@ void flash_fwd_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16
 
   const int last = min((qb + 1) * (NW * WROWS), len);   // keys of this workgroup
   const int n = (last + KV - 1) / KV;
-  Tile<D, KV, NT> tk, tv;
+  Rows<D, KV, NT> tk(sk.t), tv(sv.t);
   tk.fetch(kp, sk.t, len);
   tv.fetch(vp, sv.t, len);
   tk.store(smem);
@@ -375,12 +417,8 @@ void flash_bwd_dq_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloa
                          int Hq, int Hkv, int nq, float scale) {
   constexpr int KV = tile_rows<NW>(), NS = KV / 32, NT = NW * 64;
   const int group = Hq / Hkv;
-  int id = xcd_share(blockIdx.x, gridDim.x);
-  const int hg = id % group;
-  id /= group;
-  const int qb = nq - 1 - id % nq;
-  id /= nq;
-  const int kvh = id % Hkv, b = id / Hkv;
+  const Place pl = place(blockIdx.x, gridDim.x / (nq * group), nq, group);
+  const int qb = nq - 1 - pl.block, hg = pl.part, kvh = pl.pair % Hkv, b = pl.pair / Hkv;
   const int h = kvh * group + hg;
   const int row0 = seqs.first(b), T = seqs.len(b);
   if (qb * (NW * WROWS) >= T) return;
@@ -420,7 +458,7 @@ void flash_bwd_dq_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloa
 
   const int last = min((qb + 1) * (NW * WROWS), T);
   const int n = (last + KV - 1) / KV;
-  Tile<D, KV, NT> tk, tv;
+  Rows<D, KV, NT> tk(sk.t), tv(sv.t);
   tk.fetch(kp, sk.t, T);
   tv.fetch(vp, sv.t, T);
   tk.store(smem);
@@ -440,10 +478,13 @@ void flash_bwd_dq_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloa
       const int c0 = kv0 + s * 32;
       if (c0 > q0 + WROWS - 1 || q0 >= T) continue;     // wave-uniform
       f32x16 st = zero16(), dp = zero16();
+      __builtin_amdgcn_s_setprio(1);
       #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) st = mfma(fr.row(ks_, s, ks), qf[ks], st);
-      #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) dp = mfma(fr.row(vs_, s, ks), dof[ks], dp);
+      for (int ks = 0; ks < D / 16; ++ks) {
+        st = mfma(fr.row(ks_, s, ks), qf[ks], st);
+        dp = mfma(fr.row(vs_, s, ks), dof[ks], dp);
+      }
+      __builtin_amdgcn_s_setprio(0);
       #pragma unroll
       for (int r = 0; r < 16; ++r)
         st[r] = __builtin_amdgcn_exp2f(st[r] * scale_log2 - lse2) * (dp[r] - dl);
@@ -474,7 +515,8 @@ void flash_bwd_dq_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloa
 // hs*part .. of its group. Partials (split > 1) go to fp32 (split, B, Hkv, T, D),
 // part_rows rows a share.
 template <int D, int NW>
-__global__ __launch_bounds__(NW * 64, 2)
+__global__ // two waves' tiles take twice the registers to fetch: 23 would spill
+__launch_bounds__(NW * 64, NW == 2 && D == 128 ? 1 : 2)
 void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bfloat16* __restrict__ k,
                           const __hip_bfloat16* __restrict__ v,
                           const __hip_bfloat16* __restrict__ dout, const float* __restrict__ lse,
@@ -485,12 +527,8 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
                           int64_t part_rows, float scale) {
   constexpr int QT = 32, NT = NW * 64;
   const int group = Hq / Hkv;
-  int id = xcd_share(blockIdx.x, gridDim.x);
-  const int hs = id % split;
-  id /= split;
-  const int kb = id % nkv;              // longest columns first
-  id /= nkv;
-  const int kvh = id % Hkv, b = id / Hkv;
+  const Place pl = place(blockIdx.x, gridDim.x / (nkv * split), nkv, split);
+  const int kb = pl.block, hs = pl.part, kvh = pl.pair % Hkv, b = pl.pair / Hkv;
   const int row0 = seqs.first(b), T = seqs.len(b);
   if (kb * (NW * WROWS) >= T) return;
   const int h0 = hs * group / split, h1 = (hs + 1) * group / split;
@@ -503,7 +541,7 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int TB = QT * D * 2, SB = 2 * TB + QT * 8;  // Q, dO, lse, delta
   constexpr int KB = NW * WROWS * D * 2;
-  const Frags<D> fr;
+  const Frags<D> lane;
   // V rows stay in registers, K rows in LDS: both in registers would leave
   // 256 too few for the accumulators, one wave a SIMD, and copies to the
   // accumulation registers around every product
@@ -522,19 +560,20 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
   for (int dt = 0; dt < D / 32; ++dt) { ak[dt] = zero16(); av[dt] = zero16(); }
 
   const int first = kb * (NW * WROWS), n = (T - first + QT - 1) / QT * (h1 - h0);
-  Tile<D, QT, NT> tq, td;
-  float stat = 0.f;     // threads 0..31: lse, 32..63: delta of the tile's rows
+  Rows<D, QT, NT> tq(sq.t), td(sdo.t);
+  // threads 0..31: lse, 32..63: delta of the tile's rows. Loaded by every wave and
+  // only looked at when it is stored: a use behind a branch made the loop wait for
+  // all of the next tile's loads here, a third of its time.
+  float stat = 0.f;
+  bool stat_live = false;
+  const float* sp = ((threadIdx.x & 32) == 0 ? lse : delta) + b * seqs.b + row0;
   int fh = kvh * group + h0, fr0 = first;              // the next tile to fetch
   auto fetch = [&] {
     tq.fetch(q + b * sq.b + fh * sq.h + (int64_t)(row0 + fr0) * sq.t, sq.t, T - fr0);
     td.fetch(dout + b * sdo.b + fh * sdo.h + (int64_t)(row0 + fr0) * sdo.t, sdo.t, T - fr0);
-    if (threadIdx.x < 64) {
-      const int r = fr0 + (threadIdx.x & 31);
-      const float* p = (threadIdx.x < 32 ? lse : delta) + b * seqs.b + fh * seqs.h + row0;
-      stat = p[min(r, T - 1)];
-      // rows past the end get weight exp(-huge) = 0
-      if (threadIdx.x < 32) stat = r < T ? stat * LOG2E : 1e30f;
-    }
+    const int r = fr0 + (threadIdx.x & 31);
+    stat = sp[fh * seqs.h + min(r, T - 1)];
+    stat_live = r < T;
     fr0 += QT;
     if (fr0 >= T) { fr0 = first; ++fh; }
   };
@@ -542,10 +581,14 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
     char* s = smem + KB + (i & 1) * SB;
     tq.store(s);
     td.store(s + TB);
-    if (threadIdx.x < 64) reinterpret_cast<float*>(s + 2 * TB)[threadIdx.x] = stat;
+    // rows past the end get weight exp(-huge) = 0
+    if (threadIdx.x < 64)
+      reinterpret_cast<float*>(s + 2 * TB)[threadIdx.x] =
+          threadIdx.x >= 32 ? stat : stat_live ? stat * LOG2E : 1e30f;
   };
   fetch();
   store(0);
+  arrived<D>(vf);
   __syncthreads();
 
   int r0 = first;
@@ -555,11 +598,17 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
     const float* st_lse = reinterpret_cast<const float*>(ds_ + TB);
     if (i + 1 < n) fetch();
     if (r0 + QT - 1 >= kv0 && kv0 < T) {                // wave-uniform
+      // a tile's fragment offsets anew in every step: sixteen registers less
+      Frags<D> fr = lane;
+      asm volatile("" : "+v"(fr.row_off), "+v"(fr.tr_lo), "+v"(fr.tr_hi));
       f32x16 s = zero16(), dp = zero16();
+      __builtin_amdgcn_s_setprio(1);
       #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) s = mfma(fr.row(qs, 0, ks), fr.row(smem, wave, ks), s);
-      #pragma unroll
-      for (int ks = 0; ks < D / 16; ++ks) dp = mfma(fr.row(ds_, 0, ks), vf[ks], dp);
+      for (int ks = 0; ks < D / 16; ++ks) {
+        s = mfma(fr.row(qs, 0, ks), fr.row(smem, wave, ks), s);
+        dp = mfma(fr.row(ds_, 0, ks), vf[ks], dp);
+      }
+      __builtin_amdgcn_s_setprio(0);
       #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const f32x4 le = *reinterpret_cast<const f32x4*>(st_lse + 8 * g + 4 * half);
@@ -578,11 +627,13 @@ void flash_bwd_dkv_kernel(const __hip_bfloat16* __restrict__ q, const __hip_bflo
       #pragma unroll
       for (int k2 = 0; k2 < 2; ++k2) {
         const bf16v8 p = pack8(s, k2), ds = pack8(dp, k2);
+        __builtin_amdgcn_s_setprio(1);
         #pragma unroll
         for (int dt = 0; dt < D / 32; ++dt) {
           av[dt] = mfma(fr.col(ds_, k2 * 16, dt), p, av[dt]);
           ak[dt] = mfma(fr.col(qs, k2 * 16, dt), ds, ak[dt]);
         }
+        __builtin_amdgcn_s_setprio(0);
       }
     }
     r0 += QT;
@@ -740,7 +791,11 @@ std::vector<torch::Tensor> launch_bwd(const torch::Tensor& dout, const torch::Te
   if (blocks == 0) return grads;
   TORCH_CHECK(blocks < (1ll << 31), "flash attention: batch too large");
   const int group = Hq / Hkv;
-  const int split = (int)std::min<int64_t>(group, (1024 + kv_blocks - 1) / kv_blocks);
+  // 768 workgroups and more: below that shares of the heads, whole ones where the
+  // fullest would have two anyway. Partial sums cost: 832 blocks of the round above
+  // as they are 1140 us, in halves 1230.
+  int split = (int)std::min<int64_t>(group, (768 + kv_blocks - 1) / kv_blocks);
+  if (2 * split > group) split = group;
   torch::Tensor part;
   float *pk = nullptr, *pv = nullptr;
   if (split > 1) {
