@@ -89,6 +89,33 @@ DEV_INLINE void add_parts8(float (&v)[8], const float* p, int64_t step, int n) {
   }
 }
 
+// the same for two runs of eight, d elements apart
+DEV_INLINE void add_parts8x2(float (&v)[8], float (&w)[8], const float* p, int64_t d, int64_t step,
+                             int n) {
+  for (int z = 0; z < n; z += 4) {
+    f32x4v a[4][4];
+    #pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* q = p + min(z + i, n - 1) * step;
+      a[i][0] = *reinterpret_cast<const f32x4v*>(q);
+      a[i][1] = *reinterpret_cast<const f32x4v*>(q + 4);
+      a[i][2] = *reinterpret_cast<const f32x4v*>(q + d);
+      a[i][3] = *reinterpret_cast<const f32x4v*>(q + d + 4);
+    }
+    #pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (z + i < n) {
+        #pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[j] += a[i][0].v[j];
+          v[4 + j] += a[i][1].v[j];
+          w[j] += a[i][2].v[j];
+          w[4 + j] += a[i][3].v[j];
+        }
+      }
+  }
+}
+
 // ---- hash (counter-based random numbers) ----
 DEV_INLINE uint64_t splitmix64(uint64_t x) {
   x += 0x9E3779B97F4A7C15ull;

@@ -27,7 +27,7 @@
 // K and V are read once per sequence and kv head; bound by HBM.
 // 160 sequences of 420..1550 tokens sharing prompts, 28/4 heads of 128
 // (251 MB of distinct rows): 157 us with one lane a token on vector FMAs,
-// 76 us now; 3 sequences of 911..3777, 14/2 heads of 64: 43 -> 12.
+// 68 us now; 3 sequences of 911..3777, 14/2 heads of 64: 43 -> 12.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
@@ -141,19 +141,22 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
     constexpr int PER = D / 16;
     const int width = (H + 2 * KV) * D;
     const bool owner = z + 1 == (int)gridDim.z || c0 + slice_len >= len;
+    auto start = [&](float (&x)[8], int at) {           // the bias, or zero
+      #pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = 0.f;
+      if (src.bias) {
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(src.bias + at);
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = bf2f(v.v[j]);
+      }
+    };
     auto take = [&](float (&x)[8], int at) {
       if constexpr (SRC == ROWS) {
         const bf16x8 v = *reinterpret_cast<const bf16x8*>(src.rows + (int64_t)seq * width + at);
         #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = bf2f(v.v[j]);
       } else {
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = 0.f;
-        if (src.bias) {
-          const bf16x8 v = *reinterpret_cast<const bf16x8*>(src.bias + at);
-          #pragma unroll
-          for (int j = 0; j < 8; ++j) x[j] = bf2f(v.v[j]);
-        }
+        start(x, at);
         add_parts8(x, src.parts + (int64_t)seq * width + at, (int64_t)N * width, src.splits);
       }
     };
@@ -175,8 +178,15 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
       const int head = u / PER, c = u % PER * 8;        // head == group: the key
       const int at = (head < group ? kv * group + head : H + kv) * D + c;
       float x1[8], x2[8];
-      take(x1, at);
-      take(x2, at + D / 2);
+      if constexpr (SRC == ROWS) {
+        take(x1, at);
+        take(x2, at + D / 2);
+      } else {
+        start(x1, at);
+        start(x2, at + D / 2);
+        add_parts8x2(x1, x2, src.parts + (int64_t)seq * width + at, D / 2, (int64_t)N * width,
+                     src.splits);
+      }
       const __hip_bfloat16* nw = head < group ? src.q_norm : src.k_norm;
       if (nw) {
         float ss = 0.f;
@@ -460,7 +470,12 @@ void decode(const __hip_bfloat16* q, const torch::Tensor& kcache, const torch::T
   const int cs = slices(blocks, max_ctx), slice_len = std::max(1, CDIV(max_ctx, cs));
   #define DECODE(DD, NN) launch_decode<DD, NN, SRC>(q, kcache, vcache, bt, ctx, out, N, H, KV, \
                                                     (float)scale, q_row_stride, cs, slice_len, src)
-  if (D == 128) { if (few) DECODE(128, 8); else DECODE(128, 4); }
+  // From 513 workgroups on those of four waves with rows of 128 no longer run at
+  // once (two a CU by their LDS), those of two do: the round above 70.6 -> 67.7 us,
+  // 10 x 16 of 180..380 20.5 -> 18.1 (from partial sums 29.1 -> 21.8), 16 x 16
+  // 26.6 -> 24.0; 256 workgroups of
+  // 500..1500 would take 49.4 for 35.5, and rows of 64 fit four a CU anyway.
+  if (D == 128) { if (few) DECODE(128, 8); else if (blocks > 512) DECODE(128, 2); else DECODE(128, 4); }
   else { if (few) DECODE(64, 8); else DECODE(64, 4); }
   #undef DECODE
   HIP_CHECK_LAST();

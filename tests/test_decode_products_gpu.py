@@ -247,3 +247,22 @@ def test_decode_state(ext, N, bs, eos):
         tok, pos, ctx = torch.where(go, new, tok), pos + go, ctx + go.int()
         for a, b in zip(state, (tok, pos, ctx, limits, fin, torch.tensor([step + 1], device="cuda"), out)):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("N,H,KV", [(128, 28, 4), (129, 28, 4), (257, 4, 2)])
+def test_paged_decode_many_sequences(ext, N, H, KV):
+    """512 workgroups, one more a kv head and 514: workgroups of four and of two
+    waves, contexts of one token to several chunks; bf16 output."""
+    D, bs, g = 128, 16, torch.Generator(device="cuda").manual_seed(N)
+    lens = torch.randint(1, 300, (N,), generator=g, device="cuda", dtype=torch.int32)
+    lens[:6] = torch.tensor([1, 32, 33, 64, 65, 299], device="cuda")
+    nb = (300 + bs - 1) // bs
+    pages = torch.randperm(N * nb, generator=g, device="cuda").view(N, nb).int()
+    q, key, value = _rand((N, H, D), 1), _rand((N * nb, bs, KV, D), 2), _rand((N * nb, bs, KV, D), 3)
+    out = ext.paged_attention_decode(q, key, value, pages, lens, D ** -0.5).double()
+    for i in [*range(6), N - 1]:
+        c = int(lens[i])
+        k, v = (t[pages[i].long()].flatten(0, 1)[:c].double().repeat_interleave(H // KV, 1)
+                for t in (key, value))
+        p = (torch.einsum("hd,chd->hc", q[i].double(), k) * D ** -0.5).softmax(-1)
+        assert _rel(out[i], torch.einsum("hc,chd->hd", p, v)) < 2.0 ** -8
