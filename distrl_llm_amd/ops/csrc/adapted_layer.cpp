@@ -52,9 +52,10 @@ void scaled_mm(const Tensor& a, const Tensor& b, double scale, Tensor out) {
 
 // Adapters of projections that share an input, or of one: A (r, K), B (N, r).
 struct Adapters {
-  // From this many rows on the GPU is behind the host, and the library's products
-  // are faster on it (16 x 1550 tokens on the 1.5B model: 163 and 175 ms).
-  static constexpr int64_t MANY = 4096;
+  // Adapters of 96 columns and more re-read a wider A for every 32 rows: from this
+  // many rows on the GPU is behind the host, and the library's product faster on it
+  // (18793 x 1536: 19.5 us for 28.9; 4816: 19.4 for 10.6).
+  static constexpr int64_t MANY = 8192;
 
   Tensors A, B;
   std::vector<double> scales;
@@ -80,7 +81,7 @@ struct Adapters {
 
   // u <- the adapters' scaled inputs side by side, zeros in spare columns
   void down(const Tensor& x, const Tensor& u) const {
-    if (x.size(0) < MANY && adapter_inputs({{x, u, A, scales}}, false)) return;
+    if ((pad <= 64 || x.size(0) < MANY) && adapter_inputs({{x, u, A, scales}}, false)) return;
     if (std::equal(scales.begin() + 1, scales.end(), scales.begin())) {
       scaled_mm(x, (A.size() > 1 ? at::cat(A) : A[0]).t(), scales[0], columns(u, 0, sum));
     } else {
@@ -95,7 +96,7 @@ struct Adapters {
     for (size_t i = 0; i < B.size(); ++i)
       jobs.push_back({dy[i], i + 1 < B.size() ? part(du, i) : columns(du, at[i], pad - at[i]),
                       {B[i]}, {scales[i]}});
-    if (du.size(0) < MANY && adapter_inputs(jobs, true)) return;
+    if (adapter_inputs(jobs, true)) return;
     for (size_t i = 0; i < B.size(); ++i) scaled_mm(dy[i], B[i], scales[i], part(du, i));
     clear_spare(du);
   }

@@ -61,7 +61,13 @@ DEV_INLINE void share_sum(const Job& job, float* part, char* ty, char* tp, int n
     #pragma unroll
     for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
   u32x4 yv[4], pv[RT];
-  // rows past the end repeat the last one with weight zero
+  bool live = false;
+  const u32x4 zero = {0, 0, 0, 0};
+  // rows past the end repeat the last one with weight zero. The next step's rows
+  // are fetched before this one's products and only looked at when they are stored:
+  // cleared where they were fetched, and sunk behind the products by the compiler,
+  // they were waited for in every step (18793 rows, feed-forward half of 1536 and
+  // 8960 columns: 283 us, 263 now)
   const int yc = tid & 15, ycol = min(n0 + yc * 8, job.N - 8);
   auto fetch = [&](int64_t row) {
     #pragma unroll
@@ -70,11 +76,11 @@ DEV_INLINE void share_sum(const Job& job, float* part, char* ty, char* tp, int n
                                               ycol);
     #pragma unroll
     for (int i = 0; i < RT; ++i) {
-      const int64_t at = row + (tid >> 2);
       const int c = i * 32 + (tid & 3) * 8;
-      pv[i] = *reinterpret_cast<const u32x4*>(job.p + min(at, r1 - 1) * job.ldp + min(c, job.r - 8));
-      if (at >= r1 || c >= job.r) pv[i] = u32x4{0, 0, 0, 0};
+      pv[i] = *reinterpret_cast<const u32x4*>(job.p + min(row + (tid >> 2), r1 - 1) * job.ldp +
+                                              min(c, job.r - 8));
     }
+    live = row + (tid >> 2) < r1;
   };
   fetch(r0);
   for (int64_t row = r0; row < r1; row += ROWS) {
@@ -84,9 +90,11 @@ DEV_INLINE void share_sum(const Job& job, float* part, char* ty, char* tp, int n
       *reinterpret_cast<u32x4*>(ty + chunk((tid >> 4) + i * 16, yc)) = yv[i];
     #pragma unroll
     for (int i = 0; i < RT; ++i)
-      *reinterpret_cast<u32x4*>(tp + chunk(tid >> 2, i * 4 + (tid & 3))) = pv[i];
+      *reinterpret_cast<u32x4*>(tp + chunk(tid >> 2, i * 4 + (tid & 3))) =
+          live && i * 32 + (tid & 3) * 8 < job.r ? pv[i] : zero;
     __syncthreads();
-    fetch(min(row + ROWS, r1 - 1));
+    if (row + ROWS < r1) fetch(row + ROWS);
+    __builtin_amdgcn_sched_barrier(0);
     #pragma unroll
     for (int k = 0; k < ROWS; k += 16) {
       const bf16v8 y = column(ty, k, wave);

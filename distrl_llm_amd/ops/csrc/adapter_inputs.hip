@@ -5,14 +5,15 @@
 // These products have 32 to 128 columns and only read x or dY. The library took one
 // call for each, five forward and seven backward a layer, 17 us of the host's time
 // apiece, with another for the concatenation of the A; short micro-batches wait for
-// that: a pass of the 0.5B model over 3 x 308 tokens 20.7 -> 17.4 ms. A workgroup
+// that: a pass of the 0.5B model over 3 x 308 tokens 20.7 -> 17.2 ms. A workgroup
 // owns 32 rows and all columns; 128 of K a step pass through LDS, fetched into
 // registers up to three steps ahead, and eight waves take 16 of K each, so that few
 // workgroups have short chains. B lies with its columns innermost and is read
 // transposed (LDS transpose reads). The waves' sums meet in LDS, two and two.
-// Bound: the chain of steps, 0.3 us each. rows x K, columns, the library's product
-// against this, us: 900 x 896, 96 20.6 and 11.7; 900 x 4864, 32 18.8 and 15.1; 2400 x
-// 1536, 96 19.1 and 14.4; 4816 x 4864, 32 18.4 and 21.0.
+// Bound: HBM for many rows, else the chain of steps. rows x K, columns, the
+// library's product against this, us: 900 x 896, 96 20.1 and 7.8; 900 x 4864, 32
+// 19.6 and 11.1; 4816 x 8960, 32 20.3 and 19.1 (B 28.6 and 20.3); 18793 x 1536, 32
+// 19.2 and 13.4; 18793 x 8960, 32 76.7 and 81.3; 18793 x 1536, 96 19.5 and 28.9.
 #include <ATen/cuda/CUDAContext.h>
 #include "adapted.h"
 #include "common.h"
@@ -34,10 +35,16 @@ struct Input {
   int64_t ldx, ldo;
   float scale[PIECES];
   int first[PIECES + 1];    // columns of each adapter
-  int n, K, cols;
+  int n, K, cols, total;
 };
 
 struct Inputs { Input j[JOBS]; };
+
+// The jobs' pointers come out of an array, so the compiler does not see that they
+// are global: flat loads would wait on LDS too.
+typedef __attribute__((address_space(1))) const u32x4 global_u32x4;
+typedef __attribute__((address_space(1))) bf16v4 global_bf16v4;
+DEV_INLINE u32x4 load16(const __hip_bfloat16* p) { return *(global_u32x4*)p; }
 
 // 16 B chunk c of row k of a B tile of 32 RT columns: 4 rows over 64 B (transpose
 // reads) fall into different banks
@@ -46,6 +53,15 @@ DEV_INLINE int b_chunk(int k, int c) {
   constexpr int W = RT == 3 ? 4 : RT;
   const int swz = RT == 1 ? 0 : RT == 2 ? ((k >> 1) & 1) << 2 : (k & 3) << 2;
   return k * (W * 64) + ((c ^ swz) << 4);
+}
+
+// The adapter that column n belongs to. (By index, the job would lie in scratch.)
+struct Piece { const __hip_bfloat16* m; float scale; int first, end; };
+DEV_INLINE Piece piece(const Input& j, int n) {
+  Piece p{j.m[0], j.scale[0], 0, j.first[1]};
+  if (j.n > 1 && n >= j.first[1]) p = {j.m[1], j.scale[1], j.first[1], j.first[2]};
+  if (j.n > 2 && n >= j.first[2]) p = {j.m[2], j.scale[2], j.first[2], j.first[3]};
+  return p;
 }
 
 // grid (rows / 32, jobs)
@@ -58,7 +74,7 @@ void adapter_inputs_kernel(Inputs in, int rows) {
   const int tid = threadIdx.x, l = tid & 63, lr = l & 31, h = l >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row0 = blockIdx.x * 32, K = job.K, steps = (K + BK - 1) / BK;
-  const int total = job.first[job.n];
+  const int total = job.total;
   const u32x4 zero = {0, 0, 0, 0};
 
   // rows of 16 chunks: chunk c of row r at r * 256 + ((c ^ r % 16) << 4)
@@ -78,10 +94,9 @@ void adapter_inputs_kernel(Inputs in, int rows) {
       ms[j] = b_chunk<RT>(mk[j], mc);
     } else {
       const int n = r0 + j * 32;
-      int i = 0;
-      while (i + 1 < job.n && n >= job.first[i + 1]) ++i;
+      const Piece pc = piece(job, n);
       mok[j] = n < total;
-      mp[j] = job.m[i] + (int64_t)min(n - job.first[i], job.first[i + 1] - job.first[i] - 1) * K;
+      mp[j] = pc.m + (int64_t)min(n - pc.first, pc.end - pc.first - 1) * K;
       mk[j] = 0;
       ms[j] = n * RB + ((c ^ (n & 15)) << 4);
     }
@@ -96,10 +111,10 @@ void adapter_inputs_kernel(Inputs in, int rows) {
   // steps past the end repeat the last one; past K both operands are zero
   auto load = [&](int i, int s) {
     const int k0 = min(s, steps - 1) * BK, k = k0 + c * 8;
-    xv[i] = *reinterpret_cast<const u32x4*>(xp + min(k, K - 8));
+    xv[i] = load16(xp + min(k, K - 8));
     #pragma unroll
     for (int j = 0; j < RT; ++j)
-      mv[i][j] = *reinterpret_cast<const u32x4*>(
+      mv[i][j] = load16(
           mp[j] + (KM ? (int64_t)min(k0 + mk[j], K - 1) * total : (int64_t)min(k, K - 8)));
   };
   auto store = [&](int i, int s, int buf) {
@@ -112,6 +127,8 @@ void adapter_inputs_kernel(Inputs in, int rows) {
   };
   int buf = 0;
   auto step = [&](int i, int s) {
+    load(i, s + 3);
+    __builtin_amdgcn_sched_barrier(0);    // not behind the products
     const int at = lr * RB + (((wave * 2 + h) ^ (lr & 15)) << 4);
     const bf16v8 xf = *reinterpret_cast<const bf16v8*>(smem + buf + at);
     #pragma unroll
@@ -132,7 +149,6 @@ void adapter_inputs_kernel(Inputs in, int rows) {
     }
     buf ^= TB;
     store((i + 1) % 3, s + 1, buf);
-    load(i, s + 3);
     __syncthreads();
   };
   load(0, 0);
@@ -182,12 +198,11 @@ void adapter_inputs_kernel(Inputs in, int rows) {
     for (int q = 0; q < 4; ++q) {
       const int n = t * 32 + 8 * q + 4 * h;
       if (n >= job.cols) continue;
-      int i = 0;
-      while (i + 1 < job.n && n >= job.first[i + 1]) ++i;
+      const float scale = piece(job, n).scale;
       bf16v4 o;
       #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = (__bf16)(acc[t][4 * q + r] * job.scale[i]);
-      *reinterpret_cast<bf16v4*>(job.out + row * job.ldo + n) = o;
+      for (int r = 0; r < 4; ++r) o[r] = (__bf16)(acc[t][4 * q + r] * scale);
+      *(global_bf16v4*)(job.out + row * job.ldo + n) = o;
     }
 }
 
@@ -244,6 +259,7 @@ bool adapter_inputs(const std::vector<AdapterInput>& jobs, bool k_major) {
     if (j.out.size(1) < o.first[o.n] || j.out.size(1) > 128) return false;
     if (rows > 1 && j.out.stride(0) < j.out.size(1)) return false;   // rows over one another
     o.cols = (int)j.out.size(1);
+    o.total = o.first[o.n];
     most = std::max(most, o.cols);
     o.x = iptr(j.x);
     o.out = reinterpret_cast<__hip_bfloat16*>(j.out.data_ptr());
