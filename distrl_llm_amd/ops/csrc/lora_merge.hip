@@ -13,14 +13,11 @@
 // 13 ms with two loads in flight; 61 us for a projection of 18944 x 3584, of
 // which a copy of that size takes 55.
 //
-// The same kernel adds an adapter's output to the rows of a product, in place:
-// y += scale * u B^T (TA: A given as (K, r), staged as it lies) and
-// y += scale * u A. r 32, rows x columns, the library's addmm against this:
-// 128 x 896 3.9 and 5.3 us, 2408 x 3584 10 and 12, 2408 x 18944 41 and 40,
-// 4816 x 3584 160 and 19. On the GPU that is a draw below 4000 rows, but the
-// library's call costs 19 us of host time and this one 4, and short
-// micro-batches wait for the host: a pass of the 0.5B model over 3 x 308 tokens
-// 34.2 -> 28.0 ms; the 1.5B model's over 16 x 1550 is unchanged (within 1%).
+// The same kernel adds an adapter's output to the rows of a product, in place (the
+// prompt phase): y += scale * u B^T (TA: A given as (K, r), staged as it lies) and
+// y += scale * u A. r 32, rows x columns, the library's addmm against this, us:
+// 128 x 896 3.9 and 5.3, 2408 x 3584 10 and 12, 2408 x 18944 41 and 40, 4816 x 3584
+// 160 and 19; the library's call costs 19 us of host time and this one 4.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
