@@ -96,7 +96,11 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
   float* ml_lds = reinterpret_cast<float*>(smem + NW * (2 * CHUNK * D * 2));  // [NW][16][2]
   // fused: the heads' queries, then the new token's key and value
   __hip_bfloat16* fresh = reinterpret_cast<__hip_bfloat16*>(ml_lds + NW * 32);
-  const int last = SRC == QUERIES ? 0x7fffffff : len - 1;
+  // only the slice that has the new token makes its key and value: another one's
+  // rows past its end repeat the cache's row before (weight zero, but it must be a
+  // number)
+  const bool owner = z + 1 == (int)gridDim.z || c0 + slice_len >= len;
+  const int last = SRC == QUERIES || !owner ? 0x7fffffff : len - 1;
 
   float m = -1e30f, lsum = 0.f;
   f32x4 acc[DT];
@@ -140,7 +144,6 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
     // then the value, eight elements a thread
     constexpr int PER = D / 16;
     const int width = (H + 2 * KV) * D;
-    const bool owner = z + 1 == (int)gridDim.z || c0 + slice_len >= len;
     auto start = [&](float (&x)[8], int at) {           // the bias, or zero
       #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = 0.f;

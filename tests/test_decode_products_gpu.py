@@ -151,6 +151,47 @@ def test_paged_decode_packed(ext, H, KV, D, N, longest, bs, S, bias, norms):
     assert got[0].isnan().any(-1).sum() == KV
 
 
+@pytest.mark.parametrize("H,KV,D,N,cs", [(28, 4, 128, 16, 4), (28, 4, 128, 32, 2), (14, 2, 64, 32, 4)])
+@pytest.mark.parametrize("S", [0, 2])
+def test_paged_decode_packed_behind_a_slice_end(ext, monkeypatch, H, KV, D, N, cs, S):
+    """Contexts that end 1 to 32 tokens behind a slice whose end is no multiple
+    of 32, after a call that leaves numbers that are none in LDS: the slice does
+    not take the new token, which another one has. Against the same call in one
+    slice; both round to bf16."""
+    bs, nb, width = 16, 97, (H + 2 * KV) * D
+    room = bs * nb
+    end = (room + cs - 1) // cs
+    assert end % 32
+    behind = [z * end + d for z in range(1, cs) for d in (1, 2, 16, 27, 28, 29, 32)]
+    lens = torch.tensor((behind * N)[:N - 1] + [room], device="cuda", dtype=torch.int32)
+    pages = torch.randperm(N * nb, generator=torch.Generator().manual_seed(N)).view(N, nb)
+    pages = pages.to("cuda", torch.int32)
+    pos = lens - 1
+    slots = pages.gather(1, (pos // bs).long()[:, None])[:, 0].long() * bs + pos % bs
+    cache = [_rand((N * nb, bs, KV, D), 4 + i) for i in range(2)]
+    inv = 1.0 / 1e4 ** (torch.arange(0, D, 2, device="cuda").float() / D)
+    rows = _rand((S, N, width), 1).float() if S else _rand((N, width), 1)
+    arrived = torch.zeros(256, dtype=torch.int32, device="cuda")
+    most = 255 // KV
+
+    def call(qkv, at, slots, tables, lens):
+        return ext.paged_decode_packed(qkv, None, at, slots, inv, *cache, tables, lens, arrived, H,
+                                       D ** -0.5)
+
+    def full(value, dtype):
+        return torch.full((most,), value, dtype=dtype, device="cuda")
+
+    monkeypatch.setenv("DISTRL_PAGED_CS", "1")
+    ref = call(rows, pos, slots, pages, lens)
+    call(torch.full((most, width), float("nan"), dtype=torch.bfloat16, device="cuda"),
+         full(room - 1, torch.int32), full(-1, torch.long), pages[torch.arange(most) % N].contiguous(),
+         full(room, torch.int32))
+    monkeypatch.delenv("DISTRL_PAGED_CS")
+    out = call(rows, pos, slots, pages, lens)
+    assert bool(out.isfinite().all()) and _rel(out, ref) < 2.0 ** -8
+    assert not arrived.any()
+
+
 @pytest.mark.parametrize("name,four_bit,lora_r", [("small-qwen2", False, 8), ("small-qwen2", True, 8),
                                                   ("small-qwen3", True, 0), ("small-qwen3", False, 12)])
 @pytest.mark.parametrize("n", [3, 40, 161])
