@@ -10,7 +10,8 @@ is ~19 launches here, prepared in native code (ops/csrc/adapted_layer.cpp):
 adapters are columns of their projections' products, W laid out beside B for
 it. That costs a copy of the weights, 37 us a layer of the 1.5B model forward
 and as long backward, where adding the adapters' outputs to 18800 rows in
-passes of their own took 750. Adapter gradients are one launch and its sum
+passes of their own took 750; large weights that few rows meet are taken as
+they lie, their adapters joined to fp32 products. Adapter gradients are one launch and its sum
 (ops/csrc/adapter_grads.hip).
 """
 

@@ -32,16 +32,19 @@ namespace {
 constexpr int KC = 256;            // columns of a workgroup
 constexpr int STEPS = KC / 32;     // loads of W in flight
 
-// w and out may be one; res (or none) is added to the same sum. Rows of w and
-// out are ldw elements apart, those of b ldb. TA: a is (K, r). TILES: out in
-// tiles of 32 rows x 16 of K, [K half][row][8 elements], row n of w at row + n of
-// out, or (glu) at row + n in blocks of 16 of every 32; r may be 0.
-template <bool TA, bool TILES = false>
+// w (bf16, or fp32 sums) and out may be one; res (or none) is added to the same
+// sum. Rows of w are ldw elements apart, of out ldo, of b ldb, of res ldr (zero: one
+// for all). TA: a is (K, r). TILES: out in tiles of 32 rows x 16 of K, [K half][row][8
+// elements], row n of w at row + n of out, or (glu) at row + n in blocks of 16 of
+// every 32; r may be 0.
+template <bool TA, bool TILES = false, typename W = __hip_bfloat16>
 __global__ __launch_bounds__(256)
-void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict__ a,
+void lora_merge_kernel(const W* w, const __hip_bfloat16* __restrict__ a,
                        const __hip_bfloat16* __restrict__ b, const __hip_bfloat16* __restrict__ res,
-                       __hip_bfloat16* out, int N, int K, int r, int rows, int64_t ldw, int ldb,
-                       int64_t ldr, float scale, int row0, int glu) {
+                       __hip_bfloat16* out, int N, int K, int r, int rows, int64_t ldw, int64_t ldo,
+                       int ldb, int64_t ldr, float scale, int row0, int glu) {
+  typedef __attribute__((ext_vector_type(8))) float f32x8;
+  typedef std::conditional_t<std::is_same_v<W, float>, f32x8, bf16v8> WV;
   // A: [r32][KC], TA: [KC][r32], rows 16 B apart
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int RS = KC * 2 + 16;
@@ -62,12 +65,12 @@ void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict
   const int l = threadIdx.x & 63, g = l >> 4, lr = l & 15;
   const int end = min(N, (int)(blockIdx.y + 1) * rows);
   for (int n0 = blockIdx.y * rows + wave * 16; n0 < end; n0 += 64) {
-    const __hip_bfloat16* wrow = w + min(n0 + lr, N - 1) * ldw + g * 8;
+    const W* wrow = w + min(n0 + lr, N - 1) * ldw + g * 8;
     const __hip_bfloat16* brow = b + (int64_t)min(n0 + lr, N - 1) * ldb;
-    bf16v8 wv[STEPS];
+    WV wv[STEPS];
     #pragma unroll
     for (int i = 0; i < STEPS; ++i)                     // K % 32 == 0
-      wv[i] = *reinterpret_cast<const bf16v8*>(wrow + min(k0 + i * 32, K - 32));
+      wv[i] = *reinterpret_cast<const WV*>(wrow + min(k0 + i * 32, K - 32));
     bf16v8 rv[STEPS];
     if (res) {
       #pragma unroll
@@ -116,7 +119,7 @@ void lora_merge_kernel(const __hip_bfloat16* w, const __hip_bfloat16* __restrict
         const int n = n0 + lr, k = k0 + i * 32 + g * 8, row = row0 + (glu ? n + (n & ~15) : n);
         const int64_t at = TILES ? (int64_t)(row >> 5) * K * 32 + (k >> 4) * 512 + (k & 8) * 32 +
                                        (row & 31) * 8
-                                 : n * ldw + k;
+                                 : n * ldo + k;
         *reinterpret_cast<bf16v8*>(out + at) = o;
       }
     }
@@ -134,21 +137,23 @@ const __hip_bfloat16* lptr(const torch::Tensor& t) {
 }
 
 // rows of a (rows, columns) operand that 16 B accesses can walk
-bool lrows(const torch::Tensor& t) {
-  return t.is_cuda() && t.scalar_type() == at::kBFloat16 && t.dim() == 2 && t.stride(1) == 1 &&
+bool lrows(const torch::Tensor& t, at::ScalarType type = at::kBFloat16) {
+  return t.is_cuda() && t.scalar_type() == type && t.dim() == 2 && t.stride(1) == 1 &&
          t.stride(0) % 8 == 0 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 
-// out = w + scale * b a, or b a^T (ta); false: not these operands
+// out = w + scale * b a, or b a^T (ta), then + res; w bf16 or fp32; false: not these
+// operands
 bool launch_merge(const torch::Tensor& w, const torch::Tensor& a, const torch::Tensor& b,
                   const torch::Tensor& out, bool ta, double scale,
                   const c10::optional<torch::Tensor>& res = c10::nullopt) {
   if (w.dim() != 2 || a.dim() != 2 || b.dim() != 2) return false;
   const int N = w.size(0), K = w.size(1), r = b.size(1);
+  const bool sums = w.scalar_type() == at::kFloat;
   if (!lora_merge_takes(K, r) || (ta ? a.size(0) : a.size(1)) != K ||
       (ta ? a.size(1) : a.size(0)) != r || b.size(0) != N || out.sizes() != w.sizes() ||
-      !lrows(w) || !lrows(b) || !lrows(out) || !lrows(a) || !a.is_contiguous() ||
-      w.stride(0) != out.stride(0))
+      !lrows(w, sums ? at::kFloat : at::kBFloat16) || !lrows(b) || !lrows(out) || !lrows(a) ||
+      !a.is_contiguous() || (!sums && w.stride(0) != out.stride(0)))
     return false;
   if (N > 1 && out.stride(0) < K) return false;         // rows over one another
   if (res && (!lrows(*res) || res->sizes() != w.sizes())) return false;
@@ -159,10 +164,22 @@ bool launch_merge(const torch::Tensor& w, const torch::Tensor& a, const torch::T
   const dim3 grid(CDIV(K, KC), CDIV(N, rows)), block(256);
   auto stream = at::cuda::getCurrentCUDAStream();
   const int r32 = (r + 31) / 32 * 32, smem = ta ? KC * (r32 * 2 + 16) : r32 * (KC * 2 + 16);
-  hipLaunchKernelGGL(ta ? lora_merge_kernel<true> : lora_merge_kernel<false>, grid, block, smem,
-                     stream, lptr(w), lptr(a), lptr(b), res ? lptr(*res) : nullptr,
-                     reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), N, K, r, rows,
-                     w.stride(0), (int)b.stride(0), res ? res->stride(0) : 0, (float)scale, 0, 0);
+  auto go = [&](auto kernel, auto* from) {
+    hipLaunchKernelGGL(kernel, grid, block, smem, stream, from, lptr(a), lptr(b),
+                       res ? lptr(*res) : nullptr,
+                       reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), N, K, r, rows,
+                       w.stride(0), out.stride(0), (int)b.stride(0), res ? res->stride(0) : 0,
+                       (float)scale, 0, 0);
+  };
+  if (sums) {
+    const float* p = w.data_ptr<float>();
+    if (ta) go(lora_merge_kernel<true, false, float>, p);
+    else go(lora_merge_kernel<false, false, float>, p);
+  } else if (ta) {
+    go(lora_merge_kernel<true>, lptr(w));
+  } else {
+    go(lora_merge_kernel<false>, lptr(w));
+  }
   HIP_CHECK_LAST();
   return true;
 }
@@ -204,7 +221,8 @@ bool weight_tiles(torch::Tensor w, torch::Tensor out, int64_t row, bool glu,
                      smem, at::cuda::getCurrentCUDAStream(), lptr(w), r ? lptr(*a) : nullptr,
                      r ? lptr(*b) : nullptr, nullptr,
                      reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), N, K, r, rows, w.stride(0),
-                     r ? (int)b->stride(0) : 0, 0, (float)scale, (int)row, (int)glu);
+                     (int64_t)K, r ? (int)b->stride(0) : 0, (int64_t)0, (float)scale, (int)row,
+                     (int)glu);
   HIP_CHECK_LAST();
   return true;
 }
@@ -218,6 +236,14 @@ bool lora_add(torch::Tensor y, torch::Tensor u, torch::Tensor m, double scale,
   if (m.dim() != 2) return false;
   const bool ta = m.stride(1) != 1;
   return launch_merge(y, ta ? m.t() : m, u, y, ta, scale, res);
+}
+
+// out (M, N) bf16 = y (M, N) fp32 + u m + res if given (rows that may be one), rounded
+// once; otherwise as lora_add.
+bool lora_join(torch::Tensor y, torch::Tensor u, torch::Tensor m, torch::Tensor out,
+               c10::optional<torch::Tensor> res) {
+  const bool ta = m.stride(1) != 1;
+  return y.scalar_type() == at::kFloat && launch_merge(y, ta ? m.t() : m, u, out, ta, 1., res);
 }
 
 // ---- base and adapter weights as one matrix, so that one product does both:

@@ -334,10 +334,11 @@ def test_paged_decode_reads_packed_rows(ext):
 
 # ----------------------------------------------------- fused layer, rotary
 
-def _train_model(name, **kw):
+def _train_model(name, lora_r=8, **kw):
     from distrl_llm_amd.models import CausalLM, get_spec
-    model = CausalLM(get_spec(name), lora_r=8, lora_alpha=16, dtype=torch.bfloat16,
-                     device=torch.device("cuda"), **kw).random_init(3)
+    model = CausalLM(get_spec(name) if isinstance(name, str) else name, lora_r=lora_r,
+                     lora_alpha=16, dtype=torch.bfloat16, device=torch.device("cuda"),
+                     **kw).random_init(3)
     g = torch.Generator(device="cuda").manual_seed(5)
     with torch.no_grad():
         for n, p in model.named_parameters():
@@ -385,6 +386,36 @@ def test_fused_layer_matches_modules(name, B, T):
     # a single rounding or two of luck
     fused, plain, ref = (torch.cat([x.reshape(-1) for x in xs[1:]]) for xs in (fused, plain, ref))
     assert _rel(fused, ref) < 1.3 * _rel(plain, ref) + 2.0 ** -9
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (2, 77)])
+@pytest.mark.parametrize("lora_r,norms", [(8, False), (12, True), (96, False)])
+def test_fused_layer_takes_large_weights_as_they_lie(B, T, lora_r, norms):
+    """Few rows of a layer whose products are all past the size where weights
+    are no longer laid out beside their adapters, at ranks that the joining
+    kernel takes and that it does not: against fp64, as above."""
+    from distrl_llm_amd.models import CausalLM, fused_layer
+    from distrl_llm_amd.models.spec import ModelSpec
+    spec = ModelSpec("wide", 64, 4096, 8192, 1, 64, 8, 128, 1e6, 1e-6, True, not norms,
+                     qk_norm=norms)
+    model = _train_model(spec, lora_r=lora_r)
+    g = torch.Generator().manual_seed(T)
+    ids = torch.randint(0, 64, (B, T), generator=g).cuda()
+    mask, dout = torch.ones_like(ids), _rand((B, T, 4096), 9)
+    exact = CausalLM(spec, lora_r=lora_r, lora_alpha=16, dtype=torch.float64)
+    exact.load_state_dict({k: v.double().cpu() for k, v in model.state_dict().items()})
+    ref = _grads(exact.train(), ids.cpu(), mask.cpu(), dout.double().cpu())
+    fused = _grads(model, ids, mask, dout)
+    usable = fused_layer.usable
+    fused_layer.usable = lambda layer, x: False
+    try:
+        plain = _grads(model, ids, mask, dout)
+    finally:
+        fused_layer.usable = usable
+    for part in (slice(0, 1), slice(1, None)):
+        got, base, want = (torch.cat([x.double().cpu().reshape(-1) for x in xs[part]])
+                           for xs in (fused, plain, ref))
+        assert _rel(got, want) < 1.3 * _rel(base, want) + 2.0 ** -9
 
 
 def test_fused_layer_steps_aside():
