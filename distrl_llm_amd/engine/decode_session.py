@@ -353,6 +353,7 @@ class SessionCache:
 
     def __init__(self, engine):
         self.engine = engine
+        self.moves = 0
         self._cache = {}
 
     @staticmethod

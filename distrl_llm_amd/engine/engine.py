@@ -465,8 +465,11 @@ class Engine:
         DISTRL_GRAPH_CACHE=0 reverts to per-wave sessions."""
         from .decode_session import DecodeSession, SessionCache
         if os.environ.get("DISTRL_GRAPH_CACHE", "1") == "1":
-            if self._session_cache is None:
+            # graphs hold addresses of weights that may have moved since
+            moves = self.fused.moves if self.fused is not None else 0
+            if self._session_cache is None or self._session_cache.moves != moves:
                 self._session_cache = SessionCache(self)
+                self._session_cache.moves = moves
             try:
                 return self._session_cache.acquire(running, sp, eos_token_id)
             except MemoryError:
@@ -628,7 +631,7 @@ class Engine:
                 if apart:
                     # the 4-bit site keeps its adapter beside the base image
                     u = ext.skinny_gemm(act, lw.down_a, 0, tiles=t)
-                    base = lw.tiles["down"] if t else lw.mods["down"][0].weight
+                    base = lw.tiles["down"] if t else lw.rows("base")
                     res = ext.skinny_gemm(act, base, 1, res=res, u=u,
                                           ub=lw.down_b, tiles=t)
                 else:

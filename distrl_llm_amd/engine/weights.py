@@ -33,9 +33,11 @@ class LayerWeights:
     read (ops/csrc/stream_gemm.hip); ``tiles`` is None where the sizes do not
     tile.
     ``rows(site)``: the same row-major, for the library's products; laid out
-    when first asked for and kept current by every later refresh."""
+    when first asked for and kept current by every later refresh. One weight
+    without an adapter is the module's own; ``rows("base")`` is the down site's
+    whatever its adapter."""
 
-    __slots__ = ("layer", "tiles", "_rows", "down_apart", "qkv_b", "in_norm", "post_norm",
+    __slots__ = ("layer", "tiles", "_rows", "_own", "down_apart", "qkv_b", "in_norm", "post_norm",
                  # nf4 fragment packs (base, built once) + adapter fragment
                  # packs (rebuilt per refresh) for the fused nf4 GEMM path
                  "qkv_w4", "qkv_amax", "o_w4", "o_amax",
@@ -51,6 +53,7 @@ class LayerWeights:
     def __init__(self, layer):
         self.layer = layer
         self.tiles, self._rows = None, {}
+        self._own = set()           # sites of one weight that is copied
         self.down_apart = False     # tiles["down"] without its adapter
 
     @property
@@ -66,28 +69,43 @@ class LayerWeights:
             self._fill_rows(site)
         return self._rows[site]
 
-    def refresh_rows(self):
-        for site in self._rows:
-            self._fill_rows(site)
+    def refresh_rows(self) -> bool:
+        """Whether rows lie elsewhere now: steps captured before are stale."""
+        return any([self._fill_rows(site) for site in self._rows])
 
-    def _fill_rows(self, site: str) -> None:
-        mods, out = self.mods[site], self._rows[site]
-        if len(mods) == 1 and mods[0].r == 0:
-            w = mods[0].weight.detach()
-            if out is None:
-                self._rows[site] = w.contiguous()
-            elif out.data_ptr() != w.data_ptr():    # replaced since
-                out.copy_(w)
-            return
+    def _fill_rows(self, site: str) -> bool:
+        mods, out = self.mods["down" if site == "base" else site], self._rows[site]
+        if site == "base" or len(mods) == 1 and mods[0].r == 0:
+            return self._follow(site, mods[0].weight.detach())
         if out is None:
             out = self._rows[site] = mods[0].weight.new_empty(
                 sum(m.out_features for m in mods), mods[0].in_features)
         # IN PLACE: captured decode steps hold these storages
         if self.tiles is not None and not (site == "down" and self.down_apart):
             out.copy_(_untiled(self.tiles[site], site == "gateup"))
-            return
+            return False
         for m, rows in zip(mods, out.split([m.out_features for m in mods])):
             _merge_into(m, rows)
+        return False
+
+    def _follow(self, site: str, w: torch.Tensor) -> bool:
+        """rows(site) <- the weight w itself, or what it holds."""
+        out = self._rows[site]
+        if site in self._own:
+            out.copy_(w)
+            return False
+        if out is not None and out.data_ptr() == w.data_ptr() and w.is_contiguous():
+            return False
+        # first, or replaced: what was here before is the caller's, not written
+        if not w.is_contiguous() or out is not None and out.dtype != w.dtype:
+            self._own.add(site)
+            w = w.to(w.dtype if out is None else out.dtype, copy=True,
+                     memory_format=torch.contiguous_format)
+        if out is None:
+            self._rows[site] = w
+            return False
+        out.set_(w)
+        return True
 
     qkv_w = property(lambda self: self.rows("qkv"))
     o_w = property(lambda self: self.rows("o"))
@@ -209,6 +227,7 @@ class FusedWeights:
             and q0.weight.is_cuda and shapes_ok
             and os.environ.get("DISTRL_HYBRID_DOWN", "1") == "1")
         self.lora_r = q0.r
+        self.moves = 0      # refreshes after which captured steps are stale
         # the decode products read weights in tiles, where the tiles and the
         # row-major weights that prompts and larger steps read fit beside the
         # model (a 70B model without an adapter keeps row-major ones alone)
@@ -335,7 +354,7 @@ class FusedWeights:
         only the adapter fragment packs (A stacks, block-diagonal scaled B)
         are rebuilt per refresh — the adapter stays exact bf16.
         """
-        first = not self._built
+        first, moved = not self._built, False
         for li, layer in enumerate(self.model.model.layers):
             at = layer.self_attn
             if first:
@@ -360,12 +379,13 @@ class FusedWeights:
                 continue
             if self.tiled:
                 self._refresh_tiles(lw)
-            lw.refresh_rows()
+            moved |= lw.refresh_rows()
             if self.hybrid_down:
                 if self.lora_r > 0:
                     self._refresh_down_adapter(lw)
                 if self._nf4_down:
                     self._refresh_nf4_adapters(lw, layer, sites=("down",))
+        self.moves += moved
         self._built = True
 
     def _refresh_tiles(self, lw: "LayerWeights"):

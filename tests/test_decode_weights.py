@@ -1,0 +1,45 @@
+"""Row-major decode weights as they follow the model's tensors, on the CPU."""
+
+import pytest
+import torch
+
+from distrl_llm_amd.engine import weights
+from distrl_llm_amd.models import CausalLM, get_spec
+
+
+def _model(lora_r=0):
+    return CausalLM(get_spec("small-qwen2"), lora_r=lora_r, dtype=torch.float32).random_init(3)
+
+
+def _rand(like, seed):
+    return torch.randn(like.shape, generator=torch.Generator().manual_seed(seed), dtype=like.dtype)
+
+
+@pytest.mark.parametrize("kind", ["plain", "strided", "other type"])
+def test_replaced_weight_is_left_as_it_was(kind):
+    """A weight without an adapter replaced by another tensor, and back: the
+    rows follow, neither tensor is written, captured steps are given up."""
+    model = _model()
+    fused = weights.FusedWeights(model)
+    fused.refresh()
+    lin, lw = model.model.layers[0].self_attn.o_proj, fused.layers[0]
+    first = lin.weight.data
+    held, kept = lw.rows("o"), first.clone()
+    assert fused.moves == 0
+    other = _rand(first, 5)
+    if kind == "strided":
+        other = other.t().contiguous().t()
+    elif kind == "other type":
+        other = other.double()
+    there = other.clone()
+    for moves, data in ((1, other), (1 if kind != "plain" else 2, first), (None, other)):
+        lin.weight.data = data
+        fused.refresh()
+        assert lw.rows("o") is held and torch.equal(held, lin.weight.to(held.dtype))
+        assert torch.equal(first, kept) and torch.equal(other, there)
+        assert moves is None or fused.moves == moves
+        fused.refresh()
+    if kind != "plain":     # a copy from the first that could not be held on
+        other.add_(1.0)
+        fused.refresh()
+        assert torch.equal(held, other.to(held.dtype))
