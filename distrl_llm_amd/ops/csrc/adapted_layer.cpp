@@ -152,6 +152,32 @@ Tensor product(const Tensor& xu, const Tensors& W, const Adapters& ad,
   return at::addmm(at::cat(all), xu, WB.t());
 }
 
+// a b, from a long K, in runs of rows whose 256 x 256 tiles the chip has at once: past a
+// full wave the library's product of all rows takes as long as for two, or picks another
+// kernel (18793 x 17984 x 1536 1129 us, 16384 rows 671, 10752 rows, one wave, 384). What
+// is left beyond half a wave is a full one too, over rows that are done already: the
+// library takes 316 to 618 us for 5700 to 9400 rows of that product.
+// Sums over 24 row counts of one to four waves, all rows at once -> in runs, ms: K 9792,
+// 896 columns 4.07 -> 2.99; 6208, 1024 2.65 -> 2.59; 17984, 1536 24.8 -> 19.7 (two
+// products of half K 24.7); 22080, 2048 40.0 -> 31.6; 19520, 2560 28.9 -> 22.4; 37952,
+// 3584 67.7 -> 49.9; 28736, 4096 56.0 -> 41.1; 27712, 5120 48.9 -> 37.3; one row count
+// alone 0.47 to 1.16 of its time.
+Tensor in_waves(const Tensor& a, const Tensor& b) {
+  const int64_t rows = a.size(0), cols = b.size(1);
+  constexpr int64_t CUS = 256;
+  const int64_t wave = std::max<int64_t>(1, CUS / ((cols + 255) / 256)) * 256;
+  if (rows <= wave) return at::mm(a, b);
+  auto out = at::empty({rows, cols}, a.options());
+  for (int64_t done = 0; done < rows; done += wave) {
+    const bool full = 2 * (rows - done) > wave;
+    const int64_t from = full ? std::min(done, rows - wave) : done;
+    const int64_t n = full ? wave : rows - done;
+    auto part = out.narrow(0, from, n);
+    at::mm_out(part, a.narrow(0, from, n), b);
+  }
+  return out;
+}
+
 // dY W + du A of projections of one input, their W and A as they lie
 Tensor back_apart(const Tensors& dy, const Tensors& W, const Tensor& du, const Adapters& ad) {
   auto y = at::mm(dy[0], W[0], at::kFloat);
@@ -349,10 +375,9 @@ Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tenso
   auto act = columns(au, 0, inner), ud = columns(au, inner, d_ad.ranks[0]);
 
   const auto [dact, g2, dud] = through(g, W[2], d_ad);
-  // [dgate | du | dup]
   auto dyu = at::empty({rows, 2 * inner + in.pad}, x.options());
-  auto dgate = columns(dyu, 0, inner), du = columns(dyu, inner, in.pad),
-       dup = columns(dyu, inner + in.pad, inner);
+  auto dgate = columns(dyu, 0, inner), dup = columns(dyu, inner, inner),
+       du = columns(dyu, 2 * inner, in.pad);
   silu_mul_bwd_packed(dact, gu, dgate, dup);
   in.up({dgate, dup}, du);
   auto s = sums({{h, du, false},
@@ -367,21 +392,10 @@ Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tenso
   if (want_dx && apart(rows, 2 * inner, hidden)) {
     dx = rmsnorm_bwd_add(back_apart({dgate, dup}, {W[0], W[1]}, du, in), x, norm, g, eps);
   } else if (want_dx) {
-    const auto WA = stack_transposed({W[0], A[0], A[1], W[1]},
-                                     {0, inner, inner + in.ranks[0], inner + in.pad},
+    const auto WA = stack_transposed({W[0], W[1], A[0], A[1]},
+                                     {0, inner, 2 * inner, 2 * inner + in.ranks[0]},
                                      2 * inner + in.pad);
-    const int64_t half = inner + in.ranks[0], rest = inner + in.pad - in.ranks[0];
-    Tensor dh;
-    if (rows >= 8192 && hidden <= 2048 && half % 8 == 0) {
-      // few columns from many rows: the library's product of twice the K takes up
-      // to three times as long (18793 x 17984 x 1536: 1080 us, in two 790; from 4000
-      // rows or for 2560 columns one is the faster)
-      dh = at::mm(columns(dyu, 0, half), columns(WA, 0, half).t());
-      dh.addmm_(columns(dyu, half, rest), columns(WA, half, rest).t());
-    } else {
-      dh = at::mm(dyu, WA.t());
-    }
-    dx = rmsnorm_bwd_add(dh, x, norm, g, eps);
+    dx = rmsnorm_bwd_add(in_waves(dyu, WA.t()), x, norm, g, eps);
   }
   out.insert(out.begin(), dx);
   return out;

@@ -959,6 +959,30 @@ def test_logprob_rows(ext, rows, V):
     assert _rel(grad, ref) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("rows", [4096, 4097, 6145, 8200])
+def test_feed_forward_half_in_waves(ext, rows):
+    """Input gradients of rows whose tiles fill the chip once, of one row more,
+    of half a wave and a row more, and of three runs, against fp64: the bf16 rounding of each value on the way
+    (activation, its gradient, the sum: some 2^-9 each)."""
+    h, f, r = 4096, 64, 8
+    x, g, norm = _rand((rows, h), 1), _rand((rows, h), 2), _rand((h,), 3, 0.1) + 1
+    Ws = [_rand(s, 4 + i, 0.1) for i, s in enumerate(((f, h), (f, h), (h, f)))]
+    As = [_rand((r, w.shape[1]), 7 + i, 0.02) for i, w in enumerate(Ws)]
+    Bs = [_rand((w.shape[0], r), 10 + i, 0.1) for i, w in enumerate(Ws)]
+    scales = [0.5, 2.0, 1.0]
+    y, hu, gu, au = ext.feed_forward_half_fwd(x, norm, 1e-6, Ws, [None, None], As, Bs, scales)
+    dx = ext.feed_forward_half_bwd(g, x, norm, 1e-6, Ws, As, Bs, scales, hu, gu, au, True)[0]
+    xd = x.double().requires_grad_()
+    n = xd * torch.rsqrt((xd * xd).mean(-1, keepdim=True) + 1e-6) * norm.double()
+    wg, wu, wd = (w.double() + s * b.double() @ a.double()
+                  for w, a, b, s in zip(Ws, As, Bs, scales))
+    ref = xd + (torch.nn.functional.silu(n @ wg.t()) * (n @ wu.t())) @ wd.t()
+    want, = torch.autograd.grad(ref, xd, g.double())
+    assert _rel(y, ref.detach()) < 2.0 ** -7
+    for at in (slice(None), slice(0, 1), slice(4095, 4097), slice(rows - 1, rows)):
+        assert _rel(dx[at], want[at]) < 2.0 ** -6
+
+
 @pytest.mark.parametrize("prompts,answers", [([9, 30, 1], [40, 7, 100]), ([0, 5, 3], [4, 0, 6]),
                                              ([3], [1]), ([4, 2], [0, 0])])
 def test_learner_rows_match_padding(prompts, answers):
