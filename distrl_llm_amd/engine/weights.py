@@ -33,11 +33,12 @@ class LayerWeights:
     read (ops/csrc/stream_gemm.hip); ``tiles`` is None where the sizes do not
     tile.
     ``rows(site)``: the same row-major, for the library's products; laid out
-    when first asked for and kept current by every later refresh. One weight
-    without an adapter is the module's own; ``rows("base")`` is the down site's
-    whatever its adapter."""
+    when first asked for and kept current by every later refresh, or for every
+    call alone where there is no room beside the tiles. One weight without an
+    adapter is the module's own; ``rows("base")`` is the down site's whatever
+    its adapter."""
 
-    __slots__ = ("layer", "tiles", "_rows", "_own", "down_apart", "qkv_b", "in_norm", "post_norm",
+    __slots__ = ("layer", "tiles", "_rows", "_own", "_passing", "down_apart", "qkv_b", "in_norm", "post_norm",
                  # nf4 fragment packs (base, built once) + adapter fragment
                  # packs (rebuilt per refresh) for the fused nf4 GEMM path
                  "qkv_w4", "qkv_amax", "o_w4", "o_amax",
@@ -54,6 +55,7 @@ class LayerWeights:
         self.layer = layer
         self.tiles, self._rows = None, {}
         self._own = set()           # sites of one weight that is copied
+        self._passing = set()       # sites without room, until the next refresh
         self.down_apart = False     # tiles["down"] without its adapter
 
     @property
@@ -64,13 +66,28 @@ class LayerWeights:
                 "down": (mlp.down_proj,)}
 
     def rows(self, site: str) -> torch.Tensor:
+        if site not in self._rows and self._no_room(site):
+            self._passing.add(site)     # a capture does as its warm-up did
+            return _untiled(self.tiles[site], site == "gateup")
         if site not in self._rows:
             self._rows[site] = None
             self._fill_rows(site)
         return self._rows[site]
 
+    def _no_room(self, site: str) -> bool:
+        """Whether rows(site) must do without storage of its own: what was free
+        when the engine was made may be a learner's by the first large step."""
+        if site in self._passing:
+            return True
+        if (self.tiles is None or site == "base" or site == "down" and self.down_apart
+                or len(self.mods[site]) == 1 and self.mods[site][0].r == 0):
+            return False
+        tiles = self.tiles[site]
+        return not _room_for(tiles.numel() * tiles.element_size(), tiles.device)
+
     def refresh_rows(self) -> bool:
         """Whether rows lie elsewhere now: steps captured before are stale."""
+        self._passing.clear()
         return any([self._fill_rows(site) for site in self._rows])
 
     def _fill_rows(self, site: str) -> bool:

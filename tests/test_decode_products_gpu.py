@@ -245,6 +245,37 @@ def test_replaced_weight_reaches_row_major_storage():
     assert lw.rows("o") is held and torch.equal(held, at.o_proj.weight)
 
 
+def _cache_rows(eng, n):
+    """What a generation of n candidates leaves in the cache."""
+    from distrl_llm_amd.config import SamplingParams
+    eng.pool.allocator.reset()
+    for rows in (eng.pool.key, eng.pool.value):
+        rows.zero_()
+    eng.generate([[5, 6, 7, 8]], SamplingParams(max_tokens=4, temperature=0.0, n=n))
+    return torch.stack([eng.pool.key, eng.pool.value])
+
+
+@pytest.mark.parametrize("lora_r", [0, 8])
+def test_large_steps_on_a_full_card(monkeypatch, lora_r):
+    """Steps of more sequences than the streamed products take, the row-major
+    weights laid out within the step, twice through the captured graph: the
+    cache rows of an engine with room."""
+    from distrl_llm_amd.config import EngineConfig
+    from distrl_llm_amd.engine import Engine, weights
+    from distrl_llm_amd.models import CausalLM, get_spec
+    model = CausalLM(get_spec("small-qwen2"), lora_r=lora_r, dtype=torch.bfloat16,
+                     device=torch.device("cuda")).random_init(3).eval()
+    pools = []
+    for room in (True, False):
+        eng = Engine(model, EngineConfig(max_seq_length=64, num_kv_blocks=400, max_num_seqs=256))
+        assert eng.fused.tiled
+        with monkeypatch.context() as m:
+            m.setattr(weights, "_room_for", lambda size, device: room)
+            pools += [_cache_rows(eng, 161) for _ in range(2)][1:]
+        assert ("gateup" in eng.fused.layers[0]._rows) == room
+    assert torch.equal(*pools)
+
+
 @pytest.mark.parametrize("lora_r,four_bit", [(0, False), (8, True)])
 def test_replaced_weight_reaches_captured_steps(monkeypatch, lora_r, four_bit):
     """Row-major steps captured before a weight is another tensor: the cache
@@ -259,21 +290,12 @@ def test_replaced_weight_reaches_captured_steps(monkeypatch, lora_r, four_bit):
         model.quantize_nf4_()
     cfg = EngineConfig(max_seq_length=64, num_kv_blocks=32, max_num_seqs=8)
     eng = Engine(model, cfg)
-    before = _generate3(eng)
+    before = _cache_rows(eng, 3)
     for layer in model.model.layers:
         for lin in (layer.self_attn.o_proj, layer.mlp.down_proj):
             lin.weight.data = _rand(lin.weight.shape, 5, 0.05)
-    after = _generate3(eng)
-    assert not torch.equal(before, after) and torch.equal(after, _generate3(Engine(model, cfg)))
-
-
-def _generate3(eng):
-    from distrl_llm_amd.config import SamplingParams
-    eng.pool.allocator.reset()
-    for rows in (eng.pool.key, eng.pool.value):
-        rows.zero_()
-    eng.generate([[5, 6, 7, 8]], SamplingParams(max_tokens=4, temperature=0.0, n=3))
-    return torch.stack([eng.pool.key, eng.pool.value])
+    after = _cache_rows(eng, 3)
+    assert not torch.equal(before, after) and torch.equal(after, _cache_rows(Engine(model, cfg), 3))
 
 
 def test_no_tiles_without_room(monkeypatch):

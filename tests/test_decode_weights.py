@@ -43,3 +43,23 @@ def test_replaced_weight_is_left_as_it_was(kind):
         other.add_(1.0)
         fused.refresh()
         assert torch.equal(held, other.to(held.dtype))
+
+
+@pytest.mark.parametrize("lora_r", [0, 8])
+def test_rows_without_room_are_laid_out_for_the_call(monkeypatch, lora_r):
+    """No storage beside the tiles while the card is full; a capture does as its
+    warm-up did; the next refresh looks again."""
+    fused = weights.FusedWeights(_model(lora_r))
+    fused.refresh()
+    lw = fused.layers[0]
+    want = {site: torch.cat([weights._effective(m) for m in mods]) for site, mods in lw.mods.items()}
+    lw.tiles = {site: weights._tiled(w, site == "gateup") for site, w in want.items()}
+    kept = {"qkv", "gateup"} | ({"o", "down"} if lora_r else set())
+    for room in (False, True):
+        monkeypatch.setattr(weights, "_room_for", lambda size, device: room)
+        for site, w in want.items():
+            assert torch.equal(lw.rows(site), w)
+            assert (site in lw._rows) == (site not in kept)
+    fused.refresh()
+    for site, w in want.items():
+        assert torch.equal(lw.rows(site), w) and site in lw._rows
