@@ -386,6 +386,7 @@ class FusedWeights:
                 self.layers.append(lw)
             else:
                 lw = self.layers[li]
+                lw.layer = layer        # may be another one since
                 if lw.qkv_b is not None:
                     torch.cat([at.q_proj.bias, at.k_proj.bias,
                                at.v_proj.bias], out=lw.qkv_b)

@@ -63,3 +63,20 @@ def test_rows_without_room_are_laid_out_for_the_call(monkeypatch, lora_r):
     fused.refresh()
     for site, w in want.items():
         assert torch.equal(lw.rows(site), w) and site in lw._rows
+
+
+def test_replaced_layer_is_followed():
+    """Weights come from the model's layers as they are at the refresh."""
+    model, other = _model(), _model()
+    fused = weights.FusedWeights(model)
+    fused.refresh()
+    lw = fused.layers[0]
+    held = {site: lw.rows(site) for site in ("qkv", "o", "gateup", "down")}
+    for p in other.parameters():
+        p.data = _rand(p, 7)
+    model.model.layers[0] = other.model.layers[0]
+    fused.refresh()
+    for site, rows in held.items():
+        assert lw.rows(site) is rows
+        assert torch.equal(rows, torch.cat([m.weight for m in lw.mods[site]]))
+        assert lw.mods[site][0] in set(model.model.layers[0].modules())
