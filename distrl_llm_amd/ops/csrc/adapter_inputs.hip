@@ -256,7 +256,8 @@ bool adapter_inputs(const std::vector<AdapterInput>& jobs, bool k_major) {
       o.first[p + 1] = o.first[p] + (int)r;
       o.scale[p] = (float)j.scales[p];
     }
-    if (j.out.size(1) < o.first[o.n] || j.out.size(1) > 128) return false;
+    // columns are written by fours
+    if (j.out.size(1) < o.first[o.n] || j.out.size(1) > 128 || j.out.size(1) % 4 != 0) return false;
     if (rows > 1 && j.out.stride(0) < j.out.size(1)) return false;   // rows over one another
     o.cols = (int)j.out.size(1);
     o.total = o.first[o.n];

@@ -889,6 +889,9 @@ def test_adapter_input_refuses(ext):
     assert not ext.adapter_input(x, [m], [1.0], out[:1].expand(5, 8), False)
     assert not ext.adapter_input(x, [_rand((136, 64), 4)], [1.0], _rand((5, 136), 5), False)
     assert not ext.adapter_input(x.float(), [m], [1.0], out, False)
+    wide = torch.full((5, 16), 7.0, dtype=torch.bfloat16, device="cuda")
+    assert not ext.adapter_input(x, [m], [1.0], wide[:, :10], False)    # a part of four
+    assert (wide == 7).all()
 
 
 @pytest.mark.parametrize("N,K,ranks,pad", [((16, 8, 24), 64, (8, 8, 8), 24), ((40, 24), 136, (5, 12), 24),
