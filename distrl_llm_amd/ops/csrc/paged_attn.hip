@@ -525,12 +525,15 @@ torch::Tensor paged_decode_packed(torch::Tensor qkv, c10::optional<torch::Tensor
               qkv.scalar_type() == (parts ? at::kFloat : at::kBFloat16));
   const int N = qkv.size(-2), H = (int)n_heads, KV = kcache.size(2), D = kcache.size(3);
   TORCH_CHECK(qkv.size(-1) == (int64_t)(H + 2 * KV) * D && (parts || !bias));
-  TORCH_CHECK(kcache.is_contiguous() && vcache.is_contiguous() && vcache.sizes() == kcache.sizes() &&
-              kcache.scalar_type() == at::kBFloat16 && vcache.scalar_type() == at::kBFloat16);
+  TORCH_CHECK(vcache.sizes() == kcache.sizes() && kcache.scalar_type() == at::kBFloat16 &&
+              vcache.scalar_type() == at::kBFloat16);
+  // the kernel walks all of them as they lie on the GPU
+  for (const auto* t : {&kcache, &vcache, &positions, &slots, &inv_freq, &block_tables, &ctx_lens})
+    TORCH_CHECK(t->is_cuda() && t->is_contiguous(), "paged_decode_packed: device or layout");
   TORCH_CHECK(positions.scalar_type() == at::kInt && slots.scalar_type() == at::kLong &&
               positions.numel() == N && slots.numel() == N && inv_freq.numel() == D / 2 &&
               inv_freq.scalar_type() == at::kFloat);
-  TORCH_CHECK(block_tables.scalar_type() == at::kInt && block_tables.is_contiguous() &&
+  TORCH_CHECK(block_tables.scalar_type() == at::kInt && block_tables.dim() == 2 &&
               block_tables.size(0) == N && ctx_lens.scalar_type() == at::kInt &&
               ctx_lens.numel() == N);
   TORCH_CHECK(arrived.is_cuda() && arrived.scalar_type() == at::kInt && arrived.is_contiguous() &&

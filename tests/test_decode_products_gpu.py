@@ -151,6 +151,22 @@ def test_paged_decode_packed(ext, H, KV, D, N, longest, bs, S, bias, norms):
     assert got[0].isnan().any(-1).sum() == KV
 
 
+def test_paged_decode_packed_refuses(ext):
+    """Operands in host memory, and ones that do not lie on end."""
+    D, N = 64, 3
+    qkv, cache = _rand((N, 4 * D), 1), [_rand((4, 16, 1, D), 2 + i) for i in range(2)]
+    args = [torch.zeros(N, dtype=torch.int32, device="cuda"),
+            torch.zeros(N, dtype=torch.long, device="cuda"), torch.ones(D // 2, device="cuda"),
+            *cache, torch.zeros(N, 2, dtype=torch.int32, device="cuda"),
+            torch.ones(N, dtype=torch.int32, device="cuda"),
+            torch.zeros(N, dtype=torch.int32, device="cuda")]
+    ext.paged_decode_packed(qkv, None, *args, 2, 0.125)
+    for i, t in enumerate(args):
+        for bad in (t.cpu(), t[:1].expand(t.shape)):
+            with pytest.raises(RuntimeError):
+                ext.paged_decode_packed(qkv, None, *args[:i], bad, *args[i + 1:], 2, 0.125)
+
+
 @pytest.mark.parametrize("H,KV,D,N,cs", [(28, 4, 128, 16, 4), (28, 4, 128, 32, 2), (14, 2, 64, 32, 4)])
 @pytest.mark.parametrize("S", [0, 2])
 def test_paged_decode_packed_behind_a_slice_end(ext, monkeypatch, H, KV, D, N, cs, S):
