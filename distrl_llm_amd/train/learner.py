@@ -128,7 +128,7 @@ class Learner:
                     loss_scale: float) -> torch.Tensor:
         takes_rows = getattr(self.model, "takes_rows", None)
         if (takes_rows is not None and takes_rows()
-                and type(self)._encode_batch is Learner._encode_batch):
+                and getattr(self._encode_batch, "__func__", None) is Learner._encode_batch):
             enc = self._encode(problems, answers)
             if any(a for _, a in enc):
                 return self._rows_loss(enc, rewards, loss_scale)

@@ -89,6 +89,24 @@ def test_degenerate_batch_skipped():
         assert p.grad is None or p.grad.abs().max() == 0
 
 
+def test_replaced_batch_layout_is_used():
+    """A learner whose batch is laid out by another function gets that batch also where the model takes rows without padding."""
+    learner = _make_learner()
+    learner.model.takes_rows = lambda: True
+    learner._rows_loss = lambda *args: (_ for _ in ()).throw(AssertionError("rows"))
+    calls, layout = [], learner._encode_batch
+
+    def own(problems, answers):
+        calls.append(len(problems))
+        return layout(problems, answers)
+
+    with pytest.raises(AssertionError, match="rows"):
+        learner.accumulate_gradients(["1+1="], ["2"], [1.0])
+    learner._encode_batch = own
+    learner.accumulate_gradients(["1+1="], ["2"], [1.0])
+    assert calls == [1]
+
+
 def test_adam8bit_tracks_fp32_adam():
     torch.manual_seed(0)
     p1 = torch.nn.Parameter(torch.randn(1000))
