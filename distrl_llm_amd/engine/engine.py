@@ -555,10 +555,11 @@ class Engine:
             # waves' cached graphs pointing at freed memory (garbage u ->
             # NaN logits -> the sampler degenerates to token 0; surfaced
             # at batch 30 x 16 where pool pressure forces multiple wave
-            # sizes per round). Allocate once at max_num_seqs and slice.
+            # sizes per round). Allocate once at max_num_seqs, and what a
+            # wave is padded by, and slice.
             if getattr(self, "_u_pool_off", None) != off:
                 self._u_pool = torch.zeros(
-                    len(lws), self.cfg.max_num_seqs, off,
+                    len(lws), self.cfg.max_num_seqs + 16, off,
                     dtype=torch.float32, device=input_ids.device)
                 self._u_pool_off = off
             u_pool = self._u_pool[:, :N_batch, :]

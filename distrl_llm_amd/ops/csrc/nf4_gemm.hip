@@ -465,6 +465,7 @@ torch::Tensor nf4_gemm(torch::Tensor x, torch::Tensor w4f, torch::Tensor amaxf,
   if (has_lora) {
     TORCH_CHECK(r % 32 == 0 && bfrag.has_value());
     TORCH_CHECK(u->scalar_type() == at::kFloat && u->stride(1) == 1);
+    TORCH_CHECK(u->dim() == 2 && u->size(0) >= M && u->size(1) >= r, "nf4_gemm: rows of u");
     u_stride = u->stride(0);
   }
 
@@ -571,6 +572,7 @@ void lora_u(torch::Tensor x, torch::Tensor afrag, torch::Tensor u,
   TORCH_CHECK(u.scalar_type() == at::kFloat && u.stride(1) == 1);
   const int M = x.size(0), K = x.size(1);
   TORCH_CHECK(r % 16 == 0 && K % 32 == 0);
+  TORCH_CHECK(u.dim() == 2 && u.size(0) >= M && u.size(1) >= r, "lora_u: rows of u");
   // caller zeroes u (batched across all sites/layers per step)
   dim3 grid((M + 15) / 16, r / 16, ksplit), block(64);
   hipLaunchKernelGGL(lora_u_kernel, grid, block, 0,

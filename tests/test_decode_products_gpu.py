@@ -261,14 +261,37 @@ def test_replaced_weight_reaches_row_major_storage():
     assert lw.rows("o") is held and torch.equal(held, at.o_proj.weight)
 
 
-def _cache_rows(eng, n):
+def _cache_rows(eng, n, tokens=4):
     """What a generation of n candidates leaves in the cache."""
     from distrl_llm_amd.config import SamplingParams
     eng.pool.allocator.reset()
     for rows in (eng.pool.key, eng.pool.value):
         rows.zero_()
-    eng.generate([[5, 6, 7, 8]], SamplingParams(max_tokens=4, temperature=0.0, n=n))
+    eng.generate([[5, 6, 7, 8]], SamplingParams(max_tokens=tokens, temperature=0.0, n=n))
     return torch.stack([eng.pool.key, eng.pool.value])
+
+
+def test_four_bit_waves_are_padded_within_their_pool(monkeypatch):
+    """As many sequences as the engine takes, a wave padded beyond them: the
+    adapter inputs of the padding stay out of the next layer's. Against an
+    engine with room (atomic fp32 sums in another order: 2 %)."""
+    from distrl_llm_amd.config import EngineConfig
+    from distrl_llm_amd.engine import Engine
+    from distrl_llm_amd.models import CausalLM, get_spec
+    monkeypatch.setenv("DISTRL_DECODE_NF4", "1")
+    model = CausalLM(get_spec("small-qwen2"), lora_r=8, dtype=torch.bfloat16,
+                     device=torch.device("cuda")).random_init(3).eval()
+    with torch.no_grad():
+        for name, p in model.named_parameters():
+            if name.endswith("lora_B"):
+                p.copy_(_rand(p.shape, 7, 0.05))
+    model.quantize_nf4_()
+    pools = []
+    for most in (20, 64):
+        eng = Engine(model, EngineConfig(max_seq_length=64, num_kv_blocks=64, max_num_seqs=most))
+        assert eng.fused.nf4
+        pools.append(_cache_rows(eng, 20, 2))
+    assert _rel(*pools) < 0.02
 
 
 @pytest.mark.parametrize("lora_r", [0, 8])
