@@ -6,11 +6,12 @@ between rounds, so the engine folds it once per weight-sync:
 
     W_eff = W_base + scale * (B @ A)
 
-and concatenates the per-site projections — one qkv GEMM (q|k|v) and one
-gate|up GEMM per layer — halving GEMM launches and giving hipBLASLt fatter
-N at decode's skinny M. A refresh writes each projection's merged weight
-straight into the packed storage, one kernel a projection, once per
-generation round.
+and lays the projections of a site (q|k|v, gate|up) out as one matrix, in the
+tiles that the decode products read (ops/csrc/skinny_gemm.hip up to 16 rows,
+stream_gemm.hip up to 160); row-major beside them only for what still goes to
+the library: prompts of models without an adapter, and larger steps. A refresh
+writes each projection's merged weight straight into its tiles, one kernel a
+projection, once per generation round.
 
 Replaces the reference's per-generate adapter hot-swap into vLLM
 (``load_lora`` inside every fast_generate, reference
@@ -124,11 +125,6 @@ class LayerWeights:
         out.set_(w)
         return True
 
-    qkv_w = property(lambda self: self.rows("qkv"))
-    o_w = property(lambda self: self.rows("o"))
-    gateup_w = property(lambda self: self.rows("gateup"))
-    down_w = property(lambda self: self.rows("down"))
-
 
 def _tiled(w: torch.Tensor, glu: bool = False) -> torch.Tensor:
     """(N, K) row-major -> tiles of 32 rows x 16 of K, [K half][row][8
@@ -237,8 +233,8 @@ class FusedWeights:
                 "unavailable for this shape — cannot fall back to merged")
         # hybrid: even when the merged-bf16 cache wins overall, the fused
         # nf4 kernel BEATS hipBLASLt on the deep-K down-projection
-        # (61+13 vs 80 us/layer at decode batch 160 — profiles/r02) —
-        # run just that site through it
+        # (61+13 vs 80 us/layer at decode batch 160) — steps that the
+        # products on tiles do not take run just that site through it
         self.hybrid_down = bool(
             (not self.nf4) and q0.weight_nf4 is not None
             and q0.weight.is_cuda and shapes_ok

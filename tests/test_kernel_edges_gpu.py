@@ -645,7 +645,7 @@ def test_packed_prefill_matches_modules(name, lora_r, four_bit):
     if lora_r:
         w = w + at.k_proj.scale * at.k_proj.lora_B.double() @ at.k_proj.lora_A.double()
     q = model.spec.q_size
-    assert _rel(eng.fused.layers[1].qkv_w[q:q + model.spec.kv_size], w) < 2.0 ** -8
+    assert _rel(eng.fused.layers[1].rows("qkv")[q:q + model.spec.kv_size], w) < 2.0 ** -8
 
 
 def test_packed_prefill_after_a_changed_bias():
