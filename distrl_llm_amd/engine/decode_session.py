@@ -6,13 +6,13 @@ per-sequence state (tokens, positions, context lengths, block tables,
 finished mask, output buffer, sampler seed/step counters) in device
 tensors, pre-allocates each sequence's worst-case KV blocks up front (the
 admission control already reserved them), and expresses one decode step as
-a fixed tensor program over those buffers — embed -> 28 layers (HIP
-rmsnorm / rope / kv-scatter / paged-attention + hipBLASLt projections, or
-skinny products for few sequences) ->
-LM head -> fused sampler -> in-graph state advance. That program is
-captured once into a hipGraph and replayed per token (SURVEY.md §2.4-A:
-"hipGraph-captured decode step" north star); the host loop is just
-graph.replay() with one finished-mask sync per chunk of steps.
+a fixed tensor program over those buffers — slots of the new tokens -> embed
+-> 28 layers (products on weights in tiles, or the library's for many
+sequences; one kernel for rotation, cache write and paged attention; norms
+with the residual sum) -> LM head -> fused sampler -> state advance in one
+launch. That program is captured once into a hipGraph and replayed per token;
+the host loop is just graph.replay() with one finished-mask sync per chunk of
+steps.
 
 Sampling randomness inside the graph: the fused sampler hashes
 (per-seq seed, device step counter), and the counter increments in-graph,
@@ -230,7 +230,7 @@ class DecodeSession:
 class CachedDecodeSession(DecodeSession):
     """A DecodeSession whose device buffers (and captured hipGraph) are
     owned by a SessionCache and REUSED across generation waves
-    (docs/ROADMAP.md #4: capture cost ~0.2-0.4 s/round otherwise).
+    (capture costs ~0.2-0.4 s a round otherwise).
 
     Shapes are fixed at worst case for the cache key — N padded up, block
     tables at blocks_for(max_seq_length), out_buf at sp.max_tokens — so a

@@ -458,7 +458,7 @@ class Engine:
     def _make_session(self, running, sp, eos_token_id):
         """DecodeSession per wave, with cached state buffers + captured
         hipGraph keyed on (padded N, params) reused across waves — saves
-        the ~0.2-0.4 s/round re-capture cost (docs/ROADMAP.md #4).
+        the ~0.2-0.4 s/round re-capture cost.
         GPU-validated: cached-vs-fresh greedy equality
         (tests/test_engine_gpu.py::test_session_cache_vs_fresh_identical)
         and identical fuzz behavior over 15 randomized trials.
@@ -484,9 +484,9 @@ class Engine:
 
         GPU path: merged-LoRA fused weights (one qkv and one gate|up product
         a layer), rotation with the cache write, strided-q paged attention,
-        residual sum with the norm. Up to 16 sequences run on skinny
-        products, up to 160 on streamed ones, both on weights in tiles; more
-        on the library's.
+        residual sum with the norm. Up to 16 sequences, 32 of a small model,
+        run on skinny products, up to 160 on streamed ones, both on weights
+        in tiles; more on the library's.
         """
         if self.device.type == "cuda":
             return self._decode_forward_fused(input_ids, positions,
@@ -673,10 +673,13 @@ class Engine:
 
     def _skinny(self, n: int) -> bool:
         """Whether a decode step of n sequences runs on the skinny products:
-        every one of a layer's four fits, weights in bf16. At 32 rows the
-        library's are as fast again unless the model is small (a layer with
-        its norms and activation, 0.5B: 42 us against 59; 1.5B: 73 against
-        71; at 8 rows 4B: 80 against 104)."""
+        every one of a layer's four fits, weights in bf16. Drawn against the
+        library's (a layer with its norms and activation, us: 32 rows 0.5B 42
+        against 59, 1.5B 73 against 71; 8 rows 4B 80 against 104), where it
+        still holds for weights that do not lie in tiles. From tiles the
+        streamed products are the faster at 17 to 32 rows of a small model
+        too: 64 tokens of 17, 24 and 32 sequences, 0.5B, 90, 91 and 92 ms
+        here, 74, 75 and 76 streamed."""
         from ..ops.build import get_extension
         s, fits = self.spec, get_extension().skinny_gemm_takes
         return (self.dtype == torch.bfloat16
