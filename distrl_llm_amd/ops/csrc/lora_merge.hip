@@ -18,6 +18,9 @@
 // y += scale * u A. r 32, rows x columns, the library's addmm against this, us:
 // 128 x 896 3.9 and 5.3, 2408 x 3584 10 and 12, 2408 x 18944 41 and 40, 4816 x 3584
 // 160 and 19; the library's call costs 19 us of host time and this one 4.
+// And it joins adapter, bias and residual to an fp32 product of large weights, rounded
+// once (the learner's short micro-batches): 308 x 18944 11.8 us, 2008 x 18944 54 us,
+// 4.2 TB/s.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
