@@ -5,7 +5,9 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
+#include <atomic>
 #include <cstdint>
+#include <random>
 
 #define WAVE 64
 #define DEV_INLINE __device__ __forceinline__
@@ -123,6 +125,29 @@ DEV_INLINE uint64_t splitmix64(uint64_t x) {
   x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
   return x ^ (x >> 31);
 }
+
+// ---- arrival of workgroups ----
+// A mark that no other launch of this process has; neither half is zero.
+inline unsigned long long arrival_tag() {
+  static std::atomic<unsigned long long> calls{(unsigned long long)std::random_device{}() << 32};
+  unsigned long long x = ++calls * 0x9E3779B97F4A7C15ull;
+  x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+  return (x ^ (x >> 31)) | 0x100000001ull;
+}
+
+// What workgroups of one launch pass to each other goes past the caches of their XCDs,
+// so that a wait is all it takes to order it: a fence, which writes a whole L2 back and
+// empties it, took 50 us of 1184 workgroups that drew a token and 9 without.
+template <typename T>
+DEV_INLINE void store_through(T* p, T x) {
+  __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+DEV_INLINE T load_through(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Until this wave's stores and atomics have arrived.
+DEV_INLINE void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 #define HIP_CHECK_LAST()                                                     \
   do {                                                                       \

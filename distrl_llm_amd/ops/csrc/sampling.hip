@@ -7,23 +7,31 @@
 // cumulative probability reaches top_p (or the count top_k). The draw is the
 // argmax of z - log(-log u) over the kept set, u a counter-based hash of
 // (seed of the row, step, element): the step is read from device memory, so a
-// replayed graph draws anew. Slices add their probabilities up as integers of
-// 2^-32, whose sum does not hang on their order: a call repeats itself exactly.
-// How a row was split over workgroups (by the number of rows) shows only where
-// a cumulative probability lies within fp32 rounding of top_p.
+// replayed graph draws anew. What workgroups add up meets as integers of 2^-32,
+// whose sum does not hang on their order: a call repeats itself exactly. How a
+// row was split over workgroups (by the number of rows) shows only where a
+// cumulative probability lies within fp32 rounding of top_p.
 //
-// A row is cut into slices, so that any number of rows fills the chip: a
-// maximum pass; with a threshold two histogram passes, first over 32 groups of
-// 32 bins and then over the bins of the group in which the threshold falls;
-// and the draw, whose last slice of a row writes the token. A thread adds into
-// histogram columns of its own, so nothing collides and no atomics are needed:
-// LDS float atomics into 1024 shared bins took ~3 clocks a lane (124 us for
-// 160 rows of 152064), the two passes take 44 us.
-// An element that is kept costs ~330 cycles of hashing a wave, so sparse ones
-// are gathered into full waves first. 160 rows of 152064 at top_p 0.95: 284 us
-// as eight launches with one serial thread a row for the threshold, 95 us now
-// (draw 46, histograms 44, maximum 9), bound by the draw's integer products;
-// one row of 151936 without a threshold 24.6 -> 11.3 us, bound by two launches.
+// A row is cut into slices, so that any number of rows fills the chip, and a
+// workgroup holds its slice in registers: all its loads are in flight at once
+// and every further look at an element is free of memory.
+//  * With a threshold, two launches. The first finds a slice's maximum and the
+//    probability (count) in each of 23 steps below it. The second knows from
+//    all slices of the row to within some steps where the threshold lies: it sums
+//    and draws what lies above that window, keeps sum and best draw of
+//    each of the window's bins apart, and the row's last slice to end finds the
+//    threshold's bin and the best draw down to it.
+//  * Without one, one launch: a slice draws relative to its own maximum, and
+//    leaves out what the largest possible draw would not lift over the best of
+//    its threads' own maxima.
+// A step's probability is added up in an LDS column of the thread's own, so nothing
+// collides (LDS float atomics took ten times as long); an element that is drawn costs
+// ~330 cycles of hashing a wave, so sparse ones are gathered into full waves first.
+// 160 rows of 151936, us, against four launches that each read all logits: top_p 0.95 of
+// peaked logits 84 -> 47, of a language model's 79 -> 38, of flat ones, where most is
+// drawn, 102 -> 102; top_k 50 75 -> 41; no threshold, a model's logits 40 -> 22. One row
+// without a threshold 11.3 -> 9.5. Bound by vector work: ~14 instructions an element for
+// the steps (20 us), then the hash of what lies above the window's end.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
@@ -36,7 +44,7 @@ constexpr int NBINS = 1024;
 constexpr float ZRANGE = 32.f;        // z below -32 has no probability left
 // u is at most 1 - 2^-24 and at least 2^-24: a draw adds between -2.82 and
 // 16.64 to z. The row maximum (z = 0) reaches -2.82, nothing below -19.46 does.
-constexpr float ZDRAW = -19.5f;
+constexpr float ZDRAW = -19.5f, MOST = 16.7f;
 
 DEV_INLINE float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }
 DEV_INLINE float bf_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
@@ -87,341 +95,608 @@ DEV_INLINE float gumbel_key(uint64_t seed, int idx, float z) {
   return z - LN2 * __builtin_amdgcn_logf(-LN2 * __builtin_amdgcn_logf(u));
 }
 
-// Gathers the elements that a wave keeps and draws 64 at a time.
-struct DrawQueue {
-  uint2* q;             // 128 entries of this wave: index, z
-  uint64_t seed;
-  int head = 0, count = 0;
-  Best best;
-
-  DEV_INLINE void draw(int n) {
-    __builtin_amdgcn_wave_barrier();
-    const int lane = threadIdx.x & (WAVE - 1);
-    if (lane < n) {
-      const uint2 e = q[(head + lane) & 127];
-      best.offer(gumbel_key(seed, (int)e.x, __uint_as_float(e.y)), (int)e.x);
-    }
-    head += n;
-    count -= n;
-    __builtin_amdgcn_wave_barrier();
-  }
-  // Every lane of the wave calls it. Gathering costs a fifth of a draw: a wave
-  // that is mostly kept draws at once.
-  DEV_INLINE void push(bool keep, int idx, float z) {
-    const uint64_t mask = __ballot(keep);
-    if (mask == 0) return;
-    if (__popcll(mask) >= 48) {
-      if (keep) best.offer(gumbel_key(seed, idx, z), idx);
-      return;
-    }
-    if (keep) {
-      const int at = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                               __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
-      q[(head + count + at) & 127] = uint2{(uint32_t)idx, __float_as_uint(z)};
-    }
-    count += __popcll(mask);
-    if (count >= WAVE) draw(WAVE);
-  }
-};
-
-constexpr int GROUPS = 32, IN_GROUP = NBINS / GROUPS;
-
-// Where a running sum over 32 bins (lanes 0..31 of every wave) reaches the
-// limit: {bin, sum before it}; the last bin if it never does.
+// Sum over lanes 0..31 (and 32..63) up to this one.
 template <typename T>
-struct Crossing { int bin; T before; };
-
-template <typename T>
-DEV_INLINE Crossing<T> crossing(T x, T start, T limit) {
-  const int lane = threadIdx.x & (WAVE - 1);
-  T cum = x;
+DEV_INLINE T upto32(T x) {
   #pragma unroll
   for (int off = 1; off < 32; off <<= 1) {
-    const T y = __shfl_up(cum, off, WAVE);
-    if ((lane & 31) >= off) cum += y;
-  }
-  const uint64_t mask = __ballot(start + cum >= limit) & 0xffffffffull;
-  const int bin = mask ? __ffsll((unsigned long long)mask) - 1 : 31;
-  const T before = __shfl(cum, max(bin - 1, 0), WAVE);
-  return {bin, start + (bin ? before : T(0))};
-}
-
-DEV_INLINE float wave_total(float x) {   // lanes 0..31, in their order
-  #pragma unroll
-  for (int off = 1; off < 32; off <<= 1) {
-    const float y = __shfl_up(x, off, WAVE);
+    const T y = __shfl_up(x, off, WAVE);
     if ((threadIdx.x & 31) >= off) x += y;
   }
-  return __shfl(x, 31, WAVE);
+  return x;
 }
 
-// Sums of a row's groups and of the bins of the crossing groups, in global
-// memory: probability in units of 2^-32 (a row's is below V < 2^31) and count.
-struct Hist {
-  unsigned long long *group_p, *bin_p;     // (B, 32) each
-  int *group_c, *bin_c;
-};
-
-DEV_INLINE float prob(unsigned long long x) { return (float)x * 0x1p-32f; }
-
-// The row's crossing groups, from the group sums: every wave computes them.
-template <bool BY_P, bool BY_K>
-DEV_INLINE void crossing_groups(const Hist& h, int row, float top_p, int top_k,
-                                Crossing<float>& cp, Crossing<int>& ck, float& target) {
-  const int at = row * GROUPS + (threadIdx.x & 31);
-  if (BY_P) {
-    const float x = prob(h.group_p[at]);
-    target = top_p * wave_total(x);
-    cp = crossing(x, 0.f, target);
-  }
-  if (BY_K) ck = crossing(h.group_c[at], 0, top_k);
+// key and index in one word whose order is that of Best; 0: nothing kept
+DEV_INLINE unsigned long long word_of(const Best& b) {
+  uint32_t o = __float_as_uint(b.key);
+  o = (o >> 31) ? ~o : o | 0x80000000u;
+  return b.idx == 0x7fffffff ? 0ull
+                             : ((unsigned long long)o << 32) | (0xffffffffu - (uint32_t)b.idx);
 }
-
+DEV_INLINE int index_of(unsigned long long w) { return (int)(0xffffffffu - (uint32_t)w); }
 // ----------------------------------------------------------------- slices
-// Eight elements a thread of the block's next 2048: 16-byte loads where rows
-// are aligned for them, else one element a lane. -inf past the end.
+constexpr int CHUNKS = 10, CHUNK = 2048;       // of a slice: 80 elements a thread
+constexpr int SLICE = CHUNKS * CHUNK;
+
+// A slice of a row in a workgroup's registers, -inf past its end. 16-byte loads
+// where rows are aligned for them (eight elements on end a thread), else one
+// element a lane.
 template <typename T, bool VEC>
-DEV_INLINE void load8(const T* lr, int base, int i1, float (&x)[8], int (&id)[8]) {
-  constexpr bool BF16 = std::is_same<T, __hip_bfloat16>::value;
-  #pragma unroll
-  for (int k = 0; k < 8; ++k) id[k] = VEC ? base + threadIdx.x * 8 + k : base + k * 256 + threadIdx.x;
-  if constexpr (VEC) {
-    const int at = min(id[0], i1 - 8);
-    if constexpr (BF16) {
-      const u32x4 d = *reinterpret_cast<const u32x4*>(lr + at);
-      #pragma unroll
-      for (int w = 0; w < 4; ++w) { x[2 * w] = bf_lo(d[w]); x[2 * w + 1] = bf_hi(d[w]); }
-    } else {
-      #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const u32x4 d = *reinterpret_cast<const u32x4*>(lr + at + 4 * k);
+struct Slice {
+  static constexpr bool BF16 = std::is_same<T, __hip_bfloat16>::value;
+  static constexpr uint32_t NONE = BF16 ? 0xff80ff80u : 0xff800000u;   // -inf
+  uint32_t raw[CHUNKS][BF16 ? 4 : 8];
+
+  static DEV_INLINE int at(int c, int k) {      // element of the slice
+    return VEC ? c * CHUNK + (int)threadIdx.x * 8 + k : c * CHUNK + k * 256 + (int)threadIdx.x;
+  }
+  DEV_INLINE void load(const T* p, int n) {
+    #pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      if (c * CHUNK >= n) continue;
+      if constexpr (VEC) {
+        const T* q = p + min(at(c, 0), n - 8);
         #pragma unroll
-        for (int w = 0; w < 4; ++w) x[4 * k + w] = __uint_as_float(d[w]);
+        for (int v = 0; v < (BF16 ? 1 : 2); ++v) {
+          const u32x4 d = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(q) + 16 * v);
+          #pragma unroll
+          for (int w = 0; w < 4; ++w) raw[c][4 * v + w] = d[w];
+        }
+      } else {
+        const uint16_t* h = reinterpret_cast<const uint16_t*>(p);
+        const uint32_t* f = reinterpret_cast<const uint32_t*>(p);
+        #pragma unroll
+        for (int w = 0; w < (BF16 ? 4 : 8); ++w) {
+          if constexpr (BF16) {
+            const uint32_t lo = h[min(at(c, 2 * w), n - 1)], hi = h[min(at(c, 2 * w + 1), n - 1)];
+            raw[c][w] = lo | (hi << 16);
+          } else {
+            raw[c][w] = f[min(at(c, w), n - 1)];
+          }
+        }
       }
     }
-  } else {
     #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int at = min(id[k], i1 - 1);
-      if constexpr (BF16) x[k] = bf2f(lr[at]); else x[k] = lr[at];
+    for (int c = 0; c < CHUNKS; ++c) {
+      if ((c + 1) * CHUNK <= n || c * CHUNK >= n) continue;   // a whole chunk, or none
+      #pragma unroll
+      for (int w = 0; w < (BF16 ? 4 : 8); ++w) {
+        if constexpr (VEC) {
+          if (at(c, 0) >= n) raw[c][w] = NONE;
+        } else if constexpr (BF16) {
+          if (at(c, 2 * w) >= n) raw[c][w] = NONE;
+          else if (at(c, 2 * w + 1) >= n) raw[c][w] = (raw[c][w] & 0xffffu) | (NONE << 16);
+        } else {
+          if (at(c, w) >= n) raw[c][w] = NONE;
+        }
+      }
     }
   }
-  #pragma unroll
-  for (int k = 0; k < 8; ++k)
-    if (id[k] >= i1) x[k] = __uint_as_float(0xff800000u);
-}
+  DEV_INLINE float get(int c, int k) const {
+    if constexpr (BF16) return k & 1 ? bf_hi(raw[c][k / 2]) : bf_lo(raw[c][k / 2]);
+    else return __uint_as_float(raw[c][k]);
+  }
+  template <typename F>
+  DEV_INLINE void each(int n, F f) const {      // f(element of the slice, value)
+    #pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      if (c * CHUNK >= n) continue;
+      #pragma unroll
+      for (int k = 0; k < 8; ++k) f(at(c, k), get(c, k));
+    }
+  }
+};
 
-DEV_INLINE float row_max(const float* ms, int row, int S) {   // S <= 64
-  return wave_max(ms[row * S + min((int)(threadIdx.x & (WAVE - 1)), S - 1)]);
-}
-
-// Slice maxima; a row's first slice also clears what the later passes add to.
+// Gathers what the lanes of a wave keep of their elements, two chunks at a time, and
+// hands it on 64 at a time: f(element of the slice, value), a lane each.
 template <typename T, bool VEC>
-__global__ __launch_bounds__(256)
-void slice_max_kernel(const T* __restrict__ logits, int V, int per, float* __restrict__ ms,
-                      unsigned long long* __restrict__ top, int* __restrict__ done, Hist h) {
-  __shared__ float red[16];
-  const int row = blockIdx.x, sl = blockIdx.y;
-  const T* lr = logits + (int64_t)row * V;
-  const int i1 = min(V, (sl + 1) * per);
-  float m = -1e30f, x[8];
-  int id[8];
-  for (int base = sl * per; base < i1; base += 2048) {
-    load8<T, VEC>(lr, base, i1, x, id);
-    #pragma unroll
-    for (int k = 0; k < 8; ++k) m = fmaxf(m, x[k]);
-  }
-  m = block_max(m, red);
-  if (threadIdx.x == 0) ms[row * gridDim.y + sl] = m;
-  if (sl == 0) {
-    if (threadIdx.x == 0) { top[row] = 0ull; done[row] = 0; }
-    if (h.group_p && threadIdx.x < 32) {
-      const int at = row * 32 + threadIdx.x;
-      h.group_p[at] = h.bin_p[at] = 0ull;
-      h.group_c[at] = h.bin_c[at] = 0;
-    }
-  }
-}
+struct Gather {
+  using Entry = std::conditional_t<Slice<T, VEC>::BF16, uint32_t, unsigned long long>;
+  static constexpr int ROOM = 2 * 8 * WAVE + WAVE;
+  Entry* q;                                     // ROOM entries of this wave
+  int count = 0;
 
-// FINE false: sums of the 32 groups of bins. FINE true: sums of the bins of the
-// group where the probability (count) crosses its limit.
-template <typename T, bool VEC, bool BY_P, bool BY_K, bool FINE>
-__global__ __launch_bounds__(256)
-void slice_hist_kernel(const T* __restrict__ logits, int V, int per, float inv_temp, float top_p,
-                       int top_k, const float* __restrict__ ms, Hist h) {
-  __shared__ float hp[BY_P ? 32 * 256 : 1];     // [bin][thread]
-  __shared__ int hc[BY_K ? 32 * 256 : 1];
-  const int row = blockIdx.x, sl = blockIdx.y, tid = threadIdx.x;
-  const T* lr = logits + (int64_t)row * V;
-  const int i1 = min(V, (sl + 1) * per);
-  const float m = row_max(ms, row, gridDim.y);
-  int gp = 0, gc = 0;
-  if (FINE) {
-    Crossing<float> cp;
-    Crossing<int> ck;
-    float target;
-    crossing_groups<BY_P, BY_K>(h, row, top_p, top_k, cp, ck, target);
-    if (BY_P) gp = cp.bin;
-    if (BY_K) gc = ck.bin;
+  template <typename F>
+  DEV_INLINE void take(int at, F& f) {
+    const Entry e = q[at];
+    if constexpr (Slice<T, VEC>::BF16)
+      f((int)(e & 0xffffu), __uint_as_float(e & 0xffff0000u));
+    else
+      f((int)(e >> 32), __uint_as_float((uint32_t)e));
   }
-  for (int i = 0; i < 32; ++i) {
-    if (BY_P) hp[i * 256 + tid] = 0.f;
-    if (BY_K) hc[i * 256 + tid] = 0;
-  }
-  float x[8], next[8];
-  int id[8], next_id[8];
-  if (sl * per < i1) load8<T, VEC>(lr, sl * per, i1, next, next_id);
-  for (int base = sl * per; base < i1; base += 2048) {
+  // Every lane of the wave calls it; keep(value).
+  template <typename K, typename F>
+  DEV_INLINE void run(const Slice<T, VEC>& s, int n, K keep, F f) {
+    const int lane = threadIdx.x & (WAVE - 1);
     #pragma unroll
-    for (int k = 0; k < 8; ++k) { x[k] = next[k]; id[k] = next_id[k]; }
-    load8<T, VEC>(lr, base + 2048, i1, next, next_id);   // past the end: the last eight again
-    #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      // without branches: what does not count adds zero
-      const float z = (x[k] - m) * inv_temp;
-      const int b = bin_of(z), g = b / IN_GROUP, at = (FINE ? b % IN_GROUP : g) * 256 + tid;
-      const bool in = z > -ZRANGE;
-      if (BY_P) hp[at] += in && (!FINE || g == gp) ? __expf(z) : 0.f;
-      if (BY_K) hc[at] += in && (!FINE || g == gc) ? 1 : 0;
+    for (int c0 = 0; c0 < CHUNKS; c0 += 2) {
+      if (c0 * CHUNK >= n) continue;
+      const int two = (c0 + 1) * CHUNK < n ? 2 : 1;
+      int mine = 0;
+      #pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        if (c >= two) continue;
+        #pragma unroll
+        for (int k = 0; k < 8; ++k) mine += keep(s.get(c0 + c, k)) ? 1 : 0;
+      }
+      if (__ballot(mine > 0) == 0) continue;
+      int upto = mine;
+      #pragma unroll
+      for (int off = 1; off < WAVE; off <<= 1) {
+        const int y = __shfl_up(upto, off, WAVE);
+        if (lane >= off) upto += y;
+      }
+      int to = count + upto - mine;
+      count += __shfl(upto, WAVE - 1, WAVE);
+      #pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        if (c >= two) continue;
+        #pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const float x = s.get(c0 + c, k);
+          if (keep(x)) {
+            const uint32_t id = s.at(c0 + c, k), bits = __float_as_uint(x);
+            if constexpr (Slice<T, VEC>::BF16) q[to] = bits | id;     // SLICE < 2^16
+            else q[to] = ((unsigned long long)id << 32) | bits;
+            ++to;
+          }
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+      int done = 0;
+      for (; done + WAVE <= count; done += WAVE) take(done + lane, f);
+      count -= done;
+      if (done > 0) {
+        Entry e{};
+        if (lane < count) e = q[done + lane];
+        __builtin_amdgcn_wave_barrier();
+        if (lane < count) q[lane] = e;
+      }
+      __builtin_amdgcn_wave_barrier();
     }
+    if (lane < count) take(lane, f);
+    count = 0;
+  }
+};
+
+// The best of a workgroup's lanes, in thread 0.
+DEV_INLINE void over_block(Best& b, float* fpart, int* ipart) {
+  b.over_wave();
+  if ((threadIdx.x & (WAVE - 1)) == 0) {
+    fpart[threadIdx.x / WAVE] = b.key;
+    ipart[threadIdx.x / WAVE] = b.idx;
   }
   __syncthreads();
+  if (threadIdx.x == 0)
+    for (int w = 1; w < 4; ++w) b.offer(fpart[w], ipart[w]);
+}
+
+// --------------------------------------------------------- no threshold
+// What a slice passes on to the row's last slice to end, each word with the launch's
+// mark above it: its maximum, its best key relative to that, that key's element. A
+// mark's 32 bits might lie in old memory by chance, but not in all three.
+enum { TOP = 0, KEY = 1, ELEMENT = 2, WORDS = 3 };
+
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256)
+void draw_kernel(const T* __restrict__ logits, int V, int per, float inv_temp,
+                 const int64_t* __restrict__ seeds, const int64_t* __restrict__ step,
+                 unsigned long long* __restrict__ found, uint32_t mark, int64_t* __restrict__ out) {
+  __shared__ typename Gather<T, VEC>::Entry queue[4 * Gather<T, VEC>::ROOM];
+  __shared__ float red[16], fpart[4];
+  __shared__ int ipart[4];
+  const int row = blockIdx.x, sl = blockIdx.y, S = gridDim.y, tid = threadIdx.x;
+  const int i0 = sl * per, n = min(V - i0, per);
+  Slice<T, VEC> s;
+  s.load(logits + (int64_t)row * V + i0, n);
+  const uint64_t seed = row_seed(seeds, step, row);
+  float own = -1e30f;
+  int own_at = 0;
+  s.each(n, [&](int at, float x) {
+    if (x > own) { own = x; own_at = at; }
+  });
+  const float m = block_max(own, red);
+  // a key that is reached: nothing MOST below it can be the best
+  const float floor_key =
+      block_max(gumbel_key(seed, i0 + own_at, (own - m) * inv_temp), red) - MOST;
+  Best b;
+  Gather<T, VEC> gather{queue + (tid / WAVE) * Gather<T, VEC>::ROOM};
+  gather.run(s, n, [&](float x) { return (x - m) * inv_temp > floor_key; },
+             [&](int at, float x) {
+               b.offer(gumbel_key(seed, i0 + at, (x - m) * inv_temp), i0 + at);
+             });
+  over_block(b, fpart, ipart);
+  if (tid >= WAVE) return;
+  // Of the row's slices the last to come finds all of them here, as each looks only
+  // when its own words have arrived. Another may, too, and writes the same token.
+  // Nothing has to be cleared first; who has seen all clears them, because a replay of
+  // a captured launch has the same mark.
+  unsigned long long* const words = found + (int64_t)row * S * WORDS;
+  const unsigned long long high = (unsigned long long)mark << 32;
+  const uint32_t own_word[WORDS] = {__float_as_uint(m), __float_as_uint(b.key), (uint32_t)b.idx};
+  if (tid == 0) {
+    #pragma unroll
+    for (int i = 0; i < WORDS; ++i) store_through(words + sl * WORDS + i, high | own_word[i]);
+  }
+  stores_done();
+  float m_row = -1e30f;
+  bool all_here = true;
+  for (int i = tid; i < S; i += WAVE) {
+    unsigned long long w[WORDS];
+    #pragma unroll
+    for (int j = 0; j < WORDS; ++j) w[j] = load_through(words + i * WORDS + j);
+    #pragma unroll
+    for (int j = 0; j < WORDS; ++j) all_here = all_here && (w[j] >> 32) == mark;
+    // relative to the highest maximum that this lane has met
+    const float top = __uint_as_float((uint32_t)w[TOP]), to = fmaxf(m_row, top);
+    if (i == tid) b = Best{};
+    b.key = fmaxf(b.key + (m_row - to) * inv_temp, -1e30f);
+    m_row = to;
+    const int idx = (int)(uint32_t)w[ELEMENT];
+    if (idx != 0x7fffffff) b.offer(__uint_as_float((uint32_t)w[KEY]) + (top - to) * inv_temp, idx);
+  }
+  if (tid >= S) b = Best{};
+  if (__ballot(!all_here) != 0) return;
+  const float top = wave_max(m_row);
+  b.key = fmaxf(b.key + (m_row - top) * inv_temp, -1e30f);
+  b.over_wave();
+  if (tid == 0) out[row] = b.idx == 0x7fffffff ? 0 : b.idx;
+  for (int i = tid; i < S * WORDS; i += WAVE) words[i] = 0ull;
+}
+
+// ------------------------------------------------------------- threshold
+// Steps of -z, one wide from 0 to 20 and four wide from there to 32, where little is
+// left that a window could hold. Steps of half an octave are eleven instead of 23, but
+// with a threshold 11 below the maximum the window took in most of a row (72 us of
+// drawing for 160 rows).
+constexpr int STEPS = 23;
+DEV_INLINE int step_of(float t) { return (int)fminf(t, 15.f + 0.25f * t); }
+constexpr int LEVELS = 64;             // at which a row's steps are compared, z = 1/2 apart
+constexpr int PER_LEVEL = NBINS / LEVELS;
+// Bins in which the threshold may lie: up to a step, two levels and rounding.
+constexpr int WINDOW = 16 * PER_LEVEL;
+constexpr int POOL = 768;              // as often as they fit, in LDS
+
+// Of a slice: its maximum, probability and count down to each step below it. Of a
+// row: slices that are done; sum, count and best draw above the window (entry 0)
+// and in its bins.
+struct Sums {
+  float *top, *p;                      // (B, S), (B, S, STEPS)
+  int* c;                              // (B, S, STEPS)
+  unsigned long long *mass, *best;     // (B, 1 + WINDOW)
+  int *count, *done;                   // (B, 1 + WINDOW), (B)
+};
+
+DEV_INLINE int64_t width_at(int row) { return (int64_t)row * (1 + WINDOW); }
+
+template <typename T, bool VEC, bool BY_P, bool BY_K>
+__global__ __launch_bounds__(256)
+void steps_kernel(const T* __restrict__ logits, int V, int per, float inv_temp, Sums sums) {
+  __shared__ float hp[BY_P ? STEPS * 256 : 1];          // [step][thread]
+  __shared__ uint32_t hc[BY_K ? (STEPS + 3) / 4 * 256 : 1];   // four counts a word, 80 at most each
+  __shared__ float red[4], tp[STEPS];
+  __shared__ int tc[STEPS];
+  const int row = blockIdx.x, sl = blockIdx.y, S = gridDim.y, tid = threadIdx.x;
+  const int i0 = sl * per, n = min(V - i0, per);
+  Slice<T, VEC> s;
+  s.load(logits + (int64_t)row * V + i0, n);
+  if (sl == 0) {
+    for (int i = tid; i < 1 + WINDOW; i += 256) {
+      sums.mass[width_at(row) + i] = sums.best[width_at(row) + i] = 0ull;
+      sums.count[width_at(row) + i] = 0;
+    }
+    if (tid == 0) sums.done[row] = 0;
+  }
+  float m = -1e30f;
+  s.each(n, [&](int, float x) { m = fmaxf(m, x); });
+  if (BY_P)
+    #pragma unroll
+    for (int i = 0; i < STEPS; ++i) hp[i * 256 + tid] = 0.f;
+  if (BY_K)
+    #pragma unroll
+    for (int i = 0; i < (STEPS + 3) / 4; ++i) hc[i * 256 + tid] = 0;
+  m = block_max(m, red);
+  s.each(n, [&](int, float x) {
+    // without branches; what lies deeper adds e^-32, nothing beside the maximum's 1
+    const float below = (m - x) * inv_temp, t = fminf(below, ZRANGE - 0.01f);
+    const int g = step_of(t);
+    if (BY_P) hp[g * 256 + tid] += __expf(-t);
+    if (BY_K) hc[(g >> 2) * 256 + tid] += below < ZRANGE ? 1u << (g & 3) * 8 : 0u;
+  });
+  __syncthreads();
   const int wid = tid / WAVE, lane = tid & (WAVE - 1);
-  for (int b = wid * 8; b < wid * 8 + 8; ++b) {
+  for (int b = wid; b < STEPS; b += 4) {
     if (BY_P) {
       float v = 0.f;
       #pragma unroll
       for (int i = 0; i < 4; ++i) v += hp[b * 256 + i * WAVE + lane];
       v = wave_sum(v);
-      if (lane == 0 && v != 0.f)
-        atomicAdd(&(FINE ? h.bin_p : h.group_p)[row * 32 + b],
-                  (unsigned long long)(v * 0x1p32f + 0.5f));
+      if (lane == 0) tp[b] = v;
     }
     if (BY_K) {
       int v = 0;
       #pragma unroll
-      for (int i = 0; i < 4; ++i) v += hc[b * 256 + i * WAVE + lane];
+      for (int i = 0; i < 4; ++i) v += (hc[(b >> 2) * 256 + i * WAVE + lane] >> (b & 3) * 8) & 255;
       #pragma unroll
       for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-      if (lane == 0 && v != 0) atomicAdd(&(FINE ? h.bin_c : h.group_c)[row * 32 + b], v);
+      if (lane == 0) tc[b] = v;
     }
   }
+  __syncthreads();
+  if (tid >= 32) return;
+  const int64_t at = (int64_t)row * S + sl;
+  if (tid == 0) sums.top[at] = m;
+  const int b = min(tid, STEPS - 1);
+  if (BY_P) {
+    const float v = upto32(tid < STEPS ? tp[b] : 0.f);
+    if (tid < STEPS) sums.p[at * STEPS + b] = v;
+  }
+  if (BY_K) {
+    const int v = upto32(tid < STEPS ? tc[b] : 0);
+    if (tid < STEPS) sums.c[at * STEPS + b] = v;
+  }
+}
+
+// Bins [first, end) in which the threshold lies, from the steps of a row's slices; all
+// threads get it. With a slice's maximum at z = d a level -L is L + d below it: down to
+// there the slice holds at least the steps that end above it and at most those that
+// begin above it.
+struct Window { int first, end; float total; };
+
+// LDS of the search: the steps of as many slices as a wave has lanes, then sums of its
+// four shares.
+struct Search {
+  static constexpr int AT_ONCE = WAVE;
+  float p[AT_ONCE * STEPS], d[AT_ONCE], w[AT_ONCE];
+  int c[AT_ONCE * STEPS];
+};
+struct Shares {
+  float f[4][LEVELS][3];
+  int i[4][LEVELS][2];
+};
+
+template <bool BY_P, bool BY_K>
+DEV_INLINE Window find_window(const Sums& sums, int row, int S, float m, float inv_temp, float top_p,
+                              int top_k, char* lds) {
+  auto& in = *reinterpret_cast<Search*>(lds);
+  auto& out = *reinterpret_cast<Shares*>(lds);
+  const int tid = threadIdx.x, L = tid & (LEVELS - 1), sub = tid / LEVELS;
+  float least = 0.f, most = 0.f, total = 0.f;
+  int cleast = 0, cmost = 0;
+  for (int s0 = 0; s0 < S; s0 += Search::AT_ONCE) {
+    const int n = min(S - s0, Search::AT_ONCE);
+    const int64_t at = (int64_t)row * S + s0;
+    if (s0) __syncthreads();
+    #pragma unroll
+    for (int i = 0; i < CDIV(Search::AT_ONCE * STEPS, 256); ++i) {
+      const int j = i * 256 + tid;
+      if (BY_P && j < n * STEPS) in.p[j] = sums.p[at * STEPS + j];
+      if (BY_K && j < n * STEPS) in.c[j] = sums.c[at * STEPS + j];
+    }
+    if (tid < n) {
+      const float d = fmaxf((sums.top[at + tid] - m) * inv_temp, -1000.f);
+      in.d[tid] = d;
+      in.w[tid] = __expf(d);
+    }
+    __syncthreads();
+    for (int s = sub; s < n; s += 4) {
+      // what lies on a level's edge may have been rounded over it
+      const float t = L * (ZRANGE / LEVELS) + in.d[s], w = in.w[s];
+      const int ends = t > 2e-4f ? min(step_of(t - 1e-4f) - 1, STEPS - 1) : -1;
+      const int begins = t > -1e-4f ? min(step_of(fmaxf(t, 0.f) + 1e-4f), STEPS - 1) : -1;
+      if (BY_P) {
+        const float* p = in.p + s * STEPS;
+        least += ends >= 0 ? w * p[max(ends, 0)] : 0.f;
+        most += begins >= 0 ? w * p[max(begins, 0)] : 0.f;
+        total += w * p[STEPS - 1];
+      }
+      if (BY_K) {
+        const int* c = in.c + s * STEPS;
+        cleast += ends >= 0 ? c[max(ends, 0)] : 0;
+        cmost += begins >= 0 ? c[max(begins, 0)] : 0;
+      }
+    }
+  }
+  __syncthreads();
+  if (BY_P) { out.f[sub][L][0] = least; out.f[sub][L][1] = most; out.f[sub][L][2] = total; }
+  if (BY_K) { out.i[sub][L][0] = cleast; out.i[sub][L][1] = cmost; }
+  __syncthreads();
+  least = most = total = 0.f;
+  cleast = cmost = 0;
+  #pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (BY_P) { least += out.f[i][L][0]; most += out.f[i][L][1]; total += out.f[i][L][2]; }
+    if (BY_K) { cleast += out.i[i][L][0]; cmost += out.i[i][L][1]; }
+  }
+  // a level a lane; reached at the end of z if nowhere before
+  auto cut = [&](bool reached, bool short_of, int& first, int& end) {
+    const unsigned long long r = __ballot(reached), o = __ballot(short_of);
+    first = max(0, 63 - __clzll((long long)o));     // __clzll(0) = 64: none
+    end = min(r ? __ffsll(r) - 1 : LEVELS, first + WINDOW / PER_LEVEL);
+    end = max(end, first + 1);
+  };
+  Window w{0, LEVELS, total};
+  if (BY_P) {
+    const float target = top_p * total;
+    cut(least >= target * (1.f + 2e-6f), most < target * (1.f - 2e-6f), w.first, w.end);
+  }
+  if (BY_K) {
+    int first, end;
+    cut(cleast >= top_k, cmost < top_k, first, end);
+    w.first = BY_P ? min(w.first, first) : first;
+    w.end = BY_P ? min(w.end, end) : end;
+  }
+  w.first *= PER_LEVEL;
+  w.end *= PER_LEVEL;
+  return w;
 }
 
 template <typename T, bool VEC, bool BY_P, bool BY_K>
 __global__ __launch_bounds__(256)
-void slice_draw_kernel(const T* __restrict__ logits, int V, int per, float inv_temp, float top_p,
-                       int top_k, const float* __restrict__ ms, Hist h,
-                       const int64_t* __restrict__ seeds, const int64_t* __restrict__ step, unsigned long long* __restrict__ top,
-                       int* __restrict__ done, int64_t* __restrict__ out) {
-  __shared__ uint2 queue[4 * 128];
-  __shared__ float fpart[4];
-  __shared__ int ipart[4];
+void pick_kernel(const T* __restrict__ logits, int V, int per, float inv_temp, float top_p,
+                 int top_k, Sums sums, const int64_t* __restrict__ seeds,
+                 const int64_t* __restrict__ step, int64_t* __restrict__ out) {
+  __shared__ typename Gather<T, VEC>::Entry queue[4 * Gather<T, VEC>::ROOM];
+  __shared__ unsigned long long wmass[BY_P ? POOL : 1], wbest[POOL];   // [bin][copy]
+  __shared__ int wcount[BY_K ? POOL : 1];
+  __shared__ float red[4], fpart[4];
+  __shared__ int ipart[4], last;
+  // the search for the window comes before the gathering
+  static_assert(sizeof(queue) >= sizeof(Search) && sizeof(queue) >= sizeof(Shares), "");
   const int row = blockIdx.x, sl = blockIdx.y, S = gridDim.y, tid = threadIdx.x;
-  const T* lr = logits + (int64_t)row * V;
-  const int i1 = min(V, (sl + 1) * per);
-  const float m = row_max(ms, row, S);
-  float zlow = ZDRAW;
-  if (BY_P || BY_K) {
-    Crossing<float> cp;
-    Crossing<int> ck;
-    float target;
-    crossing_groups<BY_P, BY_K>(h, row, top_p, top_k, cp, ck, target);
-    const int at = row * 32 + (tid & 31);
-    int thr = NBINS - 1;
-    if (BY_P) thr = min(thr, cp.bin * IN_GROUP + crossing(prob(h.bin_p[at]), cp.before, target).bin);
-    if (BY_K) thr = min(thr, ck.bin * IN_GROUP + crossing(h.bin_c[at], ck.before, top_k).bin);
-    // the bins up to thr are z > -(thr + 1) / 32; the edge itself lies in the next
-    zlow = fmaxf(-(thr + 1) * (ZRANGE / NBINS), ZDRAW);
+  const int i0 = sl * per, n = min(V - i0, per);
+  Slice<T, VEC> s;
+  s.load(logits + (int64_t)row * V + i0, n);
+  for (int i = tid; i < POOL; i += 256) {
+    if (BY_P) wmass[i] = 0ull;
+    if (BY_K) wcount[i] = 0;
+    wbest[i] = 0ull;
   }
-  DrawQueue dq{queue + (tid / WAVE) * 128, row_seed(seeds, step, row)};
-  float x[8], next[8];
-  int id[8], next_id[8];
-  if (sl * per < i1) load8<T, VEC>(lr, sl * per, i1, next, next_id);
-  for (int base = sl * per; base < i1; base += 2048) {
-    #pragma unroll
-    for (int k = 0; k < 8; ++k) { x[k] = next[k]; id[k] = next_id[k]; }
-    load8<T, VEC>(lr, base + 2048, i1, next, next_id);   // past the end: the last eight again
-    #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const float z = (x[k] - m) * inv_temp;
-      dq.push(z > zlow, id[k], z);
-    }
-  }
-  dq.draw(dq.count);
-  dq.best.over_wave();
+  float m = -1e30f;
+  for (int i = tid & (WAVE - 1); i < S; i += WAVE) m = fmaxf(m, sums.top[(int64_t)row * S + i]);
+  m = wave_max(m);
+  const Window w = find_window<BY_P, BY_K>(sums, row, S, m, inv_temp, top_p, top_k,
+                                            reinterpret_cast<char*>(queue));
   __syncthreads();
-  if ((tid & (WAVE - 1)) == 0) {
-    fpart[tid / WAVE] = dq.best.key;
-    ipart[tid / WAVE] = dq.best.idx;
-  }
-  __syncthreads();
-  if (tid != 0) return;
+  const uint64_t seed = row_seed(seeds, step, row);
+  const float zlow = -w.end * (ZRANGE / NBINS);
+  const int bins = w.end - w.first;
+  const int copies = 1 << (31 - __clz(min(POOL / bins, 16))), copy = tid & (copies - 1);
   Best b;
-  for (int w = 0; w < 4; ++w) b.offer(fpart[w], ipart[w]);
-  // key and index in one word whose order is that of Best; 0: nothing kept
-  uint32_t o = __float_as_uint(b.key);
-  o = (o >> 31) ? ~o : o | 0x80000000u;
-  unsigned long long mine = b.idx == 0x7fffffff ? 0ull
-      : ((unsigned long long)o << 32) | (0xffffffffu - (uint32_t)b.idx);
-  if (S > 1) {
-    atomicMax(&top[row], mine);
-    __threadfence();
-    if (atomicAdd(&done[row], 1) != S - 1) return;
-    __threadfence();
-    mine = atomicMax(&top[row], 0ull);      // all slices have arrived
+  float above = 0.f;
+  int cabove = 0;
+  Gather<T, VEC> gather{queue + (tid / WAVE) * Gather<T, VEC>::ROOM};
+  gather.run(s, n, [&](float x) { return (x - m) * inv_temp > zlow; }, [&](int at, float x) {
+    const float z = (x - m) * inv_temp;
+    const int bin = bin_of(z);
+    const float p = BY_P ? __expf(z) : 0.f;
+    Best e;
+    if (z > ZDRAW) e.offer(gumbel_key(seed, i0 + at, z), i0 + at);
+    if (bin < w.first) {
+      above += p;
+      ++cabove;
+      b.offer(e.key, e.idx);
+    } else {
+      const int to = min(bin - w.first, bins - 1) * copies + copy;
+      if (BY_P) atomicAdd(wmass + to, (unsigned long long)(p * 0x1p32f + 0.5f));
+      if (BY_K) atomicAdd(wcount + to, 1);
+      const unsigned long long o = word_of(e);
+      if (o > wbest[to]) atomicMax(wbest + to, o);      // seldom
+    }
+  });
+  over_block(b, fpart, ipart);                  // waits for the window too
+  const int64_t at = width_at(row);
+  above = block_sum(above, red);
+  if (BY_K) {
+    #pragma unroll
+    for (int off = 32; off > 0; off >>= 1) cabove += __shfl_xor(cabove, off, WAVE);
+    if ((tid & (WAVE - 1)) == 0 && cabove) atomicAdd(sums.count + at, cabove);
   }
-  out[row] = mine == 0ull ? 0 : (int64_t)(0xffffffffu - (uint32_t)mine);
+  if (tid == 0) {
+    if (BY_P && above != 0.f)
+      atomicAdd(sums.mass + at, (unsigned long long)(above * 0x1p32f + 0.5f));
+    if (word_of(b)) atomicMax(sums.best + at, word_of(b));
+  }
+  for (int j = tid; j < bins; j += 256) {
+    unsigned long long mass = 0, best = 0;
+    int count = 0;
+    for (int i = j * copies; i < (j + 1) * copies; ++i) {
+      if (BY_P) mass += wmass[i];
+      if (BY_K) count += wcount[i];
+      best = wbest[i] > best ? wbest[i] : best;
+    }
+    if (BY_P && mass) atomicAdd(sums.mass + at + 1 + j, mass);
+    if (BY_K && count) atomicAdd(sums.count + at + 1 + j, count);
+    if (best) atomicMax(sums.best + at + 1 + j, best);
+  }
+  stores_done();
+  __syncthreads();
+  if (tid == 0) last = atomicAdd(&sums.done[row], 1) == S - 1;
+  __syncthreads();
+  if (!last) return;
+  // all slices have arrived: their sums come into LDS, and the first wave walks them
+  for (int j = tid; j < (bins + 31) / 32 * 32; j += 256) {
+    if (BY_P) wmass[j] = load_through(sums.mass + at + 1 + j);
+    if (BY_K) wcount[j] = load_through(sums.count + at + 1 + j);
+    wbest[j] = load_through(sums.best + at + 1 + j);
+  }
+  __syncthreads();
+  if (tid >= WAVE) return;
+  const float target = top_p * w.total;
+  unsigned long long best = load_through(sums.best + at);
+  unsigned long long mass = BY_P ? load_through(sums.mass + at) : 0ull;
+  int count = BY_K ? load_through(sums.count + at) : 0;
+  for (int b0 = 0; b0 < bins; b0 += 32) {
+    const int i = b0 + (tid & 31);            // POOL is a multiple of 32; zeros past the end
+    const unsigned long long pm = BY_P ? mass + upto32(wmass[i]) : 0ull;
+    const int pc = BY_K ? count + upto32(wcount[i]) : 0;
+    const uint32_t hit = (uint32_t)__ballot((BY_P && (float)pm * 0x1p-32f >= target) ||
+                                            (BY_K && pc >= top_k));
+    const int kept = hit ? __ffs((int)hit) : 32;      // down to the threshold's bin
+    unsigned long long o = (tid & 31) < kept ? wbest[i] : 0ull;
+    #pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const unsigned long long y = __shfl_xor(o, off, WAVE);
+      o = y > o ? y : o;
+    }
+    best = o > best ? o : best;
+    if (hit) break;
+    mass = __shfl(pm, 31, WAVE);
+    count = __shfl(pc, 31, WAVE);
+  }
+  if (tid == 0) out[row] = best == 0ull ? 0 : (int64_t)index_of(best);
+}
+
+// Slices of a row: two or three workgroups a CU, none longer than a workgroup's
+// registers hold or shorter than `least`. A workgroup of the threshold's launches takes
+// ~8 us whatever its slice (32 rows of 151936 in 640, 1280, 1920 workgroups 21, 26, 41
+// us; from 80 rows on the longest slices are more anyway).
+int slices(int B, int V, int least) {
+  return std::max(CDIV(V, SLICE), std::max(1, std::min(V / least, 640 / B)));
 }
 
 template <typename T, bool VEC>
 void sample_slices(const T* logits, int B, int V, float inv_t, float top_p, int top_k,
                    const torch::Tensor& seeds, const torch::Tensor& step, torch::Tensor& out) {
-  const bool by_p = top_p < 1.f, by_k = top_k > 0, filtering = by_p || by_k;
-  // enough slices for four workgroups a CU, none under one load of a block
-  int S = 1;
-  while (S < 64 && (int64_t)B * S < 1024 && V / (2 * S) >= 2048) S *= 2;
-  const int per = (CDIV(V, S) + 7) / 8 * 8;
-  auto ws = torch::empty({B * (int64_t)(12 + 4 * S + (filtering ? (8 + 4) * 2 * 32 : 0))},
-                         out.options().dtype(at::kByte));
-  char* w = reinterpret_cast<char*>(ws.data_ptr());
-  auto* top = reinterpret_cast<unsigned long long*>(w);
-  w += 8ll * B;
-  Hist h{};
-  if (filtering) {
-    h.group_p = reinterpret_cast<unsigned long long*>(w);
-    h.bin_p = h.group_p + 32ll * B;
-    h.group_c = reinterpret_cast<int*>(h.bin_p + 32ll * B);
-    h.bin_c = h.group_c + 32ll * B;
-    w = reinterpret_cast<char*>(h.bin_c + 32ll * B);
-  }
-  int* done = reinterpret_cast<int*>(w);
-  float* ms = reinterpret_cast<float*>(w + 4ll * B);
+  const bool by_p = top_p < 1.f, by_k = top_k > 0;
+  int S = slices(B, V, by_p || by_k ? 2048 : 1024);
+  const int per = CDIV(CDIV(V, S), 8) * 8;
+  S = CDIV(V, per);
+  TORCH_CHECK(per <= SLICE && (int64_t)per * S >= V && (int64_t)per * (S - 1) < V && S < 65536);
+  const int64_t rows = B, cells = rows * S;
   auto stream = at::cuda::getCurrentCUDAStream();
   const dim3 grid(B, S), block(256);
-  hipLaunchKernelGGL((slice_max_kernel<T, VEC>), grid, block, 0, stream, logits, V, per, ms, top,
-                     done, h);
-  auto hist = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream, logits, V, per, inv_t, top_p, top_k, ms, h);
+  auto room = [&](int64_t bytes) {
+    return torch::empty({bytes}, out.options().dtype(at::kByte));
   };
-  auto draw = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream, logits, V, per, inv_t, top_p, top_k, ms, h,
-                       seeds.data_ptr<int64_t>(), step.data_ptr<int64_t>(), top, done,
+  if (!by_p && !by_k) {
+    auto ws = room(cells * WORDS * 8);
+    hipLaunchKernelGGL((draw_kernel<T, VEC>), grid, block, 0, stream, logits, V, per, inv_t,
+                       seeds.data_ptr<int64_t>(), step.data_ptr<int64_t>(),
+                       reinterpret_cast<unsigned long long*>(ws.data_ptr()),
+                       (uint32_t)(arrival_tag() >> 32), out.data_ptr<int64_t>());
+    return;
+  }
+  auto ws = room(rows * (1 + WINDOW) * 20 + rows * 4 + cells * 4 * (1 + 2 * STEPS));
+  Sums sums;
+  sums.mass = reinterpret_cast<unsigned long long*>(ws.data_ptr());
+  sums.best = sums.mass + rows * (1 + WINDOW);
+  sums.count = reinterpret_cast<int*>(sums.best + rows * (1 + WINDOW));
+  sums.done = sums.count + rows * (1 + WINDOW);
+  sums.top = reinterpret_cast<float*>(sums.done + rows);
+  sums.p = sums.top + cells;
+  sums.c = reinterpret_cast<int*>(sums.p + cells * STEPS);
+  auto go = [&](auto p_, auto k_) {
+    constexpr bool P = decltype(p_)::value, K = decltype(k_)::value;
+    hipLaunchKernelGGL((steps_kernel<T, VEC, P, K>), grid, block, 0, stream, logits, V, per, inv_t,
+                       sums);
+    hipLaunchKernelGGL((pick_kernel<T, VEC, P, K>), grid, block, 0, stream, logits, V, per, inv_t,
+                       top_p, top_k, sums, seeds.data_ptr<int64_t>(), step.data_ptr<int64_t>(),
                        out.data_ptr<int64_t>());
   };
-  #define BY(P, K)                                        \
-    do {                                                  \
-      if (P || K) {                                       \
-        hist(slice_hist_kernel<T, VEC, P, K, false>);     \
-        hist(slice_hist_kernel<T, VEC, P, K, true>);      \
-      }                                                   \
-      draw(slice_draw_kernel<T, VEC, P, K>);              \
-    } while (0)
-  if (by_p && by_k) BY(true, true);
-  else if (by_p) BY(true, false);
-  else if (by_k) BY(false, true);
-  else BY(false, false);
-  #undef BY
+  if (by_p && by_k) go(std::true_type{}, std::true_type{});
+  else if (by_p) go(std::true_type{}, std::false_type{});
+  else go(std::false_type{}, std::true_type{});
 }
 
 }  // namespace

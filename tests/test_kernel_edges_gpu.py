@@ -178,6 +178,28 @@ def test_sampler_draws_as_defined(ext, B, V, dtype, temperature, top_p, top_k):
     assert got.tolist() == _sampled(logits, temperature, top_p, top_k, seeds, 11)
 
 
+@pytest.mark.parametrize("B,V,dtype", [
+    (640, 2048, "bfloat16"), (640, 2056, "bfloat16"), (641, 20480, "bfloat16"),
+    (320, 20488, "bfloat16"), (200, 20479, "float32"), (33, 61440, "bfloat16"),
+    (12, 163841, "bfloat16"), (1, 300000, "float32")])
+@pytest.mark.parametrize("spread,temperature,top_p,top_k", [
+    (3.0, 0.6, 1.0, 0), (0.5, 1.0, 0.9, 0), (3.0, 1.3, 0.97, 0), (2.0, 1.0, 0.9, 300)])
+def test_sampler_long_slices(ext, B, V, dtype, spread, temperature, top_p, top_k):
+    """Slices as long as a workgroup's registers hold, one element more and
+    less, a row in one and in more than 64; thresholds just below the maximum
+    and deep, flat rows of which most is drawn."""
+    g = torch.Generator().manual_seed(V + B)
+    logits = torch.randn(B, V, generator=g) * spread
+    logits[:, V // 3] += 4.0 * spread
+    logits = logits.to("cuda", getattr(torch, dtype))
+    seeds = torch.randint(0, 2 ** 31 - 1, (B,), generator=g)
+    got = ext.sample_tokens(logits, temperature, top_p, top_k, seeds.cuda(),
+                            torch.tensor([3], device="cuda")).tolist()
+    for at in range(0, B, max(1, B // 12)):
+        row = slice(at, at + 1)
+        assert got[row] == _sampled(logits[row], temperature, top_p, top_k, seeds[row], 3)
+
+
 def test_sampler_odd_places_and_values(ext):
     """A matrix that does not start on 16 bytes, rows with -inf, and a row
     with nothing finite below its maximum."""
