@@ -6,13 +6,13 @@ The module-by-module layer launches ~200 kernels forward and backward, most
 of them elementwise passes between the products (residual adds, adapter
 scaling, gradient sums of projections that share an input, rotary steps,
 head transposes), and short micro-batches are bound by launching them. A half
-is ~19 launches here, prepared in native code (ops/csrc/adapted_layer.cpp):
-adapters are columns of their projections' products, W laid out beside B for
-it. That costs a copy of the weights, 37 us a layer of the 1.5B model forward
-and as long backward, where adding the adapters' outputs to 18800 rows in
-passes of their own took 750; large weights that few rows meet are taken as
-they lie, their adapters joined to fp32 products. Adapter gradients are one launch and its sum
-(ops/csrc/adapter_grads.hip).
+is 7 launches forward and 9 or 10 backward here, prepared in native code
+(ops/csrc/adapted_layer.cpp): products of our own (ops/csrc/product.hip) take
+adapters as more of their projections' K, residuals, the activation and its
+gradient with them. The library's products, where many rows meet wide weights,
+have W laid out beside B for it; large weights that few rows meet are taken as
+they lie, their adapters joined to fp32 products. Adapter gradients are one
+launch and its sum (ops/csrc/adapter_grads.hip).
 """
 
 from __future__ import annotations

@@ -2,15 +2,18 @@
 // one call: attention and feed-forward with their norms, adapted projections and
 // residual sums. The autograd nodes around them are models/fused_layer.py.
 //
-// An adapter is more of its projection: u = scale * x A^T lies beside x in one
-// matrix, [x | u], and one product with [W | B] gives every projection of that
-// input, adapters and (beta = 1) the residual in its fp32 sums; backward is
-// [dY | du] [W; A]. Few rows take large weights as they lie.
+// An adapter is more of its projection: with u = scale * x A^T a projection is one
+// sum, x W^T + u B^T, with its bias or the residual; backward is dY W + du A. Own
+// products (product.hip) take all of them from where they lie, the activation and its
+// gradient with them. For the library, where it is the faster or ranks don't fit, u
+// lies beside x in one matrix, [x | u], for one product with [W | B], and few rows
+// take large weights as they lie.
 //
-// Native because short micro-batches wait for the host: the same launches from
-// Python took 25.0 ms a pass of the 0.5B model over three short samples, of which
-// the GPU worked 11.
+// Native because short micro-batches wait for the host: prepared in Python a pass of
+// the 0.5B model over three short samples took 25.0 ms, with the library's products
+// (17 us of the host each) and what they need beside them 16.0, now 11.8.
 #include "adapted.h"
+#include "product.h"
 
 using at::Tensor;
 using Tensors = std::vector<Tensor>;
@@ -44,6 +47,12 @@ Tensor columns(const Tensor& t, int64_t from, int64_t n) { return t.narrow(1, fr
 
 Tensor heads(const Tensor& t, int64_t head_dim) {
   return t.view({t.size(0), t.size(1) / head_dim, head_dim});
+}
+
+// Rows of so many columns, an odd number of 128 B apart: 18793 x 1536 x 8960 took 465
+// us with rows of 141 x 128 B, 513 with 140, 596 with 140.5.
+Tensor apart_rows(int64_t rows, int64_t cols, const at::TensorOptions& options) {
+  return columns(at::empty({rows, ((cols + 63) / 64 | 1) * 64}, options), 0, cols);
 }
 
 // out <- scale * a b, the scale in the product's epilogue
@@ -122,10 +131,28 @@ void join(const Tensor& y, const Tensor& u, const Tensor& m, const Tensor& out,
   out.copy_(y);
 }
 
-// [x | u] [W | B]^T of projections of one input, + their biases, or + a residual:
-// one rounding for all of it
-Tensor product(const Tensor& xu, const Tensors& W, const Adapters& ad,
-               const std::vector<Optional>& bias, const Optional& res = {}) {
+// Whether a product of many rows with wide weights (N, K) is the library's: its tiles
+// are the faster there, and what it needs beside them (weights laid out beside
+// adapters, the residual's copy, the activation's passes) small against that. A layer
+// of 18793 rows, us, own -> library with all of it: down 440 -> 390, the input gradient of
+// gate and up 850 -> 800, gate, up and activation 1080 -> 1060, the activation's gradient
+// 840 -> 820, its epilogue not hidden behind another tile's products; but q, k, v 127 ->
+// 160, o 111 -> 122.
+bool library(int64_t rows, int64_t N, int64_t K) { return rows > 8192 && std::max(N, K) >= 4096; }
+
+// x W^T + u B^T of projections of one input
+std::vector<ProductBlock> blocks(const Tensor& x, const Tensor& u, const Tensors& W,
+                                 const Adapters& ad, const std::vector<Optional>& bias) {
+  std::vector<ProductBlock> out;
+  for (size_t i = 0; i < W.size(); ++i)
+    out.push_back({W[i].size(0), {{x, W[i]}, {ad.part(u, i), ad.B[i]}},
+                   i < bias.size() ? bias[i] : Optional()});
+  return out;
+}
+
+// the same of [x | u], + their biases, or + a residual: one rounding for all of it
+Tensor projected(const Tensor& xu, const Tensors& W, const Adapters& ad,
+                 const std::vector<Optional>& bias, const Optional& res = {}) {
   const int64_t rows = xu.size(0), K = W[0].size(1);
   int64_t width = 0;
   bool any = false;
@@ -142,6 +169,11 @@ Tensor product(const Tensor& xu, const Tensors& W, const Adapters& ad,
       from += n;
     }
     return out;
+  }
+  if (!library(rows, width, K)) {
+    auto out = at::empty({rows, width}, xu.options());
+    if (product(blocks(columns(xu, 0, K), columns(xu, K, ad.pad), W, ad, bias), false, out, res))
+      return out;
   }
   const auto WB = adapted_weight(W, ad.B, ad.pad);
   if (res) return at::addmm(*res, xu, WB.t());
@@ -187,22 +219,43 @@ Tensor back_apart(const Tensors& dy, const Tensors& W, const Tensor& du, const A
   return out;
 }
 
-struct Through { Tensor dx, g, du; };
+struct Through { Tensor dx, du; };
 
-// g W + du A with du = scale * g B, from one product of [g | du]; g and du as parts
-// of that matrix
+// g W + du A with du = scale * g B, and du
 Through through(const Tensor& g, const Tensor& W, const Adapters& ad) {
   const int64_t N = g.size(1);
   if (apart(g.size(0), N, W.size(1))) {
     auto du = at::empty({g.size(0), ad.pad}, g.options());
     ad.up({g}, du);
-    return {back_apart({g}, {W}, du, ad), g, ad.part(du, 0)};
+    return {back_apart({g}, {W}, du, ad), ad.part(du, 0)};
+  }
+  if (!library(g.size(0), N, W.size(1))) {
+    auto du = at::empty({g.size(0), ad.pad}, g.options());
+    auto dx = at::empty({g.size(0), W.size(1)}, g.options());
+    ad.up({g}, du);
+    const auto r = ad.part(du, 0);
+    if (product({{W.size(1), {{g, W}, {r, ad.A[0]}}, {}}}, true, dx)) return {dx, r};
   }
   auto gd = at::empty({g.size(0), N + ad.pad}, g.options());
   auto g2 = columns(gd, 0, N), du = columns(gd, N, ad.pad);
   g2.copy_(g);
   ad.up({g}, du);
-  return {at::mm(gd, stack_transposed({W, ad.A[0]}, {0, N}, N + ad.pad).t()), g2, ad.part(du, 0)};
+  return {at::mm(gd, stack_transposed({W, ad.A[0]}, {0, N}, N + ad.pad).t()), ad.part(du, 0)};
+}
+
+// dx <- dY W + du A of projections of one input; false where that is the library's
+bool own_dx(Tensor& dx, const Tensors& W, const Tensors& dy, const Tensor& du, const Adapters& ad) {
+  const int64_t rows = du.size(0);
+  ProductBlock sum{W[0].size(1), {}, {}};
+  int64_t K = 0;
+  for (size_t i = 0; i < W.size(); ++i) {
+    sum.terms.push_back({dy[i], W[i]});
+    K += W[i].size(0);
+  }
+  if (library(rows, sum.width, K)) return false;
+  for (size_t i = 0; i < W.size(); ++i) sum.terms.push_back({ad.part(du, i), ad.A[i]});
+  dx = at::empty({rows, sum.width}, du.options());
+  return product({sum}, true, dx);
 }
 
 struct Job { Tensor y, p; bool by_col; };
@@ -260,11 +313,11 @@ Tensors attention_half_fwd(Tensor x, Tensor norm, double eps, Tensors W,
   const Adapters o_ad({A[3]}, {B[3]}, {scales[3]});
   const Ints sizes = {W[0].size(0), W[1].size(0), W[2].size(0)};
 
-  auto hu = at::empty({rows, hidden + in.pad}, x.options());
+  auto hu = apart_rows(rows, hidden + in.pad, x.options());
   auto h = columns(hu, 0, hidden);
   rmsnorm_fwd_into(x, norm, eps, h);
   in.down(h, columns(hu, hidden, in.pad));
-  auto qkv = product(hu, {W[0], W[1], W[2]}, in, bias);
+  auto qkv = projected(hu, {W[0], W[1], W[2]}, in, bias);
   auto q = heads(columns(qkv, 0, sizes[0]), head_dim);
   auto k = heads(columns(qkv, sizes[0], sizes[1]), head_dim);
   auto v = heads(columns(qkv, sizes[0] + sizes[1], sizes[2]), head_dim);
@@ -276,11 +329,11 @@ Tensors attention_half_fwd(Tensor x, Tensor norm, double eps, Tensors W,
     k = rmsnorm_fwd(k0, *k_norm, k_eps);
   }
   rope_rows(q, k, pos, inv_freq);
-  auto ou = at::empty({rows, sizes[0] + o_ad.pad}, x.options());
+  auto ou = apart_rows(rows, sizes[0] + o_ad.pad, x.options());
   auto o = columns(ou, 0, sizes[0]);
   auto lse = flash_varlen_fwd(q, k, v, cu, longest, scale, heads(o, head_dim))[1];
   o_ad.down(o, columns(ou, sizes[0], o_ad.pad));
-  auto y = product(ou, {W[3]}, o_ad, {}, x);
+  auto y = projected(ou, {W[3]}, o_ad, {}, x);
   return {y, hu, ou, q, k, v, lse, q0, k0};
 }
 
@@ -301,7 +354,7 @@ Tensors attention_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tensors 
   auto h = columns(hu, 0, hidden), u = columns(hu, hidden, in.pad);
   auto o = columns(ou, 0, sizes[0]), uo = columns(ou, sizes[0], o_ad.ranks[0]);
 
-  const auto [dO, g2, duo] = through(g, W[3], o_ad);
+  const auto [dO, duo] = through(g, W[3], o_ad);
   auto dyu = at::empty({rows, width + in.pad}, x.options());
   const Tensors dys = {columns(dyu, 0, sizes[0]), columns(dyu, sizes[0], sizes[1]),
                        columns(dyu, sizes[0] + sizes[1], sizes[2])};
@@ -318,7 +371,7 @@ Tensors attention_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tensors 
   in.up(dys, du);
   auto s = sums({{h, du, false},
                  {o, duo, false},
-                 {g2, uo, true},
+                 {g, uo, true},
                  {dys[0], in.part(u, 0), true},
                  {dys[1], in.part(u, 1), true},
                  {dys[2], in.part(u, 2), true}});
@@ -328,6 +381,8 @@ Tensors attention_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tensors 
   Tensor dx;
   if (want_dx && apart(rows, width, hidden)) {
     dx = rmsnorm_bwd_add(back_apart(dys, {W[0], W[1], W[2]}, du, in), x, norm, g, eps);
+  } else if (want_dx && own_dx(dx, {W[0], W[1], W[2]}, dys, du, in)) {
+    dx = rmsnorm_bwd_add(dx, x, norm, g, eps);
   } else if (want_dx) {
     const auto WA = stack_transposed({W[0], W[1], W[2], A[0], A[1], A[2]},
                                      {0, sizes[0], sizes[0] + sizes[1], width, width + in.at[1],
@@ -349,16 +404,27 @@ Tensors feed_forward_half_fwd(Tensor x, Tensor norm, double eps, Tensors W,
   const int64_t rows = x.size(0), hidden = x.size(1), inner = W[0].size(0);
   const Adapters in({A[0], A[1]}, {B[0], B[1]}, {scales[0], scales[1]});
   const Adapters d_ad({A[2]}, {B[2]}, {scales[2]});
-  auto hu = at::empty({rows, hidden + in.pad}, x.options());
+  auto hu = apart_rows(rows, hidden + in.pad, x.options());
   auto h = columns(hu, 0, hidden);
   rmsnorm_fwd_into(x, norm, eps, h);
   in.down(h, columns(hu, hidden, in.pad));
-  auto gu = product(hu, {W[0], W[1]}, in, bias);
-  auto au = at::empty({rows, inner + d_ad.pad}, x.options());
+  auto au = apart_rows(rows, inner + d_ad.pad, x.options());
   auto act = columns(au, 0, inner);
-  silu_mul_packed_into(gu, act);
+  Tensor gu;
+  if (!apart(rows, 2 * inner, hidden) && !library(rows, 2 * inner, hidden)) {
+    gu = at::empty({rows, 2 * inner}, x.options());
+    const auto both = blocks(h, columns(hu, hidden, in.pad), {W[0], W[1]}, in, bias);
+    const auto &ug = both[0].terms[1].a, &uu = both[1].terms[1].a;
+    const ProductBlock gate{inner, {both[0].terms[0], {ug, B[0]}, {uu, {}}}, bias[0]};
+    const ProductBlock up{inner, {both[1].terms[0], {ug, {}}, {uu, B[1]}}, bias[1]};
+    if (!product_glu(gate, up, gu, act)) gu = Tensor();
+  }
+  if (!gu.defined()) {
+    gu = projected(hu, {W[0], W[1]}, in, bias);
+    silu_mul_packed_into(gu, act);
+  }
   d_ad.down(act, columns(au, inner, d_ad.pad));
-  auto y = product(au, {W[2]}, d_ad, {}, x);
+  auto y = projected(au, {W[2]}, d_ad, {}, x);
   return {y, hu, gu, au};
 }
 
@@ -374,15 +440,25 @@ Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tenso
   auto h = columns(hu, 0, hidden), u = columns(hu, hidden, in.pad);
   auto act = columns(au, 0, inner), ud = columns(au, inner, d_ad.ranks[0]);
 
-  const auto [dact, g2, dud] = through(g, W[2], d_ad);
-  auto dyu = at::empty({rows, 2 * inner + in.pad}, x.options());
+  auto dyu = apart_rows(rows, 2 * inner + in.pad, x.options());
   auto dgate = columns(dyu, 0, inner), dup = columns(dyu, inner, inner),
        du = columns(dyu, 2 * inner, in.pad);
-  silu_mul_bwd_packed(dact, gu, dgate, dup);
+  Tensor dud;
+  if (!apart(rows, hidden, inner) && !library(rows, hidden, inner)) {
+    auto both = at::empty({rows, d_ad.pad}, x.options());
+    d_ad.up({g}, both);
+    dud = d_ad.part(both, 0);
+    if (!product_glu_bwd({inner, {{g, W[2]}, {dud, A[2]}}, {}}, gu, dgate, dup)) dud = Tensor();
+  }
+  if (!dud.defined()) {
+    const auto [dact, du2] = through(g, W[2], d_ad);
+    silu_mul_bwd_packed(dact, gu, dgate, dup);
+    dud = du2;
+  }
   in.up({dgate, dup}, du);
   auto s = sums({{h, du, false},
                  {act, dud, false},
-                 {g2, ud, true},
+                 {g, ud, true},
                  {dgate, in.part(u, 0), true},
                  {dup, in.part(u, 1), true}});
   Tensors out = in_order(in, s[0], &s[3]);
@@ -391,6 +467,8 @@ Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tenso
   Tensor dx;
   if (want_dx && apart(rows, 2 * inner, hidden)) {
     dx = rmsnorm_bwd_add(back_apart({dgate, dup}, {W[0], W[1]}, du, in), x, norm, g, eps);
+  } else if (want_dx && own_dx(dx, {W[0], W[1]}, {dgate, dup}, du, in)) {
+    dx = rmsnorm_bwd_add(dx, x, norm, g, eps);
   } else if (want_dx) {
     const auto WA = stack_transposed({W[0], W[1], A[0], A[1]},
                                      {0, inner, 2 * inner, 2 * inner + in.ranks[0]},

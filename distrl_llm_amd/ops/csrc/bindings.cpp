@@ -111,6 +111,12 @@ void flash_varlen_bwd(torch::Tensor dout, torch::Tensor q, torch::Tensor k,
 std::vector<torch::Tensor> adapter_grads(std::vector<torch::Tensor> y,
                                          std::vector<torch::Tensor> p,
                                          std::vector<int64_t> by_col);
+bool product_py(std::vector<std::vector<torch::Tensor>> a,
+                std::vector<std::vector<c10::optional<torch::Tensor>>> b,
+                std::vector<c10::optional<torch::Tensor>> bias,
+                std::vector<int64_t> width, std::string what,
+                std::vector<torch::Tensor> out,
+                c10::optional<torch::Tensor> res, int64_t tile);
 torch::Tensor adapted_weight(std::vector<torch::Tensor> w,
                              std::vector<torch::Tensor> b, int64_t pad);
 torch::Tensor stack_transposed(std::vector<torch::Tensor> w,
@@ -260,6 +266,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("into") = py::none());
   m.def("flash_varlen_bwd", &flash_varlen_bwd,
         "its backward, into dq, dk and dv");
+  m.def("product", &product_py, py::arg("a"), py::arg("b"), py::arg("bias"),
+        py::arg("width"), py::arg("what"), py::arg("out"),
+        py::arg("res") = py::none(), py::arg("tile") = 0,
+        "sums of products with bias, residual or SiLU*mul (tests)");
   m.def("adapter_grads", &adapter_grads,
         "p^T y of several operands, summed over the rows");
   m.def("adapted_weight", &adapted_weight,

@@ -149,6 +149,24 @@ DEV_INLINE T load_through(const T* p) {
 // Until this wave's stores and atomics have arrived.
 DEV_INLINE void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// For one whole wave of workgroup `mine` of n, whose own stores_done are behind it:
+// leaves the launch's mark in its place and says whether all n marks are there, so
+// that what the n stored through before may be joined. Of the n workgroups the last to come sees all of them; another may too, and
+// then does the same join. Nothing has to be cleared beforehand, as no place holds the
+// mark by chance; a replay of a captured launch has the same mark, so those who saw
+// all of them take them away.
+DEV_INLINE bool all_there(unsigned long long* there, int n, int mine, unsigned long long tag) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  if (lane == 0) atomicExch(there + mine, tag);
+  stores_done();
+  bool all = true;
+  for (int i = lane; i < n; i += WAVE) all = all && atomicAdd(there + i, 0ull) == tag;
+  if (__ballot(!all) != 0) return false;
+  stores_done();
+  for (int i = lane; i < n; i += WAVE) there[i] = 0ull;
+  return true;
+}
+
 #define HIP_CHECK_LAST()                                                     \
   do {                                                                       \
     hipError_t e = hipGetLastError();                                        \

@@ -1,0 +1,122 @@
+"""Products on matrix cores (ops/csrc/product.hip) at the edges of their
+tiles, shares of K and terms, against plain fp32 torch."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# Bound: operands are exact in bf16 and sums fp32, so an output is off by its
+# own rounding to 8 significant bits, 2^-8 of it at most (half of the last one's
+# 2^-7), and by a sum's 2^-24 * K, far below that.
+REL = 2.0 ** -8
+TILES = [0, 8, 7, 6, 5, 4, 128, 64, 64 + 512, 128 + 768, 64 + 2048]
+
+
+@pytest.fixture(scope="module")
+def ext():
+    from distrl_llm_amd.ops.build import build
+    return build()
+
+
+def _make(seed):
+    g = torch.Generator().manual_seed(seed)
+
+    def rand(*shape, spare=0):
+        x = torch.randn(*shape[:-1], shape[-1] + spare, generator=g).to("cuda", torch.bfloat16)
+        return x[..., :shape[-1]]
+    return rand
+
+
+def _close(x, ref):
+    assert float((x.float() - ref).norm() / ref.norm()) < REL
+
+
+@pytest.mark.parametrize("M,widths,deep,spare", [
+    (1, (8,), (32,), 0), (63, (64, 8), (32, 32), 8), (65, (72, 128, 64), (96, 32), 0),
+    (129, (136,), (64, 32, 160), 64), (257, (256, 40), (224, 64), 0), (300, (520,), (1024,), 8),
+    (513, (264, 8, 8), (320, 32), 0)])
+@pytest.mark.parametrize("tile", TILES)
+def test_sums_of_products(ext, M, widths, deep, spare, tile):
+    """Blocks of columns with their bias or a residual, terms of different
+    depths, rows further apart than they are long; b as (width, k) and (k, width)."""
+    rand = _make(M)
+    for what in ("columns", "rows"):
+        a = [[rand(M, k, spare=spare) for k in deep] for _ in widths]
+        b = [[rand(w, k, spare=spare) if what == "columns" else rand(k, w, spare=spare)
+              for k in deep] for w in widths]
+        bias = [rand(w) if i != 1 else None for i, w in enumerate(widths)]
+        ref = [sum(x.float() @ (y.float().t() if what == "columns" else y.float())
+                   for x, y in zip(xs, ys)) for xs, ys in zip(a, b)]
+        ref = torch.cat([r if c is None else r + c.float() for r, c in zip(ref, bias)], 1)
+        for res in (None, rand(M, sum(widths), spare=spare)):
+            out = rand(M, sum(widths), spare=spare)
+            assert ext.product(a, b, bias, widths, what, [out], res, tile)
+            _close(out, ref if res is None else ref + res.float())
+
+
+@pytest.mark.parametrize("M,F,K,r", [(1, 8, 32, 32), (70, 40, 96, 32), (130, 136, 64, 64),
+                                     (300, 264, 160, 32)])
+@pytest.mark.parametrize("tile", TILES)
+def test_activation(ext, M, F, K, r, tile):
+    """gate and up with an adapter each, and the activation's gradient: the
+    activation of what was rounded into [gate | up]."""
+    rand = _make(F)
+    x, ug, uu = rand(M, K), rand(M, r), rand(M, r)
+    wg, wu, bg, bu = rand(F, K), rand(F, K), rand(F, r), rand(F, r)
+    bias = [rand(F), None]
+    gu, act = rand(M, 2 * F), rand(M, F, spare=24)
+    assert ext.product([[x, ug, uu]] * 2, [[wg, bg, None], [wu, None, bu]], bias, [F, F], "glu",
+                       [gu, act], None, tile)
+    gate = x.float() @ wg.float().t() + ug.float() @ bg.float().t() + bias[0].float()
+    up = x.float() @ wu.float().t() + uu.float() @ bu.float().t()
+    _close(gu, torch.cat([gate, up], 1))
+    gate, up = gu.float().split(F, 1)
+    _close(act, torch.nn.functional.silu(gate) * up)
+
+    g, w, du, a = rand(M, K), rand(K, F), rand(M, r), rand(r, F)
+    d = rand(M, 2 * F, spare=8)
+    assert ext.product([[g, du]], [[w, a]], [None], [F], "glu_bwd", list(d.split(F, 1)), gu, tile)
+    dact = g.float() @ w.float() + du.float() @ a.float()
+    sig = gate.sigmoid()
+    _close(d, torch.cat([dact * up * sig * (1 + gate * (1 - sig)), dact * gate * sig], 1))
+
+
+def test_repeats_itself_in_a_graph(ext):
+    """Shares of K meet in their order, also when a captured launch runs again."""
+    rand = _make(3)
+    a, b, out = rand(200, 4096), rand(96, 4096), rand(200, 96)
+
+    def run(tile):
+        assert ext.product([[a]], [[b]], [None], [96], "columns", [out], None, tile)
+        return out.clone()
+
+    for tile in (64 + 2048, 128 + 1024):
+        first = run(tile)
+        _close(first, a.float() @ b.float().t())
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            again = run(tile)
+        for _ in range(5):
+            out.zero_()
+            graph.replay()
+            assert torch.equal(again, first) and torch.equal(run(tile), first)
+
+
+def test_refuses_what_it_cannot_walk(ext):
+    rand = _make(4)
+    out = rand(64, 64)
+
+    def takes(a, b, out=out, width=64):
+        return ext.product([[a]], [[b]], [None], [width], "columns", [out])
+
+    assert takes(rand(64, 64), rand(64, 64))
+    assert not takes(rand(64, 48), rand(64, 48))              # K no multiple of 32
+    assert not takes(rand(64, 64, spare=4), rand(64, 64))     # rows not on 16 bytes
+    assert not takes(rand(64, 65)[:, 1:], rand(64, 64))       # start not on 16 bytes
+    assert not takes(rand(64, 64).float(), rand(64, 64))
+    assert not takes(rand(64, 64), rand(64, 96))              # other K
+    assert not takes(rand(64, 64).t(), rand(64, 64))          # columns on end
+    assert not takes(rand(64, 64), rand(60, 64), rand(64, 60), 60)
+    assert not takes(rand(64, 64).cpu(), rand(64, 64))
