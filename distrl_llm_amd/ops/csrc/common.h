@@ -146,6 +146,15 @@ template <typename T>
 DEV_INLINE T load_through(const T* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// two floats on 8 bytes
+DEV_INLINE void store_pair(float* p, float x, float y) {
+  store_through(reinterpret_cast<unsigned long long*>(p),
+                (unsigned long long)__float_as_uint(y) << 32 | __float_as_uint(x));
+}
+DEV_INLINE float2 load_pair(const float* p) {
+  const unsigned long long v = load_through(reinterpret_cast<const unsigned long long*>(p));
+  return {__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32))};
+}
 // Until this wave's stores and atomics have arrived.
 DEV_INLINE void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 

@@ -22,12 +22,13 @@
 // partial sums and the bias, norms and rotates them, writes the new token's key
 // and value into the cache and attends over them from LDS, while the first rows
 // of the context are on their way. Slices of one sequence are joined by the last
-// of them to end. As kernels of their own rotation and join took 7.7 and 4.6 us a
+// of them to end (as a launch of its own that took 3 us). As kernels of their own rotation and join took 7.7 and 4.6 us a
 // layer at 160 sequences, 3.0 and 1.3 at eight.
 // K and V are read once per sequence and kv head; bound by HBM.
 // 160 sequences of 420..1550 tokens sharing prompts, 28/4 heads of 128
 // (251 MB of distinct rows): 157 us with one lane a token on vector FMAs,
-// 68 us now; 3 sequences of 911..3777, 14/2 heads of 64: 43 -> 12.
+// 67 us now; 3 sequences of 911..3777, 14/2 heads of 64: 43 -> 8.4, a chain of
+// length and pages, rows, products and the slices' join.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
@@ -78,17 +79,30 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
                          float* __restrict__ o_part,                // (cs, N, H, D)
                          float* __restrict__ ml_part,               // (cs, N, H, 2)
                          int H, int KV, int max_nb, int block_size, int bs_shift,
-                         float scale_log2, int64_t q_row_stride, int slice_len, Packed src) {
+                         float scale_log2, int64_t q_row_stride, int slice_len,
+                         unsigned long long* __restrict__ there,    // (N, KV, cs)
+                         unsigned long long tag, Packed src) {
   constexpr int KS = D / 32, DT = D / 16;
   constexpr int LPR = D / 8, RPL = 64 / LPR, NL = CHUNK / RPL;   // lanes of a row, rows of a load
   const int seq = blockIdx.x, kv = blockIdx.y, z = blockIdx.z, N = gridDim.x;
   const int group = H / KV;
-  const int len = ctx_lens[seq];
-  // no further than the block table reaches
-  const int c0 = z * slice_len, c1 = min(len, min(c0 + slice_len, max_nb * block_size));
-  if (z > 0 && c0 >= len) return;       // an empty slice is not read
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63, g = l >> 4, lr = l & 15;
+  const int* bt = block_tables + (int64_t)seq * max_nb;
+  const int c0 = z * slice_len;
+  auto block_of = [&](int t) { return bs_shift >= 0 ? t >> bs_shift : t / block_size; };
+  // the page of this lane's token l % 32 of a chunk, whether there is one or not
+  auto page_of = [&](int t0) {
+    return max_nb > 0 ? bt[min(block_of(t0 + (l & 31)), max_nb - 1)] : 0;
+  };
+  // What a workgroup needs first is on its way at once: the length, its pages, and
+  // below what its queries are made of. One behind the other they are a microsecond each.
+  int t0 = c0 + wave * CHUNK;
+  int page = page_of(t0);
+  const int len = ctx_lens[seq];
+  // no further than the block table reaches
+  const int c1 = min(len, min(c0 + slice_len, max_nb * block_size));
+  if (z > 0 && c0 >= len) return;       // an empty slice is not read
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
   char* ktile = smem + wave * (2 * CHUNK * D * 2);      // also 16 heads x D floats
@@ -107,16 +121,12 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
   #pragma unroll
   for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int* bt = block_tables + (int64_t)seq * max_nb;
   const int row_elems = KV * D;
   bf16v8 kf[NL], vf[NL];
-  int row;                              // of the pool, of this lane's token l % 32 of a chunk
-  auto lookup = [&](int t0) {
+  auto load = [&](int t0) {             // page: of this chunk
     const int t = min(t0 + (l & 31), c1 - 1);           // past the end: weight zero
-    const int b = bs_shift >= 0 ? t >> bs_shift : t / block_size;
-    row = bt[b] * block_size + (t - b * block_size);
-  };
-  auto load = [&] {
+    // of the pool, of this lane's token
+    const int row = __shfl(page, t - t0, WAVE) * block_size + (t - block_of(t) * block_size);
     #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int64_t at = (int64_t)__shfl(row, i * RPL + l / LPR, WAVE) * row_elems + kv * D +
@@ -126,14 +136,15 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
     }
   };
 
-  int t0 = c0 + wave * CHUNK;
-  if (t0 < c1) {
-    lookup(t0);
-    load();
-    lookup(t0 + NW * CHUNK);
-  }
+  auto begin = [&] {
+    if (t0 < c1) {
+      load(t0);
+      page = page_of(t0 + NW * CHUNK);
+    }
+  };
   bf16v8 qf[KS];
   if constexpr (SRC == QUERIES) {
+    begin();
     #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const __hip_bfloat16* qp = q + seq * q_row_stride + (kv * group + min(lr, group - 1)) * D;
@@ -144,52 +155,90 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
     // then the value, eight elements a thread
     constexpr int PER = D / 16;
     const int width = (H + 2 * KV) * D;
-    auto start = [&](float (&x)[8], int at) {           // the bias, or zero
-      #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = 0.f;
-      if (src.bias) {
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(src.bias + at);
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = bf2f(v.v[j]);
-      }
-    };
-    auto take = [&](float (&x)[8], int at) {
-      if constexpr (SRC == ROWS) {
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(src.rows + (int64_t)seq * width + at);
-        #pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = bf2f(v.v[j]);
-      } else {
-        start(x, at);
-        add_parts8(x, src.parts + (int64_t)seq * width + at, (int64_t)N * width, src.splits);
-      }
-    };
     const int64_t slot = src.slots[seq];
     const int units = (group + (owner ? 1 : 0)) * PER, all = units + (owner ? D / 8 : 0);
-    for (int u = threadIdx.x; u < all; u += NW * 64) {
+    // eight elements at `at` and eight at `other` of this sequence: the rows, or the
+    // first four partial sums of them
+    struct Raw {
       bf16x8 x, y;
+      f32x4v part[4][4];
+    };
+    auto fetch = [&](Raw& r, int at, int other) {
+      if constexpr (SRC == ROWS) {
+        const __hip_bfloat16* p = src.rows + (int64_t)seq * width;
+        r.x = *reinterpret_cast<const bf16x8*>(p + at);
+        r.y = *reinterpret_cast<const bf16x8*>(p + other);
+      } else {
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float* p = src.parts + ((int64_t)min(i, src.splits - 1) * N + seq) * width;
+          #pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            r.part[i][h] = *reinterpret_cast<const f32x4v*>(p + at + 4 * h);
+            r.part[i][2 + h] = *reinterpret_cast<const f32x4v*>(p + other + 4 * h);
+          }
+        }
+      }
+    };
+    auto take = [&](const Raw& r, float (&x)[8], float (&y)[8], int at, int other) {
+      if constexpr (SRC == ROWS) {
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) { x[j] = bf2f(r.x.v[j]); y[j] = bf2f(r.y.v[j]); }
+      } else {
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          x[j] = src.bias ? bf2f(src.bias[at + j]) : 0.f;
+          y[j] = src.bias ? bf2f(src.bias[other + j]) : 0.f;
+        }
+        #pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (i < src.splits) {
+            #pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              x[j] += r.part[i][j / 4].v[j % 4];
+              y[j] += r.part[i][2 + j / 4].v[j % 4];
+            }
+          }
+        if (src.splits > 4)
+          add_parts8x2(x, y, src.parts + ((int64_t)4 * N + seq) * width + at, other - at,
+                       (int64_t)N * width, src.splits - 4);
+      }
+    };
+    // where unit u's elements are: of the value eight, twice
+    auto places = [&](int u, int& at, int& other) {
+      if (u >= units) {
+        at = other = (H + KV + kv) * D + (u - units) * 8;
+      } else {
+        const int head = u / PER;
+        at = (head < group ? kv * group + head : H + kv) * D + u % PER * 8;
+        other = at + D / 2;
+      }
+    };
+    Raw raw;
+    int at, other;
+    if ((int)threadIdx.x < all) {
+      places(threadIdx.x, at, other);
+      fetch(raw, at, other);
+    }
+    begin();
+    for (int u = threadIdx.x; u < all; u += NW * 64) {
+      if (u >= NW * 64) {
+        places(u, at, other);
+        fetch(raw, at, other);
+      }
+      bf16x8 x, y;
+      float x1[8], x2[8];
+      take(raw, x1, x2, at, other);
       if (u >= units) {
         const int c = (u - units) * 8;
-        float v[8];
-        take(v, (H + KV + kv) * D + c);
         #pragma unroll
-        for (int j = 0; j < 8; ++j) x.v[j] = f2bf(v[j]);
+        for (int j = 0; j < 8; ++j) x.v[j] = f2bf(x1[j]);
         *reinterpret_cast<bf16x8*>(fresh + (group + 1) * D + c) = x;
         if (slot >= 0)
           *reinterpret_cast<bf16x8*>(src.vcache + (slot * KV + kv) * D + c) = x;
         continue;
       }
       const int head = u / PER, c = u % PER * 8;        // head == group: the key
-      const int at = (head < group ? kv * group + head : H + kv) * D + c;
-      float x1[8], x2[8];
-      if constexpr (SRC == ROWS) {
-        take(x1, at);
-        take(x2, at + D / 2);
-      } else {
-        start(x1, at);
-        start(x2, at + D / 2);
-        add_parts8x2(x1, x2, src.parts + (int64_t)seq * width + at, D / 2, (int64_t)N * width,
-                     src.splits);
-      }
       const __hip_bfloat16* nw = head < group ? src.q_norm : src.k_norm;
       if (nw) {
         float ss = 0.f;
@@ -243,8 +292,8 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
       *reinterpret_cast<bf16v8*>(tile + v_off<D>(r, c)) = vf[i];
     }
     if (more) {
-      load();
-      lookup(t0 + 2 * NW * CHUNK);
+      load(t0 + NW * CHUNK);
+      page = page_of(t0 + 2 * NW * CHUNK);
     }
     __builtin_amdgcn_wave_barrier();
     f32x4 st[2];
@@ -341,34 +390,58 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
       *reinterpret_cast<bf16v4*>(out + head * D + d) = y;
     } else {
       const int64_t at = (int64_t)z * N * H + head;
-      *reinterpret_cast<f32x4*>(o_part + at * D + d) = o;
-      if (d == 0) { ml_part[at * 2] = top; ml_part[at * 2 + 1] = total; }
+      #pragma unroll
+      for (int r = 0; r < 4; r += 2) store_pair(o_part + at * D + d + r, o[r], o[r + 1]);
+      if (d == 0) store_pair(ml_part + at * 2, top, total);
     }
   }
-  if constexpr (SRC != QUERIES) {
+  {
     if (whole) return;
     // the last slice of the sequence and kv head to end joins them
-    __shared__ int before;
-    __threadfence();
+    __shared__ int last;
+    stores_done();
     __syncthreads();
     const int n = min((len + slice_len - 1) / slice_len, (int)gridDim.z);
-    int* arrived = src.arrived + seq * KV + kv;
-    if (threadIdx.x == 0) before = atomicAdd(arrived, 1);
+    if constexpr (SRC == QUERIES) {
+      if (wave == 0) {
+        const bool all = all_there(there + ((int64_t)seq * KV + kv) * gridDim.z, n, z, tag);
+        if (l == 0) last = all;
+      }
+    } else {
+      if (threadIdx.x == 0) last = atomicAdd(src.arrived + seq * KV + kv, 1) == n - 1;
+    }
     __syncthreads();
-    if (before != n - 1) return;
-    __threadfence();
-    if (threadIdx.x == 0) atomicExch(arrived, 0);
+    if (!last) return;
+    if (SRC != QUERIES && threadIdx.x == 0) src.arrived[seq * KV + kv] = 0;
     for (int i = threadIdx.x; i < group * (D / 4); i += NW * 64) {
       const int h = i / (D / 4), d = i % (D / 4) * 4;
       const int64_t head = (int64_t)seq * H + kv * group + h, step = (int64_t)N * H;
+      // with the maximum of those before: one look at each
       float top = -1e30f, total = 0.f;
-      for (int s = 0; s < n; ++s) top = fmaxf(top, ml_part[(s * step + head) * 2]);
       f32x4 o = {0.f, 0.f, 0.f, 0.f};
-      for (int s = 0; s < n; ++s) {
-        const int64_t at = s * step + head;
-        const float f = __builtin_amdgcn_exp2f(ml_part[at * 2] - top);
-        total += f * ml_part[at * 2 + 1];
-        o += *reinterpret_cast<const f32x4*>(o_part + at * D + d) * f;
+      for (int s0 = 0; s0 < n; s0 += 4) {
+        float2 ml[4], lo[4], hi[4];
+        #pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int64_t at = min(s0 + s, n - 1) * step + head;
+          ml[s] = load_pair(ml_part + at * 2);
+          lo[s] = load_pair(o_part + at * D + d);
+          hi[s] = load_pair(o_part + at * D + d + 2);
+        }
+        float high = top;
+        #pragma unroll
+        for (int s = 0; s < 4; ++s) high = fmaxf(high, ml[s].x);
+        const float old = __builtin_amdgcn_exp2f(top - high);
+        total *= old;
+        o *= old;
+        top = high;
+        #pragma unroll
+        for (int s = 0; s < 4; ++s)
+          if (s0 + s < n) {
+            const float f = __builtin_amdgcn_exp2f(ml[s].x - top);
+            total += f * ml[s].y;
+            o += f32x4{lo[s].x, lo[s].y, hi[s].x, hi[s].y} * f;
+          }
       }
       const float inv = total > 0.f ? 1.f / total : 0.f;
       bf16v4 y;
@@ -377,36 +450,6 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
       *reinterpret_cast<bf16v4*>(out + head * D + d) = y;
     }
   }
-}
-
-// Joins the slices of a sequence that has more than one. grid (N, H), one wave.
-template <int D>
-__global__ __launch_bounds__(64)
-void paged_decode_combine_kernel(const float* __restrict__ o_part,
-                                 const float* __restrict__ ml_part,
-                                 const int* __restrict__ ctx_lens,
-                                 __hip_bfloat16* __restrict__ out, int H, int slice_len,
-                                 int cs) {
-  const int seq = blockIdx.x, h = blockIdx.y, N = gridDim.x, lane = threadIdx.x;
-  const int len = ctx_lens[seq];
-  if (len <= slice_len) return;                         // written already
-  const int n = min((len + slice_len - 1) / slice_len, cs);
-  const int64_t head = (int64_t)seq * H + h, step = (int64_t)N * H;
-  float top = -1e30f;
-  for (int z = 0; z < n; ++z) top = fmaxf(top, ml_part[(z * step + head) * 2]);
-  float total = 0.f, o[D / 64];
-  #pragma unroll
-  for (int e = 0; e < D / 64; ++e) o[e] = 0.f;
-  for (int z = 0; z < n; ++z) {
-    const int64_t at = z * step + head;
-    const float w = __builtin_amdgcn_exp2f(ml_part[at * 2] - top);
-    total += w * ml_part[at * 2 + 1];
-    #pragma unroll
-    for (int e = 0; e < D / 64; ++e) o[e] += w * o_part[at * D + lane + e * 64];
-  }
-  const float inv = 1.f / total;
-  #pragma unroll
-  for (int e = 0; e < D / 64; ++e) out[head * D + lane + e * 64] = f2bf(o[e] * inv);
 }
 
 template <int D, int NW, int SRC>
@@ -419,11 +462,13 @@ void launch_decode(const __hip_bfloat16* q, const torch::Tensor& kcache,
   auto stream = at::cuda::getCurrentCUDAStream();
   torch::Tensor part;
   float *o_p = nullptr, *ml_p = nullptr;
+  unsigned long long* there = nullptr;
   if (cs > 1) {
     const int64_t heads = (int64_t)cs * N * H;
-    part = torch::empty({heads * (D + 2)}, out.options().dtype(at::kFloat));
+    part = torch::empty({heads * (D + 2) + 2ll * N * KV * cs}, out.options().dtype(at::kFloat));
     o_p = part.data_ptr<float>();
     ml_p = o_p + heads * D;
+    there = reinterpret_cast<unsigned long long*>(ml_p + heads * 2);   // of QUERIES alone
   }
   auto* o = reinterpret_cast<__hip_bfloat16*>(out.data_ptr());
   const int smem = NW * (2 * CHUNK * D * 2 + 16 * 2 * 4) + (SRC == QUERIES ? 0 : (H / KV + 2) * D * 2);
@@ -432,10 +477,7 @@ void launch_decode(const __hip_bfloat16* q, const torch::Tensor& kcache,
                      reinterpret_cast<const __hip_bfloat16*>(vcache.data_ptr()),
                      bt.data_ptr<int>(), ctx.data_ptr<int>(), o, o_p, ml_p, H, KV,
                      (int)bt.size(1), block_size, shift, scale * LOG2E, q_row_stride, slice_len,
-                     src);
-  if (SRC == QUERIES && cs > 1)
-    hipLaunchKernelGGL((paged_decode_combine_kernel<D>), dim3(N, H), dim3(64), 0, stream, o_p,
-                       ml_p, ctx.data_ptr<int>(), o, H, slice_len, cs);
+                     there, cs > 1 ? arrival_tag() : 0, src);
 }
 
 // Slices of the context (known here: a table's width, not its sequence's

@@ -337,6 +337,25 @@ def test_paged_decode_stays_in_its_table(ext, N, nb):
     assert torch.equal(ext.paged_attention_decode(q, kc, vc, bt, lens, 0.1), ref)
 
 
+def test_paged_decode_slices_in_a_graph(ext):
+    """Slices of a context find each other in every replay of a capture."""
+    H, KV, D, bs, nb = 8, 2, 64, 16, 130
+    kc, vc = (_rand((3 * nb, bs, KV, D), i) for i in (1, 2))
+    q = _rand((3, H, D), 3)
+    bt = torch.randperm(3 * nb, generator=torch.Generator().manual_seed(0)).view(3, nb).int().cuda()
+    lens = torch.tensor([2080, 1, 1300], dtype=torch.int32, device="cuda")
+    ref = ext.paged_attention_decode(q, kc, vc, bt, lens, 0.125)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ext.paged_attention_decode(q, kc, vc, bt, lens, 0.125)
+    for _ in range(5):
+        out.zero_()
+        graph.replay()
+        assert torch.equal(out, ref)
+        assert torch.equal(ext.paged_attention_decode(q, kc, vc, bt, lens, 0.125), ref)
+
+
 def test_paged_decode_reads_packed_rows(ext):
     """Query heads at the head of wider rows, at any alignment."""
     H, KV, D, N = 14, 2, 64, 3
