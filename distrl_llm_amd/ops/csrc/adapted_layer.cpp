@@ -45,6 +45,10 @@ struct NoAutocast {
 
 Tensor columns(const Tensor& t, int64_t from, int64_t n) { return t.narrow(1, from, n); }
 
+// Rows from which 32 of them a workgroup fill the chip: the activation then carries its
+// adapter inputs along.
+constexpr int64_t FULL = 8192;
+
 Tensor heads(const Tensor& t, int64_t head_dim) {
   return t.view({t.size(0), t.size(1) / head_dim, head_dim});
 }
@@ -411,6 +415,7 @@ Tensors feed_forward_half_fwd(Tensor x, Tensor norm, double eps, Tensors W,
   auto au = apart_rows(rows, inner + d_ad.pad, x.options());
   auto act = columns(au, 0, inner);
   Tensor gu;
+  bool ready = false;                     // act's adapter inputs
   if (!apart(rows, 2 * inner, hidden) && !library(rows, 2 * inner, hidden)) {
     gu = at::empty({rows, 2 * inner}, x.options());
     const auto both = blocks(h, columns(hu, hidden, in.pad), {W[0], W[1]}, in, bias);
@@ -421,9 +426,10 @@ Tensors feed_forward_half_fwd(Tensor x, Tensor norm, double eps, Tensors W,
   }
   if (!gu.defined()) {
     gu = projected(hu, {W[0], W[1]}, in, bias);
-    silu_mul_packed_into(gu, act);
+    ready = rows >= FULL && silu_mul_inputs(gu, act, A[2], scales[2], columns(au, inner, d_ad.pad));
+    if (!ready) silu_mul_packed_into(gu, act);
   }
-  d_ad.down(act, columns(au, inner, d_ad.pad));
+  if (!ready) d_ad.down(act, columns(au, inner, d_ad.pad));
   auto y = projected(au, {W[2]}, d_ad, {}, x);
   return {y, hu, gu, au};
 }
@@ -444,6 +450,7 @@ Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tenso
   auto dgate = columns(dyu, 0, inner), dup = columns(dyu, inner, inner),
        du = columns(dyu, 2 * inner, in.pad);
   Tensor dud;
+  bool ready = false;                     // dgate's and dup's adapter inputs
   if (!apart(rows, hidden, inner) && !library(rows, hidden, inner)) {
     auto both = at::empty({rows, d_ad.pad}, x.options());
     d_ad.up({g}, both);
@@ -452,10 +459,12 @@ Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tenso
   }
   if (!dud.defined()) {
     const auto [dact, du2] = through(g, W[2], d_ad);
-    silu_mul_bwd_packed(dact, gu, dgate, dup);
+    ready = rows >= FULL &&
+            silu_mul_bwd_inputs(dact, gu, dgate, dup, {B[0], B[1]}, {scales[0], scales[1]}, du);
+    if (!ready) silu_mul_bwd_packed(dact, gu, dgate, dup);
     dud = du2;
   }
-  in.up({dgate, dup}, du);
+  if (!ready) in.up({dgate, dup}, du);
   auto s = sums({{h, du, false},
                  {act, dud, false},
                  {g, ud, true},

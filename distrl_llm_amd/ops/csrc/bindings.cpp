@@ -126,6 +126,12 @@ void rmsnorm_fwd_into(torch::Tensor x, torch::Tensor w, double eps,
 void silu_mul_packed_into(torch::Tensor gu, torch::Tensor out);
 void silu_mul_bwd_packed(torch::Tensor dy, torch::Tensor gu,
                          torch::Tensor dgate, torch::Tensor dup);
+bool silu_mul_inputs(torch::Tensor gu, torch::Tensor act, torch::Tensor m,
+                     double scale, torch::Tensor out);
+bool silu_mul_bwd_inputs(torch::Tensor dact, torch::Tensor gu,
+                         torch::Tensor dgate, torch::Tensor dup,
+                         std::vector<torch::Tensor> m,
+                         std::vector<double> scales, torch::Tensor out);
 bool adapter_input(torch::Tensor x, std::vector<torch::Tensor> m,
                    std::vector<double> scales, torch::Tensor out, bool k_major);
 std::vector<torch::Tensor> attention_half_fwd(
@@ -228,6 +234,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual + partial sums (+ adapter), then RMSNorm", py::arg("parts"),
         py::arg("res"), py::arg("w"), py::arg("eps"),
         py::arg("bt") = py::none());
+  m.def("silu_mul_inputs", &silu_mul_inputs,
+        "SiLU*mul with the adapter inputs of its output (tests)");
+  m.def("silu_mul_bwd_inputs", &silu_mul_bwd_inputs,
+        "SiLU*mul's gradients with their adapter inputs (tests)");
   m.def("adapter_input", &adapter_input, "scaled inputs of LoRA adapters");
   m.def("attention_half_fwd", &attention_half_fwd,
         "an adapted layer's attention half");

@@ -82,6 +82,32 @@ def test_activation(ext, M, F, K, r, tile):
     _close(d, torch.cat([dact * up * sig * (1 + gate * (1 - sig)), dact * gate * sig], 1))
 
 
+@pytest.mark.parametrize("M,F", [(1, 8), (31, 120), (33, 128), (64, 136), (100, 400), (70, 1032)])
+@pytest.mark.parametrize("r,spare", [((32, 32), 0), ((8, 24), 4), ((64, 40), 0)])
+def test_activation_with_adapter_inputs(ext, M, F, r, spare):
+    """Edges of 32 rows and steps of 128 columns; the products are those of
+    what was rounded and written, spare columns zero."""
+    rand = _make(M + F)
+    gu, act = rand(M, 2 * F), rand(M, F, spare=16)
+    m, out = rand(r[0], F), rand(M, r[0] + spare, spare=12)
+    assert ext.silu_mul_inputs(gu, act, m, 0.5, out)
+    gate, up = gu.float().split(F, 1)
+    _close(act, torch.nn.functional.silu(gate) * up)
+    _close(out[:, :r[0]], act.float() @ m.float().t() * 0.5)
+    assert not out[:, r[0]:].any()
+
+    dact, d = rand(M, F), rand(M, 2 * F + 8)
+    dgate, dup = d[:, :F], d[:, F:2 * F]
+    b, du = [rand(F, x) for x in r], rand(M, sum(r) + spare)
+    assert ext.silu_mul_bwd_inputs(dact, gu, dgate, dup, b, [0.5, 2.0], du)
+    sig = gate.sigmoid()
+    _close(dgate, dact.float() * up * sig * (1 + gate * (1 - sig)))
+    _close(dup, dact.float() * gate * sig)
+    _close(du[:, :r[0]], dgate.float() @ b[0].float() * 0.5)
+    _close(du[:, r[0]:sum(r)], dup.float() @ b[1].float() * 2.0)
+    assert not du[:, sum(r):].any()
+
+
 def test_repeats_itself_in_a_graph(ext):
     """Shares of K meet in their order, also when a captured launch runs again."""
     rand = _make(3)
