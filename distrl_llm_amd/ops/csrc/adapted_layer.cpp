@@ -487,3 +487,64 @@ Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tenso
   out.insert(out.begin(), dx);
   return out;
 }
+
+namespace {
+
+bool all_bf16(const Tensors& ts) {
+  for (const auto& t : ts)
+    if (!t.is_cuda() || t.scalar_type() != at::kBFloat16) return false;
+  return true;
+}
+
+// u of the adapters on x; undefined where own products don't take their ranks
+Tensor adapter_side(const Tensor& x, const Adapters& ad) {
+  for (const auto r : ad.ranks)
+    if (r % 32 != 0) return {};
+  auto u = at::empty({x.size(0), ad.pad}, x.options());
+  ad.down(x, u);
+  return u;
+}
+
+}  // namespace
+
+// x W^T of projections of one input side by side, with their adapters (one each, or
+// none at all) and biases, or + res, in one rounding. None where own products don't
+// take the operands.
+Optional adapted_projection(Tensor x, Tensors W, std::vector<Optional> bias, Tensors A, Tensors B,
+                            std::vector<double> scales, Optional res) {
+  if (!all_bf16(W) || !all_bf16(A) || !all_bf16(B) || !all_bf16({x}) || x.size(0) == 0) return {};
+  int64_t width = 0;
+  for (const auto& w : W) width += w.size(0);
+  std::vector<ProductBlock> sums;
+  if (A.empty()) {
+    for (size_t i = 0; i < W.size(); ++i) sums.push_back({W[i].size(0), {{x, W[i]}}, bias.at(i)});
+  } else {
+    TORCH_CHECK(A.size() == W.size());
+    const Adapters ad(A, B, scales);
+    const auto u = adapter_side(x, ad);
+    if (!u.defined()) return {};
+    sums = blocks(x, u, W, ad, bias);
+  }
+  auto out = at::empty({x.size(0), width}, x.options());
+  if (!product(sums, false, out, res)) return {};
+  return out;
+}
+
+// silu(x Wg^T) * (x Wu^T), the same way
+Optional adapted_activation(Tensor x, Tensors W, Tensors A, Tensors B, std::vector<double> scales) {
+  if (!all_bf16(W) || !all_bf16(A) || !all_bf16(B) || !all_bf16({x}) || x.size(0) == 0) return {};
+  TORCH_CHECK(W.size() == 2 && (A.empty() || A.size() == 2));
+  const int64_t inner = W[0].size(0);
+  ProductBlock gate{inner, {{x, W[0]}}, {}}, up{inner, {{x, W[1]}}, {}};
+  if (!A.empty()) {
+    const Adapters ad(A, B, scales);
+    const auto u = adapter_side(x, ad);
+    if (!u.defined()) return {};
+    const auto ug = ad.part(u, 0), uu = ad.part(u, 1);
+    gate.terms.insert(gate.terms.end(), {{ug, B[0]}, {uu, {}}});
+    up.terms.insert(up.terms.end(), {{ug, {}}, {uu, B[1]}});
+  }
+  auto act = at::empty({x.size(0), inner}, x.options());
+  if (!product_glu(gate, up, {}, act)) return {};
+  return act;
+}

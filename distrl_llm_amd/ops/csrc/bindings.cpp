@@ -126,6 +126,14 @@ void rmsnorm_fwd_into(torch::Tensor x, torch::Tensor w, double eps,
 void silu_mul_packed_into(torch::Tensor gu, torch::Tensor out);
 void silu_mul_bwd_packed(torch::Tensor dy, torch::Tensor gu,
                          torch::Tensor dgate, torch::Tensor dup);
+c10::optional<torch::Tensor> adapted_projection(
+    torch::Tensor x, std::vector<torch::Tensor> W,
+    std::vector<c10::optional<torch::Tensor>> bias, std::vector<torch::Tensor> A,
+    std::vector<torch::Tensor> B, std::vector<double> scales,
+    c10::optional<torch::Tensor> res);
+c10::optional<torch::Tensor> adapted_activation(
+    torch::Tensor x, std::vector<torch::Tensor> W, std::vector<torch::Tensor> A,
+    std::vector<torch::Tensor> B, std::vector<double> scales);
 bool silu_mul_inputs(torch::Tensor gu, torch::Tensor act, torch::Tensor m,
                      double scale, torch::Tensor out);
 bool silu_mul_bwd_inputs(torch::Tensor dact, torch::Tensor gu,
@@ -234,6 +242,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual + partial sums (+ adapter), then RMSNorm", py::arg("parts"),
         py::arg("res"), py::arg("w"), py::arg("eps"),
         py::arg("bt") = py::none());
+  m.def("adapted_projection", &adapted_projection, py::arg("x"), py::arg("w"),
+        py::arg("bias"), py::arg("a"), py::arg("b"), py::arg("scales"),
+        py::arg("res") = py::none(),
+        "projections of one input with adapters, biases or a residual, or None");
+  m.def("adapted_activation", &adapted_activation, py::arg("x"), py::arg("w"),
+        py::arg("a"), py::arg("b"), py::arg("scales"),
+        "SiLU*mul of two projections with adapters, or None");
   m.def("silu_mul_inputs", &silu_mul_inputs,
         "SiLU*mul with the adapter inputs of its output (tests)");
   m.def("silu_mul_bwd_inputs", &silu_mul_bwd_inputs,

@@ -20,10 +20,10 @@ struct ProductBlock {
 bool product(const std::vector<ProductBlock>& blocks, bool rows_of_b, const at::Tensor& out,
              const c10::optional<at::Tensor>& res = {}, int tile = 0);
 
-// gu <- [gate | up], act <- silu(gate) * up of what was rounded into gu; the terms of
+// gu, if wanted, <- [gate | up], act <- silu(gate) * up of both rounded; the terms of
 // both have the same a, one for one
-bool product_glu(const ProductBlock& gate, const ProductBlock& up, const at::Tensor& gu,
-                 const at::Tensor& act, int tile = 0);
+bool product_glu(const ProductBlock& gate, const ProductBlock& up,
+                 const c10::optional<at::Tensor>& gu, const at::Tensor& act, int tile = 0);
 
 // dgate, dup <- the activation's gradients for dact = the block, b (k, width)
 bool product_glu_bwd(const ProductBlock& block, const at::Tensor& gu, const at::Tensor& dgate,

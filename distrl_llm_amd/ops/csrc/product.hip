@@ -50,7 +50,7 @@ struct Args {
   int first[BLOCKS], terms[BLOCKS];     // of a block, or of gate and up
   int width[BLOCKS], tiles[BLOCKS];     // columns, and columns of tiles
   const __hip_bfloat16* bias[BLOCKS];
-  __hip_bfloat16* c;                    // GLU: [gate | up]
+  __hip_bfloat16* c;                    // GLU: [gate | up], or null
   int ldc;
   const __hip_bfloat16* res;
   int ldr;
@@ -402,9 +402,9 @@ void product_kernel(const Args args) {
         put(args.dgate + (int64_t)m * args.ldd + n[j], o);
         put(args.dup + (int64_t)m * args.ldd + n[j], p);
       } else {
-        put(args.c + (int64_t)m * args.ldc + c0 + n[j], o);
+        if (MODE == PLAIN || args.c) put(args.c + (int64_t)m * args.ldc + c0 + n[j], o);
         if constexpr (MODE == GLU) {
-          put(args.c + (int64_t)m * args.ldc + N + n[j], p);
+          if (args.c) put(args.c + (int64_t)m * args.ldc + N + n[j], p);
           put(args.act + (int64_t)m * args.ldact + n[j], q);
         }
       }
@@ -564,17 +564,19 @@ bool product(const std::vector<ProductBlock>& blocks, bool rows_of_b, const at::
   return true;
 }
 
-bool product_glu(const ProductBlock& gate, const ProductBlock& up, const at::Tensor& gu,
-                 const at::Tensor& act, int tile) {
+bool product_glu(const ProductBlock& gate, const ProductBlock& up,
+                 const c10::optional<at::Tensor>& gu, const at::Tensor& act, int tile) {
   Args o{};
   if (!fill(o, {&gate, &up}, false) || gate.width != up.width ||
-      gate.terms.size() != up.terms.size() || !shaped(gu, o.M, 2 * gate.width) ||
+      gate.terms.size() != up.terms.size() || (gu && !shaped(*gu, o.M, 2 * gate.width)) ||
       !shaped(act, o.M, gate.width))
     return false;
   for (size_t i = 0; i < gate.terms.size(); ++i)
     if (!gate.terms[i].a.is_same(up.terms[i].a)) return false;
-  o.c = ptr(gu);
-  o.ldc = (int)gu.stride(0);
+  if (gu) {
+    o.c = ptr(*gu);
+    o.ldc = (int)gu->stride(0);
+  }
   o.act = ptr(act);
   o.ldact = (int)act.stride(0);
   by_size<false, GLU>(o, 2, tile);

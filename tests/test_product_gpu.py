@@ -108,6 +108,41 @@ def test_activation_with_adapter_inputs(ext, M, F, r, spare):
     assert not du[:, sum(r):].any()
 
 
+@pytest.mark.parametrize("M", [1, 57, 300])
+@pytest.mark.parametrize("r", [0, 32, 64])
+def test_adapted_projection_and_activation(ext, M, r):
+    """A layer's projections with adapters or without, bias or residual."""
+    rand, K, widths = _make(M + r), 160, (96, 40, 40)
+    x, res, n = rand(M, K), rand(M, sum(widths)), len(widths) if r else 0
+    w, bias = [rand(k, K) for k in widths], [rand(k) for k in widths]
+    a, b = [rand(r, K) for _ in range(n)], [rand(k, r) for k in widths[:n]]
+    # the adapters' inputs as they are rounded: their error is not this one's
+    u = [(x.float() @ y.float().t() * 0.25).to(torch.bfloat16).float() for y in a]
+    y = [x.float() @ v.float().t() for v in w]
+    y = [v + u[i] @ b[i].float().t() if r else v for i, v in enumerate(y)]
+    # 1e-3: of u, 2^-8 at most, a few land on the other side of a rounding
+    out = ext.adapted_projection(x, w, bias, a, b, [0.25] * n)
+    ref = torch.cat([v + c.float() for v, c in zip(y, bias)], 1)
+    assert float((out.float() - ref).norm() / ref.norm()) < REL + 1e-3
+    out = ext.adapted_projection(x, w, [None] * 3, a, b, [0.25] * n, res)
+    ref = torch.cat(y, 1) + res.float()
+    assert float((out.float() - ref).norm() / ref.norm()) < REL + 1e-3
+    act = ext.adapted_activation(x, w[1:], a[1:], b[1:], [0.25] * max(n - 1, 0))
+    gate, up = (v.to(torch.bfloat16).float() for v in y[1:])
+    ref = torch.nn.functional.silu(gate) * up
+    assert float((act.float() - ref).norm() / ref.norm()) < 3 * REL   # gate, up, act
+
+
+def test_adapted_projection_leaves_the_rest(ext):
+    rand = _make(5)
+    x, w = rand(40, 64), rand(64, 64)
+    for a, b in ((rand(16, 64), rand(64, 16)), (rand(32, 64).float(), rand(64, 32).float())):
+        assert ext.adapted_projection(x, [w], [None], [a], [b], [1.0]) is None
+        assert ext.adapted_activation(x, [w, w], [a, a], [b, b], [1.0, 1.0]) is None
+    assert ext.adapted_projection(x[:0], [w], [None], [], [], []) is None
+    assert ext.adapted_projection(x.float(), [w], [None], [], [], []) is None
+
+
 def test_repeats_itself_in_a_graph(ext):
     """Shares of K meet in their order, also when a captured launch runs again."""
     rand = _make(3)
