@@ -23,7 +23,14 @@ DEV_INLINE bf16x8 load8(const __hip_bfloat16* p) {
   __builtin_memcpy(&v, p, sizeof v);
   return v;
 }
-DEV_INLINE void store8(__hip_bfloat16* p, const bf16x8& v) { __builtin_memcpy(p, &v, sizeof v); }
+// Past the caches: what is written here is of the size of the logits.
+DEV_INLINE void store8(__hip_bfloat16* p, const bf16x8& v) {
+  typedef int Four __attribute__((ext_vector_type(4)));
+  typedef Four Anywhere __attribute__((aligned(2)));
+  Four q;
+  __builtin_memcpy(&q, &v, sizeof q);
+  __builtin_nontemporal_store(q, (Anywhere*)p);
+}
 
 // One workgroup per (b, t) row; single streaming pass, online logsumexp: a
 // thread takes 32 values at a time, the next 32 on their way, compares their
@@ -146,17 +153,22 @@ void loss_rows_kernel(const float* __restrict__ token_logp, const float* __restr
   if (threadIdx.x == 0) *loss = sum;
 }
 
-// Rows are read and written once, four loads of a thread in flight: 2408 rows of 152064,
-// a quarter of them of weight zero and only written, 268 -> 258 us, the rate of a copy.
-template <typename T>
-__global__ __launch_bounds__(256)
+// Memory alone: rows are read and written once, four loads of a thread in flight. The
+// gradient goes past the caches (written through them it drove out the logits before
+// they were read, and waited for room: 2408 rows of 152064, a quarter of them of weight
+// zero and only written, 440 -> 268 us, 600 rows 127 -> 55). The rows run from the last,
+// whose logits the forward pass read last: both passes 401 -> 375 us, with THREADS 1024
+// for rows that give each four loads at least (32768 values: 242 and 242 us for 8000
+// rows) 345.
+template <typename T, int THREADS>
+__global__ __launch_bounds__(THREADS)
 void loss_bwd_kernel(const T* __restrict__ logits,
                      const int64_t* __restrict__ targets,
                      const float* __restrict__ w,
                      const float* __restrict__ lse,
                      const float* __restrict__ dloss,   // scalar, or null: 1
                      T* __restrict__ dlogits, int V) {
-  const int64_t row = blockIdx.x;
+  const int64_t row = gridDim.x - 1 - blockIdx.x;
   const T* lr = logits + row * V;
   T* dr = dlogits + row * V;
   const float wv = dloss ? w[row] * *dloss : w[row];
@@ -177,17 +189,17 @@ void loss_bwd_kernel(const T* __restrict__ logits,
       bf16x8 o;
       #pragma unroll
       for (int j = 0; j < 8; ++j) o.v[j] = f2bf(0.f);
-      for (int i = threadIdx.x; i < nvec; i += 256) store8(dr + i * 8, o);
+      for (int i = threadIdx.x; i < nvec; i += THREADS) store8(dr + i * 8, o);
     } else {
       int i = threadIdx.x;
-      for (; i + 3 * 256 < nvec; i += 1024) {
+      for (; i + 3 * THREADS < nvec; i += 4 * THREADS) {
         bf16x8 v[4];
         #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = load8(lr + (i + k * 256) * 8);
+        for (int k = 0; k < 4; ++k) v[k] = load8(lr + (i + k * THREADS) * 8);
         #pragma unroll
-        for (int k = 0; k < 4; ++k) put(i + k * 256, v[k]);
+        for (int k = 0; k < 4; ++k) put(i + k * THREADS, v[k]);
       }
-      for (; i < nvec; i += 256) put(i, load8(lr + i * 8));
+      for (; i < nvec; i += THREADS) put(i, load8(lr + i * 8));
     }
     for (int i = nvec * 8 + threadIdx.x; i < V; i += blockDim.x) {
       float g = 0.f;
@@ -281,23 +293,20 @@ torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets,
   const int64_t rows = logits.numel() / V;
   auto dlogits = torch::empty_like(logits);
   if (rows == 0) return dlogits;
-  dim3 grid(rows), block(256);
   auto stream = at::cuda::getCurrentCUDAStream();
   auto wc = w.contiguous();
   auto lsec = lse.contiguous();
-  if (logits.scalar_type() == at::kBFloat16) {
-    hipLaunchKernelGGL(loss_bwd_kernel<__hip_bfloat16>, grid, block, 0, stream,
-                       reinterpret_cast<const __hip_bfloat16*>(logits.data_ptr()),
-                       targets.contiguous().data_ptr<int64_t>(),
-                       wc.data_ptr<float>(), lsec.data_ptr<float>(), dl,
-                       reinterpret_cast<__hip_bfloat16*>(dlogits.data_ptr()), V);
-  } else {
-    hipLaunchKernelGGL(loss_bwd_kernel<float>, grid, block, 0, stream,
-                       logits.data_ptr<float>(),
-                       targets.contiguous().data_ptr<int64_t>(),
-                       wc.data_ptr<float>(), lsec.data_ptr<float>(), dl,
-                       dlogits.data_ptr<float>(), V);
-  }
+  auto tc = targets.contiguous();
+  #define BWD(T, THREADS)                                                              \
+    hipLaunchKernelGGL((loss_bwd_kernel<T, THREADS>), dim3(rows), dim3(THREADS), 0,    \
+                       stream, reinterpret_cast<const T*>(logits.data_ptr()),          \
+                       tc.data_ptr<int64_t>(), wc.data_ptr<float>(),                   \
+                       lsec.data_ptr<float>(), dl,                                     \
+                       reinterpret_cast<T*>(dlogits.data_ptr()), V)
+  if (logits.scalar_type() != at::kBFloat16) BWD(float, 256);
+  else if (V / 8 >= 4 * 1024) BWD(__hip_bfloat16, 1024);
+  else BWD(__hip_bfloat16, 256);
+  #undef BWD
   HIP_CHECK_LAST();
   return dlogits;
 }

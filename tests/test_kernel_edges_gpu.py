@@ -815,6 +815,12 @@ def test_loss_rows_at_any_element(ext, off, V):
     assert all(torch.equal(a, b) for a, b in zip((tok, lse), ext.logprob_lse_fwd(aligned, targets)))
 
 
+@pytest.mark.parametrize("off,V", [(1, 32767), (0, 32768), (3, 32775), (2, 65539)])
+def test_loss_long_rows_at_any_element(ext, off, V):
+    """Either side of the gradient's rule for 1024 threads a row."""
+    test_loss_rows_at_any_element(ext, off, V)
+
+
 @pytest.mark.parametrize("lead,mask_shape,reward_shape,host", [
     ((6,), (6,), (), False), ((6,), (6,), (1,), False), ((3, 6), (3, 6), (), False),
     ((3, 6), (3, 6), (1,), False), ((3, 6), (1, 6), (3,), False), ((3, 6), (6,), (3,), False),
