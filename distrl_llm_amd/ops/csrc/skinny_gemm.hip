@@ -9,6 +9,11 @@
 // Partial sums meet in LDS. The norm needs no pass of its own: the waves
 // multiply x by the norm weight as they read it and sum its squares on the way,
 // 1/rms scales the finished row.
+// Tiles of W are read past the caches, which hold no model's weights from one step
+// to the next (256 MB; matrices small enough to stay there would be read faster through
+// them: 9728 x 896 at one row 5.6 us, and 6.3 so). At one row, us: 19456 x 2560 22.3 ->
+// 21.3, 2560 x 9728 13.6 -> 12.7. From rows a load is half a cache line of each, whose
+// other half has to stay: 35.9 past the caches, 29.3 through them.
 // A step of a few sequences is bound by its launches' latency (~4 us each) as
 // much as by bytes, hence the fusions: on the 0.5B model at 8 rows a layer took
 // 67 us in 11 launches, 39 in 7 now (gate|up + SiLU 17 + 5 -> 11.6 us, down and
@@ -81,7 +86,10 @@ void skinny_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat
     for (int i = 0; i < U; ++i) {
       const int k = min(s + i, s1 - 1) * 32;              // past the end: the last again
       #pragma unroll
-      for (int a = 0; a < ACC; ++a) wf[i][a] = *reinterpret_cast<const bf16v8*>(wp[a] + k * (TILES ? 32 : 1));
+      for (int a = 0; a < ACC; ++a) {
+        const bf16v8* from = reinterpret_cast<const bf16v8*>(wp[a] + k * (TILES ? 32 : 1));
+        wf[i][a] = TILES ? __builtin_nontemporal_load(from) : *from;
+      }
       #pragma unroll
       for (int t = 0; t < MT; ++t)
         xf[i][t] = *reinterpret_cast<const bf16v8*>(x + (int64_t)row[t] * K + k + g * 8);

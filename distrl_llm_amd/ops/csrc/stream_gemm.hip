@@ -18,6 +18,9 @@
 // adds up on its way (the residual sum with the norm, the rotation with the cache
 // write), so the sums are rounded once. Bound: HBM where W is large, else the
 // launch with its first loads.
+// W is read past the caches, as no step finds a model's weights there (the last
+// level holds 256 MB): 37888 x 3584 at 32 and 128 rows 48.5 and 58.0 -> 43.3 and 53.2
+// us (6.3 and 5.1 TB/s), 3584 x 18944 26.8 and 33.7 -> 24.3 and 33.2; 160 rows even.
 // 160 rows, GPU time before -> now: 4608 x 3584 24.6 -> 15 us, 3584 x 3584
 // 24.6 -> 13, 3584 x 18944 (4-bit product, adapter and join) 70 -> 34.
 #include <torch/extension.h>
@@ -83,7 +86,8 @@ void stream_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat
     for (int j = 0; j < PER; ++j) xv[i][j] = *reinterpret_cast<const u32x4*>(xp[j] + k);
     #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
-      wv[i][ks] = *reinterpret_cast<const bf16v8*>(wp + (int64_t)k * 32 + ks * 512);
+      wv[i][ks] = __builtin_nontemporal_load(
+          reinterpret_cast<const bf16v8*>(wp + (int64_t)k * 32 + ks * 512));
   };
   auto store_x = [&](int i, int buf) {
     #pragma unroll
