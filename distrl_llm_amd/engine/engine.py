@@ -5,13 +5,13 @@ Native replacement for the reference's in-process vLLM engine
 sampling with a paged KV cache, n-candidate fan-out per prompt (prompt KV
 blocks shared across the n candidates via refcounting — prefill runs once
 per prompt, not n times), per-call SamplingParams, and EOS/max-token
-termination. Decode is the hot loop (SURVEY.md §3.3); on GPU every custom
+termination. Decode is the hot loop; on GPU every custom
 op routes through the gfx950 HIP extension via ops.functional and the
 step can be hipGraph-captured (engine.graph).
 
 The engine reads the SAME weight/LoRA tensors the learner trains, so
 in-process weight sync is free and cross-process sync is one RCCL
-broadcast into these tensors (SURVEY.md §2.3).
+broadcast into these tensors.
 """
 
 from __future__ import annotations
@@ -72,8 +72,7 @@ class Engine:
 
     def _derive_num_blocks(self) -> int:
         """Size the KV pool from free HBM (re-derived for 288 GB per GPU,
-        not copied from the reference's 24 GB fractions — SURVEY.md
-        §2.6-10)."""
+        not copied from the reference's 24 GB fractions)."""
         s = self.spec
         bs = self.cfg.kv_block_size
         per_block = KVCachePool.pool_size_bytes(1, s.num_layers, bs,

@@ -1,5 +1,5 @@
-// Fused log-prob + PG/GRPO loss over the 152k vocab (SURVEY.md §2.4-B
-// north star): forward emits per-token log p(target) + the row LSE in a
+// Fused log-prob + PG/GRPO loss over the 152k vocab:
+// forward emits per-token log p(target) + the row LSE in a
 // single online-logsumexp streaming pass (never materializing a (B,T,V)
 // log-prob tensor — the reference loops rows through log_softmax+gather,
 // distributed_actor.py:253-260); backward emits dlogits directly:
