@@ -69,11 +69,15 @@ struct Args {
 // what a term without b multiplies by: 32 columns, any number of times
 __device__ const uint4 ZEROS[4] = {};
 
-// 16 B a lane from base + off into LDS at lds + 16 * lane
+// 16 B a lane from base + off into LDS at lds + 16 * lane. m0 is lost to the compiler,
+// which warns that nothing keeps it: nothing has to.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 DEV_INLINE void load_to_lds(uint32_t lds, const char* base, uint32_t off) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(lds), "v"(off), "s"(base) : "memory");
+               :: "s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // Until at most VM of this wave's loads are on their way and its LDS reads are done.
 template <int VM>
 DEV_INLINE void arrived() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(VM) : "memory"); }
