@@ -175,9 +175,11 @@ Tensor projected(const Tensor& xu, const Tensors& W, const Adapters& ad,
     return out;
   }
   if (!library(rows, width, K)) {
-    auto out = at::empty({rows, width}, xu.options());
-    if (product(blocks(columns(xu, 0, K), columns(xu, K, ad.pad), W, ad, bias), false, out, res))
-      return out;
+    const auto sums = blocks(columns(xu, 0, K), columns(xu, K, ad.pad), W, ad, bias);
+    if (product_takes(sums, false)) {
+      auto out = at::empty({rows, width}, xu.options());
+      if (product(sums, false, out, res)) return out;
+    }
   }
   const auto WB = adapted_weight(W, ad.B, ad.pad);
   if (res) return at::addmm(*res, xu, WB.t());
@@ -235,10 +237,13 @@ Through through(const Tensor& g, const Tensor& W, const Adapters& ad) {
   }
   if (!library(g.size(0), N, W.size(1))) {
     auto du = at::empty({g.size(0), ad.pad}, g.options());
-    auto dx = at::empty({g.size(0), W.size(1)}, g.options());
-    ad.up({g}, du);
     const auto r = ad.part(du, 0);
-    if (product({{W.size(1), {{g, W}, {r, ad.A[0]}}, {}}}, true, dx)) return {dx, r};
+    const std::vector<ProductBlock> sum{{W.size(1), {{g, W}, {r, ad.A[0]}}, {}}};
+    if (product_takes(sum, true)) {
+      auto dx = at::empty({g.size(0), W.size(1)}, g.options());
+      ad.up({g}, du);
+      if (product(sum, true, dx)) return {dx, r};
+    }
   }
   auto gd = at::empty({g.size(0), N + ad.pad}, g.options());
   auto g2 = columns(gd, 0, N), du = columns(gd, N, ad.pad);
@@ -258,6 +263,7 @@ bool own_dx(Tensor& dx, const Tensors& W, const Tensors& dy, const Tensor& du, c
   }
   if (library(rows, sum.width, K)) return false;
   for (size_t i = 0; i < W.size(); ++i) sum.terms.push_back({ad.part(du, i), ad.A[i]});
+  if (!product_takes({sum}, true)) return false;
   dx = at::empty({rows, sum.width}, du.options());
   return product({sum}, true, dx);
 }
@@ -417,12 +423,14 @@ Tensors feed_forward_half_fwd(Tensor x, Tensor norm, double eps, Tensors W,
   Tensor gu;
   bool ready = false;                     // act's adapter inputs
   if (!apart(rows, 2 * inner, hidden) && !library(rows, 2 * inner, hidden)) {
-    gu = at::empty({rows, 2 * inner}, x.options());
     const auto both = blocks(h, columns(hu, hidden, in.pad), {W[0], W[1]}, in, bias);
     const auto &ug = both[0].terms[1].a, &uu = both[1].terms[1].a;
     const ProductBlock gate{inner, {both[0].terms[0], {ug, B[0]}, {uu, {}}}, bias[0]};
     const ProductBlock up{inner, {both[1].terms[0], {ug, {}}, {uu, B[1]}}, bias[1]};
-    if (!product_glu(gate, up, gu, act)) gu = Tensor();
+    if (product_takes({gate, up}, false)) {
+      gu = at::empty({rows, 2 * inner}, x.options());
+      if (!product_glu(gate, up, gu, act)) gu = Tensor();
+    }
   }
   if (!gu.defined()) {
     gu = projected(hu, {W[0], W[1]}, in, bias);
@@ -453,9 +461,12 @@ Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tenso
   bool ready = false;                     // dgate's and dup's adapter inputs
   if (!apart(rows, hidden, inner) && !library(rows, hidden, inner)) {
     auto both = at::empty({rows, d_ad.pad}, x.options());
-    d_ad.up({g}, both);
-    dud = d_ad.part(both, 0);
-    if (!product_glu_bwd({inner, {{g, W[2]}, {dud, A[2]}}, {}}, gu, dgate, dup)) dud = Tensor();
+    const auto r = d_ad.part(both, 0);
+    const ProductBlock dact{inner, {{g, W[2]}, {r, A[2]}}, {}};
+    if (product_takes({dact}, true)) {
+      d_ad.up({g}, both);
+      if (product_glu_bwd(dact, gu, dgate, dup)) dud = r;
+    }
   }
   if (!dud.defined()) {
     const auto [dact, du2] = through(g, W[2], d_ad);
@@ -496,15 +507,6 @@ bool all_bf16(const Tensors& ts) {
   return true;
 }
 
-// u of the adapters on x; undefined where own products don't take their ranks
-Tensor adapter_side(const Tensor& x, const Adapters& ad) {
-  for (const auto r : ad.ranks)
-    if (r % 32 != 0) return {};
-  auto u = at::empty({x.size(0), ad.pad}, x.options());
-  ad.down(x, u);
-  return u;
-}
-
 }  // namespace
 
 // x W^T of projections of one input side by side, with their adapters (one each, or
@@ -518,12 +520,14 @@ Optional adapted_projection(Tensor x, Tensors W, std::vector<Optional> bias, Ten
   std::vector<ProductBlock> sums;
   if (A.empty()) {
     for (size_t i = 0; i < W.size(); ++i) sums.push_back({W[i].size(0), {{x, W[i]}}, bias.at(i)});
+    if (!product_takes(sums, false)) return {};
   } else {
     TORCH_CHECK(A.size() == W.size());
     const Adapters ad(A, B, scales);
-    const auto u = adapter_side(x, ad);
-    if (!u.defined()) return {};
+    const auto u = at::empty({x.size(0), ad.pad}, x.options());
     sums = blocks(x, u, W, ad, bias);
+    if (!product_takes(sums, false)) return {};
+    ad.down(x, u);
   }
   auto out = at::empty({x.size(0), width}, x.options());
   if (!product(sums, false, out, res)) return {};
@@ -536,13 +540,16 @@ Optional adapted_activation(Tensor x, Tensors W, Tensors A, Tensors B, std::vect
   TORCH_CHECK(W.size() == 2 && (A.empty() || A.size() == 2));
   const int64_t inner = W[0].size(0);
   ProductBlock gate{inner, {{x, W[0]}}, {}}, up{inner, {{x, W[1]}}, {}};
-  if (!A.empty()) {
+  if (A.empty()) {
+    if (!product_takes({gate, up}, false)) return {};
+  } else {
     const Adapters ad(A, B, scales);
-    const auto u = adapter_side(x, ad);
-    if (!u.defined()) return {};
+    const auto u = at::empty({x.size(0), ad.pad}, x.options());
     const auto ug = ad.part(u, 0), uu = ad.part(u, 1);
     gate.terms.insert(gate.terms.end(), {{ug, B[0]}, {uu, {}}});
     up.terms.insert(up.terms.end(), {{ug, {}}, {uu, B[1]}});
+    if (!product_takes({gate, up}, false)) return {};
+    ad.down(x, u);
   }
   auto act = at::empty({x.size(0), inner}, x.options());
   if (!product_glu(gate, up, {}, act)) return {};

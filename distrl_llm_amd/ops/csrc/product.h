@@ -14,6 +14,10 @@ struct ProductBlock {
   c10::optional<at::Tensor> bias;
 };
 
+// Whether the products below take these operands, whatever they hold yet: what a term is
+// made of need not be launched for one that is refused. What they write is not asked for.
+bool product_takes(const std::vector<ProductBlock>& blocks, bool rows_of_b);
+
 // out <- the blocks side by side (+ res): fp32 sums, rounded once. rows_of_b: b is
 // (k, width). tile: the shape of tile, for tests; 0 picks one. All of them: false, and
 // nothing done, for what 16 B accesses and steps of 32 of K can't walk.

@@ -540,22 +540,29 @@ bool fill(Args& o, const std::vector<const ProductBlock*>& blocks, bool rows) {
   return true;
 }
 
+std::vector<const ProductBlock*> each(const std::vector<ProductBlock>& blocks) {
+  std::vector<const ProductBlock*> out;
+  for (const auto& b : blocks) out.push_back(&b);
+  return out;
+}
+
 bool shaped(const at::Tensor& t, int64_t rows, int64_t cols) {
   return walks(t, 8) && t.size(0) == rows && t.size(1) == cols;
 }
 
 }  // namespace
 
+bool product_takes(const std::vector<ProductBlock>& blocks, bool rows_of_b) {
+  Args o{};
+  return fill(o, each(blocks), rows_of_b);
+}
+
 bool product(const std::vector<ProductBlock>& blocks, bool rows_of_b, const at::Tensor& out,
              const c10::optional<at::Tensor>& res, int tile) {
   Args o{};
-  std::vector<const ProductBlock*> all;
   int64_t width = 0;
-  for (const auto& b : blocks) {
-    all.push_back(&b);
-    width += b.width;
-  }
-  if (!fill(o, all, rows_of_b) || !shaped(out, o.M, width) || (res && !shaped(*res, o.M, width)))
+  for (const auto& b : blocks) width += b.width;
+  if (!fill(o, each(blocks), rows_of_b) || !shaped(out, o.M, width) || (res && !shaped(*res, o.M, width)))
     return false;
   o.c = ptr(out);
   o.ldc = (int)out.stride(0);
@@ -563,8 +570,8 @@ bool product(const std::vector<ProductBlock>& blocks, bool rows_of_b, const at::
     o.res = ptr(*res);
     o.ldr = (int)res->stride(0);
   }
-  if (rows_of_b) by_size<true, PLAIN>(o, (int)all.size(), tile);
-  else by_size<false, PLAIN>(o, (int)all.size(), tile);
+  if (rows_of_b) by_size<true, PLAIN>(o, (int)blocks.size(), tile);
+  else by_size<false, PLAIN>(o, (int)blocks.size(), tile);
   return true;
 }
 

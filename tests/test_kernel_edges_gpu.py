@@ -390,6 +390,17 @@ def _train_model(name, lora_r=8, **kw):
     return model.train()
 
 
+def _kernels(call):
+    """What the call returns, and how often a kernel of a name ran in it."""
+    from torch.profiler import ProfilerActivity, profile
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        out = call()
+        torch.cuda.synchronize()
+    counts = [(e.key, e.count) for e in prof.key_averages()]
+    assert counts
+    return out, lambda name: sum(n for key, n in counts if name in key)
+
+
 def _grads(model, ids, mask, dout):
     out = model.forward_hidden(ids, mask)
     params = [p for p in model.parameters() if p.requires_grad]
@@ -1031,6 +1042,40 @@ def test_feed_forward_half_in_waves(ext, rows):
     assert _rel(y, ref.detach()) < 2.0 ** -7
     for at in (slice(None), slice(0, 1), slice(4095, 4097), slice(rows - 1, rows)):
         assert _rel(dx[at], want[at]) < 2.0 ** -6
+
+
+@pytest.mark.parametrize("r", [8, 16, 32])
+def test_halves_take_adapter_inputs_once(ext, r):
+    """Whatever products a rank goes through, the inputs of the adapters on one
+    matrix are one launch: those on x, then on the second product's operand, and
+    the same of the gradients."""
+    rows, h, D, f = 64, 128, 64, 256
+    x, g, norm = _rand((rows, h), 1), _rand((rows, h), 2), _rand((h,), 3, 0.1) + 1
+
+    def adapted(*shapes):
+        Ws = [_rand(s, 4 + i, 0.1) for i, s in enumerate(shapes)]
+        return (Ws, [_rand((r, w.shape[1]), 8 + i, 0.1) for i, w in enumerate(Ws)],
+                [_rand((w.shape[0], r), 12 + i, 0.1) for i, w in enumerate(Ws)])
+
+    Ws, As, Bs = adapted((h, h), (D, h), (D, h), (h, h))
+    pos = torch.arange(rows, dtype=torch.int32, device="cuda")
+    inv = 1.0 / 1e4 ** (torch.arange(0, D, 2, device="cuda").float() / D)
+    cu = torch.tensor([0, rows], dtype=torch.int32, device="cuda")
+    (y, *own), ran = _kernels(lambda: ext.attention_half_fwd(
+        x, norm, 1e-6, Ws, [None] * 3, As, Bs, [1.0] * 4, None, None, 0.0, 0.0, pos, inv, cu, rows,
+        D ** -0.5, D))
+    assert ran("adapter_inputs_kernel") == 2
+    _, ran = _kernels(lambda: ext.attention_half_bwd(
+        g, x, norm, 1e-6, Ws, As, Bs, [1.0] * 4, None, None, 0.0, 0.0, pos, -inv, cu, rows,
+        D ** -0.5, *own, True))
+    assert ran("adapter_inputs_kernel") == 2
+    Ws, As, Bs = adapted((f, h), (f, h), (h, f))
+    (y, *own), ran = _kernels(lambda: ext.feed_forward_half_fwd(
+        x, norm, 1e-6, Ws, [None] * 2, As, Bs, [1.0] * 3))
+    assert ran("adapter_inputs_kernel") == 2
+    _, ran = _kernels(lambda: ext.feed_forward_half_bwd(
+        g, x, norm, 1e-6, Ws, As, Bs, [1.0] * 3, *own, True))
+    assert ran("adapter_inputs_kernel") == 2
 
 
 @pytest.mark.parametrize("prompts,answers", [([9, 30, 1], [40, 7, 100]), ([0, 5, 3], [4, 0, 6]),
