@@ -22,8 +22,8 @@
 // partial sums and the bias, norms and rotates them, writes the new token's key
 // and value into the cache and attends over them from LDS, while the first rows
 // of the context are on their way. Slices of one sequence are joined by the last
-// of them to end (as a launch of its own that took 3 us). As kernels of their own rotation and join took 7.7 and 4.6 us a
-// layer at 160 sequences, 3.0 and 1.3 at eight.
+// of them to end (as a launch of its own that took 3 us). As kernels of their own
+// rotation and join took 7.7 and 4.6 us a layer at 160 sequences, 3.0 and 1.3 at eight.
 // K and V are read once per sequence and kv head; bound by HBM.
 // 160 sequences of 420..1550 tokens sharing prompts, 28/4 heads of 128
 // (251 MB of distinct rows): 157 us with one lane a token on vector FMAs,
@@ -158,10 +158,14 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
     const int64_t slot = src.slots[seq];
     const int units = (group + (owner ? 1 : 0)) * PER, all = units + (owner ? D / 8 : 0);
     // eight elements at `at` and eight at `other` of this sequence: the rows, or the
-    // first four partial sums of them
+    // first partial sums of them. Four hold 64 registers, 182 in all with rows of 64: two
+    // workgroups of four waves a CU instead of three (160 sequences of 30..200, 16/4
+    // heads 14.1 us, two 10.0; 96 of 100..600, 8/8 heads 22.8 and 18.8). Eight waves run
+    // one workgroup a CU, rows of 128 two with either.
+    constexpr int AHEAD = D == 64 && NW == 4 ? 2 : 4;
     struct Raw {
       bf16x8 x, y;
-      f32x4v part[4][4];
+      f32x4v part[AHEAD][4];
     };
     auto fetch = [&](Raw& r, int at, int other) {
       if constexpr (SRC == ROWS) {
@@ -170,7 +174,7 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
         r.y = *reinterpret_cast<const bf16x8*>(p + other);
       } else {
         #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < AHEAD; ++i) {
           const float* p = src.parts + ((int64_t)min(i, src.splits - 1) * N + seq) * width;
           #pragma unroll
           for (int h = 0; h < 2; ++h) {
@@ -191,7 +195,7 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
           y[j] = src.bias ? bf2f(src.bias[other + j]) : 0.f;
         }
         #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < AHEAD; ++i)
           if (i < src.splits) {
             #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -199,9 +203,9 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
               y[j] += r.part[i][2 + j / 4].v[j % 4];
             }
           }
-        if (src.splits > 4)
-          add_parts8x2(x, y, src.parts + ((int64_t)4 * N + seq) * width + at, other - at,
-                       (int64_t)N * width, src.splits - 4);
+        if (src.splits > AHEAD)
+          add_parts8x2(x, y, src.parts + ((int64_t)AHEAD * N + seq) * width + at, other - at,
+                       (int64_t)N * width, src.splits - AHEAD);
       }
     };
     // where unit u's elements are: of the value eight, twice
@@ -519,7 +523,8 @@ void decode(const __hip_bfloat16* q, const torch::Tensor& kcache, const torch::T
   // once (two a CU by their LDS), those of two do: the round above 70.6 -> 67.7 us,
   // 10 x 16 of 180..380 20.5 -> 18.1 (from partial sums 29.1 -> 21.8), 16 x 16
   // 26.6 -> 24.0; 256 workgroups of
-  // 500..1500 would take 49.4 for 35.5, and rows of 64 fit four a CU anyway.
+  // 500..1500 would take 49.4 for 35.5, and rows of 64 fit three or four a CU anyway
+  // (two waves there: 160 of 300..1500, 32/8 heads from partial sums 73 for 62).
   if (D == 128) { if (few) DECODE(128, 8); else if (blocks > 512) DECODE(128, 2); else DECODE(128, 4); }
   else { if (few) DECODE(64, 8); else DECODE(64, 4); }
   #undef DECODE

@@ -151,6 +151,12 @@ def test_paged_decode_packed(ext, H, KV, D, N, longest, bs, S, bias, norms):
     assert got[0].isnan().any(-1).sum() == KV
 
 
+@pytest.mark.parametrize("S", [2, 3, 4])
+def test_paged_decode_packed_few_partial_sums(ext, S):
+    """As many as a workgroup of four waves with rows of 64 fetches ahead, and more."""
+    test_paged_decode_packed(ext, 8, 8, 64, 130, 90, 16, S, True, False)
+
+
 def test_paged_decode_packed_refuses(ext):
     """Operands in host memory, and ones that do not lie on end."""
     D, N = 64, 3
