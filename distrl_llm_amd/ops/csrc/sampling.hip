@@ -451,7 +451,8 @@ struct Search {
   int c[AT_ONCE * STEPS];
 };
 struct Shares {
-  float f[4][LEVELS][3];
+  float f[4][LEVELS][2];
+  unsigned long long total[4];
   int i[4][LEVELS][2];
 };
 
@@ -461,7 +462,8 @@ DEV_INLINE Window find_window(const Sums& sums, int row, int S, float m, float i
   auto& in = *reinterpret_cast<Search*>(lds);
   auto& out = *reinterpret_cast<Shares*>(lds);
   const int tid = threadIdx.x, L = tid & (LEVELS - 1), sub = tid / LEVELS;
-  float least = 0.f, most = 0.f, total = 0.f;
+  float least = 0.f, most = 0.f;
+  unsigned long long total = 0;         // slices meet in it as whole numbers, as in the masses
   int cleast = 0, cmost = 0;
   for (int s0 = 0; s0 < S; s0 += Search::AT_ONCE) {
     const int n = min(S - s0, Search::AT_ONCE);
@@ -488,7 +490,7 @@ DEV_INLINE Window find_window(const Sums& sums, int row, int S, float m, float i
         const float* p = in.p + s * STEPS;
         least += ends >= 0 ? w * p[max(ends, 0)] : 0.f;
         most += begins >= 0 ? w * p[max(begins, 0)] : 0.f;
-        total += w * p[STEPS - 1];
+        total += (unsigned long long)(w * p[STEPS - 1] * 0x1p32f + 0.5f);
       }
       if (BY_K) {
         const int* c = in.c + s * STEPS;
@@ -498,14 +500,15 @@ DEV_INLINE Window find_window(const Sums& sums, int row, int S, float m, float i
     }
   }
   __syncthreads();
-  if (BY_P) { out.f[sub][L][0] = least; out.f[sub][L][1] = most; out.f[sub][L][2] = total; }
+  if (BY_P) { out.f[sub][L][0] = least; out.f[sub][L][1] = most; out.total[sub] = total; }
   if (BY_K) { out.i[sub][L][0] = cleast; out.i[sub][L][1] = cmost; }
   __syncthreads();
-  least = most = total = 0.f;
+  least = most = 0.f;
+  total = 0;
   cleast = cmost = 0;
   #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    if (BY_P) { least += out.f[i][L][0]; most += out.f[i][L][1]; total += out.f[i][L][2]; }
+    if (BY_P) { least += out.f[i][L][0]; most += out.f[i][L][1]; total += out.total[i]; }
     if (BY_K) { cleast += out.i[i][L][0]; cmost += out.i[i][L][1]; }
   }
   // a level a lane; reached at the end of z if nowhere before
@@ -515,9 +518,9 @@ DEV_INLINE Window find_window(const Sums& sums, int row, int S, float m, float i
     end = min(r ? __ffsll(r) - 1 : LEVELS, first + WINDOW / PER_LEVEL);
     end = max(end, first + 1);
   };
-  Window w{0, LEVELS, total};
+  Window w{0, LEVELS, (float)total * 0x1p-32f};
   if (BY_P) {
-    const float target = top_p * total;
+    const float target = top_p * w.total;
     cut(least >= target * (1.f + 2e-6f), most < target * (1.f - 2e-6f), w.first, w.end);
   }
   if (BY_K) {

@@ -266,6 +266,27 @@ def test_sampler_repeats_itself(ext):
             assert len(set(ext.sample_tokens(rows, 1.0, top_p, 0, seeds, step).tolist())) == 1
 
 
+def test_sampler_total_of_many_slices(ext):
+    """The total that top_p is a share of counts what single slices add little
+    to: 73 of them add e^-9.875 to 1368 each, less than half of what fp32 resolves there, and
+    with an eighth of that missing the first group alone would reach top_p. Every
+    sum here is good to 1e-7, the eighth is 3.4e-7 of it."""
+    V = 151936
+    logits = torch.full((1, V), -40.0)
+    logits[0, :1000], logits[0, 1000:2000] = 0.0, -1.0
+    logits[0, 2057::2056] = -9.875
+    small = int((logits == -9.875).sum()) * np.exp(-9.875)
+    total = 1000 + 1000 * np.exp(-1.0) + small
+    top_p, logits = float(np.float32(1000 / (total - small / 8))), logits.cuda()
+    got = []
+    for seed in range(40):
+        seeds = torch.tensor([seed])
+        got += ext.sample_tokens(logits, 1.0, top_p, 0, seeds.cuda(),
+                                 torch.tensor([0], device="cuda")).tolist()
+        assert got[-1:] == _sampled(logits, 1.0, top_p, 0, seeds, 0)
+    assert max(got) >= 1000
+
+
 def test_sampler_in_a_graph(ext):
     """Replays draw anew with the device step and match eager draws."""
     logits = _rand((5, 32768), 2, 3.0)
