@@ -7,8 +7,8 @@
 // cumulative probability reaches top_p (or the count top_k). The draw is the
 // argmax of z - log(-log u) over the kept set, u a counter-based hash of
 // (seed of the row, step, element): the step is read from device memory, so a
-// replayed graph draws anew. What workgroups add up meets as integers of 2^-32,
-// whose sum does not hang on their order: a call repeats itself exactly. How a
+// replayed graph draws anew. What workgroups add up meets as whole numbers of a small
+// unit, whose sum does not hang on their order: a call repeats itself exactly. How a
 // row was split over workgroups (by the number of rows) shows only where a
 // cumulative probability lies within fp32 rounding of top_p.
 //
@@ -365,6 +365,11 @@ struct Sums {
   int* c;                              // (B, S, STEPS)
   unsigned long long *mass, *best;     // (B, 1 + WINDOW)
   int *count, *done;                   // (B, 1 + WINDOW), (B)
+  // What probability meets in: whole numbers of 1 / unit (back), 2^-44 for 152064
+  // elements, so that the most there is, one of each, fits. Of 2^-32 100000 elements 14
+  // below the maximum, rounded one by one, were up to 1e-5 of the row too much or little.
+  float unit, back;
+  DEV_INLINE unsigned long long whole(float p) const { return (unsigned long long)(p * unit + 0.5f); }
 };
 
 DEV_INLINE int64_t width_at(int row) { return (int64_t)row * (1 + WINDOW); }
@@ -490,7 +495,7 @@ DEV_INLINE Window find_window(const Sums& sums, int row, int S, float m, float i
         const float* p = in.p + s * STEPS;
         least += ends >= 0 ? w * p[max(ends, 0)] : 0.f;
         most += begins >= 0 ? w * p[max(begins, 0)] : 0.f;
-        total += (unsigned long long)(w * p[STEPS - 1] * 0x1p32f + 0.5f);
+        total += sums.whole(w * p[STEPS - 1]);
       }
       if (BY_K) {
         const int* c = in.c + s * STEPS;
@@ -518,7 +523,7 @@ DEV_INLINE Window find_window(const Sums& sums, int row, int S, float m, float i
     end = min(r ? __ffsll(r) - 1 : LEVELS, first + WINDOW / PER_LEVEL);
     end = max(end, first + 1);
   };
-  Window w{0, LEVELS, (float)total * 0x1p-32f};
+  Window w{0, LEVELS, (float)total * sums.back};
   if (BY_P) {
     const float target = top_p * w.total;
     cut(least >= target * (1.f + 2e-6f), most < target * (1.f - 2e-6f), w.first, w.end);
@@ -581,7 +586,7 @@ void pick_kernel(const T* __restrict__ logits, int V, int per, float inv_temp, f
       b.offer(e.key, e.idx);
     } else {
       const int to = min(bin - w.first, bins - 1) * copies + copy;
-      if (BY_P) atomicAdd(wmass + to, (unsigned long long)(p * 0x1p32f + 0.5f));
+      if (BY_P) atomicAdd(wmass + to, sums.whole(p));
       if (BY_K) atomicAdd(wcount + to, 1);
       const unsigned long long o = word_of(e);
       if (o > wbest[to]) atomicMax(wbest + to, o);      // seldom
@@ -597,7 +602,7 @@ void pick_kernel(const T* __restrict__ logits, int V, int per, float inv_temp, f
   }
   if (tid == 0) {
     if (BY_P && above != 0.f)
-      atomicAdd(sums.mass + at, (unsigned long long)(above * 0x1p32f + 0.5f));
+      atomicAdd(sums.mass + at, sums.whole(above));
     if (word_of(b)) atomicMax(sums.best + at, word_of(b));
   }
   for (int j = tid; j < bins; j += 256) {
@@ -633,7 +638,7 @@ void pick_kernel(const T* __restrict__ logits, int V, int per, float inv_temp, f
     const int i = b0 + (tid & 31);            // POOL is a multiple of 32; zeros past the end
     const unsigned long long pm = BY_P ? mass + upto32(wmass[i]) : 0ull;
     const int pc = BY_K ? count + upto32(wcount[i]) : 0;
-    const uint32_t hit = (uint32_t)__ballot((BY_P && (float)pm * 0x1p-32f >= target) ||
+    const uint32_t hit = (uint32_t)__ballot((BY_P && (float)pm * sums.back >= target) ||
                                             (BY_K && pc >= top_k));
     const int kept = hit ? __ffs((int)hit) : 32;      // down to the threshold's bin
     unsigned long long o = (tid & 31) < kept ? wbest[i] : 0ull;
@@ -689,6 +694,8 @@ void sample_slices(const T* logits, int B, int V, float inv_t, float top_p, int 
   sums.top = reinterpret_cast<float*>(sums.done + rows);
   sums.p = sums.top + cells;
   sums.c = reinterpret_cast<int*>(sums.p + cells * STEPS);
+  sums.unit = std::ldexp(1.f, 30 + __builtin_clz(V));   // V times it: 2^62 at most
+  sums.back = 1.f / sums.unit;
   auto go = [&](auto p_, auto k_) {
     constexpr bool P = decltype(p_)::value, K = decltype(k_)::value;
     hipLaunchKernelGGL((steps_kernel<T, VEC, P, K>), grid, block, 0, stream, logits, V, per, inv_t,

@@ -287,6 +287,25 @@ def test_sampler_total_of_many_slices(ext):
     assert max(got) >= 1000
 
 
+def test_sampler_sums_small_probabilities(ext):
+    """100000 elements of probability 3000.55 * 2^-32, each: a sum that rounds them to
+    whole 2^-32 first is 0.45 * 2^-32 * 100000 = 1e-5 too large, reaches a top_p that is
+    half of that above the group's share, and drops the group below."""
+    V, n = 152064, 100000
+    logits = torch.full((160, V), -40.0)
+    logits[:, 0] = 0.0
+    logits[:, 1:n + 1] = float(np.log(3000.55) - 32 * np.log(2.0))
+    logits[:, n + 1:n + 50001] = -14.7
+    p = logits[0].double().exp()
+    top_p = float((1 + p[1:n + 1].sum() + 0.22 * n * 2.0 ** -32) / p.sum())
+    logits, seeds = logits.cuda(), torch.arange(160)
+    got = ext.sample_tokens(logits, 1.0, top_p, 0, seeds.cuda(),
+                            torch.tensor([3], device="cuda")).tolist()
+    assert max(got) > n
+    at = [i for i, x in enumerate(got) if x > n] + list(range(4))
+    assert [got[i] for i in at] == _sampled(logits[at], 1.0, top_p, 0, seeds[at], 3)
+
+
 def test_sampler_in_a_graph(ext):
     """Replays draw anew with the device step and match eager draws."""
     logits = _rand((5, 32768), 2, 3.0)
