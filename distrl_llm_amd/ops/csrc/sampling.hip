@@ -21,9 +21,9 @@
 //    and draws what lies above that window, keeps sum and best draw of
 //    each of the window's bins apart, and the row's last slice to end finds the
 //    threshold's bin and the best draw down to it.
-//  * Without one, one launch: a slice draws relative to its own maximum, and
-//    leaves out what the largest possible draw would not lift over the best of
-//    its threads' own maxima.
+//  * Without one, one launch, and keys that hang on no maximum: a slice leaves out
+//    what the largest possible draw would not lift over the best of its threads'
+//    own maxima.
 // A step's probability is added up in an LDS column of the thread's own, so nothing
 // collides (LDS float atomics took ten times as long); an element that is drawn costs
 // ~330 cycles of hashing a wave, so sparse ones are gathered into full waves first.
@@ -56,21 +56,23 @@ DEV_INLINE uint64_t row_seed(const int64_t* seeds, const int64_t* step, int row)
 DEV_INLINE int bin_of(float z) { return min(NBINS - 1, (int)(-z * (NBINS / ZRANGE))); }
 
 // The best key of a lane; equal keys go to the lower index.
-struct Best {
-  float key = -1e30f;
+template <typename K>
+struct BestOf {
+  K key = std::is_same<K, double>::value ? (K)-1e300 : (K)-1e30f;    // below all
   int idx = 0x7fffffff;
-  DEV_INLINE void offer(float k, int i) {
+  DEV_INLINE void offer(K k, int i) {
     if (k > key || (k == key && i < idx)) { key = k; idx = i; }
   }
   DEV_INLINE void over_wave() {
     #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
-      const float k = __shfl_xor(key, off, WAVE);
+      const K k = __shfl_xor(key, off, WAVE);
       const int i = __shfl_xor(idx, off, WAVE);
       offer(k, i);
     }
   }
 };
+using Best = BestOf<float>;
 
 // splitmix64(idx) for idx < 2^31: the first sum's upper half is a constant,
 // which leaves two of the first product's three partial products.
@@ -85,15 +87,16 @@ DEV_INLINE uint64_t mix_index(uint32_t idx) {
   return x ^ (x >> 31);
 }
 
-// z - log(-log u), u = (the hash's upper 24 bits + 1) / 2^24, kept below 1: u = 1
+// -log(-log u), u = (the hash's upper 24 bits + 1) / 2^24, kept below 1: u = 1
 // would make the key infinite and draw the element whatever its probability.
 // Neither logarithm's argument is ever denormal.
-DEV_INLINE float gumbel_key(uint64_t seed, int idx, float z) {
+DEV_INLINE float gumbel(uint64_t seed, int idx) {
   constexpr float LN2 = 0.6931471805599453f;
   const uint64_t h = splitmix64(seed ^ mix_index((uint32_t)idx));
   const float u = (float)min((uint32_t)(h >> 40) + 1u, (1u << 24) - 1u) * 0x1p-24f;
-  return z - LN2 * __builtin_amdgcn_logf(-LN2 * __builtin_amdgcn_logf(u));
+  return -LN2 * __builtin_amdgcn_logf(-LN2 * __builtin_amdgcn_logf(u));
 }
+DEV_INLINE float gumbel_key(uint64_t seed, int idx, float z) { return z + gumbel(seed, idx); }
 
 // Sum over lanes 0..31 (and 32..63) up to this one.
 template <typename T>
@@ -260,7 +263,8 @@ struct Gather {
 };
 
 // The best of a workgroup's lanes, in thread 0.
-DEV_INLINE void over_block(Best& b, float* fpart, int* ipart) {
+template <typename K>
+DEV_INLINE void over_block(BestOf<K>& b, K* fpart, int* ipart) {
   b.over_wave();
   if ((threadIdx.x & (WAVE - 1)) == 0) {
     fpart[threadIdx.x / WAVE] = b.key;
@@ -273,9 +277,13 @@ DEV_INLINE void over_block(Best& b, float* fpart, int* ipart) {
 
 // --------------------------------------------------------- no threshold
 // What a slice passes on to the row's last slice to end, each word with the launch's
-// mark above it: its maximum, its best key relative to that, that key's element. A
-// mark's 32 bits might lie in old memory by chance, but not in all three.
-enum { TOP = 0, KEY = 1, ELEMENT = 2, WORDS = 3 };
+// mark above it: the halves of its best key, and that key's element. A mark's 32 bits
+// might lie in old memory by chance, but not in all three.
+// A key is logit / temperature + the variate, in 64 bits: of nothing but its element, so
+// that a row draws the same token whatever slices it is cut into. In 32 bits, relative
+// to a slice's maximum and then moved to the row's, it was rounded twice, and keys next
+// to each other came out by how many rows were drawn together.
+enum { KEY_LOW = 0, KEY_HIGH = 1, ELEMENT = 2, WORDS = 3 };
 
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256)
@@ -283,7 +291,8 @@ void draw_kernel(const T* __restrict__ logits, int V, int per, float inv_temp,
                  const int64_t* __restrict__ seeds, const int64_t* __restrict__ step,
                  unsigned long long* __restrict__ found, uint32_t mark, int64_t* __restrict__ out) {
   __shared__ typename Gather<T, VEC>::Entry queue[4 * Gather<T, VEC>::ROOM];
-  __shared__ float red[16], fpart[4];
+  __shared__ float red[16];
+  __shared__ double kpart[4];
   __shared__ int ipart[4];
   const int row = blockIdx.x, sl = blockIdx.y, S = gridDim.y, tid = threadIdx.x;
   const int i0 = sl * per, n = min(V - i0, per);
@@ -299,13 +308,13 @@ void draw_kernel(const T* __restrict__ logits, int V, int per, float inv_temp,
   // a key that is reached: nothing MOST below it can be the best
   const float floor_key =
       block_max(gumbel_key(seed, i0 + own_at, (own - m) * inv_temp), red) - MOST;
-  Best b;
+  BestOf<double> b;
   Gather<T, VEC> gather{queue + (tid / WAVE) * Gather<T, VEC>::ROOM};
   gather.run(s, n, [&](float x) { return (x - m) * inv_temp > floor_key; },
              [&](int at, float x) {
-               b.offer(gumbel_key(seed, i0 + at, (x - m) * inv_temp), i0 + at);
+               b.offer((double)x * inv_temp + gumbel(seed, i0 + at), i0 + at);
              });
-  over_block(b, fpart, ipart);
+  over_block(b, kpart, ipart);
   if (tid >= WAVE) return;
   // Of the row's slices the last to come finds all of them here, as each looks only
   // when its own words have arrived. Another may, too, and writes the same token.
@@ -313,32 +322,25 @@ void draw_kernel(const T* __restrict__ logits, int V, int per, float inv_temp,
   // a captured launch has the same mark.
   unsigned long long* const words = found + (int64_t)row * S * WORDS;
   const unsigned long long high = (unsigned long long)mark << 32;
-  const uint32_t own_word[WORDS] = {__float_as_uint(m), __float_as_uint(b.key), (uint32_t)b.idx};
+  const unsigned long long key = (unsigned long long)__double_as_longlong(b.key);
+  const uint32_t own_word[WORDS] = {(uint32_t)key, (uint32_t)(key >> 32), (uint32_t)b.idx};
   if (tid == 0) {
     #pragma unroll
     for (int i = 0; i < WORDS; ++i) store_through(words + sl * WORDS + i, high | own_word[i]);
   }
   stores_done();
-  float m_row = -1e30f;
   bool all_here = true;
+  b = {};
   for (int i = tid; i < S; i += WAVE) {
     unsigned long long w[WORDS];
     #pragma unroll
     for (int j = 0; j < WORDS; ++j) w[j] = load_through(words + i * WORDS + j);
     #pragma unroll
     for (int j = 0; j < WORDS; ++j) all_here = all_here && (w[j] >> 32) == mark;
-    // relative to the highest maximum that this lane has met
-    const float top = __uint_as_float((uint32_t)w[TOP]), to = fmaxf(m_row, top);
-    if (i == tid) b = Best{};
-    b.key = fmaxf(b.key + (m_row - to) * inv_temp, -1e30f);
-    m_row = to;
-    const int idx = (int)(uint32_t)w[ELEMENT];
-    if (idx != 0x7fffffff) b.offer(__uint_as_float((uint32_t)w[KEY]) + (top - to) * inv_temp, idx);
+    b.offer(__longlong_as_double((long long)(w[KEY_HIGH] << 32 | (uint32_t)w[KEY_LOW])),
+            (int)(uint32_t)w[ELEMENT]);
   }
-  if (tid >= S) b = Best{};
   if (__ballot(!all_here) != 0) return;
-  const float top = wave_max(m_row);
-  b.key = fmaxf(b.key + (m_row - top) * inv_temp, -1e30f);
   b.over_wave();
   if (tid == 0) out[row] = b.idx == 0x7fffffff ? 0 : b.idx;
   for (int i = tid; i < S * WORDS; i += WAVE) words[i] = 0ull;

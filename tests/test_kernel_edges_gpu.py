@@ -306,6 +306,29 @@ def test_sampler_sums_small_probabilities(ext):
     assert [got[i] for i in at] == _sampled(logits[at], 1.0, top_p, 0, seeds[at], 3)
 
 
+def test_sampler_draw_does_not_hang_on_the_slices(ext):
+    """Alone a row is cut into 148 slices, among 640 into eight, and draws the
+    same where two keys are next to each other: the logit of one is raised to the
+    last value at which it is not drawn and the next one, at which it is. Higher
+    elements lie beside it in a short slice and in a long one."""
+    B, V, at, temperature = 640, 151936, 1500, 0.7
+    seeds, step = torch.arange(B, device="cuda"), torch.zeros(1, dtype=torch.int64, device="cuda")
+    logits = torch.full((B, V), -30.0, device="cuda")
+    logits[:, 100], logits[:, 1600], logits[:, 9000] = 0.3, 1.1, 1.7
+    low, high = (torch.full((B,), x, device="cuda") for x in (-20.0, 20.0))
+    for _ in range(60):
+        logits[:, at] = (low + high) / 2
+        drawn = ext.sample_tokens(logits, temperature, 1.0, 0, seeds, step) == at
+        low, high = torch.where(drawn, low, logits[:, at]), torch.where(drawn, logits[:, at], high)
+    assert torch.equal(torch.nextafter(low, high), high)
+    for x, drawn in ((low, False), (high, True)):
+        logits[:, at] = x
+        among = ext.sample_tokens(logits, temperature, 1.0, 0, seeds, step).tolist()
+        assert all((t == at) == drawn for t in among)
+        assert among == [ext.sample_tokens(logits[r:r + 1], temperature, 1.0, 0, seeds[r:r + 1],
+                                           step).item() for r in range(B)]
+
+
 def test_sampler_in_a_graph(ext):
     """Replays draw anew with the device step and match eager draws."""
     logits = _rand((5, 32768), 2, 3.0)
