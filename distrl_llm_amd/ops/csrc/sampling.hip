@@ -316,6 +316,8 @@ void draw_kernel(const T* __restrict__ logits, int V, int per, float inv_temp,
              });
   over_block(b, kpart, ipart);
   if (tid >= WAVE) return;
+  // a maximum of infinity: nothing is finite beside it, and the row has no draw
+  if (__float_as_uint(m) == 0x7f800000u) b = {1e300, 0x7fffffff};
   // Of the row's slices the last to come finds all of them here, as each looks only
   // when its own words have arrived. Another may, too, and writes the same token.
   // Nothing has to be cleared first; who has seen all clears them, because a replay of

@@ -329,6 +329,21 @@ def test_sampler_draw_does_not_hang_on_the_slices(ext):
                                            step).item() for r in range(B)]
 
 
+def test_sampler_without_a_finite_maximum(ext):
+    """A row with an infinite logit, or none above the lowest finite one, has no
+    element that is drawn, and answers 0, however it is cut."""
+    V = 32768
+    logits = torch.randn(3, V, generator=torch.Generator().manual_seed(1))
+    logits[0, 20000] = float("inf")
+    logits[1] = torch.finfo(torch.bfloat16).min
+    logits = logits.to("cuda", torch.bfloat16)
+    step = torch.tensor([0], device="cuda")
+    for rows in (logits, logits.repeat(200, 1)):
+        for top_p in (1.0, 0.9):
+            got = ext.sample_tokens(rows, 1.0, top_p, 0, torch.arange(len(rows), device="cuda"), step)
+            assert not got.view(-1, 3)[:, :2].any() and got.view(-1, 3)[:, 2].all()
+
+
 def test_sampler_in_a_graph(ext):
     """Replays draw anew with the device step and match eager draws."""
     logits = _rand((5, 32768), 2, 3.0)
