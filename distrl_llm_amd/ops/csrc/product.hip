@@ -550,6 +550,16 @@ bool shaped(const at::Tensor& t, int64_t rows, int64_t cols) {
   return walks(t, 8) && t.size(0) == rows && t.size(1) == cols;
 }
 
+// Whether what is read lies clear of what is written: a tile in shares of K may be
+// joined and written by two workgroups, the second after the first has written.
+bool clear_of(const at::Tensor& read, const at::Tensor& written) {
+  auto from = [](const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()); };
+  auto to = [&](const at::Tensor& t) {
+    return from(t) + ((t.size(0) - 1) * t.stride(0) + t.size(1)) * t.element_size();
+  };
+  return to(read) <= from(written) || to(written) <= from(read);
+}
+
 }  // namespace
 
 bool product_takes(const std::vector<ProductBlock>& blocks, bool rows_of_b) {
@@ -562,7 +572,8 @@ bool product(const std::vector<ProductBlock>& blocks, bool rows_of_b, const at::
   Args o{};
   int64_t width = 0;
   for (const auto& b : blocks) width += b.width;
-  if (!fill(o, each(blocks), rows_of_b) || !shaped(out, o.M, width) || (res && !shaped(*res, o.M, width)))
+  if (!fill(o, each(blocks), rows_of_b) || !shaped(out, o.M, width) ||
+      (res && !(shaped(*res, o.M, width) && clear_of(*res, out))))
     return false;
   o.c = ptr(out);
   o.ldc = (int)out.stride(0);
@@ -599,7 +610,7 @@ bool product_glu_bwd(const ProductBlock& block, const at::Tensor& gu, const at::
   Args o{};
   if (!fill(o, {&block}, true) || block.bias || !shaped(gu, o.M, 2 * block.width) ||
       !shaped(dgate, o.M, block.width) || !shaped(dup, o.M, block.width) ||
-      dgate.stride(0) != dup.stride(0))
+      dgate.stride(0) != dup.stride(0) || !clear_of(gu, dgate) || !clear_of(gu, dup))
     return false;
   o.gu = ptr(gu);
   o.ldgu = (int)gu.stride(0);

@@ -181,3 +181,17 @@ def test_refuses_what_it_cannot_walk(ext):
     assert not takes(rand(64, 64).t(), rand(64, 64))          # columns on end
     assert not takes(rand(64, 64), rand(60, 64), rand(64, 60), 60)
     assert not takes(rand(64, 64).cpu(), rand(64, 64))
+
+
+def test_refuses_a_residual_where_it_writes(ext):
+    """Shares of K may be joined twice: what is added lies clear of the output."""
+    rand = _make(6)
+    a, b, wide = rand(64, 64), rand(64, 64), rand(130, 72)
+    before = wide.clone()
+    for out, res in ((wide[:64, :64], wide[:64, :64]), (wide[:64, :64], wide[63:127, :64])):
+        assert not ext.product([[a]], [[b]], [None], [64], "columns", [out], res)
+        gu = wide.view(-1)[:64 * 128].view(64, 128)
+        assert not ext.product([[a]], [[b]], [None], [64], "glu_bwd", [out, out], gu)
+    assert torch.equal(wide, before)
+    assert ext.product([[a]], [[b]], [None], [64], "columns", [wide[:64, :64]], wide[64:128, :64])
+    _close(wide[:64, :64], a.float() @ b.float().t() + before[64:128, :64].float())
