@@ -382,18 +382,25 @@ class Engine:
     def _own_prefill(self, rows: int, site: str, rank: int) -> bool:
         """Whether a prompt phase of so many rows takes a site through products
         of our own. They take adapters, activation and residual with them and
-        a few us of the host where the library takes 17 a call; its tiles are
-        the faster on wide weights, with an adapter from some 8192 rows on,
-        without one from 60 GFLOP (700 rows, gate and up of the 7B model with
-        activation 192 us and 180; 924 rows, of the 1.5B model 66 and 80)."""
-        s = self.spec
-        n, k = {"qkv": (s.q_size + 2 * s.kv_size, s.hidden_size),
-                "o": (s.hidden_size, s.q_size),
-                "gateup": (2 * s.intermediate_size, s.hidden_size),
-                "down": (s.hidden_size, s.intermediate_size)}[site]
+        a few us of the host where the library takes 17 a call. Whole phases,
+        ms, own or by this rule -> the library's: with an adapter of rank 32
+        512, 4096 and 12288 rows of the 0.5B model 3.9, 7.8, 16.5 -> 10.1,
+        12.4, 22.8, 4B 11.1, 36, 95 -> 14.7, 42, 102, 7B 14.4, 55, 151 -> 18.7,
+        66, 169, the least gain 0.4 % (4B, 2048 rows). Without one
+        gate and up with their activation are the faster where K is short (1.5B,
+        2048 rows 8.5 -> 9.1; 4B and 7B -4 to 15 %), down where rows are few (7B,
+        512 rows 10.7 -> 12.8, 683 13.2 -> 13.2), the others only while the
+        phase waits for the host (all of the 1.5B model 200 rows 3.9 -> 4.6,
+        683 rows 5.4 -> 5.1; of the 4B model 57 rows 5.0 -> 5.8, 200 8.1 -> 6.1)."""
         if rank:
-            return rows <= 8192 or max(n, k) < 4096
-        return 2 * rows * n * k < 60e9
+            return True
+        s = self.spec
+        short = s.hidden_size <= 2048
+        if site == "gateup" and short or site == "down" and rows <= 512:
+            return True
+        layer = s.hidden_size * (2 * s.q_size + 2 * s.kv_size
+                                 + 3 * s.intermediate_size)
+        return 2 * rows * layer < (30e9 if short else 15e9)
 
     def _qk_norm(self, at, q, k):
         """Qwen3 per-head q/k RMSNorm over head_dim, applied before RoPE

@@ -206,3 +206,17 @@ def test_geom_len_mean_draws_deterministic_limits(setup):
     lens = [len(ids) for per in outs[0] for ids in per]
     assert all(1 <= L <= 20 for L in lens)
     assert len(set(lens)) > 1  # the exponential actually varies the caps
+
+
+@pytest.mark.parametrize("model,rank,rows,own", [
+    ("qwen2.5-0.5b", 0, 850, "qkv o gateup down"), ("qwen2.5-0.5b", 0, 4096, "gateup"),
+    ("qwen2.5-1.5b", 0, 57, "qkv o gateup down"), ("qwen2.5-1.5b", 0, 683, "gateup"),
+    ("qwen3-4b", 0, 57, "qkv o gateup down"), ("qwen3-4b", 0, 256, "down"),
+    ("qwen3-4b", 0, 683, ""), ("qwen2.5-7b", 0, 512, "down"), ("qwen2.5-7b", 0, 1024, ""),
+    ("qwen2.5-7b", 32, 12288, "qkv o gateup down")])
+def test_prompt_products_where_they_are_the_faster(model, rank, rows, own):
+    """Sites of a prompt phase that our own products take, as measured."""
+    from types import SimpleNamespace
+    engine = SimpleNamespace(spec=get_spec(model))
+    assert own.split() == [site for site in ("qkv", "o", "gateup", "down")
+                           if Engine._own_prefill(engine, rows, site, rank)]
