@@ -666,25 +666,26 @@ class Engine:
             # and the activation along
             t = self.fused.tiled
 
+            def product(x, w, mode, **kw):
+                return ext.skinny_gemm(x, w, mode, tiles=t,
+                                       kept=self.fused.kept, **kw)
+
             def weight(lw, site):
                 return lw.tiles[site] if t else lw.rows(site)
 
             for li, lw in enumerate(lws):
-                qkv = ext.skinny_gemm(res, weight(lw, "qkv"), 0, bias=lw.qkv_b,
-                                      norm_w=lw.in_norm, eps=eps, tiles=t)
-                res = ext.skinny_gemm(attend(qkv, li), weight(lw, "o"), 1,
-                                      res=res, tiles=t)
-                act = ext.skinny_gemm(res, weight(lw, "gateup"), 2,
-                                      norm_w=lw.post_norm, eps=eps, tiles=t)
+                qkv = product(res, weight(lw, "qkv"), 0, bias=lw.qkv_b,
+                              norm_w=lw.in_norm, eps=eps)
+                res = product(attend(qkv, li), weight(lw, "o"), 1, res=res)
+                act = product(res, weight(lw, "gateup"), 2,
+                              norm_w=lw.post_norm, eps=eps)
                 if apart:
                     # the 4-bit site keeps its adapter beside the base image
-                    u = ext.skinny_gemm(act, lw.down_a, 0, tiles=t)
+                    u = product(act, lw.down_a, 0)
                     base = lw.tiles["down"] if t else lw.rows("base")
-                    res = ext.skinny_gemm(act, base, 1, res=res, u=u,
-                                          ub=lw.down_b, tiles=t)
+                    res = product(act, base, 1, res=res, u=u, ub=lw.down_b)
                 else:
-                    res = ext.skinny_gemm(act, weight(lw, "down"), 1, res=res,
-                                          tiles=t)
+                    res = product(act, weight(lw, "down"), 1, res=res)
             return m.logits(ext.rmsnorm_fwd(res, m.model.norm.weight, eps))
 
         if streamed:

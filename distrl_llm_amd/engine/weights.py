@@ -252,6 +252,12 @@ class FusedWeights:
             and _room_for(2 * s.num_layers * 2 * s.hidden_size * (
                 2 * s.q_size + 2 * s.kv_size + 3 * s.intermediate_size),
                 q0.weight.device))
+        # whether the last-level cache (256 MB) holds the tiles from one step to
+        # the next: steps of few rows then read them through it (one row, 96
+        # tokens, ms, through and past the caches: 183 MB of layers 61.5 and
+        # 63.1, 212 MB 35.0 and 35.5, 239 MB 28.7 and 28.4; 74.3 and 74.3)
+        self.kept = 2 * s.num_layers * s.hidden_size * (
+            2 * s.q_size + 2 * s.kv_size + 3 * s.intermediate_size) < 224e6
         # the 4-bit kernel's packs of the down site: only steps beyond the
         # streamed products' rows use them
         self._nf4_down = False

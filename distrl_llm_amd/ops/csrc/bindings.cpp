@@ -59,7 +59,8 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
                           c10::optional<torch::Tensor> res,
                           c10::optional<torch::Tensor> norm_w, double eps,
                           c10::optional<torch::Tensor> u,
-                          c10::optional<torch::Tensor> ub, bool tiles);
+                          c10::optional<torch::Tensor> ub, bool tiles,
+                          bool kept);
 bool stream_gemm_takes(int64_t M, int64_t N, int64_t K);
 torch::Tensor stream_glu(torch::Tensor x, torch::Tensor w);
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
@@ -225,7 +226,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("bias") = py::none(), py::arg("res") = py::none(),
         py::arg("norm_w") = py::none(), py::arg("eps") = 0.0,
         py::arg("u") = py::none(), py::arg("ub") = py::none(),
-        py::arg("tiles") = false);
+        py::arg("tiles") = false, py::arg("kept") = false);
   m.def("stream_gemm_takes", &stream_gemm_takes,
         "whether stream_gemm and stream_glu take (M, N, K)");
   m.def("stream_glu", &stream_glu,

@@ -9,11 +9,11 @@
 // Partial sums meet in LDS. The norm needs no pass of its own: the waves
 // multiply x by the norm weight as they read it and sum its squares on the way,
 // 1/rms scales the finished row.
-// Tiles of W are read past the caches, which hold no model's weights from one step
-// to the next (256 MB; matrices small enough to stay there would be read faster through
-// them: 9728 x 896 at one row 5.6 us, and 6.3 so). At one row, us: 19456 x 2560 22.3 ->
-// 21.3, 2560 x 9728 13.6 -> 12.7. From rows a load is half a cache line of each, whose
-// other half has to stay: 35.9 past the caches, 29.3 through them.
+// Tiles of W are read past the caches where these (256 MB) hold no model's weights from
+// one step to the next, which the caller knows. At one row, us: 19456 x 2560 22.3 ->
+// 21.3, 2560 x 9728 13.6 -> 12.7; but 9728 x 896 from the caches 5.6, past them 6.3. From
+// rows a load is half a cache line of each, whose other half has to stay: 35.9 past
+// the caches, 29.3 through them.
 // A step of a few sequences is bound by its launches' latency (~4 us each) as
 // much as by bytes, hence the fusions: on the 0.5B model at 8 rows a layer took
 // 67 us in 11 launches, 39 in 7 now (gate|up + SiLU 17 + 5 -> 11.6 us, down and
@@ -30,6 +30,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 namespace {
 
 enum { PLAIN = 0, RESIDUAL = 1, GLU = 2 };
+enum { ROWS = 0, TILES = 1, KEPT = 2 };     // W, KEPT: tiles that the caches hold
 
 // Steps of K a wave has in flight: what its registers hold.
 template <int MT, int KW, int ACC, bool NORM>
@@ -38,7 +39,7 @@ constexpr int in_flight() {
   return n > 10 ? 10 : n;
 }
 
-template <int MT, int KW, int MODE, bool NORM, bool TILES>
+template <int MT, int KW, int MODE, bool NORM, int W>
 __global__ __launch_bounds__(KW * 64)
 void skinny_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat16* __restrict__ w,
                         const __hip_bfloat16* __restrict__ bias,
@@ -59,7 +60,7 @@ void skinny_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat
   const __hip_bfloat16* wp[ACC];
   #pragma unroll
   for (int a = 0; a < ACC; ++a) {
-    if (TILES) {
+    if (W != ROWS) {
       // row of the tile; SiLU*mul: 16 gate and 16 up rows
       const int n = MODE == GLU ? (n0 + wr) / 16 * 32 + a * 16 + (n0 + wr) % 16 : n0 + wr;
       wp[a] = w + (int64_t)(n >> 5) * K * 32 + (g >> 1) * 512 + (g & 1) * 256 + (n & 31) * 8;
@@ -87,8 +88,8 @@ void skinny_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat
       const int k = min(s + i, s1 - 1) * 32;              // past the end: the last again
       #pragma unroll
       for (int a = 0; a < ACC; ++a) {
-        const bf16v8* from = reinterpret_cast<const bf16v8*>(wp[a] + k * (TILES ? 32 : 1));
-        wf[i][a] = TILES ? __builtin_nontemporal_load(from) : *from;
+        const bf16v8* from = reinterpret_cast<const bf16v8*>(wp[a] + k * (W == ROWS ? 1 : 32));
+        wf[i][a] = W == TILES ? __builtin_nontemporal_load(from) : *from;
       }
       #pragma unroll
       for (int t = 0; t < MT; ++t)
@@ -197,12 +198,13 @@ bool skinny_gemm_takes(int64_t M, int64_t N, int64_t K) {
 }
 
 // mode 0: x W^T (+ bias); 1: res + x W^T (+ u ub^T); 2: silu(x Wg^T) * (x Wu^T)
-// with w = [Wg; Wu]. norm_w: x is RMS-normed first.
+// with w = [Wg; Wu]. norm_w: x is RMS-normed first. tiles: w lies in tiles; kept: and
+// stays in the caches from one call to the next.
 torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
                           c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> res,
                           c10::optional<torch::Tensor> norm_w, double eps,
                           c10::optional<torch::Tensor> u, c10::optional<torch::Tensor> ub,
-                          bool tiles) {
+                          bool tiles, bool kept) {
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous());
   TORCH_CHECK(w.is_cuda() && w.dim() == 2 && w.is_contiguous());
   TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16);
@@ -243,17 +245,18 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
   const int nt = N / 16, steps = K / 32, tr = nt <= 128 ? 8 : 16;
   const int kw = nt <= 256 ? (steps >= 64 ? 16 : steps >= 32 ? 8 : 4)
                         : (mode == GLU && steps >= 48 ? 8 : 4);
-  auto launch = [&](auto mt_, auto kw_, auto mode_, auto norm_, auto tiles_) {
+  auto launch = [&](auto mt_, auto kw_, auto mode_, auto norm_, auto w_) {
     constexpr int MT = decltype(mt_)::value, KW = decltype(kw_)::value,
                   MODE = decltype(mode_)::value;
     constexpr bool NORM = decltype(norm_)::value;
     const size_t smem = KW * (MODE == GLU ? 2 : 1) * MT * 64 * 16;
-    hipLaunchKernelGGL((skinny_gemm_kernel<MT, KW, MODE, NORM, decltype(tiles_)::value>), dim3(N / tr), dim3(KW * 64), smem,
-                       stream, ptr(x), ptr(w), b, r, nw, up, ubp, o, M, N, K, R, tr, (float)eps);
+    hipLaunchKernelGGL((skinny_gemm_kernel<MT, KW, MODE, NORM, decltype(w_)::value>), dim3(N / tr),
+                       dim3(KW * 64), smem, stream, ptr(x), ptr(w), b, r, nw, up, ubp, o, M, N, K, R, tr, (float)eps);
   };
   auto go = [&](auto mt_, auto kw_, auto mode_, auto norm_) {
-    if (tiles) launch(mt_, kw_, mode_, norm_, std::true_type{});
-    else launch(mt_, kw_, mode_, norm_, std::false_type{});
+    if (!tiles) launch(mt_, kw_, mode_, norm_, std::integral_constant<int, ROWS>{});
+    else if (kept) launch(mt_, kw_, mode_, norm_, std::integral_constant<int, KEPT>{});
+    else launch(mt_, kw_, mode_, norm_, std::integral_constant<int, TILES>{});
   };
   auto by_norm = [&](auto mt_, auto kw_, auto mode_) {
     if (nw) go(mt_, kw_, mode_, std::true_type{}); else go(mt_, kw_, mode_, std::false_type{});

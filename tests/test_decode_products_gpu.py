@@ -86,8 +86,9 @@ def test_skinny_gemm_tiles(ext, M, N, K):
     for mode, rows, tiles, args in (
             (0, half, t, {"bias": b}), (0, half, t, {"bias": b, **kw}),
             (1, half, t, {"res": res, "u": u, "ub": ub}), (2, w, tg, {}), (2, w, tg, kw)):
-        assert torch.equal(ext.skinny_gemm(x, tiles, mode, tiles=True, **args),
-                           ext.skinny_gemm(x, rows, mode, **args))
+        want = ext.skinny_gemm(x, rows, mode, **args)
+        for kept in (False, True):
+            assert torch.equal(ext.skinny_gemm(x, tiles, mode, tiles=True, kept=kept, **args), want)
 
 
 @pytest.mark.parametrize("S", [1, 3, 4, 9])
