@@ -10,8 +10,8 @@ is 7 launches forward and 9 or 10 backward here, prepared in native code
 (ops/csrc/adapted_layer.cpp): products of our own (ops/csrc/product.hip) take
 adapters as more of their projections' K, residuals, the activation and its
 gradient with them. The library's products, where many rows meet wide weights,
-have W laid out beside B for it; large weights that few rows meet are taken as
-they lie, their adapters joined to fp32 products. Adapter gradients are one
+have W laid out beside B for it; at ranks that ours don't take large weights that
+few rows meet are taken as they lie, their adapters joined to fp32 products. Adapter gradients are one
 launch and its sum (ops/csrc/adapter_grads.hip).
 """
 

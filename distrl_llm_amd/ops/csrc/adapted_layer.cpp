@@ -6,8 +6,8 @@
 // sum, x W^T + u B^T, with its bias or the residual; backward is dY W + du A. Own
 // products (product.hip) take all of them from where they lie, the activation and its
 // gradient with them. For the library, where it is the faster or ranks don't fit, u
-// lies beside x in one matrix, [x | u], for one product with [W | B], and few rows
-// take large weights as they lie.
+// lies beside x in one matrix, [x | u], for one product with [W | B]; where ranks don't
+// fit few rows take large weights as they lie.
 //
 // Native because short micro-batches wait for the host: prepared in Python a pass of
 // the 0.5B model over three short samples took 25.0 ms, with the library's products
@@ -116,14 +116,19 @@ struct Adapters {
   }
 };
 
-// Whether rows take weights (N, K) as they lie, each projection's product in fp32 and
-// its adapter joined to that, rather than laid out beside the adapter for one product.
+// Whether rows that products of our own don't take (an adapter's rank is no multiple of
+// 32) take weights (N, K) as they lie, each projection's product in fp32 and its adapter
+// joined to that, rather than laid out beside the adapter for one library product.
 // Laying out moves the weights twice whatever the rows; joining moves every row and
 // launches more, which small models wait for. A pass of a model over 62, 276, 686,
 // 1352, 2008, 3687 and 6708 rows, laid out -> as they lie, ms: 7B 37.3, 42.3, 52.4,
 // 74.4, 95.4, 146, 253 -> 27.4, 33.6, 45.2, 68.6, 93.2, 147, 262; 4B 29.5, 36.4, 45.3,
 // 59.7, 71.7, 99, 187 -> 26.7, 33.9, 42.2, 57.8, 70.2, 106, 201; the 1.5B's gate and
 // up (27.5M) at 62, 686 and 2008 rows 18.4, 23.6, 34.3 -> 19.9, 25.1, 34.6.
+// Own products, where they take the operands, are the faster: a layer of 64, 700, 1400
+// and 2048 rows, as they lie -> own, us: 7B 858, 1488, 2192, 3080 -> 570, 1270, 2188,
+// 2491; 4B 589, 878, 1222, 1579 -> 332, 734, 1061, 1610; a pass over 89, 506 and 1278
+// rows, ms: 7B 27.9, 39.6, 70.3 -> 22.8, 35.6, 63.6; 4B 25.7, 36.6, 52.9 -> 23.5, 33.0, 50.4.
 bool apart(int64_t rows, int64_t N, int64_t K) { return rows <= 2048 && N * K >= 32 << 20; }
 
 // out <- y + u m (+ res), y fp32
@@ -162,6 +167,13 @@ Tensor projected(const Tensor& xu, const Tensors& W, const Adapters& ad,
   bool any = false;
   for (const auto& w : W) width += w.size(0);
   for (const auto& b : bias) any = any || b;
+  if (!library(rows, width, K)) {
+    const auto sums = blocks(columns(xu, 0, K), columns(xu, K, ad.pad), W, ad, bias);
+    if (product_takes(sums, false)) {
+      auto out = at::empty({rows, width}, xu.options());
+      if (product(sums, false, out, res)) return out;
+    }
+  }
   if (apart(rows, width, K)) {
     auto out = at::empty({rows, width}, xu.options());
     const auto x = columns(xu, 0, K), u = columns(xu, K, ad.pad);
@@ -173,13 +185,6 @@ Tensor projected(const Tensor& xu, const Tensors& W, const Adapters& ad,
       from += n;
     }
     return out;
-  }
-  if (!library(rows, width, K)) {
-    const auto sums = blocks(columns(xu, 0, K), columns(xu, K, ad.pad), W, ad, bias);
-    if (product_takes(sums, false)) {
-      auto out = at::empty({rows, width}, xu.options());
-      if (product(sums, false, out, res)) return out;
-    }
   }
   const auto WB = adapted_weight(W, ad.B, ad.pad);
   if (res) return at::addmm(*res, xu, WB.t());
@@ -230,11 +235,6 @@ struct Through { Tensor dx, du; };
 // g W + du A with du = scale * g B, and du
 Through through(const Tensor& g, const Tensor& W, const Adapters& ad) {
   const int64_t N = g.size(1);
-  if (apart(g.size(0), N, W.size(1))) {
-    auto du = at::empty({g.size(0), ad.pad}, g.options());
-    ad.up({g}, du);
-    return {back_apart({g}, {W}, du, ad), ad.part(du, 0)};
-  }
   if (!library(g.size(0), N, W.size(1))) {
     auto du = at::empty({g.size(0), ad.pad}, g.options());
     const auto r = ad.part(du, 0);
@@ -244,6 +244,11 @@ Through through(const Tensor& g, const Tensor& W, const Adapters& ad) {
       ad.up({g}, du);
       if (product(sum, true, dx)) return {dx, r};
     }
+  }
+  if (apart(g.size(0), N, W.size(1))) {
+    auto du = at::empty({g.size(0), ad.pad}, g.options());
+    ad.up({g}, du);
+    return {back_apart({g}, {W}, du, ad), ad.part(du, 0)};
   }
   auto gd = at::empty({g.size(0), N + ad.pad}, g.options());
   auto g2 = columns(gd, 0, N), du = columns(gd, N, ad.pad);
@@ -389,10 +394,10 @@ Tensors attention_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tensors 
   out.push_back(s[1]);
   out.push_back(s[2]);
   Tensor dx;
-  if (want_dx && apart(rows, width, hidden)) {
-    dx = rmsnorm_bwd_add(back_apart(dys, {W[0], W[1], W[2]}, du, in), x, norm, g, eps);
-  } else if (want_dx && own_dx(dx, {W[0], W[1], W[2]}, dys, du, in)) {
+  if (want_dx && own_dx(dx, {W[0], W[1], W[2]}, dys, du, in)) {
     dx = rmsnorm_bwd_add(dx, x, norm, g, eps);
+  } else if (want_dx && apart(rows, width, hidden)) {
+    dx = rmsnorm_bwd_add(back_apart(dys, {W[0], W[1], W[2]}, du, in), x, norm, g, eps);
   } else if (want_dx) {
     const auto WA = stack_transposed({W[0], W[1], W[2], A[0], A[1], A[2]},
                                      {0, sizes[0], sizes[0] + sizes[1], width, width + in.at[1],
@@ -422,7 +427,7 @@ Tensors feed_forward_half_fwd(Tensor x, Tensor norm, double eps, Tensors W,
   auto act = columns(au, 0, inner);
   Tensor gu;
   bool ready = false;                     // act's adapter inputs
-  if (!apart(rows, 2 * inner, hidden) && !library(rows, 2 * inner, hidden)) {
+  if (!library(rows, 2 * inner, hidden)) {
     const auto both = blocks(h, columns(hu, hidden, in.pad), {W[0], W[1]}, in, bias);
     const auto &ug = both[0].terms[1].a, &uu = both[1].terms[1].a;
     const ProductBlock gate{inner, {both[0].terms[0], {ug, B[0]}, {uu, {}}}, bias[0]};
@@ -459,7 +464,7 @@ Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tenso
        du = columns(dyu, 2 * inner, in.pad);
   Tensor dud;
   bool ready = false;                     // dgate's and dup's adapter inputs
-  if (!apart(rows, hidden, inner) && !library(rows, hidden, inner)) {
+  if (!library(rows, hidden, inner)) {
     auto both = at::empty({rows, d_ad.pad}, x.options());
     const auto r = d_ad.part(both, 0);
     const ProductBlock dact{inner, {{g, W[2]}, {r, A[2]}}, {}};
@@ -485,10 +490,10 @@ Tensors feed_forward_half_bwd(Tensor g, Tensor x, Tensor norm, double eps, Tenso
   out.push_back(s[1]);
   out.push_back(s[2]);
   Tensor dx;
-  if (want_dx && apart(rows, 2 * inner, hidden)) {
-    dx = rmsnorm_bwd_add(back_apart({dgate, dup}, {W[0], W[1]}, du, in), x, norm, g, eps);
-  } else if (want_dx && own_dx(dx, {W[0], W[1]}, {dgate, dup}, du, in)) {
+  if (want_dx && own_dx(dx, {W[0], W[1]}, {dgate, dup}, du, in)) {
     dx = rmsnorm_bwd_add(dx, x, norm, g, eps);
+  } else if (want_dx && apart(rows, 2 * inner, hidden)) {
+    dx = rmsnorm_bwd_add(back_apart({dgate, dup}, {W[0], W[1]}, du, in), x, norm, g, eps);
   } else if (want_dx) {
     const auto WA = stack_transposed({W[0], W[1], A[0], A[1]},
                                      {0, inner, 2 * inner, 2 * inner + in.ranks[0]},

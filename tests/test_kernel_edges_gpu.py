@@ -519,11 +519,12 @@ def test_fused_layer_matches_modules(name, B, T):
 
 
 @pytest.mark.parametrize("B,T", [(1, 1), (2, 77)])
-@pytest.mark.parametrize("lora_r,norms", [(8, False), (12, True), (96, False)])
+@pytest.mark.parametrize("lora_r,norms", [(8, False), (12, True), (32, False), (96, False)])
 def test_fused_layer_takes_large_weights_as_they_lie(B, T, lora_r, norms):
     """Few rows of a layer whose products are all past the size where weights
     are no longer laid out beside their adapters, at ranks that the joining
-    kernel takes and that it does not: against fp64, as above."""
+    kernel takes and that it does not, and at two that go through our own products:
+    against fp64, as above."""
     from distrl_llm_amd.models import CausalLM, fused_layer
     from distrl_llm_amd.models.spec import ModelSpec
     spec = ModelSpec("wide", 64, 4096, 8192, 1, 64, 8, 128, 1e6, 1e-6, True, not norms,
@@ -535,7 +536,8 @@ def test_fused_layer_takes_large_weights_as_they_lie(B, T, lora_r, norms):
     exact = CausalLM(spec, lora_r=lora_r, lora_alpha=16, dtype=torch.float64)
     exact.load_state_dict({k: v.double().cpu() for k, v in model.state_dict().items()})
     ref = _grads(exact.train(), ids.cpu(), mask.cpu(), dout.double().cpu())
-    fused = _grads(model, ids, mask, dout)
+    fused, ran = _kernels(lambda: _grads(model, ids, mask, dout))
+    assert ran("product_kernel") == (0 if lora_r % 32 else 7)
     usable = fused_layer.usable
     fused_layer.usable = lambda layer, x: False
     try:
