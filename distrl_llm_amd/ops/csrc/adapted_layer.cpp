@@ -46,7 +46,10 @@ struct NoAutocast {
 Tensor columns(const Tensor& t, int64_t from, int64_t n) { return t.narrow(1, from, n); }
 
 // Rows from which 32 of them a workgroup fill the chip: the activation then carries its
-// adapter inputs along.
+// adapter inputs along. A feed-forward half forward and back with the library's
+// products, apart -> along, us: 1.5B, 2048, 4096, 7000, 9000, 16384 rows 730, 1103, 1717,
+// 2072, 3324 -> 763, 1111, 1676, 2070, 3213; 4B, 4096, 8192, 12000 1558, 2851, 3804 -> 1568,
+// 2803, 3730.
 constexpr int64_t FULL = 8192;
 
 Tensor heads(const Tensor& t, int64_t head_dim) {
@@ -147,7 +150,14 @@ void join(const Tensor& y, const Tensor& u, const Tensor& m, const Tensor& out,
 // gate and up 850 -> 800, gate, up and activation 1080 -> 1060, the activation's gradient
 // 840 -> 820, its epilogue not hidden behind another tile's products; but q, k, v 127 ->
 // 160, o 111 -> 122.
-bool library(int64_t rows, int64_t N, int64_t K) { return rows > 8192 && std::max(N, K) >= 4096; }
+// On either side of the line a feed-forward half, own -> library: 7000 and 8192 rows
+// 1.5B 1537, 1783 -> 1676, 1650, 7B (6000) 5246, 6673 -> 5414, 6596; 9000, 12000, 16384
+// rows 0.5B 828, 1022, 1350 -> 830, 1099, 1327, 1.5B 1791, 2639, 3434 -> 2030, 2453,
+// 3075, 4B 2943, 3707, 5160 -> 2961, 3583, 4926, 7B 7199, 9559, 12608 -> 6660, 9193, 11860.
+// And by width an attention half, whose widest are 6144 and 4608: 9000 and 16384 rows
+// 4B 1472, 2482 -> 1595, 2655, 7B 1495, 2637 -> 1502, 2766; the 0.5B's down (4864), with
+// the rest of its half, 807, 1329 -> 830, 1327.
+bool library(int64_t rows, int64_t N, int64_t K) { return rows > 8192 && std::max(N, K) >= 8192; }
 
 // x W^T + u B^T of projections of one input
 std::vector<ProductBlock> blocks(const Tensor& x, const Tensor& u, const Tensors& W,
