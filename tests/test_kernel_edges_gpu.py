@@ -487,22 +487,26 @@ def _grads(model, ids, mask, dout):
 
 @pytest.mark.parametrize("name", ["small-qwen2", "small-qwen3"])
 @pytest.mark.parametrize("B,T", [(1, 1), (2, 77), (3, 200)])
-def test_fused_layer_matches_modules(name, B, T):
+@pytest.mark.parametrize("lora_r", [8, 32, 64])
+def test_fused_layer_matches_modules(name, B, T, lora_r):
     """Hidden states and adapter gradients against the same model in fp64 on
     the CPU: no further off than the module path (1.3 times leaves room for
-    other roundings of the same size), with padding at the ends."""
+    other roundings of the same size), with padding at the ends; at a rank that
+    the library's products take and at two that ours do."""
     from distrl_llm_amd.models import CausalLM, fused_layer
-    model = _train_model(name)
+    model = _train_model(name, lora_r=lora_r)
     g = torch.Generator().manual_seed(T)
     ids = torch.randint(0, model.spec.vocab_size, (B, T), generator=g).cuda()
     lens = torch.randint(max(1, T // 2), T + 1, (B,), generator=g)
     mask = (torch.arange(T)[None] < lens[:, None]).long().cuda()
     dout = _rand((B, T, model.spec.hidden_size), 9) * mask.unsqueeze(-1)
-    exact = CausalLM(model.spec, lora_r=8, lora_alpha=16, dtype=torch.float64)
+    exact = CausalLM(model.spec, lora_r=lora_r, lora_alpha=16, dtype=torch.float64)
     exact.load_state_dict({k: v.double().cpu() for k, v in model.state_dict().items()})
     ref = _grads(exact.train(), ids.cpu(), mask.cpu(), dout.double().cpu())
     real = mask.bool().cpu()
-    fused = _grads(model, ids, mask, dout)
+    (fused, ran) = _kernels(lambda: _grads(model, ids, mask, dout))
+    # a layer: q|k|v, o, gate|up, down and back, but to the embedding
+    assert ran("product_kernel") == (0 if lora_r % 32 else 8 * model.spec.num_layers - 1)
     usable = fused_layer.usable
     fused_layer.usable = lambda layer, x: False
     try:
@@ -743,8 +747,9 @@ def test_lora_add(ext, M, N, r):
 
 
 @pytest.mark.parametrize("name", ["small-qwen2", "small-qwen3"])
-@pytest.mark.parametrize("lora_r,four_bit", [(0, False), (8, False), (8, True), (12, False)])
-def test_packed_prefill_matches_modules(name, lora_r, four_bit):
+@pytest.mark.parametrize("lora_r,four_bit", [(0, False), (8, False), (8, True), (12, False),
+                                             (32, False), (64, True)])
+def test_packed_prefill_matches_modules(ext, monkeypatch, name, lora_r, four_bit):
     """Logits and cache rows of a ragged batch against the module path (two
     bf16 paths of the same products: 2 %), and the merged weights against
     W + scale * B A at a rank the kernel takes and one it does not."""
@@ -762,7 +767,9 @@ def test_packed_prefill_matches_modules(name, lora_r, four_bit):
         model.quantize_nf4_()
     g = torch.Generator().manual_seed(1)
     prompts = [torch.randint(0, 4096, (n,), generator=g).tolist() for n in (3, 64, 129, 1)]
-    got = []
+    got, own = [], []
+    for f in ("adapted_projection", "adapted_activation"):
+        monkeypatch.setattr(ext, f, lambda *a, _f=getattr(ext, f): own.append(_f(*a)) or own[-1])
     for packs in (True, False):
         eng = Engine(model, EngineConfig(max_seq_length=256, num_kv_blocks=32, max_num_seqs=8))
         eng.fused.refresh()
@@ -772,6 +779,9 @@ def test_packed_prefill_matches_modules(name, lora_r, four_bit):
         got.append((logits, eng.pool.key, eng.pool.value))
     for x, y in zip(*got):
         assert _rel(x, y) < 0.02
+    # every site through our products, or through the library's
+    assert len(own) == 4 * model.spec.num_layers
+    assert all((x is None) == (lora_r % 32 != 0) for x in own)
     at = model.model.layers[1].self_attn
     w = at.k_proj.weight.double()
     if lora_r:
@@ -1122,6 +1132,47 @@ def test_feed_forward_half_in_waves(ext, rows):
     assert _rel(y, ref.detach()) < 2.0 ** -7
     for at in (slice(None), slice(0, 1), slice(4095, 4097), slice(rows - 1, rows)):
         assert _rel(dx[at], want[at]) < 2.0 ** -6
+
+
+@pytest.mark.parametrize("rows,h,f", [(70, 128, 256), (8200, 128, 256), (8200, 8192, 64)])
+@pytest.mark.parametrize("r", [8, 32, 64])
+@pytest.mark.parametrize("biased", [False, True])
+def test_feed_forward_half(ext, rows, h, f, r, biased):
+    """Output, input gradient and every adapter's gradients of one half against fp64, each
+    adapter a scale of its own and some tenth of its projection, rows and widths on
+    either side of the rules for our products and the library's. Bounds: the
+    bf16 rounding of each value on the way (adapter inputs, activation, its
+    gradient, the sum), some 2^-9 each."""
+    x, g, norm = _rand((rows, h), 1), _rand((rows, h), 2), _rand((h,), 3, 0.1) + 1
+    Ws = [_rand(s, 4 + i, s[1] ** -0.5) for i, s in enumerate(((f, h), (f, h), (h, f)))]
+    As = [_rand((r, w.shape[1]), 7 + i, w.shape[1] ** -0.5) for i, w in enumerate(Ws)]
+    Bs = [_rand((w.shape[0], r), 10 + i, 0.3 * r ** -0.5) for i, w in enumerate(Ws)]
+    scales, bias = [0.5, 2.0, 1.0], [_rand((f,), 13 + i) if biased else None for i in range(2)]
+    (y, hu, gu, au), ran = _kernels(
+        lambda: ext.feed_forward_half_fwd(x, norm, 1e-6, Ws, bias, As, Bs, scales))
+    own, wide = r % 32 == 0, rows > 8192 and h >= 8192      # as the rules have it
+    # gate|up with their activation, and down
+    assert ran("product_kernel") == (2 if own and not wide else 0)
+    assert ran("activation_inputs_kernel") == (1 if rows >= 8192 and (wide or not own) else 0)
+    (dx, *got), ran = _kernels(
+        lambda: ext.feed_forward_half_bwd(g, x, norm, 1e-6, Ws, As, Bs, scales, hu, gu, au, True))
+    assert ran("product_kernel") == (2 if own and not wide else 0)
+    leaves = [t.double().requires_grad_() for t in (x, *(m for ab in zip(As, Bs) for m in ab))]
+    xd, Ad, Bd = leaves[0], leaves[1::2], leaves[2::2]
+    n = xd * torch.rsqrt((xd * xd).mean(-1, keepdim=True) + 1e-6) * norm.double()
+
+    def proj(i, t):
+        return t @ Ws[i].double().t() + scales[i] * (t @ Ad[i].t()) @ Bd[i].t()
+
+    gate, up = (proj(i, n) + (bias[i].double() if biased else 0.0) for i in range(2))
+    ref = xd + proj(2, torch.nn.functional.silu(gate) * up)
+    want = torch.autograd.grad(ref, leaves, g.double())
+    assert _rel(gu, torch.cat([gate, up], 1).detach()) < 2.0 ** -7
+    for at in (slice(None), slice(0, 1), slice(rows - 1, rows)):
+        assert _rel(y[at], ref[at].detach()) < 2.0 ** -7
+        assert _rel(dx[at], want[0][at]) < 2.0 ** -6
+    for x, t in zip(got, want[1:]):
+        assert _rel(x, t) < 2.0 ** -6
 
 
 @pytest.mark.parametrize("r", [8, 16, 32])

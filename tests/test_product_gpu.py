@@ -6,10 +6,11 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# Bound: operands are exact in bf16 and sums fp32, so an output is off by its
-# own rounding to 8 significant bits, 2^-8 of it at most (half of the last one's
-# 2^-7), and by a sum's 2^-24 * K, far below that.
+# Bounds, of every output: operands are exact in bf16, so an output is off by its own
+# rounding to 8 significant bits, 2^-8 of it at most, and by its fp32 sum, n terms in
+# whatever order: n 2^-24 of the sum of their magnitudes.
 REL = 2.0 ** -8
+SENTINEL = 7.0
 TILES = [0, 8, 7, 6, 5, 4, 128, 64, 64 + 512, 128 + 768, 64 + 2048]
 
 
@@ -32,6 +33,30 @@ def _close(x, ref):
     assert float((x.float() - ref).norm() / ref.norm()) < REL
 
 
+def _each_close(x, ref, off):
+    """off: what else than its rounding an output may be off by, of every one."""
+    assert bool(((x.double() - ref).abs() <= REL * ref.abs() + 2 * off).all())
+
+
+def _sum(pairs, rows_of_b=False):
+    """Sums of products in fp64, and how far an fp32 sum of them may be off."""
+    pairs = [(x.double(), y.double() if rows_of_b else y.double().t()) for x, y in pairs]
+    return (sum(x @ y for x, y in pairs),
+            sum(x.abs() @ y.abs() for x, y in pairs) * (sum(x.shape[1] for x, _ in pairs) + 2) * 2.0 ** -24)
+
+
+def _room(M, width, spare):
+    """(rows to write into, whether what stands around them is untouched)"""
+    room = torch.full((M + 2, width + spare + 8), SENTINEL, dtype=torch.bfloat16, device="cuda")
+    out = room[1:-1, :width]
+
+    def untouched():
+        around = room.clone()
+        around[1:-1, :width] = SENTINEL
+        return bool((around == SENTINEL).all())
+    return out, untouched
+
+
 @pytest.mark.parametrize("M,widths,deep,spare", [
     (1, (8,), (32,), 0), (63, (64, 8), (32, 32), 8), (65, (72, 128, 64), (96, 32), 0),
     (129, (136,), (64, 32, 160), 64), (257, (256, 40), (224, 64), 0), (300, (520,), (1024,), 8),
@@ -46,13 +71,15 @@ def test_sums_of_products(ext, M, widths, deep, spare, tile):
         b = [[rand(w, k, spare=spare) if what == "columns" else rand(k, w, spare=spare)
               for k in deep] for w in widths]
         bias = [rand(w) if i != 1 else None for i, w in enumerate(widths)]
-        ref = [sum(x.float() @ (y.float().t() if what == "columns" else y.float())
-                   for x, y in zip(xs, ys)) for xs, ys in zip(a, b)]
-        ref = torch.cat([r if c is None else r + c.float() for r, c in zip(ref, bias)], 1)
+        sums = [_sum(zip(xs, ys), what == "rows") for xs, ys in zip(a, b)]
+        ref = torch.cat([r if c is None else r + c.double() for (r, _), c in zip(sums, bias)], 1)
+        off = torch.cat([o for _, o in sums], 1)
         for res in (None, rand(M, sum(widths), spare=spare)):
-            out = rand(M, sum(widths), spare=spare)
+            out, untouched = _room(M, sum(widths), spare)
             assert ext.product(a, b, bias, widths, what, [out], res, tile)
-            _close(out, ref if res is None else ref + res.float())
+            want = ref if res is None else ref + res.double()
+            _each_close(out, want, off + 2.0 ** -23 * (ref.abs() + want.abs()))
+            assert untouched()
 
 
 @pytest.mark.parametrize("M,F,K,r", [(1, 8, 32, 32), (70, 40, 96, 32), (130, 136, 64, 64),
@@ -65,21 +92,30 @@ def test_activation(ext, M, F, K, r, tile):
     x, ug, uu = rand(M, K), rand(M, r), rand(M, r)
     wg, wu, bg, bu = rand(F, K), rand(F, K), rand(F, r), rand(F, r)
     bias = [rand(F), None]
-    gu, act = rand(M, 2 * F), rand(M, F, spare=24)
+    (gu, gu_alone), (act, act_alone) = _room(M, 2 * F, 0), _room(M, F, 24)
     assert ext.product([[x, ug, uu]] * 2, [[wg, bg, None], [wu, None, bu]], bias, [F, F], "glu",
                        [gu, act], None, tile)
-    gate = x.float() @ wg.float().t() + ug.float() @ bg.float().t() + bias[0].float()
-    up = x.float() @ wu.float().t() + uu.float() @ bu.float().t()
-    _close(gu, torch.cat([gate, up], 1))
-    gate, up = gu.float().split(F, 1)
-    _close(act, torch.nn.functional.silu(gate) * up)
+    (gate, gate_off), (up, up_off) = _sum([(x, wg), (ug, bg)]), _sum([(x, wu), (uu, bu)])
+    gate = gate + bias[0].double()
+    _each_close(gu, torch.cat([gate, up], 1),
+                torch.cat([gate_off + 2.0 ** -23 * gate.abs(), up_off], 1))
+    gate, up = gu.double().split(F, 1)
+    sig = gate.sigmoid()
+    # the fast exponential and reciprocal: some 2^-22 of the result
+    _each_close(act, gate * sig * up, 2.0 ** -20 * (gate * sig * up).abs())
+    assert gu_alone() and act_alone()
 
     g, w, du, a = rand(M, K), rand(K, F), rand(M, r), rand(r, F)
-    d = rand(M, 2 * F, spare=8)
+    d, alone = _room(M, 2 * F, 0)
     assert ext.product([[g, du]], [[w, a]], [None], [F], "glu_bwd", list(d.split(F, 1)), gu, tile)
-    dact = g.float() @ w.float() + du.float() @ a.float()
-    sig = gate.sigmoid()
-    _close(d, torch.cat([dact * up * sig * (1 + gate * (1 - sig)), dact * gate * sig], 1))
+    dact, off = _sum([(g, w), (du, a)], True)
+    slope = 1 + gate * (1 - sig)
+    # the slope passes zero: its two terms are good to 2^-20 of their own
+    fast = 2.0 ** -20 * (dact * up * sig).abs() * (1 + gate.abs())
+    _each_close(d, torch.cat([dact * up * sig * slope, dact * gate * sig], 1),
+                torch.cat([off * (up * sig * slope).abs() + fast,
+                           off * (gate * sig).abs() + 2.0 ** -20 * (dact * gate * sig).abs()], 1))
+    assert alone()
 
 
 @pytest.mark.parametrize("M,F", [(1, 8), (31, 120), (33, 128), (64, 136), (100, 400), (70, 1032)])
@@ -88,24 +124,28 @@ def test_activation_with_adapter_inputs(ext, M, F, r, spare):
     """Edges of 32 rows and steps of 128 columns; the products are those of
     what was rounded and written, spare columns zero."""
     rand = _make(M + F)
-    gu, act = rand(M, 2 * F), rand(M, F, spare=16)
-    m, out = rand(r[0], F), rand(M, r[0] + spare, spare=12)
+    gu, m = rand(M, 2 * F), rand(r[0], F)
+    (act, act_alone), (out, out_alone) = _room(M, F, 16), _room(M, r[0] + spare, 12)
     assert ext.silu_mul_inputs(gu, act, m, 0.5, out)
-    gate, up = gu.float().split(F, 1)
-    _close(act, torch.nn.functional.silu(gate) * up)
-    _close(out[:, :r[0]], act.float() @ m.float().t() * 0.5)
-    assert not out[:, r[0]:].any()
-
-    dact, d = rand(M, F), rand(M, 2 * F + 8)
-    dgate, dup = d[:, :F], d[:, F:2 * F]
-    b, du = [rand(F, x) for x in r], rand(M, sum(r) + spare)
-    assert ext.silu_mul_bwd_inputs(dact, gu, dgate, dup, b, [0.5, 2.0], du)
+    gate, up = gu.double().split(F, 1)
     sig = gate.sigmoid()
-    _close(dgate, dact.float() * up * sig * (1 + gate * (1 - sig)))
-    _close(dup, dact.float() * gate * sig)
-    _close(du[:, :r[0]], dgate.float() @ b[0].float() * 0.5)
-    _close(du[:, r[0]:sum(r)], dup.float() @ b[1].float() * 2.0)
-    assert not du[:, sum(r):].any()
+    _each_close(act, gate * sig * up, 2.0 ** -20 * (gate * sig * up).abs())
+    ref, off = _sum([(act, m)])
+    _each_close(out[:, :r[0]], ref * 0.5, off * 0.5)
+    assert not out[:, r[0]:].any() and act_alone() and out_alone()
+
+    dact, (d, d_alone), (du, du_alone) = rand(M, F), _room(M, 2 * F, 0), _room(M, sum(r) + spare, 4)
+    dgate, dup = d[:, :F], d[:, F:]
+    b = [rand(F, x) for x in r]
+    assert ext.silu_mul_bwd_inputs(dact, gu, dgate, dup, b, [0.5, 2.0], du)
+    dact = dact.double()
+    _each_close(dgate, dact * up * sig * (1 + gate * (1 - sig)),
+                2.0 ** -20 * (dact * up * sig).abs() * (1 + gate.abs()))
+    _each_close(dup, dact * gate * sig, 2.0 ** -20 * (dact * gate * sig).abs())
+    for x, y, scale, at in ((dgate, b[0], 0.5, slice(0, r[0])), (dup, b[1], 2.0, slice(r[0], sum(r)))):
+        ref, off = _sum([(x, y)], True)
+        _each_close(du[:, at], ref * scale, off * scale)
+    assert not du[:, sum(r):].any() and d_alone() and du_alone()
 
 
 @pytest.mark.parametrize("M", [1, 57, 300])
