@@ -382,25 +382,27 @@ class Engine:
     def _own_prefill(self, rows: int, site: str, rank: int) -> bool:
         """Whether a prompt phase of so many rows takes a site through products
         of our own. They take adapters, activation and residual with them and
-        a few us of the host where the library takes 17 a call. Whole phases,
-        ms, own or by this rule -> the library's: with an adapter of rank 32
-        512, 4096 and 12288 rows of the 0.5B model 3.9, 7.8, 16.5 -> 10.1,
-        12.4, 22.8, 4B 11.1, 36, 95 -> 14.7, 42, 102, 7B 14.4, 55, 151 -> 18.7,
-        66, 169, the least gain 0.4 % (4B, 2048 rows). Without one
-        gate and up with their activation are the faster where K is short (1.5B,
-        2048 rows 8.5 -> 9.1; 4B and 7B -4 to 15 %), down where rows are few (7B,
-        512 rows 10.7 -> 12.8, 683 13.2 -> 13.2), the others only while the
-        phase waits for the host (all of the 1.5B model 200 rows 3.9 -> 4.6,
-        683 rows 5.4 -> 5.1; of the 4B model 57 rows 5.0 -> 5.8, 200 8.1 -> 6.1)."""
-        if rank:
-            return True
+        a few us of the host where the library takes 17 a call, and read the
+        modules' weights, where the library needs q|k|v and gate|up in one
+        matrix, which every refresh renews.
+        A call of generate for one token, ms, library -> this rule, without an
+        adapter: 57, 512, 2048 and 8192 rows 0.5B 6.5, 6.8, 7.5, 16.0 -> 3.5, 4.3,
+        5.9, 12.8, 1.5B 11.2, 10.5, 15.1, 30.3 -> 5.1, 7.0, 11.0, 26.3, 4B
+        19.1, 21.1, 31.8, 72.0 -> 9.7, 13.0, 22.7, 63.1, 7B 32.2, 37.9, 56.2, 117
+        -> 13.3, 18.8, 36.3, 99.8. o and down need no copy: own while the phase
+        waits for the host, down at few rows, and on small models (all sites own
+        instead, 2048 and 8192 rows 1.5B 12.0, 27.6, 4B 26.5, 67.8, 7B
+        36.5, 103).
+        With one of rank 32 a prompt phase alone of 512, 4096 and 12288 rows
+        0.5B 10.1, 12.4, 22.8 -> 3.9, 7.8, 16.5, 4B 14.7, 42, 102 -> 11.1, 36,
+        95, 7B 18.7, 66, 169 -> 14.4, 55, 151."""
         s = self.spec
-        short = s.hidden_size <= 2048
-        if site == "gateup" and short or site == "down" and rows <= 512:
+        if rank or site in ("qkv", "gateup") or s.hidden_size <= 1024:
             return True
         layer = s.hidden_size * (2 * s.q_size + 2 * s.kv_size
                                  + 3 * s.intermediate_size)
-        return 2 * rows * layer < (30e9 if short else 15e9)
+        return (site == "down" and rows <= 512
+                or 2 * rows * layer < (30e9 if s.hidden_size <= 2048 else 15e9))
 
     def _qk_norm(self, at, q, k):
         """Qwen3 per-head q/k RMSNorm over head_dim, applied before RoPE

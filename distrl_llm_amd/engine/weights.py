@@ -9,7 +9,7 @@ between rounds, so the engine folds it once per weight-sync:
 and lays the projections of a site (q|k|v, gate|up) out as one matrix, in the
 tiles that the decode products read (ops/csrc/skinny_gemm.hip up to 16 rows,
 stream_gemm.hip up to 160); row-major beside them only for what still goes to
-the library: large prompts of models without an adapter, and larger steps. A refresh
+the library: larger steps, and prompts whose operands our products don't take. A refresh
 writes each projection's merged weight straight into its tiles, one kernel a
 projection, once per generation round.
 

@@ -209,10 +209,9 @@ def test_geom_len_mean_draws_deterministic_limits(setup):
 
 
 @pytest.mark.parametrize("model,rank,rows,own", [
-    ("qwen2.5-0.5b", 0, 850, "qkv o gateup down"), ("qwen2.5-0.5b", 0, 4096, "gateup"),
-    ("qwen2.5-1.5b", 0, 57, "qkv o gateup down"), ("qwen2.5-1.5b", 0, 683, "gateup"),
-    ("qwen3-4b", 0, 57, "qkv o gateup down"), ("qwen3-4b", 0, 256, "down"),
-    ("qwen3-4b", 0, 683, ""), ("qwen2.5-7b", 0, 512, "down"), ("qwen2.5-7b", 0, 1024, ""),
+    ("qwen2.5-0.5b", 0, 4096, "qkv o gateup down"), ("qwen2.5-1.5b", 0, 57, "qkv o gateup down"),
+    ("qwen2.5-1.5b", 0, 683, "qkv gateup"), ("qwen3-4b", 0, 57, "qkv o gateup down"),
+    ("qwen3-4b", 0, 256, "qkv gateup down"), ("qwen3-4b", 0, 683, "qkv gateup"),
     ("qwen2.5-7b", 32, 12288, "qkv o gateup down")])
 def test_prompt_products_where_they_are_the_faster(model, rank, rows, own):
     """Sites of a prompt phase that our own products take, as measured."""
