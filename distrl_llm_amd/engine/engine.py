@@ -723,17 +723,18 @@ class Engine:
 
     def _skinny(self, n: int) -> bool:
         """Whether a decode step of n sequences runs on the skinny products:
-        every one of a layer's four fits, weights in bf16. Drawn against the
-        library's (a layer with its norms and activation, us: 32 rows 0.5B 42
-        against 59, 1.5B 73 against 71; 8 rows 4B 80 against 104), where it
-        still holds for weights that do not lie in tiles. From tiles the
-        streamed products are the faster at 17 to 32 rows of a small model
-        too: 64 tokens of 17, 24 and 32 sequences, 0.5B, 90, 91 and 92 ms
-        here, 74, 75 and 76 streamed."""
+        every one of a layer's four fits, weights in bf16. Against the library's
+        (a layer with its norms and activation, us: 32 rows 0.5B 42 against
+        59, 1.5B 73 against 71; 8 rows 4B 80 against 104), and from 17 rows on
+        against the streamed ones where weights lie in tiles: 64 tokens of
+        17, 24 and 32 sequences, ms, 0.5B 85.5, 86.6, 87.4 here, 69.6, 70.0,
+        71.1 streamed; 20 layers of 1024 and 4096 columns 56.4, 57.0, 57.2 and 54.1,
+        54.6, 55.0; 24 of 512 and 2048 54.0, 54.7, 55.5 and 54.8, 55.3, 55.7."""
         from ..ops.build import get_extension
         s, fits = self.spec, get_extension().skinny_gemm_takes
         return (self.dtype == torch.bfloat16
-                and (n <= 16 or (n <= 32 and s.hidden_size <= 1024))
+                and (n <= 16 or n <= 32 and s.hidden_size <= 1024
+                     and (s.hidden_size <= 512 or not self._streamed(n)))
                 and fits(n, s.q_size + 2 * s.kv_size, s.hidden_size)
                 and fits(n, s.hidden_size, s.q_size)
                 and fits(n, s.intermediate_size, s.hidden_size)

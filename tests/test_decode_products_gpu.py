@@ -91,6 +91,19 @@ def test_skinny_gemm_tiles(ext, M, N, K):
             assert torch.equal(ext.skinny_gemm(x, tiles, mode, tiles=True, kept=kept, **args), want)
 
 
+@pytest.mark.parametrize("model,n,tiled,skinny", [
+    ("qwen2.5-0.5b", 16, True, True), ("qwen2.5-0.5b", 17, True, False),
+    ("qwen2.5-0.5b", 32, False, True), ("qwen2.5-0.5b", 33, False, False),
+    ("small-qwen2", 32, True, True), ("qwen2.5-1.5b", 17, False, False)])
+def test_steps_on_skinny_products(model, n, tiled, skinny):
+    """The decode steps that take them, as measured."""
+    from types import SimpleNamespace
+    from distrl_llm_amd.engine import Engine
+    from distrl_llm_amd.models import get_spec
+    engine = SimpleNamespace(spec=get_spec(model), dtype=torch.bfloat16, _streamed=lambda n: tiled)
+    assert Engine._skinny(engine, n) == skinny
+
+
 @pytest.mark.parametrize("S", [1, 3, 4, 9])
 @pytest.mark.parametrize("rows,hidden,r", [(1, 64, 0), (5, 896, 32), (33, 4096, 64), (2, 4160, 128),
                                            (3, 8192, 0)])
