@@ -5,7 +5,7 @@ admission, n-candidate fan-out). For serving, concurrent requests should
 share one decode wave too: each ``generate`` call refreshes the fused
 decode weights and (on GPU) captures/replays a hipGraph sized to the
 batch, so 16 one-prompt calls cost ~16x one 16-prompt call. The reference
-has no serving surface at all (docs/ROADMAP.md #10); this is native.
+has no serving surface at all; this is native.
 
 One background thread owns the engine. ``submit`` blocks the calling
 (FastAPI threadpool) thread until its slice of the merged batch is done.

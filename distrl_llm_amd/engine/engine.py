@@ -446,7 +446,7 @@ class Engine:
             # prompts beyond the varlen kernel's score-tile cap: batch-pad
             # each prompt into its own row and run the first-party flash
             # kernel (ops/csrc/attention.hip) — native GQA, causal, no
-            # length cap, no aotriton/SDPA (docs/ROADMAP.md #9)
+            # length cap, no aotriton/SDPA
             from ..ops.build import get_extension
             ext = get_extension()
             B, Lmax = len(lens), max(lens)

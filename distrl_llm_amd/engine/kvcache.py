@@ -1,7 +1,7 @@
 """Paged KV cache pool + block allocator, sized for 288 GB HBM3E.
 
 Replaces the paged-KV machinery the reference inherits from vLLM
-(SURVEY.md §2.4-A: paged_attention, reshape_and_cache, block tables).
+(paged_attention, reshape_and_cache, block tables).
 Blocks are reference-counted so the n-candidate fan-out of one prompt
 shares the prompt's full KV blocks (prefill once per prompt instead of
 n times — the reference pays vLLM's prefix sharing here).

@@ -49,7 +49,7 @@ def spec_from_hf_config(path: str, name: Optional[str] = None) -> ModelSpec:
     if arch.startswith("Mistral") and sw is not None \
             and sw < cfg.get("max_position_embeddings", 32768):
         # pre-v0.3 Mistral uses sliding-window attention; this stack
-        # implements plain causal attention (all BASELINE.json families),
+        # implements plain causal attention (all of the registry's families),
         # so accepting the checkpoint would silently change semantics
         # beyond `sliding_window` tokens of context
         raise ValueError(

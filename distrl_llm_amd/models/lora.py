@@ -7,7 +7,7 @@ save_lora/load_lora adapter directory (reference distributed_actor.py:12,
 84-86,150). The on-disk format is the PEFT adapter directory —
 ``adapter_config.json`` + ``adapter_model.safetensors`` with
 ``base_model.model.model.layers.N.<module>.lora_{A,B}.weight`` keys — which
-is the north-star checkpoint format.
+is the reference's checkpoint format.
 """
 
 from __future__ import annotations
@@ -31,8 +31,7 @@ class LoRALinear(nn.Module):
     y = x W^T + b + scale * (x A^T) B^T, scale = alpha / r.
     A is kaiming-uniform initialized, B zeros (PEFT defaults), so a fresh
     adapter is an exact no-op — matching the reference's first-round
-    behavior of generating from base weights before any save
-    (SURVEY.md §2.6-3).
+    behavior of generating from base weights before any save.
     """
 
     def __init__(self, in_features: int, out_features: int, bias: bool,

@@ -173,9 +173,8 @@ class CausalLM(nn.Module):
 
     @torch.no_grad()
     def random_init(self, seed: int = 3407) -> "CausalLM":
-        """Deterministic random init (std 0.02) for synthetic benches
-        (random-init weights). The reference seeds LoRA with
-        random_state=3407 (reference helper.py:43)."""
+        """Deterministic random init (std 0.02) for synthetic benches. The
+        reference seeds LoRA with random_state=3407 (reference helper.py:43)."""
         dev = next(self.parameters()).device
         # generate on-device when possible (7B on CPU would take minutes);
         # deterministic for a given (seed, architecture, device type)
@@ -214,8 +213,7 @@ class CausalLM(nn.Module):
         keep_bf16=False (default for >16B models on GPU) FREES the bf16
         base image instead — every base projection (learner forward,
         prefill) then runs through the fused nf4 GEMM with on-the-fly
-        dequant for dX (SURVEY.md §2.4-B "learner nf4 GEMM" row; removes
-        the 65 GiB redundant image at 32B / the 145 GiB one at 72B that
+        dequant for dX (removes the 65 GiB redundant image at 32B / the 145 GiB one at 72B that
         OOM'd the 72B dual-role trial)."""
         if keep_bf16 is None:
             # auto: free only when the bf16 image threatens residency

@@ -1,11 +1,10 @@
 """Model architecture registry.
 
-Covers the model families the reference targets (
-Qwen2.5-{0.5B,7B,32B}, Llama-3-8B) plus tiny variants for CPU tests. Specs
+Covers the model families the reference targets
+(Qwen2.5-{0.5B,7B,32B}, Llama-3-8B) plus tiny variants for CPU tests. Specs
 are resolved from the model-name string the CLI passes (the reference
 resolves names through HF/Unsloth; offline we map known names to
-architectures and random-init weights: synthetic prompts /
-random-init weights).
+architectures and random-init weights).
 """
 
 from __future__ import annotations

@@ -3,7 +3,7 @@
 Built with torch.utils.cpp_extension (hipcc under PYTORCH_ROCM_ARCH=gfx950)
 into ``ops/_build`` INSIDE the repo, so the compiled .so travels to GPU
 boxes with the source snapshot. hipcc cross-compiles on CPU-only hosts;
-``__graft_entry__.build()`` calls :func:`build` as the driver's build check.
+``__graft_entry__.build()`` calls :func:`build` to check that everything compiles.
 """
 
 from __future__ import annotations

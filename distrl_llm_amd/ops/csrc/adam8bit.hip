@@ -1,6 +1,5 @@
-// Fused blockwise 8-bit Adam (the reference's bnb.optim.Adam8bit,
-// SURVEY.md §2.4-B): m/v states live as int8/uint8 with one fp32 absmax
-// per 256-element block; the whole dequant -> Adam -> requant -> param
+// Fused blockwise 8-bit Adam (the reference's bnb.optim.Adam8bit): m/v states
+// live as int8/uint8 with one fp32 absmax per 256-element block; the whole dequant -> Adam -> requant -> param
 // update is one kernel. One workgroup per state block (256 threads = 256
 // elements), absmax via block reduction.
 #include <torch/extension.h>

@@ -1,5 +1,5 @@
-// Paged KV-cache scatter (the reference's vLLM reshape_and_cache,
-// SURVEY.md §2.4-A): write the step's new K/V rows into their pool slots.
+// Paged KV-cache scatter (the reference's vLLM reshape_and_cache): write the
+// step's new K/V rows into their pool slots.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"

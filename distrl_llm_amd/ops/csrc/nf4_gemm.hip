@@ -1,7 +1,6 @@
 // Fused nf4-dequant + MFMA GEMM — the 4-bit weight path of both the
-// generation engine and the learner base projections (SURVEY.md §2.4:
-// "hand-written fused nf4-dequant+MFMA GEMM" north star; replaces
-// bitsandbytes kDequantizeBlockwise + cuBLAS in the reference's stack).
+// generation engine and the learner base projections (replaces bitsandbytes
+// kDequantizeBlockwise + cuBLAS in the reference's stack).
 //
 //   y[M,N] = x[M,K] @ dequant(W4)[N,K]^T (+ bias) (+ u[M,r] @ Bs[N,r]^T)
 //

@@ -633,8 +633,7 @@ torch::Tensor paged_attention_decode(torch::Tensor q, torch::Tensor kcache,
 // of the tile — lane-per-kv-token scoring against the LDS-staged q tile
 // (with causal masking), per-row softmax, PV through LDS V tiles.
 // K/V are the flat pre-RoPE'd prefill tensors (no paging needed here).
-// Completes the "prefill + decode as HIP kernels" surface (BASELINE.json
-// north star); replaces the torch-SDPA library call in the engine.
+// Replaces the torch-SDPA library call in the engine.
 namespace {
 
 // the legacy prefill kernel keeps the original 32-token V tile: the

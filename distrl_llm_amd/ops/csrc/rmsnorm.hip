@@ -1,6 +1,6 @@
 // RMSNorm forward + backward (dx only — norm weights are frozen in this
 // framework: only LoRA trains). Replaces the fused RMSNorm the reference
-// gets from vLLM/Unsloth (SURVEY.md §2.4 A+B).
+// gets from vLLM/Unsloth.
 //
 // Memory-bound: explicit bf16x8 (16 B/lane) vector loads — hipcc does not
 // auto-vectorize scalar bf16 loads (guide G13) — fp32 accumulation, one

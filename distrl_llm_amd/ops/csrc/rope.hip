@@ -1,6 +1,6 @@
 // Fused in-place RoPE for the generation path (rotate_half / neox
 // convention, matching HF Qwen2/Llama). Replaces vLLM's pos_encoding
-// kernels (SURVEY.md §2.4-A). cos/sin computed once per token into LDS and
+// kernels. cos/sin computed once per token into LDS and
 // reused across all q + kv heads.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>

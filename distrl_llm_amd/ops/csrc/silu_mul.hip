@@ -1,5 +1,5 @@
 // Fused SiLU-and-mul forward/backward (the SwiGLU activation the reference
-// gets from vLLM activation kernels / Unsloth Triton — SURVEY.md §2.4).
+// gets from vLLM activation kernels / Unsloth Triton).
 // Memory-bound elementwise: bf16x8 vector loads, grid-stride loop.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>

@@ -180,9 +180,8 @@ def sample_tokens(logits: torch.Tensor, temperature: float, top_p: float,
 # ------------------------------------------------- training RoPE fwd/bwd
 
 class _RopeTrainFn(torch.autograd.Function):
-    """First-party RoPE for the TRAINING path (SURVEY.md §2.4-B "RoPE
-    fwd/bwd" row): forward rotates q/k with the fused HIP kernel
-    (ops/csrc/rope.hip, already numerics-tested on the inference path);
+    """First-party RoPE for the TRAINING path: forward rotates q/k with the
+    fused HIP kernel (ops/csrc/rope.hip, already numerics-tested on the inference path);
     backward is the SAME kernel with NEGATED frequencies — the gradient
     of a rotation is the transposed rotation, and R(-theta) = R(theta)^T
     exactly (sin is odd, cos even). Formula verified on CPU against
@@ -229,9 +228,8 @@ def rope_training(q, k, positions, inv_freq):
 
 class _NF4LinearFn(torch.autograd.Function):
     """Base projection through the fused nf4-dequant MFMA GEMM when the
-    bf16 base image has been freed (LoRALinear.free_base_to_nf4_; big-
-    model learner path — SURVEY.md §2.4-B "learner nf4 GEMM" row). The
-    base is frozen, so backward only needs dX = dY @ W with W dequanted
+    bf16 base image has been freed (LoRALinear.free_base_to_nf4_; the
+    learner of big models). The base is frozen, so backward only needs dX = dY @ W with W dequanted
     on the fly (transient, never resident)."""
 
     @staticmethod
@@ -279,8 +277,8 @@ class _LogprobLossFn(torch.autograd.Function):
     """Fused per-token log-softmax + gather + masked PG/GRPO loss.
 
     forward returns the scalar loss; backward emits dlogits directly
-    without materializing a (B, T, V) log-prob tensor (SURVEY.md §2.4-B
-    north star). loss = -mean_b( (sum_t logp*mask / sum_t mask) * R_b ).
+    without materializing a (B, T, V) log-prob tensor.
+    loss = -mean_b( (sum_t logp*mask / sum_t mask) * R_b ).
     """
 
     @staticmethod

@@ -1,12 +1,11 @@
 """Pure-PyTorch reference implementations of every custom op.
 
 These are the numerics ground truth the HIP kernels are tested against
-("Numerics tests for a HIP kernel compare it against a plain
-PyTorch fp32 reference of the same op") and the CPU execution path for the
-gloo plumbing config.
+(a kernel is compared with a plain PyTorch fp32 reference of the same op) and
+the CPU execution path, gloo ranks among it.
 
 Op inventory mirrors the implicit kernel surface of the reference's
-dependency stack (SURVEY.md §2.4): RMSNorm, RoPE, SiLU-and-mul, KV-cache
+dependency stack: RMSNorm, RoPE, SiLU-and-mul, KV-cache
 scatter, paged attention (prefill + decode), fused sampling, nf4
 quant/dequant, and the fused log-prob + advantage loss.
 """
@@ -222,8 +221,8 @@ def pg_loss(log_probs: torch.Tensor, mask: torch.Tensor,
             rewards: torch.Tensor) -> torch.Tensor:
     """-mean_b( (sum_t logp*mask / sum_t mask) * R_b )  — the reference PG
     loss (reference distributed_actor.py:375). GRPO's surrogate
-    exp(logp - logp.detach()) has value 1 and the identical gradient
-    (SURVEY.md §2.6-6), so one implementation serves both."""
+    exp(logp - logp.detach()) has value 1 and the identical gradient,
+    so one implementation serves both."""
     m = mask.to(log_probs.dtype)
     seq_mean = (log_probs * m).sum(-1) / m.sum(-1).clamp_min(1.0)
     return -(seq_mean * rewards.to(log_probs.dtype)).mean()

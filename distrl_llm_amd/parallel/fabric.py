@@ -1,6 +1,6 @@
 """Process fabric: one process per GPU, torch.distributed over RCCL/xGMI.
 
-Native replacement for the reference's Ray transport (SURVEY.md §2.3: Ray
+Native replacement for the reference's Ray transport (Ray
 object store + shared-filesystem adapter sync, zero collectives). Here:
 
 - one ``torch.distributed`` world spans all actor + learner ranks
@@ -14,7 +14,7 @@ object store + shared-filesystem adapter sync, zero collectives). Here:
   save_lora/load_lora disk round-trip, distributed_actor.py:84-86,150).
   Payloads are tiny (~40-80 MB), so single-shot latency-bound collectives
   are the right shape for xGMI's 7x153 GB/s point-to-point links — not
-  multi-hop rings (SURVEY.md §2.3).
+  multi-hop rings.
 
 Rank layout matches the reference's GPU assignment (distributed_actor.py:
 535-537): ranks [0, num_actors) are actors, [num_actors, world) learners.

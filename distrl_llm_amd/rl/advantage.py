@@ -7,7 +7,7 @@ whitened summed reward ``(R - mean) / (std + 1e-8)`` over all n candidates
 of a group, computed BEFORE top-k filtering, and the top-k filter keeps the
 ``topk`` highest-total-reward candidates per group via argsort.
 
-Deviation (documented, SURVEY.md §2.6-2): the reference's multi-learner PG
+Deviation (documented): the reference's multi-learner PG
 path drops the baseline when flattening (merge_candidates loses the
 "baselines" key, distributed_trainer.py:221-230), training PG on raw summed
 rewards. Here the PG baseline is subtracted before any flattening, so

@@ -4,8 +4,7 @@ Mirrors the reference's data layer (reference helper.py:3-23,
 train_distributed.py:38-48): R1-style system prompt, chat templating with a
 generation prompt, and the MATH answer->solution column remap. Because this
 environment has no network, a deterministic synthetic MATH-shaped prompt
-generator is provided for benches and tests (BASELINE.json: synthetic
-prompts / random-init weights).
+generator is provided for benches and tests.
 """
 
 from __future__ import annotations

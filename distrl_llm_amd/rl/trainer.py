@@ -5,7 +5,7 @@ Every rank runs the same program (one process per GPU). Rank 0 drives the
 control flow by broadcasting (command, payload) tuples over the gloo
 control plane; all ranks execute each command's collective sequence in
 lockstep. This replaces the reference's Ray remote-call surface
-(SURVEY.md §1 L4->L3: generate / train / compute_gradients /
+(generate / train / compute_gradients /
 apply_merged_gradients / save_adapter / save_checkpoint).
 
 Round structure matches reference distributed_trainer.py:232-382:
@@ -14,7 +14,7 @@ reference README:19), rank-0 reward + advantage + top-k math, learner
 update (gradient all-reduce over the learner subgroup instead of CPU
 gather to learner 0), weight sync (RCCL broadcast instead of adapter disk
 round-trip, plus the adapter save kept for checkpoint parity), metrics
-with the reference's exact key set (SURVEY.md §5.5), periodic eval
+with the reference's exact key set, periodic eval
 (pass@1 / BoN — distributed_trainer.py:384-416) and checkpoint cadence.
 """
 
@@ -80,7 +80,7 @@ class Trainer:
     def _cmd(self, name: str, payload=None):
         """Rank 0: broadcast a command then execute it locally. Each
         command carries a monotonically increasing sequence id — the
-        explicit round handshake SURVEY.md §5.2 asks for in place of the
+        explicit round handshake in place of the
         reference's implicit adapter-file ordering."""
         assert self.fabric.rank == 0
         self._cmd_seq = getattr(self, "_cmd_seq", 0) + 1
@@ -129,7 +129,7 @@ class Trainer:
 
     def _save_checkpoint_handler(self, payload):
         """Full resumable checkpoint (extension over the reference's
-        adapter-only save, distributed_trainer.py:377-380 / SURVEY §5.4):
+        adapter-only save, distributed_trainer.py:377-380):
         PEFT adapter + rank-0 trainer counters/dataset-RNG + lead-learner
         optimizer state + per-rank engine RNG stream. With the same world
         size, ``--resume <dir>`` continues the run bit-identically."""
@@ -169,7 +169,7 @@ class Trainer:
 
         payload: (batch_dict, sp_dict). Returns (candidates, duration) on
         rank 0, None elsewhere. Candidate dicts use the reference wire
-        format (SURVEY.md §1): answers / token_lengths /
+        format: answers / token_lengths /
         solution / problem each replicated n-per-prompt.
         """
         batch, sp_dict = payload

@@ -1,7 +1,7 @@
 """Minimal OpenAI-style serving surface over the generation engine.
 
-The reference has no serving API (Engine use is in-process only —
-SURVEY.md §2.3 / docs/ROADMAP.md #10); this is a native extension so the
+The reference has no serving API (Engine use is in-process only — its
+library calls); this is a native extension so the
 paged-KV engine can also be used as a standalone completion server:
 
     python -m distrl_llm_amd.serve --model qwen2.5-7b --port 8000

@@ -7,13 +7,12 @@ to max_new_tokens — distributed_actor.py:215-239), micro-batched gradient
 accumulation over train_batch_size, bf16 autocast on GPU, the PG loss
 ``-mean((sum logp*mask / sum mask) * R)`` (distributed_actor.py:375) — which
 is also the exact GRPO gradient since the reference's one-step on-policy
-surrogate ``exp(logp - logp.detach())`` is identically 1 (SURVEY.md
-§2.6-6) — and 8-bit Adam.
+surrogate ``exp(logp - logp.detach())`` is identically 1 — and 8-bit Adam.
 
 Deviations (documented):
 - the degenerate-batch skip implements the reference's INTENT (skip when
   all advantages are zero), not its buggy ``batch_rewards.all() == 0``
-  form (SURVEY.md §2.6-4);
+  form;
 - log-probs + loss run through the fused HIP kernel emitting dlogits
   directly instead of the reference's per-row log_softmax+gather loop
   (distributed_actor.py:253-260);
@@ -70,7 +69,7 @@ class Learner:
         (prompt keeps its first max_prompt_tokens, answers their first
         max_new_tokens — distributed_actor.py:217-229) but packs instead of
         left-padding, so causal attention needs no mask (flash-capable) and
-        trailing pad compute shrinks to the batch max (SURVEY.md §2.6-8).
+        trailing pad compute shrinks to the batch max.
         """
         P, A = self.max_prompt_tokens, self.max_new_tokens
         B = len(problems)

@@ -1,6 +1,6 @@
 """Metrics logging: wandb when importable, JSONL fallback with the same keys.
 
-The key set matches the reference exactly (SURVEY.md §5.5; reference
+The key set matches the reference exactly (reference
 distributed_trainer.py:348-366,412-415): loss, mean_format_reward,
 mean_accuracy_reward, min/max_accuracy_reward, mean_token_length, episode,
 total_batch_steps, total_samples_processed, timing/update_duration,

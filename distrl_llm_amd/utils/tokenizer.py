@@ -3,7 +3,7 @@
 The reference delegates tokenization to Unsloth/HF
 (reference train_distributed.py:5,46; distributed_actor.py:217-229). Here:
 a local HF tokenizer is used when a tokenizer directory is available;
-otherwise (offline / synthetic-bench environments) a
+otherwise (offline, synthetic benches) a
 deterministic byte-level tokenizer with the model's vocab size stands in.
 
 Encoding: when the vocab is large enough, text is encoded two UTF-8 bytes

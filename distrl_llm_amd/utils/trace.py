@@ -1,4 +1,4 @@
-"""rocprof-compatible phase ranges (SURVEY.md §5.1 build note).
+"""rocprof-compatible phase ranges.
 
 ``torch.cuda.nvtx`` maps to roctx on ROCm builds, so these ranges show up
 in ``rocprofv3 --marker-trace`` (and rocprof GUI timelines) and let a

@@ -52,7 +52,7 @@ def test_process_candidates_grpo():
 def test_process_candidates_pg_baseline_subtracted():
     cands, _ = process_candidates(_candidates(), "pg", topk=4)
     r = cands[0]["rewards"][0]
-    # PG rewards are baselined before merging (deviation fix)
+    # PG rewards are baselined before merging (a deviation)
     assert abs(np.sum(r)) < 1e-9
 
 

@@ -1,8 +1,7 @@
 """The bench.py driver contract, exercised end-to-end on CPU:
 `python bench.py --cpu --tiny --steps 1 --warmup 1` must run the real
 SPMD bench loop (gloo world of 1) and print exactly one JSON line with
-every field the driver parses. Guards the round-end BENCH/SCALE runs
-against contract drift."""
+every field of its contract."""
 
 import json
 import os

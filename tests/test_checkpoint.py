@@ -1,7 +1,7 @@
 """Checkpoint/resume: full trainer-state save (adapter + optimizer +
 counters + dataset RNG + per-rank engine RNG) and bit-identical
 continuation — an extension over the reference's adapter-only
-save_checkpoint (reference distributed_trainer.py:377-380, SURVEY §5.4).
+save_checkpoint (reference distributed_trainer.py:377-380).
 """
 
 import os

@@ -90,7 +90,7 @@ def test_native_extension_is_loaded():
 
 
 def test_llama3_8b_bf16_path():
-    """BASELINE config 4 readiness: Llama-3-8B bf16 (non-quantized) decode
+    """Llama-3-8B bf16 (non-quantized) decode
     + PG learner micro-step on the same engine machinery (no qkv bias,
     GQA 4:1, vocab 128256)."""
     from distrl_llm_amd.config import EngineConfig, SamplingParams
@@ -147,7 +147,7 @@ def test_graph_vs_eager_decode_identical(setup):
 def test_session_cache_vs_fresh_identical(setup):
     """CachedDecodeSession (DISTRL_GRAPH_CACHE=1: padded lanes, reused
     buffers, hipGraph reused across waves) must produce exactly the same
-    greedy tokens as per-wave fresh sessions (docs/ROADMAP.md #4)."""
+    greedy tokens as per-wave fresh sessions."""
     import os
     model, _ = setup
     from distrl_llm_amd.config import EngineConfig, SamplingParams
@@ -174,7 +174,7 @@ def test_session_cache_vs_fresh_identical(setup):
 def test_long_prompt_prefill_no_cap(setup):
     """Prompts beyond the varlen prefill kernel's ~2200-token score-tile
     cap route through the first-party flash kernel (no SDPA/aotriton, no
-    length cap — docs/ROADMAP.md #9)."""
+    length cap)."""
     model, _ = setup
     from distrl_llm_amd.config import EngineConfig, SamplingParams
     from distrl_llm_amd.engine import Engine
@@ -192,7 +192,7 @@ def test_long_prompt_prefill_no_cap(setup):
 def test_nf4_freed_base_learner_parity():
     """free_base_to_nf4_ (bf16 image dropped, fused nf4 GEMM forward +
     on-the-fly dequant dX): forward and LoRA grads must match the
-    materialized nf4-image path (SURVEY.md §2.4-B learner nf4 GEMM)."""
+    materialized nf4-image path."""
     from distrl_llm_amd.models import CausalLM, get_spec
     spec = get_spec("small-qwen2")
     dev = torch.device("cuda:0")

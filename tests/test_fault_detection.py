@@ -1,8 +1,7 @@
 """Fail-fast fault detection: a dead rank must surface as an error on
 the surviving ranks within the fabric timeout (the reference's only
-fault handling is 240 s ray.get timeouts that crash the run — SURVEY
-§5.3; here the process-group timeout plays that role and is
-configurable via config["fabric_timeout_s"])."""
+fault handling is 240 s ray.get timeouts that crash the run; here
+the process-group timeout plays that role and is configurable via config["fabric_timeout_s"])."""
 
 import os
 import time

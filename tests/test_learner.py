@@ -33,9 +33,8 @@ def test_logprob_loss_matches_reference():
 
 
 def test_grpo_surrogate_equals_pg_gradient():
-    """exp(logp - logp.detach()) == 1 with identical gradient
-     — verify our shared implementation equals the GRPO
-    surrogate form."""
+    """exp(logp - logp.detach()) == 1 with identical gradient —
+    verify our shared implementation equals the GRPO surrogate form."""
     torch.manual_seed(1)
     B, T, V = 2, 5, 17
     logits = torch.randn(B, T, V, requires_grad=True)

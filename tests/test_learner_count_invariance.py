@@ -2,7 +2,7 @@
 1 learner (gradient accumulation) and on 2 learners (even split +
 all-reduce mean) must produce the SAME adapter — the gradient estimator
 is the mean over samples either way. This pins the distributed-update
-math the 8-GPU run relies on (SURVEY §2.2 DP-over-learners)."""
+math the 8-GPU run relies on."""
 
 import os
 

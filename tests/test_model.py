@@ -27,7 +27,7 @@ def test_forward_shapes(tiny_model):
 
 def test_fresh_lora_is_noop(tiny_model):
     """B zeros ==> adapter contributes nothing (reference first-round
-    behavior, SURVEY §2.6-3)."""
+    behavior)."""
     ids = torch.randint(0, tiny_model.spec.vocab_size, (1, 8))
     logits = tiny_model(ids)
     # disable lora by zeroing A as well; with B=0 output must be unchanged
@@ -124,8 +124,7 @@ def test_quantize_model_attaches_sidecar():
 
 def test_cli_warm_start_adapter(tmp_path):
     """--load_adapter loads a saved PEFT adapter into a fresh worker's
-    model (warm-start extension; the reference has no resume path,
-    SURVEY §5.4)."""
+    model (warm-start extension; the reference has no resume path)."""
     from distrl_llm_amd.models.lora import load_adapter, lora_state_dict, save_adapter
     spec = get_spec("tiny-qwen2")
     m1 = CausalLM(spec, lora_r=4, lora_alpha=8, dtype=torch.float32).random_init(0)

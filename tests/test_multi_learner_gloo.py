@@ -1,7 +1,7 @@
 """Multi-learner correctness: 1 actor + 2 learners over gloo. The gradient
 all-reduce + replicated optimizer must keep every learner's adapter
 bit-identical (replacing the reference's CPU gradient staging through
-learner 0, SURVEY.md §2.2), and the round weight broadcast must land the
+learner 0), and the round weight broadcast must land the
 same adapter on the actor."""
 
 import os

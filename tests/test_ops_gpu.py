@@ -1,5 +1,5 @@
 """Kernel numerics: each gfx950 HIP kernel vs the plain PyTorch fp32
-reference (SURVEY.md §4 test strategy)."""
+reference."""
 
 import math
 
@@ -384,7 +384,7 @@ def test_prefill_attention(ext, D, H, KV, lens):
 ])
 def test_flash_attention_fwd_bwd(ext, B, Hq, Hkv, T, D):
     """First-party flash attention vs fp32 torch reference: forward and all
-    three input grads (SURVEY.md §2.4-B training attention row)."""
+    three input grads."""
     torch.manual_seed(0)
     dev = torch.device("cuda:0")
     scale = D ** -0.5
@@ -425,8 +425,7 @@ def test_flash_attention_fwd_bwd(ext, B, Hq, Hkv, T, D):
 def test_rope_training_fwd_bwd(ext):
     """Training RoPE fwd/bwd (ops/functional.rope_training): the fused
     HIP kernel forward + negated-frequency backward vs fp32 torch
-    autograd (SURVEY.md §2.4-B RoPE fwd/bwd row; backward formula proven
-    in test_autograd_formulas)."""
+    autograd."""
     from distrl_llm_amd.ops import functional as OF
     from distrl_llm_amd.ops import reference as R
     torch.manual_seed(0)

@@ -1,5 +1,5 @@
 """Serving surface: OpenAI-style /v1/completions over the engine (native
-extension — the reference is in-process only, docs/ROADMAP.md #10)."""
+extension — the reference is in-process only)."""
 
 import pytest
 import torch

@@ -1,5 +1,5 @@
-"""Decode-session graph cache (DISTRL_GRAPH_CACHE=1, default off —
-docs/ROADMAP.md #4): cached state buffers + wave padding must decode
+"""Decode-session graph cache (DISTRL_GRAPH_CACHE=1, default off):
+cached state buffers + wave padding must decode
 identically to the per-wave session path, reuse state across waves, and
 never leak pool blocks (including the padding lanes' scratch block).
 On GPU the same machinery also reuses the captured hipGraph; that

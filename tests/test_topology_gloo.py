@@ -1,7 +1,7 @@
 """Mixed-topology control-plane test: 2 actors + 2 learners over gloo on
 CPU — the fullest per-node shape (actor chunking + multi-learner
-all-reduce + broadcast in one world), the same structure the driver's
-8-GPU run exercises. Verifies all four replicas converge to one adapter
+all-reduce + broadcast in one world), the structure of
+a whole node. Verifies all four replicas converge to one adapter
 and the round metrics account for every prompt exactly once."""
 
 import json

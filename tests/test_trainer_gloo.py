@@ -1,5 +1,5 @@
-"""End-to-end control-plane test: 1 actor + 1 learner over gloo on CPU —
-BASELINE.json config 1 (plumbing, no GPU). Exercises chunking, generate
+"""End-to-end control-plane test: 1 actor + 1 learner over gloo on CPU
+(plumbing, no GPU). Exercises chunking, generate
 fan-out, rewards, advantage, top-k, learner update, weight broadcast,
 adapter save, eval and metrics."""
 

@@ -1,12 +1,12 @@
 #!/usr/bin/env python3
 """Distributed RL fine-tuning CLI — flag-for-flag with the reference
-(reference train_distributed.py:11-35; SURVEY.md §5.6), running on the
+(reference train_distributed.py:11-35), running on the
 MI355X-native engine: one spawned process per GPU over RCCL/xGMI (gloo on
 CPU) instead of Ray actors.
 
 Offline behavior: if the HF dataset cannot be loaded (no network), a
-deterministic synthetic MATH-shaped dataset is used (
-synthetic prompts / random-init weights) — pass --synthetic_dataset N to
+deterministic synthetic MATH-shaped dataset is used (synthetic
+prompts / random-init weights) — pass --synthetic_dataset N to
 force it.
 """
 
