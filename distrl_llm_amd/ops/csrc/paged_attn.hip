@@ -91,14 +91,11 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
   const int* bt = block_tables + (int64_t)seq * max_nb;
   const int c0 = z * slice_len;
   auto block_of = [&](int t) { return bs_shift >= 0 ? t >> bs_shift : t / block_size; };
-  // the page of this lane's token l % 32 of a chunk, whether there is one or not
-  auto page_of = [&](int t0) {
-    return max_nb > 0 ? bt[min(block_of(t0 + (l & 31)), max_nb - 1)] : 0;
-  };
   // What a workgroup needs first is on its way at once: the length, its pages, and
   // below what its queries are made of. One behind the other they are a microsecond each.
   int t0 = c0 + wave * CHUNK;
-  int page = page_of(t0);
+  // the page of this lane's token l % 32 of the first chunk, whether there is one or not
+  int page = max_nb > 0 ? bt[min(block_of(t0 + (l & 31)), max_nb - 1)] : 0;
   const int len = ctx_lens[seq];
   // no further than the block table reaches
   const int c1 = min(len, min(c0 + slice_len, max_nb * block_size));
@@ -123,10 +120,9 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
 
   const int row_elems = KV * D;
   bf16v8 kf[NL], vf[NL];
-  auto load = [&](int t0) {             // page: of this chunk
-    const int t = min(t0 + (l & 31), c1 - 1);           // past the end: weight zero
-    // of the pool, of this lane's token
-    const int row = __shfl(page, t - t0, WAVE) * block_size + (t - block_of(t) * block_size);
+  auto token = [&](int t0) { return min(t0 + (l & 31), c1 - 1); };     // past the end: weight zero
+  auto load = [&](int page, int t0) {   // page: of this lane's token
+    const int t = token(t0), row = page * block_size + (t - block_of(t) * block_size);
     #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int64_t at = (int64_t)__shfl(row, i * RPL + l / LPR, WAVE) * row_elems + kv * D +
@@ -138,8 +134,11 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
 
   auto begin = [&] {
     if (t0 < c1) {
-      load(t0);
-      page = page_of(t0 + NW * CHUNK);
+      load(__shfl(page, token(t0) - t0, WAVE), t0);
+      // With the length known a chunk's pages are looked up where its rows end: lanes
+      // that trade them for every chunk stand in front of its rows (32 of 300..1500,
+      // 40/8 heads 26.4 us, 26.05 so; 300 of 60..400, 14/2 heads 10.1 and 10.0).
+      page = bt[block_of(token(t0 + NW * CHUNK))];
     }
   };
   bf16v8 qf[KS];
@@ -296,8 +295,8 @@ void paged_decode_kernel(const __hip_bfloat16* __restrict__ q,      // rows of q
       *reinterpret_cast<bf16v8*>(tile + v_off<D>(r, c)) = vf[i];
     }
     if (more) {
-      load(t0 + NW * CHUNK);
-      page = page_of(t0 + 2 * NW * CHUNK);
+      load(page, t0 + NW * CHUNK);
+      page = bt[block_of(token(t0 + 2 * NW * CHUNK))];
     }
     __builtin_amdgcn_wave_barrier();
     f32x4 st[2];
