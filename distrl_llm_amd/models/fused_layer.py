@@ -6,13 +6,14 @@ The module-by-module layer launches ~200 kernels forward and backward, most
 of them elementwise passes between the products (residual adds, adapter
 scaling, gradient sums of projections that share an input, rotary steps,
 head transposes), and short micro-batches are bound by launching them. A half
-is 7 launches forward and 9 or 10 backward here, prepared in native code
-(ops/csrc/adapted_layer.cpp): products of our own (ops/csrc/product.hip) take
-adapters as more of their projections' K, residuals, the activation and its
-gradient with them. The library's products, where many rows meet wide weights,
-have W laid out beside B for it; at ranks that ours don't take large weights that
-few rows meet are taken as they lie, their adapters joined to fp32 products. Adapter gradients are one
-launch and its sum (ops/csrc/adapter_grads.hip).
+is 7 launches forward and 10 or 11 backward (attention) or 5 and 7 (feed-forward)
+here, prepared in native code (ops/csrc/adapted_layer.cpp): products of our own
+(ops/csrc/product.hip) take adapters as more of their projections' K, residuals,
+the activation and its gradient with them. The library's products, where many
+rows meet wide weights, have W laid out beside B for it; at ranks that ours don't
+take large weights that few rows meet are taken as they lie, their adapters
+joined to fp32 products. Adapter gradients are one launch and its sum
+(ops/csrc/adapter_grads.hip).
 """
 
 from __future__ import annotations

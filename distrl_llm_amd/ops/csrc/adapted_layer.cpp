@@ -11,7 +11,8 @@
 //
 // Native because short micro-batches wait for the host: prepared in Python a pass of
 // the 0.5B model over three short samples took 25.0 ms, with the library's products
-// (17 us of the host each) and what they need beside them 16.0, now 11.8.
+// (17 us of the host each) and what they need beside them 17.8, now 15.6 (medians of
+// processes in turn; single ones now 11.8 to 18.7, of which 8.5 are the kernels').
 #include "adapted.h"
 #include "product.h"
 

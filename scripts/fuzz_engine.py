@@ -4,11 +4,11 @@ prefixes), EOS, n-fan-out, pool pressure, streaming callbacks and
 session-vs-eager paths, each trial cross-checked against naive
 full-recompute greedy decoding.
 
-Round-1 campaigns (CPU, tiny-qwen2): 400 eager + 300 forced-session +
+Campaigns on the CPU (tiny-qwen2): 400 eager + 300 forced-session +
 500 mixed trials, zero failures. Re-run after any engine/kernel change:
 
     python scripts/fuzz_engine.py --trials 200
-    gpurun -- 'python scripts/fuzz_engine.py --trials 50 --model small-qwen2'
+    python scripts/fuzz_engine.py --trials 50 --model small-qwen2     # on a GPU
 
 On GPU (bf16) near-argmax ties can flip greedy tokens vs the fp32 naive
 path; mismatches are reported with their divergence step so real bugs
