@@ -24,6 +24,7 @@ from __future__ import annotations
 
 from typing import List, Optional, Sequence
 
+import numpy as np
 import torch
 
 from ..models.lora import trainable_parameters
@@ -116,12 +117,19 @@ class Learner:
         dev, n_ans = self.device, torch.tensor(n_ans)
         ids = torch.tensor([t for p, a in enc for t in p + a]).to(dev)
         targets = torch.tensor([t for _, a in enc for t in a]).to(dev)
-        share = (-loss_scale / (n_ans * len(enc))).repeat_interleave(n_ans)
-        sample = torch.arange(len(enc)).repeat_interleave(n_ans)
+        # Numpy repeats: torch's wakes its threads for any size, which on a host
+        # that has fewer cores than it shows took 4 ms a call. What the loss needs
+        # is on the GPU before the layers are launched: a copy behind them waits
+        # for all of them (three short samples through the 0.5B model 15.4 to 19.6
+        # ms, 12.0 with numpy, 11.1 so).
+        share = torch.from_numpy(
+            (-loss_scale / (n_ans * len(enc))).numpy().repeat(n_ans.numpy()))
+        sample = torch.from_numpy(np.arange(len(enc)).repeat(n_ans.numpy()))
+        at = torch.cat(at).to(dev)
+        weights = rewards[sample.to(dev)] * share.to(dev)
         hidden = self.model.forward_rows(ids, [n for n in lens if n])
-        logits = self.model.logits(hidden.index_select(0, torch.cat(at).to(dev)))
-        return OF.logprob_rows(logits, targets,
-                               rewards[sample.to(dev)] * share.to(dev))
+        logits = self.model.logits(hidden.index_select(0, at))
+        return OF.logprob_rows(logits, targets, weights)
 
     def _micro_loss(self, problems, answers, rewards: torch.Tensor,
                     loss_scale: float) -> torch.Tensor:
