@@ -179,6 +179,204 @@ void skinny_gemm_kernel(const __hip_bfloat16* __restrict__ x, const __hip_bfloat
   }
 }
 
+// The same for M <= 8 rows of x. Such an x fills half of a product's 16
+// columns, and loads that repeat it (or 8 rows of W) cost as much of a CU's 64 B/clk as
+// others do, which bound the small products. Here a product's rows are 8 of W at two
+// steps of K, and its columns 8 of x at the same two: the blocks on the diagonal are the
+// two steps' sums, the others are left. Every lane loads something of its own, whole
+// cache lines of either, and the norm's work is halved; its squares are a product too.
+// Bound by the launch (1.7 us of a captured chain), the way to memory and back, and W.
+// 8 rows and cold weights in a captured chain, us, before -> now: 1152 x 896 with the norm
+// 3.95 -> 3.4, 896 x 896 3.5 -> 3.1, gate and up of 4864 x 896 8.4 -> 6.6, 896 x 4864 7.1 ->
+// 6.1; 2048 x 1536 5.2 -> 4.2, 1536 x 1536 4.6 -> 3.7, 8960 x 1536 13.5 -> 12.5, 1536 x 8960
+// 13.2 -> 11.4; 6144 x 2560 12.9 -> 10.2, 2560 x 4096 9.5 -> 7.5, 9728 x 2560 23.1 -> 19.5,
+// 2560 x 9728 17.9 -> 14.3; 3584 x 18944 32.7 -> 26.7, 18944 x 3584 55 -> 47.
+struct PairArgs {
+  const __hip_bfloat16 *x, *w, *bias, *res, *norm_w, *u, *ub;
+  __hip_bfloat16* y;
+  int M, N, K, R;
+  float eps;
+};
+
+// NG groups of 8 rows of W a workgroup, U double steps of K a wave has in flight
+template <int NG, int KW, int U, int MODE, int W>
+__global__ __launch_bounds__(KW * 64)
+void skinny_pair_kernel(const PairArgs p) {
+  constexpr bool NORM = MODE != RESIDUAL;
+  constexpr int ACC = MODE == GLU ? 2 : 1, OUT = NG / ACC, TR = OUT * 8;
+  constexpr int QUADS = OUT * 16, PARTS = WAVE / QUADS;   // four columns of a row; lanes that share one
+  __shared__ f32x4 red[KW][NG][32];
+  __shared__ float squares[NORM ? KW * 16 : 1];
+  const int M = p.M, N = p.N, K = p.K, R = p.R;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l = threadIdx.x & 63, g = l >> 4, r8 = l & 7, second = (l >> 3) & 1;
+  const int n0 = blockIdx.x * TR, ko = second * 32 + g * 8;
+  const int steps = K / 64, s0 = wave * steps / KW, s1 = (wave + 1) * steps / KW;
+
+  const __hip_bfloat16* wp[NG];
+  #pragma unroll
+  for (int a = 0; a < NG; ++a) {
+    const int n = n0 + a % OUT * 8 + r8, t = MODE == GLU ? n / 16 * 32 + a / OUT * 16 + n % 16 : n;
+    wp[a] = W == ROWS ? p.w + (int64_t)(a / OUT * N + n) * K + ko
+                      : p.w + (int64_t)(t >> 5) * K * 32 + (ko >> 4) * 512 + ((ko >> 3) & 1) * 256 +
+                            (t & 31) * 8;
+  }
+  const __hip_bfloat16* xp = p.x + (int64_t)min(r8, M - 1) * K + ko;    // spare rows repeat
+  f32x4 acc[NG];
+  #pragma unroll
+  for (int a = 0; a < NG; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 sq = f32x4{0.f, 0.f, 0.f, 0.f};     // x x^T: rows' squares on its diagonal
+  // of this lane's output, for the end
+  const int m = l & 7, n = n0 + (l % QUADS) / 16 * 8 + ((l >> 3) & 1) * 4;
+  const int64_t at = (int64_t)min(m, M - 1) * N + n;
+  bf16v4 add = {};
+  if (wave == 0) {
+    if (MODE == RESIDUAL) add = *reinterpret_cast<const bf16v4*>(p.res + at);
+    else if (MODE == PLAIN && p.bias) add = *reinterpret_cast<const bf16v4*>(p.bias + n);
+  }
+
+  for (int s = s0; s < s1; s += U) {
+    bf16v8 wf[U][NG], xf[U], nf[U];
+    #pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int k = min(s + i, s1 - 1) * 64;              // past the end: the last again
+      #pragma unroll
+      for (int a = 0; a < NG; ++a) {
+        const bf16v8* from = reinterpret_cast<const bf16v8*>(wp[a] + k * (W == ROWS ? 1 : 32));
+        wf[i][a] = W == TILES ? __builtin_nontemporal_load(from) : *from;
+      }
+      xf[i] = *reinterpret_cast<const bf16v8*>(xp + k);
+      if (NORM) nf[i] = *reinterpret_cast<const bf16v8*>(p.norm_w + ko + k);
+    }
+    #pragma unroll
+    for (int i = 0; i < U; ++i)
+      if (s + i < s1) {                                   // wave-uniform
+        if (NORM) {
+          sq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[i], xf[i], sq, 0, 0, 0);
+          #pragma unroll
+          for (int j = 0; j < 8; ++j) xf[i][j] = (__bf16)((float)xf[i][j] * (float)nf[i][j]);
+        }
+        #pragma unroll
+        for (int a = 0; a < NG; ++a)
+          acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i][a], xf[i], acc[a], 0, 0, 0);
+      }
+  }
+  if (NORM) {
+    #pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if ((l & 15) == 4 * g + r) squares[wave * 16 + (l & 15)] = sq[r];
+  }
+  if (MODE == RESIDUAL && wave == 0) {      // an adapter: more of K, elsewhere
+    for (int k0 = 0; k0 < R; k0 += 64) {
+      const int k = k0 + ko;
+      const bool there = k < R;             // an odd number of steps: zeros
+      const bf16v8 v = there ? *reinterpret_cast<const bf16v8*>(p.u + (int64_t)min(r8, M - 1) * R + k)
+                             : bf16v8{};
+      #pragma unroll
+      for (int a = 0; a < NG; ++a) {
+        const bf16v8 b = there ? *reinterpret_cast<const bf16v8*>(
+                                     p.ub + (int64_t)(n0 + a * 8 + r8) * R + k)
+                               : bf16v8{};
+        acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, v, acc[a], 0, 0, 0);
+      }
+    }
+  }
+  // the diagonal: lanes whose four rows and whose column are of the same step
+  if ((g >> 1) == second) {
+    #pragma unroll
+    for (int a = 0; a < NG; ++a) red[wave][a][second * 16 + (g & 1) * 8 + r8] = acc[a];
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  f32x4 sum[ACC];
+  const int quad = l % QUADS, part = l / QUADS;
+  #pragma unroll
+  for (int c = 0; c < ACC; ++c) {
+    sum[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    #pragma unroll
+    for (int i = 0; i < 2 * KW / PARTS; ++i) {
+      const int v = i * PARTS + part;
+      sum[c] += red[v >> 1][c * OUT + quad / 16][(v & 1) * 16 + quad % 16];
+    }
+    #pragma unroll
+    for (int off = QUADS; off < WAVE; off <<= 1)
+      #pragma unroll
+      for (int r = 0; r < 4; ++r) sum[c][r] += __shfl_xor(sum[c][r], off, WAVE);
+  }
+  if (NORM) {
+    float ss = 0.f;
+    #pragma unroll
+    for (int v = 0; v < 2 * KW; ++v) ss += squares[v * 8 + m];
+    const float r = rsqrtf(ss / K + p.eps);
+    #pragma unroll
+    for (int c = 0; c < ACC; ++c) sum[c] *= r;
+  }
+  if (m >= M || part) return;
+  bf16v4 o;
+  #pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (MODE == GLU) {
+      // gate and up round as the separate product's output does
+      const float gt = (float)(__bf16)sum[0][r], up = (float)(__bf16)sum[ACC - 1][r];
+      o[r] = (__bf16)(gt / (1.f + __expf(-gt)) * up);
+    } else {
+      o[r] = (__bf16)(MODE == RESIDUAL || p.bias ? sum[0][r] + (float)add[r] : sum[0][r]);
+    }
+  }
+  *reinterpret_cast<bf16v4*>(p.y + at) = o;
+}
+
+template <int MODE, int NG, int KW, int U>
+void launch_pair(const PairArgs& p, int kind) {
+  const dim3 grid(p.N / (NG / (MODE == GLU ? 2 : 1) * 8));
+  auto stream = at::cuda::getCurrentCUDAStream();
+  auto go = [&](auto w_) {
+    hipLaunchKernelGGL((skinny_pair_kernel<NG, KW, U, MODE, decltype(w_)::value>), grid, dim3(KW * 64),
+                       0, stream, p);
+  };
+  if (kind == ROWS) go(std::integral_constant<int, ROWS>{});
+  else if (kind == KEPT) go(std::integral_constant<int, KEPT>{});
+  else go(std::integral_constant<int, TILES>{});
+}
+
+// Rows of W a workgroup, waves and double steps in flight, from a sweep of them at 8 rows
+// and cold weights (us; rows, waves, in flight: their best). What is on its way passes
+// a CU's 32 KB of cache: where workgroups are many fewer steps are faster, few ones need
+// a wave's whole share at once. N 896 K 896 3.03 with 8/16/1 (8/8/2 3.38, 16/8/2 4.26);
+// 896 x 4864 6.12 8/8/10 (8/8/5 6.41, 16/8/10 9.5); 1536 x 8960 11.4 8/8/9; 2560 x 9728
+// 14.25 16/8/5 (16/8/10 14.84, 8/8/10 21.1); 3584 x 18944 26.7 16/8/5; 6144 x 2560 10.2
+// 16/8/5 (8/8/5 12.6); SiLU*mul of N 4864 K 896 6.4 8/8/2 (16/8/2 7.95), 8960 x 1536 12.5
+// 16/8/2 (16/8/3 14.8), 9728 x 2560 19.5 16/8/2 (16/8/5 22.1), 18944 x 3584 46.9 16/8/4.
+template <int MODE>
+void pair(const PairArgs& p, int kind) {
+  constexpr int ACC = MODE == GLU ? 2 : 1;
+  const int steps = p.K / 64, share = CDIV(steps, 8);
+  const bool narrow = p.N <= 2048 || (MODE == GLU && steps <= 16);
+  // a wave's share in even rounds of at most so many steps
+  const int most = narrow ? 10 : MODE != GLU ? 5 : share <= 6 ? 2 : 4;
+  const int u = CDIV(share, CDIV(share, most));
+  if (!narrow) {
+    if (u <= 2) launch_pair<MODE, 2 * ACC, 8, 2>(p, kind);
+    else if (u == 3) launch_pair<MODE, 2 * ACC, 8, 3>(p, kind);
+    else if (u == 4) launch_pair<MODE, 2 * ACC, 8, 4>(p, kind);
+    else launch_pair<MODE, 2 * ACC, 8, 5>(p, kind);
+  } else if (MODE != GLU && steps <= 16) {
+    launch_pair<MODE, ACC, 16, 1>(p, kind);
+  } else if (u <= 2) {
+    launch_pair<MODE, ACC, 8, 2>(p, kind);
+  } else if (u == 3) {
+    launch_pair<MODE, ACC, 8, 3>(p, kind);
+  } else if (u <= 5) {
+    launch_pair<MODE, ACC, 8, 5>(p, kind);
+  } else if (u <= 7) {
+    launch_pair<MODE, ACC, 8, 7>(p, kind);
+  } else if (u <= 9) {
+    launch_pair<MODE, ACC, 8, 9>(p, kind);
+  } else {
+    launch_pair<MODE, ACC, 8, 10>(p, kind);
+  }
+}
+
 // An operand as 16 B loads can read it: a parameter cut out of a larger buffer
 // may start anywhere.
 torch::Tensor at16(const torch::Tensor& t) {
@@ -245,6 +443,18 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
   const int nt = N / 16, steps = K / 32, tr = nt <= 128 ? 8 : 16;
   const int kw = nt <= 256 ? (steps >= 64 ? 16 : steps >= 32 ? 8 : 4)
                         : (mode == GLU && steps >= 48 ? 8 : 4);
+  TORCH_CHECK(mode != RESIDUAL || !nw, "skinny_gemm: norm with a residual sum");
+  const int kind = !tiles ? ROWS : kept ? KEPT : TILES;
+  // as a step of few sequences calls them; without a norm only adapters of 32 rows are
+  // multiplied, which wait for the launch
+  if (M <= 8 && K % 64 == 0 && (nw != nullptr) == (mode != RESIDUAL)) {
+    const PairArgs args{ptr(x), ptr(w), b, r, nw, up, ubp, o, M, N, K, R, (float)eps};
+    if (mode == PLAIN) pair<PLAIN>(args, kind);
+    else if (mode == RESIDUAL) pair<RESIDUAL>(args, kind);
+    else pair<GLU>(args, kind);
+    HIP_CHECK_LAST();
+    return y;
+  }
   auto launch = [&](auto mt_, auto kw_, auto mode_, auto norm_, auto w_) {
     constexpr int MT = decltype(mt_)::value, KW = decltype(kw_)::value,
                   MODE = decltype(mode_)::value;
@@ -254,8 +464,8 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
                        dim3(KW * 64), smem, stream, ptr(x), ptr(w), b, r, nw, up, ubp, o, M, N, K, R, tr, (float)eps);
   };
   auto go = [&](auto mt_, auto kw_, auto mode_, auto norm_) {
-    if (!tiles) launch(mt_, kw_, mode_, norm_, std::integral_constant<int, ROWS>{});
-    else if (kept) launch(mt_, kw_, mode_, norm_, std::integral_constant<int, KEPT>{});
+    if (kind == ROWS) launch(mt_, kw_, mode_, norm_, std::integral_constant<int, ROWS>{});
+    else if (kind == KEPT) launch(mt_, kw_, mode_, norm_, std::integral_constant<int, KEPT>{});
     else launch(mt_, kw_, mode_, norm_, std::integral_constant<int, TILES>{});
   };
   auto by_norm = [&](auto mt_, auto kw_, auto mode_) {
@@ -271,7 +481,6 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
     else if (kw == 8) by_mode(mt_, std::integral_constant<int, 8>{});
     else by_mode(mt_, std::integral_constant<int, 4>{});
   };
-  TORCH_CHECK(mode != RESIDUAL || !nw, "skinny_gemm: norm with a residual sum");
   if (M <= 16) by_kw(std::integral_constant<int, 1>{});
   else by_kw(std::integral_constant<int, 2>{});
   HIP_CHECK_LAST();

@@ -91,6 +91,34 @@ def test_skinny_gemm_tiles(ext, M, N, K):
             assert torch.equal(ext.skinny_gemm(x, tiles, mode, tiles=True, kept=kept, **args), want)
 
 
+@pytest.mark.parametrize("M", [1, 7, 8])
+@pytest.mark.parametrize("N,K,R", [(16, 512, 32), (896, 896, 0), (1152, 1024, 96), (2048, 1088, 64),
+                                   (2064, 576, 32), (32, 4864, 0), (2080, 8960, 32)])
+def test_skinny_gemm_few_rows(ext, M, N, K, R):
+    """Up to 8 rows: two steps of K side by side, shares of every size. Sums in fp32 of
+    products that are exact: what is left is the output's rounding, and of gate and up
+    each their own, whose errors silu at most doubles."""
+    x, w, b = _rand((M, K), 1), _rand((2 * N, K), 2, K ** -0.5), _rand((N,), 3)
+    res, kw = _rand((M, N), 4), {"norm_w": _rand((K,), 7, 0.1) + 1, "eps": 1e-6}
+    half = w[:N].contiguous()
+    xd, wd = x.double(), half.double()
+    n = (xd * kw["norm_w"].double()).to(torch.bfloat16).double() \
+        * (xd.pow(2).mean(-1, keepdim=True) + 1e-6).rsqrt()
+    assert _rel(ext.skinny_gemm(x, half, 0, b, **kw), n @ wd.t() + b.double()) < 2.0 ** -8
+    y = xd @ wd.t() + res.double()
+    assert _rel(ext.skinny_gemm(x, half, 1, res=res), y) < 2.0 ** -8
+    if R:
+        u, ub = _rand((M, R), 5), _rand((N, R), 6, 0.1)
+        got = ext.skinny_gemm(x, half, 1, res=res, u=u, ub=ub)
+        assert _rel(got, y + u.double() @ ub.double().t()) < 2.0 ** -8
+    gate, up = (n @ w.double().t()).split(N, 1)
+    assert _rel(ext.skinny_gemm(x, w, 2, **kw), torch.nn.functional.silu(gate) * up) < 2.0 ** -6
+    # a row that is no number stays by itself
+    x[0, 0] = float("inf")
+    assert ext.skinny_gemm(x, half, 1, res=res)[1:].isfinite().all()
+    assert ext.skinny_gemm(x, half, 0, **kw)[1:].isfinite().all()
+
+
 @pytest.mark.parametrize("model,n,tiled,skinny", [
     ("qwen2.5-0.5b", 16, True, True), ("qwen2.5-0.5b", 17, True, False),
     ("qwen2.5-0.5b", 32, False, True), ("qwen2.5-0.5b", 33, False, False),
