@@ -4,9 +4,15 @@
 // log-prob tensor — the reference loops rows through log_softmax+gather,
 // distributed_actor.py:253-260); backward emits dlogits directly:
 // dlogits_v = w * (1[v=target] - softmax_v), w = mask*coef*dloss.
+// Where a gradient is wanted, both are one pass over logits that a workgroup's registers
+// hold (loss_both_kernel).
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16v2;
 
 namespace {
 
@@ -161,14 +167,12 @@ void loss_rows_kernel(const float* __restrict__ token_logp, const float* __restr
 // for rows that give each four loads at least (32768 values: 242 and 242 us for 8000
 // rows) 345.
 template <typename T, int THREADS>
-__global__ __launch_bounds__(THREADS)
-void loss_bwd_kernel(const T* __restrict__ logits,
+DEV_INLINE void loss_bwd_row(const T* __restrict__ logits,
                      const int64_t* __restrict__ targets,
                      const float* __restrict__ w,
                      const float* __restrict__ lse,
                      const float* __restrict__ dloss,   // scalar, or null: 1
-                     T* __restrict__ dlogits, int V) {
-  const int64_t row = gridDim.x - 1 - blockIdx.x;
+                     T* __restrict__ dlogits, int V, int64_t row) {
   const T* lr = logits + row * V;
   T* dr = dlogits + row * V;
   const float wv = dloss ? w[row] * *dloss : w[row];
@@ -221,6 +225,184 @@ void loss_bwd_kernel(const T* __restrict__ logits,
   }
 }
 
+template <typename T, int THREADS>
+__global__ __launch_bounds__(THREADS)
+void loss_bwd_kernel(const T* __restrict__ logits, const int64_t* __restrict__ targets,
+                     const float* __restrict__ w, const float* __restrict__ lse,
+                     const float* __restrict__ dloss, T* __restrict__ dlogits, int V) {
+  loss_bwd_row<T, THREADS>(logits, targets, w, lse, dloss, dlogits, V,
+                           (int64_t)gridDim.x - 1 - blockIdx.x);
+}
+
+// The same where dlogits holds the gradient for a dloss of 1 already: a few workgroups
+// look whether it is that.
+template <typename T, int THREADS>
+__global__ __launch_bounds__(THREADS)
+void loss_anew_kernel(const T* __restrict__ logits, const int64_t* __restrict__ targets,
+                      const float* __restrict__ w, const float* __restrict__ lse,
+                      const float* __restrict__ dloss, T* __restrict__ dlogits, int V,
+                      int64_t rows) {
+  if (*dloss == 1.f) return;
+  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
+    loss_bwd_row<T, THREADS>(logits, targets, w, lse, dloss, dlogits, V, row);
+}
+
+// Both passes at once, where the gradient will be asked for: a workgroup holds a row in
+// registers, KEEP pieces of 8 values a thread, makes its log-sum-exp and writes the
+// gradient for a dloss of 1, so that logits are read once. As a piece is written the
+// next row's takes its registers: a workgroup walks rows, and reads and writes are on
+// their way all the time. Bound by memory: 2408 rows of 152064, a quarter of weight zero,
+// 308 us (4.75 TB/s read and written), 133 and 222 in two passes; with the sum over rows
+// and the look at dloss 356 -> 320. Loads or stores through or past the caches are even.
+struct RowWeights {
+  const float* w;             // of each row, or
+  const void* mask;           // (B, T), int64 or fp32, and rewards as the loss has them
+  bool mask64;
+  const float* rewards;
+  int B, T;
+  float scale;
+};
+
+template <int THREADS, int KEEP>
+__global__ __launch_bounds__(THREADS)
+void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* __restrict__ targets,
+                      RowWeights weights, float* __restrict__ token_logp,
+                      float* __restrict__ lse_out, __hip_bfloat16* __restrict__ dlogits, int rows,
+                      int V) {
+  constexpr float LOG2E = 1.4426950408889634f;
+  constexpr int NW = THREADS / WAVE;
+  __shared__ float part[2][3][NW];
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1), nvec = V / 8;
+  u32x4 v[KEEP];
+  // One offset that walks a row, as 19 addresses would take the registers: what lies past
+  // the row's end reads as zero, is left out of the sums and not written.
+  const int bytes = nvec * 16;
+  auto row_at = [&](const __hip_bfloat16* p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<__hip_bfloat16*>(p), 0, bytes, 0x00027000);
+  };
+  auto next = [&](int& off) {
+    off += THREADS * 16;
+    asm volatile("" : "+v"(off));
+  };
+  auto value = [&](int c, int j) {
+    return __uint_as_float(j & 1 ? v[c][j / 2] & 0xffff0000u : v[c][j / 2] << 16);
+  };
+  int64_t row = blockIdx.x;
+  {
+    const auto from = row_at(logits + row * V);
+    int off = tid * 16;
+    #pragma unroll
+    for (int c = 0; c < KEEP; ++c, next(off)) v[c] = __builtin_amdgcn_raw_buffer_load_b128(from, off, 0, 0);
+  }
+  for (int turn = 0; row < rows; row += gridDim.x, turn ^= 1) {
+    const __hip_bfloat16* lr = logits + row * V;
+    __hip_bfloat16* dr = dlogits + row * V;
+    const int64_t tgt = targets[row];
+    // the sequence's mask, summed beside the logits
+    float share = 0.f;
+    const int64_t seq = weights.w ? 0 : row / weights.T;
+    auto mask = [&](int64_t i) {
+      return weights.mask64 ? (float)reinterpret_cast<const int64_t*>(weights.mask)[i]
+                            : reinterpret_cast<const float*>(weights.mask)[i];
+    };
+    if (!weights.w)
+      for (int t = tid; t < weights.T; t += THREADS) share += mask(seq * weights.T + t);
+    const int at = nvec * 8 + tid;                        // of the last few
+    const float tail = at < V ? ld(lr, at) : -__builtin_inff();
+
+    float m = -1e30f, s = 0.f;     // s: sum of 2^((x - m) log2 e)
+    auto take = [&](const float* x, int n) {
+      float top = m;
+      #pragma unroll
+      for (int j = 0; j < n; ++j) top = fmaxf(top, x[j]);
+      if (top > m) {
+        s *= __builtin_amdgcn_exp2f((m - top) * LOG2E);
+        m = top;
+      }
+      const float c = m * LOG2E;
+      #pragma unroll
+      for (int j = 0; j < n; ++j) s += __builtin_amdgcn_exp2f(x[j] * LOG2E - c);
+    };
+    #pragma unroll
+    for (int c = 0; c < KEEP; ++c) {
+      if (c * THREADS >= nvec) continue;
+      if (c * THREADS + tid < nvec) {
+        float x[8];
+        #pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = value(c, j);
+        take(x, 8);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (at < V) take(&tail, 1);
+    // over the workgroup: one meeting a row, in turns of LDS
+    const float M = wave_max(m);
+    s = wave_sum(s * __builtin_amdgcn_exp2f((m - M) * LOG2E));
+    share = wave_sum(share);
+    if (lane == 0) {
+      part[turn][0][tid / WAVE] = M;
+      part[turn][1][tid / WAVE] = s;
+      part[turn][2][tid / WAVE] = share;
+    }
+    __syncthreads();
+    // a wave's lanes take a wave each, in every wave
+    const int of = lane & (NW - 1);
+    float top = part[turn][0][of], sum = part[turn][1][of], n = part[turn][2][of];
+    float high = top;
+    #pragma unroll
+    for (int off = NW / 2; off > 0; off >>= 1) high = fmaxf(high, __shfl_xor(high, off, WAVE));
+    sum *= __builtin_amdgcn_exp2f((top - high) * LOG2E);
+    #pragma unroll
+    for (int off = NW / 2; off > 0; off >>= 1) {
+      sum += __shfl_xor(sum, off, WAVE);
+      n += __shfl_xor(n, off, WAVE);
+    }
+    top = high;
+    const float l = top + __logf(sum);
+    const float wv = weights.w ? weights.w[row]
+                               : mask(row) * (-weights.rewards[seq] / fmaxf(n, 1.f) / weights.B * weights.scale);
+    if (tid == 0) lse_out[row] = l;
+    if (tid == 0 && (tgt < 0 || tgt >= V)) token_logp[row] = 0.f - l;
+    if (at < V) {
+      if (at == tgt) token_logp[row] = tail - l;
+      float g = 0.f;
+      if (wv != 0.f) g = wv * ((at == (int)tgt ? 1.f : 0.f) - __expf(tail - l));
+      dr[at] = f2bf(g);
+    }
+    const auto to = row_at(dr), from = row_at(lr + (int64_t)gridDim.x * V);
+    auto write = [&](auto more_) {
+      int off = tid * 16;
+      #pragma unroll
+      for (int c = 0; c < KEEP; ++c, next(off)) {
+        {
+          if (off == (int)(tgt >> 3) * 16 && off < bytes && tgt >= 0) {
+            float x = value(c, 0);
+            #pragma unroll
+            for (int j = 1; j < 8; ++j) x = (int)(tgt & 7) == j ? value(c, j) : x;
+            token_logp[row] = x - l;
+          }
+          u32x4 o;
+          #pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            float g[2];
+            #pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const float p = __expf(value(c, 2 * j + h) - l);
+              g[h] = wv == 0.f ? 0.f : wv * ((off / 2 + 2 * j + h == (int)tgt ? 1.f : 0.f) - p);
+            }
+            o[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{g[0], g[1]}, bf16v2));
+          }
+          __builtin_amdgcn_raw_buffer_store_b128(o, to, off, 0, 2);     // 2: past the caches
+        }
+        if (decltype(more_)::value) v[c] = __builtin_amdgcn_raw_buffer_load_b128(from, off, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (row + gridDim.x < rows) write(std::true_type{});
+    else write(std::false_type{});
+  }
+}
+
 }  // namespace
 
 std::vector<torch::Tensor> logprob_lse_fwd(torch::Tensor logits,
@@ -253,18 +435,65 @@ std::vector<torch::Tensor> logprob_lse_fwd(torch::Tensor logits,
   return {token_logp, lse};
 }
 
-// The masked PG/GRPO loss of logits (B, T, V): {loss, row weights (B, T), lse}.
-// mask int64 or fp32, rewards fp32.
+// Whether loss_both_kernel takes the rows: longer ones don't fit its registers.
+static bool takes_both(const torch::Tensor& logits) {
+  const int64_t V = logits.size(-1);
+  return logits.scalar_type() == at::kBFloat16 && logits.numel() > 0 && V >= 8 &&
+         V / 8 <= 19 * 1024 && logits.numel() / V < (1 << 30);
+}
+
+// {token_logp, lse, the gradient for a dloss of 1}
+static std::vector<torch::Tensor> logprob_both(const torch::Tensor& logits,
+                                               const torch::Tensor& targets,
+                                               const RowWeights& weights) {
+  TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() && takes_both(logits));
+  TORCH_CHECK(targets.scalar_type() == at::kLong && targets.is_contiguous());
+  const int V = logits.size(-1), nvec = V / 8;
+  const int rows = (int)(logits.numel() / V);
+  auto sizes = logits.sizes().vec();
+  sizes.pop_back();
+  auto token_logp = torch::empty(sizes, logits.options().dtype(at::kFloat));
+  auto lse = torch::empty_like(token_logp);
+  auto grad = torch::empty_like(logits);
+  // workgroups a CU by their registers
+  auto go = [&](auto threads_, auto keep_, int per_cu) {
+    constexpr int THREADS = decltype(threads_)::value, KEEP = decltype(keep_)::value;
+    hipLaunchKernelGGL((loss_both_kernel<THREADS, KEEP>), dim3(std::min(rows, 256 * per_cu)),
+                       dim3(THREADS), 0, at::cuda::getCurrentCUDAStream(),
+                       reinterpret_cast<const __hip_bfloat16*>(logits.data_ptr()),
+                       targets.data_ptr<int64_t>(), weights, token_logp.data_ptr<float>(),
+                       lse.data_ptr<float>(), reinterpret_cast<__hip_bfloat16*>(grad.data_ptr()),
+                       rows, V);
+  };
+  using Few = std::integral_constant<int, 256>;
+  using Many = std::integral_constant<int, 1024>;
+  if (nvec <= 2 * 256) go(Few{}, std::integral_constant<int, 2>{}, 8);
+  else if (nvec <= 8 * 256) go(Few{}, std::integral_constant<int, 8>{}, 6);
+  else if (nvec <= 4 * 1024) go(Many{}, std::integral_constant<int, 4>{}, 2);
+  else if (nvec <= 8 * 1024) go(Many{}, std::integral_constant<int, 8>{}, 1);
+  else if (nvec <= 16 * 1024) go(Many{}, std::integral_constant<int, 16>{}, 1);
+  else go(Many{}, std::integral_constant<int, 19>{}, 1);
+  HIP_CHECK_LAST();
+  return {token_logp, lse, grad};
+}
+
+// The masked PG/GRPO loss of logits (B, T, V): {loss, row weights (B, T), lse}, and
+// with both the gradient for a dloss of 1. mask int64 or fp32, rewards fp32.
 static std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits, torch::Tensor targets,
                                                    torch::Tensor mask, torch::Tensor rewards,
-                                                   double scale) {
+                                                   double scale, bool both) {
   TORCH_CHECK(logits.dim() == 3 && mask.is_cuda() && rewards.is_cuda());
   const int B = logits.size(0), T = logits.size(1);
   TORCH_CHECK(mask.numel() == (int64_t)B * T && targets.numel() == (int64_t)B * T &&
               rewards.numel() == B, "logprob_loss: shape mismatch");
   TORCH_CHECK(mask.is_contiguous() && rewards.is_contiguous() &&
               rewards.scalar_type() == at::kFloat);
-  auto lp = logprob_lse_fwd(logits, targets);
+  const bool mask64 = mask.scalar_type() == at::kLong;
+  TORCH_CHECK(mask64 || mask.scalar_type() == at::kFloat);
+  auto lp = both ? logprob_both(logits, targets,
+                                {nullptr, mask.data_ptr(), mask64, rewards.data_ptr<float>(), B, T,
+                                 (float)scale})
+                 : logprob_lse_fwd(logits, targets);
   auto w = torch::empty_like(lp[0]);
   auto loss = torch::empty({}, lp[0].options());
   auto stream = at::cuda::getCurrentCUDAStream();
@@ -273,16 +502,18 @@ static std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits, torch::
                        lp[0].data_ptr<float>(), mask.data_ptr<M>(),                   \
                        rewards.data_ptr<float>(), w.data_ptr<float>(),                \
                        loss.data_ptr<float>(), B, T, (float)scale)
-  if (mask.scalar_type() == at::kLong) REDUCE(int64_t);
-  else { TORCH_CHECK(mask.scalar_type() == at::kFloat); REDUCE(float); }
+  if (mask64) REDUCE(int64_t);
+  else REDUCE(float);
   #undef REDUCE
   HIP_CHECK_LAST();
+  if (both) return {loss, w, lp[1], lp[2]};
   return {loss, w, lp[1]};
 }
 
-torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets,
-                               torch::Tensor w, torch::Tensor lse,
-                               c10::optional<torch::Tensor> dloss) {
+// made: the gradient for a dloss of 1, which is kept where dloss is that
+static torch::Tensor loss_bwd(torch::Tensor logits, torch::Tensor targets, torch::Tensor w,
+                              torch::Tensor lse, c10::optional<torch::Tensor> dloss,
+                              c10::optional<torch::Tensor> made) {
   TORCH_CHECK(logits.is_cuda() && logits.is_contiguous());
   const float* dl = nullptr;
   if (dloss) {
@@ -291,47 +522,81 @@ torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets,
   }
   const int V = logits.size(-1);
   const int64_t rows = logits.numel() / V;
-  auto dlogits = torch::empty_like(logits);
+  TORCH_CHECK(!made || (dl && made->is_contiguous() && made->sizes() == logits.sizes() &&
+                        made->scalar_type() == logits.scalar_type()));
+  auto dlogits = made ? *made : torch::empty_like(logits);
   if (rows == 0) return dlogits;
   auto stream = at::cuda::getCurrentCUDAStream();
   auto wc = w.contiguous();
   auto lsec = lse.contiguous();
   auto tc = targets.contiguous();
-  #define BWD(T, THREADS)                                                              \
-    hipLaunchKernelGGL((loss_bwd_kernel<T, THREADS>), dim3(rows), dim3(THREADS), 0,    \
-                       stream, reinterpret_cast<const T*>(logits.data_ptr()),          \
+  const bool bf16 = logits.scalar_type() == at::kBFloat16;
+  const bool many = bf16 && V / 8 >= 4 * 1024;
+  #define BWD(KERNEL, T, THREADS, BLOCKS, ...)                                         \
+    hipLaunchKernelGGL((KERNEL<T, THREADS>), dim3(BLOCKS), dim3(THREADS), 0, stream,   \
+                       reinterpret_cast<const T*>(logits.data_ptr()),                  \
                        tc.data_ptr<int64_t>(), wc.data_ptr<float>(),                   \
                        lsec.data_ptr<float>(), dl,                                     \
-                       reinterpret_cast<T*>(dlogits.data_ptr()), V)
-  if (logits.scalar_type() != at::kBFloat16) BWD(float, 256);
-  else if (V / 8 >= 4 * 1024) BWD(__hip_bfloat16, 1024);
-  else BWD(__hip_bfloat16, 256);
+                       reinterpret_cast<T*>(dlogits.data_ptr()), V, ##__VA_ARGS__)
+  if (made) {
+    const int64_t blocks = std::min<int64_t>(rows, 512);
+    if (many) BWD(loss_anew_kernel, __hip_bfloat16, 1024, blocks, rows);
+    else BWD(loss_anew_kernel, __hip_bfloat16, 256, blocks, rows);
+  } else if (many) {
+    BWD(loss_bwd_kernel, __hip_bfloat16, 1024, rows);
+  } else if (bf16) {
+    BWD(loss_bwd_kernel, __hip_bfloat16, 256, rows);
+  } else {
+    BWD(loss_bwd_kernel, float, 256, rows);
+  }
   #undef BWD
   HIP_CHECK_LAST();
   return dlogits;
 }
 
-// The differentiable loss: a node of the C++ engine.
+torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets, torch::Tensor w,
+                               torch::Tensor lse, c10::optional<torch::Tensor> dloss) {
+  return loss_bwd(logits, targets, w, lse, dloss, c10::nullopt);
+}
+
+// The differentiable loss: a node of the C++ engine. Where a gradient is wanted of rows
+// that loss_both_kernel takes, forward makes it for a dloss of 1, which backward hands
+// out; any other dloss makes it anew from the logits, and so does every further backward
+// of a graph that is kept, as what was handed out is the caller's.
 namespace {
+
+bool wants_both(const torch::Tensor& logits) {
+  return at::GradMode::is_enabled() && logits.requires_grad() && logits.is_cuda() && takes_both(logits);
+}
+
+torch::Tensor handed_out(torch::autograd::AutogradContext* ctx, const torch::Tensor& dloss) {
+  const auto s = ctx->get_saved_variables();
+  c10::optional<torch::Tensor> made;
+  if (const auto it = ctx->saved_data.find("grad"); it != ctx->saved_data.end()) {
+    made = it->second.toTensor();
+    ctx->saved_data.erase(it);
+  }
+  return loss_bwd(s[0], s[1], s[2], s[3], dloss.to(at::kFloat), made);
+}
 
 struct LogprobLoss : public torch::autograd::Function<LogprobLoss> {
   static torch::Tensor forward(torch::autograd::AutogradContext* ctx, torch::Tensor logits,
                                torch::Tensor targets, torch::Tensor mask, torch::Tensor rewards,
-                               double scale) {
+                               double scale, bool both) {
     logits = logits.contiguous();
     targets = targets.contiguous();
     // int64 masks are read as they are
     auto m = mask.scalar_type() == at::kLong ? mask : mask.to(at::kFloat);
     auto r = logprob_loss_fwd(logits, targets, m.contiguous(),
-                              rewards.to(at::kFloat).contiguous(), scale);
+                              rewards.to(at::kFloat).contiguous(), scale, both);
     ctx->save_for_backward({logits, targets, r[1], r[2]});
+    if (both) ctx->saved_data["grad"] = r[3];
     return r[0];
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
-    const auto s = ctx->get_saved_variables();
-    auto d = logprob_loss_bwd(s[0], s[1], s[2], s[3], grads[0].to(at::kFloat));
-    return {d, torch::Tensor(), torch::Tensor(), torch::Tensor(), torch::Tensor()};
+    return {handed_out(ctx, grads[0]), torch::Tensor(), torch::Tensor(), torch::Tensor(),
+            torch::Tensor(), torch::Tensor()};
   }
 };
 
@@ -339,7 +604,7 @@ struct LogprobLoss : public torch::autograd::Function<LogprobLoss> {
 
 torch::Tensor logprob_loss(torch::Tensor logits, torch::Tensor targets, torch::Tensor mask,
                            torch::Tensor rewards, double scale) {
-  return LogprobLoss::apply(logits, targets, mask, rewards, scale);
+  return LogprobLoss::apply(logits, targets, mask, rewards, scale, wants_both(logits));
 }
 
 // The same sum for rows that carry weights of their own: sum_i w_i log p(target_i)
@@ -348,32 +613,32 @@ namespace {
 
 struct LogprobRows : public torch::autograd::Function<LogprobRows> {
   static torch::Tensor forward(torch::autograd::AutogradContext* ctx, torch::Tensor logits,
-                               torch::Tensor targets, torch::Tensor w) {
+                               torch::Tensor targets, torch::Tensor w, bool both) {
     TORCH_CHECK(logits.dim() == 2 && targets.is_cuda() && w.is_cuda() &&
                 targets.numel() == logits.size(0) && w.numel() == logits.size(0) &&
                 w.scalar_type() == at::kFloat, "logprob_rows: shape mismatch");
     logits = logits.contiguous();
     targets = targets.contiguous();
     w = w.contiguous();
-    auto lp = logprob_lse_fwd(logits, targets);
+    auto lp = both ? logprob_both(logits, targets, {w.data_ptr<float>()})
+                   : logprob_lse_fwd(logits, targets);
     auto loss = torch::empty({}, lp[0].options());
     hipLaunchKernelGGL(loss_rows_kernel, dim3(1), dim3(1024), 0, at::cuda::getCurrentCUDAStream(),
                        lp[0].data_ptr<float>(), w.data_ptr<float>(), loss.data_ptr<float>(),
                        logits.size(0));
     HIP_CHECK_LAST();
     ctx->save_for_backward({logits, targets, w, lp[1]});
+    if (both) ctx->saved_data["grad"] = lp[2];
     return loss;
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
-    const auto s = ctx->get_saved_variables();
-    auto d = logprob_loss_bwd(s[0], s[1], s[2], s[3], grads[0].to(at::kFloat));
-    return {d, torch::Tensor(), torch::Tensor()};
+    return {handed_out(ctx, grads[0]), torch::Tensor(), torch::Tensor(), torch::Tensor()};
   }
 };
 
 }  // namespace
 
 torch::Tensor logprob_rows(torch::Tensor logits, torch::Tensor targets, torch::Tensor w) {
-  return LogprobRows::apply(logits, targets, w);
+  return LogprobRows::apply(logits, targets, w, wants_both(logits));
 }

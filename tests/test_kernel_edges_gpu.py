@@ -1110,6 +1110,33 @@ def test_logprob_rows(ext, rows, V):
     assert _rel(grad, ref) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("rows,V", [(5, 8), (3, 4096), (700, 4104), (2, 16384), (9, 16391), (530, 32768),
+                                    (3, 65544), (2, 131079), (259, 155648), (2, 155656)])
+def test_loss_gradients_made_forward(ext, rows, V):
+    """Rows at the edges of what is held in registers, and rows beyond: one backward,
+    those behind it in a kept graph (what the first gave out is overwritten) and one
+    that is scaled give what the two passes apart do, up to the log-sum-exp's rounding
+    (some 1e-6, which moves few values over a bf16 rounding edge)."""
+    from distrl_llm_amd.ops import functional as OF
+    logits, g = _rand((rows, V), V, 2.0), torch.Generator().manual_seed(2)
+    logits[0, 1] = float("-inf")
+    targets = torch.randint(2, V, (rows,), generator=g).cuda()
+    w = torch.randn(rows, generator=g).cuda() * (torch.arange(rows, device="cuda") % 3 != 1)
+    tok, lse = ext.logprob_lse_fwd(logits, targets)
+    leaf = logits.clone().requires_grad_()
+    loss = OF.logprob_rows(leaf, targets, w)
+    assert abs(float(loss.detach()) - float((tok * w).sum())) < 1e-5 * float((tok * w).abs().sum() + 1e-30)
+    for scale in (1.0, 1.0, 3.0):
+        got, = torch.autograd.grad(loss * scale, leaf, retain_graph=True)
+        want = ext.logprob_loss_bwd(logits, targets, w * scale, lse)
+        assert _rel(got, want) < 1e-5
+        got.fill_(7.0)
+    once, = torch.autograd.grad(OF.logprob_rows(leaf, targets, w) * 3.0, leaf)
+    assert _rel(once, ext.logprob_loss_bwd(logits, targets, w * 3.0, lse)) < 1e-5
+    leaf.requires_grad_(False)                  # no gradient is wanted: none is made
+    assert not OF.logprob_rows(leaf, targets, w).requires_grad
+
+
 @pytest.mark.parametrize("rows", [4096, 4097, 6145, 8200])
 def test_feed_forward_half_in_waves(ext, rows):
     """Input gradients of rows whose tiles fill the chip once, of one row more,
