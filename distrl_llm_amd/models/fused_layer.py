@@ -135,6 +135,30 @@ class _FeedForward(torch.autograd.Function):
         return (dx, None, None, *grads)
 
 
+class Head(torch.autograd.Function):
+    """x W^T of the frozen LM head; the input's gradient is a product of our own,
+    whose sum over the vocabulary is cut into shares."""
+
+    @staticmethod
+    def forward(ctx, x, weight):
+        ctx.save_for_backward(weight)
+        return torch.nn.functional.linear(x, weight)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, g):
+        weight, = ctx.saved_tensors
+        return _ext().product_rows(g, weight), None
+
+
+def frozen_head(x, weight) -> bool:
+    """Whether Head takes x (rows, hidden) and the LM head's weight."""
+    bf16 = torch.bfloat16
+    return (x.is_cuda and x.dim() == 2 and x.dtype == weight.dtype == bf16
+            and weight.device == x.device and not weight.requires_grad
+            and type(weight) in (torch.Tensor, torch.nn.Parameter))
+
+
 def rotary(head_dim: int, theta: float, positions, cu, longest: int):
     """What the nodes need to know of the rows: int32 positions (rows,), fp32
     inverse frequencies and their negatives, the first row of every sequence

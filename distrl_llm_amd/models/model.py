@@ -320,6 +320,16 @@ class CausalLM(nn.Module):
             x = fused_layer.forward(layer, x, rotary)
         return self.model.norm(x)
 
+    def rows_logits(self, hidden: torch.Tensor) -> torch.Tensor:
+        """logits of some of forward_rows' rows (rows, H) where takes_rows(): a
+        frozen head's backward is a product of our own."""
+        head = self.lm_head
+        weight = self.model.embed_tokens.weight if head is None else head.weight
+        if ((head is None or type(head) is nn.Linear and head.bias is None)
+                and fused_layer.frozen_head(hidden, weight)):
+            return fused_layer.Head.apply(hidden, weight)
+        return self.logits(hidden)
+
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         if self.lm_head is None:
             return hidden @ self.model.embed_tokens.weight.t()

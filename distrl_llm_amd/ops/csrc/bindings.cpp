@@ -112,6 +112,7 @@ void flash_varlen_bwd(torch::Tensor dout, torch::Tensor q, torch::Tensor k,
 std::vector<torch::Tensor> adapter_grads(std::vector<torch::Tensor> y,
                                          std::vector<torch::Tensor> p,
                                          std::vector<int64_t> by_col);
+torch::Tensor product_rows(const torch::Tensor& g, const torch::Tensor& w);
 bool product_py(std::vector<std::vector<torch::Tensor>> a,
                 std::vector<std::vector<c10::optional<torch::Tensor>>> b,
                 std::vector<c10::optional<torch::Tensor>> bias,
@@ -292,6 +293,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("into") = py::none());
   m.def("flash_varlen_bwd", &flash_varlen_bwd,
         "its backward, into dq, dk and dv");
+  m.def("product_rows", &product_rows, py::arg("g"), py::arg("w"),
+        "g w, w (K, N) as it lies");
   m.def("product", &product_py, py::arg("a"), py::arg("b"), py::arg("bias"),
         py::arg("width"), py::arg("what"), py::arg("out"),
         py::arg("res") = py::none(), py::arg("tile") = 0,

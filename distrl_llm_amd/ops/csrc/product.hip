@@ -20,6 +20,9 @@
 // as many as its products. 8192 x 8192 x 8192 790 us, 1390 TFLOP/s (library 680);
 // 18793 x 2048 x 1568 121 (139); 4000 x 1536 x 8992 125 (109 and 20 for what it needs
 // beside adapters); 924 x 896 x 4896 27 (28), 924 x 1152 x 928 9.5 (19, its launch).
+// Sums over a vocabulary in shares of K, us (library's product): rows x 896 x 151936, 5 rows
+// 51 (184), 130 rows 78 (320), 561 rows 180 (437), 4801 rows 1205 (1650); 14400 x 1536 x
+// 151936 5540 (8397), 9000 x 3584 x 152064 7530 (11236).
 // One wave a SIMD with tiles of 128 x 128 each, for less LDS, spilled registers: 1530
 // us where this takes 930. Pairs of steps loaded together, for whole cache lines, were
 // slower (8192^3 870 for 770).
@@ -60,9 +63,10 @@ struct Args {
   int ldgu;
   __hip_bfloat16 *dgate, *dup;
   int ldd;
-  // shares of K a workgroup each, which the last of a tile to end adds up
+  // shares of K a workgroup each, which the last of a tile to end adds up, or (large
+  // tiles) a launch behind this one
   int splits;
-  float* part;                          // (tiles, shares, floats of a tile)
+  float* part;                          // (tiles, shares, floats of a tile), or (shares, M, N)
   unsigned long long *there, tag;       // (tiles, shares)
 };
 
@@ -103,7 +107,7 @@ void product_kernel(const Args args) {
   constexpr int NW = WM * WN, BM = WM * TM * 16, BN = WN * TN * 16;
   // pieces of 1 KB a wave loads; of A some past a tile's rows where they don't divide
   constexpr int PA = CDIV(BM / 16, NW), PB = BN / 16 / NW, EACH = PA + PB;
-  constexpr bool SPLITS = NW == 4;
+  constexpr bool SPLITS = NW == 4, SHARES = NW == 8 && MODE == PLAIN;
   constexpr int ABYTES = PA * NW * 1024, RINGBYTES = ABYTES + BN * BK * 2;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -112,11 +116,16 @@ void product_kernel(const Args args) {
 
   // An XCD takes tiles one behind the other, four rows of tiles by turns of columns, so
   // that what runs on it at once shares its L2.
-  int m_tile, n_tile;
+  // Of large tiles all of one share of K, then the next share's.
+  int m_tile, n_tile, share = SPLITS ? blockIdx.y : 0;
   {
-    const int rows = CDIV(M, BM), cols = args.cols, total = rows * cols;
-    const int x = blockIdx.x & 7;
-    const int t = x * (total >> 3) + min(x, total & 7) + (blockIdx.x >> 3);
+    const int rows = CDIV(M, BM), cols = args.cols, tiles = rows * cols;
+    const int x = blockIdx.x & 7, total = SHARES ? tiles * args.splits : tiles;
+    int t = x * (total >> 3) + min(x, total & 7) + (blockIdx.x >> 3);
+    if (SHARES && args.splits > 1) {
+      share = t / tiles;
+      t -= share * tiles;
+    }
     const int band = t / (4 * cols), in = t - band * 4 * cols, h = min(4, rows - band * 4);
     m_tile = band * 4 + in % h;
     n_tile = in / h;
@@ -165,10 +174,10 @@ void product_kernel(const Args args) {
     }
   };
   start();
-  const int share = SPLITS ? blockIdx.y : 0;
-  const int step0 = SPLITS ? (int)((int64_t)share * args.steps / args.splits) : 0;
-  const int steps = SPLITS ? (int)((int64_t)(share + 1) * args.steps / args.splits) - step0 : args.steps;
-  if (SPLITS) {
+  int step0 = 0, steps = args.steps;
+  if (SPLITS || (SHARES && args.splits > 1)) {
+    step0 = (int)((int64_t)share * args.steps / args.splits);
+    steps = (int)((int64_t)(share + 1) * args.steps / args.splits) - step0;
     int skip = step0;
     while (skip >= left) {
       skip -= left;
@@ -341,6 +350,19 @@ void product_kernel(const Args args) {
     nc[j] = min(n[j], N - 4);
   }
   auto at4 = [](const __hip_bfloat16* p) { return *reinterpret_cast<const bf16v4*>(p); };
+  if constexpr (SHARES) {
+    if (args.splits > 1) {
+      float* part = args.part + (int64_t)share * M * N;
+      #pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = row_of(i);
+        #pragma unroll
+        for (int j = 0; j < TN; ++j)
+          if (m < M && n[j] < N) *reinterpret_cast<f32x4*>(part + (int64_t)m * N + n[j]) = acc[i][j];
+      }
+      return;
+    }
+  }
   if constexpr (MODE != GLU_BWD) {
     #pragma unroll
     for (int h = 0; h < TN / HALF; ++h) {
@@ -416,6 +438,22 @@ void product_kernel(const Args args) {
   }
 }
 
+// out (rows of ld elements) <- the shares' sums in their order, (shares, M, N); four
+// columns a thread. Bound: memory.
+__global__ __launch_bounds__(256)
+void share_sum_kernel(const float* __restrict__ part, __hip_bfloat16* __restrict__ out,
+                      uint32_t cells, uint32_t N, int64_t ld, int shares) {
+  const uint32_t at = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (at >= cells) return;
+  f32x4 sum = *reinterpret_cast<const f32x4*>(part + at);
+  #pragma unroll 4
+  for (int z = 1; z < shares; ++z) sum += *reinterpret_cast<const f32x4*>(part + (int64_t)z * cells + at);
+  bf16v4 o;
+  #pragma unroll
+  for (int r = 0; r < 4; ++r) o[r] = (__bf16)sum[r];
+  *reinterpret_cast<bf16v4*>(out + at / N * ld + at % N) = o;
+}
+
 template <int WM, int WN, int TM, int TN, bool ROWS, int MODE>
 void launch(Args& a, int blocks, int splits) {
   constexpr int NW = WM * WN, BM = WM * TM * 16, BN = WN * TN * 16;
@@ -432,9 +470,17 @@ void launch(Args& a, int blocks, int splits) {
   }
   const int64_t total = (int64_t)CDIV(a.M, BM) * a.cols;
   TORCH_CHECK(total < (1 << 30), "product: size");
-  a.splits = std::max(1, std::min(splits, a.steps));
+  constexpr bool JOINS = NW == 4;       // in the kernel, in every mode
+  const bool plain = MODE == PLAIN && blocks == 1 && !a.bias[0] && !a.res;
+  a.splits = JOINS || plain ? std::max(1, std::min(splits, a.steps)) : 1;
   at::Tensor room;
-  if (a.splits > 1) {
+  const int64_t cells = (int64_t)a.M * a.width[0];
+  if (!JOINS && a.splits > 1) {
+    TORCH_CHECK(a.splits * cells < (int64_t)1 << 31 && total * a.splits < (1 << 30), "product: shares");
+    room = at::empty({a.splits * cells}, at::TensorOptions().dtype(at::kFloat).device(
+        at::kCUDA, at::cuda::current_device()));
+    a.part = room.data_ptr<float>();
+  } else if (a.splits > 1) {
     const int64_t shares = total * a.splits;
     room = at::empty({shares * (BM * BN * 4 + 8)}, at::TensorOptions().dtype(at::kByte).device(
         at::kCUDA, at::cuda::current_device()));
@@ -442,10 +488,16 @@ void launch(Args& a, int blocks, int splits) {
     a.part = reinterpret_cast<float*>(a.there + shares);
     a.tag = arrival_tag();
   }
-  hipLaunchKernelGGL((product_kernel<WM, WN, TM, TN, ROWS, MODE>), dim3(total, a.splits), dim3(NW * 64),
-                     smem,
-                     at::cuda::getCurrentCUDAStream(), a);
+  const auto stream = at::cuda::getCurrentCUDAStream();
+  hipLaunchKernelGGL((product_kernel<WM, WN, TM, TN, ROWS, MODE>),
+                     JOINS ? dim3(total, a.splits) : dim3(total * a.splits), dim3(NW * 64), smem,
+                     stream, a);
   HIP_CHECK_LAST();
+  if (!JOINS && a.splits > 1) {
+    hipLaunchKernelGGL(share_sum_kernel, dim3(CDIV(cells, 1024)), dim3(256), 0, stream, a.part, a.c,
+                       cells, a.width[0], a.ldc, a.splits);
+    HIP_CHECK_LAST();
+  }
 }
 
 template <bool ROWS, int MODE>
@@ -466,6 +518,17 @@ void by_size(Args& a, int blocks, int tile) {
   for (int tm = 8; tm >= 4; --tm) {
     const int64_t rounds = CDIV((int64_t)CDIV(a.M, 32 * tm) * columns(256), (int64_t)256);
     offer(tm, 1, a.steps * (rounds == 1 ? 0.29 + 0.043 * tm : rounds * (0.24 + 0.081 * tm)));
+    // Sums over a vocabulary (the LM head's input gradient) in shares, where tiles alone leave
+    // workgroups idle or their last round half empty: 561 x 896 x 151936 is 12 tiles. Shorter
+    // ones of few rows are the small tiles', whose shares meet without a launch. 1 GB of
+    // partial sums at most, 6 us for the launch that adds them at 4.5 TB/s.
+    const int64_t cells = (int64_t)a.M * a.width[0];
+    if (MODE != PLAIN || blocks != 1 || a.bias[0] || a.res || a.steps < 2048) continue;
+    for (int z = 2; z <= 64 && a.steps / z >= 64 && z * cells <= 1 << 28; ++z) {
+      const int64_t n = CDIV((int64_t)CDIV(a.M, 32 * tm) * columns(256) * z, (int64_t)256);
+      offer(tm, z, CDIV(a.steps, z) * (n == 1 ? 0.29 + 0.043 * tm : n * (0.24 + 0.081 * tm)) + 6. +
+                       z * cells * 8 / 4.5e6);
+    }
   }
   for (int z = 1; z <= 8 && (z == 1 || a.steps / z >= 8); ++z) {
     const double n128 = CDIV(a.M, 128) * (double)columns(128) * z / 256;
@@ -476,11 +539,11 @@ void by_size(Args& a, int blocks, int tile) {
   }
   if (tile) { pick = tile & 255; splits = std::max(1, tile >> 8); }
   switch (pick) {
-    case 8: return launch<2, 4, 8, 4, ROWS, MODE>(a, blocks, 1);
-    case 7: return launch<2, 4, 7, 4, ROWS, MODE>(a, blocks, 1);
-    case 6: return launch<2, 4, 6, 4, ROWS, MODE>(a, blocks, 1);
-    case 5: return launch<2, 4, 5, 4, ROWS, MODE>(a, blocks, 1);
-    case 4: return launch<2, 4, 4, 4, ROWS, MODE>(a, blocks, 1);
+    case 8: return launch<2, 4, 8, 4, ROWS, MODE>(a, blocks, splits);
+    case 7: return launch<2, 4, 7, 4, ROWS, MODE>(a, blocks, splits);
+    case 6: return launch<2, 4, 6, 4, ROWS, MODE>(a, blocks, splits);
+    case 5: return launch<2, 4, 5, 4, ROWS, MODE>(a, blocks, splits);
+    case 4: return launch<2, 4, 4, 4, ROWS, MODE>(a, blocks, splits);
     case 128: return launch<2, 2, 4, 4, ROWS, MODE>(a, blocks, splits);
     default: return launch<2, 2, 2, 2, ROWS, MODE>(a, blocks, splits);
   }
@@ -619,6 +682,13 @@ bool product_glu_bwd(const ProductBlock& block, const at::Tensor& gu, const at::
   o.ldd = (int)dgate.stride(0);
   by_size<true, GLU_BWD>(o, 1, tile);
   return true;
+}
+
+// g w, g (M, V), w (V, N): own products where they take them, else the library's.
+at::Tensor product_rows(const at::Tensor& g, const at::Tensor& w) {
+  auto out = at::empty({g.size(0), w.size(1)}, g.options());
+  if (g.size(0) > 0 && product({{w.size(1), {{g, w}}, {}}}, true, out)) return out;
+  return at::mm(g, w);
 }
 
 // The products above from Python, for tests. Whether they were taken.

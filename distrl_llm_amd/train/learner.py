@@ -128,7 +128,7 @@ class Learner:
         at = torch.cat(at).to(dev)
         weights = rewards[sample.to(dev)] * share.to(dev)
         hidden = self.model.forward_rows(ids, [n for n in lens if n])
-        logits = self.model.logits(hidden.index_select(0, at))
+        logits = self.model.rows_logits(hidden.index_select(0, at))
         return OF.logprob_rows(logits, targets, weights)
 
     def _micro_loss(self, problems, answers, rewards: torch.Tensor,

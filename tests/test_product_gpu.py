@@ -82,6 +82,30 @@ def test_sums_of_products(ext, M, widths, deep, spare, tile):
             assert untouched()
 
 
+@pytest.mark.parametrize("M,N,steps,spare", [(1, 8, 3, 0), (127, 264, 7, 8), (129, 248, 40, 0),
+                                             (257, 520, 11, 64)])
+@pytest.mark.parametrize("rows,shares", [(4, 2), (5, 3), (6, 7), (7, 64), (8, 5)])
+@pytest.mark.parametrize("what", ["rows", "columns"])
+def test_large_tiles_in_shares(ext, M, N, steps, spare, rows, shares, what):
+    """Shares of K of large tiles: of one step, of less than the ring, more of them than steps."""
+    rand, K = _make(M + shares), steps * 32
+    a = rand(M, K, spare=spare)
+    b = rand(K, N, spare=spare) if what == "rows" else rand(N, K, spare=spare)
+    out, untouched = _room(M, N, spare)
+    assert ext.product([[a]], [[b]], [None], [N], what, [out], None, rows | shares << 8)
+    _each_close(out, *_sum([(a, b)], what == "rows"))
+    assert untouched()
+
+
+@pytest.mark.parametrize("M,V,N", [(1, 65536, 64), (37, 65568, 96), (300, 70016, 264), (9, 32003, 64),
+                                   (0, 65536, 64)])
+def test_head_input_gradient(ext, M, V, N):
+    """Sums long enough for shares by the rule, and what goes to the library."""
+    rand = _make(M)
+    g, w = rand(M, V), rand(V, N)
+    _each_close(ext.product_rows(g, w), *_sum([(g, w)], True))
+
+
 @pytest.mark.parametrize("M,F,K,r", [(1, 8, 32, 32), (70, 40, 96, 32), (130, 136, 64, 64),
                                      (300, 264, 160, 32)])
 @pytest.mark.parametrize("tile", TILES)
