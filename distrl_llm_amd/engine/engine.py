@@ -764,7 +764,7 @@ class Engine:
         bs = self.pool.block_size
         L = len(parent.prompt_ids)
         full = L // bs  # number of completely-filled blocks
-        children = []
+        children, tails = [], []
         for i in range(n):
             self._seq_counter += 1
             child = Sequence(self._seq_counter, parent.prompt_ids,
@@ -776,12 +776,14 @@ class Engine:
                 table.append(b)
             if full < len(parent.block_table):
                 nb = self.pool.allocator.alloc()
-                self.pool.copy_block(parent.block_table[full], nb)
+                tails.append(nb)
                 table.append(nb)
             child.block_table = table
             child.context_len = L
             child.output_ids = [first_tokens[i]]
             children.append(child)
+        if tails:
+            self.pool.copy_to(parent.block_table[full], tails)
         # parent's own references are released (children hold their own)
         for b in parent.block_table:
             self.pool.allocator.free(b)
@@ -941,23 +943,30 @@ class Engine:
                 return
             with trace_range("engine/prefill"):
                 logits = self._prefill_batch(batch)
-            for i, parent in enumerate(batch):
+            # all prompts' draws are on their way before the first is waited for
+            firsts, caps = [], []
+            for i in range(len(batch)):
                 lg = logits[i:i + 1].expand(sp.n, -1).contiguous()
-                first = OF.sample_tokens(lg, sp.temperature, sp.top_p, sp.top_k,
-                                         generator=self.generator)
-                children = self._fork(parent, sp.n, first.tolist())
-                if token_limits is not None:
-                    for ci, c in enumerate(children):
-                        c.max_tokens = token_limits[parent.parent_prompt][ci]
-                elif sp.geom_len_mean:
+                firsts.append(OF.sample_tokens(
+                    lg, sp.temperature, sp.top_p, sp.top_k,
+                    generator=self.generator))
+                if token_limits is None and sp.geom_len_mean:
                     # EOS-realistic mode: per-candidate exponential caps
-                    uu = torch.rand(len(children), generator=self.generator,
+                    uu = torch.rand(sp.n, generator=self.generator,
                                     device=self.device)
-                    lims = (1.0 - float(sp.geom_len_mean)
-                            * uu.clamp_min(1e-9).log()).long() \
-                        .clamp(1, sp.max_tokens)
-                    for c, lim in zip(children, lims.tolist()):
-                        c.max_tokens = int(lim)
+                    caps.append((1.0 - float(sp.geom_len_mean)
+                                 * uu.clamp_min(1e-9).log()).long()
+                                .clamp(1, sp.max_tokens))
+            firsts = torch.stack(firsts).tolist()
+            if token_limits is not None:
+                caps = [token_limits[p.parent_prompt] for p in batch]
+            elif caps:
+                caps = torch.stack(caps).tolist()
+            for i, parent in enumerate(batch):
+                children = self._fork(parent, sp.n, firsts[i])
+                if caps:
+                    for c, cap in zip(children, caps[i]):
+                        c.max_tokens = cap
                 for c in children:
                     if stream_cb is not None:
                         stream_cb(c.parent_prompt, c.cand_index,

@@ -84,6 +84,16 @@ class KVCachePool:
         self.key[:, dst].copy_(self.key[:, src])
         self.value[:, dst].copy_(self.value[:, src])
 
+    def copy_to(self, src: int, dsts: List[int]) -> None:
+        """copy_block to each of dsts, as one launch on the GPU."""
+        if self.key.is_cuda:
+            from ..ops.functional import _require_ext
+            ext = _require_ext("kv_copy_page")
+            if ext is not None and ext.kv_copy_page(self.key, self.value, src, dsts):
+                return
+        for dst in dsts:
+            self.copy_block(src, dst)
+
     @staticmethod
     def pool_size_bytes(num_blocks: int, num_layers: int, block_size: int,
                         n_kv_heads: int, head_dim: int, dtype: torch.dtype) -> int:

@@ -31,6 +31,7 @@ torch::Tensor paged_attention_decode_strided(
     torch::Tensor q, int64_t n_heads, int64_t head_dim, int64_t q_row_stride,
     torch::Tensor kcache, torch::Tensor vcache, torch::Tensor block_tables,
     torch::Tensor ctx_lens, double scale);
+bool kv_copy_page(torch::Tensor key, torch::Tensor value, int64_t src, std::vector<int64_t> dst);
 void kv_cache_scatter(torch::Tensor k, torch::Tensor v,
                       torch::Tensor key_cache, torch::Tensor value_cache,
                       torch::Tensor slot_mapping);
@@ -204,6 +205,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "paged GQA decode attention (packed-q rows)");
   m.def("prefill_attention", &prefill_attention,
         "varlen causal prefill attention (prompt phase)");
+  m.def("kv_copy_page", &kv_copy_page, "copies of a page of all layers");
   m.def("kv_cache_scatter", &kv_cache_scatter, "paged KV cache scatter");
   m.def("paged_attention_decode", &paged_attention_decode,
         "paged GQA decode attention");

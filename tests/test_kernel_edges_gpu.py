@@ -678,6 +678,27 @@ def test_skinny_gemm_operands_anywhere(ext):
             assert torch.equal(ext.skinny_gemm(mode=mode, eps=1e-6, **args), ref), name
 
 
+@pytest.mark.parametrize("n", [1, 60, 61, 125])
+@pytest.mark.parametrize("page,dtype", [((16, 4, 128), torch.bfloat16), ((1, 1, 8), torch.bfloat16),
+                                        ((5, 3, 20), torch.float32), ((1, 1, 4), torch.bfloat16)])
+def test_page_copies(n, page, dtype):
+    """One page of every layer to n others, past what one launch takes; a page of 8 bytes,
+    which is copied by torch."""
+    from distrl_llm_amd.engine.kvcache import KVCachePool
+    pool = KVCachePool(3, 130, *page, dtype, "cuda")
+    pool.key.normal_()
+    pool.value.normal_()
+    want = pool.key.clone(), pool.value.clone()
+    dsts = [d for d in torch.randperm(130, generator=torch.Generator().manual_seed(n)).tolist() if d != 7][:n]
+    for t in want:
+        t[:, dsts] = t[:, 7:8]
+    pool.copy_to(7, dsts)
+    assert torch.equal(pool.key, want[0]) and torch.equal(pool.value, want[1])
+    if page != (1, 1, 4):
+        with pytest.raises(RuntimeError, match="no such page"):
+            pool.copy_to(7, [130])
+
+
 @pytest.mark.parametrize("D,H,KV", [(64, 3, 1), (128, 28, 4)])
 def test_rope_scatter_norms(ext, D, H, KV):
     """Per-head norms, rotation and cache write of packed projections, a
