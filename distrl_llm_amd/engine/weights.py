@@ -10,8 +10,8 @@ and lays the projections of a site (q|k|v, gate|up) out as one matrix, in the
 tiles that the decode products read (ops/csrc/skinny_gemm.hip up to 16 rows,
 stream_gemm.hip up to 160); row-major beside them only for what still goes to
 the library: larger steps, and prompts whose operands our products don't take. A refresh
-writes each projection's merged weight straight into its tiles, one kernel a
-projection, once per generation round.
+writes the projections' merged weights straight into their tiles, one kernel a
+layer, once per generation round.
 
 Replaces the reference's per-generate adapter hot-swap into vLLM
 (``load_lora`` inside every fast_generate, reference
@@ -164,21 +164,35 @@ def _merge_into(mod, out: torch.Tensor) -> None:
     out.copy_(_effective(mod))
 
 
-def _merge_tiles(mods, out: torch.Tensor, glu: bool, adapters: bool = True) -> None:
-    """out, in tiles <- the modules' weights one below the other (glu: a
-    SiLU*mul pair), with their adapters or without."""
-    from ..ops.functional import _require_ext
-    ext, row = _require_ext("decode weights"), 0
+def _tile_jobs(mods, out: torch.Tensor, glu: bool, adapters: bool):
+    """What brings the modules' weights, one below the other (glu: a SiLU*mul
+    pair), with their adapters or without, into out's tiles."""
+    row = 0
     for m in mods:
-        ab = ((m.lora_A.detach(), m.lora_B.detach(), float(m.scale))
-              if adapters and m.r > 0 else ())
-        w = m.weight.detach()
-        if ({t.dtype for t in (w, *ab[:2])} != {torch.bfloat16}
-                or not ext.weight_tiles(w, out, row, glu, *ab)):
+        a, b = ((m.lora_A.detach(), m.lora_B.detach())
+                if adapters and m.r > 0 else (None, None))
+        yield m.weight.detach(), out, row, glu, a, b, float(m.scale)
+        row += 16 if glu else m.out_features
+
+
+def _merge_tiles(sites) -> None:
+    """Of each site (modules, out, glu, adapters): out, in tiles <- its weights."""
+    from ..ops.functional import _require_ext
+    ext = _require_ext("decode weights")
+
+    def native(sites) -> bool:
+        jobs = [job for site in sites for job in _tile_jobs(*site)]
+        types = {t.dtype for w, _, _, _, a, b, _ in jobs
+                 for t in (w, a, b) if t is not None}
+        return types == {torch.bfloat16} and ext.weights_tiles(*map(list, zip(*jobs)))
+
+    if native(sites):
+        return
+    for site in sites:
+        if not native([site]):
+            mods, out, glu, adapters = site
             out.copy_(_tiled(torch.cat(
                 [_effective(m) if adapters else m.weight for m in mods]), glu))
-            return
-        row += 16 if glu else m.out_features
 
 
 def _room_for(size: int, device) -> bool:
@@ -415,7 +429,7 @@ class FusedWeights:
                     sum(m.out_features for m in mods), mods[0].in_features)
                 for site, mods in lw.mods.items()}
             lw.down_apart = self.hybrid_down and self.lora_r > 0
-        for site, mods in lw.mods.items():
-            # IN PLACE: captured decode steps hold these storages
-            _merge_tiles(mods, lw.tiles[site], site == "gateup",
-                         not (site == "down" and lw.down_apart))
+        # IN PLACE: captured decode steps hold these storages
+        _merge_tiles([(mods, lw.tiles[site], site == "gateup",
+                       not (site == "down" and lw.down_apart))
+                      for site, mods in lw.mods.items()])

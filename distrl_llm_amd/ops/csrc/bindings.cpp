@@ -66,6 +66,10 @@ bool stream_gemm_takes(int64_t M, int64_t N, int64_t K);
 torch::Tensor stream_glu(torch::Tensor x, torch::Tensor w);
 torch::Tensor stream_gemm(torch::Tensor x, torch::Tensor w,
                           c10::optional<torch::Tensor> w2);
+bool weights_tiles(std::vector<torch::Tensor> w, std::vector<torch::Tensor> out,
+                   std::vector<int64_t> row, std::vector<bool> glu,
+                   std::vector<c10::optional<torch::Tensor>> a,
+                   std::vector<c10::optional<torch::Tensor>> b, std::vector<double> scale);
 bool weight_tiles(torch::Tensor w, torch::Tensor out, int64_t row, bool glu,
                   c10::optional<torch::Tensor> a,
                   c10::optional<torch::Tensor> b, double scale);
@@ -237,6 +241,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("stream_gemm", &stream_gemm,
         "fp32 partial sums of x [w; w2]^T, W in tiles", py::arg("x"),
         py::arg("w"), py::arg("w2") = py::none());
+  m.def("weights_tiles", &weights_tiles, "weight_tiles of several weights, one launch for eight");
   m.def("weight_tiles", &weight_tiles,
         "rows of W (+ scale * B A) into tiles; false: not these operands",
         py::arg("w"), py::arg("out"), py::arg("row"), py::arg("glu"),

@@ -40,18 +40,17 @@ constexpr int STEPS = KC / 32;     // loads of W in flight
 // for all). TA: a is (K, r). TILES: out in tiles of 32 rows x 16 of K, [K half][row][8
 // elements], row n of w at row + n of out, or (glu) at row + n in blocks of 16 of
 // every 32; r may be 0.
-template <bool TA, bool TILES = false, typename W = __hip_bfloat16>
-__global__ __launch_bounds__(256)
-void lora_merge_kernel(const W* w, const __hip_bfloat16* __restrict__ a,
-                       const __hip_bfloat16* __restrict__ b, const __hip_bfloat16* __restrict__ res,
-                       __hip_bfloat16* out, int N, int K, int r, int rows, int64_t ldw, int64_t ldo,
-                       int ldb, int64_t ldr, float scale, int row0, int glu) {
+template <bool TA, bool TILES, typename W>
+DEV_INLINE void merge(const W* w, const __hip_bfloat16* __restrict__ a,
+                      const __hip_bfloat16* __restrict__ b, const __hip_bfloat16* __restrict__ res,
+                      __hip_bfloat16* out, int N, int K, int r, int rows, int64_t ldw, int64_t ldo,
+                      int ldb, int64_t ldr, float scale, int row0, int glu, int bx, int by) {
   typedef __attribute__((ext_vector_type(8))) float f32x8;
   typedef std::conditional_t<std::is_same_v<W, float>, f32x8, bf16v8> WV;
   // A: [r32][KC], TA: [KC][r32], rows 16 B apart
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int RS = KC * 2 + 16;
-  const int k0 = blockIdx.x * KC, r32 = (r + 31) / 32 * 32;
+  const int k0 = bx * KC, r32 = (r + 31) / 32 * 32;
   const int ts = r32 * 2 + 16;
   for (int i = threadIdx.x; i < r32 * (KC / 8); i += 256) {
     const int row = TA ? i / (r32 / 8) : i / (KC / 8), c = TA ? i % (r32 / 8) : i % (KC / 8);
@@ -66,8 +65,8 @@ void lora_merge_kernel(const W* w, const __hip_bfloat16* __restrict__ a,
   __syncthreads();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63, g = l >> 4, lr = l & 15;
-  const int end = min(N, (int)(blockIdx.y + 1) * rows);
-  for (int n0 = blockIdx.y * rows + wave * 16; n0 < end; n0 += 64) {
+  const int end = min(N, (by + 1) * rows);
+  for (int n0 = by * rows + wave * 16; n0 < end; n0 += 64) {
     const W* wrow = w + min(n0 + lr, N - 1) * ldw + g * 8;
     const __hip_bfloat16* brow = b + (int64_t)min(n0 + lr, N - 1) * ldb;
     WV wv[STEPS];
@@ -129,6 +128,45 @@ void lora_merge_kernel(const W* w, const __hip_bfloat16* __restrict__ a,
   }
 }
 
+template <bool TA, typename W = __hip_bfloat16>
+__global__ __launch_bounds__(256)
+void lora_merge_kernel(const W* w, const __hip_bfloat16* __restrict__ a,
+                       const __hip_bfloat16* __restrict__ b, const __hip_bfloat16* __restrict__ res,
+                       __hip_bfloat16* out, int N, int K, int r, int rows, int64_t ldw, int64_t ldo,
+                       int ldb, int64_t ldr, float scale) {
+  merge<TA, false, W>(w, a, b, res, out, N, K, r, rows, ldw, ldo, ldb, ldr, scale, 0, 0, blockIdx.x,
+                      blockIdx.y);
+}
+
+// Weights into tiles, several of them a launch: a layer's seven. A launch each left the
+// chip idle in between, where the host was the slower (0.5B, 168 of 6 us), and behind
+// the small ones (7B, of 7 to 70 us). Whole calls, their fan-out in one launch a prompt
+// in both: 160 candidates of the 7B model 167.0 -> 162.7 ms, 32 of the 4B 79.3 -> 78.3,
+// one of the 0.5B 35.7 -> 35.3.
+constexpr int JOBS = 8;
+
+struct Job {
+  const __hip_bfloat16 *w, *a, *b;
+  __hip_bfloat16* out;
+  int64_t ldw;
+  int N, K, r, rows, ldb, row0, glu, first;    // first: of the launch's workgroups
+  float scale;
+};
+struct Jobs {
+  Job job[JOBS];
+  int n;
+};
+
+__global__ __launch_bounds__(256)
+void weight_tiles_kernel(const Jobs jobs) {
+  int i = 0;
+  while (i + 1 < jobs.n && (int)blockIdx.x >= jobs.job[i + 1].first) ++i;
+  const Job& j = jobs.job[i];
+  const int at = blockIdx.x - j.first, wide = CDIV(j.K, KC);
+  merge<false, true, __hip_bfloat16>(j.w, j.a, j.b, nullptr, j.out, j.N, j.K, j.r, j.rows, j.ldw, j.K,
+                                     j.ldb, 0, j.scale, j.row0, j.glu, at % wide, at / wide);
+}
+
 }  // namespace
 
 static bool lora_merge_takes(int64_t K, int64_t r) { return K % 32 == 0 && r % 8 == 0 && r >= 8 && r <= 128; }
@@ -172,12 +210,12 @@ bool launch_merge(const torch::Tensor& w, const torch::Tensor& a, const torch::T
                        res ? lptr(*res) : nullptr,
                        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), N, K, r, rows,
                        w.stride(0), out.stride(0), (int)b.stride(0), res ? res->stride(0) : 0,
-                       (float)scale, 0, 0);
+                       (float)scale);
   };
   if (sums) {
     const float* p = w.data_ptr<float>();
-    if (ta) go(lora_merge_kernel<true, false, float>, p);
-    else go(lora_merge_kernel<false, false, float>, p);
+    if (ta) go(lora_merge_kernel<true, float>, p);
+    else go(lora_merge_kernel<false, float>, p);
   } else if (ta) {
     go(lora_merge_kernel<true>, lptr(w));
   } else {
@@ -195,11 +233,12 @@ bool lora_merge(torch::Tensor w, torch::Tensor a, torch::Tensor b, torch::Tensor
   return launch_merge(w, a, b, out, false, scale);
 }
 
-// Rows row .. of a weight in tiles (out: (rows, K), K % 32 == 0, see the kernel)
-// <- w, or w + scale * b a. glu: w is gate (row 0) or up (row 16) of a SiLU*mul
-// pair. False, and nothing done, for operands that 16 B accesses can't take.
-bool weight_tiles(torch::Tensor w, torch::Tensor out, int64_t row, bool glu,
-                  c10::optional<torch::Tensor> a, c10::optional<torch::Tensor> b, double scale) {
+namespace {
+
+// Job into `to`; false for operands that 16 B accesses can't take.
+bool tiles_job(Job& to, const torch::Tensor& w, const torch::Tensor& out, int64_t row, bool glu,
+               const c10::optional<torch::Tensor>& a, const c10::optional<torch::Tensor>& b,
+               double scale) {
   TORCH_CHECK(out.is_cuda() && out.is_contiguous() && out.dim() == 2 &&
               out.scalar_type() == at::kBFloat16 && out.size(0) % 32 == 0);
   if (w.dim() != 2 || !lrows(w) || w.size(1) != out.size(1) || w.size(1) % 32 != 0) return false;
@@ -217,16 +256,58 @@ bool weight_tiles(torch::Tensor w, torch::Tensor out, int64_t row, bool glu,
     TORCH_CHECK(a->size(1) == K && b->size(0) == N && b->size(1) == r, "weight_tiles: adapter");
     if (!lora_merge_takes(K, r)) return false;
   }
-  if (N == 0) return true;
   const int rows = (int64_t)CDIV(K, KC) * CDIV(N, 64) >= 4096 ? 256 : 64;
-  const int smem = CDIV(r, 32) * 32 * (KC * 2 + 16);
-  hipLaunchKernelGGL((lora_merge_kernel<false, true>), dim3(CDIV(K, KC), CDIV(N, rows)), dim3(256),
-                     smem, at::cuda::getCurrentCUDAStream(), lptr(w), r ? lptr(*a) : nullptr,
-                     r ? lptr(*b) : nullptr, nullptr,
-                     reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), N, K, r, rows, w.stride(0),
-                     (int64_t)K, r ? (int)b->stride(0) : 0, (int64_t)0, (float)scale, (int)row,
-                     (int)glu);
+  to = {lptr(w), r ? lptr(*a) : nullptr, r ? lptr(*b) : nullptr,
+        reinterpret_cast<__hip_bfloat16*>(out.data_ptr()), w.stride(0), N, K, r, rows,
+        r ? (int)b->stride(0) : 0, (int)row, (int)glu, 0, (float)scale};
+  return true;
+}
+
+void launch_tiles(Jobs& jobs) {
+  int64_t blocks = 0;
+  int r32 = 0;
+  for (int i = 0; i < jobs.n; ++i) {
+    Job& j = jobs.job[i];
+    j.first = (int)blocks;
+    blocks += (int64_t)CDIV(j.K, KC) * CDIV(j.N, j.rows);
+    r32 = std::max(r32, CDIV(j.r, 32) * 32);
+  }
+  if (blocks == 0) return;
+  TORCH_CHECK(blocks < (1 << 30), "weight_tiles: size");
+  hipLaunchKernelGGL(weight_tiles_kernel, dim3(blocks), dim3(256), r32 * (KC * 2 + 16),
+                     at::cuda::getCurrentCUDAStream(), jobs);
   HIP_CHECK_LAST();
+}
+
+}  // namespace
+
+// Rows row .. of a weight in tiles (out: (rows, K), K % 32 == 0, see the kernel)
+// <- w, or w + scale * b a. glu: w is gate (row 0) or up (row 16) of a SiLU*mul
+// pair. False, and nothing done, for operands that 16 B accesses can't take.
+bool weight_tiles(torch::Tensor w, torch::Tensor out, int64_t row, bool glu,
+                  c10::optional<torch::Tensor> a, c10::optional<torch::Tensor> b, double scale) {
+  Jobs jobs;
+  jobs.n = 1;
+  if (!tiles_job(jobs.job[0], w, out, row, glu, a, b, scale)) return false;
+  launch_tiles(jobs);
+  return true;
+}
+
+// The same for several weights; false, and nothing done, where one can't be taken.
+bool weights_tiles(std::vector<torch::Tensor> w, std::vector<torch::Tensor> out,
+                   std::vector<int64_t> row, std::vector<bool> glu,
+                   std::vector<c10::optional<torch::Tensor>> a,
+                   std::vector<c10::optional<torch::Tensor>> b, std::vector<double> scale) {
+  const size_t n = w.size();
+  TORCH_CHECK(out.size() == n && row.size() == n && glu.size() == n && a.size() == n &&
+              b.size() == n && scale.size() == n, "weight_tiles: lists");
+  std::vector<Jobs> all(CDIV(n, JOBS));
+  for (size_t i = 0; i < n; ++i) {
+    Jobs& to = all[i / JOBS];
+    to.n = (int)(i % JOBS) + 1;
+    if (!tiles_job(to.job[i % JOBS], w[i], out[i], row[i], glu[i], a[i], b[i], scale[i])) return false;
+  }
+  for (auto& jobs : all) launch_tiles(jobs);
   return true;
 }
 

@@ -56,6 +56,27 @@ def test_weight_tiles(ext, N1, N2, K, r):
     assert not ext.weight_tiles(_rand((N1, K + 2), 1)[:, 1:K + 1], out, 0, False)
 
 
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 17])
+def test_weights_tiles(ext, n):
+    """Weights of several shapes and ranks a launch, as one a launch; one that is refused
+    leaves all as they were."""
+    shapes = [((32, 32, 0), (256, 1056, 8), (64, 288, 128), (96, 1280, 40))[i % 4] for i in range(n)]
+    ws = [_rand((N, K), i) for i, (N, K, _) in enumerate(shapes)]
+    a = [_rand((r, K), 30 + i, 0.1) if r else None for i, (_, K, r) in enumerate(shapes)]
+    b = [_rand((N, r), 60 + i, 0.1) if r else None for i, (N, _, r) in enumerate(shapes)]
+    glu, scale = [i % 3 == 2 for i in range(n)], [0.5 + i for i in range(n)]
+    outs = [torch.full((N * (2 if g else 1) + 32, K), 3.0, dtype=torch.bfloat16, device="cuda")[:-32]
+            for (N, K, _), g in zip(shapes, glu)]
+    row, want = [16 if g else 0 for g in glu], [o.clone() for o in outs]
+    for i in range(n):
+        assert ext.weight_tiles(ws[i], want[i], row[i], glu[i], a[i], b[i], scale[i])
+    refused = ws[:-1] + [_rand((shapes[-1][0], shapes[-1][1] + 2), 1)[:, 1:-1]]
+    assert not ext.weights_tiles(refused, outs, row, glu, a, b, scale)
+    assert all(bool((o == 3).all()) for o in outs)
+    assert ext.weights_tiles(ws, outs, row, glu, a, b, scale)
+    assert all(torch.equal(o, w) for o, w in zip(outs, want))
+
+
 @pytest.mark.parametrize("M", [1, 17, 32, 33, 96, 128, 129, 160])
 @pytest.mark.parametrize("N,K", [(32, 64), (96, 192), (1152, 896), (2048, 1536), (160, 8960)])
 def test_stream_gemm(ext, M, N, K):
