@@ -191,7 +191,11 @@ struct Slice {
 };
 
 // Gathers what the lanes of a wave keep of their elements, two chunks at a time, and
-// hands it on 64 at a time: f(element of the slice, value), a lane each.
+// hands it on 64 at a time: f(element of the slice, value), a lane each. An element's
+// ballot says where each lane's goes; a chunk of which none is kept costs its maximum
+// alone. Against counts of each lane's, a prefix sum over the wave and a second look, us:
+// 160 rows of 152064, top_p 0.95 47.3 -> 45.8, no threshold 55.1 -> 51.3, 135 fp32 rows
+// 58.9 -> 51.6, 84 rows top_k 50 26.6 -> 24.5, one row 9.16 -> 8.81, 4 to 27 rows level.
 template <typename T, bool VEC>
 struct Gather {
   using Entry = std::conditional_t<Slice<T, VEC>::BF16, uint32_t, unsigned long long>;
@@ -207,42 +211,33 @@ struct Gather {
     else
       f((int)(e >> 32), __uint_as_float((uint32_t)e));
   }
-  // Every lane of the wave calls it; keep(value).
+  // Every lane of the wave calls it; keep(value), which keeps what lies above some value.
   template <typename K, typename F>
   DEV_INLINE void run(const Slice<T, VEC>& s, int n, K keep, F f) {
     const int lane = threadIdx.x & (WAVE - 1);
     #pragma unroll
     for (int c0 = 0; c0 < CHUNKS; c0 += 2) {
       if (c0 * CHUNK >= n) continue;
-      const int two = (c0 + 1) * CHUNK < n ? 2 : 1;
-      int mine = 0;
       #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        if (c >= two) continue;
+      for (int c = c0; c < c0 + 2; ++c) {
+        if (c * CHUNK >= n) continue;
+        float top = -1e30f;
         #pragma unroll
-        for (int k = 0; k < 8; ++k) mine += keep(s.get(c0 + c, k)) ? 1 : 0;
-      }
-      if (__ballot(mine > 0) == 0) continue;
-      int upto = mine;
-      #pragma unroll
-      for (int off = 1; off < WAVE; off <<= 1) {
-        const int y = __shfl_up(upto, off, WAVE);
-        if (lane >= off) upto += y;
-      }
-      int to = count + upto - mine;
-      count += __shfl(upto, WAVE - 1, WAVE);
-      #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        if (c >= two) continue;
+        for (int k = 0; k < 8; ++k) top = fmaxf(top, s.get(c, k));
+        if (__ballot(keep(top)) == 0) continue;
         #pragma unroll
         for (int k = 0; k < 8; ++k) {
-          const float x = s.get(c0 + c, k);
-          if (keep(x)) {
-            const uint32_t id = s.at(c0 + c, k), bits = __float_as_uint(x);
-            if constexpr (Slice<T, VEC>::BF16) q[to] = bits | id;     // SLICE < 2^16
+          const float x = s.get(c, k);
+          const bool kept = keep(x);
+          const unsigned long long who = __ballot(kept);
+          if (kept) {
+            const int to = count + __builtin_amdgcn_mbcnt_hi((uint32_t)(who >> 32),
+                                       __builtin_amdgcn_mbcnt_lo((uint32_t)who, 0));
+            const uint32_t id = s.at(c, k), bits = __float_as_uint(x);
+            if constexpr (Slice<T, VEC>::BF16) q[to] = bits | id;       // SLICE < 2^16
             else q[to] = ((unsigned long long)id << 32) | bits;
-            ++to;
           }
+          count += __popcll(who);
         }
       }
       __builtin_amdgcn_wave_barrier();

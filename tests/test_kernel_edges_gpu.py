@@ -678,6 +678,21 @@ def test_skinny_gemm_operands_anywhere(ext):
             assert torch.equal(ext.skinny_gemm(mode=mode, eps=1e-6, **args), ref), name
 
 
+@pytest.mark.parametrize("V,dtype", [(24000, torch.bfloat16), (20481, torch.float32), (4100, torch.bfloat16)])
+@pytest.mark.parametrize("top_p,top_k", [(1.0, 0), (0.5, 0), (1.0, 1)])
+def test_draws_at_chunk_edges(ext, V, dtype, top_p, top_k):
+    """The one likely element of each of 700 rows, which are slices of up to ten chunks,
+    at the edges of threads' pieces and of chunks, where nearly all of them keep none."""
+    places = [p for e in range(0, V, 2048) for p in (e - 1, e, e + 7, e + 8, e + 511) if 0 <= p < V] + [V - 1]
+    at = torch.tensor([places[i % len(places)] for i in range(700)], device="cuda")
+    logits = torch.zeros(700, V, dtype=dtype, device="cuda")
+    logits.scatter_(1, at[:, None], 40.0)
+    for seed in range(3):
+        seeds = torch.arange(700, device="cuda") + 1000 * seed
+        step = torch.tensor([seed], device="cuda")
+        assert torch.equal(ext.sample_tokens(logits, 1.0, top_p, top_k, seeds, step), at)
+
+
 @pytest.mark.parametrize("n", [1, 60, 61, 125])
 @pytest.mark.parametrize("page,dtype", [((16, 4, 128), torch.bfloat16), ((1, 1, 8), torch.bfloat16),
                                         ((5, 3, 20), torch.float32), ((1, 1, 4), torch.bfloat16)])
