@@ -684,10 +684,11 @@ bool product_glu_bwd(const ProductBlock& block, const at::Tensor& gu, const at::
   return true;
 }
 
-// g w, g (M, V), w (V, N): own products where they take them, else the library's.
+// g w, g (M, V), w (V, N): own products for vocabularies of models in use, else the
+// library's (500 x 1024 x 32768 67 us here, 147 there; smaller ones not measured).
 at::Tensor product_rows(const at::Tensor& g, const at::Tensor& w) {
   auto out = at::empty({g.size(0), w.size(1)}, g.options());
-  if (g.size(0) > 0 && product({{w.size(1), {{g, w}}, {}}}, true, out)) return out;
+  if (g.size(0) > 0 && g.size(1) >= 32768 && product({{w.size(1), {{g, w}}, {}}}, true, out)) return out;
   return at::mm(g, w);
 }
 

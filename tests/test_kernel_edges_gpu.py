@@ -1146,10 +1146,11 @@ def test_logprob_rows(ext, rows, V):
     assert _rel(grad, ref) < 2.0 ** -8
 
 
-@pytest.mark.parametrize("rows,V", [(5, 8), (3, 4096), (700, 4104), (2, 16384), (9, 16391), (530, 32768),
-                                    (3, 65544), (2, 131079), (259, 155648), (2, 155656)])
+@pytest.mark.parametrize("rows,V", [(5, 8), (131073, 8), (255, 4096), (256, 4096), (700, 4104), (65, 16384),
+                                    (64, 16391), (530, 32768), (17, 65544), (17, 62000), (9, 131079),
+                                    (9, 131072), (259, 155648), (9, 155656)])
 def test_loss_gradients_made_forward(ext, rows, V):
-    """Rows at the edges of what is held in registers, and rows beyond: one backward,
+    """Rows at the edges of what is held in registers, rows beyond and few rows: one backward,
     those behind it in a kept graph (what the first gave out is overwritten) and one
     that is scaled give what the two passes apart do, up to the log-sum-exp's rounding
     (some 1e-6, which moves few values over a bf16 rounding edge)."""
