@@ -30,7 +30,7 @@
 // 160 rows of 151936, us, against four launches that each read all logits: top_p 0.95 of
 // peaked logits 84 -> 47, of a language model's 79 -> 38, of flat ones, where most is
 // drawn, 102 -> 102; top_k 50 75 -> 41; no threshold, a model's logits 40 -> 22. One row
-// without a threshold 11.3 -> 9.5. Bound by vector work: ~14 instructions an element for
+// without a threshold 11.3 -> 8.8. Bound by vector work: ~14 instructions an element for
 // the steps (20 us), then the hash of what lies above the window's end.
 #include <torch/extension.h>
 #include <ATen/cuda/CUDAContext.h>
