@@ -116,7 +116,7 @@ void logprob_lse_kernel(const T* __restrict__ logits,
   }
 }
 
-// Row weights and the loss itself: w[b, t] = mask * coef_b with
+// Row weights (where w is given) and the loss itself: w[b, t] = mask * coef_b with
 // coef_b = -reward_b / max(sum mask, 1) / B * scale, loss = sum w * token_logp.
 // One wave a sequence and turn.
 template <typename M>
@@ -136,7 +136,8 @@ void loss_reduce_kernel(const float* __restrict__ token_logp, const M* __restric
       sum += token_logp[at + t] * k;
     }
     const float coef = -rewards[b] / fmaxf(wave_sum(n), 1.f) / B * scale;
-    for (int t = lane; t < T; t += WAVE) w[at + t] = (float)mask[at + t] * coef;
+    if (w)
+      for (int t = lane; t < T; t += WAVE) w[at + t] = (float)mask[at + t] * coef;
     total += wave_sum(sum) * coef;
   }
   if (lane == 0) part[wave] = total;
@@ -146,6 +147,22 @@ void loss_reduce_kernel(const float* __restrict__ token_logp, const M* __restric
     for (int i = 0; i < 16; ++i) sum += part[i];
     *loss = sum;
   }
+}
+
+// The row weights alone, before a pass over logits that makes the gradient at once, whose
+// every row would else read its sequence's whole mask: 1 x 32768 rows of 4096 1041 us, so
+// 319 (396 in two passes), 1 x 16384 of 4096 343, 127 (174), 8 x 301 of 152064 325, 323.
+// A workgroup a sequence.
+template <typename M>
+__global__ __launch_bounds__(1024)
+void loss_weights_kernel(const M* __restrict__ mask, const float* __restrict__ rewards,
+                         float* __restrict__ w, int B, int T, float scale) {
+  __shared__ float red[16];
+  const int64_t at = (int64_t)blockIdx.x * T;
+  float n = 0.f;
+  for (int t = threadIdx.x; t < T; t += 1024) n += (float)mask[at + t];
+  const float coef = -rewards[blockIdx.x] / fmaxf(block_sum(n, red), 1.f) / B * scale;
+  for (int t = threadIdx.x; t < T; t += 1024) w[at + t] = (float)mask[at + t] * coef;
 }
 
 // sum of w * token_logp over rows, in an order of its own for every row count
@@ -254,24 +271,15 @@ void loss_anew_kernel(const T* __restrict__ logits, const int64_t* __restrict__ 
 // their way all the time. Bound by memory: 2408 rows of 152064, a quarter of weight zero,
 // 308 us (4.75 TB/s read and written), 133 and 222 in two passes; with the sum over rows
 // and the look at dloss 356 -> 320. Loads or stores through or past the caches are even.
-struct RowWeights {
-  const float* w;             // of each row, or
-  const void* mask;           // (B, T), int64 or fp32, and rewards as the loss has them
-  bool mask64;
-  const float* rewards;
-  int B, T;
-  float scale;
-};
-
 template <int THREADS, int KEEP>
 __global__ __launch_bounds__(THREADS)
 void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* __restrict__ targets,
-                      RowWeights weights, float* __restrict__ token_logp,
+                      const float* __restrict__ w, float* __restrict__ token_logp,
                       float* __restrict__ lse_out, __hip_bfloat16* __restrict__ dlogits, int rows,
                       int V) {
   constexpr float LOG2E = 1.4426950408889634f;
   constexpr int NW = THREADS / WAVE;
-  __shared__ float part[2][3][NW];
+  __shared__ float part[2][2][NW];
   const int tid = threadIdx.x, lane = tid & (WAVE - 1), nvec = V / 8;
   u32x4 v[KEEP];
   // One offset that walks a row, as 19 addresses would take the registers: what lies past
@@ -298,15 +306,7 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
     const __hip_bfloat16* lr = logits + row * V;
     __hip_bfloat16* dr = dlogits + row * V;
     const int64_t tgt = targets[row];
-    // the sequence's mask, summed beside the logits
-    float share = 0.f;
-    const int64_t seq = weights.w ? 0 : row / weights.T;
-    auto mask = [&](int64_t i) {
-      return weights.mask64 ? (float)reinterpret_cast<const int64_t*>(weights.mask)[i]
-                            : reinterpret_cast<const float*>(weights.mask)[i];
-    };
-    if (!weights.w)
-      for (int t = tid; t < weights.T; t += THREADS) share += mask(seq * weights.T + t);
+    const float wv = w[row];
     const int at = nvec * 8 + tid;                        // of the last few
     const float tail = at < V ? ld(lr, at) : -__builtin_inff();
 
@@ -338,29 +338,22 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
     // over the workgroup: one meeting a row, in turns of LDS
     const float M = wave_max(m);
     s = wave_sum(s * __builtin_amdgcn_exp2f((m - M) * LOG2E));
-    share = wave_sum(share);
     if (lane == 0) {
       part[turn][0][tid / WAVE] = M;
       part[turn][1][tid / WAVE] = s;
-      part[turn][2][tid / WAVE] = share;
     }
     __syncthreads();
     // a wave's lanes take a wave each, in every wave
     const int of = lane & (NW - 1);
-    float top = part[turn][0][of], sum = part[turn][1][of], n = part[turn][2][of];
+    float top = part[turn][0][of], sum = part[turn][1][of];
     float high = top;
     #pragma unroll
     for (int off = NW / 2; off > 0; off >>= 1) high = fmaxf(high, __shfl_xor(high, off, WAVE));
     sum *= __builtin_amdgcn_exp2f((top - high) * LOG2E);
     #pragma unroll
-    for (int off = NW / 2; off > 0; off >>= 1) {
-      sum += __shfl_xor(sum, off, WAVE);
-      n += __shfl_xor(n, off, WAVE);
-    }
+    for (int off = NW / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, WAVE);
     top = high;
     const float l = top + __logf(sum);
-    const float wv = weights.w ? weights.w[row]
-                               : mask(row) * (-weights.rewards[seq] / fmaxf(n, 1.f) / weights.B * weights.scale);
     if (tid == 0) lse_out[row] = l;
     if (tid == 0 && (tgt < 0 || tgt >= V)) token_logp[row] = 0.f - l;
     if (at < V) {
@@ -449,7 +442,7 @@ static bool takes_both(const torch::Tensor& logits) {
 // {token_logp, lse, the gradient for a dloss of 1}
 static std::vector<torch::Tensor> logprob_both(const torch::Tensor& logits,
                                                const torch::Tensor& targets,
-                                               const RowWeights& weights) {
+                                               const torch::Tensor& w) {
   TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() && takes_both(logits));
   TORCH_CHECK(targets.scalar_type() == at::kLong && targets.is_contiguous());
   const int V = logits.size(-1), nvec = V / 8;
@@ -465,7 +458,7 @@ static std::vector<torch::Tensor> logprob_both(const torch::Tensor& logits,
     hipLaunchKernelGGL((loss_both_kernel<THREADS, KEEP>), dim3(std::min(rows, 256 * per_cu)),
                        dim3(THREADS), 0, at::cuda::getCurrentCUDAStream(),
                        reinterpret_cast<const __hip_bfloat16*>(logits.data_ptr()),
-                       targets.data_ptr<int64_t>(), weights, token_logp.data_ptr<float>(),
+                       targets.data_ptr<int64_t>(), w.data_ptr<float>(), token_logp.data_ptr<float>(),
                        lse.data_ptr<float>(), reinterpret_cast<__hip_bfloat16*>(grad.data_ptr()),
                        rows, V);
   };
@@ -494,17 +487,21 @@ static std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits, torch::
               rewards.scalar_type() == at::kFloat);
   const bool mask64 = mask.scalar_type() == at::kLong;
   TORCH_CHECK(mask64 || mask.scalar_type() == at::kFloat);
-  auto lp = both ? logprob_both(logits, targets,
-                                {nullptr, mask.data_ptr(), mask64, rewards.data_ptr<float>(), B, T,
-                                 (float)scale})
-                 : logprob_lse_fwd(logits, targets);
-  auto w = torch::empty_like(lp[0]);
-  auto loss = torch::empty({}, lp[0].options());
   auto stream = at::cuda::getCurrentCUDAStream();
+  auto w = torch::empty({B, T}, logits.options().dtype(at::kFloat));
+  auto loss = torch::empty({}, w.options());
+  #define WEIGHTS(M)                                                                  \
+    hipLaunchKernelGGL(loss_weights_kernel<M>, dim3(B), dim3(1024), 0, stream,        \
+                       mask.data_ptr<M>(), rewards.data_ptr<float>(),                 \
+                       w.data_ptr<float>(), B, T, (float)scale)
+  if (both && mask64) WEIGHTS(int64_t);
+  else if (both) WEIGHTS(float);
+  #undef WEIGHTS
+  auto lp = both ? logprob_both(logits, targets, w) : logprob_lse_fwd(logits, targets);
   #define REDUCE(M)                                                                   \
     hipLaunchKernelGGL(loss_reduce_kernel<M>, dim3(1), dim3(1024), 0, stream,         \
                        lp[0].data_ptr<float>(), mask.data_ptr<M>(),                   \
-                       rewards.data_ptr<float>(), w.data_ptr<float>(),                \
+                       rewards.data_ptr<float>(), both ? nullptr : w.data_ptr<float>(), \
                        loss.data_ptr<float>(), B, T, (float)scale)
   if (mask64) REDUCE(int64_t);
   else REDUCE(float);
@@ -624,8 +621,7 @@ struct LogprobRows : public torch::autograd::Function<LogprobRows> {
     logits = logits.contiguous();
     targets = targets.contiguous();
     w = w.contiguous();
-    auto lp = both ? logprob_both(logits, targets, {w.data_ptr<float>()})
-                   : logprob_lse_fwd(logits, targets);
+    auto lp = both ? logprob_both(logits, targets, w) : logprob_lse_fwd(logits, targets);
     auto loss = torch::empty({}, lp[0].options());
     hipLaunchKernelGGL(loss_rows_kernel, dim3(1), dim3(1024), 0, at::cuda::getCurrentCUDAStream(),
                        lp[0].data_ptr<float>(), w.data_ptr<float>(), loss.data_ptr<float>(),

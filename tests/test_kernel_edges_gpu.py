@@ -934,6 +934,59 @@ def test_loss_edges(B, T, V, dtype, mask_dtype):
         assert _rel(grad, ref_grad) < (2.0 ** -8 if dtype == "bfloat16" else 1e-5)
 
 
+@pytest.mark.parametrize("B,T,V", [(3, 1300, 301), (1, 20000, 64), (2, 2600, 513), (41, 60, 8192),
+                                   (300, 6, 4097), (2, 150, 40000), (290, 1, 70001), (3, 3, 152065)])
+@pytest.mark.parametrize("mask_dtype", [torch.int64, torch.float32])
+def test_masked_loss_gradients_made_forward(B, T, V, mask_dtype):
+    """Losses large enough for the gradient to be made in the forward pass: an empty mask,
+    parts of a token, more tokens than a workgroup has threads and fewer, rows that walk,
+    of every width class, a target that is no word (its gradient is the softmax alone).
+    What forward made, what is made anew behind it in a kept graph and what is made of a
+    scaled loss. The first two have the same weights: a first token of 2^24 that swallows
+    others' ones makes its sequence's sum hang on the order, and each 2^-24 by which weights
+    differ moves 2^-16 of the values over a bf16 edge. Loss sums in fp32, the gradient
+    rounds to bf16 once."""
+    from distrl_llm_amd.ops import functional as OF
+    g = torch.Generator().manual_seed(V)
+    gd = torch.Generator("cuda").manual_seed(V)
+    leaf = torch.randn(B, T, V, generator=gd, device="cuda").mul_(3).bfloat16()
+    leaf[..., 1] = float("-inf")
+    targets = torch.randint(2, V, (B, T), generator=g).cuda()
+    targets[0, 0] = -100
+    mask = torch.rand(B, T, generator=g).mul_(1.2)
+    mask = (mask if mask_dtype == torch.float32 else mask < 0.8).to(mask_dtype).cuda()
+    if mask_dtype == torch.float32:
+        mask[:, 0] = 2.0 ** 24
+    mask[1:][-1:] = 0
+    rewards = torch.randn(B, generator=g).cuda()
+    leaf.requires_grad_()
+    assert leaf.numel() >= 1 << 20
+    loss = OF.logprob_loss(leaf, targets, mask, rewards, 0.25)
+    first, = torch.autograd.grad(loss, leaf, retain_graph=True)
+    second, = torch.autograd.grad(loss, leaf, retain_graph=True)
+    assert float((first != second).float().mean()) < 2.0 ** -14
+    scaled, = torch.autograd.grad(loss * 3.0, leaf)
+    m = mask.double()
+    w = m * (-rewards.double() / m.sum(-1).clamp_min(1) / B * 0.25)[:, None]
+    tok, bad, size = 0.0, 0.0, 0.0
+    for b in range(B):                                  # fp64 of one sequence at a time
+        logp = leaf[b].detach().double().log_softmax(-1)
+        hot = torch.zeros_like(logp)
+        there = (targets[b] >= 0).nonzero()[:, 0]
+        hot[there, targets[b, there]] = 1.0
+        ref = w[b][:, None] * (hot - logp.exp())
+        lse = leaf[b].detach().double().logsumexp(-1)
+        t = torch.where(targets[b] >= 0, logp.gather(-1, targets[b].clamp_min(0)[:, None])[:, 0], -lse)
+        tok += float((w[b] * t).sum())
+        bad += float((first[b].double() - ref).square().sum())
+        bad += float((scaled[b].double() / 3 - ref).square().sum())
+        size += 2 * float(ref.square().sum())
+        if mask[b].count_nonzero() == 0:
+            assert first[b].count_nonzero() == 0 and scaled[b].count_nonzero() == 0
+    assert (bad / max(size, 1e-60)) ** 0.5 < 2.0 ** -8 or size == 0
+    assert abs(float(loss) - tok) < 1e-5 * float((w.abs() * 20).sum() + 1e-30)
+
+
 @pytest.mark.parametrize("off,V", [(1, 4096), (3, 4103), (0, 32003), (1, 7)])
 def test_loss_rows_at_any_element(ext, off, V):
     """A matrix that starts inside another and rows of an odd vocabulary give
