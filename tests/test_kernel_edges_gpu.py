@@ -1227,6 +1227,28 @@ def test_loss_gradients_made_forward(ext, rows, V):
     assert not OF.logprob_rows(leaf, targets, w).requires_grad
 
 
+@pytest.mark.parametrize("threads,pieces", [(256, k) for k in range(1, 9)] + [(512, k) for k in range(5, 9)]
+                         + [(1024, k) for k in range(5, 20)])
+def test_loss_gradients_by_pieces(ext, threads, pieces):
+    """The narrowest and the widest row of every number of pieces that a workgroup's threads
+    hold, one row more than workgroups: as the two passes apart (as above)."""
+    from distrl_llm_amd.ops import functional as OF
+    rows = 256 * (8 * 256 // threads) + 1
+    for V in (threads * 8 * (pieces - 1) + 9, threads * 8 * pieces):
+        if rows * V < 1 << 20:
+            continue
+        g = torch.Generator("cuda").manual_seed(V)
+        leaf = torch.randn(rows, V, generator=g, device="cuda").mul_(2).bfloat16().requires_grad_()
+        targets = torch.randint(0, V, (rows,), generator=g, device="cuda")
+        targets[:2] = torch.tensor([V - 1, 0])
+        w = torch.randn(rows, generator=g, device="cuda")
+        tok, lse = ext.logprob_lse_fwd(leaf.detach(), targets)
+        loss = OF.logprob_rows(leaf, targets, w)
+        assert abs(float(loss.detach()) - float((tok * w).sum())) < 1e-5 * float((tok * w).abs().sum())
+        got, = torch.autograd.grad(loss, leaf)
+        assert _rel(got, ext.logprob_loss_bwd(leaf.detach(), targets, w, lse)) < 1e-5
+
+
 @pytest.mark.parametrize("rows", [4096, 4097, 6145, 8200])
 def test_feed_forward_half_in_waves(ext, rows):
     """Input gradients of rows whose tiles fill the chip once, of one row more,
