@@ -252,7 +252,9 @@ void loss_bwd_kernel(const T* __restrict__ logits, const int64_t* __restrict__ t
 }
 
 // The same where dlogits holds the gradient for a dloss of 1 already: a few workgroups
-// look whether it is that.
+// look whether it is that. What it costs where it is not, with the pass before it, us:
+// 2400 rows of 152064 592 with rows from the first, 567 from the last (389 in two passes);
+// 8000 of 32003 486, 440 (312). The gradient at hand can't be scaled instead: it is rounded.
 template <typename T, int THREADS>
 __global__ __launch_bounds__(THREADS)
 void loss_anew_kernel(const T* __restrict__ logits, const int64_t* __restrict__ targets,
@@ -261,7 +263,7 @@ void loss_anew_kernel(const T* __restrict__ logits, const int64_t* __restrict__ 
                       int64_t rows) {
   if (*dloss == 1.f) return;
   for (int64_t row = blockIdx.x; row < rows; row += gridDim.x)
-    loss_bwd_row<T, THREADS>(logits, targets, w, lse, dloss, dlogits, V, row);
+    loss_bwd_row<T, THREADS>(logits, targets, w, lse, dloss, dlogits, V, rows - 1 - row);
 }
 
 // Both passes at once, where the gradient will be asked for: a workgroup holds a row in
@@ -573,7 +575,10 @@ torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets, torc
 // The differentiable loss: a node of the C++ engine. Where a gradient is wanted of rows
 // that loss_both_kernel takes, forward makes it for a dloss of 1, which backward hands
 // out; any other dloss makes it anew from the logits, and so does every further backward
-// of a graph that is kept, as what was handed out is the caller's.
+// of a graph that is kept, as what was handed out is the caller's. So a loss that is
+// scaled or only looked at costs more than in two passes, and one whose backward is still
+// to come holds a gradient beside its logits: the price of the one pass, which callers
+// that scale by weights and run backward at once, as the learner, do not pay.
 namespace {
 
 bool wants_both(const torch::Tensor& logits) {

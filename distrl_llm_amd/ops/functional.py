@@ -328,7 +328,15 @@ def logprob_loss(logits: torch.Tensor, targets: torch.Tensor, mask: torch.Tensor
                  rewards: torch.Tensor, loss_scale: float = 1.0) -> torch.Tensor:
     """PG/GRPO loss on answer-region logits. logits (B, T, V); targets/mask
     (B, T); rewards (B,). ``loss_scale`` folds the reference's
-    loss/num_batches scaling (reference distributed_actor.py:382)."""
+    loss/num_batches scaling (reference distributed_actor.py:382).
+
+    On the GPU the gradient of 2 MB of bf16 logits and more is made in this call
+    where one is wanted, and held for ``loss.backward()``. So scale by
+    ``loss_scale`` (or rewards), not the loss behind it, look at a loss under
+    ``no_grad``, and run each loss' backward before the next loss where room is
+    short. 2400 rows of 152064, us: loss and backward 317 (389 in two passes over
+    the logits), of a loss scaled behind the call 567 (389), whose gradient is
+    made anew, a loss alone 316 (143), under ``no_grad`` 143."""
     if logits.is_cuda:
         ext, lead = _require_ext("logprob_loss"), logits.shape[:-1]
         if (len(lead) == 2 and targets.shape == mask.shape == lead
@@ -348,5 +356,6 @@ def logprob_loss(logits: torch.Tensor, targets: torch.Tensor, mask: torch.Tensor
 def logprob_rows(logits: torch.Tensor, targets: torch.Tensor,
                  w: torch.Tensor) -> torch.Tensor:
     """sum_i w_i log p(target_i) of logits (rows, V) on the GPU: logprob_loss
-    for rows of any number of sequences, each with its weight in the loss."""
+    for rows of any number of sequences, each with its weight in the loss. What
+    a scaled or unused loss costs is as there: scale the weights."""
     return _require_ext("logprob_rows").logprob_rows(logits, targets, w)
