@@ -38,6 +38,9 @@ DEV_INLINE void store8(__hip_bfloat16* p, const bf16x8& v) {
   __builtin_nontemporal_store(q, (Anywhere*)p);
 }
 
+// A target as an element of its row, -1 where it is none
+DEV_INLINE int word_of(int64_t target, int V) { return target >= 0 && target < V ? (int)target : -1; }
+
 // One workgroup per (b, t) row; single streaming pass, online logsumexp: a
 // thread takes 32 values at a time, the next 32 on their way, compares their
 // maximum with its own once and then sums exponentials without branches (value
@@ -194,7 +197,7 @@ DEV_INLINE void loss_bwd_row(const T* __restrict__ logits,
   T* dr = dlogits + row * V;
   const float wv = dloss ? w[row] * *dloss : w[row];
   const float l = lse[row];
-  const int64_t tgt = targets[row];
+  const int tgt = word_of(targets[row], V);
   if constexpr (std::is_same<T, __hip_bfloat16>::value) {
     const int nvec = V / 8;
     auto put = [&](int i, const bf16x8& v) {
@@ -202,7 +205,7 @@ DEV_INLINE void loss_bwd_row(const T* __restrict__ logits,
       #pragma unroll
       for (int j = 0; j < 8; ++j) {
         float p = __expf(bf2f(v.v[j]) - l);
-        o.v[j] = f2bf(wv * ((i * 8 + j == (int)tgt ? 1.f : 0.f) - p));
+        o.v[j] = f2bf(wv * ((i * 8 + j == tgt ? 1.f : 0.f) - p));
       }
       store8(dr + i * 8, o);
     };
@@ -225,7 +228,7 @@ DEV_INLINE void loss_bwd_row(const T* __restrict__ logits,
     for (int i = nvec * 8 + threadIdx.x; i < V; i += blockDim.x) {
       float g = 0.f;
       if (wv != 0.f)
-        g = wv * ((i == (int)tgt ? 1.f : 0.f) - __expf(ld(lr, i) - l));
+        g = wv * ((i == tgt ? 1.f : 0.f) - __expf(ld(lr, i) - l));
       dr[i] = f2bf(g);
     }
     return;
@@ -307,7 +310,7 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
   for (int turn = 0; row < rows; row += gridDim.x, turn ^= 1) {
     const __hip_bfloat16* lr = logits + row * V;
     __hip_bfloat16* dr = dlogits + row * V;
-    const int64_t tgt = targets[row];
+    const int tgt = word_of(targets[row], V);
     const float wv = w[row];
     const int at = nvec * 8 + tid;                        // of the last few
     const float tail = at < V ? ld(lr, at) : -__builtin_inff();
@@ -357,11 +360,11 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
     top = high;
     const float l = top + __logf(sum);
     if (tid == 0) lse_out[row] = l;
-    if (tid == 0 && (tgt < 0 || tgt >= V)) token_logp[row] = 0.f - l;
+    if (tid == 0 && tgt < 0) token_logp[row] = 0.f - l;
     if (at < V) {
       if (at == tgt) token_logp[row] = tail - l;
       float g = 0.f;
-      if (wv != 0.f) g = wv * ((at == (int)tgt ? 1.f : 0.f) - __expf(tail - l));
+      if (wv != 0.f) g = wv * ((at == tgt ? 1.f : 0.f) - __expf(tail - l));
       dr[at] = f2bf(g);
     }
     const auto to = row_at(dr), from = row_at(lr + (int64_t)gridDim.x * V);
@@ -370,10 +373,10 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
       #pragma unroll
       for (int c = 0; c < KEEP; ++c, next(off)) {
         {
-          if (off == (int)(tgt >> 3) * 16 && off < bytes && tgt >= 0) {
+          if (off == (tgt >> 3) * 16 && off < bytes) {
             float x = value(c, 0);
             #pragma unroll
-            for (int j = 1; j < 8; ++j) x = (int)(tgt & 7) == j ? value(c, j) : x;
+            for (int j = 1; j < 8; ++j) x = (tgt & 7) == j ? value(c, j) : x;
             token_logp[row] = x - l;
           }
           u32x4 o;
@@ -383,7 +386,7 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
             #pragma unroll
             for (int h = 0; h < 2; ++h) {
               const float p = __expf(value(c, 2 * j + h) - l);
-              g[h] = wv == 0.f ? 0.f : wv * ((off / 2 + 2 * j + h == (int)tgt ? 1.f : 0.f) - p);
+              g[h] = wv == 0.f ? 0.f : wv * ((off / 2 + 2 * j + h == tgt ? 1.f : 0.f) - p);
             }
             o[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{g[0], g[1]}, bf16v2));
           }

@@ -1249,6 +1249,27 @@ def test_loss_gradients_by_pieces(ext, threads, pieces):
         assert _rel(got, ext.logprob_loss_bwd(leaf.detach(), targets, w, lse)) < 1e-5
 
 
+@pytest.mark.parametrize("V,dtype", [(40, torch.bfloat16), (41, torch.float32), (32777, torch.bfloat16),
+                                     (66000, torch.bfloat16)])
+def test_targets_that_are_no_word(V, dtype):
+    """Targets below a row and past it, by all of their 64 bits: the loss has no logit of
+    theirs and the gradient is the softmax alone."""
+    from distrl_llm_amd.ops import functional as OF
+    targets = torch.tensor([-1, -100, V, 2 ** 31 + 3, 2 ** 32 + 5, 2 ** 35 + 9, 2 ** 40 + V - 1, -2 ** 32 + 4,
+                            -2 ** 63, 2 ** 63 - 1, V - 1, 5], device="cuda").repeat(3)
+    leaf = _rand((len(targets), V), V, 2.0).to(dtype).requires_grad_()
+    w = torch.linspace(0.5, 1.5, len(targets), device="cuda")
+    exact = leaf.detach().double().requires_grad_()
+    there = (targets >= 0) & (targets < V)
+    tok = torch.where(there, exact.gather(1, targets.where(there, 0)[:, None])[:, 0], 0.0) - exact.logsumexp(-1)
+    ref, = torch.autograd.grad((tok * w).sum(), exact)
+    for scale in (1.0, 3.0):
+        loss = OF.logprob_rows(leaf, targets, w)
+        assert abs(float(loss.detach()) - float((tok * w).sum().detach())) < 1e-5 * float((tok * w).abs().sum().detach())
+        grad, = torch.autograd.grad(loss * scale, leaf)
+        assert _rel(grad, ref * scale) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("rows", [4096, 4097, 6145, 8200])
 def test_feed_forward_half_in_waves(ext, rows):
     """Input gradients of rows whose tiles fill the chip once, of one row more,
