@@ -7,6 +7,7 @@
 // Where a gradient is wanted, both are one pass over logits that a workgroup's registers
 // hold (loss_both_kernel).
 #include <torch/extension.h>
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/cuda/CUDAContext.h>
 #include "common.h"
 
@@ -584,8 +585,11 @@ torch::Tensor logprob_loss_bwd(torch::Tensor logits, torch::Tensor targets, torc
 // that scale by weights and run backward at once, as the learner, do not pay.
 namespace {
 
+// Not under hooks on saved tensors (checkpoints, offloading): they would drop or move the
+// logits, and the gradient, which they don't see, would stay.
 bool wants_both(const torch::Tensor& logits) {
-  return at::GradMode::is_enabled() && logits.requires_grad() && logits.is_cuda() && takes_both(logits);
+  return at::GradMode::is_enabled() && logits.requires_grad() && logits.is_cuda() &&
+         takes_both(logits) && !at::SavedTensorDefaultHooks::get_hooks();
 }
 
 torch::Tensor handed_out(torch::autograd::AutogradContext* ctx, const torch::Tensor& dloss) {

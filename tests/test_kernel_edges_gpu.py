@@ -1270,6 +1270,40 @@ def test_targets_that_are_no_word(V, dtype):
         assert _rel(grad, ref * scale) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("masked", [False, True])
+def test_loss_under_saved_tensor_hooks(masked):
+    """A loss that is checkpointed, or whose saved tensors go to the host, holds nothing
+    of its logits' size on the GPU until its backward; its gradient is the same."""
+    from torch.utils.checkpoint import checkpoint
+    from distrl_llm_amd.ops import functional as OF
+    x, w = _rand((512, 64), 1), _rand((64, 8192), 2, 0.3)
+    targets, r = torch.arange(512, device="cuda"), torch.rand(512, device="cuda")
+    size = 512 * 8192 * 2
+
+    def loss_of(x):
+        logits = x @ w
+        if masked:
+            return OF.logprob_loss(logits[None], targets[None], r[None], r[:1], 0.5)
+        return OF.logprob_rows(logits, targets, r)
+
+    grads = []
+    for how in ("plain", "checkpoint", "host"):
+        leaf = x.clone().requires_grad_()
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        if how == "checkpoint":
+            loss = checkpoint(loss_of, leaf, use_reentrant=False)
+        elif how == "host":
+            with torch.autograd.graph.save_on_cpu():
+                loss = loss_of(leaf)
+        else:
+            loss = loss_of(leaf)
+        held = torch.cuda.memory_allocated() - before
+        assert how == "plain" or held < size // 2, (how, held)
+        grads.append(torch.autograd.grad(loss, leaf)[0])
+    assert all(_rel(g, grads[0]) < 2.0 ** -8 for g in grads[1:])
+
+
 @pytest.mark.parametrize("rows", [4096, 4097, 6145, 8200])
 def test_feed_forward_half_in_waves(ext, rows):
     """Input gradients of rows whose tiles fill the chip once, of one row more,
