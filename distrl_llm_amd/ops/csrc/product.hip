@@ -515,19 +515,29 @@ void by_size(Args& a, int blocks, int tile) {
   auto offer = [&](int what, int z, double cost) {
     if (cost < least) { least = cost; pick = what; splits = z; }
   };
+  // Sums over a vocabulary (the LM head's input gradient), in shares where tiles alone leave
+  // workgroups idle or their last round half empty: 561 x 896 x 151936 is 12 tiles. Shorter
+  // ones of few rows are the small tiles', whose shares meet without a launch. 1 GB of
+  // partial sums at most, 6 us for the launch that adds them at 4.5 TB/s. Fitted apart, to 87
+  // shapes of 5 to 19200 rows, 896 to 8192 wide, over 32768 to 152064 words: within 3 % of
+  // the best for nearly all. With the costs below for them, library's product, so, us:
+  // 2408 x 4096 x 128256 2390, 2141, 2158; 1200 x 8192 x 152064 2850, 2577, 2562; 1200 x
+  // 4096 x 32768, without shares, 442, 395, 278; 6400 x 1536 x 151936 2834, 5093, 2394.
+  const int64_t cells = (int64_t)a.M * a.width[0];
+  const bool sums = MODE == PLAIN && blocks == 1 && !a.bias[0] && !a.res && a.steps >= 1024;
   for (int tm = 8; tm >= 4; --tm) {
-    const int64_t rounds = CDIV((int64_t)CDIV(a.M, 32 * tm) * columns(256), (int64_t)256);
-    offer(tm, 1, a.steps * (rounds == 1 ? 0.29 + 0.043 * tm : rounds * (0.24 + 0.081 * tm)));
-    // Sums over a vocabulary (the LM head's input gradient) in shares, where tiles alone leave
-    // workgroups idle or their last round half empty: 561 x 896 x 151936 is 12 tiles. Shorter
-    // ones of few rows are the small tiles', whose shares meet without a launch. 1 GB of
-    // partial sums at most, 6 us for the launch that adds them at 4.5 TB/s.
-    const int64_t cells = (int64_t)a.M * a.width[0];
-    if (MODE != PLAIN || blocks != 1 || a.bias[0] || a.res || a.steps < 2048) continue;
-    for (int z = 2; z <= 64 && a.steps / z >= 64 && z * cells <= 1 << 28; ++z) {
-      const int64_t n = CDIV((int64_t)CDIV(a.M, 32 * tm) * columns(256) * z, (int64_t)256);
-      offer(tm, z, CDIV(a.steps, z) * (n == 1 ? 0.29 + 0.043 * tm : n * (0.24 + 0.081 * tm)) + 6. +
-                       z * cells * 8 / 4.5e6);
+    const int64_t tiles = (int64_t)CDIV(a.M, 32 * tm) * columns(256);
+    if (!sums) {
+      const int64_t rounds = CDIV(tiles, (int64_t)256);
+      offer(tm, 1, a.steps * (rounds == 1 ? 0.29 + 0.043 * tm : rounds * (0.24 + 0.081 * tm)));
+      continue;
+    }
+    for (int z = 1; z <= 64 && (z == 1 || (a.steps / z >= 64 && z * cells <= 1 << 28)); ++z) {
+      const int64_t rounds = CDIV(tiles * z, (int64_t)256);
+      const double full = 0.27 + 0.063 * tm, half = 0.26 + 0.045 * tm;
+      const double step = rounds > 1 ? rounds * 1.02 * full
+                                     : half + (full - half) * std::max(0., tiles * z / 128. - 1);
+      offer(tm, z, CDIV(a.steps, z) * step + (z > 1 ? 6. + z * cells * 8 / 4.5e6 : 0.));
     }
   }
   for (int z = 1; z <= 8 && (z == 1 || a.steps / z >= 8); ++z) {
@@ -685,7 +695,12 @@ bool product_glu_bwd(const ProductBlock& block, const at::Tensor& gu, const at::
 }
 
 // g w, g (M, V), w (V, N): own products for vocabularies of models in use, else the
-// library's (500 x 1024 x 32768 67 us here, 147 there; smaller ones not measured).
+// library's. From 32768 words on, 1 to 19200 rows, 896 to 8192 wide, own ones take what the
+// library's do or less, within 4 % (2408 x 8192 x 32768 1160 us here, 1119 there; 1200 x 8192
+// x 152064 2562, 2579; 19200 x 8192 x 152064 38.7 ms, 38.3; 300 x 4096 x 32768 103 us, 301);
+// only 19200 rows of 512 are slower, 842 and 759. Below it either may be the faster: 9000 x
+// 512 x 4096, 16384, 32000 79, 240, 417 us here, 44, 183, 372 there, 2400 x 4096 x 24576 437,
+// 403, 300 x 1024 x 4096 25, 19; 37 x 512 x 4096, 32000 11, 30 here, 18, 116 there.
 at::Tensor product_rows(const at::Tensor& g, const at::Tensor& w) {
   auto out = at::empty({g.size(0), w.size(1)}, g.options());
   if (g.size(0) > 0 && g.size(1) >= 32768 && product({{w.size(1), {{g, w}}, {}}}, true, out)) return out;

@@ -98,7 +98,7 @@ def test_large_tiles_in_shares(ext, M, N, steps, spare, rows, shares, what):
 
 
 @pytest.mark.parametrize("M,V,N", [(1, 65536, 64), (37, 65568, 96), (300, 70016, 264), (9, 32003, 64),
-                                   (0, 65536, 64)])
+                                   (0, 65536, 64), (700, 32768, 520), (1200, 32800, 8), (2408, 32768, 1024)])
 def test_head_input_gradient(ext, M, V, N):
     """Sums long enough for shares by the rule, and what goes to the library."""
     rand = _make(M)
