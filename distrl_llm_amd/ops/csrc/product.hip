@@ -477,9 +477,14 @@ void launch(Args& a, int blocks, int splits) {
   const int64_t cells = (int64_t)a.M * a.width[0];
   if (!JOINS && a.splits > 1) {
     TORCH_CHECK(a.splits * cells < (int64_t)1 << 31 && total * a.splits < (1 << 30), "product: shares");
-    room = at::empty({a.splits * cells}, at::TensorOptions().dtype(at::kFloat).device(
-        at::kCUDA, at::cuda::current_device()));
-    a.part = room.data_ptr<float>();
+    // where memory has no room for the partial sums, tiles take all of K
+    try {
+      room = at::empty({a.splits * cells}, at::TensorOptions().dtype(at::kFloat).device(
+          at::kCUDA, at::cuda::current_device()));
+      a.part = room.data_ptr<float>();
+    } catch (const c10::OutOfMemoryError&) {
+      a.splits = 1;
+    }
   } else if (a.splits > 1) {
     const int64_t shares = total * a.splits;
     room = at::empty({shares * (BM * BN * 4 + 8)}, at::TensorOptions().dtype(at::kByte).device(

@@ -106,6 +106,28 @@ def test_head_input_gradient(ext, M, V, N):
     _each_close(ext.product_rows(g, w), *_sum([(g, w)], True))
 
 
+def test_head_input_gradient_without_room(ext):
+    """Shares whose partial sums no memory is left for: the same product, without them."""
+    rand = _make(1)
+    g, w = rand(561, 65536), rand(65536, 896)
+    want = ext.product_rows(g, w)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = torch.empty_like(want)                           # of the result, kept by the allocator
+    total, rest = torch.cuda.get_device_properties(0).total_memory, []
+    try:
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                rest.append(torch.empty(16 << 20, dtype=torch.uint8, device="cuda"))
+        del room
+        got = ext.product_rows(g, w)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    _each_close(got, *_sum([(g, w)], True))
+    assert float((got.float() - want.float()).norm() / want.float().norm()) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("M,F,K,r", [(1, 8, 32, 32), (70, 40, 96, 32), (130, 136, 64, 64),
                                      (300, 264, 160, 32)])
 @pytest.mark.parametrize("tile", TILES)
