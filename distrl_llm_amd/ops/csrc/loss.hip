@@ -454,10 +454,10 @@ static void by_pieces(int pieces, T threads, F&& f) {
   f(threads, std::integral_constant<int, FIRST>{});
 }
 
-// {token_logp, lse, the gradient for a dloss of 1}
+// {token_logp, lse}; grad <- the gradient for a dloss of 1
 static std::vector<torch::Tensor> logprob_both(const torch::Tensor& logits,
                                                const torch::Tensor& targets,
-                                               const torch::Tensor& w) {
+                                               const torch::Tensor& w, const torch::Tensor& grad) {
   TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() && takes_both(logits));
   TORCH_CHECK(targets.scalar_type() == at::kLong && targets.is_contiguous());
   const int V = logits.size(-1), nvec = V / 8;
@@ -466,7 +466,6 @@ static std::vector<torch::Tensor> logprob_both(const torch::Tensor& logits,
   sizes.pop_back();
   auto token_logp = torch::empty(sizes, logits.options().dtype(at::kFloat));
   auto lse = torch::empty_like(token_logp);
-  auto grad = torch::empty_like(logits);
   auto go = [&](auto threads_, auto keep_) {
     constexpr int THREADS = decltype(threads_)::value, KEEP = decltype(keep_)::value;
     // workgroups a CU by their registers
@@ -487,14 +486,15 @@ static std::vector<torch::Tensor> logprob_both(const torch::Tensor& logits,
   else if (nvec <= 8 * 512) by_pieces<5, 8>(CDIV(nvec, 512), std::integral_constant<int, 512>{}, go);
   else by_pieces<5, 19>(CDIV(nvec, 1024), std::integral_constant<int, 1024>{}, go);
   HIP_CHECK_LAST();
-  return {token_logp, lse, grad};
+  return {token_logp, lse};
 }
 
 // The masked PG/GRPO loss of logits (B, T, V): {loss, row weights (B, T), lse}, and
-// with both the gradient for a dloss of 1. mask int64 or fp32, rewards fp32.
+// grad, if any, <- the gradient for a dloss of 1. mask int64 or fp32, rewards fp32.
 static std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits, torch::Tensor targets,
                                                    torch::Tensor mask, torch::Tensor rewards,
-                                                   double scale, bool both) {
+                                                   double scale,
+                                                   const c10::optional<torch::Tensor>& grad) {
   TORCH_CHECK(logits.dim() == 3 && mask.is_cuda() && rewards.is_cuda());
   const int B = logits.size(0), T = logits.size(1);
   TORCH_CHECK(mask.numel() == (int64_t)B * T && targets.numel() == (int64_t)B * T &&
@@ -510,20 +510,19 @@ static std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits, torch::
     hipLaunchKernelGGL(loss_weights_kernel<M>, dim3(B), dim3(1024), 0, stream,        \
                        mask.data_ptr<M>(), rewards.data_ptr<float>(),                 \
                        w.data_ptr<float>(), B, T, (float)scale)
-  if (both && mask64) WEIGHTS(int64_t);
-  else if (both) WEIGHTS(float);
+  if (grad && mask64) WEIGHTS(int64_t);
+  else if (grad) WEIGHTS(float);
   #undef WEIGHTS
-  auto lp = both ? logprob_both(logits, targets, w) : logprob_lse_fwd(logits, targets);
+  auto lp = grad ? logprob_both(logits, targets, w, *grad) : logprob_lse_fwd(logits, targets);
   #define REDUCE(M)                                                                   \
     hipLaunchKernelGGL(loss_reduce_kernel<M>, dim3(1), dim3(1024), 0, stream,         \
                        lp[0].data_ptr<float>(), mask.data_ptr<M>(),                   \
-                       rewards.data_ptr<float>(), both ? nullptr : w.data_ptr<float>(), \
+                       rewards.data_ptr<float>(), grad ? nullptr : w.data_ptr<float>(), \
                        loss.data_ptr<float>(), B, T, (float)scale)
   if (mask64) REDUCE(int64_t);
   else REDUCE(float);
   #undef REDUCE
   HIP_CHECK_LAST();
-  if (both) return {loss, w, lp[1], lp[2]};
   return {loss, w, lp[1]};
 }
 
@@ -592,6 +591,16 @@ bool wants_both(const torch::Tensor& logits) {
          takes_both(logits) && !at::SavedTensorDefaultHooks::get_hooks();
 }
 
+// Where the gradient goes; two passes where memory has no room for it yet.
+c10::optional<torch::Tensor> gradient_room(const torch::Tensor& logits, bool both) {
+  if (!both) return c10::nullopt;
+  try {
+    return torch::empty_like(logits);
+  } catch (const c10::OutOfMemoryError&) {
+    return c10::nullopt;
+  }
+}
+
 torch::Tensor handed_out(torch::autograd::AutogradContext* ctx, const torch::Tensor& dloss) {
   const auto s = ctx->get_saved_variables();
   c10::optional<torch::Tensor> made;
@@ -610,10 +619,11 @@ struct LogprobLoss : public torch::autograd::Function<LogprobLoss> {
     targets = targets.contiguous();
     // int64 masks are read as they are
     auto m = mask.scalar_type() == at::kLong ? mask : mask.to(at::kFloat);
+    const auto grad = gradient_room(logits, both);
     auto r = logprob_loss_fwd(logits, targets, m.contiguous(),
-                              rewards.to(at::kFloat).contiguous(), scale, both);
+                              rewards.to(at::kFloat).contiguous(), scale, grad);
     ctx->save_for_backward({logits, targets, r[1], r[2]});
-    if (both) ctx->saved_data["grad"] = r[3];
+    if (grad) ctx->saved_data["grad"] = *grad;
     return r[0];
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
@@ -643,14 +653,15 @@ struct LogprobRows : public torch::autograd::Function<LogprobRows> {
     logits = logits.contiguous();
     targets = targets.contiguous();
     w = w.contiguous();
-    auto lp = both ? logprob_both(logits, targets, w) : logprob_lse_fwd(logits, targets);
+    const auto grad = gradient_room(logits, both);
+    auto lp = grad ? logprob_both(logits, targets, w, *grad) : logprob_lse_fwd(logits, targets);
     auto loss = torch::empty({}, lp[0].options());
     hipLaunchKernelGGL(loss_rows_kernel, dim3(1), dim3(1024), 0, at::cuda::getCurrentCUDAStream(),
                        lp[0].data_ptr<float>(), w.data_ptr<float>(), loss.data_ptr<float>(),
                        logits.size(0));
     HIP_CHECK_LAST();
     ctx->save_for_backward({logits, targets, w, lp[1]});
-    if (both) ctx->saved_data["grad"] = lp[2];
+    if (grad) ctx->saved_data["grad"] = *grad;
     return loss;
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,

@@ -1271,6 +1271,36 @@ def test_targets_that_are_no_word(V, dtype):
 
 
 @pytest.mark.parametrize("masked", [False, True])
+def test_loss_without_room_for_a_gradient(masked):
+    """A loss is had, with gradients enabled, where memory holds no gradient of its logits
+    yet, and its backward once there is room."""
+    from distrl_llm_amd.ops import functional as OF
+    leaf = _rand((1024, 16384), 1, 2.0).requires_grad_()
+    targets, r = torch.arange(1024, device="cuda"), torch.rand(1024, device="cuda")
+
+    def loss_of(x):
+        if masked:
+            return OF.logprob_loss(x[None], targets[None], r[None], r[:1], 0.5)
+        return OF.logprob_rows(x, targets, r)
+
+    want = loss_of(leaf)
+    ref, = torch.autograd.grad(want, leaf)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total, rest = torch.cuda.get_device_properties(0).total_memory, []
+    try:
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                rest.append(torch.empty(8 << 20, dtype=torch.uint8, device="cuda"))
+        loss = loss_of(leaf)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert abs(float(loss - want)) < 1e-5 * abs(float(want))
+    assert _rel(torch.autograd.grad(loss, leaf)[0], ref) < 1e-5
+
+
+@pytest.mark.parametrize("masked", [False, True])
 def test_loss_under_saved_tensor_hooks(masked):
     """A loss that is checkpointed, or whose saved tensors go to the host, holds nothing
     of its logits' size on the GPU until its backward; its gradient is the same."""
