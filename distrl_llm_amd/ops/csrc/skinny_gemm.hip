@@ -358,13 +358,11 @@ void pair(const PairArgs& p, int kind) {
   if (!narrow) {
     if (u <= 2) launch_pair<MODE, 2 * ACC, 8, 2>(p, kind);
     else if (u == 3) launch_pair<MODE, 2 * ACC, 8, 3>(p, kind);
-    else if (u == 4) launch_pair<MODE, 2 * ACC, 8, 4>(p, kind);
-    else launch_pair<MODE, 2 * ACC, 8, 5>(p, kind);
-  } else if (MODE != GLU && steps <= 16) {
-    launch_pair<MODE, ACC, 16, 1>(p, kind);
-  } else if (u <= 2) {
-    launch_pair<MODE, ACC, 8, 2>(p, kind);
-  } else if (u == 3) {
+    else if (MODE == GLU || u == 4) launch_pair<MODE, 2 * ACC, 8, 4>(p, kind);
+    else launch_pair<MODE, 2 * ACC, 8, MODE == GLU ? 4 : 5>(p, kind);
+  } else if (MODE == GLU ? u <= 2 : steps <= 16) {
+    launch_pair<MODE, ACC, MODE == GLU ? 8 : 16, MODE == GLU ? 2 : 1>(p, kind);
+  } else if (u <= 3) {                      // 2 only where steps <= 16
     launch_pair<MODE, ACC, 8, 3>(p, kind);
   } else if (u <= 5) {
     launch_pair<MODE, ACC, 8, 5>(p, kind);
@@ -432,8 +430,23 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
   auto y = torch::empty({M, N}, x.options());
   auto* o = reinterpret_cast<__hip_bfloat16*>(y.data_ptr());
   auto stream = at::cuda::getCurrentCUDAStream();
-  // Rows of W a workgroup takes and waves that share its K, from sweeps of both
-  // at 8 rows and cold weights (us; rows/waves): N 896, K 4864: 16/4 11.8,
+  TORCH_CHECK(mode != RESIDUAL || !nw, "skinny_gemm: norm with a residual sum");
+  const int kind = !tiles ? ROWS : kept ? KEPT : TILES;
+  // As a step of few sequences calls them; without a norm only adapters of 32 rows are
+  // multiplied, which wait for the launch. A row's sums over K are of another order here
+  // than below: its product is the same bits beside up to 7 other rows, and beside 8 to 15,
+  // but not on either side of that line (as on either side of the lines to other kernels).
+  if (M <= 8 && K % 64 == 0 && (nw != nullptr) == (mode != RESIDUAL)) {
+    const PairArgs args{ptr(x), ptr(w), b, r, nw, up, ubp, o, M, N, K, R, (float)eps};
+    if (mode == PLAIN) pair<PLAIN>(args, kind);
+    else if (mode == RESIDUAL) pair<RESIDUAL>(args, kind);
+    else pair<GLU>(args, kind);
+    HIP_CHECK_LAST();
+    return y;
+  }
+  // Rows of W a workgroup takes and waves that share its K, for 9 to 32 rows of x (and
+  // fewer where K is no multiple of 64). The lines are those of sweeps at 8 rows and cold
+  // weights, which this kernel took too then (us; rows/waves): N 896, K 4864: 16/4 11.8,
   // 16/16 10.6, 8/16 8.6, 4/16 7.8; N 1536, K 8960: 19.4, 19.6, 15.3, 24.0;
   // N 2560, K 9728: 22.7, 20.3, 28.0; N 1152, K 896: 4.6 (8/4 4.3, 8/16 8.0);
   // N 1536, K 1536: 7.1 (8/4 6.3, 8/8 5.7); SiLU*mul of N 8960, K 1536: 16/4
@@ -443,18 +456,6 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w, int64_t mode,
   const int nt = N / 16, steps = K / 32, tr = nt <= 128 ? 8 : 16;
   const int kw = nt <= 256 ? (steps >= 64 ? 16 : steps >= 32 ? 8 : 4)
                         : (mode == GLU && steps >= 48 ? 8 : 4);
-  TORCH_CHECK(mode != RESIDUAL || !nw, "skinny_gemm: norm with a residual sum");
-  const int kind = !tiles ? ROWS : kept ? KEPT : TILES;
-  // as a step of few sequences calls them; without a norm only adapters of 32 rows are
-  // multiplied, which wait for the launch
-  if (M <= 8 && K % 64 == 0 && (nw != nullptr) == (mode != RESIDUAL)) {
-    const PairArgs args{ptr(x), ptr(w), b, r, nw, up, ubp, o, M, N, K, R, (float)eps};
-    if (mode == PLAIN) pair<PLAIN>(args, kind);
-    else if (mode == RESIDUAL) pair<RESIDUAL>(args, kind);
-    else pair<GLU>(args, kind);
-    HIP_CHECK_LAST();
-    return y;
-  }
   auto launch = [&](auto mt_, auto kw_, auto mode_, auto norm_, auto w_) {
     constexpr int MT = decltype(mt_)::value, KW = decltype(kw_)::value,
                   MODE = decltype(mode_)::value;

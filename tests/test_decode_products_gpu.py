@@ -114,9 +114,12 @@ def test_skinny_gemm_tiles(ext, M, N, K):
 
 @pytest.mark.parametrize("M", [1, 7, 8])
 @pytest.mark.parametrize("N,K,R", [(16, 512, 32), (896, 896, 0), (1152, 1024, 96), (2048, 1088, 64),
-                                   (2064, 576, 32), (32, 4864, 0), (2080, 8960, 32)])
+                                   (2064, 576, 32), (32, 4864, 0), (2080, 8960, 32), (64, 2560, 0),
+                                   (48, 3584, 32), (2048, 4608, 0), (2064, 1536, 32), (2560, 4096, 0),
+                                   (2080, 4608, 0), (8960, 1536, 0), (9728, 2560, 0), (4608, 3584, 32)])
 def test_skinny_gemm_few_rows(ext, M, N, K, R):
-    """Up to 8 rows: two steps of K side by side, shares of every size. Sums in fp32 of
+    """Up to 8 rows: two steps of K side by side, every number of them that a wave has in
+    flight (1, 3, 5, 7, 9, 10, with SiLU*mul 2 for 1; more rows of W: 2 to 5, to 4). Sums in fp32 of
     products that are exact: what is left is the output's rounding, and of gate and up
     each their own, whose errors silu at most doubles."""
     x, w, b = _rand((M, K), 1), _rand((2 * N, K), 2, K ** -0.5), _rand((N,), 3)
