@@ -1433,6 +1433,29 @@ def test_halves_take_adapter_inputs_once(ext, r):
     assert ran("adapter_inputs_kernel") == 2
 
 
+@pytest.mark.parametrize("tied", [True, False])
+@pytest.mark.parametrize("V,own", [(4096, 0), (32768, 1), (65544, 0), (70016, 1)])
+def test_rows_logits(tied, V, own):
+    """Logits of rows and their gradient on either side of the LM head's line to products
+    of our own, a vocabulary that they don't take, a gradient that is laid out by columns
+    (the library's). Sums in fp32, rounded to bf16 once."""
+    import dataclasses
+    from distrl_llm_amd.models import get_spec
+    model = _train_model(dataclasses.replace(get_spec("small-qwen2"), vocab_size=V, tie_word_embeddings=tied))
+    weight = (model.model.embed_tokens if tied else model.lm_head).weight
+    assert not weight.requires_grad
+    hidden, g = _rand((37, 512), 1).requires_grad_(), _rand((37, V), 2, 0.1)
+    logits = model.rows_logits(hidden)
+    assert torch.equal(logits, model.logits(hidden))
+    (grad,), ran = _kernels(lambda: torch.autograd.grad(logits, hidden, g, retain_graph=True))
+    assert (ran("product_kernel") > 0) == bool(own)
+    ref = g.double() @ weight.double()
+    assert _rel(logits, hidden.detach().double() @ weight.double().t()) < 2.0 ** -8
+    assert _rel(grad, ref) < 2.0 ** -8
+    other, = torch.autograd.grad(logits, hidden, g.t().contiguous().t())
+    assert _rel(other, ref) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("prompts,answers", [([9, 30, 1], [40, 7, 100]), ([0, 5, 3], [4, 0, 6]),
                                              ([3], [1]), ([4, 2], [0, 0])])
 def test_learner_rows_match_padding(prompts, answers):
