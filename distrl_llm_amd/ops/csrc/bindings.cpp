@@ -70,9 +70,6 @@ bool weights_tiles(std::vector<torch::Tensor> w, std::vector<torch::Tensor> out,
                    std::vector<int64_t> row, std::vector<bool> glu,
                    std::vector<c10::optional<torch::Tensor>> a,
                    std::vector<c10::optional<torch::Tensor>> b, std::vector<double> scale);
-bool weight_tiles(torch::Tensor w, torch::Tensor out, int64_t row, bool glu,
-                  c10::optional<torch::Tensor> a,
-                  c10::optional<torch::Tensor> b, double scale);
 std::vector<torch::Tensor> add_rmsnorm_join(torch::Tensor parts,
                                             torch::Tensor res, torch::Tensor w,
                                             double eps,
@@ -242,7 +239,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "fp32 partial sums of x [w; w2]^T, W in tiles", py::arg("x"),
         py::arg("w"), py::arg("w2") = py::none());
   m.def("weights_tiles", &weights_tiles, "weight_tiles of several weights, one launch for eight");
-  m.def("weight_tiles", &weight_tiles,
+  m.def("weight_tiles",
+        [](torch::Tensor w, torch::Tensor out, int64_t row, bool glu, c10::optional<torch::Tensor> a,
+           c10::optional<torch::Tensor> b, double scale) {
+          return weights_tiles({w}, {out}, {row}, {glu}, {a}, {b}, {scale});
+        },
         "rows of W (+ scale * B A) into tiles; false: not these operands",
         py::arg("w"), py::arg("out"), py::arg("row"), py::arg("glu"),
         py::arg("a") = py::none(), py::arg("b") = py::none(),

@@ -281,19 +281,9 @@ void launch_tiles(Jobs& jobs) {
 
 }  // namespace
 
-// Rows row .. of a weight in tiles (out: (rows, K), K % 32 == 0, see the kernel)
-// <- w, or w + scale * b a. glu: w is gate (row 0) or up (row 16) of a SiLU*mul
-// pair. False, and nothing done, for operands that 16 B accesses can't take.
-bool weight_tiles(torch::Tensor w, torch::Tensor out, int64_t row, bool glu,
-                  c10::optional<torch::Tensor> a, c10::optional<torch::Tensor> b, double scale) {
-  Jobs jobs;
-  jobs.n = 1;
-  if (!tiles_job(jobs.job[0], w, out, row, glu, a, b, scale)) return false;
-  launch_tiles(jobs);
-  return true;
-}
-
-// The same for several weights; false, and nothing done, where one can't be taken.
+// Of each weight: rows row .. of out, a weight in tiles ((rows, K), K % 32 == 0, see the
+// kernel) <- w, or w + scale * b a. glu: w is gate (row 0) or up (row 16) of a SiLU*mul
+// pair. False, and nothing done, where 16 B accesses can't take an operand.
 bool weights_tiles(std::vector<torch::Tensor> w, std::vector<torch::Tensor> out,
                    std::vector<int64_t> row, std::vector<bool> glu,
                    std::vector<c10::optional<torch::Tensor>> a,

@@ -77,6 +77,33 @@ def test_weights_tiles(ext, n):
     assert all(torch.equal(o, w) for o, w in zip(outs, want))
 
 
+@pytest.mark.parametrize("N,K", [(18944, 3584), (3584, 18944)])
+def test_weights_tiles_of_all_sizes(ext, N, K):
+    """A weight of whose rows a workgroup takes 256, between small ones of whose it takes
+    64, in one launch: each is what torch makes of W + s B A, rounded once (sums in fp32
+    of products that are exact), and what lies beside it stays."""
+    from distrl_llm_amd.engine.weights import _untiled
+    jobs = []
+    for i, (n, k, r, row) in enumerate(((96, 1056, 40, 0), (N, K, 32, 16), (256, 288, 8, 32), (N, K, 0, 0),
+                                        (32, 32, 128, 0), (N, K, 16, 32))):
+        g = torch.Generator("cuda").manual_seed(i)
+        rand = lambda *s, std=1.0: torch.randn(s, generator=g, device="cuda").mul_(std).bfloat16()
+        glu = row == 16
+        out = torch.full((n * (2 if glu else 1) + 64 * (not glu), k), 3.0, dtype=torch.bfloat16, device="cuda")
+        jobs.append((rand(n, k), out, row, glu, rand(r, k, std=0.1) if r else None,
+                     rand(n, r, std=0.1) if r else None, 0.5 + i))
+    assert ext.weights_tiles(*map(list, zip(*jobs)))
+    for w, out, row, glu, a, b, scale in jobs:
+        got, first = _untiled(out, glu), len(w) if glu else row
+        there = got[first:first + len(w)]
+        assert bool((got[:first] == 3).all()) and bool((got[first + len(w):] == 3).all())
+        if a is None:
+            assert torch.equal(there, w)
+        else:
+            ref = w.double().addmm_(b.double(), a.double(), alpha=scale)
+            assert float(((there.double() - ref).abs() / ref.abs().clamp_min(2.0 ** -6)).max()) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("M", [1, 17, 32, 33, 96, 128, 129, 160])
 @pytest.mark.parametrize("N,K", [(32, 64), (96, 192), (1152, 896), (2048, 1536), (160, 8960)])
 def test_stream_gemm(ext, M, N, K):
