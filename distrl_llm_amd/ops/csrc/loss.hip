@@ -120,7 +120,7 @@ void logprob_lse_kernel(const T* __restrict__ logits,
   }
 }
 
-// Row weights (where w is given) and the loss itself: w[b, t] = mask * coef_b with
+// Row weights and the loss itself: w[b, t] = mask * coef_b with
 // coef_b = -reward_b / max(sum mask, 1) / B * scale, loss = sum w * token_logp.
 // One wave a sequence and turn.
 template <typename M>
@@ -140,8 +140,7 @@ void loss_reduce_kernel(const float* __restrict__ token_logp, const M* __restric
       sum += token_logp[at + t] * k;
     }
     const float coef = -rewards[b] / fmaxf(wave_sum(n), 1.f) / B * scale;
-    if (w)
-      for (int t = lane; t < T; t += WAVE) w[at + t] = (float)mask[at + t] * coef;
+    for (int t = lane; t < T; t += WAVE) w[at + t] = (float)mask[at + t] * coef;
     total += wave_sum(sum) * coef;
   }
   if (lane == 0) part[wave] = total;
@@ -153,16 +152,29 @@ void loss_reduce_kernel(const float* __restrict__ token_logp, const M* __restric
   }
 }
 
-// The row weights alone, before a pass over logits that makes the gradient at once, whose
-// every row would else read its sequence's whole mask: 1 x 32768 rows of 4096 1041 us, so
-// 319 (396 in two passes), 1 x 16384 of 4096 343, 127 (174), 8 x 301 of 152064 325, 323.
-// A workgroup a sequence.
+// Workgroups that count themselves: in groups on cache lines of their own, then the groups.
+// 2048 of them that end at once on one word took 17 us (8 x 600 x 4096 46 us, so 31).
+constexpr int GROUPS = 32, LINE = 32, COUNTS = (GROUPS + 1) * LINE;
+
+// Whether this one is the last; counts cleared, one thread of each
+DEV_INLINE bool last_to_end(uint32_t* counts) {
+  const uint32_t n = gridDim.x, groups = min((uint32_t)GROUPS, n), g = blockIdx.x % groups;
+  return atomicAdd(counts + (g + 1) * LINE, 1u) == (n - g - 1) / groups &&
+         atomicAdd(counts, 1u) == groups - 1;
+}
+
+// The row weights alone, ahead of a pass over logits that makes the gradient at once,
+// whose every row would else read its sequence's whole mask. A workgroup a sequence.
+// counts <- 0, for the workgroups of that pass.
 template <typename M>
 __global__ __launch_bounds__(1024)
 void loss_weights_kernel(const M* __restrict__ mask, const float* __restrict__ rewards,
-                         float* __restrict__ w, int B, int T, float scale) {
+                         float* __restrict__ w, uint32_t* __restrict__ counts, int B, int T,
+                         float scale) {
   __shared__ float red[16];
   const int64_t at = (int64_t)blockIdx.x * T;
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < COUNTS; i += 1024) counts[i] = 0;
   float n = 0.f;
   for (int t = threadIdx.x; t < T; t += 1024) n += (float)mask[at + t];
   const float coef = -rewards[blockIdx.x] / fmaxf(block_sum(n, red), 1.f) / B * scale;
@@ -277,15 +289,28 @@ void loss_anew_kernel(const T* __restrict__ logits, const int64_t* __restrict__ 
 // their way all the time. Bound by memory: 2408 rows of 152064, a quarter of weight zero,
 // 308 us (4.75 TB/s read and written), 133 and 222 in two passes; with the sum over rows
 // and the look at dloss 356 -> 320. Loads or stores through or past the caches are even.
+// With loss and counts the rows' weighted sum is made here too: a workgroup's part of it goes
+// through token_logp (an element a workgroup) to the last to end, which adds them up in
+// their order.
+struct RowWeights {
+  float* w;                   // of each row; made by it where there is
+  const void* mask;           // (B, T), int64 or fp32, with rewards as the loss has them
+  bool mask64;
+  const float* rewards;
+  int B, T;
+  float scale;
+};
+
 template <int THREADS, int KEEP>
 __global__ __launch_bounds__(THREADS)
 void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* __restrict__ targets,
-                      const float* __restrict__ w, float* __restrict__ token_logp,
-                      float* __restrict__ lse_out, __hip_bfloat16* __restrict__ dlogits, int rows,
-                      int V) {
+                      RowWeights weights, float* __restrict__ token_logp,
+                      float* __restrict__ lse_out, __hip_bfloat16* __restrict__ dlogits,
+                      float* __restrict__ loss, uint32_t* __restrict__ counts, int rows, int V) {
   constexpr float LOG2E = 1.4426950408889634f;
   constexpr int NW = THREADS / WAVE;
-  __shared__ float part[2][2][NW];
+  __shared__ float part[2][3][NW], ends[NW];
+  __shared__ bool last;
   const int tid = threadIdx.x, lane = tid & (WAVE - 1), nvec = V / 8;
   u32x4 v[KEEP];
   // One offset that walks a row, as 19 addresses would take the registers: what lies past
@@ -301,6 +326,7 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
   auto value = [&](int c, int j) {
     return __uint_as_float(j & 1 ? v[c][j / 2] & 0xffff0000u : v[c][j / 2] << 16);
   };
+  float mine = 0.f;             // of the loss
   int64_t row = blockIdx.x;
   {
     const auto from = row_at(logits + row * V);
@@ -312,7 +338,15 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
     const __hip_bfloat16* lr = logits + row * V;
     __hip_bfloat16* dr = dlogits + row * V;
     const int tgt = word_of(targets[row], V);
-    const float wv = w[row];
+    // the sequence's mask, summed beside the logits
+    float share = 0.f;
+    const int64_t seq = weights.mask ? row / weights.T : 0;
+    auto mask = [&](int64_t i) {
+      return weights.mask64 ? (float)reinterpret_cast<const int64_t*>(weights.mask)[i]
+                            : reinterpret_cast<const float*>(weights.mask)[i];
+    };
+    if (weights.mask)
+      for (int t = tid; t < weights.T; t += THREADS) share += mask(seq * weights.T + t);
     const int at = nvec * 8 + tid;                        // of the last few
     const float tail = at < V ? ld(lr, at) : -__builtin_inff();
 
@@ -344,9 +378,11 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
     // over the workgroup: one meeting a row, in turns of LDS
     const float M = wave_max(m);
     s = wave_sum(s * __builtin_amdgcn_exp2f((m - M) * LOG2E));
+    if (weights.mask) share = wave_sum(share);
     if (lane == 0) {
       part[turn][0][tid / WAVE] = M;
       part[turn][1][tid / WAVE] = s;
+      part[turn][2][tid / WAVE] = share;
     }
     __syncthreads();
     // a wave's lanes take a wave each, in every wave
@@ -360,10 +396,24 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
     for (int off = NW / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, WAVE);
     top = high;
     const float l = top + __logf(sum);
+    float wv;
+    if (weights.mask) {
+      float n = part[turn][2][of];
+      #pragma unroll
+      for (int off = NW / 2; off > 0; off >>= 1) n += __shfl_xor(n, off, WAVE);
+      wv = mask(row) * (-weights.rewards[seq] / fmaxf(n, 1.f) / weights.B * weights.scale);
+      if (tid == 0) weights.w[row] = wv;
+    } else {
+      wv = weights.w[row];
+    }
     if (tid == 0) lse_out[row] = l;
-    if (tid == 0 && tgt < 0) token_logp[row] = 0.f - l;
+    auto put = [&](float logp) {
+      if (loss) mine += wv * logp;
+      else token_logp[row] = logp;
+    };
+    if (tid == 0 && tgt < 0) put(0.f - l);
     if (at < V) {
-      if (at == tgt) token_logp[row] = tail - l;
+      if (at == tgt) put(tail - l);
       float g = 0.f;
       if (wv != 0.f) g = wv * ((at == tgt ? 1.f : 0.f) - __expf(tail - l));
       dr[at] = f2bf(g);
@@ -378,7 +428,7 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
             float x = value(c, 0);
             #pragma unroll
             for (int j = 1; j < 8; ++j) x = (tgt & 7) == j ? value(c, j) : x;
-            token_logp[row] = x - l;
+            put(x - l);
           }
           u32x4 o;
           #pragma unroll
@@ -400,6 +450,27 @@ void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* 
     if (row + gridDim.x < rows) write(std::true_type{});
     else write(std::false_type{});
   }
+  if (!loss) return;
+  auto over_block = [&](float x) {      // thread 0 has the sum
+    x = wave_sum(x);
+    if (lane == 0) ends[tid / WAVE] = x;
+    __syncthreads();
+    if (tid == 0)
+      for (int i = 1; i < NW; ++i) x += ends[i];
+    return x;
+  };
+  mine = over_block(mine);
+  if (tid == 0) {
+    store_through(token_logp + blockIdx.x, mine);
+    stores_done();
+    last = last_to_end(counts);
+  }
+  __syncthreads();
+  if (!last) return;
+  float sum = 0.f;
+  for (int i = tid; i < (int)gridDim.x; i += THREADS) sum += load_through(token_logp + i);
+  sum = over_block(sum);
+  if (tid == 0) *loss = sum;
 }
 
 }  // namespace
@@ -454,39 +525,68 @@ static void by_pieces(int pieces, T threads, F&& f) {
   f(threads, std::integral_constant<int, FIRST>{});
 }
 
-// {token_logp, lse}; grad <- the gradient for a dloss of 1
-static std::vector<torch::Tensor> logprob_both(const torch::Tensor& logits,
-                                               const torch::Tensor& targets,
-                                               const torch::Tensor& w, const torch::Tensor& grad) {
+// Threads of a workgroup of loss_both_kernel for rows of nvec pieces of 8 values, and
+// workgroups a CU by their registers.
+static int threads_of(int nvec) { return nvec <= 8 * 256 ? 256 : nvec <= 8 * 512 ? 512 : 1024; }
+static constexpr int per_cu(int threads, int pieces) {
+  return std::max(1, (8 - (pieces > 5) - (pieces > 7)) * 256 / threads);
+}
+
+// lse; grad <- the gradient for a dloss of 1, token_logp <- its values, or, with counts, the
+// workgroups' parts of loss <- the sum of w * token_logp
+static torch::Tensor logprob_both(const torch::Tensor& logits, const torch::Tensor& targets,
+                                  const RowWeights& weights, const torch::Tensor& grad,
+                                  float* token_logp, float* loss, uint32_t* counts) {
   TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() && takes_both(logits));
   TORCH_CHECK(targets.scalar_type() == at::kLong && targets.is_contiguous());
   const int V = logits.size(-1), nvec = V / 8;
   const int rows = (int)(logits.numel() / V);
   auto sizes = logits.sizes().vec();
   sizes.pop_back();
-  auto token_logp = torch::empty(sizes, logits.options().dtype(at::kFloat));
-  auto lse = torch::empty_like(token_logp);
+  auto lse = torch::empty(sizes, logits.options().dtype(at::kFloat));
   auto go = [&](auto threads_, auto keep_) {
     constexpr int THREADS = decltype(threads_)::value, KEEP = decltype(keep_)::value;
-    // workgroups a CU by their registers
-    constexpr int WAVES = 8 - (KEEP > 5) - (KEEP > 7), PER_CU = std::max(1, WAVES * 256 / THREADS);
-    hipLaunchKernelGGL((loss_both_kernel<THREADS, KEEP>), dim3(std::min(rows, 256 * PER_CU)),
+    hipLaunchKernelGGL((loss_both_kernel<THREADS, KEEP>),
+                       dim3(std::min(rows, 256 * per_cu(THREADS, KEEP))),
                        dim3(THREADS), 0, at::cuda::getCurrentCUDAStream(),
                        reinterpret_cast<const __hip_bfloat16*>(logits.data_ptr()),
-                       targets.data_ptr<int64_t>(), w.data_ptr<float>(), token_logp.data_ptr<float>(),
+                       targets.data_ptr<int64_t>(), weights, token_logp,
                        lse.data_ptr<float>(), reinterpret_cast<__hip_bfloat16*>(grad.data_ptr()),
-                       rows, V);
+                       loss, counts, rows, V);
   };
   // As many pieces as the row has: a thread's work on pieces past its end is not free, nor
   // a look whether there are any. With 2, 8 pieces of 256 threads and 4, 8, 16, 19 of 1024,
   // with a branch a piece, so, and in two passes, us: 8000 x 8192 68, 55, 53, 69; 8000 x
   // 17000 153, 144, 105, 139; 2400 x 33000 89, 80, 70, 83; 2400 x 66000 185, 170, 146, 163;
   // 300 x 70000 43, 37, 33, 36; 2400 x 152064 320, 356, 317, 389.
-  if (nvec <= 8 * 256) by_pieces<1, 8>(CDIV(nvec, 256), std::integral_constant<int, 256>{}, go);
-  else if (nvec <= 8 * 512) by_pieces<5, 8>(CDIV(nvec, 512), std::integral_constant<int, 512>{}, go);
-  else by_pieces<5, 19>(CDIV(nvec, 1024), std::integral_constant<int, 1024>{}, go);
+  const int threads = threads_of(nvec), pieces = CDIV(nvec, threads);
+  if (threads == 256) by_pieces<1, 8>(pieces, std::integral_constant<int, 256>{}, go);
+  else if (threads == 512) by_pieces<5, 8>(pieces, std::integral_constant<int, 512>{}, go);
+  else by_pieces<5, 19>(pieces, std::integral_constant<int, 1024>{}, go);
   HIP_CHECK_LAST();
-  return {token_logp, lse};
+  return lse;
+}
+
+// loss <- the sum of w * token_logp
+static void sum_rows(const torch::Tensor& token_logp, const torch::Tensor& w,
+                     const torch::Tensor& loss) {
+  hipLaunchKernelGGL(loss_rows_kernel, dim3(1), dim3(1024), 0, at::cuda::getCurrentCUDAStream(),
+                     token_logp.data_ptr<float>(), w.data_ptr<float>(), loss.data_ptr<float>(),
+                     w.numel());
+  HIP_CHECK_LAST();
+}
+
+// Whether a masked loss' row weights are made by a launch ahead, with the sum over rows
+// then in loss_both_kernel, and not by each row from its sequence's whole mask. That launch
+// and the workgroups' meeting cost 5 us more than the sum's own launch, a mask in the rows
+// some 0.7 and 0.5 for each of a thread's loads of it, on every turn of a workgroup. Masks
+// in the rows, ahead, two passes, us: 8 x 200 x 4096 17.0, 22.5, 18.1; 8 x 600 x 4096 31.7,
+// 31.1, 33.8; 4 x 1500 x 4096 40, 33.5, 44; 1 x 16384 x 4096 249, 65, 174; 2000 x 100 x 64
+// 507, 315, 513; 2 x 1200 x 32003 65, 64, 95; 8 x 100 x 152064 110, 111, 117; 8 x 301 x
+// 152064 325, 323, 360; 1 x 2400 x 152064 339, 322, 371.
+static bool weights_ahead(int rows, int T, int nvec) {
+  const int threads = threads_of(nvec), grid = 256 * per_cu(threads, CDIV(nvec, threads));
+  return std::max(1., (double)rows / grid) * (0.7 + 0.5 * T / threads) > 5.;
 }
 
 // The masked PG/GRPO loss of logits (B, T, V): {loss, row weights (B, T), lse}, and
@@ -506,18 +606,35 @@ static std::vector<torch::Tensor> logprob_loss_fwd(torch::Tensor logits, torch::
   auto stream = at::cuda::getCurrentCUDAStream();
   auto w = torch::empty({B, T}, logits.options().dtype(at::kFloat));
   auto loss = torch::empty({}, w.options());
-  #define WEIGHTS(M)                                                                  \
-    hipLaunchKernelGGL(loss_weights_kernel<M>, dim3(B), dim3(1024), 0, stream,        \
-                       mask.data_ptr<M>(), rewards.data_ptr<float>(),                 \
-                       w.data_ptr<float>(), B, T, (float)scale)
-  if (grad && mask64) WEIGHTS(int64_t);
-  else if (grad) WEIGHTS(float);
-  #undef WEIGHTS
-  auto lp = grad ? logprob_both(logits, targets, w, *grad) : logprob_lse_fwd(logits, targets);
+  if (grad && weights_ahead(B * T, T, (int)(logits.size(2) / 8))) {
+    // the workgroups' parts and their counts
+    auto parts = torch::empty({(int64_t)B * T + COUNTS}, w.options());
+    auto* counts = reinterpret_cast<uint32_t*>(parts.data_ptr<float>() + (int64_t)B * T);
+    #define WEIGHTS(M)                                                                \
+      hipLaunchKernelGGL(loss_weights_kernel<M>, dim3(B), dim3(1024), 0, stream,      \
+                         mask.data_ptr<M>(), rewards.data_ptr<float>(),               \
+                         w.data_ptr<float>(), counts, B, T, (float)scale)
+    if (mask64) WEIGHTS(int64_t);
+    else WEIGHTS(float);
+    #undef WEIGHTS
+    auto lse = logprob_both(logits, targets, {w.data_ptr<float>()}, *grad, parts.data_ptr<float>(),
+                            loss.data_ptr<float>(), counts);
+    return {loss, w, lse};
+  }
+  if (grad) {
+    auto token_logp = torch::empty({B, T}, w.options());
+    auto lse = logprob_both(logits, targets,
+                            {w.data_ptr<float>(), mask.data_ptr(), mask64, rewards.data_ptr<float>(),
+                             B, T, (float)scale},
+                            *grad, token_logp.data_ptr<float>(), nullptr, nullptr);
+    sum_rows(token_logp, w, loss);
+    return {loss, w, lse};
+  }
+  auto lp = logprob_lse_fwd(logits, targets);
   #define REDUCE(M)                                                                   \
     hipLaunchKernelGGL(loss_reduce_kernel<M>, dim3(1), dim3(1024), 0, stream,         \
                        lp[0].data_ptr<float>(), mask.data_ptr<M>(),                   \
-                       rewards.data_ptr<float>(), grad ? nullptr : w.data_ptr<float>(), \
+                       rewards.data_ptr<float>(), w.data_ptr<float>(),                \
                        loss.data_ptr<float>(), B, T, (float)scale)
   if (mask64) REDUCE(int64_t);
   else REDUCE(float);
@@ -654,13 +771,19 @@ struct LogprobRows : public torch::autograd::Function<LogprobRows> {
     targets = targets.contiguous();
     w = w.contiguous();
     const auto grad = gradient_room(logits, both);
-    auto lp = grad ? logprob_both(logits, targets, w, *grad) : logprob_lse_fwd(logits, targets);
-    auto loss = torch::empty({}, lp[0].options());
-    hipLaunchKernelGGL(loss_rows_kernel, dim3(1), dim3(1024), 0, at::cuda::getCurrentCUDAStream(),
-                       lp[0].data_ptr<float>(), w.data_ptr<float>(), loss.data_ptr<float>(),
-                       logits.size(0));
-    HIP_CHECK_LAST();
-    ctx->save_for_backward({logits, targets, w, lp[1]});
+    torch::Tensor token_logp, lse;
+    if (grad) {
+      token_logp = torch::empty({logits.size(0)}, w.options());
+      lse = logprob_both(logits, targets, {w.data_ptr<float>()}, *grad, token_logp.data_ptr<float>(),
+                         nullptr, nullptr);
+    } else {
+      auto lp = logprob_lse_fwd(logits, targets);
+      token_logp = lp[0];
+      lse = lp[1];
+    }
+    auto loss = torch::empty({}, lse.options());
+    sum_rows(token_logp, w, loss);
+    ctx->save_for_backward({logits, targets, w, lse});
     if (grad) ctx->saved_data["grad"] = *grad;
     return loss;
   }

@@ -935,12 +935,13 @@ def test_loss_edges(B, T, V, dtype, mask_dtype):
 
 
 @pytest.mark.parametrize("B,T,V", [(3, 1300, 301), (1, 20000, 64), (2, 2600, 513), (41, 60, 8192),
-                                   (300, 6, 4097), (2, 150, 40000), (290, 1, 70001), (3, 3, 152065)])
+                                   (300, 6, 4097), (2, 150, 40000), (290, 1, 70001), (3, 3, 152065),
+                                   (2, 1500, 20000), (2, 1200, 40000)])
 @pytest.mark.parametrize("mask_dtype", [torch.int64, torch.float32])
 def test_masked_loss_gradients_made_forward(B, T, V, mask_dtype):
     """Losses large enough for the gradient to be made in the forward pass: an empty mask,
-    parts of a token, more tokens than a workgroup has threads and fewer, rows that walk,
-    of every width class, a target that is no word (its gradient is the softmax alone).
+    parts of a token, more tokens than a workgroup has threads and fewer, weights made of
+    a row's mask and ahead, rows that walk, of every number of threads, a target that is no word (its gradient is the softmax alone).
     What forward made, what is made anew behind it in a kept graph and what is made of a
     scaled loss. The first two have the same weights: a first token of 2^24 that swallows
     others' ones makes its sequence's sum hang on the order, and each 2^-24 by which weights
@@ -1268,6 +1269,41 @@ def test_targets_that_are_no_word(V, dtype):
         assert abs(float(loss.detach()) - float((tok * w).sum().detach())) < 1e-5 * float((tok * w).abs().sum().detach())
         grad, = torch.autograd.grad(loss * scale, leaf)
         assert _rel(grad, ref * scale) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("B,T,V", [(3, 700, 512), (2, 300, 16391), (1, 40, 152064), (1, 20000, 64),
+                                   (2, 1200, 33000)])
+def test_masked_loss_in_a_graph(B, T, V):
+    """A captured loss and its gradient, made forward, replayed on other values with eager
+    ones in between: the workgroups' sums meet anew each time, in the same order."""
+    from distrl_llm_amd.ops import functional as OF
+    g = torch.Generator("cuda").manual_seed(V)
+    leaf = torch.randn(B, T, V, generator=g, device="cuda").bfloat16().requires_grad_()
+    targets = torch.randint(0, V, (B, T), generator=g, device="cuda")
+    mask = (torch.rand(B, T, generator=g, device="cuda") < 0.8).long()
+    rewards = torch.randn(B, generator=g, device="cuda")
+
+    def call():
+        loss = OF.logprob_loss(leaf, targets, mask, rewards, 0.5)
+        return loss.detach(), torch.autograd.grad(loss, leaf, torch.ones_like(loss))[0]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for _ in range(4):
+        with torch.no_grad():
+            leaf.copy_(torch.randn(B, T, V, generator=g, device="cuda"))
+            rewards.normal_(generator=g)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in out]
+        want = call()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
 @pytest.mark.parametrize("masked", [False, True])
