@@ -282,25 +282,26 @@ void loss_anew_kernel(const T* __restrict__ logits, const int64_t* __restrict__ 
     loss_bwd_row<T, THREADS>(logits, targets, w, lse, dloss, dlogits, V, rows - 1 - row);
 }
 
-// Both passes at once, where the gradient will be asked for: a workgroup holds a row in
-// registers, KEEP pieces of 8 values a thread, makes its log-sum-exp and writes the
-// gradient for a dloss of 1, so that logits are read once. As a piece is written the
-// next row's takes its registers: a workgroup walks rows, and reads and writes are on
-// their way all the time. Bound by memory: 2408 rows of 152064, a quarter of weight zero,
-// 308 us (4.75 TB/s read and written), 133 and 222 in two passes; with the sum over rows
-// and the look at dloss 356 -> 320. Loads or stores through or past the caches are even.
-// With loss and counts the rows' weighted sum is made here too: a workgroup's part of it goes
-// through token_logp (an element a workgroup) to the last to end, which adds them up in
-// their order.
+// Rows' weights, or what they are made of and where they go
 struct RowWeights {
-  float* w;                   // of each row; made by it where there is
-  const void* mask;           // (B, T), int64 or fp32, with rewards as the loss has them
+  float* w;
+  const void* mask;           // (B, T), int64 or fp32, or null: w is there
   bool mask64;
   const float* rewards;
   int B, T;
   float scale;
 };
 
+// Both passes at once, where the gradient will be asked for: a workgroup holds a row in
+// registers, KEEP pieces of 8 values a thread, makes its log-sum-exp and writes the
+// gradient for a dloss of 1, so that logits are read once. As a piece is written the
+// next row's takes its registers: a workgroup walks rows, and reads and writes are on
+// their way all the time. Bound by memory: 2408 rows of 152064, a quarter of weight zero,
+// 308 us (4.75 TB/s read and written), 133 and 222 in two passes; with the sum over rows
+// and the look at dloss 356 -> 315. Loads or stores through or past the caches are even.
+// With loss and counts the rows' weighted sum is made here too: a workgroup's part of it goes
+// through token_logp (an element a workgroup) to the last to end, which adds them up in
+// their order.
 template <int THREADS, int KEEP>
 __global__ __launch_bounds__(THREADS)
 void loss_both_kernel(const __hip_bfloat16* __restrict__ logits, const int64_t* __restrict__ targets,
